@@ -419,7 +419,7 @@ def main():
                      "valu_floor_from": "profiles/accumulate_knn_cfg4_sq_tcc_counters.txt @ %s" %
                                         valu_floor["measured_at"] if valu_floor else None,
                      "frac_of_achievable": round(max(floors_ms) / grad_ms[0], 4),
-                     "forward": {"kernel": "accumulate_fwd_wave_kernel, same workload, one launch",
+                     "forward": {"kernel": "accumulate_fwd_rows_kernel, same workload, one launch",
                                  "achieved": round(bytes_fwd / (fwd_ms[0] * 1e-3) / 1e9, 1),
                                  "frac": round(bytes_fwd / (fwd_ms[0] * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                                  "traffic": traffic["forward"] if traffic else None,

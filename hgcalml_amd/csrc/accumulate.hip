@@ -144,208 +144,169 @@ __global__ __launch_bounds__(256) void accumulate_fwd_kernel(const float *__rest
 }
 
 
-// ================================================================== wave-per-vertex kernels (F >= 64)
+// ================================================================== row kernel: 16 lanes per vertex
 //
-// One wave64 owns one vertex; lane l owns features [l*VEC, l*VEC+VEC) of every
-// block of 64*VEC features. The vertex index is wave-uniform, so the neighbour
-// indices and weights of its row come in through scalar loads, and gathered
-// rows are fetched with buffer loads whose address is
-//   descriptor base + scalar row offset + per-lane column offset,
-// i.e. no vector ALU is spent on addressing. The scalar row offset is not part
-// of the hardware's range check, so every row index is validated on the scalar
-// side before it is used. Chunks of U neighbour slots without
-// padding take a branch-free path with all U row loads in flight.
+// One group of 16 lanes owns a vertex and up to 64 of its features (four groups per wave), lane l
+// the VEC features from l*VEC on. The row offsets and weights of 16 slots are loaded by the group's
+// lanes at once; per slot they arrive as DPP operands, so a slot costs 2 + 5 * VEC vector
+// instructions for four groups, and a gathered row is one 16-byte load per lane. Bound by vector
+// issue with the L1 return path close behind.
+// 150,000 vertices, K = 64, F = 64 in bin order: 190 us with one wave per vertex and dword loads
+// -> 112 us; a million, K = 64, F = 128: 2.21 -> 1.9 ms.
+// A slot without a neighbour aims out of range and has weight 0: it adds 0 to a sum that started
+// at +0 and is masked out of the maximum; four slots in a row that all four groups have take the
+// path without the mask.
 
+constexpr int kNoSelf = 1 << 30;
 
-// one slot of the forward recurrence for the VEC features of this lane
-template <int VEC, bool MAX, bool SEED>
-__device__ __forceinline__ void fwd_slot(const float (&x)[VEC], float wn, int slot, float (&sum)[VEC],
-                                         float (&best)[VEC], int (&arg)[VEC]) {
+// slots Q*4 .. Q*4+3 of the current 16. VALID: every group has a neighbour in each of them
+template <int VEC, bool MAX, int Q, bool VALID>
+__device__ __forceinline__ void four_slots(__amdgpu_buffer_rsrc_t rows, uint32_t offset, float weight, uint64_t valid,
+                                           uint64_t seeds, uint32_t lane_bytes, float (&sum)[VEC], float (&best)[VEC],
+                                           int (&arg)[VEC]) {
+    float x[4][VEC];
+    load_cols<VEC>(rows, group_bcast<Q * 4>(offset) + lane_bytes, x[0]);
+    load_cols<VEC>(rows, group_bcast<Q * 4 + 1>(offset) + lane_bytes, x[1]);
+    load_cols<VEC>(rows, group_bcast<Q * 4 + 2>(offset) + lane_bytes, x[2]);
+    load_cols<VEC>(rows, group_bcast<Q * 4 + 3>(offset) + lane_bytes, x[3]);
+    const float w[4] = {group_bcast<Q * 4>(weight), group_bcast<Q * 4 + 1>(weight), group_bcast<Q * 4 + 2>(weight),
+                        group_bcast<Q * 4 + 3>(weight)};
 #pragma unroll
-    for (int e = 0; e < VEC; ++e) {
-        const float wf = x[e] * wn;
-        sum[e] = sum[e] + wf;
-        if (MAX) {
-            if (SEED) {  // slot 0 always seeds the maximum
-                best[e] = wf;
-                arg[e] = slot;
-            } else {
-                const bool take = wf >= best[e];  // ">=": a later slot wins ties
-                best[e] = take ? wf : best[e];
-                arg[e] = take ? slot : arg[e];
+    for (int u = 0; u < 4; ++u) {
+        // the groups that have a neighbour here: bit Q*4+u of each group's 16, spread over the group
+        const uint64_t first_lanes = (valid >> (Q * 4 + u)) & 0x0001000100010001ull;
+        const uint64_t has = (first_lanes << 16) - first_lanes;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            const float wf = x[u][e] * w[u];
+            sum[e] = sum[e] + wf;
+            if (MAX) {
+                uint64_t take = __builtin_amdgcn_ballot_w64(wf >= best[e]);  // ">=": a later slot wins ties
+                if (Q == 0 && u == 0) take |= seeds;                         // slot 0 always seeds the maximum
+                if (!VALID) take &= has;
+                const bool t = __builtin_amdgcn_inverse_ballot_w64(take);
+                best[e] = t ? wf : best[e];
+                arg[e] = t ? Q * 4 + u : arg[e];
             }
         }
     }
 }
 
-// Up to U slots [n_begin, n_end) of a vertex's row where some have no neighbour,
-// or the short last chunk of a row: index and weight of slot n_begin + l sit in
-// lane l and are broadcast with v_readlane (no arrays of scalars to keep alive),
-// all rows are in flight together, a slot without a neighbour fetches row 0 and
-// is skipped. Returns n_begin so that the caller's loop advances as for a full chunk.
-// (EXPW: the row's weights wait in LDS, w_lds[n] for slot n.)
-template <int VEC, bool MAX, int U, bool EXPW>
-__device__ __forceinline__ int partial_chunk(const RowMatrix &X, const int *__restrict__ irow,
-                                             const float *__restrict__ wrow, const float *w_lds, int n_begin, int n_end,
-                                             int n_vert, uint32_t lane_bytes, float (&sum)[VEC], float (&best)[VEC],
-                                             int (&arg)[VEC]) {
-    const int lane = lane_id();
-    const int n_mine = min(n_begin + lane, n_end - 1);
-    const int j_lane = n_begin + lane < n_end ? irow[n_mine] : -1;
-    const float w_lane = EXPW ? 0.f : wrow[n_mine];
-    const uint64_t valid = __ballot((uint32_t)j_lane < (uint32_t)n_vert);  // bit l: slot n_begin + l has a neighbour
-    float x[U][VEC];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const int j = __builtin_amdgcn_readlane(j_lane, u);
-        X.load<VEC>((valid >> u) & 1ull ? j : 0, lane_bytes, x[u]);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        if (!((valid >> u) & 1ull)) continue;  // wave-uniform
-        const float w = EXPW ? w_lds[n_begin + u]
-                             : __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(w_lane), u));
-        if (n_begin + u == 0)
-            fwd_slot<VEC, MAX, true>(x[u], w, 0, sum, best, arg);
-        else
-            fwd_slot<VEC, MAX, false>(x[u], w, n_begin + u, sum, best, arg);
-    }
-    return n_begin;
-}
-
-// EXPW (rows of 64 slots or fewer): `w` holds distances; lane n turns the distance of slot n into
-// the weight exp(-d) (modules/accknn_op.py:52, there a framework op of its own in front of the
-// kernel), writes it to w_out for the gradient and to LDS, from where every lane reads the slots'
-// weights (same address in all lanes) instead of the scalar loads.
+// EXPW: `w` holds distances, the weights exp(-d) are used and written to w_out for the gradient
+// (modules/accknn_op.py:52, there a framework op of its own in front of the kernel).
 template <int VEC, bool MAX, bool EXPW>
-__global__ __launch_bounds__(256) void accumulate_fwd_wave_kernel(const float *__restrict__ w,
+__global__ __launch_bounds__(256) void accumulate_fwd_rows_kernel(const float *__restrict__ w,
                                                                   const float *__restrict__ feat,
                                                                   const int *__restrict__ idx, float *__restrict__ out,
                                                                   int *__restrict__ out_maxidx,
                                                                   unsigned char *__restrict__ out_maxslot, int n_vert,
-                                                                  int K, int F, int out_cols, float kf,
+                                                                  int K, int F, int blocks, int out_cols, float kf,
                                                                   const int *__restrict__ order,
                                                                   float *__restrict__ w_out) {
-    constexpr int U = VEC == 4 ? 8 : 16;
-    const int v = wave_vertex(order, n_vert);
-    if (v >= n_vert) return;
+    constexpr int kNone = -(1 << 30);  // no maximum yet (slots are counted relative to the current 16)
+    const int l = threadIdx.x & (kRowLanes - 1);
+    const GroupTask task = group_task(order, n_vert, blocks);
+    const bool live = task.vertex >= 0;
+    const int v = live ? task.vertex : 0;
     const int *irow = idx + (size_t)v * K;
     const float *wrow = w + (size_t)v * K;
-    __shared__ float s_weights[EXPW ? 4 : 1][kWave];
-    const float *w_lds = s_weights[EXPW ? threadIdx.x >> 6 : 0];
-    if (EXPW) {
-        const int n = lane_id();
-        float w_n = 0.f;
-        if (n < K) {
-            w_n = expf(-wrow[n]);
-            w_out[(size_t)v * K + n] = w_n;
-        }
-        s_weights[threadIdx.x >> 6][n] = w_n;
-        wave_lds_fence();
-    }
-    const RowMatrix X(feat, n_vert, F);
-    int first_self = -1;  // first slot that names the vertex itself (wave-uniform, scalar ALU)
+    const __amdgpu_buffer_rsrc_t rows = make_rows(feat, (unsigned long long)n_vert * F * 4ull);
+    const int f = task.block * (kRowLanes * VEC) + l * VEC;
+    const uint32_t lane_bytes = (uint32_t)f * 4u;
 
-    for (int fb = lane_id() * VEC; fb < F; fb += kWave * VEC) {
-        const uint32_t lane_bytes = (uint32_t)fb * 4u;
-        float sum[VEC], best[VEC];
-        int arg[VEC];  // SLOT of the maximum, -1: none (translated to an index at the end)
+    float sum[VEC], best[VEC];
+    int arg[VEC];
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) {
-            sum[e] = 0.f;
-            best[e] = 0.f;
-            arg[e] = -1;
+    for (int e = 0; e < VEC; ++e) {
+        sum[e] = 0.f;
+        best[e] = 0.f;
+        arg[e] = kNone;
+    }
+    int first_self = kNoSelf;  // first slot that names the vertex itself
+    bool in_row = live && l < K;
+    int j_next = in_row ? irow[l] : -1;
+    float w_next = in_row ? wrow[l] : 0.f;
+    int c0 = 0;
+    for (; c0 < K; c0 += kRowLanes) {
+        const int j = j_next;
+        float wn = w_next;
+        if (EXPW) {
+            wn = expf(-wn);
+            if (in_row && task.block == 0) w_out[(size_t)v * K + c0 + l] = wn;
         }
-        int n0 = 0;
-        for (; n0 + U <= K; n0 += U) {
-            int j[U];
-            float wn[U];
-            float x[U][VEC];
-            uint32_t j_max = 0;  // unsigned: a negative index is the largest
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                j[u] = irow[n0 + u];
-                wn[u] = EXPW ? w_lds[n0 + u] : wrow[n0 + u];
-                j_max = max(j_max, (uint32_t)j[u]);
-            }
-            const bool all_valid = j_max < (uint32_t)n_vert;
-            if (MAX) {
-                int fs = -1;
-#pragma unroll
-                for (int u = U - 1; u >= 0; --u)
-                    if (j[u] == v) fs = n0 + u;
-                if (first_self < 0) first_self = fs;
-            }
-            if (all_valid) {  // wave-uniform: the common, padding-free chunk
-#pragma unroll
-                for (int u = 0; u < U; ++u) X.load<VEC>(j[u], lane_bytes, x[u]);
-                if (n0 == 0) {
-                    fwd_slot<VEC, MAX, true>(x[0], wn[0], 0, sum, best, arg);
-#pragma unroll
-                    for (int u = 1; u < U; ++u) fwd_slot<VEC, MAX, false>(x[u], wn[u], u, sum, best, arg);
-                } else {
-#pragma unroll
-                    for (int u = 0; u < U; ++u) fwd_slot<VEC, MAX, false>(x[u], wn[u], n0 + u, sum, best, arg);
-                }
-            } else {
-                n0 = partial_chunk<VEC, MAX, U, EXPW>(X, irow, wrow, w_lds, n0, n0 + U, n_vert, lane_bytes, sum, best,
-                                                      arg);
-            }
-        }
-        if (n0 < K) {  // K not a multiple of U
-            if (MAX) {
-                const int n_mine = min(n0 + lane_id(), K - 1);
-                const uint64_t self = __ballot(n0 + lane_id() < K && irow[n_mine] == v);
-                if (first_self < 0 && self) first_self = n0 + __builtin_ctzll(self);
-            }
-            if (K - n0 <= 4)
-                partial_chunk<VEC, MAX, 4, EXPW>(X, irow, wrow, w_lds, n0, K, n_vert, lane_bytes, sum, best, arg);
-            else if (K - n0 <= 8 || U == 8)
-                partial_chunk<VEC, MAX, 8, EXPW>(X, irow, wrow, w_lds, n0, K, n_vert, lane_bytes, sum, best, arg);
-            else
-                partial_chunk<VEC, MAX, 16, EXPW>(X, irow, wrow, w_lds, n0, K, n_vert, lane_bytes, sum, best, arg);
-        }
-        float mean[VEC];
-#pragma unroll
-        for (int e = 0; e < VEC; ++e) mean[e] = sum[e] / kf;
-        store_vec_once<VEC>(out + (size_t)v * out_cols + fb, mean);
+        in_row = live && c0 + kRowLanes + l < K;
+        j_next = in_row ? irow[c0 + kRowLanes + l] : -1;
+        w_next = in_row ? wrow[c0 + kRowLanes + l] : 0.f;
+
+        const bool has_row = (uint32_t)j < (uint32_t)n_vert;
+        const uint32_t offset = has_row ? (uint32_t)j * (uint32_t)(F * 4) : kNoRow;
+        wn = has_row ? wn : 0.f;
+        const uint64_t valid = __builtin_amdgcn_ballot_w64(has_row);
+        const uint64_t seeds = c0 == 0 ? ~0ull : 0ull;
         if (MAX) {
-            store_vec_once<VEC>(out + (size_t)v * out_cols + F + fb, best);
-            int argidx[VEC];
+            first_self = live && j == v ? min(first_self, c0 + l) : first_self;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) argidx[e] = arg[e] < 0 ? 0 : irow[arg[e]];
-            store_vec_i<VEC>(out_maxidx + (size_t)v * F + fb, argidx);
-            if (out_maxslot) {
-                // slot of the maximum; for a repeated self reference its first slot,
-                // which is the one the reference's gradient credits. A feature without a
-                // maximum (slot 0 empty, every product negative) reports index 0, and the
-                // reference's gradient compares indices: it credits the slot that names
-                // vertex 0, if the row has one.
-                bool none = false;
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) none = none || arg[e] < 0;
-                int first_zero = -1;
-                if (__ballot(none) != 0) {  // wave-uniform, rare
-                    for (int n0z = 0; n0z < K && first_zero < 0; n0z += kWave) {
-                        const int n = n0z + lane_id();
-                        const uint64_t zero = __ballot(n < K && irow[min(n, K - 1)] == 0);
-                        if (zero != 0) first_zero = n0z + __builtin_ctzll(zero);
-                    }
-                }
-                uint32_t packed = 0;
-#pragma unroll
-                for (int e = 0; e < VEC; ++e) {
-                    int sl = arg[e];
-                    if (sl < 0) sl = first_zero;
-                    else if (argidx[e] == v) sl = first_self;
-                    packed |= (uint32_t)(sl < 0 ? 255 : sl) << (8 * e);
-                }
-                unsigned char *dst = out_maxslot + (size_t)v * F + fb;
-                if constexpr (VEC == 4) *reinterpret_cast<uint32_t *>(dst) = packed;
-                else if constexpr (VEC == 2) *reinterpret_cast<uint16_t *>(dst) = (uint16_t)packed;
-                else *dst = (unsigned char)packed;
-            }
+            for (int e = 0; e < VEC; ++e) arg[e] -= kRowLanes;
         }
+#define HGC_FOUR(Q)                                                                                        \
+    if (c0 + (Q) * 4 < K) {                                                                                \
+        constexpr uint64_t all = 0x000f000f000f000full << ((Q) * 4);                                       \
+        if ((valid & all) == all)                                                                          \
+            four_slots<VEC, MAX, Q, true>(rows, offset, wn, valid, seeds, lane_bytes, sum, best, arg);     \
+        else                                                                                               \
+            four_slots<VEC, MAX, Q, false>(rows, offset, wn, valid, seeds, lane_bytes, sum, best, arg);    \
+    }
+        HGC_FOUR(0)
+        HGC_FOUR(1)
+        HGC_FOUR(2)
+        HGC_FOUR(3)
+#undef HGC_FOUR
+    }
+    const int last_base = c0 - kRowLanes;  // what `arg` is relative to
+    if (MAX && out_maxslot) first_self = group_min(first_self);
+    const int left = F - f;
+    if (!live || left <= 0) return;
+    float mean[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) mean[e] = sum[e] / kf;
+    store_cols<VEC>(out + (size_t)v * out_cols + f, mean, left);
+    if (!MAX) return;
+    store_cols<VEC>(out + (size_t)v * out_cols + F + f, best, left);
+    int slot[VEC], argidx[VEC];
+    bool none = false;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+        slot[e] = arg[e] + last_base;
+        none = none || slot[e] < 0;
+        argidx[e] = slot[e] < 0 ? 0 : irow[slot[e]];
+    }
+    store_cols<VEC>(out_maxidx + (size_t)v * F + f, argidx, left);
+    if (!out_maxslot) return;
+    // slot of the maximum; for a repeated self reference its first slot, which is the one the
+    // reference's gradient credits. A feature without a maximum (slot 0 empty, every product
+    // negative) reports index 0, and the reference's gradient compares indices: it credits the slot
+    // that names vertex 0, if the row has one.
+    int first_zero = 255;
+    if (none) {  // rare
+        for (int n = 0; n < K; ++n)
+            if (irow[n] == 0) {
+                first_zero = n;
+                break;
+            }
+    }
+    uint32_t packed = 0;
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+        const int sl = slot[e] < 0 ? first_zero : argidx[e] == v ? first_self : slot[e];
+        packed |= (uint32_t)(sl & 255) << (8 * e);
+    }
+    unsigned char *dst = out_maxslot + (size_t)v * F + f;
+    if (VEC == 4 && (F & 3) == 0) {
+        *reinterpret_cast<uint32_t *>(dst) = packed;
+    } else {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e)
+            if (e < left) dst[e] = (unsigned char)(packed >> (8 * e));
     }
 }
 
@@ -798,32 +759,37 @@ int accumulate_forward(const float *d_distances, const float *d_feat, const int 
     hipStream_t s = as_stream(stream);
     const uintptr_t align_or = reinterpret_cast<uintptr_t>(d_feat) | reinterpret_cast<uintptr_t>(d_out_feat) |
                               reinterpret_cast<uintptr_t>(d_out_maxidxs);
-    // the wave kernels address rows through 32-bit buffer offsets
-    const bool fits_32bit = (unsigned long long)n_vert * (unsigned long long)n_out_feat * 4ull < (1ull << 32);
-    const bool wave_kernel = n_feat >= 16 && fits_32bit;
-    const bool exp_in_kernel = d_out_weights && wave_kernel && n_neigh <= kWave;
-    if (d_out_weights && !exp_in_kernel) {  // the weights in a pass of their own, then as if they had been given
+    // the row kernel addresses rows through 32-bit buffer offsets
+    const bool row_kernel = n_feat >= 16 && (unsigned long long)n_vert * (unsigned long long)n_feat * 4ull <= kMaxRowBytes;
+    if (d_out_weights && !row_kernel) {  // the weights in a pass of their own, then as if they had been given
         const int rc = hgc_exp_neg(d_distances, d_out_weights, (long long)n_vert * n_neigh, stream);
         if (rc) return rc;
         d_distances = d_out_weights;
     }
-    if (wave_kernel) {  // one wave per vertex (lanes beyond a short row stay idle)
-        const int vec = wave_vec(n_feat, align_or);
-        const dim3 grid(ceil_div(n_vert, 4)), block(256);
+    if (row_kernel) {
+        int vec, blocks;
+        row_shape(n_feat, vec, blocks);
+        const dim3 grid(ceil_div((long long)n_vert * blocks, 256 / kRowLanes)), block(256);
 #define HGC_FWD(VEC, MAX, EXPW)                                                                                     \
-    accumulate_fwd_wave_kernel<VEC, MAX, EXPW><<<grid, block, 0, s>>>(d_distances, d_feat, d_idxs, d_out_feat,         \
+    accumulate_fwd_rows_kernel<VEC, MAX, EXPW><<<grid, block, 0, s>>>(d_distances, d_feat, d_idxs, d_out_feat,         \
                                                                      d_out_maxidxs, d_out_maxslots, n_vert, n_neigh, \
-                                                                     n_feat, n_out_feat, divisor, d_order, d_out_weights)
+                                                                     n_feat, blocks, n_out_feat, divisor, d_order,   \
+                                                                     d_out_weights)
 #define HGC_FWD_VEC(MAX, EXPW)                                                                                      \
-    if (vec == 4) HGC_FWD(4, MAX, EXPW); else if (vec == 2) HGC_FWD(2, MAX, EXPW); else HGC_FWD(1, MAX, EXPW)
+    switch (vec) {                                                                                                  \
+        case 1: HGC_FWD(1, MAX, EXPW); break;                                                                       \
+        case 2: HGC_FWD(2, MAX, EXPW); break;                                                                       \
+        case 3: HGC_FWD(3, MAX, EXPW); break;                                                                       \
+        default: HGC_FWD(4, MAX, EXPW);                                                                             \
+    }
         if (mean_and_max) {
-            if (exp_in_kernel) { HGC_FWD_VEC(true, true); } else { HGC_FWD_VEC(true, false); }
+            if (d_out_weights) { HGC_FWD_VEC(true, true) } else { HGC_FWD_VEC(true, false) }
         } else {
-            if (exp_in_kernel) { HGC_FWD_VEC(false, true); } else { HGC_FWD_VEC(false, false); }
+            if (d_out_weights) { HGC_FWD_VEC(false, true) } else { HGC_FWD_VEC(false, false) }
         }
 #undef HGC_FWD_VEC
 #undef HGC_FWD
-        return check_launch("accumulate_fwd_wave_kernel");
+        return check_launch("accumulate_fwd_rows_kernel");
     }
     const bool vec4 = (n_feat % 4 == 0) && (align_or & 15u) == 0;
     const long long threads = (long long)n_vert * (vec4 ? n_feat / 4 : n_feat);

@@ -127,6 +127,111 @@ __device__ __forceinline__ int wave_vertex(const int *__restrict__ order, int n_
     return (uint32_t)v < (uint32_t)n_vert ? v : n_vert;
 }
 
+// ---- four vertices per wave: one vertex per DPP row of 16 lanes ----
+//
+// Gathered rows come through the vector L1, whose return path moves 64 bytes a cycle only for
+// 16-byte loads: rows of 256 bytes gathered out of L2 with one dword per lane (one row per
+// instruction) run at 18 TB/s, with four dwords per lane and four rows per instruction at
+// 29 to 31 TB/s (rows of 512 bytes: 18 -> 31; a million rows of 512 bytes, window +-2000:
+// 17.6 -> 24.6 TB/s). So 16 lanes own a vertex, each with VEC = 1 to 4 consecutive features of a
+// block of 16 * VEC columns (wider rows: one group per block), and what belongs to one slot (row offset, weight) sits in one lane of the
+// group and reaches the others as a DPP operand (row_newbcast).
+constexpr int kRowLanes = 16;
+
+template <int U>
+__device__ __forceinline__ uint32_t group_bcast(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150 + U, 0xf, 0xf, true);
+}
+template <int U>
+__device__ __forceinline__ float group_bcast(float v) {
+    return __uint_as_float(group_bcast<U>(__float_as_uint(v)));
+}
+
+// minimum over the 16 lanes of a group, in every lane (DPP row_ror)
+__device__ __forceinline__ int group_min(int v) {
+    v = min(v, __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, true));
+    v = min(v, __builtin_amdgcn_update_dpp(0, v, 0x124, 0xf, 0xf, true));
+    v = min(v, __builtin_amdgcn_update_dpp(0, v, 0x122, 0xf, 0xf, true));
+    return min(v, __builtin_amdgcn_update_dpp(0, v, 0x121, 0xf, 0xf, true));
+}
+
+// What this lane's group works on: a vertex (see wave_vertex; -1 beyond the last one) and, for rows
+// of more than 16 * VEC features, one of its `blocks` of columns (neighbouring groups take the
+// blocks of one vertex).
+struct GroupTask {
+    int vertex, block;
+};
+__device__ __forceinline__ GroupTask group_task(const int *__restrict__ order, int n_vert, int blocks) {
+    const int tile = xcd_contiguous_block(blockIdx.x, gridDim.x);
+    const uint32_t group = (uint32_t)tile * (blockDim.x / kRowLanes) + threadIdx.x / kRowLanes;
+    const uint32_t i = blocks == 1 ? group : blocks == 2 ? group >> 1 : group / (uint32_t)blocks;
+    const int v = i < (uint32_t)n_vert ? (order ? order[i] : (int)i) : -1;
+    return {(uint32_t)v < (uint32_t)n_vert ? v : -1, (int)(group - i * (uint32_t)blocks)};
+}
+
+// A byte offset beyond every matrix the row kernels take (kMaxRowBytes): the hardware's range check
+// turns a load there into 0 without a memory access. Column offsets added to it do not wrap.
+constexpr uint32_t kNoRow = 0xffff0000u;
+constexpr unsigned long long kMaxRowBytes = 0xffff0000ull;
+
+// VEC consecutive 4-byte elements at byte offset `offset` of a raw buffer
+template <int VEC>
+__device__ __forceinline__ void load_cols(__amdgpu_buffer_rsrc_t rsrc, uint32_t offset, float (&x)[VEC]) {
+    if constexpr (VEC == 4) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)offset, 0, 0);
+        x[0] = __uint_as_float(v[0]); x[1] = __uint_as_float(v[1]);
+        x[2] = __uint_as_float(v[2]); x[3] = __uint_as_float(v[3]);
+    } else if constexpr (VEC == 3) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b96(rsrc, (int)offset, 0, 0);
+        x[0] = __uint_as_float(v[0]); x[1] = __uint_as_float(v[1]); x[2] = __uint_as_float(v[2]);
+    } else if constexpr (VEC == 2) {
+        const auto v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)offset, 0, 0);
+        x[0] = __uint_as_float(v[0]); x[1] = __uint_as_float(v[1]);
+    } else {
+        x[0] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)offset, 0, 0));
+    }
+}
+
+// the first min(VEC, left) of VEC consecutive elements; rows start on 4-byte boundaries only.
+// Result rows are touched once: non-temporal.
+template <int VEC, typename T>
+__device__ __forceinline__ void store_cols(T *p, const T (&x)[VEC], int left) {
+    typedef T vec_t __attribute__((ext_vector_type(VEC == 3 ? 4 : VEC), aligned(4)));
+    if constexpr (VEC == 3) {
+        if (left >= 3) {
+            typedef T pair_t __attribute__((ext_vector_type(2), aligned(4)));
+            pair_t v;
+            v[0] = x[0]; v[1] = x[1];
+            __builtin_nontemporal_store(v, reinterpret_cast<pair_t *>(p));
+            __builtin_nontemporal_store(x[2], p + 2);
+            return;
+        }
+    } else if (left >= VEC) {
+        if constexpr (VEC == 1) {
+            __builtin_nontemporal_store(x[0], p);
+        } else {
+            vec_t v;
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) v[e] = x[e];
+            __builtin_nontemporal_store(v, reinterpret_cast<vec_t *>(p));
+        }
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < VEC; ++e)
+        if (e < left) __builtin_nontemporal_store(x[e], p + e);
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rows(const void *base, unsigned long long bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)(uint32_t)bytes, 0x00020000);
+}
+
+// features per lane and blocks of 16 * vec features of a row of n_feat
+inline void row_shape(int n_feat, int &vec, int &blocks) {
+    blocks = ceil_div(n_feat, 4 * kRowLanes);
+    vec = ceil_div(n_feat, kRowLanes * blocks);
+}
+
 // A dense [rows, cols] matrix of 4-byte elements seen through a raw buffer
 // descriptor (stride 0, num_records = size in bytes, gfx9 data format word).
 struct RowMatrix {
