@@ -48,9 +48,9 @@ class _AccumulateExpFn(torch.autograd.Function):
     def backward(ctx, grad_out, _grad_maxidx):
         weights, features, indices, maxidx, slots = ctx.saved_tensors
         inv_off, inv_slots = ops.cached_inverse_neighbour_index(ctx.indices_ref)
-        gw, gx = torch.ops.hgcalml.accumulate_knn_grad_slots(grad_out.contiguous(), weights, features, indices,
-                                                             maxidx, slots, inv_off, inv_slots)
-        return ops.exp_neg_grad(gw, weights), gx, None, None
+        gd, gx = torch.ops.hgcalml.accumulate_knn_grad_exp_slots(grad_out.contiguous(), weights, features, indices,
+                                                                 maxidx, slots, inv_off, inv_slots)
+        return gd, gx, None, None
 
 
 class _ExpNegFn(torch.autograd.Function):

@@ -33,6 +33,14 @@ int launch_accumulate_grad_fused(const float *g, const float *w, const float *fe
                                  const unsigned char *maxslot, const int *inv_off, const int *inv_slots, float *gw,
                                  float *gfeat, int n_vert, int K, int F, int g_cols, bool mean_and_max, const int *idx,
                                  const int *order, float divisor, hipStream_t s);
+// accumulate_grad_rows.hip: rows of 16 to 128 features; returns 1 when the shape is not covered. gw == nullptr:
+// feature gradient only. negate: gw receives -(gradient * w). scratch may be null.
+size_t accumulate_grad_rows_scratch_bytes(int n_vert, int n_feat, int g_cols, float divisor);
+bool accumulate_grad_rows_covers(int n_feat, int n_neigh, bool mean_and_max, bool slots, unsigned long long g_bytes);
+int launch_accumulate_grad_rows(const float *g, const float *w, const float *feat, const unsigned char *maxslot,
+                                const int *inv_off, const int *inv_slots, float *gw, float *gfeat, int n_vert, int K, int F,
+                                int g_cols, bool mean_and_max, const int *order, float divisor, bool negate, void *scratch,
+                                size_t scratch_bytes, hipStream_t s);
 // accumulate_grad_records.hip: both gradients with the max part read from per-slot
 // records built in `records`; returns 1 when the shape is not covered or the storage is
 // too small (accumulate_grad_records_bytes is 0 where the path does not apply).
@@ -152,7 +160,7 @@ __global__ __launch_bounds__(256) void accumulate_fwd_kernel(const float *__rest
 // instructions for four groups, and a gathered row is one 16-byte load per lane. Bound by vector
 // issue with the L1 return path close behind.
 // 150,000 vertices, K = 64, F = 64 in bin order: 190 us with one wave per vertex and dword loads
-// -> 112 us; a million, K = 64, F = 128: 2.21 -> 1.9 ms.
+// -> 134 us; 240,000, K = 40, F = 32: 221 -> 95 us; a million, K = 64, F = 128: 2.21 -> 1.96 ms.
 // A slot without a neighbour aims out of range and has weight 0: it adds 0 to a sum that started
 // at +0 and is masked out of the maximum; four slots in a row that all four groups have take the
 // path without the mask.
@@ -211,7 +219,9 @@ __global__ __launch_bounds__(256) void accumulate_fwd_rows_kernel(const float *_
     const int *irow = idx + (size_t)v * K;
     const float *wrow = w + (size_t)v * K;
     const __amdgpu_buffer_rsrc_t rows = make_rows(feat, (unsigned long long)n_vert * F * 4ull);
-    const int f = task.block * (kRowLanes * VEC) + l * VEC;
+    // A lane at the end of a row that is no multiple of VEC takes the last VEC columns (never columns of the
+    // next row): what it shares with its neighbour both compute and store alike.
+    const int fb = task.block * (kRowLanes * VEC) + l * VEC, f = min(fb, F - VEC);
     const uint32_t lane_bytes = (uint32_t)f * 4u;
 
     float sum[VEC], best[VEC];
@@ -264,14 +274,13 @@ __global__ __launch_bounds__(256) void accumulate_fwd_rows_kernel(const float *_
     }
     const int last_base = c0 - kRowLanes;  // what `arg` is relative to
     if (MAX && out_maxslot) first_self = group_min(first_self);
-    const int left = F - f;
-    if (!live || left <= 0) return;
+    if (!live || fb >= F) return;
     float mean[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) mean[e] = sum[e] / kf;
-    store_cols<VEC>(out + (size_t)v * out_cols + f, mean, left);
+    store_cols<VEC>(out + (size_t)v * out_cols + f, mean);
     if (!MAX) return;
-    store_cols<VEC>(out + (size_t)v * out_cols + F + f, best, left);
+    store_cols<VEC>(out + (size_t)v * out_cols + F + f, best);
     int slot[VEC], argidx[VEC];
     bool none = false;
 #pragma unroll
@@ -280,7 +289,7 @@ __global__ __launch_bounds__(256) void accumulate_fwd_rows_kernel(const float *_
         none = none || slot[e] < 0;
         argidx[e] = slot[e] < 0 ? 0 : irow[slot[e]];
     }
-    store_cols<VEC>(out_maxidx + (size_t)v * F + f, argidx, left);
+    store_cols<VEC>(out_maxidx + (size_t)v * F + f, argidx);
     if (!out_maxslot) return;
     // slot of the maximum; for a repeated self reference its first slot, which is the one the
     // reference's gradient credits. A feature without a maximum (slot 0 empty, every product
@@ -306,7 +315,7 @@ __global__ __launch_bounds__(256) void accumulate_fwd_rows_kernel(const float *_
     } else {
 #pragma unroll
         for (int e = 0; e < VEC; ++e)
-            if (e < left) dst[e] = (unsigned char)(packed >> (8 * e));
+            dst[e] = (unsigned char)(packed >> (8 * e));
     }
 }
 
@@ -888,13 +897,23 @@ namespace hgc {
 // Gradient shared by accumulate_knn_grad (divisor = K) and push_knn (divisor = 1).
 // Either output may be null: the weight gradient needs neither the inverse index
 // nor the weights, the feature gradient needs neither the features nor the
-// neighbour table.
+// neighbour table. negate: the weights are exp(-d) and the weight gradient leaves as that of d,
+// -(gradient * w). scratch: see launch_accumulate_grad_rows.
 int accumulate_gradient(const float *d_grad_from_out_features, const float *d_distances, const float *d_feat,
                         const int *d_max_feat_indices, const unsigned char *d_max_slots, const int *d_neigh_indices,
                         const int *d_inv_offsets, const int *d_inv_slots, float *d_out_grad_distances,
                         float *d_out_grad_features, int n_vert, int n_neigh, int n_feat, int n_grad_from_out_feat,
                         int mean_and_max, float divisor, const int *d_order, void *records, size_t records_bytes,
-                        hgc_stream_t stream) {
+                        bool negate, void *scratch, size_t scratch_bytes, hgc_stream_t stream) {
+    if (negate && (records || !accumulate_grad_rows_covers(n_feat, n_neigh, mean_and_max, d_max_slots != nullptr,
+                                                           (unsigned long long)n_vert * n_grad_from_out_feat * 4ull))) {
+        const int rc = accumulate_gradient(d_grad_from_out_features, d_distances, d_feat, d_max_feat_indices, d_max_slots,
+                                           d_neigh_indices, d_inv_offsets, d_inv_slots, d_out_grad_distances,
+                                           d_out_grad_features, n_vert, n_neigh, n_feat, n_grad_from_out_feat, mean_and_max,
+                                           divisor, d_order, records, records_bytes, false, scratch, scratch_bytes, stream);
+        if (rc || n_vert == 0) return rc;
+        return hgc_exp_neg_grad(d_out_grad_distances, d_distances, d_out_grad_distances, (long long)n_vert * n_neigh, stream);
+    }
     const bool want_w = d_out_grad_distances != nullptr, want_f = d_out_grad_features != nullptr;
     HGC_REQUIRE(n_vert >= 0 && n_neigh >= 1 && n_feat >= 1, "bad sizes");
     HGC_REQUIRE(n_grad_from_out_feat == n_feat * (mean_and_max ? 2 : 1),
@@ -921,6 +940,13 @@ int accumulate_gradient(const float *d_grad_from_out_features, const float *d_di
                                                       d_out_grad_features, n_vert, n_neigh, n_feat, d_neigh_indices,
                                                       d_order, divisor, records, records_bytes, s);
         if (rc <= 0) return rc;  // 1: shape not covered
+    }
+    if (want_f && (want_w || !mean_and_max)) {
+        const int rc = launch_accumulate_grad_rows(d_grad_from_out_features, d_distances, d_feat, d_max_slots, d_inv_offsets,
+                                                   d_inv_slots, d_out_grad_distances, d_out_grad_features, n_vert, n_neigh,
+                                                   n_feat, n_grad_from_out_feat, mean_and_max != 0, d_order, divisor, negate,
+                                                   scratch, scratch_bytes, s);
+        if (rc <= 0) return rc;
     }
     if (fits_32bit && want_f && (want_w || !mean_and_max)) {
         const int rc = launch_accumulate_grad_fused(d_grad_from_out_features, d_distances, d_feat, d_max_feat_indices,
@@ -1042,7 +1068,27 @@ int hgc_accumulate_knn_grad_slots(const float *d_grad_from_out_features, const f
     return accumulate_gradient(d_grad_from_out_features, d_distances, d_feat, d_max_feat_indices, d_max_slots,
                                d_neigh_indices, d_inv_offsets, d_inv_slots, d_out_grad_distances, d_out_grad_features,
                                n_vert, n_neigh, n_feat, n_grad_from_out_feat, mean_and_max, (float)n_neigh,
-                               d_vertex_order, nullptr, 0, stream);
+                               d_vertex_order, nullptr, 0, false, nullptr, 0, stream);
+}
+
+size_t hgc_accumulate_knn_grad_scratch_bytes(int n_vert, int n_neigh, int n_feat, int mean_and_max) {
+    return accumulate_grad_rows_scratch_bytes(n_vert, n_feat, n_feat * (mean_and_max ? 2 : 1), (float)n_neigh);
+}
+
+int hgc_accumulate_knn_grad_scratch(const float *d_grad_from_out_features, const float *d_distances, const float *d_feat,
+                                    const int *d_max_feat_indices, const unsigned char *d_max_slots,
+                                    const int *d_neigh_indices, const int *d_inv_offsets, const int *d_inv_slots,
+                                    const int *d_vertex_order, float *d_out_grad_distances, float *d_out_grad_features,
+                                    int n_vert, int n_neigh, int n_feat, int n_grad_from_out_feat, int mean_and_max,
+                                    int weights_are_exp, void *scratch, size_t scratch_bytes, hgc_stream_t stream) {
+    HGC_REQUIRE(n_vert <= 0 || (d_out_grad_distances && d_out_grad_features), "null pointer");
+    if (scratch && (!aligned256(scratch) ||
+                    scratch_bytes < hgc_accumulate_knn_grad_scratch_bytes(n_vert, n_neigh, n_feat, mean_and_max)))
+        return fail(HGC_ERR_WORKSPACE, "accumulate_knn_grad_scratch: scratch memory misaligned or too small");
+    return accumulate_gradient(d_grad_from_out_features, d_distances, d_feat, d_max_feat_indices, d_max_slots,
+                               d_neigh_indices, d_inv_offsets, d_inv_slots, d_out_grad_distances, d_out_grad_features,
+                               n_vert, n_neigh, n_feat, n_grad_from_out_feat, mean_and_max, (float)n_neigh,
+                               d_vertex_order, nullptr, 0, weights_are_exp != 0, scratch, scratch_bytes, stream);
 }
 
 size_t hgc_accumulate_knn_grad_records_workspace_bytes(int n_vert, int n_neigh, int n_feat, int mean_and_max) {
@@ -1067,7 +1113,7 @@ int hgc_accumulate_knn_grad_records(const float *d_grad_from_out_features, const
     return accumulate_gradient(d_grad_from_out_features, d_distances, d_feat, d_max_feat_indices, d_max_slots,
                                d_neigh_indices, d_inv_offsets, d_inv_slots, d_out_grad_distances, d_out_grad_features,
                                n_vert, n_neigh, n_feat, n_grad_from_out_feat, mean_and_max, (float)n_neigh,
-                               d_vertex_order, need != 0 ? workspace : nullptr, workspace_bytes, stream);
+                               d_vertex_order, need != 0 ? workspace : nullptr, workspace_bytes, false, nullptr, 0, stream);
 }
 
 int hgc_accumulate_knn_grad(const float *d_grad_from_out_features, const float *d_distances, const float *d_feat,

@@ -17,6 +17,9 @@
 // The same kernel without the dot products (no weight gradient wanted, mean
 // only) is the ordered gather push_knn needs: out[m] = sum of w[v,n] * feat[v].
 //
+// Taken for rows of 129 to 256 features, and for narrower ones when no slot table is given
+// (accumulate_grad_rows.hip has the others).
+//
 // Scalar-unit economy: the per-entry metadata (flat slot -> vertex, row offset,
 // weight, arg-max key) is computed by the 64 lanes for 64 entries at once and
 // broadcast per entry with v_readlane; the hot loop carries no scalar loads and
@@ -321,10 +324,14 @@ int launch_fused(const float *g, const float *w, const float *feat, const int *m
     accumulate_grad_fused_kernel<VEC, NB, MAX, P2, SL, WG, PARTIAL><<<grid, block, 0, s>>>(g, w, feat, maxidx, maxslot, inv_off, \
                                                                                   inv_slots, gw, gfeat, n_vert, K, F,    \
                                                                                   g_cols, div_k, idx, order, divisor)
-    if (!want_w) { if (pow2k) HGC_FUSED(false, true, false, false); else HGC_FUSED(false, false, false, false); }
-    else if (mean_and_max && slots) { if (pow2k) HGC_FUSED(true, true, true, true); else HGC_FUSED(true, false, true, true); }
-    else if (mean_and_max) { if (pow2k) HGC_FUSED(true, true, false, true); else HGC_FUSED(true, false, false, true); }
-    else { if (pow2k) HGC_FUSED(false, true, false, true); else HGC_FUSED(false, false, false, true); }
+    if constexpr (VEC * NB >= 3) {
+        if (!want_w) { if (pow2k) HGC_FUSED(false, true, false, false); else HGC_FUSED(false, false, false, false); }
+        else if (slots) { if (pow2k) HGC_FUSED(true, true, true, true); else HGC_FUSED(true, false, true, true); }
+        else if (mean_and_max) { if (pow2k) HGC_FUSED(true, true, false, true); else HGC_FUSED(true, false, false, true); }
+        else { if (pow2k) HGC_FUSED(false, true, false, true); else HGC_FUSED(false, false, false, true); }
+    } else {  // up to 128 features: without a slot table only, the row kernel takes the others
+        if (pow2k) HGC_FUSED(true, true, false, true); else HGC_FUSED(true, false, false, true);
+    }
 #undef HGC_FUSED
     return check_launch("accumulate_grad_fused_kernel");
 }
@@ -351,6 +358,10 @@ int launch_accumulate_grad_fused(const float *g, const float *w, const float *fe
     // rows are addressed through 32-bit buffer offsets
     if ((unsigned long long)n_vert * (unsigned long long)g_cols * 4ull >= (1ull << 32)) return 1;
     if (maxslot && K > 254) maxslot = nullptr;
+    if (F <= 2 * kWave) {  // accumulate_grad_rows.hip
+        if (!mean_and_max) return 1;
+        maxslot = nullptr;
+    }
     const int vec = partial ? 1 : wave_vec(F, align_or);
     const int nb = ceil_div(F, kWave * vec);
     // wider rows would not fit the register budget that keeps 5+ waves per SIMD resident

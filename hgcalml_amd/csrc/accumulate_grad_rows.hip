@@ -1,0 +1,440 @@
+// Gradient of the GravNet neighbour accumulation for rows of 16 to 128 features: both outputs from one
+// gather over the inverse neighbour index, 16 lanes per target vertex.
+//
+// Reference behaviour restated here:
+//   modules/compiled/accumulate_knn_grad_kernel.cc:36-97   (feature gradient)
+//   modules/compiled/accumulate_knn_grad_kernel.cc:99-165  (weight gradient)
+//
+// For an entry (v, n) of target m's inverse list (idx[v, n] == m) the feature gradient of m adds
+// (g[v,f]/K)*w[v,n] + max part, in ascending (v, n) order (the reference CPU kernel's order: the
+// result is bit-identical to it), and the weight gradient of slot (v, n) is the dot product of
+// g[v, :] with feat[m, :], which the group holds in registers.
+//
+// Layout as in the forward (accumulate_rows.hpp): a group of 16 lanes owns a target and up to 64 of its
+// features, lane l VEC consecutive ones; four groups per wave. The group's lanes fetch the list
+// entries, weights and row offsets of 16 entries at once and hand them on as DPP operands. What a
+// gathered row costs is then one 16-byte load per lane for the mean half, one dword for the
+// arg-max slots and a masked 16-byte load for the few features whose maximum sits at this entry,
+// for four targets together. One wave per target with one dword per lane ran its three loads
+// per entry at the L1's narrow-load rate (95 % busy, vector issue 62 %):
+// 150,000 vertices, K = 64, F = 64 in bin order 574 -> 320 us; K = 40, F = 32, 240,000 590 -> 278 us;
+// a million, K = 64, F = 128 5.75 -> 4.45 ms. What bounds it now: the L1's address and return path
+// (77 and 90 % busy at 150,000 vertices), vector issue at 66 %, and at a million vertices the
+// L2 misses (37 % of the return path's time).
+//
+// The loads of an entry depend on one another (slots, then the max half they gate), so two entries at a
+// time move through a pipeline: slots two steps ahead, rows one step ahead, arithmetic.
+// The dot products of four entries are reduced across the 16 lanes by a transposing exchange (three
+// instructions per value with DPP).
+#include "accumulate_rows.hpp"
+
+namespace hgc {
+
+namespace {
+
+using namespace acc;
+
+// How the mean part (g / divisor) * w is formed with the bits of the two operations:
+//   kPow2    divisor a power of two: g * (w / divisor), exact apart from subnormal quotients
+//   kScaled  g has been divided beforehand
+//   kDivide  an IEEE divide per element and entry
+enum Scale { kPow2, kScaled, kDivide };
+
+struct GradRows {
+    const float *g, *g_max;       // mean and max half of the upstream gradient, rows of `pitch` floats
+    const float *w, *feat;
+    const unsigned char *maxslot;
+    const int *inv_off, *inv_slots, *order;
+    float *gw, *gfeat;
+    unsigned long long g_bytes, g_max_bytes, slot_bytes;  // sizes seen by the hardware's range check
+    int n_vert, K, F, blocks, pitch;
+    FastDiv div_k;
+    float divisor;
+    uint32_t slot_shift;  // maxslot has been moved down by this many bytes onto a multiple of 4
+    bool negate;  // gw receives -(gradient * w): the chain rule through w = exp(-d)
+};
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_from(float v) {
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+
+// sums of val[0..3] over the group's 16 lanes (fixed order): lane l receives that of val[l >> 2]
+__device__ __forceinline__ float group_sum_4(const float (&val)[4], int lane) {
+    const bool upper8 = (lane & 8) != 0, upper4 = (lane & 4) != 0;
+    const float a = (upper8 ? val[2] : val[0]) + dpp_from<0x128>(upper8 ? val[0] : val[2]);  // row_ror:8, lane ^ 8
+    const float b = (upper8 ? val[3] : val[1]) + dpp_from<0x128>(upper8 ? val[1] : val[3]);
+    float r = (upper4 ? b : a) + dpp_from<0x141>(upper4 ? a : b);  // row_half_mirror, lane ^ 7
+    r = r + dpp_from<0x1b>(r);                                     // quad_perm [3,2,1,0], lane ^ 3
+    return r + dpp_from<0xb1>(r);                                  // quad_perm [1,0,3,2], lane ^ 1
+}
+
+// Entry e of a chunk of 16 sits in lane entry_lane(e) of its group (4 x 4 transposed): that is the lane
+// that ends up with the entry's dot product. The map is its own inverse.
+constexpr int entry_lane(int e) { return 4 * (e & 3) + (e >> 2); }
+
+// Does byte E of `packed` equal `key`? One SDWA compare.
+template <int E>
+__device__ __forceinline__ uint64_t byte_is(uint32_t packed, uint32_t key) {
+    uint64_t mask;
+    if constexpr (E == 0) asm("v_cmp_eq_u32_sdwa %0, %1, %2 src0_sel:BYTE_0 src1_sel:DWORD" : "=s"(mask) : "v"(packed), "v"(key));
+    else if constexpr (E == 1) asm("v_cmp_eq_u32_sdwa %0, %1, %2 src0_sel:BYTE_1 src1_sel:DWORD" : "=s"(mask) : "v"(packed), "v"(key));
+    else if constexpr (E == 2) asm("v_cmp_eq_u32_sdwa %0, %1, %2 src0_sel:BYTE_2 src1_sel:DWORD" : "=s"(mask) : "v"(packed), "v"(key));
+    else asm("v_cmp_eq_u32_sdwa %0, %1, %2 src0_sel:BYTE_3 src1_sel:DWORD" : "=s"(mask) : "v"(packed), "v"(key));
+    return mask;
+}
+
+// Arg-max slots of VEC features, packed in one word. ALIGNED: they start on a multiple of VEC (1, 2 or 4)
+// and come in one load of that width; otherwise out of the eight bytes around them, which start on a
+// multiple of 4 and end with the table's last word (last_pair: where the last eight bytes begin).
+template <int VEC, bool ALIGNED>
+struct SlotBytes {
+    uint32_t v[ALIGNED ? 1 : 3];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rsrc, uint32_t offset, uint32_t last_pair) {
+        if constexpr (ALIGNED) {
+            if constexpr (VEC == 4) v[0] = __builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)offset, 0, 0);
+            else if constexpr (VEC == 2) v[0] = __builtin_amdgcn_raw_buffer_load_b16(rsrc, (int)offset, 0, 0);
+            else v[0] = __builtin_amdgcn_raw_buffer_load_b8(rsrc, (int)offset, 0, 0);
+        } else {
+            // (the offset of an entry beyond the list is moved into the table here: its row still reads zeros)
+            const uint32_t at = min(offset & ~3u, last_pair);
+            const auto two = __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)at, 0, 0);
+            v[0] = two[0];
+            v[1] = two[1];
+            v[2] = (offset - at) * 8u;
+        }
+    }
+    __device__ __forceinline__ uint32_t packed() const {
+        if constexpr (ALIGNED) return v[0];
+        else return (uint32_t)((((uint64_t)v[1] << 32) | v[0]) >> (v[2] & 63u));
+    }
+};
+
+// what the group's lanes hold of 16 entries
+struct Entries {
+    uint32_t row;    // byte offset of the gradient row, kNoRow beyond the list
+    uint32_t slots;  // byte offset of the arg-max slots
+    uint32_t key;    // slot of the entry
+    float w, w_mean; // weight, and what the mean half is multiplied by
+};
+
+// Two entries on their way through the pipeline: arg-max slots (requested two steps ahead), gradient
+// rows (requested one step ahead, the max half by the slots), arithmetic.
+template <int VEC, bool MAX, bool ALIGNED>
+struct Step {
+    SlotBytes<VEC, ALIGNED> sb[2];
+    float gm[2][VEC], gx[2][VEC];
+    uint64_t hit[2][VEC];
+
+    template <int E>
+    __device__ __forceinline__ void request_slots(__amdgpu_buffer_rsrc_t MS, const Entries &en, uint32_t lane_col, uint32_t last_pair) {
+        if constexpr (MAX) {
+            sb[0].load(MS, group_bcast<entry_lane(E)>(en.slots) + lane_col, last_pair);
+            sb[1].load(MS, group_bcast<entry_lane(E + 1)>(en.slots) + lane_col, last_pair);
+        }
+    }
+    template <int U>
+    __device__ __forceinline__ void request_row(__amdgpu_buffer_rsrc_t G, __amdgpu_buffer_rsrc_t GX, uint32_t at, uint32_t key) {
+        load_cols<VEC>(G, at, gm[U]);
+        if constexpr (MAX) {
+            const uint32_t slots = sb[U].packed();
+            hit[U][0] = byte_is<0>(slots, key);
+            uint64_t any = hit[U][0];
+            if constexpr (VEC > 1) any |= hit[U][1] = byte_is<1>(slots, key);
+            if constexpr (VEC > 2) any |= hit[U][2] = byte_is<2>(slots, key);
+            if constexpr (VEC > 3) any |= hit[U][3] = byte_is<3>(slots, key);
+            // about F/K features of a row have their maximum at one entry: the other lanes aim out of range
+            load_cols<VEC>(GX, __builtin_amdgcn_inverse_ballot_w64(any) ? at : kNoRow, gx[U]);
+        }
+    }
+    template <int E>
+    __device__ __forceinline__ void request_rows(__amdgpu_buffer_rsrc_t G, __amdgpu_buffer_rsrc_t GX, const Entries &en,
+                                                 uint32_t lane_bytes) {
+        request_row<0>(G, GX, group_bcast<entry_lane(E)>(en.row) + lane_bytes, group_bcast<entry_lane(E)>(en.key));
+        request_row<1>(G, GX, group_bcast<entry_lane(E + 1)>(en.row) + lane_bytes, group_bcast<entry_lane(E + 1)>(en.key));
+    }
+    // An entry beyond its list reads zeros and has weight 0: it adds 0 to a sum that started at +0.
+    // w_max: 0 in the lanes of repeated self references, whose max part counts for the weight gradient only.
+    template <int U, Scale SCALE, bool WGRAD>
+    __device__ __forceinline__ void add(float w, float w_mean, float w_max, const float (&xo)[VEC], const float (&xk)[VEC],
+                                        float divisor, float (&acc)[VEC], float &val) const {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            const float g = gm[U][e];
+            const float part = SCALE == kDivide ? (g / divisor) * w : g * w_mean;
+            if (WGRAD) val = __builtin_fmaf(g, xk[e], val);
+            if constexpr (MAX) {
+                const float gsel = VEC == 1 ? gx[U][e] : __builtin_amdgcn_inverse_ballot_w64(hit[U][e]) ? gx[U][e] : 0.f;
+                if (WGRAD) val = __builtin_fmaf(gsel, xo[e], val);
+                const float part_max = gsel * w_max;
+                const float sum = part + part_max;
+                acc[e] = acc[e] + sum;
+            } else {
+                acc[e] = acc[e] + part;  // the reference's "+ 0" cannot change the sum
+            }
+        }
+    }
+};
+
+__device__ __forceinline__ bool group_lane_of(uint64_t mask, int lane_in_group) {
+    const uint64_t first_lanes = (mask >> lane_in_group) & 0x0001000100010001ull;
+    return __builtin_amdgcn_inverse_ballot_w64((first_lanes << 16) - first_lanes);
+}
+
+template <int VEC, bool MAX, Scale SCALE, bool ALIGNED, bool WGRAD>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) void accumulate_grad_rows_kernel(const GradRows p) {
+    const int lane = lane_id(), l = lane & (kRowLanes - 1);
+    if (WGRAD) {
+        // weight gradient of padded slots: they sort behind the last target's entries
+        const int first = p.inv_off[p.n_vert], total = p.n_vert * p.K;
+        for (long long i = first + (long long)blockIdx.x * blockDim.x + threadIdx.x; i < total;
+             i += (long long)gridDim.x * blockDim.x)
+            p.gw[p.inv_slots[i]] = 0.f;
+    }
+    // The groups of a workgroup trade their targets so that those of a wave have lists of similar length: a
+    // wave runs for as long as its longest one (kNN tables, mean 64 of standard deviation 23: 79 entries of
+    // time per list as they come, 74 sorted; a group pair that shares a target stays together).
+    __shared__ int s_vertex[16], s_block[16], s_begin[16], s_count[16], s_from[16];
+    const int group = threadIdx.x / kRowLanes;
+    {
+        const GroupTask first = group_task(p.order, p.n_vert, p.blocks);
+        if (l == 0) {
+            const int begin = first.vertex >= 0 ? p.inv_off[first.vertex] : 0;
+            s_vertex[group] = first.vertex;
+            s_block[group] = first.block;
+            s_begin[group] = begin;
+            s_count[group] = first.vertex >= 0 ? p.inv_off[first.vertex + 1] - begin : 0;
+        }
+        __syncthreads();
+        const int own = s_count[group], other = s_count[l];
+        const uint64_t below = __builtin_amdgcn_ballot_w64(other < own || (other == own && l < group));
+        if (l == 0) s_from[__popcll((below >> (lane & 48)) & 0xffffull)] = group;
+        __syncthreads();
+    }
+    const int from = s_from[group];
+    const GroupTask task = {s_vertex[from], s_block[from]};
+    const bool live = task.vertex >= 0;
+    const int m = live ? task.vertex : 0;
+    const int begin = s_begin[from], count = s_count[from];
+    // of the wave's longest list
+    const int longest = max(max(readlane_i32(count, 0), readlane_i32(count, 16)),
+                            max(readlane_i32(count, 32), readlane_i32(count, 48)));
+
+    const __amdgpu_buffer_rsrc_t G = make_rows(p.g, p.g_bytes);
+    const __amdgpu_buffer_rsrc_t GX = make_rows(p.g_max, MAX ? p.g_max_bytes : 0);
+    const __amdgpu_buffer_rsrc_t MS = make_rows(p.maxslot, MAX ? p.slot_bytes : 0);
+    const float inv_divisor = 1.f / p.divisor;
+
+    // A lane at the end of a row that is no multiple of VEC, and the lanes behind it, take the last VEC
+    // columns (never columns of the next row): what they share with another lane they compute too
+    // and store alike, but it counts once in the dot products.
+    const int fb = task.block * (kRowLanes * VEC) + l * VEC;
+    const int f = min(fb, p.F - VEC);
+    const uint32_t lane_bytes = (uint32_t)f * 4u, lane_col = (uint32_t)f + p.slot_shift;
+    const uint32_t last_pair = (uint32_t)p.slot_bytes - 8u;
+    float xo[VEC], xk[VEC], acc[VEC];
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+        xo[e] = WGRAD && live && f + e >= fb ? p.feat[(size_t)m * p.F + f + e] : 0.f;
+        xk[e] = SCALE == kScaled ? xo[e] : (float)((double)xo[e] * (1.0 / (double)p.divisor));
+        acc[e] = 0.f;
+    }
+
+    const int *list = p.inv_slots + begin + entry_lane(l);
+    const int mine = count - entry_lane(l);  // this lane has an entry of chunk c0 if c0 < mine
+    auto entries_of = [&](int slot, float w, int c0) {
+        Entries en;
+        const bool here = c0 < mine;
+        const int v = fast_div(slot, p.div_k);
+        en.key = (uint32_t)(slot - v * p.K);
+        en.row = here ? (uint32_t)v * (uint32_t)(p.pitch * 4) : kNoRow;
+        en.slots = here ? (uint32_t)v * (uint32_t)p.F : kNoRow;
+        en.w = w;
+        en.w_mean = SCALE == kPow2 ? w * inv_divisor : w;
+        return en;
+    };
+
+    // slots of the list two chunks ahead, weights and offsets one chunk ahead
+    int slot = 0 < mine ? list[0] : 0;
+    int slot_next = kRowLanes < mine ? list[kRowLanes] : 0;
+    Entries en = entries_of(slot, 0 < mine ? p.w[slot] : 0.f, 0);
+    int self_key = 0;
+    bool self_seen = false;
+    uint64_t repeats = 0;
+    // Entries that name the target itself: the first one (lowest slot) carries the max part; later ones
+    // (padding by repeated self references) are compared with that slot too, for the weight gradient.
+    auto mark_repeats = [&](Entries &e, int c0) {
+        uint64_t rep = 0;
+        if (MAX) {
+            const bool self = c0 < mine && e.row == (uint32_t)m * (uint32_t)(p.pitch * 4);
+            if (__builtin_amdgcn_ballot_w64(self)) {
+                const int lowest = group_min(self ? (int)e.key : 1 << 30);
+                if (!self_seen && lowest < (1 << 30)) self_key = lowest;
+                const bool repeat = self && (self_seen || (int)e.key != self_key);
+                rep = __builtin_amdgcn_ballot_w64(repeat);
+                if (repeat) e.key = (uint32_t)self_key;
+                self_seen = self_seen || lowest < (1 << 30);
+            }
+        }
+        return rep;
+    };
+    repeats = mark_repeats(en, 0);
+
+    Step<VEC, MAX, ALIGNED> st[2];
+    st[0].template request_slots<0>(MS, en, lane_col, last_pair);
+    st[1].template request_slots<2>(MS, en, lane_col, last_pair);
+    st[0].template request_rows<0>(G, GX, en, lane_bytes);
+    for (int c0 = 0; c0 < longest; c0 += kRowLanes) {
+        const int slot_after = c0 + 2 * kRowLanes < mine ? list[c0 + 2 * kRowLanes] : 0;
+        const float w_next = c0 + kRowLanes < mine ? p.w[slot_next] : 0.f;
+        Entries next = entries_of(slot_next, 0.f, c0 + kRowLanes);
+        const uint64_t next_repeats = mark_repeats(next, c0 + kRowLanes);
+        float r[4] = {0.f, 0.f, 0.f, 0.f}, val[4];
+        // step I: rows of step I + 1 and slots of step I + 2 are requested, then step I is added up
+#define HGC_STEP(I)                                                                                                           \
+    {                                                                                                                         \
+        constexpr int kRows = (I) * 2 + 2, kSlots = (I) * 2 + 4;                                                              \
+        st[((I) + 1) & 1].template request_rows<(kRows & 15)>(G, GX, kRows < 16 ? en : next, lane_bytes);                     \
+        st[(I) & 1].template request_slots<(kSlots & 15)>(MS, kSlots < 16 ? en : next, lane_col, last_pair);                             \
+        __builtin_amdgcn_sched_barrier(0);                                                                                    \
+        constexpr int kA = entry_lane((I) * 2), kB = entry_lane((I) * 2 + 1);                                                 \
+        const float wa = group_bcast<kA>(en.w), wb = group_bcast<kB>(en.w);                                                   \
+        val[((I) & 1) * 2] = val[((I) & 1) * 2 + 1] = 0.f;                                                                    \
+        st[(I) & 1].template add<0, SCALE, WGRAD>(wa, SCALE == kPow2 ? group_bcast<kA>(en.w_mean) : wa,                       \
+                                                  group_lane_of(repeats, kA) ? 0.f : wa, xo, xk, p.divisor, acc, val[((I) & 1) * 2]);    \
+        st[(I) & 1].template add<1, SCALE, WGRAD>(wb, SCALE == kPow2 ? group_bcast<kB>(en.w_mean) : wb,                       \
+                                                  group_lane_of(repeats, kB) ? 0.f : wb, xo, xk, p.divisor, acc, val[((I) & 1) * 2 + 1]); \
+        if (WGRAD && ((I) & 1)) r[(I) >> 1] = group_sum_4(val, lane);                                                         \
+        __builtin_amdgcn_sched_barrier(0);                                                                                    \
+    }
+        HGC_STEP(0)
+        HGC_STEP(1)
+        HGC_STEP(2)
+        HGC_STEP(3)
+        if (c0 + 8 < longest) {
+            HGC_STEP(4)
+            HGC_STEP(5)
+            next.w = w_next;
+            next.w_mean = SCALE == kPow2 ? w_next * inv_divisor : w_next;
+            HGC_STEP(6)
+            HGC_STEP(7)
+        }
+#undef HGC_STEP
+        if (WGRAD) {
+            float sum = (l & 2) ? ((l & 1) ? r[3] : r[2]) : ((l & 1) ? r[1] : r[0]);
+            if (p.blocks == 2) sum = sum + __shfl_xor(sum, kRowLanes, kWave);  // the other half of the row
+            if (c0 < mine && task.block == 0) p.gw[slot] = p.negate ? -(sum * en.w) : sum;
+        }
+        slot = slot_next;
+        slot_next = slot_after;
+        en = next;
+        repeats = next_repeats;
+    }
+    if (live && fb < p.F) store_cols<VEC>(p.gfeat + (size_t)m * p.F + f, acc);
+}
+
+template <int VEC, bool MAX, Scale SCALE, bool WGRAD>
+void launch_packed(const GradRows &p, hipStream_t s) {
+    const dim3 grid(ceil_div((long long)p.n_vert * p.blocks, 256 / kRowLanes)), block(256);
+    if constexpr (MAX && VEC != 3) {
+        if (p.F % VEC == 0 && p.slot_shift == 0) {
+            accumulate_grad_rows_kernel<VEC, MAX, SCALE, true, WGRAD><<<grid, block, 0, s>>>(p);
+            return;
+        }
+    }
+    accumulate_grad_rows_kernel<VEC, MAX, SCALE, false, WGRAD><<<grid, block, 0, s>>>(p);
+}
+
+template <int VEC>
+int launch_rows(const GradRows &p, bool mean_and_max, bool want_w, Scale scale, hipStream_t s) {
+#define HGC_SCALES(MAX, WG)                                                        \
+    do {                                                                           \
+        if (scale == kPow2) launch_packed<VEC, MAX, kPow2, WG>(p, s);              \
+        else if (scale == kScaled) launch_packed<VEC, MAX, kScaled, WG>(p, s);     \
+        else launch_packed<VEC, MAX, kDivide, WG>(p, s);                           \
+    } while (0)
+    if (!want_w) HGC_SCALES(false, false);
+    else if (mean_and_max) HGC_SCALES(true, true);
+    else HGC_SCALES(false, true);
+#undef HGC_SCALES
+    return check_launch("accumulate_grad_rows_kernel");
+}
+
+// the mean half of the gradient divided by the divisor, rows of the gradient's own width
+__global__ __launch_bounds__(256) void divide_mean_half_kernel(const float *__restrict__ g, float *__restrict__ out,
+                                                               long long total, int F, int pitch, float divisor) {
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= total) return;
+    const long long v = t / F;
+    const size_t at = (size_t)v * pitch + (size_t)(t - v * F);
+    out[at] = g[at] / divisor;
+}
+
+}  // namespace
+
+size_t accumulate_grad_rows_scratch_bytes(int n_vert, int n_feat, int g_cols, float divisor) {
+    if (n_feat < kRowLanes || n_feat > 8 * kRowLanes) return 0;
+    if (divisor == (float)(int)divisor && is_pow2((int)divisor)) return 0;
+    return align_up((size_t)n_vert * g_cols * sizeof(float));
+}
+
+bool accumulate_grad_rows_covers(int n_feat, int n_neigh, bool mean_and_max, bool slots, unsigned long long g_bytes) {
+    return n_feat >= kRowLanes && n_feat <= 8 * kRowLanes && (!mean_and_max || (slots && n_neigh <= 254)) &&
+           g_bytes <= kMaxRowBytes;
+}
+
+// Returns 1 where the shape is not covered. gw == nullptr: feature gradient only (mean only). scratch
+// (accumulate_grad_rows_scratch_bytes, may be null) holds the quotients g / divisor where the divisor is
+// no power of two: N F divides in a pass of their own instead of N K F inside the gather
+// (150,000 vertices, K = 40, F = 64: 287 -> 262 us).
+int launch_accumulate_grad_rows(const float *g, const float *w, const float *feat, const unsigned char *maxslot,
+                                const int *inv_off, const int *inv_slots, float *gw, float *gfeat, int n_vert, int K, int F,
+                                int g_cols, bool mean_and_max, const int *order, float divisor, bool negate, void *scratch,
+                                size_t scratch_bytes, hipStream_t s) {
+    const bool want_w = gw != nullptr;
+    const unsigned long long g_bytes = (unsigned long long)n_vert * g_cols * 4ull;
+    if (!accumulate_grad_rows_covers(F, K, mean_and_max, maxslot != nullptr, g_bytes) || (mean_and_max && !want_w)) return 1;
+    GradRows p;
+    Scale scale = kDivide;
+    p.g = g;
+    if (divisor == (float)(int)divisor && is_pow2((int)divisor)) {
+        scale = kPow2;
+    } else if (scratch && scratch_bytes >= accumulate_grad_rows_scratch_bytes(n_vert, F, g_cols, divisor)) {
+        scale = kScaled;
+        const long long total = (long long)n_vert * F;
+        divide_mean_half_kernel<<<ceil_div(total, 256), 256, 0, s>>>(g, static_cast<float *>(scratch), total, F, g_cols, divisor);
+        const int rc = check_launch("divide_mean_half_kernel");
+        if (rc) return rc;
+        p.g = static_cast<const float *>(scratch);
+    }
+    p.g_max = mean_and_max ? g + F : nullptr;
+    p.w = w;
+    p.feat = feat;
+    p.inv_off = inv_off;
+    p.inv_slots = inv_slots;
+    p.order = order;
+    p.gw = gw;
+    p.gfeat = gfeat;
+    p.g_bytes = g_bytes;
+    p.g_max_bytes = g_bytes - (unsigned long long)F * 4ull;
+    p.slot_shift = (uint32_t)(reinterpret_cast<uintptr_t>(maxslot) & 3u);
+    p.maxslot = maxslot - p.slot_shift;
+    p.slot_bytes = ((unsigned long long)n_vert * F + p.slot_shift + 3ull) / 4 * 4;  // whole words
+    p.n_vert = n_vert;
+    p.K = K;
+    p.F = F;
+    p.pitch = g_cols;
+    p.div_k = make_fast_div(K);
+    p.divisor = divisor;
+    p.negate = negate;
+    int vec;
+    row_shape(F, vec, p.blocks);
+    switch (vec) {
+        case 1: return launch_rows<1>(p, mean_and_max, want_w, scale, s);
+        case 2: return launch_rows<2>(p, mean_and_max, want_w, scale, s);
+        case 3: return launch_rows<3>(p, mean_and_max, want_w, scale, s);
+        default: return launch_rows<4>(p, mean_and_max, want_w, scale, s);
+    }
+}
+
+}  // namespace hgc

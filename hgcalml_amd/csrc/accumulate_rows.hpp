@@ -192,34 +192,22 @@ __device__ __forceinline__ void load_cols(__amdgpu_buffer_rsrc_t rsrc, uint32_t 
     }
 }
 
-// the first min(VEC, left) of VEC consecutive elements; rows start on 4-byte boundaries only.
-// Result rows are touched once: non-temporal.
+// VEC consecutive elements of a result row (touched once: non-temporal); rows start on 4-byte boundaries only
 template <int VEC, typename T>
-__device__ __forceinline__ void store_cols(T *p, const T (&x)[VEC], int left) {
-    typedef T vec_t __attribute__((ext_vector_type(VEC == 3 ? 4 : VEC), aligned(4)));
-    if constexpr (VEC == 3) {
-        if (left >= 3) {
-            typedef T pair_t __attribute__((ext_vector_type(2), aligned(4)));
-            pair_t v;
-            v[0] = x[0]; v[1] = x[1];
-            __builtin_nontemporal_store(v, reinterpret_cast<pair_t *>(p));
-            __builtin_nontemporal_store(x[2], p + 2);
-            return;
-        }
-    } else if (left >= VEC) {
-        if constexpr (VEC == 1) {
-            __builtin_nontemporal_store(x[0], p);
-        } else {
-            vec_t v;
+__device__ __forceinline__ void store_cols(T *p, const T (&x)[VEC]) {
+    if constexpr (VEC == 1) {
+        __builtin_nontemporal_store(x[0], p);
+    } else if constexpr (VEC == 3) {
+        const T pair[2] = {x[0], x[1]};
+        store_cols<2>(p, pair);
+        __builtin_nontemporal_store(x[2], p + 2);
+    } else {
+        typedef T vec_t __attribute__((ext_vector_type(VEC), aligned(4)));
+        vec_t v;
 #pragma unroll
-            for (int e = 0; e < VEC; ++e) v[e] = x[e];
-            __builtin_nontemporal_store(v, reinterpret_cast<vec_t *>(p));
-        }
-        return;
+        for (int e = 0; e < VEC; ++e) v[e] = x[e];
+        __builtin_nontemporal_store(v, reinterpret_cast<vec_t *>(p));
     }
-#pragma unroll
-    for (int e = 0; e < VEC; ++e)
-        if (e < left) __builtin_nontemporal_store(x[e], p + e);
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rows(const void *base, unsigned long long bytes) {

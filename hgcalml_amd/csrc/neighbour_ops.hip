@@ -27,7 +27,7 @@ int accumulate_gradient(const float *d_grad_from_out_features, const float *d_di
                         const int *d_inv_offsets, const int *d_inv_slots, float *d_out_grad_distances,
                         float *d_out_grad_features, int n_vert, int n_neigh, int n_feat, int n_grad_from_out_feat,
                         int mean_and_max, float divisor, const int *d_order, void *records, size_t records_bytes,
-                        hgc_stream_t stream);
+                        bool negate, void *scratch, size_t scratch_bytes, hgc_stream_t stream);
 
 namespace {
 
@@ -246,8 +246,9 @@ __global__ __launch_bounds__(256) void exp_neg_kernel(const float *__restrict__ 
     }
 }
 
-__global__ __launch_bounds__(256) void exp_neg_grad_kernel(const float *__restrict__ gw, const float *__restrict__ w,
-                                                           float *__restrict__ gd, long long n) {
+// (gd may be gw)
+__global__ __launch_bounds__(256) void exp_neg_grad_kernel(const float *gw, const float *__restrict__ w, float *gd,
+                                                           long long n) {
     const long long i = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (i + 4 <= n) {
         const float4 a = *reinterpret_cast<const float4 *>(gw + i), b = *reinterpret_cast<const float4 *>(w + i);
@@ -445,7 +446,7 @@ int hgc_push_knn_ordered(const float *d_weights, const float *d_feat, const int 
     // feature gradient of the accumulation with `feat` as upstream gradient, not divided by K
     return accumulate_gradient(d_feat, d_weights, nullptr, nullptr, nullptr, nullptr, d_inv_offsets, d_inv_slots,
                                nullptr, d_out_feat, n_vert, n_neigh, n_feat, n_feat, 0, 1.f, d_vertex_order, nullptr, 0,
-                               stream);
+                               false, nullptr, 0, stream);
 }
 
 int hgc_push_knn(const float *d_weights, const float *d_feat, const int *d_idxs, const int *d_inv_offsets,
@@ -474,7 +475,7 @@ int hgc_push_knn_grad(const float *d_grad, const float *d_weights, const float *
     // w_grad[v, n] = sum_f grad[idx[v,n], f] * feat[v, f]: the weight gradient with the roles of the
     // vertex's own row (feat) and the gathered rows (grad) as in the accumulation's
     return accumulate_gradient(d_feat, nullptr, d_grad, nullptr, nullptr, d_idxs, nullptr, nullptr, d_w_grad, nullptr,
-                               n_vert, n_neigh, n_feat, n_feat, 0, 1.f, nullptr, nullptr, 0, stream);
+                               n_vert, n_neigh, n_feat, n_feat, 0, 1.f, nullptr, nullptr, 0, false, nullptr, 0, stream);
 }
 
 int hgc_exp_neg(const float *d_distances, float *d_weights, long long n_values, hgc_stream_t stream) {

@@ -421,7 +421,8 @@ def invalidate_neighbour_table(indices):
 
 
 def _accumulate_backward(grad_from_out_features, distances, features, neigh_indices, max_feat_indices, max_slots,
-                         inv_offsets, inv_slots):
+                         inv_offsets, inv_slots, exp_weights=False):
+    """exp_weights: the weights are exp(-d), the first result is the gradient w.r.t. d"""
     dev = require_device(grad_from_out_features, distances, features, neigh_indices, max_feat_indices)
     g, w, x = f32(grad_from_out_features), f32(distances), f32(features)
     idx, mi = i32(neigh_indices), i32(max_feat_indices)
@@ -432,20 +433,24 @@ def _accumulate_backward(grad_from_out_features, distances, features, neigh_indi
         max_slots = None
     gw = torch.empty((n, k), dtype=torch.float32, device=dev)
     gx = torch.empty((n, f), dtype=torch.float32, device=dev)
-    # with the slot table: one record per (vertex, slot) in scratch memory carries the max part to the gather
+    # on request, with the slot table: one record per (vertex, slot) in scratch memory carries the max part to the gather
     need = 0
-    if max_slots is not None and gl.acc_grad_hit_records is not False:
-        if gl.acc_grad_hit_records or lib.hgc_accumulate_knn_grad_records_pays(n, k, f, int(mean_and_max)):
-            need = lib.hgc_accumulate_knn_grad_records_workspace_bytes(n, k, f, int(mean_and_max))
+    if max_slots is not None and gl.acc_grad_hit_records:
+        need = lib.hgc_accumulate_knn_grad_records_workspace_bytes(n, k, f, int(mean_and_max))
     if need:
         ws = workspace(need, dev)
         check(lib.hgc_accumulate_knn_grad_records(p(g), p(w), p(x), p(mi), p(max_slots), p(idx), p(inv_offsets),
                                                   p(inv_slots), p(vertex_order_of(neigh_indices)), p(gw), p(gx), n, k,
                                                   f, g.shape[1], 0, int(mean_and_max), p(ws), ws.numel(), stream()))
-        return gw, gx
-    check(lib.hgc_accumulate_knn_grad_slots(p(g), p(w), p(x), p(mi), p(max_slots), p(idx), p(inv_offsets),
-                                            p(inv_slots), p(vertex_order_of(neigh_indices)), p(gw), p(gx), n, k, f,
-                                            g.shape[1], 0, int(mean_and_max), stream()))
+        return (exp_neg_grad(gw, w) if exp_weights else gw), gx
+    if exp_weights and w.data_ptr() % 16:
+        w = w.clone()
+    need = lib.hgc_accumulate_knn_grad_scratch_bytes(n, k, f, int(mean_and_max))
+    ws = workspace(need, dev) if need else None
+    check(lib.hgc_accumulate_knn_grad_scratch(p(g), p(w), p(x), p(mi), p(max_slots), p(idx), p(inv_offsets),
+                                              p(inv_slots), p(vertex_order_of(neigh_indices)), p(gw), p(gx), n, k, f,
+                                              g.shape[1], int(mean_and_max), int(exp_weights), p(ws),
+                                              ws.numel() if need else 0, stream()))
     return gw, gx
 
 
@@ -466,6 +471,17 @@ def accumulate_knn_grad_slots(grad_from_out_features: torch.Tensor, distances: t
     """accumulate_knn_grad fed with the slot table of accumulate_knn_slots"""
     return _accumulate_backward(grad_from_out_features, distances, features, neigh_indices, max_feat_indices,
                                 max_slots, inv_offsets, inv_slots)
+
+
+@torch.library.custom_op("hgcalml::accumulate_knn_grad_exp_slots", mutates_args=())
+def accumulate_knn_grad_exp_slots(grad_from_out_features: torch.Tensor, weights: torch.Tensor, features: torch.Tensor,
+                                  neigh_indices: torch.Tensor, max_feat_indices: torch.Tensor, max_slots: torch.Tensor,
+                                  inv_offsets: torch.Tensor, inv_slots: torch.Tensor
+                                  ) -> tuple[torch.Tensor, torch.Tensor]:
+    """gradients of accumulate_knn_exp_slots w.r.t. the distances and the features
+    (modules/accknn_op.py:52,71-89)"""
+    return _accumulate_backward(grad_from_out_features, weights, features, neigh_indices, max_feat_indices, max_slots,
+                                inv_offsets, inv_slots, exp_weights=True)
 
 
 # --------------------------------------------------------------------------- ops next to the accumulation
@@ -706,6 +722,11 @@ def _(grad_from_out_features, distances, features, neigh_indices, max_feat_indic
 @accumulate_knn_grad_slots.register_fake
 def _(grad_from_out_features, distances, features, neigh_indices, max_feat_indices, max_slots, inv_offsets,
       inv_slots):
+    return _accumulate_grad_shapes(features, neigh_indices)
+
+
+@accumulate_knn_grad_exp_slots.register_fake
+def _(grad_from_out_features, weights, features, neigh_indices, max_feat_indices, max_slots, inv_offsets, inv_slots):
     return _accumulate_grad_shapes(features, neigh_indices)
 
 

@@ -385,10 +385,11 @@ int hgc_accumulate_knn_grad_slots(const float *d_grad_from_out_features, const f
  * record pass does not cover (n_feat outside 16..128, n_neigh > 254, gradient
  * matrix of 4 GiB or more, !mean_and_max); the call then behaves exactly like
  * hgc_accumulate_knn_grad_slots and accepts a NULL workspace, as it does when
- * d_max_slots is NULL. hgc_accumulate_knn_grad_records_pays says where the
- * record pass has measured faster (n_neigh >= 48, n_neigh < n_feat <= 2 n_neigh
- * and n_vert * n_feat of 12 Mi elements or more: cfg4 5.8 -> 4.7 ms); elsewhere
- * hgc_accumulate_knn_grad_slots is the better call. */
+ * d_max_slots is NULL. hgc_accumulate_knn_grad_records_pays says for which
+ * shapes the record pass comes near hgc_accumulate_knn_grad_slots (n_neigh >= 48,
+ * n_neigh < n_feat <= 2 n_neigh and n_vert * n_feat of 12 Mi elements or more: a
+ * million rows, 64 neighbours, 128 features, banded table 4.70 ms against 4.62 ms,
+ * kNN table 5.9 against 4.45); elsewhere it costs half as much again or more. */
 size_t hgc_accumulate_knn_grad_records_workspace_bytes(int n_vert, int n_neigh, int n_feat,
                                                        int mean_and_max);
 int hgc_accumulate_knn_grad_records_pays(int n_vert, int n_neigh, int n_feat, int mean_and_max);
@@ -401,6 +402,26 @@ int hgc_accumulate_knn_grad_records(const float *d_grad_from_out_features, const
                                     int n_vert, int n_neigh, int n_feat, int n_grad_from_out_feat,
                                     int n_moments, int mean_and_max,
                                     void *workspace, size_t workspace_bytes, hgc_stream_t stream);
+
+/* hgc_accumulate_knn_grad_slots with scratch memory (may be NULL) for the
+ * quotients g / n_neigh where n_neigh is no power of two and n_feat is 16..128
+ * (the query returns 0 elsewhere): one pass of n_vert * n_feat divides instead
+ * of one divide per gathered element. Same bits either way. With
+ * weights_are_exp the weights are exp(-d) and d_out_grad_distances receives the
+ * gradient w.r.t. d, -(gradient w.r.t. the weight * weight), the bits of
+ * hgc_exp_neg_grad behind this call (outputs and d_distances then on 16-byte
+ * boundaries). No single counterpart in the reference
+ * (modules/accknn_op.py:52,71-89). */
+size_t hgc_accumulate_knn_grad_scratch_bytes(int n_vert, int n_neigh, int n_feat, int mean_and_max);
+int hgc_accumulate_knn_grad_scratch(const float *d_grad_from_out_features, const float *d_distances,
+                                    const float *d_feat, const int *d_max_feat_indices,
+                                    const unsigned char *d_max_slots, const int *d_neigh_indices,
+                                    const int *d_inv_offsets, const int *d_inv_slots,
+                                    const int *d_vertex_order,
+                                    float *d_out_grad_distances, float *d_out_grad_features,
+                                    int n_vert, int n_neigh, int n_feat, int n_grad_from_out_feat,
+                                    int mean_and_max, int weights_are_exp,
+                                    void *scratch, size_t scratch_bytes, hgc_stream_t stream);
 
 /* ------------------------------------------------------------------ */
 /* Ops over the same neighbour table, either side of the accumulation  */

@@ -65,3 +65,42 @@ def test_forward_at_the_ends_of_tiles(oracle, n, K, F):
                 sl = slots.cpu().numpy().astype(int)
                 named = np.where(sl < K, np.take_along_axis(idx, np.minimum(sl, K - 1), 1), 0)
                 assert (named == rarg).all()
+
+
+@pytest.mark.parametrize("n,K,F", SHAPES)
+def test_gradient_at_the_ends_of_tiles(oracle, n, K, F):
+    """both gradients with and without the quotients' scratch memory, w.r.t. weights and (weights_are_exp) distances;
+    lists of very different length in one workgroup"""
+    from hgcalml_amd import ops
+    from hgcalml_amd._lib import check, lib, p, stream
+    rng = np.random.default_rng(n + 200 * K + 20000 * F)
+    idx = table(rng, n, K)
+    hub = rng.integers(0, min(n, 5), n)  # many rows name the same few vertices
+    for v in range(0, n, 3):
+        if K > 1 and hub[v] not in idx[v]:
+            idx[v, K - 1] = hub[v]
+    x = rng.standard_normal((n, F)).astype(np.float32)
+    w = rng.random((n, K), dtype=np.float32)
+    ti, tw, tx = t(idx), t(w), t(x)
+    inv = ops.inverse_neighbour_index(ti)
+    for mm in (True, False):
+        g = rng.standard_normal((n, 2 * F if mm else F)).astype(np.float32)
+        _, rarg = oracle.AccumulateLinKnn(w, x, idx, mm)
+        rgw, rgx = oracle.accumulate_knn_grad_kernel(g, w, x, idx, rarg)
+        _, arg, slots = torch.ops.hgcalml.accumulate_knn_slots(tw, tx, ti, 0, mm)
+        need = lib.hgc_accumulate_knn_grad_scratch_bytes(n, K, F, int(mm))
+        # 1e-5 of the sum of the absolute terms of a dot product of F (2 F) float32 products
+        absx = np.abs(x[np.maximum(idx, 0)])
+        tol = 1e-5 * (absx * (np.abs(g[:, :F]) / K + (np.abs(g[:, F:]) if mm else 0))[:, None, :]).sum(-1) + 1e-30
+        order = t(rng.permutation(n).astype(np.int32))
+        for with_scratch, exp in ((False, False), (True, False), (True, True)):
+            gw, gx = torch.empty_like(tw), torch.empty_like(tx)
+            scratch = torch.empty(max(need, 256), dtype=torch.uint8, device=DEV) if with_scratch else None
+            check(lib.hgc_accumulate_knn_grad_scratch(p(t(g)), p(tw), p(tx), p(arg), p(slots) if slots.numel() else None, p(ti),
+                                                      p(inv[0]), p(inv[1]), p(order) if exp else None, p(gw), p(gx), n, K, F,
+                                                      g.shape[1], int(mm), int(exp), p(scratch),
+                                                      scratch.numel() if with_scratch else 0, stream()))
+            assert (bits(gx.cpu().numpy()) == bits(rgx)).all()
+            got, want = gw.cpu().numpy(), -(rgw * w) if exp else rgw
+            assert (np.abs(got - want) <= tol).all()
+            assert (got[idx < 0] == 0).all()
