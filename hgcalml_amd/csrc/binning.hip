@@ -752,7 +752,7 @@ int hgc_sort_by_bin(const int *d_flat_bin, int n_vert, int n_total_bins, int *d_
         return fail(HGC_ERR_WORKSPACE, "sort_by_bin workspace missing, misaligned or too small");
     // a stable counting sort by bin yields the order and the boundary table at once
     if (stable_key_sort_supported(n_vert, n_total_bins, hits_per_bin(n_vert, n_total_bins)))
-        return stable_key_sort(d_flat_bin, nullptr, n_vert, n_total_bins, hits_per_bin(n_vert, n_total_bins),
+        return stable_key_sort(d_flat_bin, n_vert, n_total_bins, hits_per_bin(n_vert, n_total_bins),
                                d_bin_boundaries, d_sorting, workspace, workspace_bytes, s);
     Carver carve(workspace);
     int *iota = carve.take<int>(n_vert);

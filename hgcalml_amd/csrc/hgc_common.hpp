@@ -113,15 +113,14 @@ int shift_and_bin(const float *d_coords, const uint32_t *d_min_bits, const uint3
                   int n_total_bins, float *d_shifted, float *d_bin_width, int *d_n_bins, int *d_assigned_bin,
                   int *d_flat_bin, hipStream_t s);
 
-// Stable sort of `total` items by integer key (split_sort.hip). Item i has the key
-// d_keys[d_values ? d_values[i] : i] and the value d_values ? d_values[i] : i; keys outside
-// [0, n_keys) count as n_keys and sort last. d_order [total] receives the values in key order,
+// Stable sort of `total` items by integer key (split_sort.hip). Item i has the key d_keys[i];
+// keys outside [0, n_keys) count as n_keys and sort last. d_order [total] receives the item numbers in key order,
 // d_offsets (may be null) [n_keys + 1] the first position of every key. `per_key_hint`: items
 // expected per key (sizes the tiles). Not every shape is supported (key ranges of 2^22 and more).
 bool stable_key_sort_supported(long long total, int n_keys, int per_key_hint);
 size_t stable_key_sort_workspace_bytes(long long total, int n_keys, int per_key_hint);
-int stable_key_sort(const int *d_keys, const int *d_values, long long total, int n_keys, int per_key_hint,
-                    int *d_offsets, int *d_order, void *workspace, size_t workspace_bytes, hipStream_t s);
+int stable_key_sort(const int *d_keys, long long total, int n_keys, int per_key_hint, int *d_offsets, int *d_order,
+                    void *workspace, size_t workspace_bytes, hipStream_t s);
 
 // hgc_binned_select_knn_fused over a boundary table with stride 2^boundary_shift.
 // fine_bits > 0 (= n_bin_dim): d_bin_idx holds the half-bin cells of bin_grouping's spatial mode

@@ -81,7 +81,7 @@ int hgc_inverse_neighbour_index(const int *d_idxs, int n_vert, int n_neigh, int 
         return fail(HGC_ERR_WORKSPACE, "inverse_neighbour_index workspace missing, misaligned or too small");
     const long long total = (long long)n_vert * n_neigh;
     if (stable_key_sort_supported(total, n_vert, n_neigh))
-        return stable_key_sort(d_idxs, nullptr, total, n_vert, n_neigh, d_inv_offsets, d_inv_slots, workspace,
+        return stable_key_sort(d_idxs, total, n_vert, n_neigh, d_inv_offsets, d_inv_slots, workspace,
                                workspace_bytes, s);
 
     // Keys and values are generated on the fly: key = the slot's target (invalid

@@ -1,0 +1,31 @@
+"""The two-level key sort behind the inverse neighbour index where its variants and batches end: numbers of tiles around
+1536 and 4096 (one counter per wave and tile, two passes of 6 and of 7 bits), stretches of a few items, of exactly one
+batch of 12,288 and of one more, tiles beyond the 20,480 items that are held in registers."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("n,k,kind", [(1, 5, "random"), (63, 65, "random"), (64, 64, "random"), (4096, 1, "random"), (4097, 1, "random"),
+                                      (12288, 1, "random"), (49152, 64, "random"), (49153, 64, "random"), (1572863, 1, "random"),
+                                      (1572864, 2, "random"), (4194303, 1, "random"), (4194304, 1, "random"), (60000, 40, "few"),
+                                      (2000000, 3, "sorted")])
+def test_inverse_index_at_the_ends_of_batches_and_tiles(n, k, kind):
+    from hgcalml_amd import ops
+    rng = np.random.default_rng(n + 7 * k)
+    idx = rng.integers(0, n, (n, k)).astype(np.int32)
+    if kind == "few":       # tiles of a hundred thousand items next to empty ones
+        idx = (idx % 900).astype(np.int32)
+    if kind == "sorted":
+        idx = np.repeat(np.arange(n, dtype=np.int32)[:, None], k, 1)
+    idx[rng.random((n, k)) < 0.03] = -1
+    off, slots = ops.inverse_neighbour_index(torch.from_numpy(idx).to(DEV))
+    flat = torch.from_numpy(idx.reshape(-1)).to(DEV).to(torch.int64)
+    key = torch.where(flat < 0, torch.full_like(flat, n), flat)
+    order = torch.sort(key, stable=True).indices
+    assert torch.equal(slots[:n * k].to(torch.int64), order)
+    assert torch.equal(off.to(torch.int64), torch.searchsorted(key[order], torch.arange(n + 1, device=DEV)))
