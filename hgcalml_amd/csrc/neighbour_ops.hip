@@ -1,9 +1,8 @@
 // Ops next to the accumulate path that run over the same neighbour table:
-//   * coordinate gradient of the kNN distances (SelectKnnGrad),
+//   * squared distances to listed neighbours (LocalDistance),
 //   * push_knn forward and gradient.
 //
 // Reference behaviour restated here:
-//   modules/compiled/select_knn_grad_kernel.cu.cc:81-164
 //   modules/compiled/push_knn_kernel.cc:40-62
 //   modules/compiled/push_knn_grad_kernel.cc:23-71
 //   modules/compiled/local_distance_kernel.cc:18-70
@@ -31,78 +30,8 @@ int accumulate_gradient(const float *d_grad_from_out_features, const float *d_di
 
 namespace {
 
-// One thread per (vertex i, coordinate c). d(dist_ik)/d(x_i) summed over the
-// vertex's own neighbours first, in slot order, then the terms of every (v, n)
-// that names i, in ascending (v, n) order. Each term is formed in double and
-// rounded once, as the reference's `2. * g * (x_k - x_i)` is. With a processing
-// order (a permutation of the vertices, e.g. the kNN's bin order) neighbouring
-// threads work on vertices that share neighbours, whose coordinates then come
-// from the first-level cache; the results do not depend on it.
-__global__ __launch_bounds__(256) void select_knn_grad_kernel(const float *__restrict__ grad_dist,
-                                                              const int *__restrict__ idx,
-                                                              const float *__restrict__ coord,
-                                                              const int *__restrict__ inv_off,
-                                                              const int *__restrict__ inv_slots,
-                                                              float *__restrict__ grad_coord, int n_vert, int K, int C,
-                                                              const acc::FastDiv div_k,
-                                                              const int *__restrict__ order) {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int r = (int)(t / C);
-    if (r >= n_vert) return;
-    const int c = (int)(t - (long long)r * C);
-    const int i = order ? order[r] : r;
-    if ((uint32_t)i >= (uint32_t)n_vert) return;  // not a permutation: that vertex is left out
-    const float xi = coord[(size_t)i * C + c];
-
-    // loads of U slots are issued together; the additions stay in slot / list order
-    constexpr int U = 8;
-    float sum = 0.f;
-    for (int n0 = 0; n0 < K; n0 += U) {
-        int k[U];
-        float g[U], xk[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int n = min(n0 + u, K - 1);
-            k[u] = idx[(size_t)i * K + n];
-            g[u] = grad_dist[(size_t)i * K + n];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const bool ok = n0 + u < K && k[u] >= 0 && k[u] < n_vert;
-            k[u] = ok ? k[u] : -1;
-            xk[u] = coord[(size_t)(ok ? k[u] : i) * C + c];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (k[u] < 0) continue;
-            const float diff = xk[u] - xi;
-            sum = (float)((double)sum - 2. * (double)g[u] * (double)diff);
-        }
-    }
-    const int begin = inv_off[i], end = inv_off[i + 1];
-    for (int e0 = begin; e0 < end; e0 += U) {
-        int slot[U];
-        float g[U], xv[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) slot[u] = inv_slots[min(e0 + u, end - 1)];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            g[u] = grad_dist[slot[u]];
-            xv[u] = coord[(size_t)acc::fast_div(slot[u], div_k) * C + c];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (e0 + u >= end) break;
-            const float diff = xi - xv[u];
-            const float add = (float)(2. * (double)g[u] * (double)diff);
-            sum = sum + add;
-        }
-    }
-    grad_coord[(size_t)i * C + c] = sum;
-}
-
 // one thread per (vertex, slot): serial fp32 sum over the coordinates, 0 for a
-// missing neighbour and for the vertex itself (order: see select_knn_grad_kernel)
+// missing neighbour and for the vertex itself (order: the vertices are worked on in it)
 __global__ __launch_bounds__(256) void local_distance_kernel(const int *__restrict__ idx,
                                                              const float *__restrict__ coord,
                                                              float *__restrict__ dist, int C, int n_in_vert,
@@ -392,29 +321,6 @@ int hgc_neighbour_covariance(const float *d_coords, const float *d_weights, cons
     }
 #undef HGC_COV
     return HGC_ERR_UNSUPPORTED;
-}
-
-int hgc_select_knn_grad_ordered(const float *d_grad_dist, const int *d_indices, const float *d_dist,
-                                const float *d_coord, const int *d_inv_offsets, const int *d_inv_slots,
-                                const int *d_vertex_order, float *d_grad_coord, int n_vert, int n_neigh, int n_coords,
-                                hgc_stream_t stream) {
-    (void)d_dist;  // carried by the reference op, not used by its kernels
-    HGC_REQUIRE(n_vert >= 0 && n_neigh >= 1 && n_coords >= 1, "bad sizes");
-    HGC_REQUIRE((long long)n_vert * std::max(n_neigh, n_coords) < (1ll << 31), "tensor too large for int32 indexing");
-    if (n_vert == 0) return HGC_OK;
-    HGC_REQUIRE(d_grad_dist && d_indices && d_coord && d_inv_offsets && d_inv_slots && d_grad_coord, "null pointer");
-    const long long threads = (long long)n_vert * n_coords;
-    select_knn_grad_kernel<<<ceil_div(threads, 256), 256, 0, as_stream(stream)>>>(
-        d_grad_dist, d_indices, d_coord, d_inv_offsets, d_inv_slots, d_grad_coord, n_vert, n_neigh, n_coords,
-        acc::make_fast_div(n_neigh), d_vertex_order);
-    return check_launch("select_knn_grad_kernel");
-}
-
-int hgc_select_knn_grad(const float *d_grad_dist, const int *d_indices, const float *d_dist, const float *d_coord,
-                        const int *d_inv_offsets, const int *d_inv_slots, float *d_grad_coord, int n_vert, int n_neigh,
-                        int n_coords, hgc_stream_t stream) {
-    return hgc_select_knn_grad_ordered(d_grad_dist, d_indices, d_dist, d_coord, d_inv_offsets, d_inv_slots, nullptr,
-                                       d_grad_coord, n_vert, n_neigh, n_coords, stream);
 }
 
 int hgc_local_distance_ordered(const int *d_neigh_idxs, const float *d_coords, const int *d_vertex_order,
