@@ -27,7 +27,8 @@ def check_condensate_counts(assignment, n_condensates, row_splits):
 
 def merge_noise_as_indiv_cp(assignment, asso_idx, alpha_idx, is_cond, n_condensates, row_splits):
     """Every noise hit becomes a condensation point of its own, numbered before
-    the real ones inside each event (modules/assign_condensate_op.py:16-44)."""
+    the real ones inside each event (modules/assign_condensate_op.py:16-44).
+    For outputs that are already there, on any device; the wrapper below has it done by the library."""
     dev = assignment.device
     n = assignment.shape[0]
     rs = row_splits.to(device=dev, dtype=torch.int64)
@@ -85,10 +86,8 @@ def BuildAndAssignCondensatesBinned(ccoords, betas, dist, row_splits, beta_thres
     n_bins_sc = max(4, min(int(math.ceil(math.pow(n / 5, 1 / 3))), 25))
     assignment, asso, alpha_idx, is_cond, n_condensates = ops.build_and_assign_condensates(
         ccoords, betas, dist, no_condensation_mask, row_splits, beta_threshold, distance_threshold,
-        assign_by_max_beta, nbin_dims, n_bins_sc)
+        assign_by_max_beta, nbin_dims, n_bins_sc, bool(keep_noise))
     out = (assignment[:, None], asso, alpha_idx, is_cond[:, None], n_condensates)
-    if keep_noise:
-        out = merge_noise_as_indiv_cp(*out, row_splits)
     if gl.debug_checks:
         check_condensate_counts(out[0], out[4], row_splits)
     return out

@@ -601,8 +601,8 @@ def binned_assign_to_condensates(ccoords: torch.Tensor, dist: torch.Tensor, beta
 
 
 def build_and_assign_condensates(ccoords, betas, dist, mask, row_splits, beta_threshold, distance_threshold,
-                                 assign_by_max_beta, nbin_dims, n_bins_scalar):
-    """modules/assign_condensate_op.py:210-373 (without keep_noise) as one call into the library;
+                                 assign_by_max_beta, nbin_dims, n_bins_scalar, keep_noise=False):
+    """modules/assign_condensate_op.py:210-373 as one call into the library (two with keep_noise);
     returns (assignment [n], association [n], alpha_idx [n_condensates], is_cond [n] bool,
     n_condensates [events + 1]). One host synchronisation, for the length of alpha_idx."""
     dev = require_device(ccoords, betas, dist)
@@ -624,8 +624,16 @@ def build_and_assign_condensates(ccoords, betas, dist, mask, row_splits, beta_th
                                                    int(assign_by_max_beta), nbin_dims, n_bins_scalar, p(assignment),
                                                    p(asso), p(alpha), p(is_cond), p(ncond), p(ws), ws.numel(),
                                                    stream()))
-    total = int(ncond[-1]) if n > 0 else 0
-    return assignment, asso, alpha[:total], is_cond, ncond
+    if keep_noise and n > 0:
+        real, alpha = alpha, torch.empty((2 * n,), dtype=torch.int32, device=dev)
+        real_ncond, ncond = ncond, torch.empty_like(ncond)
+        total = torch.empty((1,), dtype=torch.int32, device=dev)
+        ws = workspace(lib.hgc_keep_noise_condensates_workspace_bytes(n, num_rows), dev)
+        check(lib.hgc_keep_noise_condensates(p(row_splits), n, num_rows, p(real), p(real_ncond), p(assignment), p(asso),
+                                             p(is_cond), p(alpha), p(ncond), p(total), p(ws), ws.numel(), stream()))
+    else:
+        total = ncond[-1]
+    return assignment, asso, alpha[:int(total) if n > 0 else 0], is_cond, ncond
 
 
 def exp_neg(distances):

@@ -606,6 +606,20 @@ int hgc_build_and_assign_condensates(const float *d_ccoords, const float *d_beta
                                      int *d_alpha_idx, unsigned char *d_is_cond, int *d_n_condensates,
                                      void *workspace, size_t workspace_bytes, hgc_stream_t stream);
 
+/* keep_noise of that wrapper (merge_noise_as_indiv_cp, modules/assign_condensate_op.py:16-44)
+ * on the outputs of hgc_build_and_assign_condensates: every hit without an
+ * assignment becomes a condensation point of its own, numbered before the real
+ * ones of its event. d_assignment, d_association and d_is_cond are updated in
+ * place; d_out_n_condensates [num_rows + 1] and the list of condensation points
+ * d_out_alpha_idx (room for 2 * n_vert entries, noise hits first in every
+ * event) are written, and its length to *d_out_n_alpha. No host
+ * synchronisation. */
+size_t hgc_keep_noise_condensates_workspace_bytes(int n_vert, int num_rows);
+int hgc_keep_noise_condensates(const int *d_row_splits, int n_vert, int num_rows, const int *d_alpha_idx,
+                               const int *d_n_condensates, int *d_assignment, int *d_association,
+                               unsigned char *d_is_cond, int *d_out_alpha_idx, int *d_out_n_condensates,
+                               int *d_out_n_alpha, void *workspace, size_t workspace_bytes, hgc_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
