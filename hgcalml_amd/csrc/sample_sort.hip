@@ -20,7 +20,9 @@
 // between lanes (ds_bpermute) and, for the few steps across waves, through LDS.
 // Buckets hold ~2000 keys; with eight or more sampled keys per bucket one four
 // times that size is out of reach for keys in any order that was not built
-// against the sampling positions. A bucket beyond 8192 keys is still sorted: runs
+// against the sampling positions.
+// Up to 16384 keys one launch does it: every key's place is the number of smaller
+// keys, counted (rank_kernel). A bucket beyond 8192 keys is still sorted: runs
 // of that size, then pairwise merges through global memory by the same workgroup
 // (slow, never seen on real inputs, exercised by the tests through a smaller run
 // size).
@@ -38,6 +40,9 @@ constexpr int kBucketStage = 8192;   // keys of a bucket that are sorted in LDS 
 constexpr int kMaxBuckets = 512;     // at least eight sampled keys per bucket
 constexpr int kMoveBlock = 256;      // threads of the counting and moving kernels
 constexpr int kMoveItems = 8;        // keys per thread there
+// Ranking grows with n^2, the sample sort little below 10^5 keys (a call, ranking against sample sort: 700 keys 7.0
+// against 7.5 us, 5000 12 against 44, 8192 16 against 46, 16384 28 against 59).
+constexpr int kRankLimit = 16384;
 constexpr uint64_t kPadKey = ~0ull;  // sorts behind every real key
 
 __device__ __forceinline__ uint64_t key_from_lane(uint64_t v, int src_lane) {
@@ -313,6 +318,44 @@ __global__ __launch_bounds__(kSortBlock) void bucket_sort_kernel(uint64_t *bucke
     for (int o = tid; o < count; o += kSortBlock) values_out[start + o] = (int)(src[o] & value_mask);
 }
 
+// The place of a key is the number of smaller ones. A workgroup ranks 64 keys (one per lane), each of its 16 waves
+// against a sixteenth of all keys, which are the same for every lane and come as scalar loads: two vector instructions
+// per pair (64-bit compare, add with carry), no LDS and no barrier but the last sum. Bound by vector issue, n^2 / 2^16
+// pairs per SIMD at most. The bitonic network over the same 5000 keys in one workgroup is 91 dependent exchange steps
+// (44 us, a fifth of a condensate call).
+__global__ __launch_bounds__(kSortBlock) void rank_kernel(const uint64_t *__restrict__ keys, int n, uint64_t value_mask,
+                                                          int *__restrict__ values_out) {
+    constexpr int waves = kSortBlock / kWave;
+    __shared__ int s_below[waves][kWave];
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = blockIdx.x * kWave + lane;
+    const uint64_t mine = i < n ? keys[i] : 0ull;
+    const int per_wave = (n + waves - 1) / waves;
+    const int begin = min(n, wave * per_wave), end = min(n, begin + per_wave);
+    // equal keys keep their order: those in front of this workgroup's count, those behind it do not
+    const int own = min(max((int)blockIdx.x * kWave, begin), end);
+    const int behind = min(max(((int)blockIdx.x + 1) * kWave, begin), end);
+    int below = 0;
+    int j = begin;
+    for (; j + 8 <= own; j += 8)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) below += keys[j + u] <= mine ? 1 : 0;
+    for (; j < own; ++j) below += keys[j] <= mine ? 1 : 0;
+    for (; j < behind; ++j) below += (keys[j] < mine || (keys[j] == mine && j < i)) ? 1 : 0;
+    for (; j + 8 <= end; j += 8)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) below += keys[j + u] < mine ? 1 : 0;
+    for (; j < end; ++j) below += keys[j] < mine ? 1 : 0;
+    s_below[wave][lane] = below;
+    __syncthreads();
+    if (wave == 0 && i < n) {
+        int place = 0;
+#pragma unroll
+        for (int w = 0; w < waves; ++w) place += s_below[w][lane];
+        values_out[place] = (int)(mine & value_mask);
+    }
+}
+
 int buckets_for(long long n) {
     if (n <= kBucketStage) return 1;
     int buckets = 2;
@@ -336,13 +379,17 @@ int sample_sort_values(uint64_t *d_keys, uint64_t *d_spare, long long n, int val
                        void *workspace, size_t workspace_bytes, int stage, hipStream_t s) {
     HGC_REQUIRE(sample_sort_supported(n), "sample sort: too many keys");
     HGC_REQUIRE(value_bits >= 1 && value_bits <= 31, "sample sort: 1 <= value bits <= 31");
-    if (stage == 0) stage = kBucketStage;
-    HGC_REQUIRE(stage >= 2 && stage <= kBucketStage && (stage & (stage - 1)) == 0, "sample sort: bad stage");
+    HGC_REQUIRE(stage == 0 || (stage >= 2 && stage <= kBucketStage && (stage & (stage - 1)) == 0), "sample sort: bad stage");
     if (n == 0) return HGC_OK;
     HGC_REQUIRE(d_keys && d_spare && d_values, "null pointer");
     if (!workspace || !aligned256(workspace) || workspace_bytes < sample_sort_workspace_bytes())
         return fail(HGC_ERR_WORKSPACE, "sample sort workspace missing, misaligned or too small");
     const uint64_t mask = (1ull << value_bits) - 1ull;
+    if (stage == 0 && n <= kRankLimit) {
+        rank_kernel<<<ceil_div(n, kWave), kSortBlock, 0, s>>>(d_keys, (int)n, mask, d_values);
+        return check_launch("rank");
+    }
+    if (stage == 0) stage = kBucketStage;
     const int buckets = buckets_for(n);
     if (buckets == 1) {
         bucket_sort_kernel<<<1, kSortBlock, 0, s>>>(d_keys, d_spare, nullptr, 1, (int)n, stage, mask, d_values);
