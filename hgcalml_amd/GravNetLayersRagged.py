@@ -11,6 +11,7 @@ and through the dense layers (torch).
 import torch
 from torch import nn
 
+from . import globals as gl
 from . import ops
 from .accknn_op import AccumulateKnn, AccumulateKnnSumw
 from .binned_select_knn_op import BinnedSelectKnn
@@ -24,6 +25,60 @@ def eye_init_(weight, mean=0.0, stddev=0.1, eye_scaling=1.0):
         n_out, n_in = weight.shape
         weight += torch.eye(n_in, n_out, dtype=weight.dtype, device=weight.device).t() * eye_scaling
     return weight
+
+
+def _library_takes(*tensors):
+    """whether the library's passes stand for the tensor operations: float32 on one GPU, at least one row, no
+    derivative of the derivative asked for, and neither switch that asks for differentiable compositions"""
+    if gl.knn_ops_use_tf_gradients or gl.acc_ops_use_tf_gradients:
+        return False
+    return all(t.is_cuda and t.dtype == torch.float32 and t.numel() > 0 and t.device == tensors[0].device
+               for t in tensors)
+
+
+def _sum_rows(t):
+    """t.sum(0)"""
+    if torch.is_grad_enabled() or not _library_takes(t) or t[0].numel() > 1 << 20:
+        return t.sum(0)
+    return ops.column_sums(t.reshape(t.shape[0], -1)).view(t.shape[1:])
+
+
+class _DropSelfFn(torch.autograd.Function):
+    """table and distances without the self column, and the distances themselves: the gradients of both come back in
+    one pass"""
+
+    @staticmethod
+    def forward(ctx, idx, dist):
+        ctx.set_materialize_grads(False)
+        nidx, ndist = ops.gravnet_drop_self(idx, dist)
+        ctx.mark_non_differentiable(nidx)
+        return nidx, ndist, dist
+
+    @staticmethod
+    def backward(ctx, _grad_nidx, grad_narrow, grad_wide):
+        if grad_narrow is None:
+            return None, grad_wide
+        if torch.is_grad_enabled():
+            grad = torch.nn.functional.pad(grad_narrow, (1, 0))
+            return None, grad if grad_wide is None else grad + grad_wide
+        return None, ops.gravnet_drop_self_grad(grad_narrow, grad_wide)
+
+
+class _JoinFn(torch.autograd.Function):
+    """[accumulated - (features | features) | x] and its gradients, one pass each"""
+
+    @staticmethod
+    def forward(ctx, accumulated, features, x):
+        ctx.n_features = features.shape[1]
+        return ops.gravnet_join(accumulated, features, x)
+
+    @staticmethod
+    def backward(ctx, grad):
+        f = ctx.n_features
+        if torch.is_grad_enabled():
+            return grad[:, :2 * f], -grad[:, :f] - grad[:, f:2 * f], grad[:, 2 * f:]
+        out = ops.gravnet_join_grad(grad, f, *ctx.needs_input_grad)
+        return tuple(g if want else None for g, want in zip(out, ctx.needs_input_grad))
 
 
 class _TallLinearFn(torch.autograd.Function):
@@ -50,12 +105,13 @@ class _TallLinearFn(torch.autograd.Function):
             whole = n // s * s
             if whole >= 64 * s:
                 grad_w = torch.bmm(g[:whole].view(s, -1, g.shape[1]).transpose(1, 2),
-                                   x[:whole].view(s, -1, x.shape[1])).sum(0)
+                                   x[:whole].view(s, -1, x.shape[1]))
+                grad_w = _sum_rows(grad_w)
                 if whole < n:
                     grad_w = grad_w + g[whole:].t() @ x[whole:]
             else:
                 grad_w = g.t() @ x
-        grad_b = g.sum(0) if ctx.has_bias and ctx.needs_input_grad[2] else None
+        grad_b = _sum_rows(g) if ctx.has_bias and ctx.needs_input_grad[2] else None
         return grad_x, grad_w, grad_b
 
 
@@ -101,6 +157,9 @@ class RaggedGravNet(nn.Module):
         if not self.training:
             return
         with torch.no_grad():
+            if _library_takes(dist, self.dynamic_radius):
+                self.dynamic_radius += ops.gravnet_radius_step(dist, self.dynamic_radius)
+                return
             lindist = torch.sqrt(dist)
             update = lindist.max() * 1.05
             mean_dist = lindist.mean()
@@ -111,11 +170,13 @@ class RaggedGravNet(nn.Module):
     def compute_neighbours_and_distancesq(self, coordinates, row_splits):
         idx, dist = BinnedSelectKnn(self.n_neighbours + 1, coordinates, row_splits, max_radius=-1.0,
                                     tf_compatible=False, n_bins=self.n_knn_bins)
-        dist = torch.where(idx < 0, torch.zeros_like(dist), dist)
-        self.update_dynamic_radius(dist.detach())
+        self.update_dynamic_radius(dist.detach())  # missing neighbours have distance 0
         # the table without its self column, as tensors of their own; it lists the
         # same vertices row by row, so the kNN's processing order applies to it too
-        nidx, ndist = idx[:, 1:].contiguous(), dist[:, 1:].contiguous()
+        if _library_takes(dist):
+            nidx, ndist, dist = _DropSelfFn.apply(idx, dist)
+        else:
+            nidx, ndist = idx[:, 1:].contiguous(), dist[:, 1:].contiguous()
         ops.share_vertex_order(idx, nidx)
         ops.declare_without_first_column(nidx, idx)
         if self.return_self:
@@ -132,8 +193,11 @@ class RaggedGravNet(nn.Module):
         prev_feat = features
         features = self.collect_neighbours(features, neighbour_indices, distancesq)
         features = features.reshape(-1, prev_feat.shape[1] * 2)
-        features = features - prev_feat.repeat(1, 2)
-        return torch.relu(self.output_feature_transform(torch.cat([features, x], dim=-1)))
+        if _library_takes(features, prev_feat, x):
+            joined = _JoinFn.apply(features, prev_feat, x)
+        else:
+            joined = torch.cat([features - prev_feat.repeat(1, 2), x], dim=-1)
+        return torch.relu(self.output_feature_transform(joined))
 
     def forward(self, x, row_splits):
         assert x.dim() == 2 and row_splits.dim() == 1

@@ -64,6 +64,14 @@ _SIGNATURES = {
     "hgc_push_knn_grad": (_c_int, [_ptr] * 6 + [_c_int] * 3 + [_ptr]),
     "hgc_exp_neg": (_c_int, [_ptr, _ptr, ctypes.c_longlong, _ptr]),
     "hgc_exp_neg_grad": (_c_int, [_ptr, _ptr, _ptr, ctypes.c_longlong, _ptr]),
+    "hgc_gravnet_drop_self": (_c_int, [_ptr] * 2 + [_c_int] * 2 + [_ptr] * 3),
+    "hgc_gravnet_drop_self_grad": (_c_int, [_ptr] * 2 + [_c_int] * 2 + [_ptr] * 2),
+    "hgc_gravnet_radius_step_workspace_bytes": (_c_size, []),
+    "hgc_gravnet_radius_step": (_c_int, [_ptr, ctypes.c_longlong] + [_ptr] * 3 + [_c_size, _ptr]),
+    "hgc_gravnet_join": (_c_int, [_ptr] * 3 + [_c_int] * 3 + [_ptr] * 2),
+    "hgc_gravnet_join_grad": (_c_int, [_ptr] + [_c_int] * 3 + [_ptr] * 4),
+    "hgc_column_sums_workspace_bytes": (_c_size, [_c_int] * 2),
+    "hgc_column_sums": (_c_int, [_ptr] + [_c_int] * 2 + [_ptr] * 2 + [_c_size, _ptr]),
     "hgc_binned_assign_to_condensates_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int]),
     "hgc_binned_assign_to_condensates": (_c_int, [_c_int, _c_int] + [_ptr] * 21 + [_c_int] * 4 + [_ptr, _ptr, _c_size, _ptr]),
     "hgc_build_and_assign_condensates_workspace_bytes": (_c_size, [_c_int] * 5),

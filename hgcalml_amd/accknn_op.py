@@ -20,10 +20,13 @@ class _AccumulateFn(torch.autograd.Function):
         ctx.save_for_backward(weights, features, indices, maxidx, slots)
         ctx.indices_ref = indices
         ctx.mark_non_differentiable(maxidx)
+        ctx.set_materialize_grads(False)  # no zeros for the index output
         return out, maxidx
 
     @staticmethod
     def backward(ctx, grad_out, _grad_maxidx):
+        if grad_out is None:
+            return None, None, None, None
         weights, features, indices, maxidx, slots = ctx.saved_tensors
         inv_off, inv_slots = ops.cached_inverse_neighbour_index(ctx.indices_ref)
         gw, gx = torch.ops.hgcalml.accumulate_knn_grad_slots(grad_out.contiguous(), weights, features, indices,
@@ -42,10 +45,13 @@ class _AccumulateExpFn(torch.autograd.Function):
         ctx.save_for_backward(weights, features, indices, maxidx, slots)
         ctx.indices_ref = indices
         ctx.mark_non_differentiable(maxidx)
+        ctx.set_materialize_grads(False)  # no zeros for the index output
         return out, maxidx
 
     @staticmethod
     def backward(ctx, grad_out, _grad_maxidx):
+        if grad_out is None:
+            return None, None, None, None
         weights, features, indices, maxidx, slots = ctx.saved_tensors
         inv_off, inv_slots = ops.cached_inverse_neighbour_index(ctx.indices_ref)
         gd, gx = torch.ops.hgcalml.accumulate_knn_grad_exp_slots(grad_out.contiguous(), weights, features, indices,

@@ -31,10 +31,13 @@ class _BinnedSelectKnnFn(torch.autograd.Function):
                                                    max_radius)
         ctx.save_for_backward(coords, idx, dist)
         ctx.mark_non_differentiable(idx)
+        ctx.set_materialize_grads(False)  # no zeros for the index output
         return idx, dist
 
     @staticmethod
     def backward(ctx, _grad_idx, grad_dist):
+        if grad_dist is None:
+            return (None,) * 8
         coords, idx, dist = ctx.saved_tensors
         grad_coords = torch.ops.hgcalml.select_knn_grad(grad_dist.contiguous(), idx, dist, coords)
         return grad_coords, None, None, None, None, None, None, None

@@ -1,0 +1,404 @@
+// The memory passes of the GravNet block around its search and accumulation
+// (modules/GravNetLayersRagged.py:3095-3283): the neighbour table and distances without the self column, the update of
+// the dynamic radius, the row [mean - p | max - p | x] that the last dense layer reads, and sums over the rows for the
+// gradients of the dense layers. All of them stream; as single tensor operations they were 40 launches and, at 150k
+// vertices, K = 64, F = 64, 0.6 of the 2.45 ms of a training step, most of it intermediates written and read again; the
+// step takes 2.19 ms with these (240k vertices, K = 40, F = 32 with the weights' sum: 2.97 -> 2.72). What is left of them
+// runs at 4 to 5 TB/s: at 150k vertices 36 us each for the join and its gradient (115 and 154 MB), the table and its
+// gradient, 13 us for the radius.
+#include <algorithm>
+#include <cmath>
+
+#include "hgc_common.hpp"
+
+namespace hgc {
+namespace {
+
+constexpr int kThreads = 256;
+
+// ---- table and distances without column 0 -------------------------------------------------------------------------
+
+// A thread moves four consecutive entries of the narrow table (16-byte stores); the wide rows start anywhere, their
+// loads are four dwords each that neighbouring lanes complete to whole lines.
+__global__ __launch_bounds__(kThreads) void drop_self_kernel(const int *__restrict__ idx, const float *__restrict__ dist,
+                                                             unsigned total, unsigned narrow, int *__restrict__ out_idx,
+                                                             float *__restrict__ out_dist) {
+    const unsigned first = (blockIdx.x * kThreads + threadIdx.x) * 4u;
+    if (first >= total) return;
+    unsigned row = first / narrow, col = first - row * narrow;
+    int ai[4];
+    float di[4];
+    const unsigned count = min(4u, total - first);
+#pragma unroll
+    for (unsigned u = 0; u < 4; ++u) {
+        if (u < count) {
+            ai[u] = idx[first + u + row + 1];  // row * (narrow + 1) + col + 1
+            di[u] = dist[first + u + row + 1];
+        }
+        if (++col == narrow) col = 0, ++row;
+    }
+    if (count == 4) {
+        *reinterpret_cast<int4 *>(out_idx + first) = int4{ai[0], ai[1], ai[2], ai[3]};
+        *reinterpret_cast<float4 *>(out_dist + first) = float4{di[0], di[1], di[2], di[3]};
+    } else {
+#pragma unroll
+        for (unsigned u = 0; u < 3; ++u)
+            if (u < count) out_idx[first + u] = ai[u], out_dist[first + u] = di[u];
+    }
+}
+
+// gradient w.r.t. the wide distances: that of the narrow ones moved up by a column, plus that of the wide ones (if any)
+__global__ __launch_bounds__(kThreads) void drop_self_grad_kernel(const float *__restrict__ g_narrow,
+                                                                  const float *__restrict__ g_wide, unsigned total,
+                                                                  unsigned wide, float *__restrict__ out) {
+    const unsigned first = (blockIdx.x * kThreads + threadIdx.x) * 4u;
+    if (first >= total) return;
+    unsigned row = first / wide, col = first - row * wide;
+    const unsigned count = min(4u, total - first);
+    float vi[4] = {0.f, 0.f, 0.f, 0.f};
+    if (g_wide && count == 4) {
+        const float4 v = *reinterpret_cast<const float4 *>(g_wide + first);
+        vi[0] = v.x, vi[1] = v.y, vi[2] = v.z, vi[3] = v.w;
+    } else if (g_wide) {
+#pragma unroll
+        for (unsigned u = 0; u < 3; ++u)
+            if (u < count) vi[u] = g_wide[first + u];
+    }
+#pragma unroll
+    for (unsigned u = 0; u < 4; ++u) {
+        if (u < count && col > 0) vi[u] += g_narrow[first + u - row - 1];
+        if (++col == wide) col = 0, ++row;
+    }
+    if (count == 4) {
+        *reinterpret_cast<float4 *>(out + first) = float4{vi[0], vi[1], vi[2], vi[3]};
+    } else {
+#pragma unroll
+        for (unsigned u = 0; u < 3; ++u)
+            if (u < count) out[first + u] = vi[u];
+    }
+}
+
+// ---- dynamic radius -----------------------------------------------------------------------------------------------
+
+constexpr int kRadiusBlocks = 512;
+
+struct MaxSum {
+    double sum;
+    float max;
+};
+
+__device__ __forceinline__ void fold(MaxSum &a, float max, double sum) {
+    a.max = (max > a.max || max != max) ? max : a.max;  // NaN stays, as in torch's max
+    a.sum += sum;
+}
+
+__device__ __forceinline__ MaxSum block_fold(MaxSum a) {
+    __shared__ MaxSum s_wave[kThreads / kWave];
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+        const float m = __shfl_xor(a.max, off);
+        const double sum = __shfl_xor(a.sum, off);
+        fold(a, m, sum);
+    }
+    if (lane_id() == 0) s_wave[threadIdx.x / kWave] = a;
+    __syncthreads();
+    a = s_wave[0];
+    for (int w = 1; w < kThreads / kWave; ++w) fold(a, s_wave[w].max, s_wave[w].sum);
+    return a;
+}
+
+// largest distance and sum of the distances (roots of the squares), one pair per workgroup
+__global__ __launch_bounds__(kThreads) void radius_parts_kernel(const float *__restrict__ distsq, long long total,
+                                                                MaxSum *__restrict__ parts) {
+    MaxSum a{0.0, 0.f};  // no distance is negative
+    const long long whole = total / 4;
+    for (long long i = (long long)blockIdx.x * kThreads + threadIdx.x; i < whole; i += (long long)gridDim.x * kThreads) {
+        const float4 v = reinterpret_cast<const float4 *>(distsq)[i];
+        const float x = sqrtf(v.x), y = sqrtf(v.y), z = sqrtf(v.z), w = sqrtf(v.w);
+        fold(a, x, 0.0);
+        fold(a, y, 0.0);
+        fold(a, z, 0.0);
+        fold(a, w, (double)x + (double)y + ((double)z + (double)w));
+    }
+    if (blockIdx.x == 0 && threadIdx.x < total - whole * 4) {
+        const float x = sqrtf(distsq[whole * 4 + threadIdx.x]);
+        fold(a, x, x);
+    }
+    a = block_fold(a);
+    if (threadIdx.x == 0) parts[blockIdx.x] = a;
+}
+
+// 0.05 (update - radius), update = max(min(1.05 largest, 2), 2 mean) + 1e-3
+__global__ __launch_bounds__(kThreads) void radius_step_kernel(const MaxSum *__restrict__ parts, int n_parts,
+                                                               long long total, const float *__restrict__ radius,
+                                                               float *__restrict__ step) {
+    MaxSum a{0.0, 0.f};
+    for (int i = threadIdx.x; i < n_parts; i += kThreads) fold(a, parts[i].max, parts[i].sum);
+    a = block_fold(a);
+    if (threadIdx.x == 0) {
+        const float reach = a.max * 1.05f;
+        const float low = reach > 2.f ? 2.f : reach;  // NaN stays
+        const float twice = 2.f * (float)(a.sum / (double)total);
+        const float update = (low > twice ? low : twice) + 1e-3f;
+        *step = 0.05f * (update - *radius);
+    }
+}
+
+// ---- the last dense layer's input ---------------------------------------------------------------------------------
+
+// VEC consecutive columns of a row per thread; a workgroup takes `rows` whole rows
+template <int VEC>
+struct Vec;
+template <>
+struct Vec<1> {
+    using type = float;
+};
+template <>
+struct Vec<4> {
+    using type = float4;
+};
+
+__device__ __forceinline__ float minus(float a, float b) { return a - b; }
+__device__ __forceinline__ float4 minus(float4 a, float4 b) { return {a.x - b.x, a.y - b.y, a.z - b.z, a.w - b.w}; }
+__device__ __forceinline__ float minus_sum(float a, float b) { return -a - b; }
+__device__ __forceinline__ float4 minus_sum(float4 a, float4 b) { return {-a.x - b.x, -a.y - b.y, -a.z - b.z, -a.w - b.w}; }
+
+// out row: acc[0..F) - p | acc[F..2F) - p | x; widths in units of VEC columns
+template <int VEC>
+__global__ __launch_bounds__(kThreads) void join_rows_kernel(const float *__restrict__ acc, const float *__restrict__ p,
+                                                             const float *__restrict__ x, int n, int rows, unsigned f,
+                                                             unsigned w_x, float *__restrict__ out) {
+    using V = typename Vec<VEC>::type;
+    const unsigned width = 2 * f + w_x;
+    const long long first = (long long)blockIdx.x * rows;
+    const unsigned items = (unsigned)min((long long)rows, n - first) * width;
+    const V *acc_v = reinterpret_cast<const V *>(acc) + first * 2 * f;
+    const V *p_v = reinterpret_cast<const V *>(p) + first * f;
+    const V *x_v = reinterpret_cast<const V *>(x) + first * w_x;
+    V *out_v = reinterpret_cast<V *>(out) + first * width;
+    for (unsigned t = threadIdx.x; t < items; t += kThreads) {
+        const unsigned row = t / width, col = t - row * width;
+        V v;
+        if (col < 2 * f)
+            v = minus(acc_v[row * 2 * f + col], p_v[row * f + (col < f ? col : col - f)]);
+        else
+            v = x_v[row * w_x + (col - 2 * f)];
+        out_v[t] = v;
+    }
+}
+
+// its gradient: to acc (2F columns), to p (-(first half) - (second half)), to x; outputs may be null
+template <int VEC>
+__global__ __launch_bounds__(kThreads) void join_rows_grad_kernel(const float *__restrict__ g, int n, int rows, unsigned f,
+                                                                  unsigned w_x, float *__restrict__ g_acc,
+                                                                  float *__restrict__ g_p, float *__restrict__ g_x) {
+    using V = typename Vec<VEC>::type;
+    const unsigned width = 2 * f + w_x, tasks = f + w_x;
+    const long long first = (long long)blockIdx.x * rows;
+    const unsigned items = (unsigned)min((long long)rows, n - first) * tasks;
+    const V *g_v = reinterpret_cast<const V *>(g) + first * width;
+    V *acc_v = reinterpret_cast<V *>(g_acc) + first * 2 * f;
+    V *p_v = reinterpret_cast<V *>(g_p) + first * f;
+    V *x_v = reinterpret_cast<V *>(g_x) + first * w_x;
+    for (unsigned t = threadIdx.x; t < items; t += kThreads) {
+        const unsigned row = t / tasks, col = t - row * tasks;
+        if (col < f) {
+            const V a = g_v[row * width + col], b = g_v[row * width + f + col];
+            if (g_acc) acc_v[row * 2 * f + col] = a, acc_v[row * 2 * f + f + col] = b;
+            if (g_p) p_v[row * f + col] = minus_sum(a, b);
+        } else if (g_x) {
+            x_v[row * w_x + (col - f)] = g_v[row * width + f + col];
+        }
+    }
+}
+
+// ---- sums over the rows -------------------------------------------------------------------------------------------
+
+// Columns are cut into tiles of `tile` vectors (grid.y), rows into grid.x slabs; a thread adds its columns of every
+// (256 / tile)-th row of the slab, four loads under way at a time, the groups of a workgroup meet in LDS. With one slab the
+// results are final, otherwise one row per slab is left and added by a second launch of the same kernel.
+template <int VEC>
+__global__ __launch_bounds__(kThreads) void column_sums_kernel(const float *__restrict__ x, int n_rows, int cols_v,
+                                                               int tile_width, int slab, float *__restrict__ out) {
+    using V = typename Vec<VEC>::type;
+    __shared__ float s_part[kThreads * VEC];
+    const int tile = blockIdx.y * tile_width;
+    const int width = min(tile_width, cols_v - tile);
+    const int groups = kThreads / width;
+    const int group = threadIdx.x / width, col = threadIdx.x - group * width;
+    const int begin = blockIdx.x * slab, end = min(n_rows, begin + slab);
+    const V *src = reinterpret_cast<const V *>(x) + tile + col;
+    float sum[VEC] = {};
+    auto add = [&](const V &v) {
+        const float *f = reinterpret_cast<const float *>(&v);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) sum[e] += f[e];
+    };
+    if (group < groups) {
+        int r = begin + group;
+        for (; r + 3 * groups < end; r += 4 * groups) {
+            const V a = src[(size_t)r * cols_v], b = src[(size_t)(r + groups) * cols_v];
+            const V c = src[(size_t)(r + 2 * groups) * cols_v], d = src[(size_t)(r + 3 * groups) * cols_v];
+            add(a), add(b), add(c), add(d);
+        }
+        for (; r < end; r += groups) add(src[(size_t)r * cols_v]);
+    }
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) s_part[e * kThreads + threadIdx.x] = sum[e];
+    __syncthreads();
+    if (threadIdx.x < width) {
+        float *o = out + ((size_t)blockIdx.x * cols_v + tile + col) * VEC;
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            float s = s_part[e * kThreads + threadIdx.x];
+            for (int g = 1; g < groups; ++g) s += s_part[e * kThreads + g * width + threadIdx.x];
+            o[e] = s;
+        }
+    }
+}
+
+struct SumsPlan {
+    int vec, cols_v, tile, slab, slabs;
+};
+
+// First pass: tiles of 32 vectors (128 or 512 bytes of a row), 16 rows or more per thread, up to about 512 workgroups.
+SumsPlan sums_plan(int n_rows, int cols, int vec) {
+    SumsPlan p;
+    p.vec = vec;
+    p.cols_v = cols / vec;
+    p.tile = std::min(32, p.cols_v);
+    const int most = std::max(1, 512 / ceil_div(p.cols_v, p.tile));
+    p.slab = std::max(16 * (kThreads / p.tile), ceil_div(n_rows, most));
+    p.slabs = ceil_div(n_rows, p.slab);
+    return p;
+}
+
+int launch_column_sums(const float *x, int n_rows, const SumsPlan &p, float *out, hipStream_t s) {
+    const dim3 grid(p.slabs, ceil_div(p.cols_v, p.tile));
+    if (p.vec == 4)
+        column_sums_kernel<4><<<grid, kThreads, 0, s>>>(x, n_rows, p.cols_v, p.tile, p.slab, out);
+    else
+        column_sums_kernel<1><<<grid, kThreads, 0, s>>>(x, n_rows, p.cols_v, p.tile, p.slab, out);
+    return check_launch("column_sums");
+}
+
+int rows_per_block(unsigned items_per_row) { return std::max(1, (int)(4 * kThreads / std::max(1u, items_per_row))); }
+
+bool aligned16(std::initializer_list<const void *> pointers) {
+    for (const void *p : pointers)
+        if (reinterpret_cast<uintptr_t>(p) & 15u) return false;
+    return true;
+}
+
+}  // namespace
+}  // namespace hgc
+
+using namespace hgc;
+
+extern "C" {
+
+int hgc_gravnet_drop_self(const int *d_idxs, const float *d_dist, int n_vert, int n_neigh, int *d_out_idxs,
+                          float *d_out_dist, hgc_stream_t stream) {
+    HGC_REQUIRE(n_vert >= 0 && n_neigh >= 2, "n_vert >= 0, n_neigh >= 2");
+    HGC_REQUIRE((long long)n_vert * n_neigh < (1ll << 31) - 4, "n_vert * n_neigh must stay below 2^31");
+    if (n_vert == 0) return HGC_OK;
+    HGC_REQUIRE(d_idxs && d_dist && d_out_idxs && d_out_dist, "null pointer");
+    HGC_REQUIRE(aligned16({d_out_idxs, d_out_dist}), "outputs must lie on 16-byte boundaries");
+    const unsigned total = (unsigned)n_vert * (unsigned)(n_neigh - 1);
+    drop_self_kernel<<<ceil_div(total, 4 * kThreads), kThreads, 0, as_stream(stream)>>>(
+        d_idxs, d_dist, total, (unsigned)(n_neigh - 1), d_out_idxs, d_out_dist);
+    return check_launch("gravnet_drop_self");
+}
+
+int hgc_gravnet_drop_self_grad(const float *d_grad_narrow, const float *d_grad_wide, int n_vert, int n_neigh,
+                               float *d_out_grad, hgc_stream_t stream) {
+    HGC_REQUIRE(n_vert >= 0 && n_neigh >= 2, "n_vert >= 0, n_neigh >= 2");
+    HGC_REQUIRE((long long)n_vert * n_neigh < (1ll << 31) - 4, "n_vert * n_neigh must stay below 2^31");
+    if (n_vert == 0) return HGC_OK;
+    HGC_REQUIRE(d_grad_narrow && d_out_grad, "null pointer");
+    HGC_REQUIRE(aligned16({d_grad_wide, d_out_grad}), "wide gradients must lie on 16-byte boundaries");
+    const unsigned total = (unsigned)n_vert * (unsigned)n_neigh;
+    drop_self_grad_kernel<<<ceil_div(total, 4 * kThreads), kThreads, 0, as_stream(stream)>>>(
+        d_grad_narrow, d_grad_wide, total, (unsigned)n_neigh, d_out_grad);
+    return check_launch("gravnet_drop_self_grad");
+}
+
+size_t hgc_gravnet_radius_step_workspace_bytes(void) { return align_up(kRadiusBlocks * sizeof(MaxSum)); }
+
+int hgc_gravnet_radius_step(const float *d_distsq, long long total, const float *d_radius, float *d_step, void *workspace,
+                            size_t workspace_bytes, hgc_stream_t stream) {
+    HGC_REQUIRE(total >= 1, "the largest of no distances is not defined");
+    HGC_REQUIRE(d_distsq && d_radius && d_step, "null pointer");
+    HGC_REQUIRE(aligned16({d_distsq}), "distances must lie on a 16-byte boundary");
+    if (!workspace || !aligned256(workspace) || workspace_bytes < hgc_gravnet_radius_step_workspace_bytes())
+        return fail(HGC_ERR_WORKSPACE, "radius step workspace missing, misaligned or too small");
+    MaxSum *parts = static_cast<MaxSum *>(workspace);
+    const int blocks = (int)std::max(1ll, std::min<long long>(kRadiusBlocks, total / (16 * kThreads)));
+    radius_parts_kernel<<<blocks, kThreads, 0, as_stream(stream)>>>(d_distsq, total, parts);
+    radius_step_kernel<<<1, kThreads, 0, as_stream(stream)>>>(parts, blocks, total, d_radius, d_step);
+    return check_launch("gravnet_radius_step");
+}
+
+int hgc_gravnet_join(const float *d_acc, const float *d_features, const float *d_x, int n_vert, int n_feat, int n_x,
+                     float *d_out, hgc_stream_t stream) {
+    HGC_REQUIRE(n_vert >= 0 && n_feat >= 1 && n_x >= 1 && n_feat <= 1 << 20 && n_x <= 1 << 20, "bad sizes");
+    if (n_vert == 0) return HGC_OK;
+    HGC_REQUIRE(d_acc && d_features && d_x && d_out, "null pointer");
+    const bool wide = n_feat % 4 == 0 && n_x % 4 == 0 && aligned16({d_acc, d_features, d_x, d_out});
+    const int vec = wide ? 4 : 1;
+    const unsigned f = n_feat / vec, w = n_x / vec;
+    const int rows = rows_per_block(2 * f + w);
+    const int grid = ceil_div(n_vert, rows);
+    if (wide)
+        join_rows_kernel<4><<<grid, kThreads, 0, as_stream(stream)>>>(d_acc, d_features, d_x, n_vert, rows, f, w, d_out);
+    else
+        join_rows_kernel<1><<<grid, kThreads, 0, as_stream(stream)>>>(d_acc, d_features, d_x, n_vert, rows, f, w, d_out);
+    return check_launch("gravnet_join");
+}
+
+int hgc_gravnet_join_grad(const float *d_grad, int n_vert, int n_feat, int n_x, float *d_grad_acc, float *d_grad_features,
+                          float *d_grad_x, hgc_stream_t stream) {
+    HGC_REQUIRE(n_vert >= 0 && n_feat >= 1 && n_x >= 1 && n_feat <= 1 << 20 && n_x <= 1 << 20, "bad sizes");
+    if (n_vert == 0) return HGC_OK;
+    HGC_REQUIRE(d_grad, "null pointer");
+    const bool wide = n_feat % 4 == 0 && n_x % 4 == 0 && aligned16({d_grad, d_grad_acc, d_grad_features, d_grad_x});
+    const int vec = wide ? 4 : 1;
+    const unsigned f = n_feat / vec, w = n_x / vec;
+    const int rows = rows_per_block(f + w);
+    const int grid = ceil_div(n_vert, rows);
+    if (wide)
+        join_rows_grad_kernel<4><<<grid, kThreads, 0, as_stream(stream)>>>(d_grad, n_vert, rows, f, w, d_grad_acc,
+                                                                          d_grad_features, d_grad_x);
+    else
+        join_rows_grad_kernel<1><<<grid, kThreads, 0, as_stream(stream)>>>(d_grad, n_vert, rows, f, w, d_grad_acc,
+                                                                          d_grad_features, d_grad_x);
+    return check_launch("gravnet_join_grad");
+}
+
+size_t hgc_column_sums_workspace_bytes(int n_rows, int n_cols) {
+    if (n_rows < 1 || n_cols < 1) return 0;
+    // one row of partial sums per slab, whichever vector width the call takes
+    int slabs = sums_plan(n_rows, n_cols, 1).slabs;
+    if (n_cols % 4 == 0) slabs = std::max(slabs, sums_plan(n_rows, n_cols, 4).slabs);
+    return slabs > 1 ? align_up((size_t)slabs * n_cols * sizeof(float)) : 0;
+}
+
+int hgc_column_sums(const float *d_x, int n_rows, int n_cols, float *d_sums, void *workspace, size_t workspace_bytes,
+                    hgc_stream_t stream) {
+    HGC_REQUIRE(n_rows >= 1 && n_cols >= 1 && n_cols <= 1 << 20, "bad sizes");
+    HGC_REQUIRE(d_x && d_sums, "null pointer");
+    const size_t need = hgc_column_sums_workspace_bytes(n_rows, n_cols);
+    if (need && (!workspace || !aligned256(workspace) || workspace_bytes < need))
+        return fail(HGC_ERR_WORKSPACE, "column sums workspace missing, misaligned or too small");
+    hipStream_t s = as_stream(stream);
+    const SumsPlan p = sums_plan(n_rows, n_cols, n_cols % 4 == 0 && aligned16({d_x, d_sums}) ? 4 : 1);
+    if (p.slabs == 1) return launch_column_sums(d_x, n_rows, p, d_sums, s);
+    float *parts = static_cast<float *>(workspace);
+    if (int rc = launch_column_sums(d_x, n_rows, p, parts, s)) return rc;
+    SumsPlan last = p;  // few rows: narrow tiles, so that many groups share them
+    last.tile = std::min(8, p.cols_v);
+    last.slab = p.slabs;
+    last.slabs = 1;
+    return launch_column_sums(parts, p.slabs, last, d_sums, s);
+}
+
+}  // extern "C"

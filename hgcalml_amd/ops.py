@@ -660,6 +660,106 @@ def exp_neg_grad(weight_grad, weights):
     return out
 
 
+# --------------------------------------------------------------------------- GravNet block
+
+# Several of these run per training step of a small event, where host time counts: defined below custom_op, whose
+# wrapper costs more than the launches.
+_FRAGMENT = torch.library.Library("hgcalml", "FRAGMENT")
+
+
+def _op(schema):
+    name = schema.split("(")[0]
+    _FRAGMENT.define(schema)
+
+    def register(fn):
+        _FRAGMENT.impl(name, fn, "CUDA")
+        return getattr(torch.ops.hgcalml, name).default
+    return register
+
+
+def _aligned(t):
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+@_op("gravnet_drop_self(Tensor indices, Tensor distances) -> (Tensor, Tensor)")
+def gravnet_drop_self(indices, distances):
+    """neighbour table and squared distances without their first column"""
+    dev = require_device(indices, distances)
+    idx, d = i32(indices), f32(distances)
+    n, k = idx.shape
+    if d.shape != idx.shape or k < 2:
+        raise ValueError("gravnet_drop_self: indices and distances [N, K >= 2] expected")
+    out_idx = torch.empty((n, k - 1), dtype=torch.int32, device=dev)
+    out = torch.empty((n, k - 1), dtype=torch.float32, device=dev)
+    check(lib.hgc_gravnet_drop_self(p(idx), p(d), n, k, p(out_idx), p(out), stream()))
+    return out_idx, out
+
+
+@_op("gravnet_drop_self_grad(Tensor grad_narrow, Tensor? grad_wide) -> Tensor")
+def gravnet_drop_self_grad(grad_narrow, grad_wide):
+    """gradient of gravnet_drop_self w.r.t. the distances, added to their own gradient (if there is one)"""
+    dev = require_device(grad_narrow, grad_wide)
+    narrow = f32(grad_narrow)
+    wide = None if grad_wide is None else _aligned(f32(grad_wide))
+    n, k = narrow.shape[0], narrow.shape[1] + 1
+    if wide is not None and wide.shape != (n, k):
+        raise ValueError("gravnet_drop_self_grad: gradients of shape [N, K - 1] and [N, K] expected")
+    out = torch.empty((n, k), dtype=torch.float32, device=dev)
+    check(lib.hgc_gravnet_drop_self_grad(p(narrow), p(wide), n, k, p(out), stream()))
+    return out
+
+
+@_op("gravnet_radius_step(Tensor distances, Tensor radius) -> Tensor")
+def gravnet_radius_step(distances, radius):
+    """what one training step adds to the dynamic radius (modules/GravNetLayersRagged.py:3180-3193)"""
+    dev = require_device(distances, radius)
+    d = _aligned(f32(distances))
+    step = torch.empty((), dtype=torch.float32, device=dev)
+    ws = workspace(lib.hgc_gravnet_radius_step_workspace_bytes(), dev)
+    check(lib.hgc_gravnet_radius_step(p(d), d.numel(), p(radius), p(step), p(ws), ws.numel(), stream()))
+    return step
+
+
+@_op("gravnet_join(Tensor accumulated, Tensor features, Tensor x) -> Tensor")
+def gravnet_join(accumulated, features, x):
+    """[accumulated - (features | features) | x], the input rows of the block's last dense layer"""
+    dev = require_device(accumulated, features, x)
+    acc, feat, x = f32(accumulated), f32(features), f32(x)
+    n, f = feat.shape
+    if acc.shape != (n, 2 * f) or x.dim() != 2 or x.shape[0] != n:
+        raise ValueError("gravnet_join: [N, 2F], [N, F] and [N, X] expected")
+    out = torch.empty((n, 2 * f + x.shape[1]), dtype=torch.float32, device=dev)
+    check(lib.hgc_gravnet_join(p(acc), p(feat), p(x), n, f, x.shape[1], p(out), stream()))
+    return out
+
+
+@_op("gravnet_join_grad(Tensor grad, int n_features, bool for_accumulated, bool for_features, bool for_x) "
+     "-> (Tensor, Tensor, Tensor)")
+def gravnet_join_grad(grad, n_features, for_accumulated, for_features, for_x):
+    """gradients of gravnet_join; an empty tensor where none is wanted"""
+    dev = require_device(grad)
+    g = f32(grad)
+    n, f, w = g.shape[0], n_features, g.shape[1] - 2 * n_features
+    wanted = ((for_accumulated, 2 * f), (for_features, f), (for_x, w))
+    out = [torch.empty((n, width) if want else (0,), dtype=torch.float32, device=dev) for want, width in wanted]
+    check(lib.hgc_gravnet_join_grad(p(g), n, f, w, *(p(t) if want else None for t, (want, _) in zip(out, wanted)),
+                                    stream()))
+    return tuple(out)
+
+
+@_op("column_sums(Tensor x) -> Tensor")
+def column_sums(x):
+    """x.sum(0) of a float32 matrix"""
+    dev = require_device(x)
+    x = f32(x)
+    n, c = x.shape
+    out = torch.empty((c,), dtype=torch.float32, device=dev)
+    need = lib.hgc_column_sums_workspace_bytes(n, c)
+    ws = workspace(need, dev) if need else None
+    check(lib.hgc_column_sums(p(x), n, c, p(out), p(ws), ws.numel() if need else 0, stream()))
+    return out
+
+
 # --------------------------------------------------------------------------- shapes without data
 
 # Fake ("meta") implementations: output shapes and dtypes from input shapes alone, so that
@@ -765,3 +865,37 @@ def _(ccoords, dist, beta, no_condensation_mask, bins_flat, bin_splits, indices_
     n, nh, rows = ccoords.shape[0], beta_h.numel(), row_splits.numel() - 1
     return (_i32_like((nh,), ccoords), _i32_like((n,), ccoords), _i32_like((nh,), ccoords), _i32_like((n,), ccoords),
             _i32_like((rows + 1,), ccoords))
+
+
+@torch.library.register_fake("hgcalml::gravnet_drop_self")
+def _(indices, distances):
+    n, k = indices.shape
+    return _i32_like((n, k - 1), indices), _f32_like((n, k - 1), indices)
+
+
+@torch.library.register_fake("hgcalml::gravnet_drop_self_grad")
+def _(grad_narrow, grad_wide):
+    n, k = grad_narrow.shape
+    return _f32_like((n, k + 1), grad_narrow)
+
+
+@torch.library.register_fake("hgcalml::gravnet_radius_step")
+def _(distances, radius):
+    return _f32_like((), radius)
+
+
+@torch.library.register_fake("hgcalml::gravnet_join")
+def _(accumulated, features, x):
+    return _f32_like((x.shape[0], accumulated.shape[1] + x.shape[1]), x)
+
+
+@torch.library.register_fake("hgcalml::gravnet_join_grad")
+def _(grad, n_features, for_accumulated, for_features, for_x):
+    n, f = grad.shape[0], n_features
+    wanted = ((for_accumulated, 2 * f), (for_features, f), (for_x, grad.shape[1] - 2 * f))
+    return tuple(_f32_like((n, width) if want else (0,), grad) for want, width in wanted)
+
+
+@torch.library.register_fake("hgcalml::column_sums")
+def _(x):
+    return _f32_like((x.shape[1],), x)

@@ -544,6 +544,42 @@ int hgc_sort_distinct_keys(unsigned long long *d_keys, long long n, int value_bi
 /* Condensate assignment                                               */
 /* ------------------------------------------------------------------ */
 
+/* ---- the GravNet block around its search and accumulation
+ * (modules/GravNetLayersRagged.py:3095-3283, tensor operations there) ---- */
+
+/* Table and squared distances [n_vert, n_neigh] without column 0, the self
+ * entry: outputs [n_vert, n_neigh - 1] on 16-byte boundaries. The gradient
+ * w.r.t. the wide distances is that of the narrow ones moved up by a column
+ * plus d_grad_wide (may be NULL: 0). */
+int hgc_gravnet_drop_self(const int *d_idxs, const float *d_dist, int n_vert, int n_neigh,
+                          int *d_out_idxs, float *d_out_dist, hgc_stream_t stream);
+int hgc_gravnet_drop_self_grad(const float *d_grad_narrow, const float *d_grad_wide, int n_vert,
+                               int n_neigh, float *d_out_grad, hgc_stream_t stream);
+
+/* What update_dynamic_radius adds to the radius (GravNetLayersRagged.py:3180-3193):
+ * 0.05 (u - radius), u = max(min(1.05 largest distance, 2), 2 mean distance) + 1e-3,
+ * over `total` >= 1 squared distances (16-byte boundary). d_radius, d_step: one
+ * float each on the device. */
+size_t hgc_gravnet_radius_step_workspace_bytes(void);
+int hgc_gravnet_radius_step(const float *d_distsq, long long total, const float *d_radius,
+                            float *d_step, void *workspace, size_t workspace_bytes, hgc_stream_t stream);
+
+/* Input rows of the block's last dense layer, [n_vert, 2 n_feat + n_x]:
+ * acc[:, :n_feat] - features | acc[:, n_feat:] - features | x. The gradient goes
+ * to d_grad_acc [n_vert, 2 n_feat], d_grad_features [n_vert, n_feat] and
+ * d_grad_x [n_vert, n_x], each of which may be NULL. */
+int hgc_gravnet_join(const float *d_acc, const float *d_features, const float *d_x, int n_vert,
+                     int n_feat, int n_x, float *d_out, hgc_stream_t stream);
+int hgc_gravnet_join_grad(const float *d_grad, int n_vert, int n_feat, int n_x, float *d_grad_acc,
+                          float *d_grad_features, float *d_grad_x, hgc_stream_t stream);
+
+/* Sums over the rows of a row-major [n_rows, n_cols] matrix (bias gradients,
+ * slices of weight gradients), in a fixed order. The query returns 0 where one
+ * launch does it and a NULL workspace is accepted. */
+size_t hgc_column_sums_workspace_bytes(int n_rows, int n_cols);
+int hgc_column_sums(const float *d_x, int n_rows, int n_cols, float *d_sums, void *workspace,
+                    size_t workspace_bytes, hgc_stream_t stream);
+
 /* Greedy highest-beta-first condensate selection and hit assignment per event.
  * Replaces BinnedCondensatesFinderOpFunctor
  * (modules/compiled/binned_assign_to_condensates_kernel.h, _kernel.cc:23-241);

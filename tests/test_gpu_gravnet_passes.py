@@ -1,0 +1,92 @@
+"""The memory passes of the GravNet block against the tensor operations they stand for: equal bits where nothing is
+summed, at odd widths, single rows and the ends of workgroups; the block with the passes against the block without."""
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("n,k", [(1, 2), (3, 3), (5, 2), (127, 4), (255, 17), (1000, 65), (1025, 41)])
+def test_drop_self(n, k):
+    from hgcalml_amd import ops
+    g = torch.Generator().manual_seed(n * k)
+    idx = torch.randint(-1, n, (n, k), generator=g, dtype=torch.int32).to(DEV)
+    d = torch.rand(n, k, generator=g).to(DEV)
+    got_idx, got = ops.gravnet_drop_self(idx, d)
+    assert torch.equal(got_idx, idx[:, 1:]) and torch.equal(got, d[:, 1:])
+    narrow, wide = torch.randn(n, k - 1, generator=g).to(DEV), torch.randn(n, k, generator=g).to(DEV)
+    padded = torch.nn.functional.pad(narrow, (1, 0))
+    assert torch.equal(ops.gravnet_drop_self_grad(narrow, None), padded)
+    assert torch.equal(ops.gravnet_drop_self_grad(narrow, wide), wide + padded)
+    assert torch.equal(ops.gravnet_drop_self_grad(narrow, wide.t().contiguous().t()), wide + padded)
+    odd = torch.randn(n * k + 1, generator=g).to(DEV)[1:].view(n, k)  # not on a 16-byte boundary
+    assert torch.equal(ops.gravnet_drop_self_grad(narrow, odd), odd + padded)
+
+
+@pytest.mark.parametrize("n,f,w", [(1, 1, 1), (7, 3, 5), (64, 16, 4), (333, 22, 29), (100, 64, 64), (257, 32, 48),
+                                   (3, 300, 700), (2, 4, 4), (1000, 5, 8)])
+def test_join(n, f, w):
+    from hgcalml_amd import ops
+    g = torch.Generator().manual_seed(n + f + w)
+    acc, p, x = (torch.randn(n, c, generator=g).to(DEV) for c in (2 * f, f, w))
+    assert torch.equal(ops.gravnet_join(acc, p, x), torch.cat([acc - p.repeat(1, 2), x], dim=1))
+    grad = torch.randn(n, 2 * f + w, generator=g).to(DEV)
+    for wanted in ((True, True, True), (False, True, False), (True, False, False), (False, False, True)):
+        got = ops.gravnet_join_grad(grad, f, *wanted)
+        for a, b, want in zip(got, (grad[:, :2 * f], -grad[:, :f] - grad[:, f:2 * f], grad[:, 2 * f:]), wanted):
+            assert torch.equal(a, b) if want else a.numel() == 0
+
+
+@pytest.mark.parametrize("n,c", [(1, 1), (1, 130), (255, 7), (256, 48), (513, 1), (2477, 48), (64, 24576), (64, 4099),
+                                 (150000, 128), (70001, 33), (8192, 4), (9000, 516)])
+def test_column_sums(n, c):
+    from hgcalml_amd import ops
+    x = torch.randn(n, c, generator=torch.Generator().manual_seed(n + c))
+    want = x.double().sum(0)
+    # float32 sums: at most 1024 serial additions per column and level, of terms whose absolute sum bounds the partial sums
+    bound = 1024 * 2.0 ** -24 * x.double().abs().sum(0)
+    got = ops.column_sums(x.to(DEV)).cpu().double()
+    assert ((got - want).abs() <= bound).all()
+    shifted = torch.randn(n * c + 1, generator=torch.Generator().manual_seed(c)).to(DEV)[1:].view(n, c)
+    want = shifted.cpu().double()
+    assert ((ops.column_sums(shifted).cpu().double() - want.sum(0)).abs() <= 1024 * 2.0 ** -24 * want.abs().sum(0)).all()
+
+
+@pytest.mark.parametrize("total,high", [(1, 1.0), (2, 30.0), (1023, 0.01), (4097, 1.0), (3000001, 9.0)])
+def test_radius_step(total, high):
+    from hgcalml_amd import ops
+    d = torch.rand(total, 1, generator=torch.Generator().manual_seed(total)).to(DEV) * high
+    radius = torch.tensor(0.7, device=DEV)
+
+    def step(d, radius):
+        dist = d.double().sqrt()
+        return 0.05 * (torch.maximum((dist.max() * 1.05).clamp(max=2.0), 2.0 * dist.mean()) + 1e-3 - radius.double())
+    # a root, three products and a rounded sum in float32, each off by 2^-24 of values below 6
+    assert abs(float(ops.gravnet_radius_step(d, radius)) - float(step(d, radius))) <= 6 * 8 * 2.0 ** -24
+    d[total // 2] = float("nan")
+    assert torch.isnan(ops.gravnet_radius_step(d, radius))
+
+
+@pytest.mark.parametrize("return_self", [True, False])
+def test_block_with_and_without_the_passes(return_self, monkeypatch):
+    """same operations in the same order but for sums over rows and the order of two gradients added: 1e-5"""
+    from hgcalml_amd import GravNetLayersRagged as module
+    torch.manual_seed(5)
+    layer = module.RaggedGravNet(13, 9, 3, 30, 11, return_self=return_self).to(DEV)
+    x = torch.randn(901, 13, device=DEV)
+    rs = torch.tensor([0, 5, 400, 901], dtype=torch.int32, device=DEV)  # the first event has padded rows
+
+    def once():
+        layer.dynamic_radius.fill_(1.0)
+        xx = x.clone().requires_grad_(True)
+        out, coords, idx, dist = layer(xx, rs)
+        loss = (out * out).sum() + (dist * torch.linspace(0, 1, dist.numel(), device=DEV).view(dist.shape)).sum()
+        return [out, coords, idx, dist, layer.dynamic_radius.clone()] + list(
+            torch.autograd.grad(loss, [xx] + list(layer.parameters())))
+    fused = once()
+    monkeypatch.setattr(module, "_library_takes", lambda *tensors: False)
+    for a, b in zip(fused, once()):
+        assert a.shape == b.shape and a.dtype == b.dtype
+        assert (a.double() - b.double()).norm() <= 1e-5 * b.double().norm()
