@@ -72,6 +72,7 @@ __global__ __launch_bounds__(256) void column_minmax_kernel(const float *__restr
     __shared__ float s_lo[4][kMaxBinDims], s_hi[4][kMaxBinDims];
 #pragma unroll
     for (int c = 0; c < kMaxBinDims; ++c) {
+        if (c >= n_dims) break;
         float a = lo[c], b = hi[c];
         for (int off = 32; off > 0; off >>= 1) {
             a = fminf(a, __shfl_xor(a, off, kWave));
@@ -83,7 +84,7 @@ __global__ __launch_bounds__(256) void column_minmax_kernel(const float *__restr
         }
     }
     __syncthreads();
-    if (threadIdx.x < kMaxBinDims) {
+    if (threadIdx.x < n_dims) {
         int c = threadIdx.x;
         float a = fminf(fminf(s_lo[0][c], s_lo[1][c]), fminf(s_lo[2][c], s_lo[3][c]));
         float b = fmaxf(fmaxf(s_hi[0][c], s_hi[1][c]), fmaxf(s_hi[2][c], s_hi[3][c]));
@@ -130,6 +131,7 @@ __global__ __launch_bounds__(64) void grid_params_kernel(const float *__restrict
     float lo[kMaxBinDims], hi[kMaxBinDims];
 #pragma unroll
     for (int c = 0; c < kMaxBinDims; ++c) {
+        if (c >= n_dims) break;
         float a = FLT_MAX, b = -FLT_MAX;
         for (int i = threadIdx.x; i < n_partial; i += kWave) {
             a = fminf(a, partial[((size_t)i * 2 + 0) * kMaxBinDims + c]);
@@ -306,6 +308,74 @@ __global__ __launch_bounds__(256) void index_replacer_kernel(const int *__restri
 // counters): every block folds the column minima / maxima and derives the grid
 // itself, so there is no separate launch for that.
 
+struct PointBin {
+    int event, cell, half, flags;
+    int k[kMaxBinDims];
+};
+
+// bin of point p, flat over all events, and the half of the bin it lies in per dimension
+__device__ __forceinline__ PointBin bin_of_point(const float *coords, int stride, int p, const int *row_splits, int n_rs,
+                                                 int n_dims, const float *shift, float bw, const int *n_bins,
+                                                 int n_bins_bound) {
+    PointBin b;
+    b.half = b.flags = 0;
+    int mul = 1, cell = 0;
+#pragma unroll
+    for (int c = kMaxBinDims - 1; c >= 0; --c) {
+        if (c >= n_dims) continue;
+        const float raw = coords[(size_t)p * stride + c];
+        if (!isfinite(raw)) b.flags |= HGC_FLAG_COORDINATE_NOT_FINITE;
+        const float x = raw - shift[c];
+        const float in_bins = x / bw;
+        int k = (int)in_bins;
+        const int nb = n_bins[c];
+        if (k < 0 || k >= nb) {
+            k = 0;
+            b.flags |= HGC_FLAG_COORDINATE_OUT_OF_GRID;
+        } else if (in_bins - (float)k >= 0.5f) {
+            b.half |= 1 << (n_dims - 1 - c);  // upper half of the bin in this dimension (last dimension: bit 0)
+        }
+        b.k[c] = k;
+        cell += k * mul;
+        mul *= nb;
+    }
+    int lo = 1, hi = n_rs;  // event: number of row splits (from the second on) that are <= p
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (row_splits[mid] > p)
+            hi = mid;
+        else
+            lo = mid + 1;
+    }
+    b.event = lo - 1;
+    cell += b.event * mul;
+    b.cell = min(cell, n_bins_bound - 1);  // no effect for row splits that end at n_vert
+    return b;
+}
+
+__device__ __forceinline__ void store_bin_row(int *binass, size_t row, int n_dims, const PointBin &b) {
+    if (n_dims == 3) {  // one 16-byte row (the arrays are aligned)
+        reinterpret_cast<int4 *>(binass)[row] = make_int4(b.event, b.k[0], b.k[1], b.k[2]);
+    } else {
+        binass[row * (n_dims + 1)] = b.event;
+#pragma unroll
+        for (int c = 0; c < kMaxBinDims; ++c)
+            if (c < n_dims) binass[row * (n_dims + 1) + c + 1] = b.k[c];
+    }
+}
+
+__device__ __forceinline__ void copy_coords_row(const float *coords, int from, float *out, int to, int n_coords,
+                                                int rows_aligned) {
+    if (n_coords == 4 && rows_aligned) {
+        reinterpret_cast<float4 *>(out)[to] = reinterpret_cast<const float4 *>(coords)[from];
+    } else if (n_coords == 3) {  // one 12-byte store per row instead of three of 4 bytes to a scattered address
+        struct __attribute__((packed, aligned(4))) Row3 { float v[3]; };
+        reinterpret_cast<Row3 *>(out)[to] = reinterpret_cast<const Row3 *>(coords)[from];
+    } else {
+        for (int c = 0; c < n_coords; ++c) out[(size_t)to * n_coords + c] = coords[(size_t)from * n_coords + c];
+    }
+}
+
 __global__ __launch_bounds__(256) void bin_points_ranked_kernel(
     const float *__restrict__ coords, int stride, const float *__restrict__ partial, int n_partial,
     const int *__restrict__ row_splits, int n_vert, int n_dims, int n_rs, int n_bins_scalar,
@@ -317,6 +387,7 @@ __global__ __launch_bounds__(256) void bin_points_ranked_kernel(
     __shared__ int s_nb[kMaxBinDims];
 #pragma unroll
     for (int c = 0; c < kMaxBinDims; ++c) {
+        if (c >= n_dims) break;
         float a = FLT_MAX, b = -FLT_MAX;
         for (int i = threadIdx.x; i < n_partial; i += blockDim.x) {
             a = fminf(a, partial[((size_t)i * 2 + 0) * kMaxBinDims + c]);
@@ -334,7 +405,7 @@ __global__ __launch_bounds__(256) void bin_points_ranked_kernel(
     __syncthreads();
     if (threadIdx.x == 0) {
         float lo[kMaxBinDims], hi[kMaxBinDims];
-        for (int c = 0; c < kMaxBinDims; ++c) {
+        for (int c = 0; c < n_dims; ++c) {
             lo[c] = fminf(fminf(s_lo[0][c], s_lo[1][c]), fminf(s_lo[2][c], s_lo[3][c]));
             hi[c] = fmaxf(fmaxf(s_hi[0][c], s_hi[1][c]), fmaxf(s_hi[2][c], s_hi[3][c]));
         }
@@ -350,51 +421,135 @@ __global__ __launch_bounds__(256) void bin_points_ranked_kernel(
     __syncthreads();
     const float bw = s_bw;
     for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n_vert; p += gridDim.x * blockDim.x) {
-        int mul = 1, cell = 0, flags = 0, half = 0;
-        int ks[kMaxBinDims];
-        for (int c = n_dims - 1; c >= 0; --c) {
-            const float raw = coords[(size_t)p * stride + c];
-            if (!isfinite(raw)) flags |= HGC_FLAG_COORDINATE_NOT_FINITE;
-            const float x = raw - s_shift[c];
-            const float in_bins = x / bw;
-            int k = (int)in_bins;
-            const int nb = s_nb[c];
-            if (k < 0 || k >= nb) {
-                k = 0;
-                flags |= HGC_FLAG_COORDINATE_OUT_OF_GRID;
-            } else if (in_bins - (float)k >= 0.5f) {
-                half |= 1 << (n_dims - 1 - c);  // upper half of the bin in this dimension (last dimension: bit 0)
-            }
-            ks[c] = k;
-            cell += k * mul;
-            mul *= nb;
-        }
-        int lo = 1, hi = n_rs;  // event: number of row splits (from the second on) that are <= p
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (row_splits[mid] > p)
-                hi = mid;
-            else
-                lo = mid + 1;
-        }
-        const int ev = lo - 1;
-        cell += ev * mul;
-        if (flags && status) atomicOr(status, flags);
-        cell = min(cell, n_bins_bound - 1);  // no effect for row splits that end at n_vert
-        if (n_dims == 3) {  // one 16-byte row (the workspace is aligned)
-            reinterpret_cast<int4 *>(binass)[p] = make_int4(ev, ks[0], ks[1], ks[2]);
-        } else {
-            binass[(size_t)p * (n_dims + 1)] = ev;
-            for (int c = 0; c < n_dims; ++c) binass[(size_t)p * (n_dims + 1) + c + 1] = ks[c];
-        }
+        const PointBin b = bin_of_point(coords, stride, p, row_splits, n_rs, n_dims, s_shift, bw, s_nb, n_bins_bound);
+        if (b.flags && status) atomicOr(status, b.flags);
+        store_bin_row(binass, p, n_dims, b);
         // Every bin has 2^sub_shift counters, so that the increments of a crowded bin queue up on
         // several addresses instead of one. spatial (sub_shift = n_dims): the counter is the half of
         // the bin the point lies in, per dimension -- the bin's points then come grouped by these
         // 2^n_dims sub-cells, a grid of half the bin width nested in the bins, and the flat index
         // names the sub-cell. Otherwise a point takes the counter its index names.
-        const int counter = (cell << sub_shift) | (spatial ? half : (p & ((1 << sub_shift) - 1)));
-        flat[p] = spatial ? counter : cell;
+        const int counter = (b.cell << sub_shift) | (spatial ? b.half : (p & ((1 << sub_shift) - 1)));
+        flat[p] = spatial ? counter : b.cell;
         rank[p] = atomicAdd(&counts[counter], 1);
+    }
+}
+
+// All of the grouping by one workgroup, for a few thousand points whose counters fit into its LDS: bounding box, grid,
+// bins, counters (16 bits each, two in a word; a bin's rank in it is the order of arrival), their prefix sums and the move
+// into bin order, with barriers where the general path has launches. A point's bin and rank stay in its thread's registers.
+// Bound by latencies: seven barriers' worth of LDS and L2 round trips, 9 us for 700 points where the five launches took 23
+// (a call of BinnedSelectKnn 36.7 -> 24.5 us). Beyond 2048 points one compute unit has too much to write where the nested
+// grid has its 10^4 cells: a call with 4 dimensions and K = 64 takes 47 us against 53 in five launches at 2000 points, 59
+// against 56 at 3000 and 76 against 65 at 4096.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallItems = 2;
+constexpr int kSmallPoints = kSmallThreads * kSmallItems;
+constexpr int kSmallWords = 16384;  // pairs of counters
+
+__global__ __launch_bounds__(kSmallThreads) void group_small_kernel(
+    const float *__restrict__ coords, int n_coords, const int *__restrict__ direction, const int *__restrict__ row_splits,
+    int n_vert, int n_dims, int n_rs, int n_bins_scalar, int n_bins_bound, int spatial, int rows_aligned,
+    float *__restrict__ shift_out, float *__restrict__ bin_width_out, int *__restrict__ n_bins_out,
+    int *__restrict__ boundaries, int *__restrict__ bin_starts, int *__restrict__ sorting, float *__restrict__ scoords,
+    int *__restrict__ sflat, int *__restrict__ sbinass, int *__restrict__ sdir, int *__restrict__ status) {
+    constexpr int waves = kSmallThreads / kWave;
+    __shared__ uint32_t s_count[kSmallWords];
+    __shared__ float s_lo[waves][kMaxBinDims], s_hi[waves][kMaxBinDims];
+    __shared__ float s_shift[kMaxBinDims], s_bw;
+    __shared__ int s_nb[kMaxBinDims], s_wave[waves];
+    const int tid = threadIdx.x, wave = tid / kWave;
+    const int bits = spatial ? n_dims : 0;
+    const int n_counters = (n_bins_bound << bits) + 1;
+    const int n_words = (n_counters + 1) / 2;
+    for (int w = tid; w < n_words; w += kSmallThreads) s_count[w] = 0;
+    {
+        float lo[kMaxBinDims], hi[kMaxBinDims];
+#pragma unroll
+        for (int c = 0; c < kMaxBinDims; ++c) lo[c] = FLT_MAX, hi[c] = -FLT_MAX;
+#pragma unroll
+        for (int u = 0; u < kSmallItems; ++u) {
+            const int p = u * kSmallThreads + tid;
+#pragma unroll
+            for (int c = 0; c < kMaxBinDims; ++c)
+                if (c < n_dims && p < n_vert) {
+                    const float x = coords[(size_t)p * n_coords + c];
+                    lo[c] = fminf(lo[c], x);
+                    hi[c] = fmaxf(hi[c], x);
+                }
+        }
+#pragma unroll
+        for (int c = 0; c < kMaxBinDims; ++c) {
+            if (c >= n_dims) break;
+            float a = lo[c], b = hi[c];
+            for (int off = 32; off > 0; off >>= 1) {
+                a = fminf(a, __shfl_xor(a, off, kWave));
+                b = fmaxf(b, __shfl_xor(b, off, kWave));
+            }
+            if (lane_id() == 0) s_lo[wave][c] = a, s_hi[wave][c] = b;
+        }
+    }
+    __syncthreads();
+    if (tid == 0) {
+        float lo[kMaxBinDims], hi[kMaxBinDims];
+        for (int c = 0; c < n_dims; ++c) {
+            lo[c] = s_lo[0][c], hi[c] = s_hi[0][c];
+            for (int w = 1; w < waves; ++w) lo[c] = fminf(lo[c], s_lo[w][c]), hi[c] = fmaxf(hi[c], s_hi[w][c]);
+        }
+        derive_grid(lo, hi, n_dims, 0, n_bins_scalar, nullptr, s_shift, &s_bw, s_nb);
+        for (int c = 0; c < n_dims; ++c) {
+            shift_out[c] = s_shift[c];
+            n_bins_out[c] = s_nb[c];
+        }
+        bin_width_out[0] = s_bw;
+    }
+    __syncthreads();
+    const float bw = s_bw;
+    PointBin bin[kSmallItems];
+    int rank[kSmallItems];
+#pragma unroll
+    for (int u = 0; u < kSmallItems; ++u) {
+        const int p = u * kSmallThreads + tid;
+        if (p >= n_vert) continue;
+        bin[u] = bin_of_point(coords, n_coords, p, row_splits, n_rs, n_dims, s_shift, bw, s_nb, n_bins_bound);
+        if (bin[u].flags && status) atomicOr(status, bin[u].flags);
+        if (spatial) bin[u].cell = (bin[u].cell << bits) | bin[u].half;
+        const int half_word = (bin[u].cell & 1) * 16;
+        rank[u] = (int)((atomicAdd(&s_count[bin[u].cell >> 1], 1u << half_word) >> half_word) & 0xffffu);
+    }
+    __syncthreads();
+    {   // counts to exclusive prefix sums, in place (n_vert fits into 16 bits); a thread owns a run of words
+        const int per = (n_words + kSmallThreads - 1) / kSmallThreads;
+        const int first = tid * per, last = min(n_words, first + per);
+        int own = 0;
+        for (int w = first; w < last; ++w) own += (int)(s_count[w] & 0xffffu) + (int)(s_count[w] >> 16);
+        const int upto = wave_inclusive_sum(own);
+        if (lane_id() == kWave - 1) s_wave[wave] = upto;
+        __syncthreads();
+        int at = upto - own;
+        for (int w = 0; w < wave; ++w) at += s_wave[w];
+        for (int w = first; w < last; ++w) {
+            const uint32_t pair = s_count[w];
+            const int mid = at + (int)(pair & 0xffffu);
+            s_count[w] = (uint32_t)at | ((uint32_t)mid << 16);
+            at = mid + (int)(pair >> 16);
+        }
+    }
+    __syncthreads();
+    auto prefix = [&](int counter) { return (int)((s_count[counter >> 1] >> ((counter & 1) * 16)) & 0xffffu); };
+    if (spatial)
+        for (int i = tid; i < n_counters; i += kSmallThreads) boundaries[i] = prefix(i);
+    for (int i = tid; i <= n_bins_bound; i += kSmallThreads) bin_starts[i] = prefix(i << bits);
+#pragma unroll
+    for (int u = 0; u < kSmallItems; ++u) {
+        const int p = u * kSmallThreads + tid;
+        if (p >= n_vert) continue;
+        const int at = prefix(bin[u].cell) + rank[u];
+        sorting[at] = p;
+        sflat[at] = bin[u].cell;
+        copy_coords_row(coords, p, scoords, at, n_coords, rows_aligned);
+        store_bin_row(sbinass, at, n_dims, bin[u]);
+        if (direction) sdir[at] = direction[p];
     }
 }
 
@@ -411,14 +566,7 @@ __global__ __launch_bounds__(256) void move_to_bin_order_kernel(
     const int at = boundaries[spatial ? (size_t)cell : ((size_t)cell << sub_shift) | (p & ((1 << sub_shift) - 1))] + rank[p];
     sorting[at] = p;
     sflat[at] = cell;
-    if (n_coords == 4 && rows_aligned) {
-        reinterpret_cast<float4 *>(scoords)[at] = reinterpret_cast<const float4 *>(coords)[p];
-    } else if (n_coords == 3) {  // one 12-byte store per row instead of three of 4 bytes to a scattered address
-        struct __attribute__((packed, aligned(4))) Row3 { float v[3]; };
-        reinterpret_cast<Row3 *>(scoords)[at] = reinterpret_cast<const Row3 *>(coords)[p];
-    } else {
-        for (int c = 0; c < n_coords; ++c) scoords[(size_t)at * n_coords + c] = coords[(size_t)p * n_coords + c];
-    }
+    copy_coords_row(coords, p, scoords, at, n_coords, rows_aligned);
     if (n_dims == 3) {
         reinterpret_cast<int4 *>(sbinass)[at] = reinterpret_cast<const int4 *>(binass)[p];
     } else {
@@ -537,9 +685,13 @@ int launch_fill_i32(int *p, int value, long long n, hipStream_t s) {
 }
 
 
-// few blocks fold the bounding box (every binning block reads all their partial
-// results again), many assign the bins
-static int grouping_blocks(int n_vert) { return std::max(1, std::min(128, ceil_div(n_vert, 1024))); }
+// the blocks that fold the bounding box: every binning block reads all their partial results again
+static int grouping_blocks(int n_vert) { return std::max(1, std::min(128, ceil_div(n_vert, 256))); }
+
+// the whole grouping in one workgroup (see group_small_kernel)
+static bool grouping_is_small(int n_vert, int n_bins_bound, int n_bin_dims, bool spatial) {
+    return n_vert <= kSmallPoints && ((size_t)n_bins_bound << (spatial ? n_bin_dims : 0)) + 2 <= 2 * (size_t)kSmallWords;
+}
 
 bool bin_grouping_spatial(int n_bins_bound, int n_bin_dims) {
     return n_bin_dims >= 2 && n_bin_dims <= 4 && (((size_t)n_bins_bound << n_bin_dims) + 1) <= ((size_t)1 << 22);
@@ -585,6 +737,15 @@ int bin_grouping(const float *d_coords, const int *d_row_splits, const int *d_di
     if (!workspace || !aligned256(workspace) ||
         workspace_bytes < bin_grouping_workspace_bytes(n_vert, n_bins_bound, n_bin_dims, spatial))
         return fail(HGC_ERR_WORKSPACE, "bin grouping workspace missing, misaligned or too small");
+    const int rows_aligned =
+        ((reinterpret_cast<uintptr_t>(d_coords) | reinterpret_cast<uintptr_t>(d_scoords)) & 15u) == 0;
+    if (d_bin_starts && grouping_is_small(n_vert, n_bins_bound, n_bin_dims, spatial)) {
+        group_small_kernel<<<1, kSmallThreads, 0, s>>>(d_coords, n_coords, d_direction, d_row_splits, n_vert, n_bin_dims,
+                                                       n_rs, n_bins_scalar, n_bins_bound, spatial ? 1 : 0, rows_aligned,
+                                                       d_shift, d_bin_width, d_n_bins, d_boundaries, d_bin_starts,
+                                                       d_sorting, d_scoords, d_sflat, d_sbinass, d_sdir, status_word());
+        return check_launch("group_small");
+    }
     const int blocks = grouping_blocks(n_vert);
     Carver carve(workspace);
     float *partial = carve.take<float>((size_t)blocks * 2 * kMaxBinDims);
@@ -623,8 +784,6 @@ int bin_grouping(const float *d_coords, const int *d_row_splits, const int *d_di
         rc = check_launch("bin boundary table");
     }
     if (rc) return rc;
-    const int rows_aligned =
-        ((reinterpret_cast<uintptr_t>(d_coords) | reinterpret_cast<uintptr_t>(d_scoords)) & 15u) == 0;
     move_to_bin_order_kernel<<<ceil_div(n_vert, 256), 256, 0, s>>>(d_coords, binass, flat, rank, d_direction,
                                                                    d_boundaries, n_vert, n_coords, n_bin_dims,
                                                                    sub_shift, spatial ? 1 : 0, rows_aligned, d_sorting,

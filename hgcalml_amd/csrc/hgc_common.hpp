@@ -92,6 +92,7 @@ int sample_sort_values(uint64_t *d_keys, uint64_t *d_spare, long long n, int val
 // every table entry is the boundary of such a sub-cell, and d_sflat holds sub-cell indices
 // (bin << n_bin_dims | bits) instead of bin indices.
 // d_bin_starts (may be null): n_bins_bound + 1 entries, the boundary of every bin without a stride.
+// A few thousand points with d_bin_starts take one launch, which writes d_boundaries only if spatial.
 bool bin_grouping_spatial(int n_bins_bound, int n_bin_dims);
 int bin_grouping_sub_shift(int n_bins_bound, int n_bin_dims, bool spatial);
 size_t bin_grouping_workspace_bytes(int n_vert, int n_bins_bound, int n_bin_dims, bool spatial);
