@@ -62,6 +62,7 @@ _SIGNATURES = {
     "hgc_push_knn": (_c_int, [_ptr] * 6 + [_c_int] * 3 + [_ptr]),
     "hgc_push_knn_ordered": (_c_int, [_ptr] * 7 + [_c_int] * 3 + [_ptr]),
     "hgc_push_knn_grad": (_c_int, [_ptr] * 6 + [_c_int] * 3 + [_ptr]),
+    "hgc_push_knn_grad_ordered": (_c_int, [_ptr] * 7 + [_c_int] * 3 + [_ptr]),
     "hgc_exp_neg": (_c_int, [_ptr, _ptr, ctypes.c_longlong, _ptr]),
     "hgc_exp_neg_grad": (_c_int, [_ptr, _ptr, _ptr, ctypes.c_longlong, _ptr]),
     "hgc_gravnet_drop_self": (_c_int, [_ptr] * 2 + [_c_int] * 2 + [_ptr] * 3),

@@ -54,25 +54,6 @@ struct GradRows {
     bool negate;  // gw receives -(gradient * w): the chain rule through w = exp(-d)
 };
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_from(float v) {
-    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
-}
-
-// sums of val[0..3] over the group's 16 lanes (fixed order): lane l receives that of val[l >> 2]
-__device__ __forceinline__ float group_sum_4(const float (&val)[4], int lane) {
-    const bool upper8 = (lane & 8) != 0, upper4 = (lane & 4) != 0;
-    const float a = (upper8 ? val[2] : val[0]) + dpp_from<0x128>(upper8 ? val[0] : val[2]);  // row_ror:8, lane ^ 8
-    const float b = (upper8 ? val[3] : val[1]) + dpp_from<0x128>(upper8 ? val[1] : val[3]);
-    float r = (upper4 ? b : a) + dpp_from<0x141>(upper4 ? a : b);  // row_half_mirror, lane ^ 7
-    r = r + dpp_from<0x1b>(r);                                     // quad_perm [3,2,1,0], lane ^ 3
-    return r + dpp_from<0xb1>(r);                                  // quad_perm [1,0,3,2], lane ^ 1
-}
-
-// Entry e of a chunk of 16 sits in lane entry_lane(e) of its group (4 x 4 transposed): that is the lane
-// that ends up with the entry's dot product. The map is its own inverse.
-constexpr int entry_lane(int e) { return 4 * (e & 3) + (e >> 2); }
-
 // Does byte E of `packed` equal `key`? One SDWA compare.
 template <int E>
 __device__ __forceinline__ uint64_t byte_is(uint32_t packed, uint32_t key) {

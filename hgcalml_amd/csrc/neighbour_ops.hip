@@ -57,102 +57,123 @@ __global__ __launch_bounds__(256) void local_distance_kernel(const int *__restri
     dist[t] = dsq;
 }
 
-// Gradient of push_knn, both outputs from one gather: a wave owns vertex v,
-// fetches the upstream gradient rows of its K neighbours once and forms
+// Gradient of push_knn, both outputs from one gather: a group of 16 lanes owns vertex v, fetches the
+// upstream gradient rows of its K neighbours once and forms
 //   feat_grad[v, f] = sum_n grad[idx[v,n], f] * w[v,n]   (serial, slot order: the reference's sum)
 //   w_grad[v, n]    = sum_f grad[idx[v,n], f] * feat[v, f]
-// the second as per-lane partial dot products that a fixed transpose-butterfly
-// reduces for 32 slots at a time. Lane l owns features [l*VEC, l*VEC+VEC) of each
-// of the NB blocks of 64*VEC features.
+// the second as dot products per lane that a fixed exchange over the group adds up, four slots at a
+// time. Lane l owns the VEC features from l*VEC on of each of the NB blocks of 16*VEC (rows of up to
+// 256 features). Index and weight of 16 slots sit one per lane, slot s in lane entry_lane(s), which is
+// the lane that ends up with the slot's dot product. Bound by vector issue like the accumulation's
+// forward pass. On kNN tables (3-D Gaussian, processed in bin order) against one wave per vertex, or two
+// separate passes where 64 does not divide the columns: 60,000 vertices, K = 24, F = 48 97 -> 23 us;
+// 150,000, K = 64, F = 64 356 -> 125; 300,000, K = 64, F = 128 1346 -> 547; 200,000, K = 40, F = 256
+// 1169 -> 477 (on tables that need no order 65 -> 21, 322 -> 123, 700 -> 527, 498 -> 438).
 template <int VEC, int NB>
-__global__ __launch_bounds__(256) void push_grad_wave_kernel(const float *__restrict__ grad, const float *__restrict__ w,
+__global__ __launch_bounds__(256) void push_grad_rows_kernel(const float *__restrict__ grad, const float *__restrict__ w,
                                                              const float *__restrict__ feat, const int *__restrict__ idx,
-                                                             float *__restrict__ feat_grad, float *__restrict__ w_grad,
-                                                             int n_vert, int K, int F) {
+                                                             const int *__restrict__ order, float *__restrict__ feat_grad,
+                                                             float *__restrict__ w_grad, int n_vert, int K, int F) {
     using namespace acc;
-    constexpr int G = 32;  // slots per reduction
-    constexpr int U = 8;   // gathered rows in flight
-    const int v = wave_vertex(nullptr, n_vert);
-    if (v >= n_vert) return;
-    const int lane = lane_id();
+    const int lane = lane_id(), l = lane & (kRowLanes - 1);
+    const GroupTask task = group_task(order, n_vert, 1);
+    const bool live = task.vertex >= 0;
+    const int v = live ? task.vertex : 0;
     const int *irow = idx + (size_t)v * K;
     const float *wrow = w + (size_t)v * K;
-    const RowMatrix X(grad, n_vert, F);
+    const __amdgpu_buffer_rsrc_t rows = make_rows(grad, (unsigned long long)n_vert * F * 4ull);
+    // A lane at the end of a row that is no multiple of VEC takes the last VEC columns; those it shares with its
+    // neighbour count in the neighbour's dot product only.
     uint32_t lane_bytes[NB];
     float own[NB][VEC], sum[NB][VEC];
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-        const int fb = (b * kWave + lane) * VEC;
-        lane_bytes[b] = (uint32_t)fb * 4u;
-        load_vec<VEC>(feat + (size_t)v * F + fb, own[b]);
+        const int fb = (b * kRowLanes + l) * VEC, f = min(fb, F - VEC);
+        lane_bytes[b] = (uint32_t)f * 4u;
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) sum[b][e] = 0.f;
-    }
-    for (int l0 = 0; l0 < K; l0 += G) {
-        float val[G];
-#pragma unroll
-        for (int i = 0; i < G; ++i) val[i] = 0.f;
-#pragma unroll
-        for (int u0 = 0; u0 < G; u0 += U) {
-            if (l0 + u0 >= K) break;  // wave-uniform
-            int j[U];
-            float wl[U];
-            float x[U][NB][VEC];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int l = min(l0 + u0 + u, K - 1);
-                j[u] = l0 + u0 + u < K ? irow[l] : -1;
-                wl[u] = wrow[l];
-            }
-            // slots without a neighbour read row 0 and are left out of the sum; their
-            // weight gradient is overwritten with 0 below
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int b = 0; b < NB; ++b)
-                    X.load<VEC>((uint32_t)j[u] < (uint32_t)n_vert ? j[u] : 0, lane_bytes[b], x[u][b]);
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const bool valid = (uint32_t)j[u] < (uint32_t)n_vert;  // wave-uniform
-#pragma unroll
-                for (int b = 0; b < NB; ++b)
-#pragma unroll
-                    for (int e = 0; e < VEC; ++e) {
-                        val[u0 + u] = __builtin_fmaf(own[b][e], x[u][b][e], val[u0 + u]);
-                        if (valid) sum[b][e] = sum[b][e] + x[u][b][e] * wl[u];
-                    }
-            }
+        for (int e = 0; e < VEC; ++e) {
+            const float x = feat[(size_t)v * F + f + e];
+            own[b][e] = f + e >= fb ? x : 0.f;
+            sum[b][e] = 0.f;
         }
-        const float r = transpose_reduce_32(val);  // lane L: slot l0 + (L & 31)
-        const int l = l0 + lane;
-        if (lane < G && l < K) w_grad[(size_t)v * K + l] = (uint32_t)irow[l] < (uint32_t)n_vert ? r : 0.f;
     }
+    const int mine = entry_lane(l);
+    bool in_row = live && mine < K;
+    int j_next = in_row ? irow[mine] : -1;
+    float w_next = in_row ? wrow[mine] : 0.f;
+    for (int c0 = 0; c0 < K; c0 += kRowLanes) {
+        const bool store = in_row;
+        const bool has_row = (uint32_t)j_next < (uint32_t)n_vert;
+        const uint32_t offset = has_row ? (uint32_t)j_next * (uint32_t)(F * 4) : kNoRow;  // no row: 0 is read ...
+        const float wn = has_row ? w_next : 0.f;                                           // ... and adds 0
+        in_row = live && c0 + kRowLanes + mine < K;
+        j_next = in_row ? irow[c0 + kRowLanes + mine] : -1;
+        w_next = in_row ? wrow[c0 + kRowLanes + mine] : 0.f;
+        float r[4] = {};
+#define HGC_PUSH_SLOT(Q, U)                                                                                  \
+    {                                                                                                        \
+        const uint32_t row = group_bcast<entry_lane((Q) * 4 + (U))>(offset);                                 \
+        _Pragma("unroll") for (int b = 0; b < NB; ++b) load_cols<VEC>(rows, row + lane_bytes[b], x[U][b]);    \
+        ws[U] = group_bcast<entry_lane((Q) * 4 + (U))>(wn);                                                  \
+    }
+#define HGC_PUSH_FOUR(Q)                                                                                     \
+    if (c0 + (Q) * 4 < K) {                                                                                  \
+        float x[4][NB][VEC], ws[4], val[4];                                                                  \
+        HGC_PUSH_SLOT(Q, 0)                                                                                  \
+        HGC_PUSH_SLOT(Q, 1)                                                                                  \
+        HGC_PUSH_SLOT(Q, 2)                                                                                  \
+        HGC_PUSH_SLOT(Q, 3)                                                                                  \
+        _Pragma("unroll") for (int u = 0; u < 4; ++u) {                                                      \
+            val[u] = 0.f;                                                                                    \
+            _Pragma("unroll") for (int b = 0; b < NB; ++b) _Pragma("unroll") for (int e = 0; e < VEC; ++e) { \
+                val[u] = __builtin_fmaf(own[b][e], x[u][b][e], val[u]);                                      \
+                sum[b][e] = sum[b][e] + x[u][b][e] * ws[u];                                                  \
+            }                                                                                                \
+        }                                                                                                    \
+        r[Q] = group_sum_4(val, lane);                                                                       \
+    }
+        HGC_PUSH_FOUR(0)
+        HGC_PUSH_FOUR(1)
+        HGC_PUSH_FOUR(2)
+        HGC_PUSH_FOUR(3)
+#undef HGC_PUSH_FOUR
+#undef HGC_PUSH_SLOT
+        // lane l holds the sums of slot 4 q + (l >> 2) in r[q]; its own slot has q = l & 3
+        const float dot = (l & 2) ? ((l & 1) ? r[3] : r[2]) : ((l & 1) ? r[1] : r[0]);
+        if (store) w_grad[(size_t)v * K + c0 + mine] = has_row ? dot : 0.f;
+    }
+    if (!live) return;
 #pragma unroll
-    for (int b = 0; b < NB; ++b) store_vec<VEC>(feat_grad + (size_t)v * F + (lane_bytes[b] >> 2), sum[b]);
+    for (int b = 0; b < NB; ++b)
+        if ((b * kRowLanes + l) * VEC < F) store_cols<VEC>(feat_grad + (size_t)v * F + (lane_bytes[b] >> 2), sum[b]);
 }
 
 // returns 1 when the shape is not covered
-int launch_push_grad_wave(const float *grad, const float *w, const float *feat, const int *idx, float *feat_grad,
-                          float *w_grad, int n_vert, int K, int F, hipStream_t s) {
+int launch_push_grad_rows(const float *grad, const float *w, const float *feat, const int *idx, const int *order,
+                          float *feat_grad, float *w_grad, int n_vert, int K, int F, hipStream_t s) {
     using namespace acc;
-    if (F % kWave != 0 || (unsigned long long)n_vert * (unsigned long long)F * 4ull >= (1ull << 32)) return 1;
-    const uintptr_t align_or = reinterpret_cast<uintptr_t>(grad) | reinterpret_cast<uintptr_t>(feat) |
-                               reinterpret_cast<uintptr_t>(feat_grad);
-    const int vec = wave_vec(F, align_or);
-    const int nb = F / (kWave * vec);
-    const dim3 grid(ceil_div(n_vert, 4)), block(256);
-#define HGC_PUSH_GRAD(VEC, NB) \
-    push_grad_wave_kernel<VEC, NB><<<grid, block, 0, s>>>(grad, w, feat, idx, feat_grad, w_grad, n_vert, K, F)
+    if (F > 256 || (unsigned long long)n_vert * (unsigned long long)F * 4ull > kMaxRowBytes) return 1;
+    int vec, nb;
+    row_shape(F, vec, nb);
+    const dim3 grid(ceil_div(n_vert, 256 / kRowLanes)), block(256);
+#define HGC_PUSH_GRAD(VEC, NB)                                                                                         \
+    case VEC * 10 + NB:                                                                                                \
+        push_grad_rows_kernel<VEC, NB><<<grid, block, 0, s>>>(grad, w, feat, idx, order, feat_grad, w_grad, n_vert, K, F); \
+        break
     switch (vec * 10 + nb) {
-        case 11: HGC_PUSH_GRAD(1, 1); break;
-        case 12: HGC_PUSH_GRAD(1, 2); break;
-        case 13: HGC_PUSH_GRAD(1, 3); break;
-        case 21: HGC_PUSH_GRAD(2, 1); break;
-        case 41: HGC_PUSH_GRAD(4, 1); break;
+        HGC_PUSH_GRAD(1, 1);
+        HGC_PUSH_GRAD(2, 1);
+        HGC_PUSH_GRAD(3, 1);
+        HGC_PUSH_GRAD(4, 1);
+        HGC_PUSH_GRAD(3, 2);
+        HGC_PUSH_GRAD(4, 2);
+        HGC_PUSH_GRAD(3, 3);
+        HGC_PUSH_GRAD(4, 3);
+        HGC_PUSH_GRAD(4, 4);
         default: return 1;
     }
 #undef HGC_PUSH_GRAD
-    return check_launch("push_grad_wave_kernel");
+    return check_launch("push_grad_rows_kernel");
 }
 
 }  // namespace
@@ -205,6 +226,27 @@ __global__ __launch_bounds__(256) void exp_neg_grad_kernel(const float *gw, cons
 
 __device__ __forceinline__ float divide_no_nan(float a, float b) { return b == 0.f ? 0.f : a / b; }
 
+// Both kernels walk the slots four at a time, indices and weights one step ahead, so that a step's gathers are under
+// way together (one slot after the other: 40,000 vertices, K = 32, F = 8, C = 4 74 us for both, now 65). What bounds them is the L1's
+// address rate: index, weight and coordinates are the same for the lanes of a vertex. Workgroups of one XCD take consecutive vertices of the processing order.
+constexpr int kMomentSlots = 4;
+
+struct SlotStep {
+    int j[kMomentSlots];  // -1: no neighbour
+    float w[kMomentSlots];
+};
+
+__device__ __forceinline__ void fetch_slots(const int *irow, const float *wrow, int n0, int n_neigh, int n_vert,
+                                            SlotStep &step) {
+#pragma unroll
+    for (int u = 0; u < kMomentSlots; ++u) {
+        const int n = min(n0 + u, n_neigh - 1);
+        const int j = irow[n];
+        step.j[u] = n0 + u < n_neigh && (unsigned)j < (unsigned)n_vert ? j : -1;
+        step.w[u] = wrow[n];
+    }
+}
+
 template <int C>
 __global__ __launch_bounds__(256) void neighbour_means_kernel(const float *__restrict__ coords,
                                                               const float *__restrict__ weights,
@@ -212,24 +254,38 @@ __global__ __launch_bounds__(256) void neighbour_means_kernel(const float *__res
                                                               float *__restrict__ sumw, float *__restrict__ means,
                                                               const int *__restrict__ order, int n_vert, int n_feat,
                                                               int n_neigh) {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long t = (long long)xcd_contiguous_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     const int i = (int)(t / n_feat);
     if (i >= n_vert) return;
     const int f = (int)(t - (long long)i * n_feat);
     const int v = order ? order[i] : i;  // processing order with locality: results do not depend on it
     if ((unsigned)v >= (unsigned)n_vert) return;
     const float kf = (float)n_neigh;
+    const int *irow = idx + (size_t)v * n_neigh;
+    const float *wrow = weights + (size_t)v * n_neigh;
     float s = 0.f, sc[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) sc[c] = 0.f;
-    for (int n = 0; n < n_neigh; ++n) {
-        const int j = idx[(size_t)v * n_neigh + n];
-        if ((unsigned)j >= (unsigned)n_vert) continue;
-        const float w = weights[(size_t)v * n_neigh + n];
-        const float a = feats[(size_t)j * n_feat + f];
-        s = s + a * w;
+    SlotStep next;
+    fetch_slots(irow, wrow, 0, n_neigh, n_vert, next);
+    for (int n0 = 0; n0 < n_neigh; n0 += kMomentSlots) {
+        const SlotStep now = next;
+        float a[kMomentSlots], x[kMomentSlots][C];
 #pragma unroll
-        for (int c = 0; c < C; ++c) sc[c] = sc[c] + (coords[(size_t)j * C + c] * a) * w;
+        for (int u = 0; u < kMomentSlots; ++u) {
+            const size_t j = max(now.j[u], 0);
+            a[u] = feats[j * n_feat + f];
+#pragma unroll
+            for (int c = 0; c < C; ++c) x[u][c] = coords[j * C + c];
+        }
+        if (n0 + kMomentSlots < n_neigh) fetch_slots(irow, wrow, n0 + kMomentSlots, n_neigh, n_vert, next);
+#pragma unroll
+        for (int u = 0; u < kMomentSlots; ++u) {
+            if (now.j[u] < 0) continue;
+            s = s + a[u] * now.w[u];
+#pragma unroll
+            for (int c = 0; c < C; ++c) sc[c] = sc[c] + (x[u][c] * a[u]) * now.w[u];
+        }
     }
     const float S = (s / kf) * kf;
     sumw[(size_t)v * n_feat + f] = S;
@@ -246,30 +302,41 @@ __global__ __launch_bounds__(256) void neighbour_covariance_kernel(const float *
                                                                    const float *__restrict__ means, float *__restrict__ cov,
                                                                    const int *__restrict__ order, int n_vert, int n_feat,
                                                                    int n_neigh) {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long long t = (long long)xcd_contiguous_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     const int i = (int)(t / n_feat);
     if (i >= n_vert) return;
     const int f = (int)(t - (long long)i * n_feat);
     const int v = order ? order[i] : i;
     if ((unsigned)v >= (unsigned)n_vert) return;
     const float kf = (float)n_neigh;
+    const int *irow = idx + (size_t)v * n_neigh;
+    const float *wrow = weights + (size_t)v * n_neigh;
     float acc[C][C];  // the lower triangle is accumulated, the products are symmetric bit for bit
 #pragma unroll
     for (int c = 0; c < C; ++c)
 #pragma unroll
         for (int d = 0; d < C; ++d) acc[c][d] = 0.f;
-    for (int n = 0; n < n_neigh; ++n) {
-        const int j = idx[(size_t)v * n_neigh + n];
-        if ((unsigned)j >= (unsigned)n_vert) continue;
-        const float w = weights[(size_t)v * n_neigh + n];
-        const float a = feats[(size_t)j * n_feat + f];
-        float cen[C];
+    SlotStep next;
+    fetch_slots(irow, wrow, 0, n_neigh, n_vert, next);
+    for (int n0 = 0; n0 < n_neigh; n0 += kMomentSlots) {
+        const SlotStep now = next;
+        float a[kMomentSlots], cen[kMomentSlots][C];
 #pragma unroll
-        for (int c = 0; c < C; ++c) cen[c] = coords[(size_t)j * C + c] - means[((size_t)j * n_feat + f) * C + c];
+        for (int u = 0; u < kMomentSlots; ++u) {
+            const size_t j = max(now.j[u], 0);
+            a[u] = feats[j * n_feat + f];
 #pragma unroll
-        for (int c = 0; c < C; ++c)
+            for (int c = 0; c < C; ++c) cen[u][c] = coords[j * C + c] - means[(j * n_feat + f) * C + c];
+        }
+        if (n0 + kMomentSlots < n_neigh) fetch_slots(irow, wrow, n0 + kMomentSlots, n_neigh, n_vert, next);
 #pragma unroll
-            for (int d = 0; d <= c; ++d) acc[c][d] = acc[c][d] + ((cen[c] * cen[d]) * a) * w;
+        for (int u = 0; u < kMomentSlots; ++u) {
+            if (now.j[u] < 0) continue;
+#pragma unroll
+            for (int c = 0; c < C; ++c)
+#pragma unroll
+                for (int d = 0; d <= c; ++d) acc[c][d] = acc[c][d] + ((cen[u][c] * cen[u][d]) * a[u]) * now.w[u];
+        }
     }
     const float den = sumw[(size_t)v * n_feat + f] + 1e-3f;
     float *out = cov + ((size_t)v * n_feat + f) * C * C;
@@ -361,8 +428,9 @@ int hgc_push_knn(const float *d_weights, const float *d_feat, const int *d_idxs,
                                 n_neigh, n_feat, stream);
 }
 
-int hgc_push_knn_grad(const float *d_grad, const float *d_weights, const float *d_feat, const int *d_idxs,
-                      float *d_feat_grad, float *d_w_grad, int n_vert, int n_neigh, int n_feat, hgc_stream_t stream) {
+int hgc_push_knn_grad_ordered(const float *d_grad, const float *d_weights, const float *d_feat, const int *d_idxs,
+                              const int *d_vertex_order, float *d_feat_grad, float *d_w_grad, int n_vert, int n_neigh,
+                              int n_feat, hgc_stream_t stream) {
     HGC_REQUIRE(n_vert <= 0 || (d_feat_grad && d_w_grad), "null pointer");
     HGC_REQUIRE(n_vert >= 0 && n_neigh >= 1 && n_feat >= 1, "bad sizes");
     HGC_REQUIRE((long long)n_vert * n_neigh < (1ll << 31), "n_vert * n_neigh must stay below 2^31");
@@ -370,18 +438,24 @@ int hgc_push_knn_grad(const float *d_grad, const float *d_weights, const float *
     HGC_REQUIRE(d_grad && d_weights && d_feat && d_idxs, "null pointer");
     {
         // both gradients from one gather pass where that kernel covers the shape
-        const int rc = launch_push_grad_wave(d_grad, d_weights, d_feat, d_idxs, d_feat_grad, d_w_grad, n_vert, n_neigh,
-                                             n_feat, as_stream(stream));
+        const int rc = launch_push_grad_rows(d_grad, d_weights, d_feat, d_idxs, d_vertex_order, d_feat_grad, d_w_grad,
+                                             n_vert, n_neigh, n_feat, as_stream(stream));
         if (rc <= 0) return rc;
     }
     // feat_grad[v, f] = sum_n grad[idx[v,n], f] * w[v,n]: the mean-only forward over `grad`, not divided by K
     int rc = accumulate_forward(d_weights, d_grad, d_idxs, d_feat_grad, nullptr, nullptr, n_vert, n_neigh, n_feat,
-                                n_feat, 0, 1.f, nullptr, nullptr, stream);
+                                n_feat, 0, 1.f, d_vertex_order, nullptr, stream);
     if (rc) return rc;
     // w_grad[v, n] = sum_f grad[idx[v,n], f] * feat[v, f]: the weight gradient with the roles of the
     // vertex's own row (feat) and the gathered rows (grad) as in the accumulation's
     return accumulate_gradient(d_feat, nullptr, d_grad, nullptr, nullptr, d_idxs, nullptr, nullptr, d_w_grad, nullptr,
                                n_vert, n_neigh, n_feat, n_feat, 0, 1.f, nullptr, nullptr, 0, false, nullptr, 0, stream);
+}
+
+int hgc_push_knn_grad(const float *d_grad, const float *d_weights, const float *d_feat, const int *d_idxs,
+                      float *d_feat_grad, float *d_w_grad, int n_vert, int n_neigh, int n_feat, hgc_stream_t stream) {
+    return hgc_push_knn_grad_ordered(d_grad, d_weights, d_feat, d_idxs, nullptr, d_feat_grad, d_w_grad, n_vert, n_neigh,
+                                     n_feat, stream);
 }
 
 int hgc_exp_neg(const float *d_distances, float *d_weights, long long n_values, hgc_stream_t stream) {

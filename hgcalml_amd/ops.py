@@ -554,7 +554,8 @@ def push_knn_grad(grad: torch.Tensor, weights: torch.Tensor, features: torch.Ten
     n, k = idx.shape
     wgrad = torch.empty_like(w)
     fgrad = torch.empty_like(x)
-    check(lib.hgc_push_knn_grad(p(g), p(w), p(x), p(idx), p(fgrad), p(wgrad), n, k, x.shape[1], stream()))
+    check(lib.hgc_push_knn_grad_ordered(p(g), p(w), p(x), p(idx), p(vertex_order_of(indices)), p(fgrad), p(wgrad), n, k,
+                                        x.shape[1], stream()))
     return wgrad, fgrad
 
 
