@@ -129,13 +129,13 @@ def require_device(*tensors):
 
 def p(t):
     """device pointer of a (contiguous) tensor, or NULL"""
-    if t is None:
-        return None
-    return ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """handle of torch's current stream on the current device. (The stream object that torch.cuda.current_stream()
+    makes costs 5 us a call, as much as a launch: a training step of the GravNet block asks 13 times.)"""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def workspace(nbytes, device):
