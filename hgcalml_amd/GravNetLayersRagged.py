@@ -13,7 +13,7 @@ from torch import nn
 
 from . import globals as gl
 from . import ops
-from .accknn_op import AccumulateKnn, AccumulateKnnSumw
+from .accknn_op import AccumulateKnn, AccumulateKnnSumw, _AccumulateSumwFn
 from .binned_select_knn_op import BinnedSelectKnn
 
 
@@ -184,6 +184,8 @@ class RaggedGravNet(nn.Module):
         return nidx, ndist, None, None
 
     def collect_neighbours(self, features, neighbour_indices, distancesq):
+        if self.sumwnorm and _library_takes(distancesq, features):
+            return _AccumulateSumwFn.apply(10.0 * distancesq, features, neighbour_indices)
         acc = AccumulateKnnSumw if self.sumwnorm else AccumulateKnn
         f, _ = acc(10.0 * distancesq, features, neighbour_indices, mean_and_max=True)
         return f

@@ -71,6 +71,9 @@ _SIGNATURES = {
     "hgc_gravnet_radius_step": (_c_int, [_ptr, ctypes.c_longlong] + [_ptr] * 3 + [_c_size, _ptr]),
     "hgc_gravnet_join": (_c_int, [_ptr] * 3 + [_c_int] * 3 + [_ptr] * 2),
     "hgc_gravnet_join_grad": (_c_int, [_ptr] + [_c_int] * 3 + [_ptr] * 4),
+    "hgc_sumw_normalise": (_c_int, [_ptr] * 2 + [_c_int] * 3 + [_ptr] * 3),
+    "hgc_sumw_grad": (_c_int, [_ptr] * 3 + [_c_int] * 3 + [_ptr] * 3),
+    "hgc_sumw_distance_grad": (_c_int, [_ptr] * 3 + [_c_int] * 2 + [_ptr] * 2),
     "hgc_column_sums_workspace_bytes": (_c_size, [_c_int] * 2),
     "hgc_column_sums": (_c_int, [_ptr] + [_c_int] * 2 + [_ptr] * 2 + [_c_size, _ptr]),
     "hgc_binned_assign_to_condensates_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int]),

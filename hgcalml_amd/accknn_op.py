@@ -59,6 +59,41 @@ class _AccumulateExpFn(torch.autograd.Function):
         return gd, gx, None, None
 
 
+class _AccumulateSumwFn(torch.autograd.Function):
+    """what AccumulateKnnSumw(distances, features, indices, mean_and_max=True) returns first, without the column of
+    ones: the weights' sum is taken from the weights"""
+
+    @staticmethod
+    def forward(ctx, distances, features, indices):
+        out, maxidx, slots, weights = torch.ops.hgcalml.accumulate_knn_exp_slots(distances, features, indices, 0, True)
+        idx = ops.i32(indices)
+        norm = ops.sumw_normalise(weights, idx, out)
+        ctx.save_for_backward(weights, features, indices, maxidx, slots, out, norm)
+        ctx.indices_ref = indices
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        weights, features, indices, maxidx, slots, out, norm = ctx.saved_tensors
+        k, f = indices.shape[1], features.shape[1]
+        if torch.is_grad_enabled():
+            # differentiable up to the accumulation's gradient, which says itself that it has none
+            empty = (norm == 0)[:, None]
+            over = torch.where(empty, torch.zeros_like(grad_out[:, :f]),
+                               grad_out[:, :f] / torch.where(empty, torch.ones_like(norm)[:, None], norm[:, None]))
+            g_acc, g_norm = torch.cat([over, grad_out[:, f:]], dim=1), -(over * out[:, :f]).sum(1) / k
+        else:
+            g_acc, g_norm = ops.sumw_grad(grad_out, out, norm, k)
+        inv_off, inv_slots = ops.cached_inverse_neighbour_index(ctx.indices_ref)
+        gd, gx = torch.ops.hgcalml.accumulate_knn_grad_exp_slots(g_acc, weights, features, indices, maxidx, slots, inv_off,
+                                                                 inv_slots)
+        if torch.is_grad_enabled():
+            gd = gd - torch.where(indices < 0, torch.zeros_like(weights), g_norm[:, None] * weights)
+        else:
+            ops.sumw_distance_grad(g_norm, weights, ops.i32(indices), gd)
+        return gd, gx, None
+
+
 class _ExpNegFn(torch.autograd.Function):
     """weights = exp(-distances) (modules/accknn_op.py:52) and its chain rule, one kernel each"""
 

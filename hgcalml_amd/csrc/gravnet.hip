@@ -3,13 +3,13 @@
 // the dynamic radius, the row [mean - p | max - p | x] that the last dense layer reads, and sums over the rows for the
 // gradients of the dense layers. All of them stream; as single tensor operations they were 40 launches and, at 150k
 // vertices, K = 64, F = 64, 0.6 of the 2.45 ms of a training step, most of it intermediates written and read again; the
-// step takes 2.19 ms with these (240k vertices, K = 40, F = 32 with the weights' sum: 2.97 -> 2.72). What is left of them
+// step takes 2.19 ms with these (240k vertices, K = 40, F = 32 with the weights' sum: 2.97 -> 2.27). What is left of them
 // runs at 4 to 5 TB/s: at 150k vertices 36 us each for the join and its gradient (115 and 154 MB), the table and its
 // gradient, 13 us for the radius.
 #include <algorithm>
 #include <cmath>
 
-#include "hgc_common.hpp"
+#include "accumulate_rows.hpp"
 
 namespace hgc {
 namespace {
@@ -211,6 +211,104 @@ __global__ __launch_bounds__(kThreads) void join_rows_grad_kernel(const float *_
     }
 }
 
+// ---- mean over the weights' sum instead of the number of slots ------------------------------------------------------
+//
+// AccumulateKnnSumw (modules/GravNetLayersRagged.py:35-62) sends a column of ones through the accumulation and divides by
+// what arrives there: the sum of the weights over the slots, divided by K. The sum needs the weights only, so here the
+// features keep their own width (33 columns instead of 32 cost the accumulation 75 us forward and 155 us backward of 240,000
+// vertices with K = 40) and three streaming passes do the rest. Same bits forward; backward the sum's share
+// of a weight's gradient is added after the dot product instead of inside it.
+
+constexpr int kGroup = acc::kRowLanes;  // lanes per vertex
+
+template <int U>
+__device__ __forceinline__ void add_slots(float mine, float &sum) {
+    if constexpr (U < kGroup) {
+        sum = sum + acc::group_bcast<U>(mine);
+        add_slots<U + 1>(mine, sum);
+    }
+}
+
+// norm[v] = (sum of the weights, slot after slot) / K; the mean columns of `out` [n, 2F] divided by it (0 where it is 0)
+__global__ __launch_bounds__(kThreads) void sumw_normalise_kernel(const float *__restrict__ weights,
+                                                                  const int *__restrict__ idx, int n, int K, int F, float kf,
+                                                                  float *__restrict__ out, float *__restrict__ norm) {
+    const int v = blockIdx.x * (kThreads / kGroup) + threadIdx.x / kGroup, l = threadIdx.x % kGroup;
+    const bool live = v < n;
+    float sum = 0.f;
+    for (int c0 = 0; c0 < K; c0 += kGroup) {
+        const size_t at = (size_t)v * K + c0 + l;
+        const bool in_row = live && c0 + l < K;
+        const bool has = in_row && (uint32_t)idx[in_row ? at : 0] < (uint32_t)n;
+        add_slots<0>(has ? weights[at] : 0.f, sum);  // a sum from +0 on: adding 0 changes nothing
+    }
+    if (!live) return;
+    const float d = sum / kf;
+    if (l == 0) norm[v] = d;
+    float *row = out + (size_t)v * 2 * F;
+    for (int c = l; c < F; c += kGroup) row[c] = d == 0.f ? 0.f : row[c] / d;
+}
+
+// From the gradient g [n, 2F] of the normalised rows: that of the accumulation's rows, and 1/K of that of norm
+__global__ __launch_bounds__(kThreads) void sumw_grad_kernel(const float *__restrict__ g, const float *__restrict__ out,
+                                                             const float *__restrict__ norm, int n, int F, float kf,
+                                                             float *__restrict__ g_acc, float *__restrict__ g_norm) {
+    const int v = blockIdx.x * (kThreads / kGroup) + threadIdx.x / kGroup, l = threadIdx.x % kGroup;
+    if (v >= n) return;
+    const float d = norm[v];
+    const size_t row = (size_t)v * 2 * F;
+    float part = 0.f;
+    for (int c = l; c < F; c += kGroup) {
+        const float gm = g[row + c], gx = g[row + F + c], mean = out[row + c];
+        if (d != 0.f) part = part - gm * (mean / d);
+        g_acc[row + c] = d == 0.f ? 0.f : gm / d;
+        g_acc[row + F + c] = gx;
+    }
+    part += acc::dpp_from<0x128>(part);  // over the 16 lanes: ror 8, 4, 2, 1
+    part += acc::dpp_from<0x124>(part);
+    part += acc::dpp_from<0x122>(part);
+    part += acc::dpp_from<0x121>(part);
+    if (l == 0) g_norm[v] = part / kf;
+}
+
+// the weights' sum in the gradient of the distances, w = exp(-d): g_dist -= g_norm * w where there is a neighbour
+__global__ __launch_bounds__(kThreads) void sumw_distance_grad_kernel(const float *__restrict__ g_norm,
+                                                                      const float *__restrict__ weights,
+                                                                      const int *__restrict__ idx, unsigned total,
+                                                                      unsigned K, unsigned n, float *__restrict__ g_dist) {
+    const unsigned first = (blockIdx.x * kThreads + threadIdx.x) * 4u;
+    if (first >= total) return;
+    unsigned row = first / K, col = first - row * K;
+    const unsigned count = min(4u, total - first);
+    float w[4], g[4];
+    int j[4];
+    if (count == 4) {
+        const float4 a = *reinterpret_cast<const float4 *>(weights + first), b = *reinterpret_cast<float4 *>(g_dist + first);
+        const int4 c = *reinterpret_cast<const int4 *>(idx + first);
+        w[0] = a.x, w[1] = a.y, w[2] = a.z, w[3] = a.w;
+        g[0] = b.x, g[1] = b.y, g[2] = b.z, g[3] = b.w;
+        j[0] = c.x, j[1] = c.y, j[2] = c.z, j[3] = c.w;
+    } else {
+#pragma unroll
+        for (unsigned u = 0; u < 4; ++u) {
+            const unsigned at = min(first + u, total - 1);
+            w[u] = weights[at], g[u] = g_dist[at], j[u] = idx[at];
+        }
+    }
+#pragma unroll
+    for (unsigned u = 0; u < 4; ++u) {
+        if (u < count && (unsigned)j[u] < n) g[u] = g[u] - g_norm[row] * w[u];
+        if (++col == K) col = 0, ++row;
+    }
+    if (count == 4) {
+        *reinterpret_cast<float4 *>(g_dist + first) = float4{g[0], g[1], g[2], g[3]};
+    } else {
+#pragma unroll
+        for (unsigned u = 0; u < 3; ++u)
+            if (u < count) g_dist[first + u] = g[u];
+    }
+}
+
 // ---- sums over the rows -------------------------------------------------------------------------------------------
 
 // Columns are cut into tiles of `tile` vectors (grid.y), rows into grid.x slabs; a thread adds its columns of every
@@ -372,6 +470,39 @@ int hgc_gravnet_join_grad(const float *d_grad, int n_vert, int n_feat, int n_x, 
         join_rows_grad_kernel<1><<<grid, kThreads, 0, as_stream(stream)>>>(d_grad, n_vert, rows, f, w, d_grad_acc,
                                                                           d_grad_features, d_grad_x);
     return check_launch("gravnet_join_grad");
+}
+
+int hgc_sumw_normalise(const float *d_weights, const int *d_idxs, int n_vert, int n_neigh, int n_feat, float *d_out_feat,
+                       float *d_norm, hgc_stream_t stream) {
+    HGC_REQUIRE(n_vert >= 0 && n_neigh >= 1 && n_feat >= 1, "bad sizes");
+    if (n_vert == 0) return HGC_OK;
+    HGC_REQUIRE(d_weights && d_idxs && d_out_feat && d_norm, "null pointer");
+    sumw_normalise_kernel<<<ceil_div(n_vert, kThreads / kGroup), kThreads, 0, as_stream(stream)>>>(
+        d_weights, d_idxs, n_vert, n_neigh, n_feat, (float)n_neigh, d_out_feat, d_norm);
+    return check_launch("sumw_normalise");
+}
+
+int hgc_sumw_grad(const float *d_grad, const float *d_out_feat, const float *d_norm, int n_vert, int n_neigh, int n_feat,
+                  float *d_grad_accumulated, float *d_grad_norm, hgc_stream_t stream) {
+    HGC_REQUIRE(n_vert >= 0 && n_neigh >= 1 && n_feat >= 1, "bad sizes");
+    if (n_vert == 0) return HGC_OK;
+    HGC_REQUIRE(d_grad && d_out_feat && d_norm && d_grad_accumulated && d_grad_norm, "null pointer");
+    sumw_grad_kernel<<<ceil_div(n_vert, kThreads / kGroup), kThreads, 0, as_stream(stream)>>>(
+        d_grad, d_out_feat, d_norm, n_vert, n_feat, (float)n_neigh, d_grad_accumulated, d_grad_norm);
+    return check_launch("sumw_grad");
+}
+
+int hgc_sumw_distance_grad(const float *d_grad_norm, const float *d_weights, const int *d_idxs, int n_vert, int n_neigh,
+                           float *d_grad_distances, hgc_stream_t stream) {
+    HGC_REQUIRE(n_vert >= 0 && n_neigh >= 1, "bad sizes");
+    HGC_REQUIRE((long long)n_vert * n_neigh < (1ll << 31) - 4, "n_vert * n_neigh must stay below 2^31");
+    if (n_vert == 0) return HGC_OK;
+    HGC_REQUIRE(d_grad_norm && d_weights && d_idxs && d_grad_distances, "null pointer");
+    HGC_REQUIRE(aligned16({d_weights, d_idxs, d_grad_distances}), "arrays must lie on 16-byte boundaries");
+    const unsigned total = (unsigned)n_vert * (unsigned)n_neigh;
+    sumw_distance_grad_kernel<<<ceil_div(total, 4 * kThreads), kThreads, 0, as_stream(stream)>>>(
+        d_grad_norm, d_weights, d_idxs, total, (unsigned)n_neigh, (unsigned)n_vert, d_grad_distances);
+    return check_launch("sumw_distance_grad");
 }
 
 size_t hgc_column_sums_workspace_bytes(int n_rows, int n_cols) {

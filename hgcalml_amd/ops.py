@@ -748,6 +748,36 @@ def gravnet_join_grad(grad, n_features, for_accumulated, for_features, for_x):
     return tuple(out)
 
 
+@_op("sumw_normalise(Tensor weights, Tensor indices, Tensor(a!) accumulated) -> Tensor")
+def sumw_normalise(weights, indices, accumulated):
+    """mean half of the accumulation's rows over the weights' sum, in place; returns that sum / K"""
+    dev = require_device(weights, indices, accumulated)
+    n, k = indices.shape
+    norm = torch.empty((n,), dtype=torch.float32, device=dev)
+    check(lib.hgc_sumw_normalise(p(weights), p(indices), n, k, accumulated.shape[1] // 2, p(accumulated), p(norm),
+                                 stream()))
+    return norm
+
+
+@_op("sumw_grad(Tensor grad, Tensor normalised, Tensor norm, int n_neighbours) -> (Tensor, Tensor)")
+def sumw_grad(grad, normalised, norm, n_neighbours):
+    """gradients w.r.t. the accumulation's rows and (divided by K) the weights' sum"""
+    dev = require_device(grad, normalised, norm)
+    g = f32(grad)
+    g_acc, g_norm = torch.empty_like(g), torch.empty_like(norm)
+    check(lib.hgc_sumw_grad(p(g), p(normalised), p(norm), g.shape[0], n_neighbours, g.shape[1] // 2, p(g_acc), p(g_norm),
+                            stream()))
+    return g_acc, g_norm
+
+
+@_op("sumw_distance_grad(Tensor norm_grad, Tensor weights, Tensor indices, Tensor(a!) distance_grad) -> ()")
+def sumw_distance_grad(norm_grad, weights, indices, distance_grad):
+    """the weights' sum's share of the distances' gradient, added in place"""
+    require_device(norm_grad, weights, indices, distance_grad)
+    w, idx = _aligned(weights), _aligned(indices)
+    check(lib.hgc_sumw_distance_grad(p(norm_grad), p(w), p(idx), idx.shape[0], idx.shape[1], p(distance_grad), stream()))
+
+
 @_op("column_sums(Tensor x) -> Tensor")
 def column_sums(x):
     """x.sum(0) of a float32 matrix"""
@@ -900,3 +930,18 @@ def _(grad, n_features, for_accumulated, for_features, for_x):
 @torch.library.register_fake("hgcalml::column_sums")
 def _(x):
     return _f32_like((x.shape[1],), x)
+
+
+@torch.library.register_fake("hgcalml::sumw_normalise")
+def _(weights, indices, accumulated):
+    return _f32_like((indices.shape[0],), accumulated)
+
+
+@torch.library.register_fake("hgcalml::sumw_grad")
+def _(grad, normalised, norm, n_neighbours):
+    return _f32_like(grad.shape, grad), _f32_like(norm.shape, norm)
+
+
+@torch.library.register_fake("hgcalml::sumw_distance_grad")
+def _(norm_grad, weights, indices, distance_grad):
+    return None

@@ -579,6 +579,23 @@ int hgc_gravnet_join(const float *d_acc, const float *d_features, const float *d
 int hgc_gravnet_join_grad(const float *d_grad, int n_vert, int n_feat, int n_x, float *d_grad_acc,
                           float *d_grad_features, float *d_grad_x, hgc_stream_t stream);
 
+/* AccumulateKnnSumw (modules/GravNetLayersRagged.py:35-62) without its column
+ * of ones, around hgc_accumulate_knn_exp_slots with mean and maximum:
+ * d_norm[v] = (sum over the slots with a neighbour of d_weights[v,n]) / n_neigh;
+ * the mean half of d_out_feat [n_vert, 2 n_feat] is divided by it in place (0
+ * where it is 0). Backward: hgc_sumw_grad turns the gradient of the normalised
+ * rows into that of the accumulation's rows and d_grad_norm [n_vert] = 1/n_neigh of that
+ * of d_norm; hgc_sumw_distance_grad subtracts d_grad_norm[v] * d_weights[v,n] from
+ * the distance gradient of every slot with a neighbour (arrays [n_vert, n_neigh]
+ * on 16-byte boundaries). */
+int hgc_sumw_normalise(const float *d_weights, const int *d_idxs, int n_vert, int n_neigh, int n_feat,
+                       float *d_out_feat, float *d_norm, hgc_stream_t stream);
+int hgc_sumw_grad(const float *d_grad, const float *d_out_feat, const float *d_norm, int n_vert,
+                  int n_neigh, int n_feat, float *d_grad_accumulated, float *d_grad_norm,
+                  hgc_stream_t stream);
+int hgc_sumw_distance_grad(const float *d_grad_norm, const float *d_weights, const int *d_idxs,
+                           int n_vert, int n_neigh, float *d_grad_distances, hgc_stream_t stream);
+
 /* Sums over the rows of a row-major [n_rows, n_cols] matrix (bias gradients,
  * slices of weight gradients), in a fixed order. The query returns 0 where one
  * launch does it and a NULL workspace is accepted. */

@@ -69,12 +69,12 @@ def test_radius_step(total, high):
     assert torch.isnan(ops.gravnet_radius_step(d, radius))
 
 
-@pytest.mark.parametrize("return_self", [True, False])
-def test_block_with_and_without_the_passes(return_self, monkeypatch):
+@pytest.mark.parametrize("return_self,sumw", [(True, False), (False, False), (True, True)])
+def test_block_with_and_without_the_passes(return_self, sumw, monkeypatch):
     """same operations in the same order but for sums over rows and the order of two gradients added: 1e-5"""
     from hgcalml_amd import GravNetLayersRagged as module
     torch.manual_seed(5)
-    layer = module.RaggedGravNet(13, 9, 3, 30, 11, return_self=return_self).to(DEV)
+    layer = module.RaggedGravNet(13, 9, 3, 30, 11, return_self=return_self, sumwnorm=sumw).to(DEV)
     x = torch.randn(901, 13, device=DEV)
     rs = torch.tensor([0, 5, 400, 901], dtype=torch.int32, device=DEV)  # the first event has padded rows
 
@@ -90,3 +90,26 @@ def test_block_with_and_without_the_passes(return_self, monkeypatch):
     for a, b in zip(fused, once()):
         assert a.shape == b.shape and a.dtype == b.dtype
         assert (a.double() - b.double()).norm() <= 1e-5 * b.double().norm()
+
+
+@pytest.mark.parametrize("n,k,f", [(1, 1, 1), (17, 5, 3), (33, 16, 15), (100, 17, 32), (64, 40, 33), (90, 70, 130)])
+def test_weights_sum(n, k, f):
+    """against the composition with a column of ones: equal bits forward; backward the order of a sum of 2 f + 1 products and
+    the rounding of 1 / norm differ"""
+    from hgcalml_amd import AccumulateKnnSumw
+    from hgcalml_amd.accknn_op import _AccumulateSumwFn
+    g = torch.Generator().manual_seed(n + k + f)
+    idx = torch.rand(n, n, generator=g).argsort(1)[:, :k].to(torch.int32)   # different neighbours in each row
+    idx[torch.rand(n, generator=g) < 0.2, k // 2:] = -1
+    idx[0] = -1                                      # a row without neighbours: 0, and no gradient
+    idx = idx.to(DEV)
+    d = torch.rand(n, k, generator=g).to(DEV).requires_grad_(True)
+    x = torch.randn(n, f, generator=g).to(DEV).requires_grad_(True)
+    grad = torch.randn(n, 2 * f, generator=g).to(DEV)
+    want = AccumulateKnnSumw(d, x, idx, mean_and_max=True)[0]
+    got = _AccumulateSumwFn.apply(d, x, idx)
+    assert torch.equal(got, want)
+    for a, b in zip(torch.autograd.grad(got, [d, x], grad), torch.autograd.grad(want, [d, x], grad)):
+        assert torch.isfinite(a).all()
+        assert (a - b).norm() <= 1e-5 * b.norm() + 1e-30
+    assert (torch.autograd.grad(_AccumulateSumwFn.apply(d, x, idx), d, grad)[0][idx < 0] == 0).all()
