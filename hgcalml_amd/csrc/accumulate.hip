@@ -578,6 +578,71 @@ __global__ __launch_bounds__(256) void drop_first_column_kernel(const int *__res
     }
 }
 
+// The slots without a neighbour, which both indices list behind the last target: those of columns 1.. move up in
+// order. Parts of `part` entries of that tail (its length is only known on the device; parts beyond it are empty): counts
+// of what stays, their prefix sums, the move.
+__global__ __launch_bounds__(256) void tail_counts_kernel(const int *__restrict__ inv_off,
+                                                          const int *__restrict__ inv_slots, int n_vert,
+                                                          long long total, int part, const acc::FastDiv div_k, int K,
+                                                          int *__restrict__ counts) {
+    __shared__ int s_count;
+    if (threadIdx.x == 0) s_count = 0;
+    __syncthreads();
+    const long long begin = inv_off[n_vert] + (long long)blockIdx.x * part, end = min(begin + part, total);
+    int count = 0;
+    for (long long e = begin + threadIdx.x; e - lane_id() < end; e += blockDim.x) {
+        const int slot = e < end ? inv_slots[e] : 0;
+        count += __popcll(__ballot(slot - acc::fast_div(slot, div_k) * K != 0));
+    }
+    if (lane_id() == 0 && count) atomicAdd(&s_count, count);
+    __syncthreads();
+    if (threadIdx.x == 0) counts[blockIdx.x] = s_count;
+}
+
+__global__ __launch_bounds__(1024) void tail_scan_kernel(int *__restrict__ counts, int n_parts) {
+    __shared__ int s_wave[16];
+    int run = 0;
+    for (int base = 0; base < n_parts; base += 1024) {
+        const int i = base + threadIdx.x;
+        const int mine = i < n_parts ? counts[i] : 0;
+        const int upto = wave_inclusive_sum(mine);
+        if (lane_id() == kWave - 1) s_wave[threadIdx.x / kWave] = upto;
+        __syncthreads();
+        int before = run + upto - mine;
+        for (int w = 0; w < 16; ++w) {
+            if (w < (int)(threadIdx.x / kWave)) before += s_wave[w];
+            run += s_wave[w];
+        }
+        if (i < n_parts) counts[i] = before;
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(256) void tail_move_kernel(const int *__restrict__ inv_off,
+                                                        const int *__restrict__ inv_slots, int n_vert, long long total,
+                                                        int part, const acc::FastDiv div_k, int K,
+                                                        const int *__restrict__ before, const int *__restrict__ out_off,
+                                                        int *__restrict__ out_slots) {
+    __shared__ int s_kept[4];
+    const long long begin = inv_off[n_vert] + (long long)blockIdx.x * part, end = min(begin + part, total);
+    int at = out_off[n_vert] + before[blockIdx.x];
+    for (long long e0 = begin; e0 < end; e0 += blockDim.x) {
+        const long long e = e0 + threadIdx.x;
+        const int slot = e < end ? inv_slots[e] : 0;
+        const int v = acc::fast_div(slot, div_k), n = slot - v * K;
+        const uint64_t kept = __ballot(n != 0);
+        if (lane_id() == 0) s_kept[threadIdx.x / kWave] = __popcll(kept);
+        __syncthreads();
+        int mine = at;
+        for (int w = 0; w < 4; ++w) {
+            if (w < (int)(threadIdx.x / kWave)) mine += s_kept[w];
+            at += s_kept[w];
+        }
+        if (n != 0) out_slots[mine + __popcll(kept & ((1ull << lane_id()) - 1ull))] = v * (K - 1) + n - 1;
+        __syncthreads();
+    }
+}
+
 // ------------------------------------------------------------------ feature gradient
 
 // gfeat[m, f] = sum over (v, n) naming m, ascending, of ((g[v,f]/K)*w[v,n] + max part)
@@ -887,7 +952,15 @@ int hgc_inverse_index_without_first_column(const int *d_inv_offsets, const int *
                                     rocprim::plus<int>(), s));
     drop_first_column_kernel<<<blocks, 256, 0, s>>>(d_inv_offsets, d_inv_slots, dropped_before, n_vert, div_k,
                                                     n_neigh, d_out_offsets, d_out_slots);
-    return check_launch("drop_first_column");
+    if ((rc = check_launch("drop_first_column"))) return rc;
+    // the parts' counts take the place of the targets': no more than n_vert + 1 parts
+    const long long total = (long long)n_vert * n_neigh;
+    const int part = std::max(4096, (n_neigh + 255) / 256 * 256), n_parts = ceil_div(total, part);
+    tail_counts_kernel<<<n_parts, 256, 0, s>>>(d_inv_offsets, d_inv_slots, n_vert, total, part, div_k, n_neigh, dropped);
+    tail_scan_kernel<<<1, 1024, 0, s>>>(dropped, n_parts);
+    tail_move_kernel<<<n_parts, 256, 0, s>>>(d_inv_offsets, d_inv_slots, n_vert, total, part, div_k, n_neigh, dropped,
+                                             d_out_offsets, d_out_slots);
+    return check_launch("inverse index tail");
 }
 
 }  // extern "C"
