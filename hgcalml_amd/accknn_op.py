@@ -53,7 +53,8 @@ class _AccumulateExpFn(torch.autograd.Function):
         if grad_out is None:
             return None, None, None, None
         weights, features, indices, maxidx, slots = ctx.saved_tensors
-        inv_off, inv_slots = ops.cached_inverse_neighbour_index(ctx.indices_ref)
+        inv_off, inv_slots = ops.accumulate_gradient_index(ctx.indices_ref, features.shape[1],
+                                                           grad_out.shape[1] > features.shape[1])
         gd, gx = torch.ops.hgcalml.accumulate_knn_grad_exp_slots(grad_out.contiguous(), weights, features, indices,
                                                                  maxidx, slots, inv_off, inv_slots)
         return gd, gx, None, None
@@ -84,7 +85,7 @@ class _AccumulateSumwFn(torch.autograd.Function):
             g_acc, g_norm = torch.cat([over, grad_out[:, f:]], dim=1), -(over * out[:, :f]).sum(1) / k
         else:
             g_acc, g_norm = ops.sumw_grad(grad_out, out, norm, k)
-        inv_off, inv_slots = ops.cached_inverse_neighbour_index(ctx.indices_ref)
+        inv_off, inv_slots = ops.accumulate_gradient_index(ctx.indices_ref, f, True)
         gd, gx = torch.ops.hgcalml.accumulate_knn_grad_exp_slots(g_acc, weights, features, indices, maxidx, slots, inv_off,
                                                                  inv_slots)
         if torch.is_grad_enabled():

@@ -39,7 +39,7 @@ size_t accumulate_grad_rows_scratch_bytes(int n_vert, int n_feat, int g_cols, fl
 bool accumulate_grad_rows_covers(int n_feat, int n_neigh, bool mean_and_max, bool slots, unsigned long long g_bytes);
 int launch_accumulate_grad_rows(const float *g, const float *w, const float *feat, const unsigned char *maxslot,
                                 const int *inv_off, const int *inv_slots, float *gw, float *gfeat, int n_vert, int K, int F,
-                                int g_cols, bool mean_and_max, const int *order, float divisor, bool negate, void *scratch,
+                                int g_cols, bool mean_and_max, const int *order, float divisor, bool negate, int skip, void *scratch,
                                 size_t scratch_bytes, hipStream_t s);
 // accumulate_grad_records.hip: both gradients with the max part read from per-slot
 // records built in `records`; returns 1 when the shape is not covered or the storage is
@@ -1017,8 +1017,7 @@ int accumulate_gradient(const float *d_grad_from_out_features, const float *d_di
     if (want_f && (want_w || !mean_and_max)) {
         const int rc = launch_accumulate_grad_rows(d_grad_from_out_features, d_distances, d_feat, d_max_slots, d_inv_offsets,
                                                    d_inv_slots, d_out_grad_distances, d_out_grad_features, n_vert, n_neigh,
-                                                   n_feat, n_grad_from_out_feat, mean_and_max != 0, d_order, divisor, negate,
-                                                   scratch, scratch_bytes, s);
+                                                   n_feat, n_grad_from_out_feat, mean_and_max != 0, d_order, divisor, negate, 0, scratch, scratch_bytes, s);
         if (rc <= 0) return rc;
     }
     if (fits_32bit && want_f && (want_w || !mean_and_max)) {
@@ -1162,6 +1161,30 @@ int hgc_accumulate_knn_grad_scratch(const float *d_grad_from_out_features, const
                                d_neigh_indices, d_inv_offsets, d_inv_slots, d_out_grad_distances, d_out_grad_features,
                                n_vert, n_neigh, n_feat, n_grad_from_out_feat, mean_and_max, (float)n_neigh,
                                d_vertex_order, nullptr, 0, weights_are_exp != 0, scratch, scratch_bytes, stream);
+}
+
+int hgc_accumulate_knn_grad_whole_index_covers(int n_vert, int n_neigh, int n_feat, int mean_and_max) {
+    return n_vert >= 1 && n_neigh >= 1 && (long long)n_vert * (n_neigh + 1ll) < (1ll << 31) &&
+           accumulate_grad_rows_covers(n_feat, n_neigh, mean_and_max != 0, true,
+                                       (unsigned long long)n_vert * n_feat * (mean_and_max ? 2ull : 1ull) * 4ull);
+}
+
+int hgc_accumulate_knn_grad_whole_index(const float *d_grad_from_out_features, const float *d_distances, const float *d_feat,
+                                        const unsigned char *d_max_slots, const int *d_inv_offsets, const int *d_inv_slots,
+                                        const int *d_vertex_order, float *d_out_grad_distances, float *d_out_grad_features,
+                                        int n_vert, int n_neigh, int n_feat, int n_grad_from_out_feat, int mean_and_max,
+                                        int weights_are_exp, void *scratch, size_t scratch_bytes, hgc_stream_t stream) {
+    HGC_REQUIRE(hgc_accumulate_knn_grad_whole_index_covers(n_vert, n_neigh, n_feat, mean_and_max), "shape not covered");
+    HGC_REQUIRE(n_grad_from_out_feat == n_feat * (mean_and_max ? 2 : 1), "bad gradient width");
+    HGC_REQUIRE(d_grad_from_out_features && d_distances && d_feat && d_inv_offsets && d_inv_slots &&
+                    d_out_grad_distances && d_out_grad_features && (d_max_slots || !mean_and_max), "null pointer");
+    if (scratch && (!aligned256(scratch) ||
+                    scratch_bytes < hgc_accumulate_knn_grad_scratch_bytes(n_vert, n_neigh, n_feat, mean_and_max)))
+        return fail(HGC_ERR_WORKSPACE, "accumulate_knn_grad_whole_index: scratch memory misaligned or too small");
+    return launch_accumulate_grad_rows(d_grad_from_out_features, d_distances, d_feat, mean_and_max ? d_max_slots : nullptr,
+                                       d_inv_offsets, d_inv_slots, d_out_grad_distances, d_out_grad_features, n_vert, n_neigh,
+                                       n_feat, n_grad_from_out_feat, mean_and_max != 0, d_vertex_order, (float)n_neigh,
+                                       weights_are_exp != 0, 1, scratch, scratch_bytes, as_stream(stream));
 }
 
 size_t hgc_accumulate_knn_grad_records_workspace_bytes(int n_vert, int n_neigh, int n_feat, int mean_and_max) {

@@ -22,6 +22,10 @@
 // (77 and 90 % busy at 150,000 vertices), vector issue at 66 %, and at a million vertices the
 // L2 misses (37 % of the return path's time).
 //
+// GravNet accumulates over a table without its self column and needs the inverse index of the whole table for the
+// distances: `skip` lets the gather run on that one and pass over the entries of column 0 (one in K + 1), instead of
+// deriving a second index (a training step at 150,000 vertices, K = 64: 2.17 -> 2.11 ms; 240,000, K = 40: 2.27 -> 2.17).
+//
 // The loads of an entry depend on one another (slots, then the max half they gate), so two entries at a
 // time move through a pipeline: slots two steps ahead, rows one step ahead, arithmetic.
 // The dot products of four entries are reduced across the 16 lanes by a transposing exchange (three
@@ -48,7 +52,8 @@ struct GradRows {
     float *gw, *gfeat;
     unsigned long long g_bytes, g_max_bytes, slot_bytes;  // sizes seen by the hardware's range check
     int n_vert, K, F, blocks, pitch;
-    FastDiv div_k;
+    int skip;  // 1: the inverse index is that of a table with one more column in front (K + 1), which is left out
+    FastDiv div_k;  // by K + skip
     float divisor;
     uint32_t slot_shift;  // maxslot has been moved down by this many bytes onto a multiple of 4
     bool negate;  // gw receives -(gradient * w): the chain rule through w = exp(-d)
@@ -96,6 +101,7 @@ struct Entries {
     uint32_t row;    // byte offset of the gradient row, kNoRow beyond the list
     uint32_t slots;  // byte offset of the arg-max slots
     uint32_t key;    // slot of the entry
+    int slot;        // its flat number v K + slot, -1 beyond the list
     float w, w_mean; // weight, and what the mean half is multiplied by
 };
 
@@ -167,10 +173,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
     const int lane = lane_id(), l = lane & (kRowLanes - 1);
     if (WGRAD) {
         // weight gradient of padded slots: they sort behind the last target's entries
-        const int first = p.inv_off[p.n_vert], total = p.n_vert * p.K;
+        const int first = p.inv_off[p.n_vert], total = p.n_vert * (p.K + p.skip);
         for (long long i = first + (long long)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-             i += (long long)gridDim.x * blockDim.x)
-            p.gw[p.inv_slots[i]] = 0.f;
+             i += (long long)gridDim.x * blockDim.x) {
+            const int slot = p.inv_slots[i], v = fast_div(slot, p.div_k);
+            if (slot - v * (p.K + p.skip) >= p.skip) p.gw[slot - (v + 1) * p.skip] = 0.f;
+        }
     }
     // The groups of a workgroup trade their targets so that those of a wave have lists of similar length: a
     // wave runs for as long as its longest one (kNN tables, mean 64 of standard deviation 23: 79 entries of
@@ -223,22 +231,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
 
     const int *list = p.inv_slots + begin + entry_lane(l);
     const int mine = count - entry_lane(l);  // this lane has an entry of chunk c0 if c0 < mine
-    auto entries_of = [&](int slot, float w, int c0) {
+    auto entries_of = [&](int slot, int c0) {
         Entries en;
-        const bool here = c0 < mine;
-        const int v = fast_div(slot, p.div_k);
-        en.key = (uint32_t)(slot - v * p.K);
+        const int v = fast_div(slot, p.div_k), n = slot - v * (p.K + p.skip) - p.skip;
+        const bool here = c0 < mine && n >= 0;  // column 0 of an index of the whole table is nobody's
+        en.key = (uint32_t)n;
+        en.slot = here ? slot - (v + 1) * p.skip : -1;
         en.row = here ? (uint32_t)v * (uint32_t)(p.pitch * 4) : kNoRow;
         en.slots = here ? (uint32_t)v * (uint32_t)p.F : kNoRow;
-        en.w = w;
-        en.w_mean = SCALE == kPow2 ? w * inv_divisor : w;
         return en;
+    };
+    auto weight_of = [&](const Entries &e) { return e.slot >= 0 ? p.w[e.slot] : 0.f; };
+    auto set_weight = [&](Entries &e, float w) {
+        e.w = w;
+        e.w_mean = SCALE == kPow2 ? w * inv_divisor : w;
     };
 
     // slots of the list two chunks ahead, weights and offsets one chunk ahead
-    int slot = 0 < mine ? list[0] : 0;
+    const int slot = 0 < mine ? list[0] : 0;
     int slot_next = kRowLanes < mine ? list[kRowLanes] : 0;
-    Entries en = entries_of(slot, 0 < mine ? p.w[slot] : 0.f, 0);
+    Entries en = entries_of(slot, 0);
+    set_weight(en, weight_of(en));
     int self_key = 0;
     bool self_seen = false;
     uint64_t repeats = 0;
@@ -267,8 +280,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
     st[0].template request_rows<0>(G, GX, en, lane_bytes);
     for (int c0 = 0; c0 < longest; c0 += kRowLanes) {
         const int slot_after = c0 + 2 * kRowLanes < mine ? list[c0 + 2 * kRowLanes] : 0;
-        const float w_next = c0 + kRowLanes < mine ? p.w[slot_next] : 0.f;
-        Entries next = entries_of(slot_next, 0.f, c0 + kRowLanes);
+        Entries next = entries_of(slot_next, c0 + kRowLanes);
+        const float w_next = weight_of(next);
+        set_weight(next, 0.f);
         const uint64_t next_repeats = mark_repeats(next, c0 + kRowLanes);
         float r[4] = {0.f, 0.f, 0.f, 0.f}, val[4];
         // step I: rows of step I + 1 and slots of step I + 2 are requested, then step I is added up
@@ -295,8 +309,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
         if (c0 + 8 < longest) {
             HGC_STEP(4)
             HGC_STEP(5)
-            next.w = w_next;
-            next.w_mean = SCALE == kPow2 ? w_next * inv_divisor : w_next;
+            set_weight(next, w_next);
             HGC_STEP(6)
             HGC_STEP(7)
         }
@@ -304,9 +317,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
         if (WGRAD) {
             float sum = (l & 2) ? ((l & 1) ? r[3] : r[2]) : ((l & 1) ? r[1] : r[0]);
             if (p.blocks == 2) sum = sum + __shfl_xor(sum, kRowLanes, kWave);  // the other half of the row
-            if (c0 < mine && task.block == 0) p.gw[slot] = p.negate ? -(sum * en.w) : sum;
+            if (en.slot >= 0 && task.block == 0) p.gw[en.slot] = p.negate ? -(sum * en.w) : sum;
         }
-        slot = slot_next;
         slot_next = slot_after;
         en = next;
         repeats = next_repeats;
@@ -370,8 +382,8 @@ bool accumulate_grad_rows_covers(int n_feat, int n_neigh, bool mean_and_max, boo
 // (150,000 vertices, K = 40, F = 64: 287 -> 262 us).
 int launch_accumulate_grad_rows(const float *g, const float *w, const float *feat, const unsigned char *maxslot,
                                 const int *inv_off, const int *inv_slots, float *gw, float *gfeat, int n_vert, int K, int F,
-                                int g_cols, bool mean_and_max, const int *order, float divisor, bool negate, void *scratch,
-                                size_t scratch_bytes, hipStream_t s) {
+                                int g_cols, bool mean_and_max, const int *order, float divisor, bool negate, int skip,
+                                void *scratch, size_t scratch_bytes, hipStream_t s) {
     const bool want_w = gw != nullptr;
     const unsigned long long g_bytes = (unsigned long long)n_vert * g_cols * 4ull;
     if (!accumulate_grad_rows_covers(F, K, mean_and_max, maxslot != nullptr, g_bytes) || (mean_and_max && !want_w)) return 1;
@@ -405,7 +417,8 @@ int launch_accumulate_grad_rows(const float *g, const float *w, const float *fea
     p.K = K;
     p.F = F;
     p.pitch = g_cols;
-    p.div_k = make_fast_div(K);
+    p.skip = skip;
+    p.div_k = make_fast_div(K + skip);
     p.divisor = divisor;
     p.negate = negate;
     int vec;

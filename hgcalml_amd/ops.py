@@ -405,6 +405,20 @@ def cached_inverse_neighbour_index(indices):
     return value
 
 
+def accumulate_gradient_index(indices, n_features, mean_and_max):
+    """The inverse index the gradient of an accumulation over `indices` is called with: that of the whole table where
+    `indices` is declared to be its columns 1.. and the gradient's kernel can leave the first column out (recognised by
+    its length, n (k + 1) slots), the table's own one otherwise."""
+    declared = getattr(indices, "_hgc_without_first_column_of", None)
+    if declared is not None and not gl.acc_grad_hit_records:
+        whole, part_version, whole_version = declared
+        n, k = indices.shape
+        if (part_version == indices._version and whole_version == whole._version and
+                lib.hgc_accumulate_knn_grad_whole_index_covers(n, k, n_features, int(mean_and_max))):
+            return cached_inverse_neighbour_index(whole)
+    return cached_inverse_neighbour_index(indices)
+
+
 def invalidate_neighbour_table(indices):
     """Forgets what is cached for the neighbour table `indices` (inverse index, processing
     order), also under other tensor objects on the same memory. Needed only after the table
@@ -433,6 +447,16 @@ def _accumulate_backward(grad_from_out_features, distances, features, neigh_indi
         max_slots = None
     gw = torch.empty((n, k), dtype=torch.float32, device=dev)
     gx = torch.empty((n, f), dtype=torch.float32, device=dev)
+    if n and inv_slots.numel() == n * (k + 1):  # accumulate_gradient_index: the index of the whole table
+        if exp_weights and w.data_ptr() % 16:
+            w = w.clone()
+        need = lib.hgc_accumulate_knn_grad_scratch_bytes(n, k, f, int(mean_and_max))
+        ws = workspace(need, dev) if need else None
+        check(lib.hgc_accumulate_knn_grad_whole_index(p(g), p(w), p(x), p(max_slots), p(inv_offsets), p(inv_slots),
+                                                      p(vertex_order_of(neigh_indices)), p(gw), p(gx), n, k, f, g.shape[1],
+                                                      int(mean_and_max), int(exp_weights), p(ws),
+                                                      ws.numel() if need else 0, stream()))
+        return gw, gx
     # on request, with the slot table: one record per (vertex, slot) in scratch memory carries the max part to the gather
     need = 0
     if max_slots is not None and gl.acc_grad_hit_records:

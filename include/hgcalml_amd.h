@@ -551,6 +551,22 @@ int hgc_sort_distinct_keys(unsigned long long *d_keys, long long n, int value_bi
 /* Condensate assignment                                               */
 /* ------------------------------------------------------------------ */
 
+/* hgc_accumulate_knn_grad_scratch for a table that is columns 1.. of another
+ * one [n_vert, n_neigh + 1] (GravNet drops the self column of its kNN result),
+ * fed with the inverse index of that whole table, which the distance gradient
+ * needs anyway: the entries of its column 0 are left out. Same results as with
+ * the index of the table itself. For shapes the query accepts (rows of 16 to 128
+ * features, d_max_slots given with mean_and_max). No counterpart in the
+ * reference. */
+int hgc_accumulate_knn_grad_whole_index_covers(int n_vert, int n_neigh, int n_feat, int mean_and_max);
+int hgc_accumulate_knn_grad_whole_index(const float *d_grad_from_out_features, const float *d_distances,
+                                        const float *d_feat, const unsigned char *d_max_slots,
+                                        const int *d_inv_offsets, const int *d_inv_slots,
+                                        const int *d_vertex_order, float *d_out_grad_distances,
+                                        float *d_out_grad_features, int n_vert, int n_neigh, int n_feat,
+                                        int n_grad_from_out_feat, int mean_and_max, int weights_are_exp,
+                                        void *scratch, size_t scratch_bytes, hgc_stream_t stream);
+
 /* ---- the GravNet block around its search and accumulation
  * (modules/GravNetLayersRagged.py:3095-3283, tensor operations there) ---- */
 

@@ -113,3 +113,31 @@ def test_weights_sum(n, k, f):
         assert torch.isfinite(a).all()
         assert (a - b).norm() <= 1e-5 * b.norm() + 1e-30
     assert (torch.autograd.grad(_AccumulateSumwFn.apply(d, x, idx), d, grad)[0][idx < 0] == 0).all()
+
+
+@pytest.mark.parametrize("n,k,f", [(2, 1, 16), (17, 3, 17), (66, 15, 33), (67, 16, 64), (90, 17, 65), (83, 40, 128), (70, 64, 48),
+                                   (40, 5, 130), (40, 5, 8)])
+@pytest.mark.parametrize("mean_and_max", [True, False])
+def test_gradient_with_the_index_of_the_whole_table(n, k, f, mean_and_max):
+    """bit for bit the gradients with the narrow table's own index, for padded rows and whatever column 0 holds; shapes the
+    kernel does not cover are given the narrow index"""
+    from hgcalml_amd import AccumulateKnn, ops
+    g = torch.Generator().manual_seed(n + k + f)
+    part = torch.rand(n, n, generator=g).argsort(1)[:, :k].to(torch.int32)
+    part[torch.rand(n, generator=g) < 0.3, k // 2:] = -1
+    first = torch.where(torch.rand(n, generator=g) < 0.7, torch.arange(n), torch.randint(-1, n, (n,), generator=g))
+    whole = torch.cat([first.to(torch.int32)[:, None], part], dim=1).to(DEV)
+    d = torch.rand(n, k, generator=g).to(DEV).requires_grad_(True)
+    x = torch.randn(n, f, generator=g).to(DEV).requires_grad_(True)
+    grad = torch.randn(n, 2 * f if mean_and_max else f, generator=g).to(DEV)
+    results = []
+    for declared in (False, True):
+        table = part.to(DEV)
+        if declared:
+            ops.declare_without_first_column(table, whole)
+            index = ops.accumulate_gradient_index(table, f, mean_and_max)
+            assert index[1].numel() == n * (k + 1 if 16 <= f <= 128 else k)
+        out = AccumulateKnn(d, x, table, mean_and_max=mean_and_max)[0]
+        results.append(torch.autograd.grad(out, [d, x], grad))
+    for a, b in zip(*results):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
