@@ -364,18 +364,6 @@ __device__ __forceinline__ void store_bin_row(int *binass, size_t row, int n_dim
     }
 }
 
-__device__ __forceinline__ void copy_coords_row(const float *coords, int from, float *out, int to, int n_coords,
-                                                int rows_aligned) {
-    if (n_coords == 4 && rows_aligned) {
-        reinterpret_cast<float4 *>(out)[to] = reinterpret_cast<const float4 *>(coords)[from];
-    } else if (n_coords == 3) {  // one 12-byte store per row instead of three of 4 bytes to a scattered address
-        struct __attribute__((packed, aligned(4))) Row3 { float v[3]; };
-        reinterpret_cast<Row3 *>(out)[to] = reinterpret_cast<const Row3 *>(coords)[from];
-    } else {
-        for (int c = 0; c < n_coords; ++c) out[(size_t)to * n_coords + c] = coords[(size_t)from * n_coords + c];
-    }
-}
-
 __global__ __launch_bounds__(256) void bin_points_ranked_kernel(
     const float *__restrict__ coords, int stride, const float *__restrict__ partial, int n_partial,
     const int *__restrict__ row_splits, int n_vert, int n_dims, int n_rs, int n_bins_scalar,

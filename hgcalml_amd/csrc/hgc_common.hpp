@@ -182,6 +182,19 @@ __device__ __forceinline__ int xcd_chunked_block(int bid, int nblocks) {
     return ((k / CHUNK) * kNumXcd + xcd) * CHUNK + k % CHUNK;
 }
 
+// out[to, :] = coords[from, :]; rows_aligned: both matrices start on 16-byte boundaries
+__device__ __forceinline__ void copy_coords_row(const float *coords, int from, float *out, int to, int n_coords,
+                                                int rows_aligned) {
+    if (n_coords == 4 && rows_aligned) {
+        reinterpret_cast<float4 *>(out)[to] = reinterpret_cast<const float4 *>(coords)[from];
+    } else if (n_coords == 3) {  // one 12-byte store per row instead of three of 4 bytes to a scattered address
+        struct __attribute__((packed, aligned(4))) Row3 { float v[3]; };
+        reinterpret_cast<Row3 *>(out)[to] = reinterpret_cast<const Row3 *>(coords)[from];
+    } else {
+        for (int c = 0; c < n_coords; ++c) out[(size_t)to * n_coords + c] = coords[(size_t)from * n_coords + c];
+    }
+}
+
 __device__ __forceinline__ int readlane_i32(int v, int lane) {
     return __builtin_amdgcn_readlane(v, lane);
 }
