@@ -18,9 +18,8 @@ into a HIP graph (same kernels, same buffers); the faster of the two is reported
 The `roofline` object is measured in a second timed loop of the same run (also
 K iterations, HIP events on the stream the kernels are launched on) at cfg4
 (N=1,000,000, K=64, F=128, banded neighbour table): the dominant piece, one call
-of the accumulate_knn gradient (algorithmic bytes 4*N*(3K+5F); two kernels: the
-streaming pass that builds the per-slot hit records and the gather over the
-inverse index), with the forward launch (4*N*(2K+4F)), the forward+gradient pair
+of the accumulate_knn gradient (algorithmic bytes 4*N*(3K+5F); one kernel, a gather
+over the inverse index), with the forward launch (4*N*(2K+4F)), the forward+gradient pair
 and the pair plus one build of the inverse neighbour index next to it, against
 the 8 TB/s HBM peak. Next to the fraction of the HBM roofline it states two
 floors of what this formulation can reach on this memory system: the same
@@ -280,18 +279,18 @@ def main():
     import hgcalml_amd.globals as gl
     grad_ms = event_ms(lambda: torch.ops.hgcalml.accumulate_knn_grad_slots(g4, w4, x4, i4, arg4, slots4, *inv),
                        r_steps, r_warm)
-    # the same gradient through the gather that compares slot bytes (no records, no streaming pass)
-    gl.acc_grad_hit_records = False
-    grad_slots_ms = event_ms(lambda: torch.ops.hgcalml.accumulate_knn_grad_slots(g4, w4, x4, i4, arg4, slots4, *inv),
-                             max(3, r_steps // 2), 2)
+    # the same gradient with a streaming pass that hands the max part to the gather as records
+    gl.acc_grad_hit_records = True
+    grad_records_ms = event_ms(lambda: torch.ops.hgcalml.accumulate_knn_grad_slots(g4, w4, x4, i4, arg4, slots4, *inv),
+                               max(3, r_steps // 2), 2)
     gl.acc_grad_hit_records = None
     # the K-fold gather of this table with one multiply-add per gathered element and nothing else
     push_ms = event_ms(lambda: torch.ops.hgcalml.push_knn(w4, x4, i4), max(3, r_steps // 2), 2)
     bytes_fwd = 4.0 * n4 * (2 * K4 + 4 * F4)
     bytes_bwd = 4.0 * n4 * (3 * K4 + 5 * F4)
     achieved = (bytes_fwd + bytes_bwd) / ((fwd_ms[0] + grad_ms[0]) * 1e-3) / 1e9
-    log("bench: cfg4 fwd %.3f ms, grad %.3f ms (slot-byte gather %.3f ms, bare ordered gather %.3f ms), inverse index "
-        "(one-off) %.3f ms -> %.1f GB/s" % (fwd_ms[0], grad_ms[0], grad_slots_ms[0], push_ms[0], inv_ms[0], achieved))
+    log("bench: cfg4 fwd %.3f ms, grad %.3f ms (through records %.3f ms, bare ordered gather %.3f ms), inverse index "
+        "(one-off) %.3f ms -> %.1f GB/s" % (fwd_ms[0], grad_ms[0], grad_records_ms[0], push_ms[0], inv_ms[0], achieved))
 
     if args.section == "streams":
         # same table, same inputs: the gradient without the max half (no slot bytes, no max-half loads), and the
@@ -402,16 +401,15 @@ def main():
         "accumulate_fwd_grad_GBps": round(achieved, 1),
         # the dominant kernel of the graded path: one launch of the one-pass gradient kernel
         "roofline": {"bound": "hbm",
-                     "kernel": "hit_records_kernel + accumulate_grad_records_kernel + weight_grad_to_table_kernel: one "
-                               "call of the accumulate_knn gradient (weights + features), cfg4 (N=%d, K=%d, F=%d)"
-                               % (n4, K4, F4),
+                     "kernel": "accumulate_grad_rows_kernel: one call of the accumulate_knn gradient (weights + features), "
+                               "cfg4 (N=%d, K=%d, F=%d)" % (n4, K4, F4),
                      "achieved": round(bytes_bwd / (grad_ms[0] * 1e-3) / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(bytes_bwd / (grad_ms[0] * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
                      "traffic": traffic["gradient"] if traffic else None,
                      "traffic_measured_at": traffic["measured_at"] if traffic else None,
                      "algorithmic_bytes": bytes_bwd, "launch_ms": round(grad_ms[0], 4),
-                     # the same call through the gather that compares slot bytes (one kernel, no records)
-                     "launch_ms_slot_byte_gather": round(grad_slots_ms[0], 4),
+                     # the same gradient through a streaming pass of records (three kernels)
+                     "launch_ms_records": round(grad_records_ms[0], 4),
                      # floors of this formulation on this memory system: the bare K-fold gather of the same rows
                      # (PushKnn, timed above), the issue time of the gradient's vector instructions (counters)
                      "l2_gather_floor_ms": round(push_ms[0], 4),
