@@ -105,7 +105,18 @@ __device__ __forceinline__ int lanes_below(uint64_t mask) {
 
 constexpr int kAhead = 8;  // steps of 64 items whose loads are issued together (memory-level parallelism)
 
-// item i has the key keys[i] and the value i
+// Positions are counted from where a workgroup's stretch (or its tile, level 2) begins: a walk looks up to a batch
+// beyond the end of its stretch, which as a position among all items, of which there may be 2^31 - 1, would not
+// fit into an int.
+struct Stretch {
+    int first, count;
+};
+__device__ __forceinline__ Stretch stretch_of(int group, int per_group, int total) {
+    const long long first = min((long long)group * per_group, (long long)total);
+    return {(int)first, (int)min((long long)per_group, total - first)};
+}
+
+// keys[first], keys[first + STRIDE], ...
 template <int STRIDE, int N>
 __device__ __forceinline__ void load_items(const int *__restrict__ keys, int first, int last, int (&key)[N]) {
     // loads past the end re-read the last item: no branch, all of them in flight together
@@ -121,14 +132,13 @@ __global__ __launch_bounds__(kCountThreads) void tile_count_kernel(const int *__
     extern __shared__ int s_count[];  // [n_tiles]
     for (int t = threadIdx.x; t < n_tiles; t += blockDim.x) s_count[t] = 0;
     __syncthreads();
-    const long long first = (long long)blockIdx.x * per_group;
-    const int begin = (int)min(first, (long long)total), end = (int)min(first + per_group, (long long)total);
-    for (int e0 = begin + (int)threadIdx.x; e0 - (int)threadIdx.x < end; e0 += kCountThreads * kAhead) {
+    const Stretch own = stretch_of(blockIdx.x, per_group, total);
+    for (int e0 = (int)threadIdx.x; e0 - (int)threadIdx.x < own.count; e0 += kCountThreads * kAhead) {
         int raw[kAhead];
-        load_items<kCountThreads>(keys, e0, end - 1, raw);
+        load_items<kCountThreads>(keys + own.first, e0, own.count - 1, raw);
 #pragma unroll
         for (int a = 0; a < kAhead; ++a)
-            if (e0 + a * kCountThreads < end) atomicAdd(&s_count[clamp_key(raw[a], n_keys) >> lo_bits], 1);
+            if (e0 + a * kCountThreads < own.count) atomicAdd(&s_count[clamp_key(raw[a], n_keys) >> lo_bits], 1);
     }
     __syncthreads();
     for (int t = threadIdx.x; t < n_tiles; t += blockDim.x) counts[(size_t)t * n_groups + blockIdx.x] = s_count[t];
@@ -161,17 +171,16 @@ __global__ __launch_bounds__(kMoveThreads) void tile_move_kernel(const int *__re
     const int wave = threadIdx.x >> 6, lane = lane_id();
     uint16_t *const mine = s_count + wave * row;
     for (int t = threadIdx.x; t < n_tiles; t += kMoveThreads) s_next[t] = starts[(size_t)t * n_groups + blockIdx.x];
-    const long long first = (long long)blockIdx.x * per_group;
-    const int begin = (int)min(first, (long long)total), end = (int)min(first + per_group, (long long)total);
+    const Stretch own = stretch_of(blockIdx.x, per_group, total);
     const int tiles_per_thread = (n_tiles + kMoveThreads - 1) / kMoveThreads;
 
-    for (int b0 = begin; b0 < end; b0 += kBatch) {
-        const int in_batch = min(kBatch, end - b0);
+    for (int b0 = 0; b0 < own.count; b0 += kBatch) {
+        const int in_batch = min(kBatch, own.count - b0);
         const int per_wave = ((in_batch + kMoveWaves - 1) / kMoveWaves + kWave - 1) / kWave * kWave;
         const int w0 = min(wave * per_wave, in_batch), w1 = min(w0 + per_wave, in_batch);
         int key[kMoveSteps];
         for (int i = threadIdx.x; i < kMoveWaves * row / 2; i += kMoveThreads) reinterpret_cast<uint32_t *>(s_count)[i] = 0;
-        load_items<kWave>(keys, b0 + w0 + lane, end - 1, key);
+        load_items<kWave>(keys + own.first, b0 + w0 + lane, own.count - 1, key);
         lds_barrier();
 #pragma unroll
         for (int a = 0; a < kMoveSteps; ++a) {
@@ -217,7 +226,7 @@ __global__ __launch_bounds__(kMoveThreads) void tile_move_kernel(const int *__re
             lds_order_point();
             if (valid && rank == 0) mine[tile] = (uint16_t)(place + (int)__popcll(peers));
             lds_order_point();
-            if (valid) s_stage[place + rank] = make_uint2((uint32_t)key[a], (uint32_t)(b0 + w0 + a * kWave + lane));
+            if (valid) s_stage[place + rank] = make_uint2((uint32_t)key[a], (uint32_t)own.first + (uint32_t)(b0 + w0 + a * kWave + lane));
         }
         lds_barrier();
         for (int i = threadIdx.x; i < in_batch; i += kMoveThreads) {
@@ -289,19 +298,18 @@ __global__ __launch_bounds__(kMoveThreads) void tile_move_wide_kernel(const int 
     uint16_t *const s_local = reinterpret_cast<uint16_t *>(s_next + n_tiles);  // its first place in the batch (where it has items)
     const int wave = threadIdx.x >> 6, lane = lane_id();
     for (int t = threadIdx.x; t < n_tiles; t += kMoveThreads) s_next[t] = starts[(size_t)t * n_groups + blockIdx.x];
-    const long long first = (long long)blockIdx.x * per_group;
-    const int begin = (int)min(first, (long long)total), end = (int)min(first + per_group, (long long)total);
+    const Stretch own = stretch_of(blockIdx.x, per_group, total);
 
-    for (int b0 = begin; b0 < end; b0 += kBatch) {
-        const int in_batch = min(kBatch, end - b0);
+    for (int b0 = 0; b0 < own.count; b0 += kBatch) {
+        const int in_batch = min(kBatch, own.count - b0);
         const int per_wave = ((in_batch + kMoveWaves - 1) / kMoveWaves + kWave - 1) / kWave * kWave;
         const int w0 = min(wave * per_wave, in_batch), w1 = min(w0 + per_wave, in_batch);
         int key[kMoveSteps], val[kMoveSteps];
-        load_items<kWave>(keys, b0 + w0 + lane, end - 1, key);
+        load_items<kWave>(keys + own.first, b0 + w0 + lane, own.count - 1, key);
 #pragma unroll
         for (int a = 0; a < kMoveSteps; ++a) {
             key[a] = (int)clamp_key(key[a], n_keys);
-            val[a] = b0 + w0 + a * kWave + lane;
+            val[a] = (int)((uint32_t)own.first + (uint32_t)(b0 + w0 + a * kWave + lane));
         }
         batch_pass<BITS>(key, val, w0, w1, lo_bits, s_counters, s_wave_sums, s_stage);
 #pragma unroll
@@ -387,24 +395,26 @@ __global__ __launch_bounds__(kSortWaves *kWave) void tile_sort_kernel(const uint
     __shared__ int s_stage[kHeldItems];
     const int wave = threadIdx.x >> 6, lane = lane_id();
     const int tile = blockIdx.x;
-    const int begin_tile = starts[(size_t)tile * n_groups], end_tile = starts[(size_t)(tile + 1) * n_groups];
-    const bool held = end_tile - begin_tile <= kHeldItems;
+    const int begin_tile = starts[(size_t)tile * n_groups], in_tile = starts[(size_t)(tile + 1) * n_groups] - begin_tile;
+    const bool held = in_tile <= kHeldItems;
+    order += begin_tile;
     for (int t = threadIdx.x; t < T * kSortWaves; t += blockDim.x) (&s_cursor[0][0])[t] = 0;
-    const int per_wave = ((end_tile - begin_tile + kSortWaves - 1) / kSortWaves + kWave - 1) / kWave * kWave;
-    const int begin = min(begin_tile + wave * per_wave, end_tile), end = min(begin + per_wave, end_tile);
+    const int per_wave = (max(in_tile - 1, 0) / (kSortWaves * kWave) + 1) * kWave;
+    const Stretch own = stretch_of(wave, per_wave, in_tile);
+    records += (size_t)begin_tile + own.first;
     uint2 rec[kSortSteps];
     if (held) {
 #pragma unroll
         for (int a = 0; a < kSortSteps; ++a)
-            if (begin + a * kWave < end) rec[a] = records[min(begin + a * kWave + lane, end - 1)];  // wave-uniform
+            if (a * kWave < own.count) rec[a] = records[min(a * kWave + lane, own.count - 1)];  // wave-uniform
     }
     lds_barrier();
     if (held) {
 #pragma unroll
         for (int a = 0; a < kSortSteps; ++a)
-            if (begin + a * kWave + lane < end) atomicAdd(&s_cursor[wave][rec[a].x & (T - 1)], 1);
+            if (a * kWave + lane < own.count) atomicAdd(&s_cursor[wave][rec[a].x & (T - 1)], 1);
     } else {
-        for (int e = begin + lane; e < end; e += kWave) atomicAdd(&s_cursor[wave][records[e].x & (T - 1)], 1);
+        for (int e = lane; e < own.count; e += kWave) atomicAdd(&s_cursor[wave][records[e].x & (T - 1)], 1);
     }
     lds_barrier();
     // per key: the waves' counts become their first positions inside the key's run
@@ -455,19 +465,19 @@ __global__ __launch_bounds__(kSortWaves *kWave) void tile_sort_kernel(const uint
     if (held) {
 #pragma unroll
         for (int a = 0; a < kSortSteps; ++a) {
-            if (begin + a * kWave >= end) break;  // wave-uniform
-            const bool valid = begin + a * kWave + lane < end;
+            if (a * kWave >= own.count) break;  // wave-uniform
+            const bool valid = a * kWave + lane < own.count;
             const int place = place_of(rec[a].x, valid);
             if (valid) s_stage[place] = (int)rec[a].y;
         }
         lds_barrier();
-        for (int i = threadIdx.x; i < end_tile - begin_tile; i += blockDim.x) order[(size_t)begin_tile + i] = s_stage[i];
+        for (int i = threadIdx.x; i < in_tile; i += blockDim.x) order[i] = s_stage[i];
     } else {
-        for (int c0 = begin; c0 < end; c0 += kWave) {  // wave-uniform
-            const uint2 r = records[min(c0 + lane, end - 1)];
-            const bool valid = c0 + lane < end;
+        for (int c0 = 0; c0 < own.count; c0 += kWave) {  // wave-uniform
+            const uint2 r = records[min(c0 + lane, own.count - 1)];
+            const bool valid = c0 + lane < own.count;
             const int place = place_of(r.x, valid);
-            if (valid) order[(size_t)begin_tile + place] = (int)r.y;
+            if (valid) order[place] = (int)r.y;
         }
     }
 }

@@ -29,3 +29,35 @@ def test_inverse_index_at_the_ends_of_batches_and_tiles(n, k, kind):
     order = torch.sort(key, stable=True).indices
     assert torch.equal(slots[:n * k].to(torch.int64), order)
     assert torch.equal(off.to(torch.int64), torch.searchsorted(key[order], torch.arange(n + 1, device=DEV)))
+
+
+@pytest.mark.parametrize("n,k", [(8388607, 256), (1000, 2147483)])
+def test_inverse_index_of_the_largest_tables(n, k):
+    """2^31 - 256 and 2^31 - 648 slots: the walks look ahead beyond the largest int"""
+    from hgcalml_amd import ops
+    total = n * k
+    assert 2 ** 31 - 12288 < total < 2 ** 31
+    if torch.cuda.mem_get_info()[0] < 64 << 30:
+        pytest.skip("needs 64 GB of device memory")
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(n)
+    idx = torch.randint(-1, n, (n, k), dtype=torch.int32, device=DEV, generator=gen)
+    off, slots = ops.inverse_neighbour_index(idx)
+    flat = idx.view(-1)
+    # the first position of every key, with that of the slots without a neighbour and the end behind them
+    begin = torch.cat([off.to(torch.int64), torch.tensor([total], device=DEV)])
+    assert int(begin[0]) == 0 and bool((begin.diff() >= 0).all())
+    last_key, last_slot = -1, -1
+    for s in range(0, total, 1 << 27):
+        part = slots[s:min(total, s + (1 << 27))].to(torch.int64)
+        assert int(part.min()) >= 0 and int(part.max()) < total
+        key = flat[part].to(torch.int64)
+        key[key < 0] = n
+        at = torch.arange(s, s + len(part), device=DEV)
+        assert bool((begin[key] <= at).all()) and bool((at < begin[key + 1]).all())
+        step, same = part.diff(), key.diff() == 0
+        assert bool((key.diff() >= 0).all()) and bool((step[same] > 0).all())     # sorted, and stable: no slot twice
+        assert int(key[0]) > last_key or (int(key[0]) == last_key and int(part[0]) > last_slot)
+        last_key, last_slot = int(key[-1]), int(part[-1])
+    del idx, flat, off, slots, part, key, at, step, same
+    torch.cuda.empty_cache()
