@@ -19,7 +19,8 @@
 //            way (count per wave, scan over the tile's keys, ordered walk) into a
 //            stage in LDS, from where the tile's values leave in whole lines,
 //            together with the first position of every key. Tiles of up to
-//            20,480 items are held in registers between the count and the walk.
+//            20,480 items are held in registers between the count and the walk, larger
+//            ones are read twice.
 // 9.75 M items, 150,000 keys (the inverse index of a kNN table): 205 -> 119 us; 64 M items, a million
 // keys: 1.32 -> 0.84 ms (kNN table), 0.92 -> 0.80 (banded). Bound by vector issue and LDS latency of
 // the walks (16 waves per CU); the memory traffic alone would take 60 us and 0.4 ms.
@@ -381,9 +382,15 @@ constexpr int kSortWaves = 16;  // counters (4 bytes per wave and key) and stage
 constexpr int kSortSteps = 20;  // steps of 64 records a wave holds in registers between the count and the walk
 constexpr int kHeldItems = kSortWaves * kWave * kSortSteps;
 
+// What the stage holds: twice as many items as a tile aims at where the counters leave the room
+constexpr int stage_items(int lo_bits) { return lo_bits <= 8 ? 32768 : kHeldItems; }
+
 // One workgroup per tile. The tile's values leave through a stage in LDS, so that global memory
 // sees whole lines instead of one 4-byte write per slot. A tile with more items than the registers
-// and the stage hold reads its records twice and writes its values one by one.
+// hold (few keys, or a few that most items share) reads its records twice, kAhead steps at a time, one with
+// more than the stage holds writes its values one by one. (Step by step every wave waits for one load after
+// the other: 5 M items of 300 keys 540 us, now 402; the index of 6.4 M slots that name 2000 of 100,000
+// vertices 569, now 427.)
 template <int LO_BITS>
 __global__ __launch_bounds__(kSortWaves *kWave) void tile_sort_kernel(const uint2 *__restrict__ records,
                                                                       const int *__restrict__ starts, int n_groups,
@@ -392,11 +399,12 @@ __global__ __launch_bounds__(kSortWaves *kWave) void tile_sort_kernel(const uint
     constexpr int T = 1 << LO_BITS;
     __shared__ int s_cursor[kSortWaves][T];
     __shared__ int s_total[T];
-    __shared__ int s_stage[kHeldItems];
+    constexpr int kStage = stage_items(LO_BITS);
+    __shared__ int s_stage[kStage];
     const int wave = threadIdx.x >> 6, lane = lane_id();
     const int tile = blockIdx.x;
     const int begin_tile = starts[(size_t)tile * n_groups], in_tile = starts[(size_t)(tile + 1) * n_groups] - begin_tile;
-    const bool held = in_tile <= kHeldItems;
+    const bool held = in_tile <= kHeldItems, staged = in_tile <= kStage;
     order += begin_tile;
     for (int t = threadIdx.x; t < T * kSortWaves; t += blockDim.x) (&s_cursor[0][0])[t] = 0;
     const int per_wave = (max(in_tile - 1, 0) / (kSortWaves * kWave) + 1) * kWave;
@@ -414,7 +422,14 @@ __global__ __launch_bounds__(kSortWaves *kWave) void tile_sort_kernel(const uint
         for (int a = 0; a < kSortSteps; ++a)
             if (a * kWave + lane < own.count) atomicAdd(&s_cursor[wave][rec[a].x & (T - 1)], 1);
     } else {
-        for (int e = lane; e < own.count; e += kWave) atomicAdd(&s_cursor[wave][records[e].x & (T - 1)], 1);
+        for (int e0 = lane; e0 - lane < own.count; e0 += kWave * kAhead) {
+            uint32_t key[kAhead];
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a) key[a] = records[min(e0 + a * kWave, own.count - 1)].x;
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a)
+                if (e0 + a * kWave < own.count) atomicAdd(&s_cursor[wave][key[a] & (T - 1)], 1);
+        }
     }
     lds_barrier();
     // per key: the waves' counts become their first positions inside the key's run
@@ -470,16 +485,24 @@ __global__ __launch_bounds__(kSortWaves *kWave) void tile_sort_kernel(const uint
             const int place = place_of(rec[a].x, valid);
             if (valid) s_stage[place] = (int)rec[a].y;
         }
-        lds_barrier();
-        for (int i = threadIdx.x; i < in_tile; i += blockDim.x) order[i] = s_stage[i];
     } else {
-        for (int c0 = 0; c0 < own.count; c0 += kWave) {  // wave-uniform
-            const uint2 r = records[min(c0 + lane, own.count - 1)];
-            const bool valid = c0 + lane < own.count;
-            const int place = place_of(r.x, valid);
-            if (valid) order[place] = (int)r.y;
+        for (int c0 = 0; c0 < own.count; c0 += kWave * kAhead) {  // wave-uniform
+            uint2 r[kAhead];
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a) r[a] = records[min(c0 + a * kWave + lane, own.count - 1)];
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a) {
+                if (c0 + a * kWave >= own.count) break;  // wave-uniform
+                const bool valid = c0 + a * kWave + lane < own.count;
+                const int place = place_of(r[a].x, valid);
+                if (valid && staged) s_stage[place] = (int)r[a].y;
+                if (valid && !staged) order[place] = (int)r[a].y;
+            }
         }
+        if (!staged) return;
     }
+    lds_barrier();
+    for (int i = threadIdx.x; i < in_tile; i += blockDim.x) order[i] = s_stage[i];
 }
 
 

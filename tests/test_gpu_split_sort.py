@@ -13,7 +13,10 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("n,k,kind", [(1, 5, "random"), (63, 65, "random"), (64, 64, "random"), (4096, 1, "random"), (4097, 1, "random"),
                                       (12288, 1, "random"), (49152, 64, "random"), (49153, 64, "random"), (1572863, 1, "random"),
                                       (1572864, 2, "random"), (4194303, 1, "random"), (4194304, 1, "random"), (60000, 40, "few"),
-                                      (2000000, 3, "sorted")])
+                                      (2000000, 3, "sorted"),
+                                      # one tile: held in registers up to 20,480 slots, staged in LDS up to 32,768
+                                      (16, 1280, "random"), (1, 20481, "random"), (16, 2048, "random"), (1, 32769, "random"),
+                                      (31, 8200, "random"), (3, 512, "random"), (3, 513, "random")])
 def test_inverse_index_at_the_ends_of_batches_and_tiles(n, k, kind):
     from hgcalml_amd import ops
     rng = np.random.default_rng(n + 7 * k)
