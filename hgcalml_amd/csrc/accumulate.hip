@@ -219,6 +219,7 @@ __global__ __launch_bounds__(256) void accumulate_fwd_rows_kernel(const float *_
     const int *irow = idx + (size_t)v * K;
     const float *wrow = w + (size_t)v * K;
     const __amdgpu_buffer_rsrc_t rows = make_rows(feat, (unsigned long long)n_vert * F * 4ull);
+    const uint32_t no_row = no_row_offset(F);
     // A lane at the end of a row that is no multiple of VEC takes the last VEC columns (never columns of the
     // next row): what it shares with its neighbour both compute and store alike.
     const int fb = task.block * (kRowLanes * VEC) + l * VEC, f = min(fb, F - VEC);
@@ -249,7 +250,7 @@ __global__ __launch_bounds__(256) void accumulate_fwd_rows_kernel(const float *_
         w_next = in_row ? wrow[c0 + kRowLanes + l] : 0.f;
 
         const bool has_row = (uint32_t)j < (uint32_t)n_vert;
-        const uint32_t offset = has_row ? (uint32_t)j * (uint32_t)(F * 4) : kNoRow;
+        const uint32_t offset = has_row ? (uint32_t)j * (uint32_t)(F * 4) : no_row;
         wn = has_row ? wn : 0.f;
         const uint64_t valid = __builtin_amdgcn_ballot_w64(has_row);
         const uint64_t seeds = c0 == 0 ? ~0ull : 0ull;
@@ -834,7 +835,7 @@ int accumulate_forward(const float *d_distances, const float *d_feat, const int 
     const uintptr_t align_or = reinterpret_cast<uintptr_t>(d_feat) | reinterpret_cast<uintptr_t>(d_out_feat) |
                               reinterpret_cast<uintptr_t>(d_out_maxidxs);
     // the row kernel addresses rows through 32-bit buffer offsets
-    const bool row_kernel = n_feat >= 16 && (unsigned long long)n_vert * (unsigned long long)n_feat * 4ull <= kMaxRowBytes;
+    const bool row_kernel = n_feat >= 16 && rows_addressable(n_vert, n_feat);
     if (d_out_weights && !row_kernel) {  // the weights in a pass of their own, then as if they had been given
         const int rc = hgc_exp_neg(d_distances, d_out_weights, (long long)n_vert * n_neigh, stream);
         if (rc) return rc;

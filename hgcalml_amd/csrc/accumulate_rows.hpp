@@ -189,9 +189,14 @@ __device__ __forceinline__ GroupTask group_task(const int *__restrict__ order, i
 }
 
 // A byte offset beyond every matrix the row kernels take (kMaxRowBytes): the hardware's range check
-// turns a load there into 0 without a memory access. Column offsets added to it do not wrap.
+// turns a load there into 0 without a memory access. Column offsets of rows of up to 256 features, which is
+// what the gradients' kernels take, do not wrap when they are added to it.
 constexpr uint32_t kNoRow = 0xffff0000u;
 constexpr unsigned long long kMaxRowBytes = 0xffff0000ull;
+
+// The same for rows of any length: behind the matrix, and a whole row in front of the end of the 32 bits
+__host__ __device__ constexpr uint32_t no_row_offset(int cols) { return 0xffffffe0u - (uint32_t)cols * 4u; }
+inline bool rows_addressable(int n_rows, int cols) { return (n_rows + 1ull) * (unsigned long long)cols * 4ull <= 0xffffffe0ull; }
 
 // VEC consecutive 4-byte elements at byte offset `offset` of a raw buffer
 template <int VEC>
