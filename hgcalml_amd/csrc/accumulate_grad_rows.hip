@@ -105,9 +105,18 @@ struct Entries {
     float w, w_mean; // weight, and what the mean half is multiplied by
 };
 
+// What a lane holds of another lane's columns (rows that do not fill their lanes) must not reach the dot
+// products, whatever its value: 0 * infinity is no 0.
+//   kFull      every lane has VEC columns of its own
+//   kLanes     a lane has VEC columns of its own or none: its dot products are left out
+//   kElements  a lane may share some of its columns: these elements are taken as 0 and not stored either
+// own[e]: the lanes whose element e is theirs. (150,000 vertices, own features of 0 in their place and now:
+// K = 40, F = 22 178 and 177 us, F = 50 229 and 231; K = 16, F = 127 208 and 212.)
+enum Tail { kFull, kLanes, kElements };
+
 // Two entries on their way through the pipeline: arg-max slots (requested two steps ahead), gradient
 // rows (requested one step ahead, the max half by the slots), arithmetic.
-template <int VEC, bool MAX, bool ALIGNED>
+template <int VEC, bool MAX, bool ALIGNED, Tail TAIL>
 struct Step {
     SlotBytes<VEC, ALIGNED> sb[2];
     float gm[2][VEC], gx[2][VEC];
@@ -144,15 +153,17 @@ struct Step {
     // w_max: 0 in the lanes of repeated self references, whose max part counts for the weight gradient only.
     template <int U, Scale SCALE, bool WGRAD>
     __device__ __forceinline__ void add(float w, float w_mean, float w_max, const float (&xo)[VEC], const float (&xk)[VEC],
-                                        float divisor, float (&acc)[VEC], float &val) const {
+                                        const uint64_t (&own)[VEC], float divisor, float (&acc)[VEC], float &val) const {
+        float dot = 0.f;
 #pragma unroll
         for (int e = 0; e < VEC; ++e) {
-            const float g = gm[U][e];
+            const float g = TAIL != kElements || __builtin_amdgcn_inverse_ballot_w64(own[e]) ? gm[U][e] : 0.f;
             const float part = SCALE == kDivide ? (g / divisor) * w : g * w_mean;
-            if (WGRAD) val = __builtin_fmaf(g, xk[e], val);
+            if (WGRAD) dot = __builtin_fmaf(g, xk[e], dot);
             if constexpr (MAX) {
-                const float gsel = VEC == 1 ? gx[U][e] : __builtin_amdgcn_inverse_ballot_w64(hit[U][e]) ? gx[U][e] : 0.f;
-                if (WGRAD) val = __builtin_fmaf(gsel, xo[e], val);
+                const uint64_t here = TAIL == kElements ? hit[U][e] & own[e] : hit[U][e];
+                const float gsel = VEC == 1 ? gx[U][e] : __builtin_amdgcn_inverse_ballot_w64(here) ? gx[U][e] : 0.f;
+                if (WGRAD) dot = __builtin_fmaf(gsel, xo[e], dot);
                 const float part_max = gsel * w_max;
                 const float sum = part + part_max;
                 acc[e] = acc[e] + sum;
@@ -160,6 +171,7 @@ struct Step {
                 acc[e] = acc[e] + part;  // the reference's "+ 0" cannot change the sum
             }
         }
+        val = TAIL != kLanes || __builtin_amdgcn_inverse_ballot_w64(own[0]) ? dot : 0.f;
     }
 };
 
@@ -168,7 +180,7 @@ __device__ __forceinline__ bool group_lane_of(uint64_t mask, int lane_in_group) 
     return __builtin_amdgcn_inverse_ballot_w64((first_lanes << 16) - first_lanes);
 }
 
-template <int VEC, bool MAX, Scale SCALE, bool ALIGNED, bool WGRAD>
+template <int VEC, bool MAX, Scale SCALE, bool ALIGNED, Tail TAIL, bool WGRAD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) void accumulate_grad_rows_kernel(const GradRows p) {
     const int lane = lane_id(), l = lane & (kRowLanes - 1);
     if (WGRAD) {
@@ -215,15 +227,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
     const float inv_divisor = 1.f / p.divisor;
 
     // A lane at the end of a row that is no multiple of VEC, and the lanes behind it, take the last VEC
-    // columns (never columns of the next row): what they share with another lane they compute too
-    // and store alike, but it counts once in the dot products.
+    // columns (never columns of the next row); what they share with another lane counts there (see TAIL).
     const int fb = task.block * (kRowLanes * VEC) + l * VEC;
     const int f = min(fb, p.F - VEC);
     const uint32_t lane_bytes = (uint32_t)f * 4u, lane_col = (uint32_t)f + p.slot_shift;
     const uint32_t last_pair = (uint32_t)p.slot_bytes - 8u;
     float xo[VEC], xk[VEC], acc[VEC];
+    uint64_t own[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
+        own[e] = __builtin_amdgcn_ballot_w64(f + e >= fb);
         xo[e] = WGRAD && live && f + e >= fb ? p.feat[(size_t)m * p.F + f + e] : 0.f;
         xk[e] = SCALE == kScaled ? xo[e] : (float)((double)xo[e] * (1.0 / (double)p.divisor));
         acc[e] = 0.f;
@@ -274,7 +287,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
     };
     repeats = mark_repeats(en, 0);
 
-    Step<VEC, MAX, ALIGNED> st[2];
+    Step<VEC, MAX, ALIGNED, TAIL> st[2];
     st[0].template request_slots<0>(MS, en, lane_col, last_pair);
     st[1].template request_slots<2>(MS, en, lane_col, last_pair);
     st[0].template request_rows<0>(G, GX, en, lane_bytes);
@@ -294,11 +307,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
         __builtin_amdgcn_sched_barrier(0);                                                                                    \
         constexpr int kA = entry_lane((I) * 2), kB = entry_lane((I) * 2 + 1);                                                 \
         const float wa = group_bcast<kA>(en.w), wb = group_bcast<kB>(en.w);                                                   \
-        val[((I) & 1) * 2] = val[((I) & 1) * 2 + 1] = 0.f;                                                                    \
         st[(I) & 1].template add<0, SCALE, WGRAD>(wa, SCALE == kPow2 ? group_bcast<kA>(en.w_mean) : wa,                       \
-                                                  group_lane_of(repeats, kA) ? 0.f : wa, xo, xk, p.divisor, acc, val[((I) & 1) * 2]);    \
+                                                  group_lane_of(repeats, kA) ? 0.f : wa, xo, xk, own, p.divisor, acc, val[((I) & 1) * 2]);    \
         st[(I) & 1].template add<1, SCALE, WGRAD>(wb, SCALE == kPow2 ? group_bcast<kB>(en.w_mean) : wb,                       \
-                                                  group_lane_of(repeats, kB) ? 0.f : wb, xo, xk, p.divisor, acc, val[((I) & 1) * 2 + 1]); \
+                                                  group_lane_of(repeats, kB) ? 0.f : wb, xo, xk, own, p.divisor, acc, val[((I) & 1) * 2 + 1]); \
         if (WGRAD && ((I) & 1)) r[(I) >> 1] = group_sum_4(val, lane);                                                         \
         __builtin_amdgcn_sched_barrier(0);                                                                                    \
     }
@@ -323,19 +335,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
         en = next;
         repeats = next_repeats;
     }
-    if (live && fb < p.F) store_cols<VEC>(p.gfeat + (size_t)m * p.F + f, acc);
+    if (!live || fb >= p.F) return;
+    float *const out = p.gfeat + (size_t)m * p.F + f;
+    if (TAIL == kElements && f < fb) {
+#pragma unroll
+        for (int e = 1; e < VEC; ++e)
+            if (f + e >= fb) __builtin_nontemporal_store(acc[e], out + e);
+    } else {
+        store_cols<VEC>(out, acc);
+    }
 }
 
 template <int VEC, bool MAX, Scale SCALE, bool WGRAD>
 void launch_packed(const GradRows &p, hipStream_t s) {
     const dim3 grid(ceil_div((long long)p.n_vert * p.blocks, 256 / kRowLanes)), block(256);
-    if constexpr (MAX && VEC != 3) {
-        if (p.F % VEC == 0 && p.slot_shift == 0) {
-            accumulate_grad_rows_kernel<VEC, MAX, SCALE, true, WGRAD><<<grid, block, 0, s>>>(p);
-            return;
-        }
+#define HGC_ROWS(ALIGNED, TAIL) accumulate_grad_rows_kernel<VEC, MAX, SCALE, ALIGNED, TAIL, WGRAD><<<grid, block, 0, s>>>(p)
+    const bool full = p.F == kRowLanes * VEC * p.blocks, whole = p.F % VEC == 0;
+    if constexpr (VEC == 1) {  // rows of 16 features
+        HGC_ROWS(MAX, kFull);
+    } else if constexpr (MAX && VEC != 3) {
+        if (p.slot_shift != 0 || !whole) HGC_ROWS(false, kElements);  // (right for full lanes too)
+        else if (full) HGC_ROWS(true, kFull);
+        else HGC_ROWS(true, kLanes);
+    } else {
+        if (full) HGC_ROWS(false, kFull);
+        else if (whole) HGC_ROWS(false, kLanes);
+        else HGC_ROWS(false, kElements);
     }
-    accumulate_grad_rows_kernel<VEC, MAX, SCALE, false, WGRAD><<<grid, block, 0, s>>>(p);
+#undef HGC_ROWS
 }
 
 template <int VEC>

@@ -35,3 +35,43 @@ def test_empty_slots_of_wide_rows(oracle, F):
         assert np.isfinite(ref[1:]).all() and same(out.cpu().numpy(), ref)
         if mm:
             assert (arg.cpu().numpy() == rarg).all()
+
+
+def named_once(rng, n, K):
+    """K different neighbours a row, the vertex itself not among them"""
+    return np.stack([rng.permutation(np.delete(np.arange(n), v))[:K] for v in range(n)]).astype(np.int32)
+
+
+def close(got, ref, bound):
+    """non-finite values alike, finite ones within the bound"""
+    finite = np.isfinite(ref)
+    return same(got[~finite], ref[~finite]) and (np.abs(got[finite] - ref[finite]) <= bound[finite]).all()
+
+
+@pytest.mark.parametrize("F", [16, 17, 18, 22, 31, 33, 45, 50, 65, 66, 100, 127, 128])
+@pytest.mark.parametrize("mean_and_max", [True, False])
+def test_infinite_gradient_in_the_last_columns(oracle, F, mean_and_max):
+    """lanes beyond the end of a row hold the last columns again: what is infinite there counts once, and not times 0"""
+    from hgcalml_amd import ops  # noqa: F401
+    rng = np.random.default_rng(F)
+    n, K = 40, 7
+    idx = named_once(rng, n, K)
+    x = (rng.random((n, F)) + 0.5).astype(np.float32)
+    w = (rng.random((n, K)) + 0.5).astype(np.float32)
+    g = (rng.random((n, 2 * F if mean_and_max else F)) + 0.5).astype(np.float32)
+    g[::3, F - 1] = np.inf
+    other = np.arange(1, n, 3)
+    g[other, F - 2 - np.arange(len(other)) % 3] = -np.inf
+    if mean_and_max:
+        g[::4, 2 * F - 1] = np.inf
+        g[other, 2 * F - 1] = 1
+    _, arg = oracle.AccumulateLinKnn(w, x, idx, mean_and_max)
+    rgw, rgx = oracle.accumulate_knn_grad_kernel(g, w, x, idx, arg)
+    assert np.isinf(rgw).any() and not np.isnan(rgw).any()
+    tw, tx, ti = t(w).requires_grad_(True), t(x).requires_grad_(True), t(idx)
+    from hgcalml_amd import AccumulateLinKnn
+    gw, gx = torch.autograd.grad(AccumulateLinKnn(tw, tx, ti, mean_and_max)[0], [tw, tx], t(g))
+    # up to 2 F products below 2.25 and their sums in float32, in another order
+    bound = np.full(rgw.shape, (2 * F + 8) * 2.0 ** -24 * 4.5 * F)
+    assert close(gw.cpu().numpy(), rgw, bound)
+    assert same(gx.cpu().numpy(), rgx)
