@@ -105,17 +105,10 @@ struct Entries {
     float w, w_mean; // weight, and what the mean half is multiplied by
 };
 
-// What a lane holds of another lane's columns (rows that do not fill their lanes) must not reach the dot
-// products, whatever its value: 0 * infinity is no 0.
-//   kFull      every lane has VEC columns of its own
-//   kLanes     a lane has VEC columns of its own or none: its dot products are left out
-//   kElements  a lane may share some of its columns: these elements are taken as 0 and not stored either
-// own[e]: the lanes whose element e is theirs. (150,000 vertices, own features of 0 in their place and now:
-// K = 40, F = 22 178 and 177 us, F = 50 229 and 231; K = 16, F = 127 208 and 212.)
-enum Tail { kFull, kLanes, kElements };
-
 // Two entries on their way through the pipeline: arg-max slots (requested two steps ahead), gradient
-// rows (requested one step ahead, the max half by the slots), arithmetic.
+// rows (requested one step ahead, the max half by the slots), arithmetic. own[e]: the lanes whose element e
+// is theirs. (150,000 vertices, own features of 0 in the place of the others and now: K = 40, F = 22 178 and
+// 177 us, F = 50 229 and 231; K = 16, F = 127 208 and 212.)
 template <int VEC, bool MAX, bool ALIGNED, Tail TAIL>
 struct Step {
     SlotBytes<VEC, ALIGNED> sb[2];
@@ -350,16 +343,16 @@ template <int VEC, bool MAX, Scale SCALE, bool WGRAD>
 void launch_packed(const GradRows &p, hipStream_t s) {
     const dim3 grid(ceil_div((long long)p.n_vert * p.blocks, 256 / kRowLanes)), block(256);
 #define HGC_ROWS(ALIGNED, TAIL) accumulate_grad_rows_kernel<VEC, MAX, SCALE, ALIGNED, TAIL, WGRAD><<<grid, block, 0, s>>>(p)
-    const bool full = p.F == kRowLanes * VEC * p.blocks, whole = p.F % VEC == 0;
+    const Tail tail = row_tail(p.F, VEC, p.blocks);
     if constexpr (VEC == 1) {  // rows of 16 features
         HGC_ROWS(MAX, kFull);
     } else if constexpr (MAX && VEC != 3) {
-        if (p.slot_shift != 0 || !whole) HGC_ROWS(false, kElements);  // (right for full lanes too)
-        else if (full) HGC_ROWS(true, kFull);
+        if (p.slot_shift != 0 || tail == kElements) HGC_ROWS(false, kElements);  // (right for full lanes too)
+        else if (tail == kFull) HGC_ROWS(true, kFull);
         else HGC_ROWS(true, kLanes);
     } else {
-        if (full) HGC_ROWS(false, kFull);
-        else if (whole) HGC_ROWS(false, kLanes);
+        if (tail == kFull) HGC_ROWS(false, kFull);
+        else if (tail == kLanes) HGC_ROWS(false, kLanes);
         else HGC_ROWS(false, kElements);
     }
 #undef HGC_ROWS

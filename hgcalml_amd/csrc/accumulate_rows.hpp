@@ -244,6 +244,16 @@ inline void row_shape(int n_feat, int &vec, int &blocks) {
     vec = ceil_div(n_feat, kRowLanes * blocks);
 }
 
+// A lane at the end of a row that is no multiple of VEC, and the lanes behind it, hold the last VEC columns. What
+// they hold of another lane's columns must not reach a dot product, whatever its value: 0 * infinity is no 0.
+//   kFull      every lane has VEC columns of its own
+//   kLanes     a lane has VEC columns of its own or none: its share of the dot products is left out
+//   kElements  a lane may share some of its columns: these elements are left out one by one
+enum Tail { kFull, kLanes, kElements };
+inline Tail row_tail(int n_feat, int vec, int blocks) {
+    return n_feat == kRowLanes * vec * blocks ? kFull : n_feat % vec == 0 ? kLanes : kElements;
+}
+
 // A dense [rows, cols] matrix of 4-byte elements seen through a raw buffer
 // descriptor (stride 0, num_records = size in bytes, gfx9 data format word).
 struct RowMatrix {

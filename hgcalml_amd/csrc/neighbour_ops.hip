@@ -69,7 +69,7 @@ __global__ __launch_bounds__(256) void local_distance_kernel(const int *__restri
 // separate passes where 64 does not divide the columns: 60,000 vertices, K = 24, F = 48 97 -> 23 us;
 // 150,000, K = 64, F = 64 356 -> 125; 300,000, K = 64, F = 128 1346 -> 547; 200,000, K = 40, F = 256
 // 1169 -> 477 (on tables that need no order 65 -> 21, 322 -> 123, 700 -> 527, 498 -> 438).
-template <int VEC, int NB>
+template <int VEC, int NB, acc::Tail TAIL>
 __global__ __launch_bounds__(256) void push_grad_rows_kernel(const float *__restrict__ grad, const float *__restrict__ w,
                                                              const float *__restrict__ feat, const int *__restrict__ idx,
                                                              const int *__restrict__ order, float *__restrict__ feat_grad,
@@ -82,10 +82,11 @@ __global__ __launch_bounds__(256) void push_grad_rows_kernel(const float *__rest
     const int *irow = idx + (size_t)v * K;
     const float *wrow = w + (size_t)v * K;
     const __amdgpu_buffer_rsrc_t rows = make_rows(grad, (unsigned long long)n_vert * F * 4ull);
-    // A lane at the end of a row that is no multiple of VEC takes the last VEC columns; those it shares with its
-    // neighbour count in the neighbour's dot product only.
+    // Columns that a lane at the end of a row shares with its neighbour count in the neighbour's dot product only (see
+    // Tail; only the last block of a row has any). owned[e]: the lanes whose element e of that block is theirs.
     uint32_t lane_bytes[NB];
     float own[NB][VEC], sum[NB][VEC];
+    uint64_t owned[VEC];
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
         const int fb = (b * kRowLanes + l) * VEC, f = min(fb, F - VEC);
@@ -95,6 +96,7 @@ __global__ __launch_bounds__(256) void push_grad_rows_kernel(const float *__rest
             const float x = feat[(size_t)v * F + f + e];
             own[b][e] = f + e >= fb ? x : 0.f;
             sum[b][e] = 0.f;
+            if (b == NB - 1) owned[e] = __builtin_amdgcn_ballot_w64(f + e >= fb);
         }
     }
     const int mine = entry_lane(l);
@@ -125,10 +127,16 @@ __global__ __launch_bounds__(256) void push_grad_rows_kernel(const float *__rest
         HGC_PUSH_SLOT(Q, 3)                                                                                  \
         _Pragma("unroll") for (int u = 0; u < 4; ++u) {                                                      \
             val[u] = 0.f;                                                                                    \
-            _Pragma("unroll") for (int b = 0; b < NB; ++b) _Pragma("unroll") for (int e = 0; e < VEC; ++e) { \
-                val[u] = __builtin_fmaf(own[b][e], x[u][b][e], val[u]);                                      \
-                sum[b][e] = sum[b][e] + x[u][b][e] * ws[u];                                                  \
+            float before = 0.f;                                                                              \
+            _Pragma("unroll") for (int b = 0; b < NB; ++b) {                                                 \
+                if (b == NB - 1) before = val[u];                                                            \
+                _Pragma("unroll") for (int e = 0; e < VEC; ++e) {                                            \
+                    const bool counts = TAIL != kElements || b < NB - 1 || __builtin_amdgcn_inverse_ballot_w64(owned[e]);\
+                    val[u] = __builtin_fmaf(own[b][e], counts ? x[u][b][e] : 0.f, val[u]);                   \
+                    sum[b][e] = sum[b][e] + x[u][b][e] * ws[u];                                              \
+                }                                                                                            \
             }                                                                                                \
+            if (TAIL == kLanes) val[u] = __builtin_amdgcn_inverse_ballot_w64(owned[0]) ? val[u] : before;    \
         }                                                                                                    \
         r[Q] = group_sum_4(val, lane);                                                                       \
     }
@@ -155,10 +163,15 @@ int launch_push_grad_rows(const float *grad, const float *w, const float *feat, 
     if (F > 256 || (unsigned long long)n_vert * (unsigned long long)F * 4ull > kMaxRowBytes) return 1;
     int vec, nb;
     row_shape(F, vec, nb);
+    const Tail tail = row_tail(F, vec, nb);
     const dim3 grid(ceil_div(n_vert, 256 / kRowLanes)), block(256);
-#define HGC_PUSH_GRAD(VEC, NB)                                                                                         \
-    case VEC * 10 + NB:                                                                                                \
-        push_grad_rows_kernel<VEC, NB><<<grid, block, 0, s>>>(grad, w, feat, idx, order, feat_grad, w_grad, n_vert, K, F); \
+#define HGC_PUSH_TAIL(VEC, NB, TAIL) \
+    push_grad_rows_kernel<VEC, NB, TAIL><<<grid, block, 0, s>>>(grad, w, feat, idx, order, feat_grad, w_grad, n_vert, K, F)
+#define HGC_PUSH_GRAD(VEC, NB)                                   \
+    case VEC * 10 + NB:                                          \
+        if (tail == kFull) HGC_PUSH_TAIL(VEC, NB, kFull);        \
+        else if (tail == kLanes) HGC_PUSH_TAIL(VEC, NB, kLanes); \
+        else HGC_PUSH_TAIL(VEC, NB, kElements);                  \
         break
     switch (vec * 10 + nb) {
         HGC_PUSH_GRAD(1, 1);
@@ -173,6 +186,7 @@ int launch_push_grad_rows(const float *grad, const float *w, const float *feat, 
         default: return 1;
     }
 #undef HGC_PUSH_GRAD
+#undef HGC_PUSH_TAIL
     return check_launch("push_grad_rows_kernel");
 }
 

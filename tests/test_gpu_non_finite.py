@@ -75,3 +75,27 @@ def test_infinite_gradient_in_the_last_columns(oracle, F, mean_and_max):
     bound = np.full(rgw.shape, (2 * F + 8) * 2.0 ** -24 * 4.5 * F)
     assert close(gw.cpu().numpy(), rgw, bound)
     assert same(gx.cpu().numpy(), rgx)
+
+
+@pytest.mark.parametrize("F", [1, 5, 16, 17, 22, 31, 48, 50, 64, 65, 100, 127, 129, 150, 193, 255, 256])
+def test_infinite_push_gradient_in_the_last_columns(F):
+    from hgcalml_amd import ops  # noqa: F401
+    rng = np.random.default_rng(200 + F)
+    n, K = 40, 7
+    idx = named_once(rng, n, K)
+    idx[5, 2:] = -1
+    x = (rng.random((n, F)) + 0.5).astype(np.float32)
+    w = (rng.random((n, K)) + 0.5).astype(np.float32)
+    g = (rng.random((n, F)) + 0.5).astype(np.float32)
+    g[::3, F - 1] = np.inf
+    other = np.arange(1, n, 3)
+    g[other, np.maximum(F - 2 - np.arange(len(other)) % 3, 0)] = -np.inf
+    rows = np.where((idx < 0)[..., None], 0, g[idx]).astype(np.float64)
+    want_w = (rows * x[:, None, :]).sum(-1)
+    with np.errstate(invalid="ignore"):
+        want_x = (rows * w[..., None]).sum(1)
+    assert np.isinf(want_w).any() and not np.isnan(want_w).any()
+    gw, gx = torch.ops.hgcalml.push_knn_grad(t(g), t(w), t(x), t(idx))
+    # sums of F (K) products below 2.25
+    assert close(gw.cpu().numpy(), want_w, np.full(want_w.shape, (F + 8) * 2.0 ** -24 * 2.25 * F))
+    assert close(gx.cpu().numpy(), want_x, np.full(want_x.shape, (K + 8) * 2.0 ** -24 * 2.25 * K))
