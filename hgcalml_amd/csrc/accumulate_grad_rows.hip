@@ -143,9 +143,8 @@ struct Step {
         request_row<1>(G, GX, group_bcast<entry_lane(E + 1)>(en.row) + lane_bytes, group_bcast<entry_lane(E + 1)>(en.key));
     }
     // An entry beyond its list reads zeros and has weight 0: it adds 0 to a sum that started at +0.
-    // w_max: 0 in the lanes of repeated self references, whose max part counts for the weight gradient only.
     template <int U, Scale SCALE, bool WGRAD>
-    __device__ __forceinline__ void add(float w, float w_mean, float w_max, const float (&xo)[VEC], const float (&xk)[VEC],
+    __device__ __forceinline__ void add(float w, float w_mean, const float (&xo)[VEC], const float (&xk)[VEC],
                                         const uint64_t (&own)[VEC], float divisor, float (&acc)[VEC], float &val) const {
         float dot = 0.f;
 #pragma unroll
@@ -157,7 +156,7 @@ struct Step {
                 const uint64_t here = TAIL == kElements ? hit[U][e] & own[e] : hit[U][e];
                 const float gsel = VEC == 1 ? gx[U][e] : __builtin_amdgcn_inverse_ballot_w64(here) ? gx[U][e] : 0.f;
                 if (WGRAD) dot = __builtin_fmaf(gsel, xo[e], dot);
-                const float part_max = gsel * w_max;
+                const float part_max = gsel * w;
                 const float sum = part + part_max;
                 acc[e] = acc[e] + sum;
             } else {
@@ -167,11 +166,6 @@ struct Step {
         val = TAIL != kLanes || __builtin_amdgcn_inverse_ballot_w64(own[0]) ? dot : 0.f;
     }
 };
-
-__device__ __forceinline__ bool group_lane_of(uint64_t mask, int lane_in_group) {
-    const uint64_t first_lanes = (mask >> lane_in_group) & 0x0001000100010001ull;
-    return __builtin_amdgcn_inverse_ballot_w64((first_lanes << 16) - first_lanes);
-}
 
 template <int VEC, bool MAX, Scale SCALE, bool ALIGNED, Tail TAIL, bool WGRAD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) void accumulate_grad_rows_kernel(const GradRows p) {
@@ -258,27 +252,31 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
     int slot_next = kRowLanes < mine ? list[kRowLanes] : 0;
     Entries en = entries_of(slot, 0);
     set_weight(en, weight_of(en));
-    int self_key = 0;
+    // Entries that name the target itself: the first one (lowest slot) carries the max part. Later ones (padding by
+    // repeated self references) have a slot that no maximum names; the weight gradient counts the maxima of the
+    // first one for them too, on the same gradient row: theirs is the dot product of the first.
+    constexpr uint32_t kNoSlot = 0x1ff;
+    struct Selves {
+        uint64_t first, repeats;  // lanes whose entry is one
+    };
     bool self_seen = false;
-    uint64_t repeats = 0;
-    // Entries that name the target itself: the first one (lowest slot) carries the max part; later ones
-    // (padding by repeated self references) are compared with that slot too, for the weight gradient.
-    auto mark_repeats = [&](Entries &e, int c0) {
-        uint64_t rep = 0;
+    auto mark_selves = [&](Entries &e, int c0) {
+        Selves s{0, 0};
         if (MAX) {
             const bool self = c0 < mine && e.row == (uint32_t)m * (uint32_t)(p.pitch * 4);
             if (__builtin_amdgcn_ballot_w64(self)) {
                 const int lowest = group_min(self ? (int)e.key : 1 << 30);
-                if (!self_seen && lowest < (1 << 30)) self_key = lowest;
-                const bool repeat = self && (self_seen || (int)e.key != self_key);
-                rep = __builtin_amdgcn_ballot_w64(repeat);
-                if (repeat) e.key = (uint32_t)self_key;
+                const bool first = self && !self_seen && (int)e.key == lowest;
+                s.first = __builtin_amdgcn_ballot_w64(first);
+                s.repeats = __builtin_amdgcn_ballot_w64(self && !first);
+                if (self && !first) e.key = kNoSlot;
                 self_seen = self_seen || lowest < (1 << 30);
             }
         }
-        return rep;
+        return s;
     };
-    repeats = mark_repeats(en, 0);
+    Selves selves = mark_selves(en, 0);
+    float self_dot = 0.f;
 
     Step<VEC, MAX, ALIGNED, TAIL> st[2];
     st[0].template request_slots<0>(MS, en, lane_col, last_pair);
@@ -289,7 +287,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
         Entries next = entries_of(slot_next, c0 + kRowLanes);
         const float w_next = weight_of(next);
         set_weight(next, 0.f);
-        const uint64_t next_repeats = mark_repeats(next, c0 + kRowLanes);
+        const Selves next_selves = mark_selves(next, c0 + kRowLanes);
         float r[4] = {0.f, 0.f, 0.f, 0.f}, val[4];
         // step I: rows of step I + 1 and slots of step I + 2 are requested, then step I is added up
 #define HGC_STEP(I)                                                                                                           \
@@ -300,10 +298,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
         __builtin_amdgcn_sched_barrier(0);                                                                                    \
         constexpr int kA = entry_lane((I) * 2), kB = entry_lane((I) * 2 + 1);                                                 \
         const float wa = group_bcast<kA>(en.w), wb = group_bcast<kB>(en.w);                                                   \
-        st[(I) & 1].template add<0, SCALE, WGRAD>(wa, SCALE == kPow2 ? group_bcast<kA>(en.w_mean) : wa,                       \
-                                                  group_lane_of(repeats, kA) ? 0.f : wa, xo, xk, own, p.divisor, acc, val[((I) & 1) * 2]);    \
-        st[(I) & 1].template add<1, SCALE, WGRAD>(wb, SCALE == kPow2 ? group_bcast<kB>(en.w_mean) : wb,                       \
-                                                  group_lane_of(repeats, kB) ? 0.f : wb, xo, xk, own, p.divisor, acc, val[((I) & 1) * 2 + 1]); \
+        st[(I) & 1].template add<0, SCALE, WGRAD>(wa, SCALE == kPow2 ? group_bcast<kA>(en.w_mean) : wa, xo, xk, own, p.divisor,  \
+                                                  acc, val[((I) & 1) * 2]);                                                   \
+        st[(I) & 1].template add<1, SCALE, WGRAD>(wb, SCALE == kPow2 ? group_bcast<kB>(en.w_mean) : wb, xo, xk, own, p.divisor,  \
+                                                  acc, val[((I) & 1) * 2 + 1]);                                               \
         if (WGRAD && ((I) & 1)) r[(I) >> 1] = group_sum_4(val, lane);                                                         \
         __builtin_amdgcn_sched_barrier(0);                                                                                    \
     }
@@ -322,11 +320,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
         if (WGRAD) {
             float sum = (l & 2) ? ((l & 1) ? r[3] : r[2]) : ((l & 1) ? r[1] : r[0]);
             if (p.blocks == 2) sum = sum + __shfl_xor(sum, kRowLanes, kWave);  // the other half of the row
+            if (MAX && selves.first) {
+                const uint32_t in_group = (uint32_t)(selves.first >> (lane & 48)) & 0xffffu;
+                const float dot = __shfl(sum, (lane & 48) + __builtin_ctz(in_group | 0x10000u), kWave);
+                self_dot = in_group ? dot : self_dot;
+            }
+            if (MAX && selves.repeats) sum = __builtin_amdgcn_inverse_ballot_w64(selves.repeats) ? self_dot : sum;
             if (en.slot >= 0 && task.block == 0) p.gw[en.slot] = p.negate ? -(sum * en.w) : sum;
         }
         slot_next = slot_after;
         en = next;
-        repeats = next_repeats;
+        selves = next_selves;
     }
     if (!live || fb >= p.F) return;
     float *const out = p.gfeat + (size_t)m * p.F + f;

@@ -99,3 +99,29 @@ def test_infinite_push_gradient_in_the_last_columns(F):
     # sums of F (K) products below 2.25
     assert close(gw.cpu().numpy(), want_w, np.full(want_w.shape, (F + 8) * 2.0 ** -24 * 2.25 * F))
     assert close(gx.cpu().numpy(), want_x, np.full(want_x.shape, (K + 8) * 2.0 ** -24 * 2.25 * K))
+
+
+@pytest.mark.parametrize("F", [16, 22, 64, 100])
+def test_infinite_gradient_of_a_maximum_at_repeated_self_references(oracle, F):
+    """rows padded with the vertex itself: the max part of the feature gradient counts once, the weight gradient of every one
+    of these slots has it"""
+    from hgcalml_amd import AccumulateLinKnn
+    rng = np.random.default_rng(100 + F)
+    n, K = 40, 37
+    idx = named_once(rng, n, K)
+    idx[:, 3:6] = np.arange(n)[:, None]
+    idx[::2, 20:] = np.arange(n)[::2, None]   # over the borders of 16 entries
+    x = (rng.random((n, F)) + 0.5).astype(np.float32)
+    w = (rng.random((n, K)) + 0.5).astype(np.float32)
+    w[:, 3:6] = 3.0
+    w[::2, 20:] = 3.0
+    g = (rng.random((n, 2 * F)) + 0.5).astype(np.float32)
+    g[::3, F:] = np.inf
+    _, arg = oracle.AccumulateLinKnn(w, x, idx, True)
+    assert (arg == np.arange(n)[:, None]).mean() > 0.1
+    rgw, rgx = oracle.accumulate_knn_grad_kernel(g, w, x, idx, arg)
+    assert np.isinf(rgx).any() and not np.isnan(rgx).any() and not np.isnan(rgw).any()
+    tw, tx = t(w).requires_grad_(True), t(x).requires_grad_(True)
+    gw, gx = torch.autograd.grad(AccumulateLinKnn(tw, tx, t(idx), True)[0], [tw, tx], t(g))
+    assert close(gw.cpu().numpy(), rgw, np.full(rgw.shape, (2 * F + 8) * 2.0 ** -24 * 4.5 * F))
+    assert same(gx.cpu().numpy(), rgx)
