@@ -59,15 +59,11 @@ struct GradRows {
     bool negate;  // gw receives -(gradient * w): the chain rule through w = exp(-d)
 };
 
-// Does byte E of `packed` equal `key`? One SDWA compare.
+// Does byte E of `packed` equal `key`? The compiler makes one SDWA compare of it, and keeps the wait states between
+// a compare and a vector use of its mask.
 template <int E>
 __device__ __forceinline__ uint64_t byte_is(uint32_t packed, uint32_t key) {
-    uint64_t mask;
-    if constexpr (E == 0) asm("v_cmp_eq_u32_sdwa %0, %1, %2 src0_sel:BYTE_0 src1_sel:DWORD" : "=s"(mask) : "v"(packed), "v"(key));
-    else if constexpr (E == 1) asm("v_cmp_eq_u32_sdwa %0, %1, %2 src0_sel:BYTE_1 src1_sel:DWORD" : "=s"(mask) : "v"(packed), "v"(key));
-    else if constexpr (E == 2) asm("v_cmp_eq_u32_sdwa %0, %1, %2 src0_sel:BYTE_2 src1_sel:DWORD" : "=s"(mask) : "v"(packed), "v"(key));
-    else asm("v_cmp_eq_u32_sdwa %0, %1, %2 src0_sel:BYTE_3 src1_sel:DWORD" : "=s"(mask) : "v"(packed), "v"(key));
-    return mask;
+    return __builtin_amdgcn_ballot_w64(((packed >> (8 * E)) & 255u) == key);
 }
 
 // Arg-max slots of VEC features, packed in one word. ALIGNED: they start on a multiple of VEC (1, 2 or 4)
