@@ -98,14 +98,17 @@ __global__ __launch_bounds__(kGradWaves *kWave) void knn_grad_kernel(const float
     // chunk is added up.
     int k_next[kPairs];
     float g_next[kPairs], x_next[kPairs][C];
+    uint64_t counts[kPairs];  // lanes whose pair has a neighbour; the others hand over 0 (inf - inf is no 0)
     auto hand_over = [&](bool own) {  // own: neighbour minus vertex, otherwise vertex minus namer
         wave_lds_fence();
 #pragma unroll
         for (int p = 0; p < kPairs; ++p) {
             const int v = p * (kWave / kChunk) + lane / kChunk;
 #pragma unroll
-            for (int c = 0; c < C; ++c)
-                diff[v * kRow + s * kLanes + c] = own ? x_next[p][c] - x[p][c] : x[p][c] - x_next[p][c];
+            for (int c = 0; c < C; ++c) {
+                const float d = own ? x_next[p][c] - x[p][c] : x[p][c] - x_next[p][c];
+                diff[v * kRow + s * kLanes + c] = __builtin_amdgcn_inverse_ballot_w64(counts[p]) ? d : 0.f;
+            }
             grad[v * (kChunk + 1) + s] = 2.f * g_next[p];
         }
         wave_lds_fence();
@@ -118,6 +121,7 @@ __global__ __launch_bounds__(kGradWaves *kWave) void knn_grad_kernel(const float
 #pragma unroll
         for (int p = 0; p < kPairs; ++p) {
             const bool ok = (uint32_t)k_next[p] < (uint32_t)n_vert;
+            counts[p] = __builtin_amdgcn_ballot_w64(ok);
             const size_t at = (size_t)max(vertex[p], 0) * K + min(n0 + s, K - 1);
             g_next[p] = ok ? grad_a[at] : 0.f;
             if (grad_b) g_next[p] = ok ? g_next[p] + grad_b[at] : 0.f;
@@ -132,6 +136,7 @@ __global__ __launch_bounds__(kGradWaves *kWave) void knn_grad_kernel(const float
 #pragma unroll
         for (int p = 0; p < kPairs; ++p) {
             const bool ok = k_next[p] >= 0;
+            counts[p] = __builtin_amdgcn_ballot_w64(ok);
             g_next[p] = ok ? grad_a[k_next[p]] : 0.f;
             if (grad_b) g_next[p] = ok ? g_next[p] + grad_b[k_next[p]] : 0.f;
             load_row<C>(coord, ok ? fast_div(k_next[p], div_k) : max(vertex[p], 0), x_next[p]);

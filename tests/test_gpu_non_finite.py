@@ -125,3 +125,22 @@ def test_infinite_gradient_of_a_maximum_at_repeated_self_references(oracle, F):
     gw, gx = torch.autograd.grad(AccumulateLinKnn(tw, tx, t(idx), True)[0], [tw, tx], t(g))
     assert close(gw.cpu().numpy(), rgw, np.full(rgw.shape, (2 * F + 8) * 2.0 ** -24 * 4.5 * F))
     assert same(gx.cpu().numpy(), rgx)
+
+
+@pytest.mark.parametrize("C", [1, 2, 3, 4, 5, 8, 9, 12])
+def test_distance_gradient_of_vertices_that_lie_nowhere(oracle, C):
+    """slots without a neighbour and the places behind a row or list count nothing, also where the vertex's own coordinates are
+    infinite or NaN"""
+    from hgcalml_amd import ops  # noqa: F401
+    rng = np.random.default_rng(300 + C)
+    n, K = 50, 19
+    idx = named_once(rng, n, K)
+    idx[idx >= 45] = -1        # nobody names the last five vertices
+    idx[45:] = -1              # and they name nobody
+    x = rng.standard_normal((n, C)).astype(np.float32)
+    x[45], x[46], x[47, C - 1] = np.inf, np.nan, -np.inf
+    g = rng.standard_normal((n, K)).astype(np.float32)
+    ref = oracle.select_knn_grad_kernel(g, idx, x)
+    assert np.isfinite(ref).all() and not ref[45:].any()
+    got = torch.ops.hgcalml.select_knn_grad(t(g), t(idx), t(np.zeros_like(g)), t(x))
+    assert same(got.cpu().numpy(), ref)
