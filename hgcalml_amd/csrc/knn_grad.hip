@@ -46,16 +46,14 @@ __device__ __forceinline__ void load_row(const float *__restrict__ coord, int ro
     }
 }
 
-// grad_b (may be null): a second gradient of the distances, added to the first. Results in rows of out_pitch.
 template <int C>
-__global__ __launch_bounds__(kGradWaves *kWave) void knn_grad_kernel(const float *__restrict__ grad_a,
-                                                                    const float *__restrict__ grad_b,
+__global__ __launch_bounds__(kGradWaves *kWave) void knn_grad_kernel(const float *__restrict__ grad_dist,
                                                                     const int *__restrict__ idx,
                                                                     const float *__restrict__ coord,
                                                                     const int *__restrict__ inv_off,
                                                                     const int *__restrict__ inv_slots,
-                                                                    float *__restrict__ out, int out_pitch, int n_vert,
-                                                                    int K, const FastDiv div_k,
+                                                                    float *__restrict__ out, int n_vert, int K,
+                                                                    const FastDiv div_k,
                                                                     const int *__restrict__ order) {
     constexpr int kLanes = C <= 4 ? 4 : 8;          // lanes per vertex
     constexpr int kVertices = kWave / kLanes;       // per wave
@@ -123,8 +121,7 @@ __global__ __launch_bounds__(kGradWaves *kWave) void knn_grad_kernel(const float
             const bool ok = (uint32_t)k_next[p] < (uint32_t)n_vert;
             counts[p] = __builtin_amdgcn_ballot_w64(ok);
             const size_t at = (size_t)max(vertex[p], 0) * K + min(n0 + s, K - 1);
-            g_next[p] = ok ? grad_a[at] : 0.f;
-            if (grad_b) g_next[p] = ok ? g_next[p] + grad_b[at] : 0.f;
+            g_next[p] = ok ? grad_dist[at] : 0.f;
             load_row<C>(coord, ok ? k_next[p] : max(vertex[p], 0), x_next[p]);
         }
     };
@@ -137,8 +134,7 @@ __global__ __launch_bounds__(kGradWaves *kWave) void knn_grad_kernel(const float
         for (int p = 0; p < kPairs; ++p) {
             const bool ok = k_next[p] >= 0;
             counts[p] = __builtin_amdgcn_ballot_w64(ok);
-            g_next[p] = ok ? grad_a[k_next[p]] : 0.f;
-            if (grad_b) g_next[p] = ok ? g_next[p] + grad_b[k_next[p]] : 0.f;
+            g_next[p] = ok ? grad_dist[k_next[p]] : 0.f;
             load_row<C>(coord, ok ? fast_div(k_next[p], div_k) : max(vertex[p], 0), x_next[p]);
         }
     };
@@ -177,18 +173,17 @@ __global__ __launch_bounds__(kGradWaves *kWave) void knn_grad_kernel(const float
     const int r = r0 + cv;
     if (cc < C && r < n_vert) {
         const int i = order ? order[r] : r;
-        if ((uint32_t)i < (uint32_t)n_vert) out[(size_t)i * out_pitch + cc] = sum;
+        if ((uint32_t)i < (uint32_t)n_vert) out[(size_t)i * C + cc] = sum;
     }
 }
 
 // more than 8 coordinates: one thread per coordinate
-__global__ __launch_bounds__(256) void knn_grad_wide_kernel(const float *__restrict__ grad_a,
-                                                            const float *__restrict__ grad_b,
+__global__ __launch_bounds__(256) void knn_grad_wide_kernel(const float *__restrict__ grad_dist,
                                                             const int *__restrict__ idx,
                                                             const float *__restrict__ coord,
                                                             const int *__restrict__ inv_off,
                                                             const int *__restrict__ inv_slots, float *__restrict__ out,
-                                                            int out_pitch, int n_vert, int K, int C,
+                                                            int n_vert, int K, int C,
                                                             const FastDiv div_k, const int *__restrict__ order) {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const int r = (int)(t / C);
@@ -197,34 +192,32 @@ __global__ __launch_bounds__(256) void knn_grad_wide_kernel(const float *__restr
     const int i = order ? order[r] : r;
     if ((uint32_t)i >= (uint32_t)n_vert) return;
     const float xi = coord[(size_t)i * C + c];
-    auto gradient = [&](size_t at) { return grad_b ? grad_a[at] + grad_b[at] : grad_a[at]; };
     float sum = 0.f;
     for (int n = 0; n < K; ++n) {
         const size_t at = (size_t)i * K + n;
         const int k = idx[at];
         if ((uint32_t)k >= (uint32_t)n_vert) continue;
         const float diff = coord[(size_t)k * C + c] - xi;
-        sum = __builtin_fmaf(-2.f * gradient(at), diff, sum);
+        sum = __builtin_fmaf(-2.f * grad_dist[at], diff, sum);
     }
     for (int e = inv_off[i]; e < inv_off[i + 1]; ++e) {
         const int slot = inv_slots[e];
         const float diff = xi - coord[(size_t)fast_div(slot, div_k) * C + c];
-        const float add = 2.f * gradient(slot) * diff;
+        const float add = 2.f * grad_dist[slot] * diff;
         sum = sum + add;
     }
-    out[(size_t)i * out_pitch + c] = sum;
+    out[(size_t)i * C + c] = sum;
 }
 
 }  // namespace
 
-int launch_knn_grad(const float *grad_a, const float *grad_b, const int *idx, const float *coord, const int *inv_off,
-                    const int *inv_slots, const int *order, float *out, int out_pitch, int n_vert, int K, int C,
-                    hipStream_t s) {
+int launch_knn_grad(const float *grad_dist, const int *idx, const float *coord, const int *inv_off, const int *inv_slots,
+                    const int *order, float *out, int n_vert, int K, int C, hipStream_t s) {
     const FastDiv div_k = make_fast_div(K);
 #define HGC_KNN_GRAD(N)                                                                                              \
     case N:                                                                                                          \
         knn_grad_kernel<N><<<ceil_div(n_vert, kGradWaves * kWave / (N <= 4 ? 4 : 8)), kGradWaves * kWave, 0, s>>>(   \
-            grad_a, grad_b, idx, coord, inv_off, inv_slots, out, out_pitch, n_vert, K, div_k, order);                \
+            grad_dist, idx, coord, inv_off, inv_slots, out, n_vert, K, div_k, order);                                \
         break
     switch (C) {
         HGC_KNN_GRAD(1);
@@ -237,8 +230,8 @@ int launch_knn_grad(const float *grad_a, const float *grad_b, const int *idx, co
         HGC_KNN_GRAD(8);
         default: {
             const long long threads = (long long)n_vert * C;
-            knn_grad_wide_kernel<<<ceil_div(threads, 256), 256, 0, s>>>(grad_a, grad_b, idx, coord, inv_off, inv_slots, out,
-                                                                       out_pitch, n_vert, K, C, div_k, order);
+            knn_grad_wide_kernel<<<ceil_div(threads, 256), 256, 0, s>>>(grad_dist, idx, coord, inv_off, inv_slots, out, n_vert,
+                                                                       K, C, div_k, order);
         }
     }
 #undef HGC_KNN_GRAD
@@ -260,8 +253,8 @@ int hgc_select_knn_grad_ordered(const float *d_grad_dist, const int *d_indices, 
     HGC_REQUIRE((long long)n_vert * std::max(n_neigh, n_coords) < (1ll << 31), "tensor too large for int32 indexing");
     if (n_vert == 0) return HGC_OK;
     HGC_REQUIRE(d_grad_dist && d_indices && d_coord && d_inv_offsets && d_inv_slots && d_grad_coord, "null pointer");
-    return launch_knn_grad(d_grad_dist, nullptr, d_indices, d_coord, d_inv_offsets, d_inv_slots, d_vertex_order, d_grad_coord,
-                           n_coords, n_vert, n_neigh, n_coords, as_stream(stream));
+    return launch_knn_grad(d_grad_dist, d_indices, d_coord, d_inv_offsets, d_inv_slots, d_vertex_order, d_grad_coord, n_vert,
+                           n_neigh, n_coords, as_stream(stream));
 }
 
 int hgc_select_knn_grad(const float *d_grad_dist, const int *d_indices, const float *d_dist, const float *d_coord,
