@@ -177,7 +177,8 @@ __global__ __launch_bounds__(kGradWaves *kWave) void knn_grad_kernel(const float
     }
 }
 
-// more than 8 coordinates: one thread per coordinate
+// More than 8 coordinates: one thread per coordinate. The loads of eight slots (list entries) are issued together; the
+// additions stay in their order.
 __global__ __launch_bounds__(256) void knn_grad_wide_kernel(const float *__restrict__ grad_dist,
                                                             const int *__restrict__ idx,
                                                             const float *__restrict__ coord,
@@ -192,19 +193,49 @@ __global__ __launch_bounds__(256) void knn_grad_wide_kernel(const float *__restr
     const int i = order ? order[r] : r;
     if ((uint32_t)i >= (uint32_t)n_vert) return;
     const float xi = coord[(size_t)i * C + c];
+    constexpr int U = 8;
     float sum = 0.f;
-    for (int n = 0; n < K; ++n) {
-        const size_t at = (size_t)i * K + n;
-        const int k = idx[at];
-        if ((uint32_t)k >= (uint32_t)n_vert) continue;
-        const float diff = coord[(size_t)k * C + c] - xi;
-        sum = __builtin_fmaf(-2.f * grad_dist[at], diff, sum);
+    for (int n0 = 0; n0 < K; n0 += U) {
+        int k[U];
+        float g[U], x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const size_t at = (size_t)i * K + min(n0 + u, K - 1);
+            k[u] = idx[at];
+            g[u] = grad_dist[at];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool ok = n0 + u < K && (uint32_t)k[u] < (uint32_t)n_vert;
+            k[u] = ok ? k[u] : -1;
+            x[u] = coord[(size_t)(ok ? k[u] : i) * C + c];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (k[u] < 0) continue;
+            const float diff = x[u] - xi;
+            sum = __builtin_fmaf(-2.f * g[u], diff, sum);
+        }
     }
-    for (int e = inv_off[i]; e < inv_off[i + 1]; ++e) {
-        const int slot = inv_slots[e];
-        const float diff = xi - coord[(size_t)fast_div(slot, div_k) * C + c];
-        const float add = 2.f * grad_dist[slot] * diff;
-        sum = sum + add;
+    const int begin = inv_off[i], count = inv_off[i + 1] - begin;
+    const int *const list = inv_slots + begin;
+    for (int e0 = 0; e0 < count; e0 += U) {
+        int slot[U];
+        float g[U], x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) slot[u] = list[min(e0 + u, count - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            g[u] = grad_dist[slot[u]];
+            x[u] = coord[(size_t)fast_div(slot[u], div_k) * C + c];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (e0 + u >= count) break;
+            const float diff = xi - x[u];
+            const float add = 2.f * g[u] * diff;
+            sum = sum + add;
+        }
     }
     out[(size_t)i * C + c] = sum;
 }
