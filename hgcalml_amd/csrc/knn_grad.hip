@@ -8,7 +8,8 @@
 // every term rounded into the float sum one after the other. The reference's `2. * g * (x_k - x_i)` is exact in
 // double; subtracted from the sum there and rounded to float it is a fused multiply-add (apart from
 // roundings that the double subtraction moves onto the middle between two floats, one in 2^29), rounded to
-// float and added it is a float product and a float sum.
+// float and added it is a float product and a float sum. The factor 2 goes to the difference: coordinates whose
+// differences it could take beyond the largest float have infinite distances, a gradient may be that large.
 //
 // Both sums are chains, so a lane owns one coordinate of one vertex and walks its slots and list entries
 // serially; what it walks over is fetched by the wave together: 16 slots (entries) of its 16 vertices (8
@@ -105,9 +106,9 @@ __global__ __launch_bounds__(kGradWaves *kWave) void knn_grad_kernel(const float
 #pragma unroll
             for (int c = 0; c < C; ++c) {
                 const float d = own ? x_next[p][c] - x[p][c] : x[p][c] - x_next[p][c];
-                diff[v * kRow + s * kLanes + c] = __builtin_amdgcn_inverse_ballot_w64(counts[p]) ? d : 0.f;
+                diff[v * kRow + s * kLanes + c] = __builtin_amdgcn_inverse_ballot_w64(counts[p]) ? 2.f * d : 0.f;
             }
-            grad[v * (kChunk + 1) + s] = 2.f * g_next[p];
+            grad[v * (kChunk + 1) + s] = g_next[p];
         }
         wave_lds_fence();
     };
@@ -214,7 +215,7 @@ __global__ __launch_bounds__(256) void knn_grad_wide_kernel(const float *__restr
         for (int u = 0; u < U; ++u) {
             if (k[u] < 0) continue;
             const float diff = x[u] - xi;
-            sum = __builtin_fmaf(-2.f * g[u], diff, sum);
+            sum = __builtin_fmaf(-g[u], 2.f * diff, sum);
         }
     }
     const int begin = inv_off[i], count = inv_off[i + 1] - begin;
@@ -233,7 +234,7 @@ __global__ __launch_bounds__(256) void knn_grad_wide_kernel(const float *__restr
         for (int u = 0; u < U; ++u) {
             if (e0 + u >= count) break;
             const float diff = xi - x[u];
-            const float add = 2.f * g[u] * diff;
+            const float add = g[u] * (2.f * diff);
             sum = sum + add;
         }
     }

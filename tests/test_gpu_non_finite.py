@@ -144,3 +144,20 @@ def test_distance_gradient_of_vertices_that_lie_nowhere(oracle, C):
     assert np.isfinite(ref).all() and not ref[45:].any()
     got = torch.ops.hgcalml.select_knn_grad(t(g), t(idx), t(np.zeros_like(g)), t(x))
     assert same(got.cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("C", [1, 3, 4, 7, 9])
+def test_distance_gradient_of_the_largest_gradients(oracle, C):
+    """twice such a gradient is beyond the largest float, times the difference of two coordinates it is not"""
+    from hgcalml_amd import ops  # noqa: F401
+    rng = np.random.default_rng(400 + C)
+    n, K = 60, 5
+    idx = named_once(rng, n, K)
+    x = (rng.random((n, C)) * 1e-3).astype(np.float32)
+    x[1] = x[0]
+    idx[0, 1] = 1              # a difference of 0
+    g = (rng.choice([-1, 1], (n, K)) * np.float32(3e38)).astype(np.float32)
+    ref = oracle.select_knn_grad_kernel(g, idx, x)
+    assert np.isfinite(ref).all() and np.abs(ref).max() > 1e34
+    got = torch.ops.hgcalml.select_knn_grad(t(g), t(idx), t(np.zeros_like(g)), t(x))
+    assert same(got.cpu().numpy(), ref)
