@@ -35,7 +35,7 @@ int launch_accumulate_grad_fused(const float *g, const float *w, const float *fe
                                  const int *order, float divisor, hipStream_t s);
 // accumulate_grad_rows.hip: rows of 16 to 128 features; returns 1 when the shape is not covered. gw == nullptr:
 // feature gradient only. negate: gw receives -(gradient * w). scratch may be null.
-size_t accumulate_grad_rows_scratch_bytes(int n_vert, int n_feat, int g_cols, float divisor);
+size_t accumulate_grad_rows_scratch_bytes(int n_vert, int n_feat, int n_neigh, bool mean_and_max, float divisor);
 bool accumulate_grad_rows_covers(int n_feat, int n_neigh, bool mean_and_max, bool slots, unsigned long long g_bytes);
 int launch_accumulate_grad_rows(const float *g, const float *w, const float *feat, const unsigned char *maxslot,
                                 const int *inv_off, const int *inv_slots, float *gw, float *gfeat, int n_vert, int K, int F,
@@ -1145,7 +1145,7 @@ int hgc_accumulate_knn_grad_slots(const float *d_grad_from_out_features, const f
 }
 
 size_t hgc_accumulate_knn_grad_scratch_bytes(int n_vert, int n_neigh, int n_feat, int mean_and_max) {
-    return accumulate_grad_rows_scratch_bytes(n_vert, n_feat, n_feat * (mean_and_max ? 2 : 1), (float)n_neigh);
+    return accumulate_grad_rows_scratch_bytes(n_vert, n_feat, n_neigh, mean_and_max != 0, (float)n_neigh);
 }
 
 int hgc_accumulate_knn_grad_scratch(const float *d_grad_from_out_features, const float *d_distances, const float *d_feat,

@@ -30,6 +30,8 @@
 // time move through a pipeline: slots two steps ahead, rows one step ahead, arithmetic.
 // The dot products of four entries are reduced across the 16 lanes by a transposing exchange (three
 // instructions per value with DPP).
+#include <algorithm>
+
 #include "accumulate_rows.hpp"
 
 namespace hgc {
@@ -40,12 +42,12 @@ using namespace acc;
 
 // How the mean part (g / divisor) * w is formed with the bits of the two operations:
 //   kPow2    divisor a power of two: g * (w / divisor), exact apart from subnormal quotients
-//   kScaled  g has been divided beforehand
+//   kScaled  g has been divided beforehand: rows of F quotients, so that with a max half its rows are twice as long
 //   kDivide  an IEEE divide per element and entry
 enum Scale { kPow2, kScaled, kDivide };
 
 struct GradRows {
-    const float *g, *g_max;       // mean and max half of the upstream gradient, rows of `pitch` floats
+    const float *g, *g_max;       // mean and max half of the upstream gradient, rows of `pitch` floats (g_max: 2F)
     const float *w, *feat;
     const unsigned char *maxslot;
     const int *inv_off, *inv_slots, *order;
@@ -92,9 +94,13 @@ struct SlotBytes {
     }
 };
 
+// Behind a matrix of half of kMaxRowBytes, and twice of it behind one of kMaxRowBytes
+constexpr uint32_t kNoHalfRow = 0x7fffe000u;
+static_assert(kNoHalfRow >= kMaxRowBytes / 2 && 2ull * kNoHalfRow >= kMaxRowBytes && 2ull * kNoHalfRow + 8 * kRowLanes * 4 < 1ull << 32);
+
 // what the group's lanes hold of 16 entries
 struct Entries {
-    uint32_t row;    // byte offset of the gradient row, kNoRow beyond the list
+    uint32_t row;    // byte offset of the (mean half's) gradient row, behind the matrices beyond the list
     uint32_t slots;  // byte offset of the arg-max slots
     uint32_t key;    // slot of the entry
     int slot;        // its flat number v K + slot, -1 beyond the list
@@ -105,7 +111,8 @@ struct Entries {
 // rows (requested one step ahead, the max half by the slots), arithmetic. own[e]: the lanes whose element e
 // is theirs. (150,000 vertices, own features of 0 in the place of the others and now: K = 40, F = 22 178 and
 // 177 us, F = 50 229 and 231; K = 16, F = 127 208 and 212.)
-template <int VEC, bool MAX, bool ALIGNED, Tail TAIL>
+// TWICE: the max half lies in rows twice as long as those of the mean half.
+template <int VEC, bool MAX, bool ALIGNED, Tail TAIL, bool TWICE>
 struct Step {
     SlotBytes<VEC, ALIGNED> sb[2];
     float gm[2][VEC], gx[2][VEC];
@@ -119,7 +126,9 @@ struct Step {
         }
     }
     template <int U>
-    __device__ __forceinline__ void request_row(__amdgpu_buffer_rsrc_t G, __amdgpu_buffer_rsrc_t GX, uint32_t at, uint32_t key) {
+    __device__ __forceinline__ void request_row(__amdgpu_buffer_rsrc_t G, __amdgpu_buffer_rsrc_t GX, uint32_t row, uint32_t lane_bytes,
+                                                uint32_t key) {
+        const uint32_t at = row + lane_bytes;
         load_cols<VEC>(G, at, gm[U]);
         if constexpr (MAX) {
             const uint32_t slots = sb[U].packed();
@@ -129,14 +138,15 @@ struct Step {
             if constexpr (VEC > 2) any |= hit[U][2] = byte_is<2>(slots, key);
             if constexpr (VEC > 3) any |= hit[U][3] = byte_is<3>(slots, key);
             // about F/K features of a row have their maximum at one entry: the other lanes aim out of range
-            load_cols<VEC>(GX, __builtin_amdgcn_inverse_ballot_w64(any) ? at : kNoRow, gx[U]);
+            const uint32_t at_max = TWICE ? (row << 1) + lane_bytes : at;
+            load_cols<VEC>(GX, __builtin_amdgcn_inverse_ballot_w64(any) ? at_max : kNoRow, gx[U]);
         }
     }
     template <int E>
     __device__ __forceinline__ void request_rows(__amdgpu_buffer_rsrc_t G, __amdgpu_buffer_rsrc_t GX, const Entries &en,
                                                  uint32_t lane_bytes) {
-        request_row<0>(G, GX, group_bcast<entry_lane(E)>(en.row) + lane_bytes, group_bcast<entry_lane(E)>(en.key));
-        request_row<1>(G, GX, group_bcast<entry_lane(E + 1)>(en.row) + lane_bytes, group_bcast<entry_lane(E + 1)>(en.key));
+        request_row<0>(G, GX, group_bcast<entry_lane(E)>(en.row), lane_bytes, group_bcast<entry_lane(E)>(en.key));
+        request_row<1>(G, GX, group_bcast<entry_lane(E + 1)>(en.row), lane_bytes, group_bcast<entry_lane(E + 1)>(en.key));
     }
     // An entry beyond its list reads zeros and has weight 0: it adds 0 to a sum that started at +0.
     template <int U, Scale SCALE, bool WGRAD>
@@ -225,6 +235,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
         acc[e] = 0.f;
     }
 
+    constexpr bool kTwice = MAX && SCALE == kScaled;
+    constexpr uint32_t no_row = kTwice ? kNoHalfRow : kNoRow;
     const int *list = p.inv_slots + begin + entry_lane(l);
     const int mine = count - entry_lane(l);  // this lane has an entry of chunk c0 if c0 < mine
     auto entries_of = [&](int slot, int c0) {
@@ -233,7 +245,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
         const bool here = c0 < mine && n >= 0;  // column 0 of an index of the whole table is nobody's
         en.key = (uint32_t)n;
         en.slot = here ? slot - (v + 1) * p.skip : -1;
-        en.row = here ? (uint32_t)v * (uint32_t)(p.pitch * 4) : kNoRow;
+        en.row = here ? (uint32_t)v * (uint32_t)(p.pitch * 4) : no_row;
         en.slots = here ? (uint32_t)v * (uint32_t)p.F : kNoRow;
         return en;
     };
@@ -274,7 +286,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
     Selves selves = mark_selves(en, 0);
     float self_dot = 0.f;
 
-    Step<VEC, MAX, ALIGNED, TAIL> st[2];
+    Step<VEC, MAX, ALIGNED, TAIL, kTwice> st[2];
     st[0].template request_slots<0>(MS, en, lane_col, last_pair);
     st[1].template request_slots<2>(MS, en, lane_col, last_pair);
     st[0].template request_rows<0>(G, GX, en, lane_bytes);
@@ -373,27 +385,27 @@ int launch_rows(const GradRows &p, bool mean_and_max, bool want_w, Scale scale, 
     return check_launch("accumulate_grad_rows_kernel");
 }
 
-// the mean half of the gradient divided by the divisor, rows of the gradient's own width
+// the mean half of the gradient (rows of `pitch` floats) divided by the divisor, rows of F
 __global__ __launch_bounds__(256) void divide_mean_half_kernel(const float *__restrict__ g, float *__restrict__ out,
                                                                long long total, int F, int pitch, float divisor) {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= total) return;
     const long long v = t / F;
-    const size_t at = (size_t)v * pitch + (size_t)(t - v * F);
-    out[at] = g[at] / divisor;
+    out[t] = g[(size_t)v * pitch + (size_t)(t - v * F)] / divisor;
 }
 
 }  // namespace
 
-size_t accumulate_grad_rows_scratch_bytes(int n_vert, int n_feat, int g_cols, float divisor) {
-    if (n_feat < kRowLanes || n_feat > 8 * kRowLanes) return 0;
-    if (divisor == (float)(int)divisor && is_pow2((int)divisor)) return 0;
-    return align_up((size_t)n_vert * g_cols * sizeof(float));
-}
-
 bool accumulate_grad_rows_covers(int n_feat, int n_neigh, bool mean_and_max, bool slots, unsigned long long g_bytes) {
     return n_feat >= kRowLanes && n_feat <= 8 * kRowLanes && (!mean_and_max || (slots && n_neigh <= 254)) &&
            g_bytes <= kMaxRowBytes;
+}
+
+size_t accumulate_grad_rows_scratch_bytes(int n_vert, int n_feat, int n_neigh, bool mean_and_max, float divisor) {
+    const unsigned long long n = (unsigned long long)std::max(n_vert, 0) * std::max(n_feat, 0) * sizeof(float);
+    if (!accumulate_grad_rows_covers(n_feat, n_neigh, mean_and_max, true, n * (mean_and_max ? 2 : 1))) return 0;
+    if (divisor == (float)(int)divisor && is_pow2((int)divisor)) return 0;
+    return align_up((size_t)n);
 }
 
 // Returns 1 where the shape is not covered. gw == nullptr: feature gradient only (mean only). scratch
@@ -412,7 +424,7 @@ int launch_accumulate_grad_rows(const float *g, const float *w, const float *fea
     p.g = g;
     if (divisor == (float)(int)divisor && is_pow2((int)divisor)) {
         scale = kPow2;
-    } else if (scratch && scratch_bytes >= accumulate_grad_rows_scratch_bytes(n_vert, F, g_cols, divisor)) {
+    } else if (scratch && scratch_bytes >= accumulate_grad_rows_scratch_bytes(n_vert, F, K, mean_and_max, divisor)) {
         scale = kScaled;
         const long long total = (long long)n_vert * F;
         divide_mean_half_kernel<<<ceil_div(total, 256), 256, 0, s>>>(g, static_cast<float *>(scratch), total, F, g_cols, divisor);
@@ -428,7 +440,7 @@ int launch_accumulate_grad_rows(const float *g, const float *w, const float *fea
     p.order = order;
     p.gw = gw;
     p.gfeat = gfeat;
-    p.g_bytes = g_bytes;
+    p.g_bytes = scale == kScaled ? (unsigned long long)n_vert * F * 4ull : g_bytes;
     p.g_max_bytes = g_bytes - (unsigned long long)F * 4ull;
     p.slot_shift = (uint32_t)(reinterpret_cast<uintptr_t>(maxslot) & 3u);
     p.maxslot = maxslot - p.slot_shift;
@@ -436,7 +448,7 @@ int launch_accumulate_grad_rows(const float *g, const float *w, const float *fea
     p.n_vert = n_vert;
     p.K = K;
     p.F = F;
-    p.pitch = g_cols;
+    p.pitch = scale == kScaled ? F : g_cols;
     p.skip = skip;
     p.div_k = make_fast_div(K + skip);
     p.divisor = divisor;

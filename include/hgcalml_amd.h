@@ -405,9 +405,11 @@ int hgc_accumulate_knn_grad_records(const float *d_grad_from_out_features, const
                                     void *workspace, size_t workspace_bytes, hgc_stream_t stream);
 
 /* hgc_accumulate_knn_grad_slots with scratch memory (may be NULL) for the
- * quotients g / n_neigh where n_neigh is no power of two and n_feat is 16..128
- * (the query returns 0 elsewhere): one pass of n_vert * n_feat divides instead
- * of one divide per gathered element. Same bits either way. With
+ * quotients g / n_neigh, n_vert * n_feat floats, where n_neigh is no power of
+ * two and n_feat is 16..128 (the query returns 0 elsewhere, with mean_and_max
+ * also beyond 254 neighbours, and for gradient matrices beyond 32-bit offsets):
+ * one pass of n_vert * n_feat divides instead of one divide per gathered
+ * element. Same bits either way. With
  * weights_are_exp the weights are exp(-d) and d_out_grad_distances receives the
  * gradient w.r.t. d, -(gradient w.r.t. the weight * weight), the bits of
  * hgc_exp_neg_grad behind this call (outputs and d_distances then on 16-byte

@@ -99,6 +99,19 @@ def test_host_side_argument_checks(capi):
     assert h(one, 10, 10, one, one, null, 0, null) == -2
 
 
+def test_scratch_of_the_accumulation_gradient(capi):
+    """one float per vertex and feature, and none where the kernel that reads it is not taken"""
+    f = capi.hgc_accumulate_knn_grad_scratch_bytes
+    f.restype, f.argtypes = ctypes.c_size_t, [ctypes.c_int] * 4
+    for mean_and_max in (0, 1):
+        assert f(1000, 40, 64, mean_and_max) == 1000 * 64 * 4
+        assert f(1000, 64, 64, mean_and_max) == 0                       # a power of two: no quotients needed
+        assert f(1000, 40, 15, mean_and_max) == 0 and f(1000, 40, 129, mean_and_max) == 0
+        assert f(0, 40, 64, mean_and_max) == 0
+    assert f(1000, 255, 64, 1) == 0 and f(1000, 255, 64, 0) == 1000 * 64 * 4    # arg-max slots are bytes
+    assert f(5000000, 40, 128, 1) == 0 and f(5000000, 40, 128, 0) == 5000000 * 128 * 4   # rows beyond 32-bit offsets
+
+
 def test_settings_are_per_thread(capi):
     """the status word, the choice of the kNN grid and the last error text belong to the thread that set
     them: another thread sees the initial state, and what it sets does not leak back"""

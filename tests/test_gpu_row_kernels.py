@@ -104,3 +104,42 @@ def test_gradient_at_the_ends_of_tiles(oracle, n, K, F):
             got, want = gw.cpu().numpy(), -(rgw * w) if exp else rgw
             assert (np.abs(got - want) <= tol).all()
             assert (got[idx < 0] == 0).all()
+
+
+def test_gradient_of_the_largest_matrix_of_quotients():
+    """8,388,480 rows of 64 features, K no power of two: the gradient matrix ends where 32-bit offsets do, that of its quotients
+    at half of it; lists of two entries, so that most of the 16 places of a step lie beyond them"""
+    from hgcalml_amd import ops
+    if torch.cuda.mem_get_info()[0] < 48 << 30:
+        pytest.skip("needs 48 GB of device memory")
+    n, K, F = 8388480, 3, 64
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(7)
+    v = torch.arange(n, device=DEV, dtype=torch.int32)
+    idx = torch.stack([v, (v + 1) % n, torch.full_like(v, -1)], 1)
+    w = torch.rand(n, K, device=DEV, generator=gen)
+    x = torch.randn(n, F, device=DEV, generator=gen)
+    g = torch.randn(n, 2 * F, device=DEV, generator=gen)
+    slots = torch.randint(0, 3, (n, F), device=DEV, generator=gen, dtype=torch.uint8)   # 2: nobody's
+    arg = torch.zeros(n, F, device=DEV, dtype=torch.int32)                              # not read where there are slots
+    gw, gx = torch.ops.hgcalml.accumulate_knn_grad_slots(g, w, x, idx, arg, slots, *ops.inverse_neighbour_index(idx))
+    del arg
+
+    divisor = torch.full((F,), float(K), device=DEV)   # (torch multiplies by the reciprocal of a number)
+
+    def part(rows, slot):
+        up, ww = g[rows], w[rows, slot, None]
+        return up[:, :F] / divisor * ww + torch.where(slots[rows] == slot, up[:, F:], torch.zeros_like(up[:, F:])) * ww
+    for s in range(0, n, 1 << 20):
+        rows = torch.arange(s, min(n, s + (1 << 20)), device=DEV)
+        own, named = part(rows, 0), part((rows - 1) % n, 1)
+        assert torch.equal(gx[rows], torch.where((rows == 0)[:, None], own + named, named + own))   # ascending (vertex, slot)
+        for slot in (0, 1):
+            xx, up = x[(rows + slot) % n].double(), g[rows].double()
+            terms = up[:, :F] * xx / K + torch.where(slots[rows] == slot, up[:, F:] * xx, torch.zeros_like(xx))
+            # at most 2 F products, sums and one quotient, each rounded once
+            assert bool(((gw[rows, slot].double() - terms.sum(1)).abs() <=
+                         (2 * F + 2) * 2.0 ** -24 * ((up[:, :F] * xx).abs().sum(1) + (up[:, F:] * xx).abs().sum(1))).all())
+        assert not gw[rows, 2].any()
+    del g, x, w, slots, gw, gx, idx, v
+    torch.cuda.empty_cache()
