@@ -540,6 +540,7 @@ __global__ __launch_bounds__(256) void weight_grad_wave_kernel(const float *__re
 // The inverse index of a neighbour table without its first column, from the inverse
 // index of the whole table: the entries of column 0 leave every target's list and
 // flat slot v*K+n becomes v*(K-1)+n-1. One wave per target, its list across the lanes.
+// (Positions in a list, not in the index, which may have 2^31 - 1 entries: the wave's step beyond its end fits.)
 __global__ __launch_bounds__(256) void first_column_entries_kernel(const int *__restrict__ inv_off,
                                                                    const int *__restrict__ inv_slots, int n_vert,
                                                                    const acc::FastDiv div_k, int K,
@@ -548,10 +549,11 @@ __global__ __launch_bounds__(256) void first_column_entries_kernel(const int *__
     if (m > n_vert) return;
     int count = 0;
     if (m < n_vert) {
-        const int begin = inv_off[m], end = inv_off[m + 1];
-        for (int e = begin + lane_id(); e - lane_id() < end; e += kWave) {
-            const int slot = e < end ? inv_slots[e] : 1;
-            count += __popcll(__ballot(e < end && slot - acc::fast_div(slot, div_k) * K == 0));
+        const int begin = inv_off[m], in_list = inv_off[m + 1] - begin;
+        const int *const list = inv_slots + begin;
+        for (int e0 = 0; e0 < in_list; e0 += kWave) {
+            const int e = e0 + lane_id(), slot = e < in_list ? list[e] : 1;
+            count += __popcll(__ballot(e < in_list && slot - acc::fast_div(slot, div_k) * K == 0));
         }
     }
     if (lane_id() == 0) dropped[m] = count;
@@ -568,11 +570,12 @@ __global__ __launch_bounds__(256) void drop_first_column_kernel(const int *__res
     int at = inv_off[m] - dropped_before[m];
     if (lane_id() == 0) out_off[m] = at;
     if (m == n_vert) return;
-    const int begin = inv_off[m], end = inv_off[m + 1];
-    for (int e = begin + lane_id(); e - lane_id() < end; e += kWave) {
-        const int slot = e < end ? inv_slots[e] : 0;
+    const int begin = inv_off[m], in_list = inv_off[m + 1] - begin;
+    const int *const list = inv_slots + begin;
+    for (int e0 = 0; e0 < in_list; e0 += kWave) {
+        const int e = e0 + lane_id(), slot = e < in_list ? list[e] : 0;
         const int v = acc::fast_div(slot, div_k), n = slot - v * K;
-        const bool keep = e < end && n != 0;
+        const bool keep = e < in_list && n != 0;
         const uint64_t kept = __ballot(keep);
         if (keep) out_slots[at + __popcll(kept & ((1ull << lane_id()) - 1ull))] = v * (K - 1) + n - 1;
         at += __popcll(kept);

@@ -19,3 +19,23 @@ def test_derived_index_lists_the_empty_slots(n, k, empty):
     offsets, slots = ops.inverse_index_without_first_column(ops.inverse_neighbour_index(whole), n, k)
     want_offsets, want_slots = ops.inverse_neighbour_index(whole[:, 1:].contiguous())
     assert torch.equal(offsets, want_offsets) and torch.equal(slots, want_slots)
+
+
+def test_derived_index_of_the_largest_table():
+    """2^31 - 256 slots: the last list ends where a wave's step beyond it is no int any more. Row v names v alone, apart
+    from its first slot, so that both indices list the slots in order."""
+    from hgcalml_amd import ops
+    n, k = 8388607, 256
+    if torch.cuda.mem_get_info()[0] < 64 << 30:
+        pytest.skip("needs 64 GB of device memory")
+    offsets = (torch.arange(n + 1, device=DEV) * k).to(torch.int32)
+    slots = torch.arange(n * k, dtype=torch.int32, device=DEV)
+    got_offsets, got_slots = ops.inverse_index_without_first_column((offsets, slots), n, k)
+    del slots
+    assert torch.equal(got_offsets, (torch.arange(n + 1, device=DEV) * (k - 1)).to(torch.int32))
+    total = n * (k - 1)
+    for s in range(0, total, 1 << 28):
+        e = min(total, s + (1 << 28))
+        assert torch.equal(got_slots[s:e], torch.arange(s, e, dtype=torch.int32, device=DEV))
+    del got_slots
+    torch.cuda.empty_cache()
