@@ -397,7 +397,7 @@ extern "C" {
 int hgc_gravnet_drop_self(const int *d_idxs, const float *d_dist, int n_vert, int n_neigh, int *d_out_idxs,
                           float *d_out_dist, hgc_stream_t stream) {
     HGC_REQUIRE(n_vert >= 0 && n_neigh >= 2, "n_vert >= 0, n_neigh >= 2");
-    HGC_REQUIRE((long long)n_vert * n_neigh < (1ll << 31) - 4, "n_vert * n_neigh must stay below 2^31");
+    HGC_REQUIRE((long long)n_vert * n_neigh < (1ll << 31), "n_vert * n_neigh must stay below 2^31");
     if (n_vert == 0) return HGC_OK;
     HGC_REQUIRE(d_idxs && d_dist && d_out_idxs && d_out_dist, "null pointer");
     HGC_REQUIRE(aligned16({d_out_idxs, d_out_dist}), "outputs must lie on 16-byte boundaries");
@@ -410,7 +410,7 @@ int hgc_gravnet_drop_self(const int *d_idxs, const float *d_dist, int n_vert, in
 int hgc_gravnet_drop_self_grad(const float *d_grad_narrow, const float *d_grad_wide, int n_vert, int n_neigh,
                                float *d_out_grad, hgc_stream_t stream) {
     HGC_REQUIRE(n_vert >= 0 && n_neigh >= 2, "n_vert >= 0, n_neigh >= 2");
-    HGC_REQUIRE((long long)n_vert * n_neigh < (1ll << 31) - 4, "n_vert * n_neigh must stay below 2^31");
+    HGC_REQUIRE((long long)n_vert * n_neigh < (1ll << 31), "n_vert * n_neigh must stay below 2^31");
     if (n_vert == 0) return HGC_OK;
     HGC_REQUIRE(d_grad_narrow && d_out_grad, "null pointer");
     HGC_REQUIRE(aligned16({d_grad_wide, d_out_grad}), "wide gradients must lie on 16-byte boundaries");
@@ -438,7 +438,7 @@ int hgc_gravnet_radius_step(const float *d_distsq, long long total, const float 
 
 int hgc_gravnet_join(const float *d_acc, const float *d_features, const float *d_x, int n_vert, int n_feat, int n_x,
                      float *d_out, hgc_stream_t stream) {
-    HGC_REQUIRE(n_vert >= 0 && n_feat >= 1 && n_x >= 1 && n_feat <= 1 << 20 && n_x <= 1 << 20, "bad sizes");
+    HGC_REQUIRE(n_vert >= 0 && n_feat >= 1 && n_x >= 1 && n_feat <= 1 << 30 && n_x <= 1 << 30, "bad sizes");
     if (n_vert == 0) return HGC_OK;
     HGC_REQUIRE(d_acc && d_features && d_x && d_out, "null pointer");
     const bool wide = n_feat % 4 == 0 && n_x % 4 == 0 && aligned16({d_acc, d_features, d_x, d_out});
@@ -455,7 +455,7 @@ int hgc_gravnet_join(const float *d_acc, const float *d_features, const float *d
 
 int hgc_gravnet_join_grad(const float *d_grad, int n_vert, int n_feat, int n_x, float *d_grad_acc, float *d_grad_features,
                           float *d_grad_x, hgc_stream_t stream) {
-    HGC_REQUIRE(n_vert >= 0 && n_feat >= 1 && n_x >= 1 && n_feat <= 1 << 20 && n_x <= 1 << 20, "bad sizes");
+    HGC_REQUIRE(n_vert >= 0 && n_feat >= 1 && n_x >= 1 && n_feat <= 1 << 30 && n_x <= 1 << 30, "bad sizes");
     if (n_vert == 0) return HGC_OK;
     HGC_REQUIRE(d_grad, "null pointer");
     const bool wide = n_feat % 4 == 0 && n_x % 4 == 0 && aligned16({d_grad, d_grad_acc, d_grad_features, d_grad_x});
@@ -495,7 +495,7 @@ int hgc_sumw_grad(const float *d_grad, const float *d_out_feat, const float *d_n
 int hgc_sumw_distance_grad(const float *d_grad_norm, const float *d_weights, const int *d_idxs, int n_vert, int n_neigh,
                            float *d_grad_distances, hgc_stream_t stream) {
     HGC_REQUIRE(n_vert >= 0 && n_neigh >= 1, "bad sizes");
-    HGC_REQUIRE((long long)n_vert * n_neigh < (1ll << 31) - 4, "n_vert * n_neigh must stay below 2^31");
+    HGC_REQUIRE((long long)n_vert * n_neigh < (1ll << 31), "n_vert * n_neigh must stay below 2^31");
     if (n_vert == 0) return HGC_OK;
     HGC_REQUIRE(d_grad_norm && d_weights && d_idxs && d_grad_distances, "null pointer");
     HGC_REQUIRE(aligned16({d_weights, d_idxs, d_grad_distances}), "arrays must lie on 16-byte boundaries");

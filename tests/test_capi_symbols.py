@@ -99,6 +99,24 @@ def test_host_side_argument_checks(capi):
     assert h(one, 10, 10, one, one, null, 0, null) == -2
 
 
+def test_limits_of_the_gravnet_passes(capi):
+    """tables of up to 2^31 - 1 slots, as everywhere else, and rows of any width a tensor has: what is missing here is only the
+    pointers"""
+    capi.hgc_last_error.restype = ctypes.c_char_p
+    p, i = ctypes.c_void_p, ctypes.c_int
+    null = p(None)
+    for f, before, after in ((capi.hgc_gravnet_drop_self, 2, 3), (capi.hgc_gravnet_drop_self_grad, 2, 2),
+                             (capi.hgc_sumw_distance_grad, 3, 2)):
+        f.argtypes = [p] * before + [i, i] + [p] * after
+        for n, k, text in ((32537631, 66, b"null pointer"), (1 << 25, 64, b"2^31")):   # 2^31 - 2 and 2^31 slots
+            assert f(*[null] * before, n, k, *[null] * after) == -1 and text in capi.hgc_last_error()
+    capi.hgc_gravnet_join.argtypes = [p] * 3 + [i] * 3 + [p] * 2
+    capi.hgc_gravnet_join_grad.argtypes = [p] + [i] * 3 + [p] * 4
+    for f, x in ((4, 3 << 20), (3 << 20, 4)):
+        assert capi.hgc_gravnet_join(*[null] * 3, 5, f, x, *[null] * 2) == -1 and b"null pointer" in capi.hgc_last_error()
+        assert capi.hgc_gravnet_join_grad(null, 5, f, x, *[null] * 4) == -1 and b"null pointer" in capi.hgc_last_error()
+
+
 def test_scratch_of_the_accumulation_gradient(capi):
     """one float per vertex and feature, and none where the kernel that reads it is not taken"""
     f = capi.hgc_accumulate_knn_grad_scratch_bytes
