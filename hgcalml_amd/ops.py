@@ -447,15 +447,14 @@ def _accumulate_backward(grad_from_out_features, distances, features, neigh_indi
         max_slots = None
     gw = torch.empty((n, k), dtype=torch.float32, device=dev)
     gx = torch.empty((n, f), dtype=torch.float32, device=dev)
-    if n and inv_slots.numel() == n * (k + 1):  # accumulate_gradient_index: the index of the whole table
-        if exp_weights and w.data_ptr() % 16:
+    if exp_weights and n and inv_slots.numel() == n * (k + 1):  # accumulate_gradient_index: the index of the whole table
+        if w.data_ptr() % 16:
             w = w.clone()
         need = lib.hgc_accumulate_knn_grad_scratch_bytes(n, k, f, int(mean_and_max))
         ws = workspace(need, dev) if need else None
         check(lib.hgc_accumulate_knn_grad_whole_index(p(g), p(w), p(x), p(max_slots), p(inv_offsets), p(inv_slots),
                                                       p(vertex_order_of(neigh_indices)), p(gw), p(gx), n, k, f, g.shape[1],
-                                                      int(mean_and_max), int(exp_weights), p(ws),
-                                                      ws.numel() if need else 0, stream()))
+                                                      int(mean_and_max), 1, p(ws), ws.numel() if need else 0, stream()))
         return gw, gx
     # on request, with the slot table: one record per (vertex, slot) in scratch memory carries the max part to the gather
     need = 0

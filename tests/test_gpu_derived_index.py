@@ -21,6 +21,21 @@ def test_derived_index_lists_the_empty_slots(n, k, empty):
     assert torch.equal(offsets, want_offsets) and torch.equal(slots, want_slots)
 
 
+def test_gradient_with_an_index_that_is_longer_than_the_table():
+    """only the entries that the offsets name count: n (K + 1) of them are not taken for a wider table's index"""
+    from hgcalml_amd import ops
+    g = torch.Generator().manual_seed(1)
+    n, k, f = 50, 7, 16
+    idx = torch.randint(0, n, (n, k), generator=g, dtype=torch.int32).to(DEV)
+    w, x, up = (torch.rand(n, c, generator=g).to(DEV) for c in (k, f, 2 * f))
+    _, arg, slots = torch.ops.hgcalml.accumulate_knn_slots(w, x, idx, 0, True)
+    off, inv = ops.inverse_neighbour_index(idx)
+    longer = torch.cat([inv, torch.zeros(n, dtype=torch.int32, device=DEV)])
+    for a, b in zip(torch.ops.hgcalml.accumulate_knn_grad_slots(up, w, x, idx, arg, slots, off, inv),
+                    torch.ops.hgcalml.accumulate_knn_grad_slots(up, w, x, idx, arg, slots, off, longer)):
+        assert torch.equal(a, b)
+
+
 def test_derived_index_of_the_largest_table():
     """2^31 - 256 slots: the last list ends where a wave's step beyond it is no int any more. Row v names v alone, apart
     from its first slot, so that both indices list the slots in order."""
