@@ -39,19 +39,36 @@ def test_join(n, f, w):
             assert torch.equal(a, b) if want else a.numel() == 0
 
 
+def additions(n, c, vec):
+    """the longest chain of float32 additions a column goes through: the rows of a thread one after the other, the workgroup's
+    groups of threads one after the other, and both again over the slabs' sums (the split column_sums takes)"""
+    cols = c // vec
+    tile = min(32, cols)
+    slab = max(16 * (256 // tile), -(-n // max(1, 512 // -(-cols // tile))))
+    slabs = -(-n // slab)
+    chain = -(-min(slab, n) // (256 // tile)) + 256 // tile
+    narrowest = min(tile, cols % tile or tile)   # a narrow last tile has the more groups, none has longer chains of rows
+    chain = max(chain, -(-min(slab, n) // (256 // narrowest)) + 256 // narrowest)
+    if slabs > 1:
+        last = min(8, cols)
+        narrowest = min(last, cols % last or last)
+        chain += max(-(-slabs // (256 // w)) + 256 // w for w in (last, narrowest))
+    return chain
+
+
 @pytest.mark.parametrize("n,c", [(1, 1), (1, 130), (255, 7), (256, 48), (513, 1), (2477, 48), (64, 24576), (64, 4099),
                                  (150000, 128), (70001, 33), (8192, 4), (9000, 516)])
 def test_column_sums(n, c):
+    """every addition of a chain is off by 2^-24 of a partial sum, which the sum of the absolute values bounds"""
     from hgcalml_amd import ops
     x = torch.randn(n, c, generator=torch.Generator().manual_seed(n + c))
-    want = x.double().sum(0)
-    # float32 sums: at most 1024 serial additions per column and level, of terms whose absolute sum bounds the partial sums
-    bound = 1024 * 2.0 ** -24 * x.double().abs().sum(0)
-    got = ops.column_sums(x.to(DEV)).cpu().double()
-    assert ((got - want).abs() <= bound).all()
     shifted = torch.randn(n * c + 1, generator=torch.Generator().manual_seed(c)).to(DEV)[1:].view(n, c)
-    want = shifted.cpu().double()
-    assert ((ops.column_sums(shifted).cpu().double() - want.sum(0)).abs() <= 1024 * 2.0 ** -24 * want.abs().sum(0)).all()
+    for on_gpu, vec in ((x.to(DEV), 4 if c % 4 == 0 else 1), (shifted, 1)):
+        exact, got = on_gpu.cpu().double(), ops.column_sums(on_gpu).cpu().double()
+        bound = additions(n, c, vec) * 2.0 ** -24 * exact.abs().sum(0)
+        assert ((got - exact.sum(0)).abs() <= 1.0001 * bound).all()
+    # (about a hundred additions for a tall matrix of ordinary width)
+    assert additions(150000, 128, 4) == 37 + 8 + 16 + 32
 
 
 @pytest.mark.parametrize("total,high", [(1, 1.0), (2, 30.0), (1023, 0.01), (4097, 1.0), (3000001, 9.0)])
