@@ -45,14 +45,15 @@ def _sum_rows(t):
 
 class _DropSelfFn(torch.autograd.Function):
     """table and distances without the self column, and the distances themselves: the gradients of both come back in
-    one pass"""
+    one pass. The distances leave as a tensor of their own on the same memory, which may be written to (an input handed
+    back would be a view that refuses it): the block reads them no more, and neither does the search's gradient."""
 
     @staticmethod
     def forward(ctx, idx, dist):
         ctx.set_materialize_grads(False)
         nidx, ndist = ops.gravnet_drop_self(idx, dist)
         ctx.mark_non_differentiable(nidx)
-        return nidx, ndist, dist
+        return nidx, ndist, dist.data
 
     @staticmethod
     def backward(ctx, _grad_nidx, grad_narrow, grad_wide):
@@ -177,6 +178,8 @@ class RaggedGravNet(nn.Module):
             nidx, ndist, dist = _DropSelfFn.apply(idx, dist)
         else:
             nidx, ndist = idx[:, 1:].contiguous(), dist[:, 1:].contiguous()
+            if self.return_self:
+                dist = dist.clone()  # may be written to: the search keeps its own
         ops.share_vertex_order(idx, nidx)
         ops.declare_without_first_column(nidx, idx)
         if self.return_self:

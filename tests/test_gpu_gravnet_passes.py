@@ -109,6 +109,26 @@ def test_block_with_and_without_the_passes(return_self, sumw, monkeypatch):
         assert (a.double() - b.double()).norm() <= 1e-5 * b.double().norm()
 
 
+@pytest.mark.parametrize("return_self", [True, False])
+@pytest.mark.parametrize("passes", [True, False])
+def test_returned_distances_may_be_written_to(return_self, passes, monkeypatch):
+    """in place, before the gradient is asked for: what it is without writing, times the factor"""
+    from hgcalml_amd import GravNetLayersRagged as module
+    if not passes:
+        monkeypatch.setattr(module, "_library_takes", lambda *tensors: False)
+    torch.manual_seed(6)
+    layer = module.RaggedGravNet(5, 4, 3, 6, 7, return_self=return_self).to(DEV)
+    x = torch.randn(200, 5, device=DEV, requires_grad=True)
+    rs = torch.tensor([0, 3, 200], dtype=torch.int32, device=DEV)
+
+    def gradient(in_place):
+        _, _, _, dist = layer(x, rs)
+        dist = dist.mul_(4.0) if in_place else dist * 4.0
+        return dist.detach().clone(), torch.autograd.grad(dist.sum(), x)[0]
+    for a, b in zip(gradient(True), gradient(False)):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("n,k,f", [(1, 1, 1), (17, 5, 3), (33, 16, 15), (100, 17, 32), (64, 40, 33), (90, 70, 130)])
 def test_weights_sum(n, k, f):
     """against the composition with a column of ones: equal bits forward; backward the order of a sum of 2 f + 1 products and
