@@ -38,7 +38,7 @@ def _library_takes(*tensors):
 
 def _sum_rows(t):
     """t.sum(0)"""
-    if torch.is_grad_enabled() or not _library_takes(t) or t[0].numel() > 1 << 20:
+    if torch.is_grad_enabled() or not _library_takes(t) or t.shape[0] >= 1 << 31 or t[0].numel() > 1 << 20:
         return t.sum(0)
     return ops.column_sums(t.reshape(t.shape[0], -1)).view(t.shape[1:])
 

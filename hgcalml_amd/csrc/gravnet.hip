@@ -323,7 +323,8 @@ __global__ __launch_bounds__(kThreads) void column_sums_kernel(const float *__re
     const int width = min(tile_width, cols_v - tile);
     const int groups = kThreads / width;
     const int group = threadIdx.x / width, col = threadIdx.x - group * width;
-    const int begin = blockIdx.x * slab, end = min(n_rows, begin + slab);
+    // rows and what lies a step beyond a slab's end fit into 32 bits without a sign: up to 2^31 - 1 rows
+    const unsigned begin = blockIdx.x * (unsigned)slab, end = min((unsigned)n_rows, begin + (unsigned)slab);
     const V *src = reinterpret_cast<const V *>(x) + tile + col;
     float sum[VEC] = {};
     auto add = [&](const V &v) {
@@ -332,7 +333,7 @@ __global__ __launch_bounds__(kThreads) void column_sums_kernel(const float *__re
         for (int e = 0; e < VEC; ++e) sum[e] += f[e];
     };
     if (group < groups) {
-        int r = begin + group;
+        unsigned r = begin + group;
         for (; r + 3 * groups < end; r += 4 * groups) {
             const V a = src[(size_t)r * cols_v], b = src[(size_t)(r + groups) * cols_v];
             const V c = src[(size_t)(r + 2 * groups) * cols_v], d = src[(size_t)(r + 3 * groups) * cols_v];

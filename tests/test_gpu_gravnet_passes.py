@@ -71,6 +71,21 @@ def test_column_sums(n, c):
     assert additions(150000, 128, 4) == 37 + 8 + 16 + 32
 
 
+@pytest.mark.parametrize("n", [2**31 - 1, 2**31 - 257, 2**31 + 5])
+def test_column_sums_of_the_tallest_matrices(n):
+    """the last rows of the last slab, and more rows than the library counts; whole numbers, so that every order is exact"""
+    from hgcalml_amd import ops
+    from hgcalml_amd.GravNetLayersRagged import _sum_rows
+    x = torch.zeros(n, 1, device=DEV)
+    marks = [0, 1, n // 2, n - 5000000, n - 300, n - 2, n - 1]
+    for i, row in enumerate(marks):
+        x[row] = 2.0 ** i
+    with torch.no_grad():
+        assert _sum_rows(x).tolist() == [2.0 ** len(marks) - 1]
+    if n < 2**31:
+        assert ops.column_sums(x).tolist() == [2.0 ** len(marks) - 1]
+
+
 @pytest.mark.parametrize("total,high", [(1, 1.0), (2, 30.0), (1023, 0.01), (4097, 1.0), (3000001, 9.0)])
 def test_radius_step(total, high):
     from hgcalml_amd import ops
