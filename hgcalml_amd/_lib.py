@@ -75,6 +75,8 @@ _SIGNATURES = {
     "hgc_gravnet_join_grad": (_c_int, [_ptr] + [_c_int] * 3 + [_ptr] * 4),
     "hgc_sumw_normalise": (_c_int, [_ptr] * 2 + [_c_int] * 3 + [_ptr] * 3),
     "hgc_sumw_grad": (_c_int, [_ptr] * 3 + [_c_int] * 3 + [_ptr] * 3),
+    "hgc_sumw_normalise_keep": (_c_int, [_ptr] * 2 + [_c_int] * 3 + [_ptr] * 4),
+    "hgc_sumw_grad_kept": (_c_int, [_ptr] * 3 + [_c_int] * 3 + [_ptr] * 3),
     "hgc_sumw_distance_grad": (_c_int, [_ptr] * 3 + [_c_int] * 2 + [_ptr] * 2),
     "hgc_column_sums_workspace_bytes": (_c_size, [_c_int] * 2),
     "hgc_column_sums": (_c_int, [_ptr] + [_c_int] * 2 + [_ptr] * 2 + [_c_size, _ptr]),

@@ -68,23 +68,25 @@ class _AccumulateSumwFn(torch.autograd.Function):
     def forward(ctx, distances, features, indices):
         out, maxidx, slots, weights = torch.ops.hgcalml.accumulate_knn_exp_slots(distances, features, indices, 0, True)
         idx = ops.i32(indices)
-        norm = ops.sumw_normalise(weights, idx, out)
-        ctx.save_for_backward(weights, features, indices, maxidx, slots, out, norm)
+        # the gradient reads a mean half of its own: the result may be written to
+        mean = out.new_empty(features.shape) if any(ctx.needs_input_grad) else None
+        norm = ops.sumw_normalise(weights, idx, out, mean)
+        ctx.save_for_backward(weights, features, indices, maxidx, slots, mean, norm)
         ctx.indices_ref = indices
         return out
 
     @staticmethod
     def backward(ctx, grad_out):
-        weights, features, indices, maxidx, slots, out, norm = ctx.saved_tensors
+        weights, features, indices, maxidx, slots, mean, norm = ctx.saved_tensors
         k, f = indices.shape[1], features.shape[1]
         if torch.is_grad_enabled():
             # differentiable up to the accumulation's gradient, which says itself that it has none
             empty = (norm == 0)[:, None]
             over = torch.where(empty, torch.zeros_like(grad_out[:, :f]),
                                grad_out[:, :f] / torch.where(empty, torch.ones_like(norm)[:, None], norm[:, None]))
-            g_acc, g_norm = torch.cat([over, grad_out[:, f:]], dim=1), -(over * out[:, :f]).sum(1) / k
+            g_acc, g_norm = torch.cat([over, grad_out[:, f:]], dim=1), -(over * mean).sum(1) / k
         else:
-            g_acc, g_norm = ops.sumw_grad(grad_out, out, norm, k)
+            g_acc, g_norm = ops.sumw_grad(grad_out, mean, norm, k)
         inv_off, inv_slots = ops.accumulate_gradient_index(ctx.indices_ref, f, True)
         gd, gx = torch.ops.hgcalml.accumulate_knn_grad_exp_slots(g_acc, weights, features, indices, maxidx, slots, inv_off,
                                                                  inv_slots)

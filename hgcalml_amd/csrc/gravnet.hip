@@ -229,10 +229,12 @@ __device__ __forceinline__ void add_slots(float mine, float &sum) {
     }
 }
 
-// norm[v] = (sum of the weights, slot after slot) / K; the mean columns of `out` [n, 2F] divided by it (0 where it is 0)
+// norm[v] = (sum of the weights, slot after slot) / K; the mean columns of `out` [n, 2F] divided by it (0 where it is 0),
+// and again to `kept` [n, F] (may be null): what the gradient reads, so that `out` may be written to by then
 __global__ __launch_bounds__(kThreads) void sumw_normalise_kernel(const float *__restrict__ weights,
                                                                   const int *__restrict__ idx, int n, int K, int F, float kf,
-                                                                  float *__restrict__ out, float *__restrict__ norm) {
+                                                                  float *__restrict__ out, float *__restrict__ kept,
+                                                                  float *__restrict__ norm) {
     const int v = blockIdx.x * (kThreads / kGroup) + threadIdx.x / kGroup, l = threadIdx.x % kGroup;
     const bool live = v < n;
     float sum = 0.f;
@@ -246,12 +248,17 @@ __global__ __launch_bounds__(kThreads) void sumw_normalise_kernel(const float *_
     const float d = sum / kf;
     if (l == 0) norm[v] = d;
     float *row = out + (size_t)v * 2 * F;
-    for (int c = l; c < F; c += kGroup) row[c] = d == 0.f ? 0.f : row[c] / d;
+    for (int c = l; c < F; c += kGroup) {
+        const float mean = d == 0.f ? 0.f : row[c] / d;
+        row[c] = mean;
+        if (kept) kept[(size_t)v * F + c] = mean;
+    }
 }
 
-// From the gradient g [n, 2F] of the normalised rows: that of the accumulation's rows, and 1/K of that of norm
-__global__ __launch_bounds__(kThreads) void sumw_grad_kernel(const float *__restrict__ g, const float *__restrict__ out,
-                                                             const float *__restrict__ norm, int n, int F, float kf,
+// From the gradient g [n, 2F] of the normalised rows: that of the accumulation's rows, and 1/K of that of norm (means:
+// rows of `pitch` floats)
+__global__ __launch_bounds__(kThreads) void sumw_grad_kernel(const float *__restrict__ g, const float *__restrict__ means,
+                                                             size_t pitch, const float *__restrict__ norm, int n, int F, float kf,
                                                              float *__restrict__ g_acc, float *__restrict__ g_norm) {
     const int v = blockIdx.x * (kThreads / kGroup) + threadIdx.x / kGroup, l = threadIdx.x % kGroup;
     if (v >= n) return;
@@ -259,7 +266,7 @@ __global__ __launch_bounds__(kThreads) void sumw_grad_kernel(const float *__rest
     const size_t row = (size_t)v * 2 * F;
     float part = 0.f;
     for (int c = l; c < F; c += kGroup) {
-        const float gm = g[row + c], gx = g[row + F + c], mean = out[row + c];
+        const float gm = g[row + c], gx = g[row + F + c], mean = means[v * pitch + c];
         if (d != 0.f) part = part - gm * (mean / d);
         g_acc[row + c] = d == 0.f ? 0.f : gm / d;
         g_acc[row + F + c] = gx;
@@ -473,24 +480,40 @@ int hgc_gravnet_join_grad(const float *d_grad, int n_vert, int n_feat, int n_x, 
     return check_launch("gravnet_join_grad");
 }
 
-int hgc_sumw_normalise(const float *d_weights, const int *d_idxs, int n_vert, int n_neigh, int n_feat, float *d_out_feat,
-                       float *d_norm, hgc_stream_t stream) {
+int hgc_sumw_normalise_keep(const float *d_weights, const int *d_idxs, int n_vert, int n_neigh, int n_feat,
+                            float *d_out_feat, float *d_kept_mean, float *d_norm, hgc_stream_t stream) {
     HGC_REQUIRE(n_vert >= 0 && n_neigh >= 1 && n_feat >= 1, "bad sizes");
     if (n_vert == 0) return HGC_OK;
     HGC_REQUIRE(d_weights && d_idxs && d_out_feat && d_norm, "null pointer");
     sumw_normalise_kernel<<<ceil_div(n_vert, kThreads / kGroup), kThreads, 0, as_stream(stream)>>>(
-        d_weights, d_idxs, n_vert, n_neigh, n_feat, (float)n_neigh, d_out_feat, d_norm);
+        d_weights, d_idxs, n_vert, n_neigh, n_feat, (float)n_neigh, d_out_feat, d_kept_mean, d_norm);
     return check_launch("sumw_normalise");
+}
+
+int hgc_sumw_normalise(const float *d_weights, const int *d_idxs, int n_vert, int n_neigh, int n_feat, float *d_out_feat,
+                       float *d_norm, hgc_stream_t stream) {
+    return hgc_sumw_normalise_keep(d_weights, d_idxs, n_vert, n_neigh, n_feat, d_out_feat, nullptr, d_norm, stream);
+}
+
+static int sumw_grad(const float *d_grad, const float *d_means, size_t pitch, const float *d_norm, int n_vert, int n_neigh,
+                     int n_feat, float *d_grad_accumulated, float *d_grad_norm, hgc_stream_t stream) {
+    if (n_vert == 0) return HGC_OK;
+    HGC_REQUIRE(d_grad && d_means && d_norm && d_grad_accumulated && d_grad_norm, "null pointer");
+    sumw_grad_kernel<<<ceil_div(n_vert, kThreads / kGroup), kThreads, 0, as_stream(stream)>>>(
+        d_grad, d_means, pitch, d_norm, n_vert, n_feat, (float)n_neigh, d_grad_accumulated, d_grad_norm);
+    return check_launch("sumw_grad");
 }
 
 int hgc_sumw_grad(const float *d_grad, const float *d_out_feat, const float *d_norm, int n_vert, int n_neigh, int n_feat,
                   float *d_grad_accumulated, float *d_grad_norm, hgc_stream_t stream) {
     HGC_REQUIRE(n_vert >= 0 && n_neigh >= 1 && n_feat >= 1, "bad sizes");
-    if (n_vert == 0) return HGC_OK;
-    HGC_REQUIRE(d_grad && d_out_feat && d_norm && d_grad_accumulated && d_grad_norm, "null pointer");
-    sumw_grad_kernel<<<ceil_div(n_vert, kThreads / kGroup), kThreads, 0, as_stream(stream)>>>(
-        d_grad, d_out_feat, d_norm, n_vert, n_feat, (float)n_neigh, d_grad_accumulated, d_grad_norm);
-    return check_launch("sumw_grad");
+    return sumw_grad(d_grad, d_out_feat, 2ull * n_feat, d_norm, n_vert, n_neigh, n_feat, d_grad_accumulated, d_grad_norm, stream);
+}
+
+int hgc_sumw_grad_kept(const float *d_grad, const float *d_kept_mean, const float *d_norm, int n_vert, int n_neigh, int n_feat,
+                       float *d_grad_accumulated, float *d_grad_norm, hgc_stream_t stream) {
+    HGC_REQUIRE(n_vert >= 0 && n_neigh >= 1 && n_feat >= 1, "bad sizes");
+    return sumw_grad(d_grad, d_kept_mean, n_feat, d_norm, n_vert, n_neigh, n_feat, d_grad_accumulated, d_grad_norm, stream);
 }
 
 int hgc_sumw_distance_grad(const float *d_grad_norm, const float *d_weights, const int *d_idxs, int n_vert, int n_neigh,

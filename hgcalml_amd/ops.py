@@ -771,25 +771,27 @@ def gravnet_join_grad(grad, n_features, for_accumulated, for_features, for_x):
     return tuple(out)
 
 
-@_op("sumw_normalise(Tensor weights, Tensor indices, Tensor(a!) accumulated) -> Tensor")
-def sumw_normalise(weights, indices, accumulated):
-    """mean half of the accumulation's rows over the weights' sum, in place; returns that sum / K"""
+@_op("sumw_normalise(Tensor weights, Tensor indices, Tensor(a!) accumulated, Tensor(b!)? kept=None) -> Tensor")
+def sumw_normalise(weights, indices, accumulated, kept=None):
+    """mean half of the accumulation's rows over the weights' sum, in place, and to `kept` [N, F]; returns that sum / K"""
     dev = require_device(weights, indices, accumulated)
     n, k = indices.shape
     norm = torch.empty((n,), dtype=torch.float32, device=dev)
-    check(lib.hgc_sumw_normalise(p(weights), p(indices), n, k, accumulated.shape[1] // 2, p(accumulated), p(norm),
-                                 stream()))
+    check(lib.hgc_sumw_normalise_keep(p(weights), p(indices), n, k, accumulated.shape[1] // 2, p(accumulated), p(kept),
+                                      p(norm), stream()))
     return norm
 
 
 @_op("sumw_grad(Tensor grad, Tensor normalised, Tensor norm, int n_neighbours) -> (Tensor, Tensor)")
 def sumw_grad(grad, normalised, norm, n_neighbours):
-    """gradients w.r.t. the accumulation's rows and (divided by K) the weights' sum"""
+    """gradients w.r.t. the accumulation's rows and (divided by K) the weights' sum, from the normalised rows [N, 2F] or
+    their mean half [N, F]"""
     dev = require_device(grad, normalised, norm)
     g = f32(grad)
     g_acc, g_norm = torch.empty_like(g), torch.empty_like(norm)
-    check(lib.hgc_sumw_grad(p(g), p(normalised), p(norm), g.shape[0], n_neighbours, g.shape[1] // 2, p(g_acc), p(g_norm),
-                            stream()))
+    whole = normalised.shape[1] == g.shape[1]
+    call = lib.hgc_sumw_grad if whole else lib.hgc_sumw_grad_kept
+    check(call(p(g), p(normalised), p(norm), g.shape[0], n_neighbours, g.shape[1] // 2, p(g_acc), p(g_norm), stream()))
     return g_acc, g_norm
 
 
@@ -956,7 +958,7 @@ def _(x):
 
 
 @torch.library.register_fake("hgcalml::sumw_normalise")
-def _(weights, indices, accumulated):
+def _(weights, indices, accumulated, kept=None):
     return _f32_like((indices.shape[0],), accumulated)
 
 

@@ -606,12 +606,20 @@ int hgc_gravnet_join_grad(const float *d_grad, int n_vert, int n_feat, int n_x, 
  * rows into that of the accumulation's rows and d_grad_norm [n_vert] = 1/n_neigh of that
  * of d_norm; hgc_sumw_distance_grad subtracts d_grad_norm[v] * d_weights[v,n] from
  * the distance gradient of every slot with a neighbour (arrays [n_vert, n_neigh]
- * on 16-byte boundaries). */
+ * on 16-byte boundaries). The _keep form also writes the normalised mean half to
+ * d_kept_mean [n_vert, n_feat] (may be NULL), and the _kept form reads that instead of
+ * d_out_feat, which may be written to in between. */
 int hgc_sumw_normalise(const float *d_weights, const int *d_idxs, int n_vert, int n_neigh, int n_feat,
                        float *d_out_feat, float *d_norm, hgc_stream_t stream);
 int hgc_sumw_grad(const float *d_grad, const float *d_out_feat, const float *d_norm, int n_vert,
                   int n_neigh, int n_feat, float *d_grad_accumulated, float *d_grad_norm,
                   hgc_stream_t stream);
+int hgc_sumw_normalise_keep(const float *d_weights, const int *d_idxs, int n_vert, int n_neigh,
+                            int n_feat, float *d_out_feat, float *d_kept_mean, float *d_norm,
+                            hgc_stream_t stream);
+int hgc_sumw_grad_kept(const float *d_grad, const float *d_kept_mean, const float *d_norm, int n_vert,
+                       int n_neigh, int n_feat, float *d_grad_accumulated, float *d_grad_norm,
+                       hgc_stream_t stream);
 int hgc_sumw_distance_grad(const float *d_grad_norm, const float *d_weights, const int *d_idxs,
                            int n_vert, int n_neigh, float *d_grad_distances, hgc_stream_t stream);
 

@@ -165,6 +165,12 @@ def test_weights_sum(n, k, f):
         assert torch.isfinite(a).all()
         assert (a - b).norm() <= 1e-5 * b.norm() + 1e-30
     assert (torch.autograd.grad(_AccumulateSumwFn.apply(d, x, idx), d, grad)[0][idx < 0] == 0).all()
+    # the result may be written to in place before its gradient is asked for
+    written = _AccumulateSumwFn.apply(d, x, idx)
+    written -= x.detach().repeat(1, 2)
+    for a, b in zip(torch.autograd.grad(written, [d, x], grad),
+                    torch.autograd.grad(_AccumulateSumwFn.apply(d, x, idx), [d, x], grad)):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("n,k,f", [(2, 1, 16), (17, 3, 17), (66, 15, 33), (67, 16, 64), (90, 17, 65), (83, 40, 128), (70, 64, 48),
