@@ -10,8 +10,9 @@
 // 4*(3K + 5F). The K-fold re-read of feature / gradient rows is a gather that
 // must be served by L2 / Infinity Cache, not HBM.
 //
-// Layout: consecutive lanes hold consecutive features of one vertex (float4
-// per lane when F % 4 == 0), so every gathered row is one coalesced request.
+// Layout: rows of 16 features and more have 16 lanes per vertex, up to four
+// consecutive features per lane (accumulate_rows.hpp); narrower rows, and matrices beyond
+// 32-bit offsets, a thread per element with consecutive lanes on consecutive features.
 // The forward and the feature gradient add their terms in exactly the
 // reference CPU order (slot order, resp. ascending (vertex, slot) per target
 // through the inverse neighbour index), which makes them bit-identical to it;
@@ -159,8 +160,9 @@ __global__ __launch_bounds__(256) void accumulate_fwd_kernel(const float *__rest
 // lanes at once; per slot they arrive as DPP operands, so a slot costs 2 + 5 * VEC vector
 // instructions for four groups, and a gathered row is one 16-byte load per lane. Bound by vector
 // issue with the L1 return path close behind.
-// 150,000 vertices, K = 64, F = 64 in bin order: 190 us with one wave per vertex and dword loads
-// -> 134 us; 240,000, K = 40, F = 32: 221 -> 95 us; a million, K = 64, F = 128: 2.21 -> 1.96 ms.
+// kNN tables of Gaussian points in bin order, one wave per vertex and dword loads against this kernel:
+// 150,000 vertices, 4-D, K = 64, F = 64 171 -> 121 us (with exp(-d) inside 186 -> 147); 240,000, 3-D,
+// K = 40, F = 32 221 -> 101 us (224 -> 117). A million, banded table, K = 64, F = 128 2.21 -> 1.90 ms.
 // A slot without a neighbour aims out of range and has weight 0: it adds 0 to a sum that started
 // at +0 and is masked out of the maximum; four slots in a row that all four groups have take the
 // path without the mask.
@@ -1008,9 +1010,9 @@ int accumulate_gradient(const float *d_grad_from_out_features, const float *d_di
     const bool pow2k = divisor == (float)(int)divisor && is_pow2((int)divisor);
 
     const bool fits_32bit = (unsigned long long)n_vert * (unsigned long long)(2 * n_feat) * 4ull < (1ull << 32);
-    // both gradients from one gather pass where that kernel covers the shape (rows of
-    // 16 to 256 features), or the mean-only feature gradient alone: the gather without
-    // the dot products
+    // both gradients from one gather pass where a kernel covers the shape (16 lanes per target: rows of
+    // 16 to 128 features; a wave per target: up to 256), or the mean-only feature gradient alone: the gather
+    // without the dot products
     if (fits_32bit && want_f && want_w && mean_and_max && d_max_slots && records) {
         const int rc = launch_accumulate_grad_records(d_grad_from_out_features, d_distances, d_feat, d_max_slots,
                                                       d_inv_offsets, d_inv_slots, d_out_grad_distances,

@@ -576,8 +576,8 @@ size_t accumulate_grad_records_bytes(int n_vert, int K, int F) {
 
 // Where the record pass comes near the gather that reads the slot table (accumulate_grad_rows.hip):
 // rows wider than K features with two hits or fewer per slot on average, 48 neighbours or more, and
-// gathered rows that add up to more than the L2 caches keep. (K = 64, F = 128, a million rows: 4.70 ms
-// against 4.62 on a banded table, 5.9 against 4.45 on a kNN table; narrower rows and fewer neighbours
+// gathered rows that add up to more than the L2 caches keep. (K = 64, F = 128, a million rows: 4.75 ms
+// against 4.55 on a banded table, 5.9 against 4.45 on a kNN table; narrower rows and fewer neighbours
 // are further apart.)
 bool accumulate_grad_records_pays(int n_vert, int K, int F) {
     return accumulate_grad_records_bytes(n_vert, K, F) != 0 && K >= 48 && F > K && F <= 2 * K &&

@@ -17,8 +17,8 @@
 // arg-max slots and a masked 16-byte load for the few features whose maximum sits at this entry,
 // for four targets together. One wave per target with one dword per lane ran its three loads
 // per entry at the L1's narrow-load rate (95 % busy, vector issue 62 %):
-// 150,000 vertices, K = 64, F = 64 in bin order 574 -> 320 us; K = 40, F = 32, 240,000 590 -> 278 us;
-// a million, K = 64, F = 128 5.75 -> 4.45 ms. What bounds it now: the L1's address and return path
+// Gaussian points in bin order, 150,000 vertices, 4-D, K = 64, F = 64 535 -> 294 us; 240,000, 3-D, K = 40,
+// F = 32 571 -> 293 us; a million, K = 64, F = 128 5.75 -> 4.45 ms. What bounds it now: the L1's address and return path
 // (77 and 90 % busy at 150,000 vertices), vector issue at 66 %, and at a million vertices the
 // L2 misses (37 % of the return path's time).
 //

@@ -426,7 +426,7 @@ __global__ __launch_bounds__(256) void bin_points_ranked_kernel(
 // All of the grouping by one workgroup, for a few thousand points whose counters fit into its LDS: bounding box, grid,
 // bins, counters (16 bits each, two in a word; a bin's rank in it is the order of arrival), their prefix sums and the move
 // into bin order, with barriers where the general path has launches. A point's bin and rank stay in its thread's registers.
-// Bound by latencies: seven barriers' worth of LDS and L2 round trips, 9 us for 700 points where the five launches took 23
+// Bound by latencies: five barriers' worth of LDS and L2 round trips, 9 us for 700 points where the five launches took 23
 // (a call of BinnedSelectKnn 36.7 -> 24.5 us). Beyond 2048 points one compute unit has too much to write where the nested
 // grid has its 10^4 cells: a call with 4 dimensions and K = 64 takes 47 us against 53 in five launches at 2000 points, 59
 // against 56 at 3000 and 76 against 65 at 4096.

@@ -3,9 +3,9 @@
 // the dynamic radius, the row [mean - p | max - p | x] that the last dense layer reads, and sums over the rows for the
 // gradients of the dense layers. All of them stream; as single tensor operations they were 40 launches and, at 150k
 // vertices, K = 64, F = 64, 0.6 of the 2.45 ms of a training step, most of it intermediates written and read again; the
-// step takes 2.19 ms with these (240k vertices, K = 40, F = 32 with the weights' sum: 2.97 -> 2.27). What is left of them
-// runs at 4 to 5 TB/s: at 150k vertices 36 us each for the join and its gradient (115 and 154 MB), the table and its
-// gradient, 13 us for the radius.
+// step took 2.19 ms with these (240k vertices, K = 40, F = 32 with the weights' sum: 2.97 -> 2.27). Reads and writes
+// together run at what a large copy reaches (5.3 TB/s): at 150k vertices 42 and 49 us for the join and its gradient
+// (269 MB each), 27 and 23 us for the table (155 MB) and its gradient (116 MB), 13 us for the radius (39 MB).
 #include <algorithm>
 #include <cmath>
 

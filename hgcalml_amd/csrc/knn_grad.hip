@@ -15,8 +15,9 @@
 // serially; what it walks over is fetched by the wave together: 16 slots (entries) of its 16 vertices (8
 // with more than 4 coordinates) at a time, one lane per slot for index, gradient and coordinate row,
 // handed over through LDS as differences. (One thread per coordinate doing its own loads fetched every
-// index and gradient C times and issued 16 distinct lines per load: 150,000 vertices, K = 65, C = 4 in bin
-// order 263 -> 168 us; 240,000, K = 41, C = 3 263 -> 131.) What bounds it is the L2: 24 M lines at
+// index and gradient C times and issued 16 distinct lines per load: Gaussian points in bin order, 150,000,
+// K = 65, C = 4 224 -> 138 us (160 in a training step, with other kernels' data in the caches); 240,000,
+// K = 41, C = 3 248 -> 127.) What bounds it is the L2: 24 M lines at
 // 136 G/s for gathers of 4 and 16 bytes; vector issue 12 %. Consecutive workgroups of an XCD take
 // consecutive vertices of the processing order, which keeps the scattered gradients of the second sum in
 // that XCD's L2.

@@ -389,7 +389,7 @@ int hgc_accumulate_knn_grad_slots(const float *d_grad_from_out_features, const f
  * d_max_slots is NULL. hgc_accumulate_knn_grad_records_pays says for which
  * shapes the record pass comes near hgc_accumulate_knn_grad_slots (n_neigh >= 48,
  * n_neigh < n_feat <= 2 n_neigh and n_vert * n_feat of 12 Mi elements or more: a
- * million rows, 64 neighbours, 128 features, banded table 4.70 ms against 4.62 ms,
+ * million rows, 64 neighbours, 128 features, banded table 4.75 ms against 4.55 ms,
  * kNN table 5.9 against 4.45); elsewhere it costs half as much again or more. */
 size_t hgc_accumulate_knn_grad_records_workspace_bytes(int n_vert, int n_neigh, int n_feat,
                                                        int mean_and_max);
