@@ -163,6 +163,8 @@ __global__ __launch_bounds__(256) void accumulate_fwd_kernel(const float *__rest
 // kNN tables of Gaussian points in bin order, one wave per vertex and dword loads against this kernel:
 // 150,000 vertices, 4-D, K = 64, F = 64 171 -> 121 us (with exp(-d) inside 186 -> 147); 240,000, 3-D,
 // K = 40, F = 32 221 -> 101 us (224 -> 117). A million, banded table, K = 64, F = 128 2.21 -> 1.90 ms.
+// (Without locality, points in random order and no processing order, rows come from beyond the L2 and some widths
+// are 3 to 6 % slower: 60,000, K = 64, F = 64 102 -> 107 us.)
 // A slot without a neighbour aims out of range and has weight 0: it adds 0 to a sum that started
 // at +0 and is masked out of the maximum; four slots in a row that all four groups have take the
 // path without the mask.
@@ -319,6 +321,209 @@ __global__ __launch_bounds__(256) void accumulate_fwd_rows_kernel(const float *_
 #pragma unroll
         for (int e = 0; e < VEC; ++e)
             dst[e] = (unsigned char)(packed >> (8 * e));
+    }
+}
+
+
+// ================================================================== wave kernel: rows of whole waves of 16-byte loads
+//
+// Rows of 256 features, or a multiple, are 16-byte loads of every lane of a wave, so that a wave takes one vertex: index
+// and weight of a slot are the same for all lanes and come as scalar loads, the row as a buffer load with a
+// scalar offset, and no vector instruction goes into addressing or broadcasts. The scalar offset is not part
+// of the hardware's range check: every index is compared with the number of rows before it is used.
+// Eight slots without padding take a path without branches, with all their rows under way.
+//
+// Where it pays, against 16 lanes per vertex (Gaussian 3-D points in bin order): means alone, F = 256 100,000
+// vertices, K = 8 57 against 63 us; 60,000, K = 40 101 against 107; F = 512, 60,000, K = 64 281 against 308; 100,000,
+// K = 20 equal. With the maximum, F = 256 and 32 neighbours or more: 60,000, K = 40 109 against 114 us, K = 64
+// 158 against 169; with fewer neighbours 16 lanes are the faster ones (100,000, K = 20 131 against 117, K = 8
+// 76 and 76, with exp(-d) inside 97 against 77), and for wider rows (F = 512, 100,000, K = 16 348 against 246).
+
+// one slot of the forward recurrence for the VEC features of this lane
+template <int VEC, bool MAX, bool SEED>
+__device__ __forceinline__ void fwd_slot(const float (&x)[VEC], float wn, int slot, float (&sum)[VEC],
+                                         float (&best)[VEC], int (&arg)[VEC]) {
+#pragma unroll
+    for (int e = 0; e < VEC; ++e) {
+        const float wf = x[e] * wn;
+        sum[e] = sum[e] + wf;
+        if (MAX) {
+            if (SEED) {  // slot 0 always seeds the maximum
+                best[e] = wf;
+                arg[e] = slot;
+            } else {
+                const bool take = wf >= best[e];  // ">=": a later slot wins ties
+                best[e] = take ? wf : best[e];
+                arg[e] = take ? slot : arg[e];
+            }
+        }
+    }
+}
+
+// Up to U slots [n_begin, n_end) of a vertex's row where some have no neighbour,
+// or the short last chunk of a row: index and weight of slot n_begin + l sit in
+// lane l and are broadcast with v_readlane (no arrays of scalars to keep alive),
+// all rows are in flight together, a slot without a neighbour fetches row 0 and
+// is skipped. Returns n_begin so that the caller's loop advances as for a full chunk.
+// (EXPW: the row's weights wait in LDS, w_lds[n] for slot n.)
+template <int VEC, bool MAX, int U, bool EXPW>
+__device__ __forceinline__ int partial_chunk(const RowMatrix &X, const int *__restrict__ irow,
+                                             const float *__restrict__ wrow, const float *w_lds, int n_begin, int n_end,
+                                             int n_vert, uint32_t lane_bytes, float (&sum)[VEC], float (&best)[VEC],
+                                             int (&arg)[VEC]) {
+    const int lane = lane_id();
+    const int n_mine = min(n_begin + lane, n_end - 1);
+    const int j_lane = n_begin + lane < n_end ? irow[n_mine] : -1;
+    const float w_lane = EXPW ? 0.f : wrow[n_mine];
+    const uint64_t valid = __ballot((uint32_t)j_lane < (uint32_t)n_vert);  // bit l: slot n_begin + l has a neighbour
+    float x[U][VEC];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int j = __builtin_amdgcn_readlane(j_lane, u);
+        X.load<VEC>((valid >> u) & 1ull ? j : 0, lane_bytes, x[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if (!((valid >> u) & 1ull)) continue;  // wave-uniform
+        const float w = EXPW ? w_lds[n_begin + u]
+                             : __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(w_lane), u));
+        if (n_begin + u == 0)
+            fwd_slot<VEC, MAX, true>(x[u], w, 0, sum, best, arg);
+        else
+            fwd_slot<VEC, MAX, false>(x[u], w, n_begin + u, sum, best, arg);
+    }
+    return n_begin;
+}
+
+// EXPW (rows of 64 slots or fewer): `w` holds distances; lane n turns the distance of slot n into
+// the weight exp(-d) (modules/accknn_op.py:52, there a framework op of its own in front of the
+// kernel), writes it to w_out for the gradient and to LDS, from where every lane reads the slots'
+// weights (same address in all lanes) instead of the scalar loads.
+template <bool MAX, bool EXPW>
+__global__ __launch_bounds__(256) void accumulate_fwd_wave_kernel(const float *__restrict__ w,
+                                                                  const float *__restrict__ feat,
+                                                                  const int *__restrict__ idx, float *__restrict__ out,
+                                                                  int *__restrict__ out_maxidx,
+                                                                  unsigned char *__restrict__ out_maxslot, int n_vert,
+                                                                  int K, int F, int out_cols, float kf,
+                                                                  const int *__restrict__ order,
+                                                                  float *__restrict__ w_out) {
+    constexpr int VEC = 4, U = 8;
+    const int v = wave_vertex(order, n_vert);
+    if (v >= n_vert) return;
+    const int *irow = idx + (size_t)v * K;
+    const float *wrow = w + (size_t)v * K;
+    __shared__ float s_weights[EXPW ? 4 : 1][kWave];
+    const float *w_lds = s_weights[EXPW ? threadIdx.x >> 6 : 0];
+    if (EXPW) {
+        const int n = lane_id();
+        float w_n = 0.f;
+        if (n < K) {
+            w_n = expf(-wrow[n]);
+            w_out[(size_t)v * K + n] = w_n;
+        }
+        s_weights[threadIdx.x >> 6][n] = w_n;
+        wave_lds_fence();
+    }
+    const RowMatrix X(feat, n_vert, F);
+    int first_self = -1;  // first slot that names the vertex itself (wave-uniform, scalar ALU)
+
+    for (int fb = lane_id() * VEC; fb < F; fb += kWave * VEC) {
+        const uint32_t lane_bytes = (uint32_t)fb * 4u;
+        float sum[VEC], best[VEC];
+        int arg[VEC];  // SLOT of the maximum, -1: none (translated to an index at the end)
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            sum[e] = 0.f;
+            best[e] = 0.f;
+            arg[e] = -1;
+        }
+        int n0 = 0;
+        for (; n0 + U <= K; n0 += U) {
+            int j[U];
+            float wn[U];
+            float x[U][VEC];
+            uint32_t j_max = 0;  // unsigned: a negative index is the largest
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                j[u] = irow[n0 + u];
+                wn[u] = EXPW ? w_lds[n0 + u] : wrow[n0 + u];
+                j_max = max(j_max, (uint32_t)j[u]);
+            }
+            const bool all_valid = j_max < (uint32_t)n_vert;
+            if (MAX) {
+                int fs = -1;
+#pragma unroll
+                for (int u = U - 1; u >= 0; --u)
+                    if (j[u] == v) fs = n0 + u;
+                if (first_self < 0) first_self = fs;
+            }
+            if (all_valid) {  // wave-uniform: the common, padding-free chunk
+#pragma unroll
+                for (int u = 0; u < U; ++u) X.load<VEC>(j[u], lane_bytes, x[u]);
+                if (n0 == 0) {
+                    fwd_slot<VEC, MAX, true>(x[0], wn[0], 0, sum, best, arg);
+#pragma unroll
+                    for (int u = 1; u < U; ++u) fwd_slot<VEC, MAX, false>(x[u], wn[u], u, sum, best, arg);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < U; ++u) fwd_slot<VEC, MAX, false>(x[u], wn[u], n0 + u, sum, best, arg);
+                }
+            } else {
+                n0 = partial_chunk<VEC, MAX, U, EXPW>(X, irow, wrow, w_lds, n0, n0 + U, n_vert, lane_bytes, sum, best,
+                                                      arg);
+            }
+        }
+        if (n0 < K) {  // K not a multiple of U
+            if (MAX) {
+                const int n_mine = min(n0 + lane_id(), K - 1);
+                const uint64_t self = __ballot(n0 + lane_id() < K && irow[n_mine] == v);
+                if (first_self < 0 && self) first_self = n0 + __builtin_ctzll(self);
+            }
+            if (K - n0 <= 4)
+                partial_chunk<VEC, MAX, 4, EXPW>(X, irow, wrow, w_lds, n0, K, n_vert, lane_bytes, sum, best, arg);
+            else
+                partial_chunk<VEC, MAX, U, EXPW>(X, irow, wrow, w_lds, n0, K, n_vert, lane_bytes, sum, best, arg);
+        }
+        float mean[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) mean[e] = sum[e] / kf;
+        store_vec_once<VEC>(out + (size_t)v * out_cols + fb, mean);
+        if (MAX) {
+            store_vec_once<VEC>(out + (size_t)v * out_cols + F + fb, best);
+            int argidx[VEC];
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) argidx[e] = arg[e] < 0 ? 0 : irow[arg[e]];
+            store_vec_i<VEC>(out_maxidx + (size_t)v * F + fb, argidx);
+            if (out_maxslot) {
+                // slot of the maximum; for a repeated self reference its first slot,
+                // which is the one the reference's gradient credits. A feature without a
+                // maximum (slot 0 empty, every product negative) reports index 0, and the
+                // reference's gradient compares indices: it credits the slot that names
+                // vertex 0, if the row has one.
+                bool none = false;
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) none = none || arg[e] < 0;
+                int first_zero = -1;
+                if (__ballot(none) != 0) {  // wave-uniform, rare
+                    for (int n0z = 0; n0z < K && first_zero < 0; n0z += kWave) {
+                        const int n = n0z + lane_id();
+                        const uint64_t zero = __ballot(n < K && irow[min(n, K - 1)] == 0);
+                        if (zero != 0) first_zero = n0z + __builtin_ctzll(zero);
+                    }
+                }
+                uint32_t packed = 0;
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) {
+                    int sl = arg[e];
+                    if (sl < 0) sl = first_zero;
+                    else if (argidx[e] == v) sl = first_self;
+                    packed |= (uint32_t)(sl < 0 ? 255 : sl) << (8 * e);
+                }
+                unsigned char *dst = out_maxslot + (size_t)v * F + fb;
+                *reinterpret_cast<uint32_t *>(dst) = packed;
+            }
+        }
     }
 }
 
@@ -845,6 +1050,23 @@ int accumulate_forward(const float *d_distances, const float *d_feat, const int 
         const int rc = hgc_exp_neg(d_distances, d_out_weights, (long long)n_vert * n_neigh, stream);
         if (rc) return rc;
         d_distances = d_out_weights;
+    }
+    // a wave per vertex where its lanes' 16-byte loads make up whole rows (see there for where that pays)
+    if (row_kernel && n_feat % (4 * kWave) == 0 && (!mean_and_max || (n_feat == 4 * kWave && n_neigh >= 32)) &&
+        (align_or & 15u) == 0 && (reinterpret_cast<uintptr_t>(d_out_maxslots) & 3u) == 0 &&
+        (!d_out_weights || n_neigh <= kWave)) {
+        const dim3 grid(ceil_div(n_vert, 4)), block(256);
+#define HGC_FWD(MAX, EXPW)                                                                                             \
+    accumulate_fwd_wave_kernel<MAX, EXPW><<<grid, block, 0, s>>>(d_distances, d_feat, d_idxs, d_out_feat, d_out_maxidxs, \
+                                                                 d_out_maxslots, n_vert, n_neigh, n_feat, n_out_feat,  \
+                                                                 divisor, d_order, d_out_weights)
+        if (mean_and_max) {
+            if (d_out_weights) HGC_FWD(true, true); else HGC_FWD(true, false);
+        } else {
+            if (d_out_weights) HGC_FWD(false, true); else HGC_FWD(false, false);
+        }
+#undef HGC_FWD
+        return check_launch("accumulate_fwd_wave_kernel");
     }
     if (row_kernel) {
         int vec, blocks;

@@ -44,7 +44,13 @@ SHAPES = [(1, 1, 16), (2, 3, 17), (3, 4, 31), (5, 5, 32), (17, 15, 33), (66, 16,
           (40, 7, 260), (33, 80, 22)]
 
 
-@pytest.mark.parametrize("n,K,F", SHAPES)
+# rows of whole waves of 16-byte loads, which a wave per vertex takes: slots around its eight at a time and the 64 whose
+# weights it forms itself
+WAVE_SHAPES = [(1, 1, 256), (5, 4, 256), (33, 7, 256), (40, 8, 256), (41, 9, 512), (50, 13, 256), (30, 16, 768), (40, 31, 256),
+               (50, 32, 256), (47, 37, 256), (60, 43, 256), (81, 64, 256), (83, 65, 256), (90, 66, 512)]
+
+
+@pytest.mark.parametrize("n,K,F", SHAPES + WAVE_SHAPES)
 def test_forward_at_the_ends_of_tiles(oracle, n, K, F):
     from hgcalml_amd import ops
     rng = np.random.default_rng(n + 100 * K + 10000 * F)
@@ -65,6 +71,29 @@ def test_forward_at_the_ends_of_tiles(oracle, n, K, F):
                 sl = slots.cpu().numpy().astype(int)
                 named = np.where(sl < K, np.take_along_axis(idx, np.minimum(sl, K - 1), 1), 0)
                 assert (named == rarg).all()
+
+
+@pytest.mark.parametrize("n,K,F", WAVE_SHAPES)
+@pytest.mark.parametrize("mm", [True, False])
+def test_forward_of_whole_waves_against_sixteen_lanes(n, K, F, mm):
+    """bit for bit what 16 lanes per vertex give, which take the same rows from a matrix that is not on a 16-byte
+    boundary; infinities and NaN among the features, exp(-d) inside and outside"""
+    rng = np.random.default_rng(n + K + F)
+    idx = table(rng, n, K)
+    x = rng.standard_normal((n, F)).astype(np.float32)
+    x[rng.random((n, F)) < 0.05] = np.inf
+    x[rng.random((n, F)) < 0.05] = -np.inf
+    x[rng.random((n, F)) < 0.02] = np.nan
+    x[0] = np.nan
+    d, ti = t(rng.random((n, K), dtype=np.float32)), t(idx)
+    shifted = torch.empty(n * F + 1, device=DEV)[1:].view(n, F)
+    shifted.copy_(t(x))
+    for op in (torch.ops.hgcalml.accumulate_knn_slots, torch.ops.hgcalml.accumulate_knn_exp_slots):
+        for a, b in zip(op(d, t(x), ti, 0, mm), op(d, shifted, ti, 0, mm)):
+            if a.dtype == torch.float32:
+                assert torch.equal(torch.isnan(a), torch.isnan(b))
+                a, b = torch.nan_to_num(a, nan=0.5), torch.nan_to_num(b, nan=0.5)
+            assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("n,K,F", SHAPES)
