@@ -446,12 +446,19 @@ size_t hgc_binned_select_knn_pipeline_workspace_bytes(int n_vert, int n_coords, 
     const SearchGrid asked = callers_grid(n_coords, n_bins_scalar, max_bin_dims);
     if (n_vert < 0 || n_coords < 1 || n_rs < 2 || n_bins_scalar < 1 || asked.n_bin_dims < 1 || asked.n_bin_dims > 5)
         return 0;
-    // enough for either grid, whichever hgc_set_knn_grid selects at the time of the call, and for
-    // the library's own grid at any number of neighbours (the coarser grids of larger numbers can be
-    // nested ones where the finest is not)
+    // enough for either grid, whichever hgc_set_knn_grid selects at the time of the call, and for the library's own
+    // grid at any number of neighbours. Fewer bins may need more: the boundary table's counters per bin, and the
+    // nested grid, are what a table of their number of bins has room for. So every number of bins between
+    // those of the smallest and the largest number of neighbours counts, with and without the nested grid.
     size_t bytes = knn_layout(n_vert, n_coords, asked, n_rs, use_direction).total;
-    for (int k = kSmallestGridK; k <= kLargestGridK; k *= 2)
-        bytes = std::max(bytes, knn_layout(n_vert, n_coords, own_grid(n_vert, n_coords, n_rs, k), n_rs, use_direction).total);
+    auto cover = [&](int smallest_k, int largest_k) {
+        SearchGrid grid = own_grid(n_vert, n_coords, n_rs, smallest_k);
+        const int fewest = own_grid(n_vert, n_coords, n_rs, largest_k).n_bins;
+        for (; grid.n_bins >= fewest; --grid.n_bins)
+            bytes = std::max(bytes, knn_layout(n_vert, n_coords, grid, n_rs, use_direction).total);
+    };
+    cover(kSmallestGridK, kSmallestNestedK - 1);
+    cover(kSmallestNestedK, kLargestGridK);
     return bytes;
 }
 
@@ -459,8 +466,12 @@ int hgc_binned_select_knn_pipeline_static(const float *d_coords, const int *d_ro
                                           int n_vert, int n_coords, int n_rs, int n_neigh, int n_bins_scalar,
                                           int max_bin_dims, int tf_compat, float max_radius, int *d_indices,
                                           float *d_dist, int *d_out_sorting, hgc_stream_t stream) {
-    const size_t need = hgc_binned_select_knn_pipeline_workspace_bytes(n_vert, n_coords, n_rs, n_bins_scalar,
-                                                                       max_bin_dims, d_direction != nullptr);
+    // what this call needs; the query covers any number of neighbours and either grid (0: bad arguments, refused below)
+    size_t need = hgc_binned_select_knn_pipeline_workspace_bytes(n_vert, n_coords, n_rs, n_bins_scalar, max_bin_dims,
+                                                                 d_direction != nullptr);
+    if (need > (size_t)HGC_STATIC_SCRATCH_BYTES)
+        need = knn_layout(n_vert, n_coords, search_grid(n_vert, n_coords, n_rs, n_neigh, n_bins_scalar, max_bin_dims), n_rs,
+                          d_direction != nullptr).total;
     if (need > (size_t)HGC_STATIC_SCRATCH_BYTES)
         return fail(HGC_ERR_WORKSPACE,
                     "this call needs %zu bytes of scratch, the built-in array holds %zu: use "

@@ -238,10 +238,11 @@ int hgc_binned_select_knn_pipeline(const float *d_coords, const int *d_row_split
  * counterpart in the reference. The scratch memory is an array of
  * HGC_STATIC_SCRATCH_BYTES inside the library's device image; every GPU the
  * library is used on holds it from the first call to the end of the process.
- * The call allocates and frees nothing. A problem whose
- * hgc_binned_select_knn_pipeline_workspace_bytes(...) exceeds
- * HGC_STATIC_SCRATCH_BYTES is refused with HGC_ERR_WORKSPACE (N = 150,000 points
- * with 4 coordinates, one event and n_bins = 30 need 42.1 MiB). All calls on
+ * The call allocates and frees nothing. A problem that needs more than
+ * HGC_STATIC_SCRATCH_BYTES is refused with HGC_ERR_WORKSPACE; one whose
+ * hgc_binned_select_knn_pipeline_workspace_bytes(...), which covers any number of
+ * neighbours, does not exceed it is not (N = 150,000 points with 4 coordinates, one
+ * event and n_bins = 30: 29.0 MiB). All calls on
  * one GPU share that GPU's array: calls that overlap on one GPU (different
  * streams or threads) race and must be ordered by the caller. The first call on
  * a device looks the array's address up (hipGetSymbolAddress, under a lock):

@@ -167,3 +167,22 @@ def test_package_refuses_cpu_tensors(capi):
     from hgcalml_amd import AccumulateLinKnn
     with pytest.raises(RuntimeError, match="GPU"):
         AccumulateLinKnn(torch.ones(4, 2), torch.ones(4, 3), torch.zeros(4, 2, dtype=torch.int32))
+
+
+def test_knn_workspace_query_covers_every_number_of_neighbours(capi):
+    """the size is checked before anything is launched; without a GPU the launch that follows is an error of its own.
+    (A call with 2-D points, one event of 30,000 and K = 43 was refused with the workspace that the query asks for.)"""
+    torch = pytest.importorskip("torch")
+    if torch.cuda.is_available():
+        pytest.skip("the pointers of this test lead nowhere")
+    query, call = capi.hgc_binned_select_knn_pipeline_workspace_bytes, capi.hgc_binned_select_knn_pipeline
+    query.restype = ctypes.c_size_t
+    somewhere, null = ctypes.c_void_p(1 << 20), ctypes.c_void_p(None)
+    for c in (2, 3, 4, 5, 6):
+        for events in (1, 2, 7, 64):
+            for n in (1, 100, 1000, 5000, 20000, 30000, 100000, 150000, 500000, 1000000):
+                need = query(n, c, events + 1, 30, 3, 0)
+                for k in list(range(2, 70)) + [100, 300]:
+                    rc = call(somewhere, somewhere, null, n, c, events + 1, k, 30, 3, 0, ctypes.c_float(-1.0), somewhere,
+                              somewhere, null, somewhere, ctypes.c_size_t(need), null)
+                    assert rc not in (0, -2), (c, events, n, k)

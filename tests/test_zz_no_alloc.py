@@ -79,3 +79,15 @@ def test_static_scratch_refuses_what_does_not_fit():
     rc = lib.hgc_binned_select_knn_pipeline_static(p(c), p(rs), None, n, C, 2, K, 30, 3, 0, -1.0, p(idx), p(dist), None,
                                                    stream())
     assert rc == -2 and b"scratch" in lib.hgc_last_error()
+
+
+@pytest.mark.parametrize("n,C,K", [(30000, 2, 43), (30000, 2, 58), (30000, 5, 61), (3000, 3, 50)])
+def test_every_number_of_neighbours_has_its_workspace(n, C, K):
+    """grids between those of 32 and of 64 neighbours; the list of K neighbours is the head of that of 64"""
+    import torch
+    from hgcalml_amd import BinnedSelectKnn
+    x = torch.randn(n, C, generator=torch.Generator().manual_seed(n + C)).to("cuda:0")
+    rs = torch.tensor([0, n // 3, n] if C == 5 else [0, n], dtype=torch.int32, device="cuda:0")
+    idx, dist = BinnedSelectKnn(K, x, rs)
+    want_idx, want = BinnedSelectKnn(64, x, rs)
+    assert torch.equal(idx, want_idx[:, :K]) and torch.equal(dist, want[:, :K])
