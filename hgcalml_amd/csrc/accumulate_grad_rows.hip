@@ -21,6 +21,10 @@
 // F = 32 571 -> 293 us; a million, K = 64, F = 128 5.75 -> 4.45 ms. What bounds it now: the L1's address and return path
 // (77 and 90 % busy at 150,000 vertices), vector issue at 66 %, and at a million vertices the
 // L2 misses (37 % of the return path's time).
+// Where this split loses: tables without locality (60,000 vertices, K = 24, targets drawn at random, F = 100 and 128 212 ->
+// 232 us, F = 64 136 -> 144), and a few targets that the whole table names, where a list's entries are one serial
+// chain, longer per entry with four targets a wave (50 targets, F = 64 3.96 -> 5.32 ms). The host does not know a
+// table's lists, and tables of a neighbour search have neither.
 //
 // GravNet accumulates over a table without its self column and needs the inverse index of the whole table for the
 // distances: `skip` lets the gather run on that one and pass over the entries of column 0 (one in K + 1), instead of
