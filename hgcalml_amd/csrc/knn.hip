@@ -6,7 +6,8 @@
 //   modules/binned_select_knn_op.py:92-95               (un-sort, fused when a sorting is given)
 //   modules/compiled/select_knn_kernel.cc:158,244-245   (radius rule)
 //
-// Design (gfx950, wave64):
+// Two searches, chosen by collects(): collect_nearest (every coordinate binned, up to 129 neighbours), described where
+// it stands, and walk_shells for the rest. walk_shells' design (gfx950, wave64):
 //   * Points arrive grouped by bin, so the bins of one row of the grid (last
 //     binned dimension running) are one contiguous range of points. A shell of
 //     half-width d is cut into such ranges ("segments"); the 64 lanes look up 64
@@ -59,7 +60,6 @@ struct KnnParams {
     int *status;      // may be null: device status word for data errors
     float radius_sq;  // < 0: no radius
     int n_vert, K, n_coords, n_bin_dim, n_bboundaries, tf_compat, use_direction;
-    int boundary_shift;  // the boundary of bin b sits at bin_boundaries[b << boundary_shift]
     int rank_base;       // WINDOW kernels: the neighbour ranks below this one are in the output already
     // fine_bits = n_bin_dim: bin_idx is that of the spatial grouping, bin_idx[q] = bin << fine_bits |
     // half-bin bits, and the points of a bin are grouped by these cells. NESTED kernels: a query
@@ -74,8 +74,13 @@ __device__ __forceinline__ float dist_sq(const float (&q)[C > 0 ? C : 1], const 
     float acc = 0.f;
     if constexpr (C > 0) {
         // uniform base + 32-bit byte offset: the load takes its base from scalar registers
-        const float *r = reinterpret_cast<const float *>(reinterpret_cast<const char *>(coord) +
-                                                         (uint32_t)j * (uint32_t)(C * sizeof(float)));
+        uint32_t offset = (uint32_t)j * (uint32_t)(C * sizeof(float));
+        if constexpr (C == 3) {  // 12 j by a shift and a shift-add: a 32-bit multiplication takes four issue slots
+            uint32_t j4 = (uint32_t)j << 2;
+            asm("" : "+v"(j4));
+            offset = (j4 << 1) + j4;
+        }
+        const float *r = reinterpret_cast<const float *>(reinterpret_cast<const char *>(coord) + offset);
         float x[C];
         if constexpr (C == 4 || C == 8) {  // rows are 16-byte aligned (checked on the host)
 #pragma unroll
@@ -99,7 +104,7 @@ __device__ __forceinline__ float dist_sq(const float (&q)[C > 0 ? C : 1], const 
 #pragma unroll
         for (int c = 0; c < C; ++c) {
             const float d = q[c] - x[c];
-            acc = acc + d * d;
+            acc = c == 0 ? d * d : acc + d * d;  // 0 + a square is the square
         }
     } else {
         const float *r = coord + (size_t)j * n_coords;
@@ -273,12 +278,6 @@ constexpr float kNearFirst = 0.45f;
 // strip of segment marks (one byte of LDS each); a multiple of 512.
 constexpr int kMarkCap = 2048;
 
-// Waves (= queries) per workgroup. Queries differ a lot in cost, and a wave slot
-// of a workgroup is handed on only when the whole workgroup has ended: one wave
-// per workgroup measured fastest (150k clustered points in 4-D, K = 64: 0.75 ms
-// against 0.78 ms with 4 and 0.95 ms with 8).
-constexpr int kQueriesPerBlock = 1;
-
 // q = x / w, r = x % w for 0 <= x < 2^22 and w < 2^13, without an integer divide: with inv_w
 // within an ulp of 1 / w (the hardware's approximate reciprocal will do) the float quotient is
 // off by at most one, the remainder says which way
@@ -402,8 +401,8 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
             if (FINE)
                 with_own_bin = p.cell_boundaries[own_cell + 1] - p.cell_boundaries[own_cell] <= Kn;
             else
-                with_own_bin = p.bin_boundaries[(size_t)(own_bin + 1) << p.boundary_shift] -
-                                   p.bin_boundaries[(size_t)own_bin << p.boundary_shift] <= Kn;
+                with_own_bin = p.bin_boundaries[own_bin + 1] -
+                                   p.bin_boundaries[own_bin] <= Kn;
         }
         for (int d = uniform(with_own_bin ? 1 : 0); d <= reach_max; ++d) {
             if (FINE && d > kFineMaxShell) return false;
@@ -576,8 +575,8 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
                             const int first = event_base + cell * nb_last + lo;
                             const int last = event_base + cell * nb_last + hi + 1;
                             if (last < p.n_bboundaries) {
-                                seg_start = p.bin_boundaries[(size_t)first << p.boundary_shift];
-                                seg_len = p.bin_boundaries[(size_t)last << p.boundary_shift] - seg_start;
+                                seg_start = p.bin_boundaries[first];
+                                seg_len = p.bin_boundaries[last] - seg_start;
                             } else if (p.status) {  // the reference prints "idx out of range" and skips the bin
                                 atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
                             }
@@ -687,6 +686,491 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
     return true;
 }
 
+// ---- the search of up to 129 neighbours: collect, cut, sort once ----
+//
+// Bound by the issue of vector instructions (90 % busy), as walk_shells is, and most of those went into resolving the
+// segments of one small shell after another, steps with a few candidates, and sorted inserts of keys that leave the
+// list again. Here a query collects candidates, unsorted, in LDS:
+//   * first the cube of bins around it that holds enough points (the boundary table says how many, before any
+//     distance), or the next larger ones until Kn candidates are collected;
+//   * then the Kn-th distance is bounded by bisection (counts are ballots) and what lies beyond is dropped;
+//   * then one pass over the rows of bins outside the cube that the bound reaches;
+//   * then the keys that are left are sorted, once.
+// Vector instructions per query: 16 events of 1.14 M 3-D points, K = 32, radius 0.1 about 700 -> 465, 150,000 4-D
+// points, K = 65 1475 -> 1126. The whole search, by shells -> collected: these two 1399 -> 1173 us and 429 -> 372 us;
+// 240,000 3-D points, K = 41 367 -> 307; 4-D Gaussian, K = 65 467 -> 410; 4-D uniform, K = 64 361 -> 305; 2-D
+// clusters, K = 32 186 -> 130; 3-D clusters, K = 96 489 -> 319. Tried and taken back: first regions that leave out the
+// corners of the cube (fewer candidates, but a second pass for every query: 4 to 13 % slower), up to three pieces of a
+// row per lane on the nested grid (level in 4-D, 3-D 7 % slower), two queries per wave one after the other (level).
+constexpr int kBufferKeys = 256;  // collected keys per query, in LDS
+// The first cube holds more than Kn + Kn / 2 points. 16 events of 3-D points, K = 32, radius 0.1: 1188 / 1186 / 1182 /
+// 1173 / 1163 us for 1 / 1.125 / 1.25 / 1.5 / 2 Kn; 4-D Gaussian, K = 32: 408 us up to 1.5, 437 at 2; others level.
+constexpr int kFirstCubeShift = 1;
+constexpr int kFineMaxCube = 3;  // on the nested grid a query gives up beyond this half-width
+
+// keys 0 .. n of `buffer` cut down to between Kn and `most` of the smallest (Kn <= most <= n): returns how many are
+// left; `cut` becomes a distance pattern that the Kn-th smallest does not exceed. Distances first, and where more
+// than `most` keys share the Kn-th distance the indices decide.
+__device__ __forceinline__ int cut_to_smallest(uint64_t *const buffer, const int lane, const int n, const int Kn,
+                                               const int most, uint32_t &cut) {
+    constexpr int kRegs = kBufferKeys / kWave;
+    uint64_t k[kRegs];
+    uint32_t largest = 0;
+#pragma unroll
+    for (int u = 0; u < kRegs; ++u) {
+        k[u] = kEmptyKey;
+        if (u * kWave < n) {
+            const bool there = u * kWave + lane < n;
+            if (there) k[u] = buffer[u * kWave + lane];
+            largest = max(largest, there ? (uint32_t)(k[u] >> 32) : 0u);
+        }
+    }
+    uint32_t hi = (uint32_t)readlane_i32((int)wave_inclusive_max(largest), kWave - 1);
+    // (empty lanes count when hi is the pattern of all ones; no square has it)
+    auto count = [&](uint32_t limit) {
+        int c = 0;
+#pragma unroll
+        for (int u = 0; u < kRegs; ++u)
+            if (u * kWave < n) c += (int)__popcll(__builtin_amdgcn_ballot_w64((uint32_t)(k[u] >> 32) <= limit));
+        return c;
+    };
+    int left = n;
+    uint32_t tie_limit = 0xffffffffu;  // keys at distance `hi` stay up to this index
+    if (n > most) {
+        uint32_t lo = 0, step = 2u << 23;  // count(lo) < Kn, or lo = 0
+        for (;;) {
+            lo = hi > step ? hi - step : 0;
+            if (lo == 0) break;
+            const int c = count(lo);
+            if (c < Kn) break;
+            hi = lo;
+            left = c;
+            step = min(2 * step, 1u << 30);
+            if (left <= most) break;
+        }
+        while (left > most && hi - lo > 1) {
+            const uint32_t mid = lo + ((hi - lo) >> 1);
+            const int c = count(mid);
+            if (c >= Kn) {
+                hi = mid;
+                left = c;
+            } else {
+                lo = mid;
+            }
+        }
+        if (left > most && lo == 0) {
+            const int c = count(0);
+            if (c >= Kn) {
+                hi = 0;
+                left = c;
+            }
+        }
+        if (left > most) {  // more than `most` - Kn keys share the Kn-th distance
+            uint32_t tie_lo = 0;  // fewer than Kn keys with this limit, or 0
+            while (left > most && tie_limit - tie_lo > 1) {
+                const uint32_t mid = tie_lo + ((tie_limit - tie_lo) >> 1);
+                const uint64_t limit = (uint64_t)hi << 32 | mid;
+                int c = 0;
+#pragma unroll
+                for (int u = 0; u < kRegs; ++u) c += (int)__popcll(__builtin_amdgcn_ballot_w64(k[u] <= limit));
+                if (c >= Kn) {
+                    tie_limit = mid;
+                    left = c;
+                } else {
+                    tie_lo = mid;
+                }
+            }
+        }
+        const uint64_t limit = (uint64_t)hi << 32 | tie_limit;
+        int at = 0;
+        wave_lds_fence();
+#pragma unroll
+        for (int u = 0; u < kRegs; ++u) {
+            if (u * kWave < n) {
+                const uint64_t m = __builtin_amdgcn_ballot_w64(k[u] <= limit && u * kWave + lane < n);
+                const int before = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+                if (__builtin_amdgcn_inverse_ballot_w64(m)) buffer[at + before] = k[u];
+                at += (int)__popcll(m);
+            }
+        }
+        wave_lds_fence();
+        left = at;
+    }
+    cut = min(cut, hi);
+    return left;
+}
+
+// table[i] with the table in scalar registers and a 32-bit byte offset (tables of collect_nearest stay below 2^30 entries)
+__device__ __forceinline__ int table_entry(const int *__restrict__ table, int i) {
+    return *reinterpret_cast<const int *>(reinterpret_cast<const char *>(table) + ((uint32_t)i << 2));
+}
+
+// Taken where every coordinate is binned and up to 129 neighbours are asked for. With more coordinates the Kn-th
+// distance is many bins wide, and the walk by shells, which tightens it as it goes, looks at fewer candidates (80,000
+// points in 5-D, 4 of them binned, K = 32: 423 us by shells, 635 us collected).
+constexpr bool collects(int C, int NB, int S, bool window) { return C == NB && NB >= 2 && NB <= 4 && S <= 2 && !window; }
+
+// a bound of the squared distances with this pattern or a smaller one; at least the smallest normal number, since the
+// hardware's square root takes smaller ones as zero
+__device__ __forceinline__ float bound_of(uint32_t pattern) { return __uint_as_float(max(pattern, 0x00800000u)); }
+
+// The Kn smallest keys of query q, ascending, in `key` (ranks beyond the points there are: the empty key). FINE as in
+// walk_shells. False: nothing is decided (the grid of bins, or walk_shells, has to do it).
+template <int C, int NB, int S, bool MAPPED, bool FINE>
+__device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q, const int lane, uint8_t *const marks,
+                                                uint64_t *const buffer, const int Kn, uint64_t (&key)[S]) {
+    static_assert(C > 0 && NB >= 2 && NB <= 4 && S <= 2);
+    constexpr int B = NB;
+    float qc[C];
+    const float *qrow = p.coord + (size_t)q * C;
+#pragma unroll
+    for (int c = 0; c < C; ++c) qc[c] = qrow[c];
+
+    // Dimension i of the query's place in the grid is worked out in lane i (one vector instruction for all of them)
+    // and read from there.
+    const int own_cell = uniform(p.bin_idx[q]);
+    const int own_bin = own_cell >> p.fine_bits;
+    const int dim = min(lane, B - 1);
+    int nb_v = p.n_bins[dim], qb_v = p.dim_bin_idx[(size_t)q * (B + 1) + 1 + dim];
+    int in_event = 0;  // number of the own bin inside its event
+#pragma unroll
+    for (int i = 0; i < B; ++i) in_event = in_event * readlane_i32(nb_v, i) + readlane_i32(qb_v, i);
+    const int event_base = own_bin - in_event;
+    if (FINE) {
+        nb_v *= 2;
+        qb_v = 2 * qb_v + ((own_cell >> (B - 1 - dim)) & 1);
+    }
+    const int top_v = nb_v - 1 - qb_v;  // bins above the own one
+    int nb[B], qb[B];
+    long long grid_rows = 1;
+    bool rows_fit = true;
+#pragma unroll
+    for (int i = 0; i < B; ++i) {
+        nb[i] = readlane_i32(nb_v, i);
+        qb[i] = readlane_i32(qb_v, i);
+        if (i < B - 1) {
+            grid_rows *= nb[i];
+            rows_fit = rows_fit && nb[i] < (1 << 13);
+        }
+    }
+    const int nb_last = nb[B - 1], qb_last = qb[B - 1];
+    const int bins_last = FINE ? nb_last >> 1 : nb_last;
+    grid_rows *= FINE ? bins_last + 1 : 2;  // slots of a pass
+    if (!rows_fit || grid_rows >= (1ll << 22) || event_base < 0) {  // see divmod_small; a bin that no grid gives
+        if (FINE) return false;  // the grid of bins may do
+        if (p.status && lane == 0) atomicOr(p.status, event_base < 0 ? HGC_FLAG_BIN_BEYOND_TABLE : HGC_FLAG_SHELL_TOO_WIDE);
+        return true;  // the list stays empty
+    }
+    const float bw = FINE ? 0.5f * p.bin_width[0] : p.bin_width[0];
+    // Coordinates without bounds leave widths without a meaning: then nothing is pruned, the whole grid is walked.
+    const bool prunes = bw > 1e-30f && bw < 1e18f;  // (the square stays finite)
+    const float inv_bw = __builtin_amdgcn_rcpf(bw);  // within an ulp; used with margins of a thousandth of a bin
+    const float bins_per_unit = prunes ? 1.001f * inv_bw : 3.0e38f;
+    const float gap_scale = prunes ? 0.999f * (bw * bw) : 0.f;  // bounds are generous by 0.1 %
+
+    // lower bounds of the distance to the edges of the own bin, in bin widths, as in walk_shells
+    float tl_v = 0.f, tu_v = 0.f;
+    if (p.shift) {
+        const float frac = (qrow[dim] - p.shift[dim]) * inv_bw - (float)qb_v;
+        if (frac >= 0.f && frac <= 1.f) {
+            tl_v = fmaxf(frac - 1e-3f, 0.f);
+            tu_v = fmaxf(1.f - frac - 1e-3f, 0.f);
+        }
+    }
+    float from_lower[B], from_upper[B];  // 1 - these bounds
+#pragma unroll
+    for (int i = 0; i < B - 1; ++i) {
+        from_lower[i] = __int_as_float(readlane_i32(__float_as_int(1.f - tl_v), i));
+        from_upper[i] = __int_as_float(readlane_i32(__float_as_int(1.f - tu_v), i));
+    }
+    const float tl_last = __int_as_float(readlane_i32(__float_as_int(tl_v), B - 1));
+    const float tu_last = __int_as_float(readlane_i32(__float_as_int(tu_v), B - 1));
+
+    const bool has_radius = p.radius_sq >= 0.f;
+    // candidates beyond this distance pattern are not collected: the radius, then the bound of the Kn-th distance
+    uint32_t cut = has_radius ? __float_as_uint(p.radius_sq) : 0xffffffffu;
+    const int kept = Kn + (Kn >> 2) + 4;  // a cut leaves up to so many keys
+
+    // The first cube: the smallest one that holds more than `enough` points, of half-width 0 .. kCubes (no wider than
+    // the radius asks for). One lane per row of bins (on the nested grid per row and bin that the row's three cells
+    // touch, always two).
+    const int enough = Kn + (Kn >> kFirstCubeShift);
+    int d_out, d_radius = 1 << 30;  // the cube of half-width d_radius holds everything within the radius
+    if (has_radius && prunes)
+        d_radius = max(1, uniform((int)fminf(__builtin_ceilf(__builtin_amdgcn_sqrtf(bound_of(__float_as_uint(p.radius_sq))) * bins_per_unit), 1.0e9f)));
+    int seg_start = 0, seg_len = 0;
+    {
+        int off[B], ring = 0;
+        bool in_grid = true;
+        if constexpr (FINE) {
+            int row = lane >> 1;
+            in_grid = row < (B == 2 ? 3 : B == 3 ? 9 : 27);
+#pragma unroll
+            for (int i = B - 2; i >= 0; --i) {
+                off[i] = (i > 0 ? row % 3 : row) - 1;
+                row /= 3;
+            }
+        } else if constexpr (B == 4) {
+            off[0] = (lane >> 4) - 1, off[1] = ((lane >> 2) & 3) - 1, off[2] = (lane & 3) - 1;
+        } else if constexpr (B == 3) {
+            off[0] = (lane >> 3) - 3, off[1] = (lane & 7) - 3;
+        } else {
+            off[0] = lane - 3;
+        }
+        int cell = 0, halves = 0;
+#pragma unroll
+        for (int i = 0; i < B - 1; ++i) {
+            const int k = qb[i] + off[i];
+            in_grid = in_grid && (uint32_t)k < (uint32_t)nb[i];
+            ring = max(ring, abs(off[i]));
+            if (FINE) {
+                cell = (int)__umul24(cell, nb[i] >> 1) + (k >> 1);
+                halves = (halves << 1) | (k & 1);
+            } else {
+                cell = (int)__umul24(cell, nb[i]) + k;
+            }
+        }
+        if constexpr (FINE) {
+            const int own = uniform(p.cell_boundaries[own_cell + 1]) - uniform(p.cell_boundaries[own_cell]);
+            d_out = own > enough ? 0 : 1;
+            const int bin_last = ((qb_last - 1) >> 1) + (lane & 1);
+            const int lo = max(max(qb_last - d_out, 0), 2 * bin_last), hi = min(min(qb_last + d_out, nb_last - 1), 2 * bin_last + 1);
+            const int bin = event_base + (int)__umul24(cell, bins_last) + bin_last;
+            if (in_grid && ring <= d_out && lo <= hi && bin + 1 < p.n_bboundaries) {
+                const int base = ((bin << (B - 1)) | halves) << 1;
+                seg_start = table_entry(p.cell_boundaries, base | (lo & 1));
+                seg_len = table_entry(p.cell_boundaries, (base | (hi & 1)) + 1) - seg_start;
+            }
+        } else {
+            constexpr int kCubes = B == 4 ? 1 : 3;
+            // lanes without a row look at the own one
+            const int row = in_grid ? event_base + (int)__umul24(cell, nb_last) : own_bin - qb_last;
+            auto look = [&](int d) {  // the part of the row inside the cube of half-width d
+                const int from = max(qb_last - d, 0), to = min(qb_last + d, nb_last - 1) + 1;
+                const bool wanted = in_grid && ring <= d && row < p.n_bboundaries - to;
+                seg_start = seg_len = 0;
+                if (wanted) {
+                    seg_start = table_entry(p.bin_boundaries + from, row);
+                    seg_len = table_entry(p.bin_boundaries + to, row) - seg_start;
+                }
+                if (p.status && in_grid && ring <= d && !wanted)  // the reference prints "idx out of range" and skips the bin
+                    atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
+                return readlane_i32(wave_inclusive_sum(seg_len), kWave - 1);
+            };
+            d_out = 1;
+            const int held = look(1);
+            if (kCubes > 1 && held <= enough && d_radius > 1) {
+                d_out = 2;
+                if (look(2) <= enough && d_radius > 2) {
+                    d_out = 3;
+                    look(3);
+                }
+            } else if (held > 4 * enough && own_bin + 1 < p.n_bboundaries &&
+                       uniform(p.bin_boundaries[own_bin + 1]) - uniform(p.bin_boundaries[own_bin]) > enough) {
+                d_out = 0;  // crowded: the own bin does
+                look(0);
+            }
+            d_out = uniform(d_out);
+        }
+    }
+
+    int n_kept = 0;  // keys in the buffer
+    int d_in = -1;   // the cube of this half-width has been walked (-1: none)
+    for (;;) {
+        const bool bounded = prunes && cut < 0x7f000000u;
+        const bool last_pass = bounded && d_in >= 0;  // everything within the bound
+        int below[B], width[B], below_in[B], width_in[B];
+        float inv_width[B], inv_width_in[B];
+        int n_rows = 1, n_inner = 1, lo_last = 0, hi_last = 0, first_bin = 0, P = 1, n_slots = 1;
+        bool low_caps = false, high_caps = false;
+        float inv_P = 1.f;
+        if (d_in >= 0) {
+            float reach_bins = 3.0e9f;
+            if (bounded) reach_bins = __builtin_amdgcn_sqrtf(bound_of(cut)) * bins_per_unit + 1.001f;
+            if (FINE && (last_pass ? reach_bins > (float)(kFineMaxCube + 2) : d_out > kFineMaxCube)) return false;
+            const int d_most = last_pass ? 1 << 30 : d_out;
+            const int lo_v = min(min(d_most, qb_v), (int)fminf(reach_bins - tl_v, 1.0e9f));
+            const int hi_v = min(min(d_most, top_v), (int)fminf(reach_bins - tu_v, 1.0e9f));
+            bool beyond = false;  // anything outside the cube walked before
+#pragma unroll
+            for (int i = 0; i < B - 1; ++i) {
+                const int lo_i = readlane_i32(lo_v, i), hi_i = readlane_i32(hi_v, i);
+                below[i] = lo_i;
+                width[i] = lo_i + hi_i + 1;
+                below_in[i] = min(lo_i, d_in);
+                width_in[i] = below_in[i] + min(hi_i, d_in) + 1;
+                inv_width[i] = inv_width_in[i] = 1.f;
+                if (i > 0) {
+                    inv_width[i] = __builtin_amdgcn_rcpf((float)width[i]);
+                    inv_width_in[i] = __builtin_amdgcn_rcpf((float)width_in[i]);
+                }
+                n_rows *= width[i];
+                n_inner *= width_in[i];
+                beyond = beyond || lo_i > d_in || hi_i > d_in;
+            }
+            lo_last = readlane_i32(lo_v, B - 1);
+            hi_last = readlane_i32(hi_v, B - 1);
+            low_caps = lo_last > d_in;
+            high_caps = hi_last > d_in;
+            if (!beyond && !low_caps && !high_caps) break;
+            if (FINE) {
+                first_bin = (qb_last - lo_last) >> 1;
+                P = ((qb_last + hi_last) >> 1) - first_bin + 1;
+                inv_P = __builtin_amdgcn_rcpf((float)P);
+            }
+            // one slot per row and, where both end caps of the rows that cross the walked cube matter, one more for those
+            n_slots = FINE ? n_rows * P : low_caps && high_caps ? n_rows + n_inner : n_rows;
+        }
+
+        for (int slot0 = 0; slot0 < n_slots; slot0 += kWave) {
+            const float reach2 = prunes && cut < 0x7f000000u ? bound_of(cut) : 3.0e38f;
+            const int slot = slot0 + lane;
+            if (d_in >= 0) seg_start = seg_len = 0;
+            if (d_in >= 0 && slot < n_slots) {
+                int row, piece = 0;
+                bool inner = false;
+                if (FINE) {
+                    divmod_small(slot, P, inv_P, row, piece);
+                } else {
+                    inner = slot >= n_rows;
+                    row = inner ? slot - n_rows : slot;
+                }
+                int off[B];
+#pragma unroll
+                for (int i = B - 2; i >= 0; --i) {
+                    const int below_i = inner ? below_in[i] : below[i];
+                    if (i > 0) {
+                        int digit;
+                        divmod_small(row, inner ? width_in[i] : width[i], inner ? inv_width_in[i] : inv_width[i], row, digit);
+                        off[i] = digit - below_i;
+                    } else {
+                        off[i] = row - below_i;
+                    }
+                }
+                bool on_face = false;
+                int cell = 0, halves = 0;
+                float gap2 = 0.f;  // squared lower bound of the distance to this row, in bin widths
+#pragma unroll
+                for (int i = 0; i < B - 1; ++i) {
+                    const int o = off[i], k = qb[i] + o;
+                    on_face = on_face || abs(o) > d_in;
+                    if (FINE) {
+                        cell = (int)__umul24(cell, nb[i] >> 1) + (k >> 1);
+                        halves = (halves << 1) | (k & 1);
+                    } else {
+                        cell = (int)__umul24(cell, nb[i]) + k;
+                    }
+                    const float of = (float)o;
+                    const float g = fmaxf(fmaxf(of - from_upper[i], -of - from_lower[i]), 0.f);
+                    gap2 = __builtin_fmaf(g, g, gap2);
+                }
+                gap2 *= gap_scale;
+                // bins of the row within reach (bound generous by 0.1 % and a thousandth of a bin)
+                const float rest = reach2 - gap2;
+                const float span = __builtin_amdgcn_sqrtf(fmaxf(rest, 0.f)) * bins_per_unit + 1.001f;
+                int lo = -min(lo_last, (int)fminf(span - tl_last, 1.0e9f));
+                int hi = min(hi_last, (int)fminf(span - tu_last, 1.0e9f));
+                if (FINE) {
+                    // the part inside one bin, less the cells walked before
+                    const int bin = first_bin + piece;
+                    lo = max(lo, 2 * bin - qb_last);
+                    hi = min(hi, 2 * bin + 1 - qb_last);
+                    if (!on_face) {
+                        if (lo < -d_in) hi = min(hi, -d_in - 1);
+                        else lo = max(lo, d_in + 1);
+                    }
+                } else if (!on_face) {
+                    if (low_caps && !inner) hi = min(hi, -d_in - 1);
+                    else lo = max(lo, d_in + 1);
+                }
+                if (rest >= 0.f && lo <= hi) {
+                    if (FINE) {
+                        const int bin = event_base + (int)__umul24(cell, bins_last) + ((qb_last + lo) >> 1);
+                        if (bin + 1 < p.n_bboundaries) {
+                            const int base = ((bin << (B - 1)) | halves) << 1;
+                            seg_start = table_entry(p.cell_boundaries, base | ((qb_last + lo) & 1));
+                            seg_len = table_entry(p.cell_boundaries, (base | ((qb_last + hi) & 1)) + 1) - seg_start;
+                        } else if (p.status) {
+                            atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
+                        }
+                    } else {
+                        const int first = event_base + (int)__umul24(cell, nb_last) + qb_last + lo;
+                        const int last = first + (hi - lo) + 1;
+                        if (last < p.n_bboundaries) {
+                            seg_start = table_entry(p.bin_boundaries, first);
+                            seg_len = table_entry(p.bin_boundaries, last) - seg_start;
+                        } else if (p.status) {
+                            atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
+                        }
+                    }
+                }
+            }
+            const int seg_end = wave_inclusive_sum(seg_len);
+            const int seg_off = seg_end - seg_len;
+            const int total = readlane_i32(seg_end, kWave - 1);
+            // kept one lane up, so that the mark (lane number + 1) is the lane to read it from: see walk_shells
+            const int seg_delta = __builtin_amdgcn_update_dpp(0, seg_start - seg_off, 0x13c, 0xf, 0xf, false);
+            uint32_t owner_carry = 0;
+            for (int c0 = 0; c0 < total; c0 += kMarkCap) {
+                const int chunk = min(kMarkCap, total - c0);
+                for (int base = 0; base < chunk; base += kWave * 8)
+                    *reinterpret_cast<uint64_t *>(marks + base + lane * 8) = 0;
+                wave_lds_fence();
+                const int rel = seg_off - c0;
+                if (seg_len > 0 && rel >= 0 && rel < chunk) marks[rel] = (uint8_t)(lane + 1);
+                wave_lds_fence();
+                for (int t = 0; t < chunk; t += kWave) {
+                    const int c = c0 + t + lane;
+                    uint32_t owner = wave_inclusive_max(marks[t + lane]);
+                    owner = max(owner, owner_carry);
+                    owner_carry = (uint32_t)readlane_i32((int)owner, kWave - 1);
+                    const int j = c + from_lane_i32(seg_delta, (int)owner);
+                    const bool in_list = c < total;
+                    uint64_t valid = __builtin_amdgcn_ballot_w64(in_list) & __builtin_amdgcn_ballot_w64(j != q);
+                    const int jj = in_list ? j : q;
+                    const uint32_t id = MAPPED ? *reinterpret_cast<const uint32_t *>(
+                                                     reinterpret_cast<const char *>(p.sorting) + ((uint32_t)jj << 2))
+                                               : (uint32_t)jj;
+                    const float dsq = dist_sq<C>(qc, p.coord, jj, C, qrow);
+                    if (p.use_direction) {
+                        const int dj = p.direction[jj];
+                        valid &= ~__builtin_amdgcn_ballot_w64(dj == 1 || dj == 2);  // may not be a neighbour
+                    }
+                    uint64_t enters = valid & __builtin_amdgcn_ballot_w64(__float_as_uint(dsq) <= cut);
+                    if (enters) {
+                        if (n_kept + (int)__popcll(enters) > kBufferKeys) {
+                            wave_lds_fence();
+                            n_kept = cut_to_smallest(buffer, lane, n_kept, Kn, kept, cut);
+                            enters &= __builtin_amdgcn_ballot_w64(__float_as_uint(dsq) <= cut);
+                        }
+                        const int at = n_kept + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(enters >> 32),
+                                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)enters, 0));
+                        if (__builtin_amdgcn_inverse_ballot_w64(enters)) buffer[at] = (uint64_t)__float_as_uint(dsq) << 32 | id;
+                        n_kept += (int)__popcll(enters);
+                    }
+                }
+            }
+        }
+        // done: everything within the bound, the radius or the grid has been seen
+        if (last_pass || d_out >= d_radius || !__builtin_amdgcn_ballot_w64(max(qb_v, top_v) > d_out)) break;
+        d_in = d_out;
+        if (n_kept >= Kn) {
+            wave_lds_fence();
+            n_kept = cut_to_smallest(buffer, lane, n_kept, Kn, kept, cut);
+        }
+        d_out = d_out < 4 ? d_out + 1 : d_out + (d_out >> 1);
+    }
+
+    wave_lds_fence();
+    if (n_kept > S * kWave) n_kept = cut_to_smallest(buffer, lane, n_kept, Kn, S * kWave, cut);
+    key[0] = wave_sort_u64(lane < n_kept ? buffer[lane] : kEmptyKey);
+    if constexpr (S == 2) {
+        key[1] = kEmptyKey;
+        if (n_kept > kWave) merge_batch<S>(key, wave_sort_u64(kWave + lane < n_kept ? buffer[kWave + lane] : kEmptyKey));
+    }
+    return true;
+}
+
 // C: coordinates per point, NB: binned dimensions (0 for either: taken from the
 // arguments), S: registers of the sorted list per lane, MAPPED: results in the
 // index space and at the positions of `sorting`.
@@ -698,24 +1182,16 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
 // NESTED: the search runs over a nested grid (see KnnParams::fine_bits): a query whose bin holds more
 // than fine_min_population points walks the nested grid (and the grid of bins after all when that
 // walk gives up), the others the grid of bins.
-template <int C, int NB, int S, bool MAPPED, bool WINDOW = false, bool NESTED = false>
-__global__ __launch_bounds__(kQueriesPerBlock * kWave)
-__attribute__((amdgpu_waves_per_eu(S <= 2 ? 8 : 1, 8)))
-void knn_wave_kernel(const KnnParams p) {
-    __shared__ __attribute__((aligned(8))) uint8_t mark_strips[kQueriesPerBlock][kMarkCap];
-    const int lane = lane_id();
-    // queries come in bin order and differ a lot in cost from region to region:
-    // chunks of 512 of them are dealt to the XCDs in turn
-    const int tile = xcd_chunked_block<512>(blockIdx.x, gridDim.x);
-    const int q = tile * kQueriesPerBlock + (threadIdx.x >> 6);  // one query per wave
-    uint8_t *const marks = mark_strips[threadIdx.x >> 6];
-    if (q >= p.n_vert) return;
+template <int C, int NB, int S, bool MAPPED, bool WINDOW, bool NESTED>
+__device__ __forceinline__ void search_query(const KnnParams &p, const int q, const int lane, uint8_t *const marks,
+                                             uint64_t *const buffer) {
+    constexpr bool kCollects = collects(C, NB, S, WINDOW);
     bool crowded = false;
     if constexpr (NESTED) {
         const int own_bin = uniform(p.bin_idx[q]) >> p.fine_bits;
         if (own_bin + 1 < p.n_bboundaries)
-            crowded = p.bin_boundaries[(size_t)(own_bin + 1) << p.boundary_shift] -
-                          p.bin_boundaries[(size_t)own_bin << p.boundary_shift] > p.fine_min_population;
+            crowded = p.bin_boundaries[own_bin + 1] -
+                          p.bin_boundaries[own_bin] > p.fine_min_population;
     }
 
     const int K = p.K;
@@ -743,16 +1219,23 @@ void knn_wave_kernel(const KnnParams p) {
     for (int s = 0; s < S; ++s) key[s] = kEmptyKey;
 
     if (searching) {
-        if constexpr (NESTED) {
-            if (!crowded) {
-                walk_shells<C, NB, S, MAPPED, WINDOW, false, NESTED>(p, q, lane, marks, Kn, floor_key, key);
-            } else if (!walk_shells<C, NB, S, MAPPED, WINDOW, true, NESTED>(p, q, lane, marks, Kn, floor_key, key)) {
-#pragma unroll
-                for (int s = 0; s < S; ++s) key[s] = kEmptyKey;
-                walk_shells<C, NB, S, MAPPED, WINDOW, false, NESTED>(p, q, lane, marks, Kn, floor_key, key);
+        if constexpr (kCollects) {
+            if constexpr (NESTED) {
+                if (!crowded || !collect_nearest<C, NB, S, MAPPED, true>(p, q, lane, marks, buffer, Kn, key))
+                    collect_nearest<C, NB, S, MAPPED, false>(p, q, lane, marks, buffer, Kn, key);
+            } else {
+                collect_nearest<C, NB, S, MAPPED, false>(p, q, lane, marks, buffer, Kn, key);
             }
         } else {
-            walk_shells<C, NB, S, MAPPED, WINDOW, false, NESTED>(p, q, lane, marks, Kn, floor_key, key);
+            bool found = false;
+            if constexpr (NESTED) {
+                found = crowded && walk_shells<C, NB, S, MAPPED, WINDOW, true, NESTED>(p, q, lane, marks, Kn, floor_key, key);
+                if (!found) {
+#pragma unroll
+                    for (int s = 0; s < S; ++s) key[s] = kEmptyKey;
+                }
+            }
+            if (!found) walk_shells<C, NB, S, MAPPED, WINDOW, false, NESTED>(p, q, lane, marks, Kn, floor_key, key);
         }
     }
 
@@ -772,10 +1255,22 @@ void knn_wave_kernel(const KnnParams p) {
     }
 }
 
+template <int C, int NB, int S, bool MAPPED, bool WINDOW = false, bool NESTED = false>
+__global__ __launch_bounds__(kWave)
+__attribute__((amdgpu_waves_per_eu(S <= 2 ? 8 : 1, 8)))
+void knn_wave_kernel(const KnnParams p) {
+    __shared__ __attribute__((aligned(8))) uint8_t marks[kMarkCap];
+    __shared__ uint64_t buffer[collects(C, NB, S, WINDOW) ? kBufferKeys : 1];
+    // queries come in bin order and differ a lot in cost from region to region:
+    // chunks of 512 of them are dealt to the XCDs in turn
+    const int q = xcd_chunked_block<512>(blockIdx.x, gridDim.x);
+    search_query<C, NB, S, MAPPED, WINDOW, NESTED>(p, q, lane_id(), marks, buffer);
+}
+
 template <int C, int NB, bool MAPPED>
 int launch_levels(const KnnParams &p, hipStream_t s) {
     const int levels = std::max(1, ceil_div(p.K - 1, kWave));
-    const dim3 grid(ceil_div(p.n_vert, kQueriesPerBlock)), block(kQueriesPerBlock * kWave);
+    const dim3 grid(p.n_vert), block(kWave);
     if (levels > kBulkInsertMaxRuns) {  // more neighbours than the registers hold: one launch per window of ranks
         KnnParams window = p;
         for (window.rank_base = 0; window.rank_base < p.K - 1; window.rank_base += kBulkInsertMaxRuns * kWave) {
@@ -811,7 +1306,9 @@ int launch_levels(const KnnParams &p, hipStream_t s) {
 // wrapper's default, or min(4, coordinates), the pipeline's own grid) get kernels with both
 // numbers fixed at compile time, anything else the one that reads them.
 template <bool MAPPED>
-int launch_coords(const KnnParams &p, hipStream_t s) {
+int launch_coords(const KnnParams &p, int bins_bound, hipStream_t s) {
+    // collect_nearest: 32-bit offsets into the table, 24-bit factors of bin numbers
+    if (p.n_bboundaries >= 1 << 30 || bins_bound >= 1 << 24) return launch_levels<0, 0, MAPPED>(p, s);
     if (p.n_coords == 2 && p.n_bin_dim == 2) return launch_levels<2, 2, MAPPED>(p, s);
     if (p.n_coords == 3 && p.n_bin_dim == 3) return launch_levels<3, 3, MAPPED>(p, s);
     if (p.n_coords == 4 && p.n_bin_dim == 3) return launch_levels<4, 3, MAPPED>(p, s);
@@ -830,11 +1327,11 @@ int launch_coords(const KnnParams &p, hipStream_t s) {
 }  // namespace
 
 int binned_select_knn_strided(const float *d_coord, const int *d_bin_idx, const int *d_direction,
-                              const int *d_dim_bin_idx, const int *d_bin_boundaries, int boundary_shift,
+                              const int *d_dim_bin_idx, const int *d_bin_boundaries,
                               const int *d_n_bins, const float *d_bin_width, const int *d_sorting,
                               const float *d_shift, float max_radius, int *d_indices, float *d_dist, int n_vert,
                               int n_neigh, int n_coords, int n_bin_dim, int n_bboundaries, int tf_compat,
-                              int use_direction, const int *d_cell_boundaries, int fine_bits,
+                              int use_direction, int bins_bound, const int *d_cell_boundaries, int fine_bits,
                               int fine_min_population, hipStream_t s) {
     // same conditions as the reference op (binned_select_knn_kernel.cc:336-352)
     HGC_REQUIRE(n_bin_dim > 1, "BinnedSelectKnnOp expects at least 2 binning dimensions.");
@@ -848,7 +1345,6 @@ int binned_select_knn_strided(const float *d_coord, const int *d_bin_idx, const 
     HGC_REQUIRE((unsigned long long)n_vert * (unsigned long long)n_coords * sizeof(float) < (1ull << 32),
                 "coordinate matrix must stay below 4 GiB");
     HGC_REQUIRE(n_bboundaries >= 2, "bin boundary table too short");
-    HGC_REQUIRE(boundary_shift >= 0 && boundary_shift < 8, "bad boundary stride");
     HGC_REQUIRE(fine_bits == 0 || (fine_bits == n_bin_dim && fine_bits <= 4),
                 "a nested grid has one bit per binned dimension, four at most");
     if (n_vert == 0) return HGC_OK;
@@ -882,12 +1378,11 @@ int binned_select_knn_strided(const float *d_coord, const int *d_bin_idx, const 
     p.n_bboundaries = n_bboundaries;
     p.tf_compat = tf_compat;
     p.use_direction = use_direction;
-    p.boundary_shift = boundary_shift;
     p.rank_base = 0;
     p.cell_boundaries = d_cell_boundaries;
     p.fine_bits = fine_bits;
     p.fine_min_population = fine_min_population;
-    return d_sorting ? launch_coords<true>(p, s) : launch_coords<false>(p, s);
+    return d_sorting ? launch_coords<true>(p, bins_bound, s) : launch_coords<false>(p, bins_bound, s);
 }
 
 }  // namespace hgc
@@ -902,9 +1397,9 @@ int hgc_binned_select_knn_fused(const float *d_coord, const int *d_bin_idx, cons
                                 const float *d_shift, float max_radius, int *d_indices, float *d_dist, int n_vert, int n_neigh,
                                 int n_coords, int n_bin_dim, int n_bboundaries, int tf_compat,
                                 int use_direction, hgc_stream_t stream) {
-    return binned_select_knn_strided(d_coord, d_bin_idx, d_direction, d_dim_bin_idx, d_bin_boundaries, 0, d_n_bins,
+    return binned_select_knn_strided(d_coord, d_bin_idx, d_direction, d_dim_bin_idx, d_bin_boundaries, d_n_bins,
                                      d_bin_width, d_sorting, d_shift, max_radius, d_indices, d_dist, n_vert, n_neigh,
-                                     n_coords, n_bin_dim, n_bboundaries, tf_compat, use_direction, nullptr, 0, 0,
+                                     n_coords, n_bin_dim, n_bboundaries, tf_compat, use_direction, n_bboundaries, nullptr, 0, 0,
                                      as_stream(stream));
 }
 
