@@ -240,120 +240,180 @@ __global__ __launch_bounds__(256) void exp_neg_grad_kernel(const float *gw, cons
 
 __device__ __forceinline__ float divide_no_nan(float a, float b) { return b == 0.f ? 0.f : a / b; }
 
-// Both kernels walk the slots four at a time, indices and weights one step ahead, so that a step's gathers are under
-// way together (one slot after the other: 40,000 vertices, K = 32, F = 8, C = 4 74 us for both, now 65). What bounds them is the L1's
-// address rate: index, weight and coordinates are the same for the lanes of a vertex. Workgroups of one XCD take consecutive vertices of the processing order.
-constexpr int kMomentSlots = 4;
+// A wave's 64 (vertex, feature) pairs belong to a few consecutive vertices of the processing order. It puts indices and
+// weights of 32 of their slots (16 where a wave has more than 16 vertices) into its own part of LDS, one lane per slot,
+// and each lane reads them there two slots per 16-byte load; the rows of four slots are gathered together.
+// Index and weight as loads of every lane (the same address for the lanes of a vertex) cost as much of the L1's address
+// rate as the gathers themselves: 40,000 vertices, K = 32, F = 8, C = 4 26 us for the means and 37 for the covariance
+// before, the whole call with its search 161 -> 141 us. What bounds them now is the latency of the gathered rows, at
+// five waves per SIMD.
+// Workgroups of one XCD take consecutive vertices.
+constexpr int kMomentSlots = 4, kMomentWaves = 4;
 
-struct SlotStep {
-    int j[kMomentSlots];  // -1: no neighbour
-    float w[kMomentSlots];
+struct alignas(8) Slot {
+    int j;  // -1: no neighbour
+    float w;
 };
 
-__device__ __forceinline__ void fetch_slots(const int *irow, const float *wrow, int n0, int n_neigh, int n_vert,
-                                            SlotStep &step) {
+// vertices that 64 consecutive pairs can belong to, slots of each that are in LDS at a time
+inline int moment_vertices(int n_feat) { return std::min(kWave, (kWave - 2 + n_feat) / n_feat + 1); }
+inline int moment_chunk(int n_feat) { return moment_vertices(n_feat) > 16 ? 16 : 32; }
+inline size_t moment_lds_bytes(int n_feat) {
+    // two slots of padding: rows of 36 or 68 dwords, the 16-byte reads of up to 16 vertices meet no bank twice
+    return (size_t)kMomentWaves * moment_vertices(n_feat) * (moment_chunk(n_feat) + 2) * sizeof(Slot);
+}
+
+// Calls term(j, w, valid) for the four slots of every step, in order, with the rows of a step requested by gather(u, j).
+template <typename Gather, typename Term>
+__device__ __forceinline__ void for_each_slot(Slot *const staged, const int lane, const int local, const int n_local,
+                                              const int my_row, const int chunk_bits, const int *__restrict__ idx,
+                                              const float *__restrict__ weights, const int n_neigh, const int n_vert,
+                                              Gather gather, Term term) {
+    const int chunk = 1 << chunk_bits, stride = chunk + 2;
+    const Slot *const mine = staged + local * stride;
+    for (int n0 = 0; n0 < n_neigh; n0 += chunk) {
+        for (int e0 = 0; e0 < n_local << chunk_bits; e0 += kWave) {
+            const int e = e0 + lane, v = e >> chunk_bits, n = n0 + (e & (chunk - 1));
+            const int row = __shfl(my_row, v & (kWave - 1));
+            if (v < n_local) {
+                Slot slot{-1, 0.f};
+                if (row >= 0 && n < n_neigh) {
+                    const int at = row * n_neigh + n;
+                    slot = {idx[at], weights[at]};
+                    if ((unsigned)slot.j >= (unsigned)n_vert) slot.j = -1;
+                }
+                staged[v * stride + (e & (chunk - 1))] = slot;
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int n_steps = min(chunk, n_neigh - n0);
+        for (int n = 0; n < n_steps; n += kMomentSlots) {
+            Slot slot[kMomentSlots];
 #pragma unroll
-    for (int u = 0; u < kMomentSlots; ++u) {
-        const int n = min(n0 + u, n_neigh - 1);
-        const int j = irow[n];
-        step.j[u] = n0 + u < n_neigh && (unsigned)j < (unsigned)n_vert ? j : -1;
-        step.w[u] = wrow[n];
+            for (int u = 0; u < kMomentSlots; u += 2) {
+                const int4 two = *reinterpret_cast<const int4 *>(mine + n + u);
+                slot[u] = {two.x, __int_as_float(two.y)};
+                slot[u + 1] = {two.z, __int_as_float(two.w)};
+            }
+            int any_missing = 0;
+#pragma unroll
+            for (int u = 0; u < kMomentSlots; ++u) {
+                gather(u, (unsigned)max(slot[u].j, 0));
+                any_missing |= slot[u].j;
+            }
+            if (__all(any_missing >= 0)) {
+#pragma unroll
+                for (int u = 0; u < kMomentSlots; ++u) term(u, slot[u].w);
+            } else {
+#pragma unroll
+                for (int u = 0; u < kMomentSlots; ++u)
+                    if (slot[u].j >= 0) term(u, slot[u].w);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // the next chunk overwrites what was read here
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
+// the pair a lane owns: vertex (-1 past the end) and feature, and its place among the wave's vertices
+struct MomentPair {
+    int v, f, local, n_local, row_of_lane;
+};
+
+__device__ __forceinline__ MomentPair moment_pair(const int *__restrict__ order, const int lane, int n_vert, int n_feat) {
+    const long long wave_first = ((long long)xcd_contiguous_block(blockIdx.x, gridDim.x) * kMomentWaves + (threadIdx.x >> 6)) * kWave;
+    const long long t = wave_first + lane;
+    const int first = (int)(wave_first / n_feat), i = (int)(t / n_feat);
+    MomentPair m;
+    m.f = (int)(t - (long long)i * n_feat);
+    m.local = i - first;
+    m.n_local = min((int)((wave_first + kWave - 1) / n_feat), n_vert - 1) - first + 1;
+    // processing order with locality: results do not depend on it
+    int row = -1;
+    if (lane < m.n_local) row = order ? order[first + lane] : first + lane;
+    if ((unsigned)row >= (unsigned)n_vert) row = -1;
+    m.row_of_lane = row;
+    const int v = __shfl(row, m.local & (kWave - 1));
+    m.v = i < n_vert ? v : -1;
+    return m;
+}
+
 template <int C>
-__global__ __launch_bounds__(256) void neighbour_means_kernel(const float *__restrict__ coords,
-                                                              const float *__restrict__ weights,
-                                                              const float *__restrict__ feats, const int *__restrict__ idx,
-                                                              float *__restrict__ sumw, float *__restrict__ means,
-                                                              const int *__restrict__ order, int n_vert, int n_feat,
-                                                              int n_neigh) {
-    const long long t = (long long)xcd_contiguous_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    const int i = (int)(t / n_feat);
-    if (i >= n_vert) return;
-    const int f = (int)(t - (long long)i * n_feat);
-    const int v = order ? order[i] : i;  // processing order with locality: results do not depend on it
-    if ((unsigned)v >= (unsigned)n_vert) return;
-    const float kf = (float)n_neigh;
-    const int *irow = idx + (size_t)v * n_neigh;
-    const float *wrow = weights + (size_t)v * n_neigh;
-    float s = 0.f, sc[C];
+__global__ __launch_bounds__(kMomentWaves *kWave) void neighbour_means_kernel(
+    const float *__restrict__ coords, const float *__restrict__ weights, const float *__restrict__ feats,
+    const int *__restrict__ idx, float *__restrict__ sumw, float *__restrict__ means, const int *__restrict__ order,
+    int n_vert, int n_feat, int n_neigh, int chunk_bits, int wave_slots) {
+    extern __shared__ __align__(16) char s_slots[];
+    Slot *const staged = reinterpret_cast<Slot *>(s_slots) + (threadIdx.x >> 6) * wave_slots;
+    const int lane = threadIdx.x & (kWave - 1);
+    const MomentPair m = moment_pair(order, lane, n_vert, n_feat);
+    if (m.n_local <= 0) return;
+    const int local = m.v >= 0 ? m.local : 0;
+    float s = 0.f, sc[C], a[kMomentSlots], x[kMomentSlots][C];
 #pragma unroll
     for (int c = 0; c < C; ++c) sc[c] = 0.f;
-    SlotStep next;
-    fetch_slots(irow, wrow, 0, n_neigh, n_vert, next);
-    for (int n0 = 0; n0 < n_neigh; n0 += kMomentSlots) {
-        const SlotStep now = next;
-        float a[kMomentSlots], x[kMomentSlots][C];
-#pragma unroll
-        for (int u = 0; u < kMomentSlots; ++u) {
-            const size_t j = max(now.j[u], 0);
-            a[u] = feats[j * n_feat + f];
+    for_each_slot(
+        staged, lane, local, m.n_local, m.row_of_lane, chunk_bits, idx, weights, n_neigh, n_vert,
+        [&](int u, unsigned j) {
+            a[u] = feats[j * (unsigned)n_feat + m.f];
 #pragma unroll
             for (int c = 0; c < C; ++c) x[u][c] = coords[j * C + c];
-        }
-        if (n0 + kMomentSlots < n_neigh) fetch_slots(irow, wrow, n0 + kMomentSlots, n_neigh, n_vert, next);
+        },
+        [&](int u, float w) {
+            s = s + a[u] * w;
 #pragma unroll
-        for (int u = 0; u < kMomentSlots; ++u) {
-            if (now.j[u] < 0) continue;
-            s = s + a[u] * now.w[u];
-#pragma unroll
-            for (int c = 0; c < C; ++c) sc[c] = sc[c] + (x[u][c] * a[u]) * now.w[u];
-        }
-    }
+            for (int c = 0; c < C; ++c) sc[c] = sc[c] + (x[u][c] * a[u]) * w;
+        });
+    if (m.v < 0) return;
+    const float kf = (float)n_neigh;
     const float S = (s / kf) * kf;
-    sumw[(size_t)v * n_feat + f] = S;
+    const size_t out = (size_t)m.v * n_feat + m.f;
+    sumw[out] = S;
 #pragma unroll
-    for (int c = 0; c < C; ++c) means[((size_t)v * n_feat + f) * C + c] = divide_no_nan((sc[c] / kf) * kf, S + 1e-3f);
+    for (int c = 0; c < C; ++c) means[out * C + c] = divide_no_nan((sc[c] / kf) * kf, S + 1e-3f);
 }
 
 template <int C>
-__global__ __launch_bounds__(256) void neighbour_covariance_kernel(const float *__restrict__ coords,
-                                                                   const float *__restrict__ weights,
-                                                                   const float *__restrict__ feats,
-                                                                   const int *__restrict__ idx,
-                                                                   const float *__restrict__ sumw,
-                                                                   const float *__restrict__ means, float *__restrict__ cov,
-                                                                   const int *__restrict__ order, int n_vert, int n_feat,
-                                                                   int n_neigh) {
-    const long long t = (long long)xcd_contiguous_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    const int i = (int)(t / n_feat);
-    if (i >= n_vert) return;
-    const int f = (int)(t - (long long)i * n_feat);
-    const int v = order ? order[i] : i;
-    if ((unsigned)v >= (unsigned)n_vert) return;
-    const float kf = (float)n_neigh;
-    const int *irow = idx + (size_t)v * n_neigh;
-    const float *wrow = weights + (size_t)v * n_neigh;
-    float acc[C][C];  // the lower triangle is accumulated, the products are symmetric bit for bit
+__global__ __launch_bounds__(kMomentWaves *kWave) void neighbour_covariance_kernel(
+    const float *__restrict__ coords, const float *__restrict__ weights, const float *__restrict__ feats,
+    const int *__restrict__ idx, const float *__restrict__ sumw, const float *__restrict__ means, float *__restrict__ cov,
+    const int *__restrict__ order, int n_vert, int n_feat, int n_neigh, int chunk_bits, int wave_slots) {
+    extern __shared__ __align__(16) char s_slots[];
+    Slot *const staged = reinterpret_cast<Slot *>(s_slots) + (threadIdx.x >> 6) * wave_slots;
+    const int lane = threadIdx.x & (kWave - 1);
+    const MomentPair m = moment_pair(order, lane, n_vert, n_feat);
+    if (m.n_local <= 0) return;
+    const int local = m.v >= 0 ? m.local : 0;
+    // the lower triangle is accumulated, the products are symmetric bit for bit
+    float acc[C][C], a[kMomentSlots], x[kMomentSlots][C], mean[kMomentSlots][C];
 #pragma unroll
     for (int c = 0; c < C; ++c)
 #pragma unroll
         for (int d = 0; d < C; ++d) acc[c][d] = 0.f;
-    SlotStep next;
-    fetch_slots(irow, wrow, 0, n_neigh, n_vert, next);
-    for (int n0 = 0; n0 < n_neigh; n0 += kMomentSlots) {
-        const SlotStep now = next;
-        float a[kMomentSlots], cen[kMomentSlots][C];
+    for_each_slot(
+        staged, lane, local, m.n_local, m.row_of_lane, chunk_bits, idx, weights, n_neigh, n_vert,
+        [&](int u, unsigned j) {
+            const unsigned at = j * (unsigned)n_feat + m.f;
+            a[u] = feats[at];
 #pragma unroll
-        for (int u = 0; u < kMomentSlots; ++u) {
-            const size_t j = max(now.j[u], 0);
-            a[u] = feats[j * n_feat + f];
+            for (int c = 0; c < C; ++c) x[u][c] = coords[j * C + c], mean[u][c] = means[(size_t)at * C + c];
+        },
+        [&](int u, float w) {
+            float cen[C];
 #pragma unroll
-            for (int c = 0; c < C; ++c) cen[u][c] = coords[j * C + c] - means[(j * n_feat + f) * C + c];
-        }
-        if (n0 + kMomentSlots < n_neigh) fetch_slots(irow, wrow, n0 + kMomentSlots, n_neigh, n_vert, next);
-#pragma unroll
-        for (int u = 0; u < kMomentSlots; ++u) {
-            if (now.j[u] < 0) continue;
+            for (int c = 0; c < C; ++c) cen[c] = x[u][c] - mean[u][c];
 #pragma unroll
             for (int c = 0; c < C; ++c)
 #pragma unroll
-                for (int d = 0; d <= c; ++d) acc[c][d] = acc[c][d] + ((cen[u][c] * cen[u][d]) * a[u]) * now.w[u];
-        }
-    }
-    const float den = sumw[(size_t)v * n_feat + f] + 1e-3f;
-    float *out = cov + ((size_t)v * n_feat + f) * C * C;
+                for (int d = 0; d <= c; ++d) acc[c][d] = acc[c][d] + ((cen[c] * cen[d]) * a[u]) * w;
+        });
+    if (m.v < 0) return;
+    const float kf = (float)n_neigh;
+    const size_t at = (size_t)m.v * n_feat + m.f;
+    const float den = sumw[at] + 1e-3f;
+    float *out = cov + at * C * C;
 #pragma unroll
     for (int c = 0; c < C; ++c)
 #pragma unroll
@@ -364,13 +424,16 @@ template <int C>
 int launch_neighbour_covariance(const float *coords, const float *weights, const float *feats, const int *idx, float *cov,
                                 float *means, float *sumw, const int *order, int n_vert, int n_feat, int n_neigh,
                                 hipStream_t s) {
-    const int blocks = ceil_div((long long)n_vert * n_feat, 256);
-    neighbour_means_kernel<C><<<blocks, 256, 0, s>>>(coords, weights, feats, idx, sumw, means, order, n_vert, n_feat,
-                                                     n_neigh);
+    const int blocks = ceil_div((long long)n_vert * n_feat, kMomentWaves * kWave);
+    const int chunk = moment_chunk(n_feat), chunk_bits = chunk == 32 ? 5 : 4;
+    const int wave_slots = moment_vertices(n_feat) * (chunk + 2);
+    const size_t lds = moment_lds_bytes(n_feat);
+    neighbour_means_kernel<C><<<blocks, kMomentWaves * kWave, lds, s>>>(coords, weights, feats, idx, sumw, means, order,
+                                                                        n_vert, n_feat, n_neigh, chunk_bits, wave_slots);
     int rc = check_launch("neighbour_means_kernel");
     if (rc) return rc;
-    neighbour_covariance_kernel<C><<<blocks, 256, 0, s>>>(coords, weights, feats, idx, sumw, means, cov, order, n_vert,
-                                                          n_feat, n_neigh);
+    neighbour_covariance_kernel<C><<<blocks, kMomentWaves * kWave, lds, s>>>(
+        coords, weights, feats, idx, sumw, means, cov, order, n_vert, n_feat, n_neigh, chunk_bits, wave_slots);
     return check_launch("neighbour_covariance_kernel");
 }
 
