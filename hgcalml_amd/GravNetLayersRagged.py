@@ -43,6 +43,15 @@ def _sum_rows(t):
     return ops.column_sums(t.reshape(t.shape[0], -1)).view(t.shape[1:])
 
 
+def _weight_grad_in_one_pass(g, x):
+    """Whether weight and bias gradient of a dense layer come from the library's one pass over g and x. Wide layers over
+    many rows are the batched product's (us with the bias' sums, one pass / batched: 240,000 rows, 160 x 352 376 / 290;
+    150,000, 160 x 256 140 / 135, 128 x 256 101 / 115; 60,000, 160 x 352 104 / 121; 20,000 43 / 69)."""
+    widths = g.shape[1] * x.shape[1]
+    return (not torch.is_grad_enabled() and _library_takes(g, x) and
+            (widths <= 1 << 15 or (widths <= 1 << 16 and x.shape[0] <= 1 << 16)))
+
+
 class _DropSelfFn(torch.autograd.Function):
     """table and distances without the self column, and the distances themselves: the gradients of both come back in
     one pass. The distances leave as a tensor of their own on the same memory, which may be written to (an input handed
@@ -83,9 +92,9 @@ class _JoinFn(torch.autograd.Function):
 
 
 class _TallLinearFn(torch.autograd.Function):
-    """y = x W^T + b for x of very many rows. The weight gradient g^T x reduces over those rows
-    into a small matrix; as one GEMM it runs on a handful of workgroups (0.35-0.44 ms for 150k rows
-    of 64-192 columns), as a batch of 64 row slices added up afterwards it takes 0.07-0.11 ms."""
+    """y = x W^T + b for x of very many rows. The weight gradient g^T x reduces over those rows into a small matrix; as one
+    GEMM it runs on a handful of workgroups (0.35-0.44 ms for 150k rows of 64-192 columns). The library's pass forms it
+    together with the bias gradient; where that one is not taken, a batch of 64 row slices is added up afterwards."""
 
     SLICES = 64
 
@@ -101,6 +110,10 @@ class _TallLinearFn(torch.autograd.Function):
         g = g.contiguous()
         grad_x = g @ weight if ctx.needs_input_grad[0] else None
         grad_w = None
+        want_b = ctx.has_bias and ctx.needs_input_grad[2]
+        if ctx.needs_input_grad[1] and _weight_grad_in_one_pass(g, x):
+            grad_w, grad_b = ops.dense_weight_grad(g, x)
+            return grad_x, grad_w, grad_b if want_b else None
         if ctx.needs_input_grad[1]:
             n, s = x.shape[0], _TallLinearFn.SLICES
             whole = n // s * s
@@ -112,7 +125,7 @@ class _TallLinearFn(torch.autograd.Function):
                     grad_w = grad_w + g[whole:].t() @ x[whole:]
             else:
                 grad_w = g.t() @ x
-        grad_b = _sum_rows(g) if ctx.has_bias and ctx.needs_input_grad[2] else None
+        grad_b = _sum_rows(g) if want_b else None
         return grad_x, grad_w, grad_b
 
 

@@ -80,6 +80,8 @@ _SIGNATURES = {
     "hgc_sumw_distance_grad": (_c_int, [_ptr] * 3 + [_c_int] * 2 + [_ptr] * 2),
     "hgc_column_sums_workspace_bytes": (_c_size, [_c_int] * 2),
     "hgc_column_sums": (_c_int, [_ptr] + [_c_int] * 2 + [_ptr] * 2 + [_c_size, _ptr]),
+    "hgc_dense_weight_grad_workspace_bytes": (_c_size, [ctypes.c_longlong] + [_c_int] * 2),
+    "hgc_dense_weight_grad": (_c_int, [_ptr] * 2 + [ctypes.c_longlong] + [_c_int] * 2 + [_ptr] * 3 + [_c_size, _ptr]),
     "hgc_binned_assign_to_condensates_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int]),
     "hgc_binned_assign_to_condensates": (_c_int, [_c_int, _c_int] + [_ptr] * 21 + [_c_int] * 4 + [_ptr, _ptr, _c_size, _ptr]),
     "hgc_build_and_assign_condensates_workspace_bytes": (_c_size, [_c_int] * 5),

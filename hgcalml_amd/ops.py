@@ -816,6 +816,23 @@ def column_sums(x):
     return out
 
 
+@_op("dense_weight_grad(Tensor grad, Tensor x) -> (Tensor, Tensor)")
+def dense_weight_grad(grad, x):
+    """(grad.t() @ x, grad.sum(0)) of float32 matrices of very many rows: weight and bias gradient of a dense layer"""
+    dev = require_device(grad, x)
+    grad, x = f32(grad), f32(x)
+    (n, n_out), n_in = grad.shape, x.shape[1]
+    if x.shape[0] != n:
+        raise ValueError("dense_weight_grad expects as many rows of x as of the gradient")
+    weight = torch.empty((n_out, n_in), dtype=torch.float32, device=dev)
+    bias = torch.empty((n_out,), dtype=torch.float32, device=dev)
+    need = lib.hgc_dense_weight_grad_workspace_bytes(n, n_out, n_in)
+    ws = workspace(need, dev) if need else None
+    check(lib.hgc_dense_weight_grad(p(grad), p(x), n, n_out, n_in, p(weight), p(bias), p(ws), ws.numel() if need else 0,
+                                    stream()))
+    return weight, bias
+
+
 # --------------------------------------------------------------------------- shapes without data
 
 # Fake ("meta") implementations: output shapes and dtypes from input shapes alone, so that
@@ -955,6 +972,11 @@ def _(grad, n_features, for_accumulated, for_features, for_x):
 @torch.library.register_fake("hgcalml::column_sums")
 def _(x):
     return _f32_like((x.shape[1],), x)
+
+
+@torch.library.register_fake("hgcalml::dense_weight_grad")
+def _(grad, x):
+    return _f32_like((grad.shape[1], x.shape[1]), grad), _f32_like((grad.shape[1],), grad)
 
 
 @torch.library.register_fake("hgcalml::sumw_normalise")

@@ -631,6 +631,16 @@ size_t hgc_column_sums_workspace_bytes(int n_rows, int n_cols);
 int hgc_column_sums(const float *d_x, int n_rows, int n_cols, float *d_sums, void *workspace,
                     size_t workspace_bytes, hgc_stream_t stream);
 
+/* Gradients of a dense layer y = x W^T + b over row-major matrices grad
+ * [n_rows, n_out] and x [n_rows, n_in]: weight [n_out, n_in] = grad^T x and
+ * bias [n_out] = sum over the rows of grad (d_bias_grad may be NULL), in a fixed
+ * order; n_out * n_in <= 2^20. The query returns 0 where one launch does it and a
+ * NULL workspace is accepted. No counterpart in the reference (Keras does it). */
+size_t hgc_dense_weight_grad_workspace_bytes(long long n_rows, int n_out, int n_in);
+int hgc_dense_weight_grad(const float *d_grad, const float *d_x, long long n_rows, int n_out,
+                          int n_in, float *d_weight_grad, float *d_bias_grad, void *workspace,
+                          size_t workspace_bytes, hgc_stream_t stream);
+
 /* Greedy highest-beta-first condensate selection and hit assignment per event.
  * Replaces BinnedCondensatesFinderOpFunctor
  * (modules/compiled/binned_assign_to_condensates_kernel.h, _kernel.cc:23-241);
