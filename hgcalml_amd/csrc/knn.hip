@@ -766,7 +766,7 @@ __device__ __forceinline__ int cut_to_smallest(uint64_t *const buffer, const int
             }
         }
         if (left > most) {  // more than `most` - Kn keys share the Kn-th distance
-            uint32_t tie_lo = 0;  // fewer than Kn keys with this limit, or 0
+            uint32_t tie_lo = 0;  // fewer than Kn keys with this limit, or 0 (Kn at most)
             while (left > most && tie_limit - tie_lo > 1) {
                 const uint32_t mid = tie_lo + ((tie_limit - tie_lo) >> 1);
                 const uint64_t limit = (uint64_t)hi << 32 | mid;
@@ -780,6 +780,8 @@ __device__ __forceinline__ int cut_to_smallest(uint64_t *const buffer, const int
                     tie_lo = mid;
                 }
             }
+            // one too many with the limit 1: points 0 and 1 share the Kn-th distance, and point 0 completes the list
+            if (left > most) tie_limit = 0;
         }
         const uint64_t limit = (uint64_t)hi << 32 | tie_limit;
         int at = 0;

@@ -73,6 +73,20 @@ def test_matches_brute_force(dims, kind, K, radius, directed):
 
 
 @pytest.mark.parametrize("dims", [2, 3, 4])
+@pytest.mark.parametrize("K", [17, 65, 129])  # a list that fills its registers exactly, and one that does not
+def test_first_two_points_share_the_last_distance(dims, K):
+    """points 0 and 1 coincide and are the farthest ones of a query that has one neighbour too many"""
+    gen = torch.Generator().manual_seed(dims)
+    x = torch.rand(K + 1, dims, generator=gen) * 0.3 + 0.7
+    x[:2] = 0.0
+    idx, dist = BinnedSelectKnn(K, x.to(DEV), torch.tensor([0, K + 1], dtype=torch.int32, device=DEV))
+    want = brute_force(x, [0, K + 1], K, 0, None)
+    assert (want[0][2:, K - 1] == 0).all()
+    assert torch.equal(idx.cpu(), want[0])
+    assert torch.equal(dist.cpu().view(torch.int32), want[1].view(torch.int32))
+
+
+@pytest.mark.parametrize("dims", [2, 3, 4])
 @pytest.mark.parametrize("bad", [float("inf"), -float("inf"), float("nan")])
 def test_unbounded_coordinates_end(dims, bad):
     """one such coordinate leaves bin widths without a meaning: the search ends and the finite points keep each other"""
