@@ -980,7 +980,9 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
     int d_in = -1;   // the cube of this half-width has been walked (-1: none)
     for (;;) {
         const bool bounded = prunes && cut < 0x7f000000u;
-        const bool last_pass = bounded && d_in >= 0;  // everything within the bound
+        // Everything within the bound; where the list is not full and a radius reaches far, larger cubes come first (with
+        // radius 3 in the unit square, 60,000 points, K = 40 one pass over everything takes 1045 us, this 102).
+        const bool last_pass = bounded && d_in >= 0 && (n_kept >= Kn || d_radius <= 2 * d_in + 2);
         int below[B], width[B], below_in[B], width_in[B];
         float inv_width[B], inv_width_in[B];
         int n_rows = 1, n_inner = 1, lo_last = 0, hi_last = 0, first_bin = 0, P = 1, n_slots = 1;

@@ -73,6 +73,19 @@ def test_matches_brute_force(dims, kind, K, radius, directed):
 
 
 @pytest.mark.parametrize("dims", [2, 3, 4])
+@pytest.mark.parametrize("K,radius", [(17, 0.02), (17, 0.2), (40, 0.9), (40, 5.0), (100, 5.0)])
+@pytest.mark.parametrize("kind", ["uniform", "clump", "line"])
+def test_radius_of_many_bins(dims, K, radius, kind):
+    """from a radius inside one bin to one that reaches across the grid while the first bins hold too few points"""
+    gen = torch.Generator().manual_seed(dims)
+    x = points(kind, 3000, dims, gen) ** 2  # denser towards one corner
+    got = BinnedSelectKnn(K, x.to(DEV), torch.tensor([0, 3000], dtype=torch.int32, device=DEV), max_radius=radius)
+    want = brute_force(x, [0, 3000], K, radius, None)
+    assert torch.equal(got[0].cpu(), want[0])
+    assert torch.equal(got[1].cpu().view(torch.int32), want[1].view(torch.int32))
+
+
+@pytest.mark.parametrize("dims", [2, 3, 4])
 @pytest.mark.parametrize("K", [17, 65, 129])  # a list that fills its registers exactly, and one that does not
 def test_first_two_points_share_the_last_distance(dims, K):
     """points 0 and 1 coincide and are the farthest ones of a query that has one neighbour too many"""
