@@ -932,11 +932,29 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
                 cell = (int)__umul24(cell, nb[i]) + k;
             }
         }
+        // What the radius leaves of a row: with bins wider than the radius the cube is mostly beyond it (60,000 4-D Gaussian
+        // points, radius 0.1, K = 40: 139 -> 82 us a call; 16 events of 1.14 M points, radius 0.1: 1183 -> 1171).
+        int lo_most = 1 << 30, hi_most = 1 << 30;
+        if (has_radius && prunes) {
+            float gap2 = 0.f;
+#pragma unroll
+            for (int i = 0; i < B - 1; ++i) {
+                const float of = (float)off[i];
+                const float g = fmaxf(fmaxf(of - from_upper[i], -of - from_lower[i]), 0.f);
+                gap2 = __builtin_fmaf(g, g, gap2);
+            }
+            const float rest = bound_of(cut) - gap2 * gap_scale;
+            const float span = __builtin_amdgcn_sqrtf(fmaxf(rest, 0.f)) * bins_per_unit + 1.001f;
+            in_grid = in_grid && rest >= 0.f;
+            lo_most = (int)fminf(span - tl_last, 1.0e9f);
+            hi_most = (int)fminf(span - tu_last, 1.0e9f);
+        }
         if constexpr (FINE) {
             const int own = uniform(p.cell_boundaries[own_cell + 1]) - uniform(p.cell_boundaries[own_cell]);
             d_out = own > enough ? 0 : 1;
             const int bin_last = ((qb_last - 1) >> 1) + (lane & 1);
-            const int lo = max(max(qb_last - d_out, 0), 2 * bin_last), hi = min(min(qb_last + d_out, nb_last - 1), 2 * bin_last + 1);
+            const int lo = max(max(qb_last - min(d_out, lo_most), 0), 2 * bin_last);
+            const int hi = min(min(qb_last + min(d_out, hi_most), nb_last - 1), 2 * bin_last + 1);
             const int bin = event_base + (int)__umul24(cell, bins_last) + bin_last;
             if (in_grid && ring <= d_out && lo <= hi && bin + 1 < p.n_bboundaries) {
                 const int base = ((bin << (B - 1)) | halves) << 1;
@@ -948,12 +966,12 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
             // lanes without a row look at the own one
             const int row = in_grid ? event_base + (int)__umul24(cell, nb_last) : own_bin - qb_last;
             auto look = [&](int d) {  // the part of the row inside the cube of half-width d
-                const int from = max(qb_last - d, 0), to = min(qb_last + d, nb_last - 1) + 1;
+                const int from = max(qb_last - min(d, lo_most), 0), to = min(qb_last + min(d, hi_most), nb_last - 1) + 1;
                 const bool wanted = in_grid && ring <= d && row < p.n_bboundaries - to;
                 seg_start = seg_len = 0;
                 if (wanted) {
-                    seg_start = table_entry(p.bin_boundaries + from, row);
-                    seg_len = table_entry(p.bin_boundaries + to, row) - seg_start;
+                    seg_start = table_entry(p.bin_boundaries, row + from);
+                    seg_len = table_entry(p.bin_boundaries, row + to) - seg_start;
                 }
                 if (p.status && in_grid && ring <= d && !wanted)  // the reference prints "idx out of range" and skips the bin
                     atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
