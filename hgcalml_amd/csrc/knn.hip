@@ -688,7 +688,7 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
 
 // ---- the search of up to 129 neighbours: collect, cut, sort once ----
 //
-// Bound by the issue of vector instructions (90 % busy), as walk_shells is, and most of those went into resolving the
+// Bound by the issue of vector instructions (80 % busy), as walk_shells is, and most of those went into resolving the
 // segments of one small shell after another, steps with a few candidates, and sorted inserts of keys that leave the
 // list again. Here a query collects candidates, unsorted, in LDS:
 //   * first the cube of bins around it that holds enough points (the boundary table says how many, before any
@@ -697,7 +697,7 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
 //   * then one pass over the rows of bins outside the cube that the bound reaches;
 //   * then the keys that are left are sorted, once.
 // Vector instructions per query: 16 events of 1.14 M 3-D points, K = 32, radius 0.1 about 700 -> 465, 150,000 4-D
-// points, K = 65 1475 -> 1126. The whole search, by shells -> collected: these two 1399 -> 1173 us and 429 -> 372 us;
+// points, K = 65 1475 -> 1087. The whole search, by shells -> collected: these two 1399 -> 1173 us and 429 -> 372 us;
 // 240,000 3-D points, K = 41 367 -> 307; 4-D Gaussian, K = 65 467 -> 410; 4-D uniform, K = 64 361 -> 305; 2-D
 // clusters, K = 32 186 -> 130; 3-D clusters, K = 96 489 -> 319. Tried and taken back: first regions that leave out the
 // corners of the cube (fewer candidates, but a second pass for every query: 4 to 13 % slower), up to three pieces of a
