@@ -382,9 +382,10 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
                 grid_rows = min(grid_rows * nb[i], 1ll << 40);
                 rows_fit = rows_fit && nb[i] < (1 << 13);
             }
-            if (!rows_fit || grid_rows >= (1ll << 22)) {
+            if (!rows_fit || grid_rows >= (1ll << 22) || event_base < 0) {  // or a bin that no grid gives
                 if (FINE) return false;  // the grid of bins may do
-                if (p.status && lane == 0) atomicOr(p.status, HGC_FLAG_SHELL_TOO_WIDE);
+                if (p.status && lane == 0)
+                    atomicOr(p.status, event_base < 0 ? HGC_FLAG_BIN_BEYOND_TABLE : HGC_FLAG_SHELL_TOO_WIDE);
                 return true;  // the list stays empty
             }
         }
@@ -397,7 +398,7 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
         // with shell 1: every row of that shell then takes its whole run of the last
         // dimension, and the run of the centre row contains the own bin.
         bool with_own_bin = false;
-        if (reach_max > 0 && own_bin + 1 < p.n_bboundaries) {
+        if (reach_max > 0 && own_bin >= 0 && own_bin + 1 < p.n_bboundaries) {
             if (FINE)
                 with_own_bin = p.cell_boundaries[own_cell + 1] - p.cell_boundaries[own_cell] <= Kn;
             else
@@ -834,10 +835,22 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
     const int own_bin = own_cell >> p.fine_bits;
     const int dim = min(lane, B - 1);
     int nb_v = p.n_bins[dim], qb_v = p.dim_bin_idx[(size_t)q * (B + 1) + 1 + dim];
-    int in_event = 0;  // number of the own bin inside its event
+    int in_event = 0, cells_per_event = 1;  // number of the own bin inside its event
 #pragma unroll
-    for (int i = 0; i < B; ++i) in_event = in_event * readlane_i32(nb_v, i) + readlane_i32(qb_v, i);
-    const int event_base = own_bin - in_event;
+    for (int i = 0; i < B; ++i) {
+        in_event = in_event * readlane_i32(nb_v, i) + readlane_i32(qb_v, i);
+        cells_per_event *= readlane_i32(nb_v, i);
+    }
+    int event_base = uniform(p.dim_bin_idx[(size_t)q * (B + 1)]) * cells_per_event;
+    bool placed = own_bin - event_base == in_event && !__builtin_amdgcn_ballot_w64((uint32_t)qb_v >= (uint32_t)nb_v);
+    if (!placed) {
+        // The bin says which event it is (a division, which rows of a binning are spared). A row outside the grid, or of
+        // another bin than the own one, does not say where the query is: then the whole grid of the event is walked
+        // from the nearest bin inside, and nothing is pruned.
+        event_base = own_bin - own_bin % max(cells_per_event, 1);
+        placed = own_bin - event_base == in_event && !__builtin_amdgcn_ballot_w64((uint32_t)qb_v >= (uint32_t)nb_v);
+        if (!placed) qb_v = max(min(qb_v, nb_v - 1), 0);
+    }
     if (FINE) {
         nb_v *= 2;
         qb_v = 2 * qb_v + ((own_cell >> (B - 1 - dim)) & 1);
@@ -865,7 +878,7 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
     }
     const float bw = FINE ? 0.5f * p.bin_width[0] : p.bin_width[0];
     // Coordinates without bounds leave widths without a meaning: then nothing is pruned, the whole grid is walked.
-    const bool prunes = bw > 1e-30f && bw < 1e18f;  // (the square stays finite)
+    const bool prunes = placed && bw > 1e-30f && bw < 1e18f;  // (the square stays finite)
     const float inv_bw = __builtin_amdgcn_rcpf(bw);  // within an ulp; used with margins of a thousandth of a bin
     const float bins_per_unit = prunes ? 1.001f * inv_bw : 3.0e38f;
     const float gap_scale = prunes ? 0.999f * (bw * bw) : 0.f;  // bounds are generous by 0.1 %
@@ -956,25 +969,29 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
             const int lo = max(max(qb_last - min(d_out, lo_most), 0), 2 * bin_last);
             const int hi = min(min(qb_last + min(d_out, hi_most), nb_last - 1), 2 * bin_last + 1);
             const int bin = event_base + (int)__umul24(cell, bins_last) + bin_last;
-            if (in_grid && ring <= d_out && lo <= hi && bin + 1 < p.n_bboundaries) {
-                const int base = ((bin << (B - 1)) | halves) << 1;
-                seg_start = table_entry(p.cell_boundaries, base | (lo & 1));
-                seg_len = table_entry(p.cell_boundaries, (base | (hi & 1)) + 1) - seg_start;
+            if (in_grid && ring <= d_out && lo <= hi) {
+                if (bin + 1 < p.n_bboundaries) {
+                    const int base = ((bin << (B - 1)) | halves) << 1;
+                    seg_start = table_entry(p.cell_boundaries, base | (lo & 1));
+                    seg_len = table_entry(p.cell_boundaries, (base | (hi & 1)) + 1) - seg_start;
+                } else if (p.status) {
+                    atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
+                }
             }
         } else {
             constexpr int kCubes = B == 4 ? 1 : 3;
-            // lanes without a row look at the own one
-            const int row = in_grid ? event_base + (int)__umul24(cell, nb_last) : own_bin - qb_last;
+            const int row = event_base + (int)__umul24(cell, nb_last);
             auto look = [&](int d) {  // the part of the row inside the cube of half-width d
                 const int from = max(qb_last - min(d, lo_most), 0), to = min(qb_last + min(d, hi_most), nb_last - 1) + 1;
-                const bool wanted = in_grid && ring <= d && row < p.n_bboundaries - to;
                 seg_start = seg_len = 0;
-                if (wanted) {
-                    seg_start = table_entry(p.bin_boundaries, row + from);
-                    seg_len = table_entry(p.bin_boundaries, row + to) - seg_start;
+                if (in_grid && ring <= d && from < to) {
+                    if (row < p.n_bboundaries - to) {
+                        seg_start = table_entry(p.bin_boundaries, row + from);
+                        seg_len = table_entry(p.bin_boundaries, row + to) - seg_start;
+                    } else if (p.status) {  // the reference prints "idx out of range" and skips the bin
+                        atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
+                    }
                 }
-                if (p.status && in_grid && ring <= d && !wanted)  // the reference prints "idx out of range" and skips the bin
-                    atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
                 return readlane_i32(wave_inclusive_sum(seg_len), kWave - 1);
             };
             d_out = 1;
@@ -985,7 +1002,7 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
                     d_out = 3;
                     look(3);
                 }
-            } else if (held > 4 * enough && own_bin + 1 < p.n_bboundaries &&
+            } else if (held > 4 * enough && placed && own_bin + 1 < p.n_bboundaries &&
                        uniform(p.bin_boundaries[own_bin + 1]) - uniform(p.bin_boundaries[own_bin]) > enough) {
                 d_out = 0;  // crowded: the own bin does
                 look(0);

@@ -1,0 +1,91 @@
+"""The raw search op on rows and tables that no grid of this package gives: rows outside the grid or of another bin, and
+boundary tables that end early. Nothing is read beyond a table, and what the table holds is answered."""
+import numpy as np
+import pytest
+import torch
+
+from test_data_errors import _status_after
+from test_gpu_collected_search import brute_force
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+SPLITS = [0, 250, 600]
+
+
+class Binned:
+    """two events in bin order with the tables of the reference's own binning, and the op on them"""
+
+    def __init__(self, oracle, dims, n_bins=5):
+        rng = np.random.default_rng(dims)
+        x = rng.random((SPLITS[-1], dims)).astype(np.float32)
+        self.rows, self.flat, self.n_bins, self.width, count = oracle.BinByCoordinates(x, np.array(SPLITS, np.int32), n_bins=n_bins)
+        order = np.argsort(self.flat, kind="stable")
+        self.x, self.rows, self.flat = x[order], self.rows[order].copy(), self.flat[order]
+        self.bounds = np.concatenate([[0], np.cumsum(count)]).astype(np.int32)
+        self.cells = int(np.prod(self.n_bins))
+
+    def search(self, K, radius=0.0, table=None, rows=None):
+        """indices, squared distances and the flags that the call left"""
+        from hgcalml_amd._lib import check, lib, p, stream
+        on_gpu = [torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+                  for a in (self.x, self.flat, self.rows if rows is None else rows, self.bounds if table is None else table,
+                            self.n_bins, self.width)]
+        x, flat, rows, table, n_bins, width = on_gpu
+        n, dims = x.shape
+        idx = torch.empty((n, K), dtype=torch.int32, device=DEV)
+        dist = torch.empty((n, K), dtype=torch.float32, device=DEV)
+        flags = _status_after(lambda: check(lib.hgc_binned_select_knn_fused(
+            p(x), p(flat), None, p(rows), p(table), p(n_bins), p(width), None, None, radius or -1.0, p(idx), p(dist), n, K, dims,
+            dims, len(table), 0, 0, stream())))
+        return idx.cpu(), dist.cpu(), flags
+
+
+def wrong_rows(binned, kind):
+    """every seventh row names a bin outside the grid, or one of the grid that is not the point's own"""
+    rows = binned.rows.copy()
+    some = np.arange(0, len(rows), 7)
+    rng = np.random.default_rng(1)
+    if kind == "above":
+        rows[some, -1] = binned.n_bins[-1] + rng.integers(0, 40, len(some))
+    elif kind == "far above":
+        rows[some, -1] = 1 << 20
+    elif kind == "event":  # the entry that names the event is not looked at
+        rows[some, 0] = rng.integers(-2, 3, len(some))
+    elif kind == "below":
+        rows[some, 1] = -1 - rng.integers(0, 40, len(some))
+    else:
+        rows[some, 1:] = rng.integers(0, binned.n_bins, (len(some), len(binned.n_bins)))
+    return rows
+
+
+@pytest.mark.parametrize("dims", [2, 3, 4])
+@pytest.mark.parametrize("kind", ["above", "far above", "below", "another", "event"])
+@pytest.mark.parametrize("K,radius", [(6, 0.0), (6, 0.2), (100, 0.0)])
+def test_rows_that_do_not_name_the_own_bin(oracle, dims, kind, K, radius):
+    """such a row says nothing about where its point is: the whole event is searched, of the event that its bin names"""
+    from hgcalml_amd import ops
+    binned = Binned(oracle, dims)
+    want = brute_force(torch.from_numpy(binned.x), SPLITS, K, radius, None)
+    idx, dist, flags = binned.search(K, radius, rows=wrong_rows(binned, kind))
+    assert flags == 0
+    assert torch.equal(idx, want[0]) and torch.equal(dist, want[1])
+    # the table ends with the first event: the second one's points have no neighbours
+    idx, dist, flags = binned.search(K, radius, table=binned.bounds[:binned.cells + 1], rows=wrong_rows(binned, kind))
+    assert flags == ops.FLAG_BIN_BEYOND_TABLE
+    first = SPLITS[1]
+    assert torch.equal(idx[:first], want[0][:first]) and torch.equal(dist[:first], want[1][:first])
+    assert (idx[first:, 1:] == -1).all() and (dist[first:] == 0).all()
+
+
+@pytest.mark.parametrize("dims", [2, 3, 4])
+@pytest.mark.parametrize("K", [6, 140])  # collected, and by shells
+def test_bins_below_every_event_have_no_neighbours(oracle, dims, K):
+    from hgcalml_amd import ops
+    binned = Binned(oracle, dims)
+    want = binned.search(K)
+    bad = torch.arange(len(binned.x)) % 11 == 0
+    binned.flat[bad.numpy()] = -binned.cells - 3
+    idx, dist, flags = binned.search(K)
+    assert want[2] == 0 and flags == ops.FLAG_BIN_BEYOND_TABLE
+    assert torch.equal(idx[~bad], want[0][~bad]) and torch.equal(dist[~bad], want[1][~bad])
+    assert (idx[bad, 1:] == -1).all() and (dist[bad] == 0).all()
