@@ -123,7 +123,8 @@ size_t stable_key_sort_workspace_bytes(long long total, int n_keys, int per_key_
 int stable_key_sort(const int *d_keys, long long total, int n_keys, int per_key_hint, int *d_offsets, int *d_order,
                     void *workspace, size_t workspace_bytes, hipStream_t s);
 
-// hgc_binned_select_knn_fused with a nested grid; bins_bound: no dimension has more bins.
+// hgc_binned_select_knn_fused with a nested grid; bins_bound: no dimension has more bins; callers_table: bin rows and
+// boundary table were handed over by a caller and need not fit together.
 // fine_bits > 0 (= n_bin_dim): d_bin_idx holds the half-bin cells of bin_grouping's spatial mode
 // and d_cell_boundaries is that mode's table (one entry per cell); a query whose bin holds more
 // than fine_min_population points then walks the nested grid of half the bin width instead of
@@ -133,8 +134,8 @@ int binned_select_knn_strided(const float *d_coord, const int *d_bin_idx, const 
                               const int *d_n_bins, const float *d_bin_width, const int *d_sorting,
                               const float *d_shift, float max_radius, int *d_indices, float *d_dist, int n_vert,
                               int n_neigh, int n_coords, int n_bin_dim, int n_bboundaries, int tf_compat,
-                              int use_direction, int bins_bound, const int *d_cell_boundaries, int fine_bits,
-                              int fine_min_population, hipStream_t s);
+                              int use_direction, int bins_bound, bool callers_table,
+                              const int *d_cell_boundaries, int fine_bits, int fine_min_population, hipStream_t s);
 
 // hgc_binned_assign_to_condensates with two more arguments: with d_high set, the *_h
 // arrays are the arrays of all hits themselves (n_vert_h == n_vert, d_indices_to_filtered[i]

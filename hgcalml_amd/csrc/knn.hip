@@ -320,7 +320,8 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
         const int own_cell = uniform(p.bin_idx[q]);   // with fine_bits: bin and half-bin bits
         const int own_bin = own_cell >> p.fine_bits;
         int nb[kDims], qb[kDims];
-        int cells_per_event = 1;
+        int cells_per_event = 1, in_event = 0;
+        int outside = 0;  // negative: the row lies outside the grid
         int reach_max = 0;  // beyond this shell distance no bin is inside the grid
 #pragma unroll
         for (int i = 0; i < kDims; ++i) {
@@ -330,6 +331,8 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
                 nb[i] = uniform(p.n_bins[i]);
                 qb[i] = uniform(p.dim_bin_idx[(size_t)q * (B + 1) + 1 + i]);
                 cells_per_event *= nb[i];
+                in_event = in_event * nb[i] + qb[i];
+                outside |= qb[i] | (nb[i] - 1 - qb[i]);
                 if (FINE) {
                     nb[i] *= 2;
                     qb[i] = 2 * qb[i] + ((own_cell >> (B - 1 - i)) & 1);
@@ -337,10 +340,22 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
                 reach_max = max(reach_max, max(qb[i], nb[i] - 1 - qb[i]));
             }
         }
-        const int event_base = cells_per_event * (own_bin / cells_per_event);
+        const int event_base = own_bin - own_bin % max(cells_per_event, 1);
+        // A row outside the grid, or of another bin than the own one, does not say where the query is: then the whole grid
+        // of the event is walked from the nearest bin inside, and (with bins of no width) nothing is pruned.
+        const bool placed = outside >= 0 && own_bin - event_base == in_event;
+        if (!placed) {
+            reach_max = 0;
+#pragma unroll
+            for (int i = 0; i < kDims; ++i)
+                if (i < B) {
+                    qb[i] = max(min(qb[i], nb[i] - 1), 0);
+                    reach_max = max(reach_max, max(qb[i], nb[i] - 1 - qb[i]));
+                }
+        }
         const int nb_last = nb[B - 1], qb_last = qb[B - 1];
         const int bins_last = FINE ? nb_last >> 1 : nb_last;  // bins (not cells) along the last dimension
-        const float bw = FINE ? 0.5f * p.bin_width[0] : p.bin_width[0];
+        const float bw = !placed ? 0.f : FINE ? 0.5f * p.bin_width[0] : p.bin_width[0];
         const float inv_bw = 1.f / bw;
         const float bins_per_unit = 1.001f * inv_bw;  // generous by 0.1 %, for the pruning bound only
 
@@ -377,15 +392,17 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
         // a row on the nested grid.
         {
             long long grid_rows = FINE ? nb_last / 2 + 2 : 2;
-            bool rows_fit = true;
+            bool rows_fit = true, is_grid = event_base >= 0 && nb_last > 0;  // false: a bin, or numbers of bins, that no grid has
             for (int i = 0; i < B - 1; ++i) {
                 grid_rows = min(grid_rows * nb[i], 1ll << 40);
                 rows_fit = rows_fit && nb[i] < (1 << 13);
+                is_grid = is_grid && nb[i] > 0;
             }
-            if (!rows_fit || grid_rows >= (1ll << 22) || event_base < 0) {  // or a bin that no grid gives
+            // (flat bins are 32 bits)
+            if (!FINE && grid_rows < (1ll << 22)) is_grid = is_grid && 2ll * event_base + grid_rows * nb_last <= 1ll << 32;
+            if (!rows_fit || grid_rows >= (1ll << 22) || !is_grid) {
                 if (FINE) return false;  // the grid of bins may do
-                if (p.status && lane == 0)
-                    atomicOr(p.status, event_base < 0 ? HGC_FLAG_BIN_BEYOND_TABLE : HGC_FLAG_SHELL_TOO_WIDE);
+                if (p.status && lane == 0) atomicOr(p.status, is_grid ? HGC_FLAG_SHELL_TOO_WIDE : HGC_FLAG_BIN_BEYOND_TABLE);
                 return true;  // the list stays empty
             }
         }
@@ -575,12 +592,13 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
                         } else {
                             const int first = event_base + cell * nb_last + lo;
                             const int last = event_base + cell * nb_last + hi + 1;
-                            if (last < p.n_bboundaries) {
+                            // bins beyond the table are skipped, as by the reference, which prints "idx out of range"
+                            const int there = min(last, p.n_bboundaries - 1);
+                            if (first < there) {
                                 seg_start = p.bin_boundaries[first];
-                                seg_len = p.bin_boundaries[last] - seg_start;
-                            } else if (p.status) {  // the reference prints "idx out of range" and skips the bin
-                                atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
+                                seg_len = p.bin_boundaries[there] - seg_start;
                             }
+                            if (p.status && there < last) atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
                         }
                     }
                 }
@@ -818,8 +836,10 @@ constexpr bool collects(int C, int NB, int S, bool window) { return C == NB && N
 __device__ __forceinline__ float bound_of(uint32_t pattern) { return __uint_as_float(max(pattern, 0x00800000u)); }
 
 // The Kn smallest keys of query q, ascending, in `key` (ranks beyond the points there are: the empty key). FINE as in
-// walk_shells. False: nothing is decided (the grid of bins, or walk_shells, has to do it).
-template <int C, int NB, int S, bool MAPPED, bool FINE>
+// walk_shells. False: nothing is decided (the grid of bins, or walk_shells, has to do it). CALLERS: bin rows and boundary table
+// were handed over by a caller, may contradict each other and be of any size; without, they are those of the package's own
+// binning, which need no such checks (1.14 M points in 16 events on 43 bins: 1130 us with them, 1040 without, 1185 by shells).
+template <int C, int NB, int S, bool MAPPED, bool FINE, bool CALLERS>
 __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q, const int lane, uint8_t *const marks,
                                                 uint64_t *const buffer, const int Kn, uint64_t (&key)[S]) {
     static_assert(C > 0 && NB >= 2 && NB <= 4 && S <= 2);
@@ -841,12 +861,11 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
         in_event = in_event * readlane_i32(nb_v, i) + readlane_i32(qb_v, i);
         cells_per_event *= readlane_i32(nb_v, i);
     }
-    int event_base = uniform(p.dim_bin_idx[(size_t)q * (B + 1)]) * cells_per_event;
-    bool placed = own_bin - event_base == in_event && !__builtin_amdgcn_ballot_w64((uint32_t)qb_v >= (uint32_t)nb_v);
-    if (!placed) {
-        // The bin says which event it is (a division, which rows of a binning are spared). A row outside the grid, or of
-        // another bin than the own one, does not say where the query is: then the whole grid of the event is walked
-        // from the nearest bin inside, and nothing is pruned.
+    int event_base = own_bin - in_event;
+    bool placed = true;
+    if constexpr (CALLERS) {
+        // The bin says which event it is. A row outside the grid, or of another bin than the own one, does not say where
+        // the query is: then the whole grid of the event is walked from the nearest bin inside, and nothing is pruned.
         event_base = own_bin - own_bin % max(cells_per_event, 1);
         placed = own_bin - event_base == in_event && !__builtin_amdgcn_ballot_w64((uint32_t)qb_v >= (uint32_t)nb_v);
         if (!placed) qb_v = max(min(qb_v, nb_v - 1), 0);
@@ -865,23 +884,42 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
         qb[i] = readlane_i32(qb_v, i);
         if (i < B - 1) {
             grid_rows *= nb[i];
-            rows_fit = rows_fit && nb[i] < (1 << 13);
+            rows_fit = rows_fit && nb[i] < (1 << 13) && (!CALLERS || nb[i] > 0);
         }
     }
     const int nb_last = nb[B - 1], qb_last = qb[B - 1];
     const int bins_last = FINE ? nb_last >> 1 : nb_last;
     grid_rows *= FINE ? bins_last + 1 : 2;  // slots of a pass
-    if (!rows_fit || grid_rows >= (1ll << 22) || event_base < 0) {  // see divmod_small; a bin that no grid gives
+    bool no_grid = event_base < 0;  // a bin, or numbers of bins, that no grid has
+    if (CALLERS && grid_rows < (1ll << 22))  // (grid_rows is twice the rows here; flat bins are 32 bits)
+        no_grid = no_grid || grid_rows <= 0 || nb_last < 1 || event_base >= p.n_bboundaries - 1 || 2ll * event_base + grid_rows * nb_last > 1ll << 32;
+    if (!rows_fit || grid_rows >= (1ll << 22) || no_grid) {  // see divmod_small
         if (FINE) return false;  // the grid of bins may do
-        if (p.status && lane == 0) atomicOr(p.status, event_base < 0 ? HGC_FLAG_BIN_BEYOND_TABLE : HGC_FLAG_SHELL_TOO_WIDE);
+        if (p.status && lane == 0) atomicOr(p.status, no_grid ? HGC_FLAG_BIN_BEYOND_TABLE : HGC_FLAG_SHELL_TOO_WIDE);
         return true;  // the list stays empty
     }
-    const float bw = FINE ? 0.5f * p.bin_width[0] : p.bin_width[0];
+    const float bw = !placed ? 0.f : FINE ? 0.5f * p.bin_width[0] : p.bin_width[0];
     // Coordinates without bounds leave widths without a meaning: then nothing is pruned, the whole grid is walked.
-    const bool prunes = placed && bw > 1e-30f && bw < 1e18f;  // (the square stays finite)
+    const bool prunes = bw > 1e-30f && bw < 1e18f;  // (the square stays finite)
     const float inv_bw = __builtin_amdgcn_rcpf(bw);  // within an ulp; used with margins of a thousandth of a bin
     const float bins_per_unit = prunes ? 1.001f * inv_bw : 3.0e38f;
     const float gap_scale = prunes ? 0.999f * (bw * bw) : 0.f;  // bounds are generous by 0.1 %
+
+    // number of the first bin of a row of the grid, from the number of the row
+    auto row_base = [&](int row) {
+        return event_base + (CALLERS ? row * bins_last : (int)__umul24(row, bins_last));
+    };
+    // a caller's table: the points of bins first .. last - 1 of a row, without the bins beyond the table, which are skipped
+    // as by the reference, which prints "idx out of range"
+    int seg_start = 0, seg_len = 0;
+    [[maybe_unused]] auto callers_run = [&](int first, int last) {
+        const int there = min(last, p.n_bboundaries - 1);
+        if (first < there) {
+            seg_start = p.bin_boundaries[first];
+            seg_len = p.bin_boundaries[there] - seg_start;
+        }
+        if (p.status && there < last) atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
+    };
 
     // lower bounds of the distance to the edges of the own bin, in bin widths, as in walk_shells
     float tl_v = 0.f, tu_v = 0.f;
@@ -913,7 +951,6 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
     int d_out, d_radius = 1 << 30;  // the cube of half-width d_radius holds everything within the radius
     if (has_radius && prunes)
         d_radius = max(1, uniform((int)fminf(__builtin_ceilf(__builtin_amdgcn_sqrtf(bound_of(__float_as_uint(p.radius_sq))) * bins_per_unit), 1.0e9f)));
-    int seg_start = 0, seg_len = 0;
     {
         int off[B], ring = 0;
         bool in_grid = true;
@@ -968,29 +1005,29 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
             const int bin_last = ((qb_last - 1) >> 1) + (lane & 1);
             const int lo = max(max(qb_last - min(d_out, lo_most), 0), 2 * bin_last);
             const int hi = min(min(qb_last + min(d_out, hi_most), nb_last - 1), 2 * bin_last + 1);
-            const int bin = event_base + (int)__umul24(cell, bins_last) + bin_last;
-            if (in_grid && ring <= d_out && lo <= hi) {
-                if (bin + 1 < p.n_bboundaries) {
-                    const int base = ((bin << (B - 1)) | halves) << 1;
-                    seg_start = table_entry(p.cell_boundaries, base | (lo & 1));
-                    seg_len = table_entry(p.cell_boundaries, (base | (hi & 1)) + 1) - seg_start;
-                } else if (p.status) {
-                    atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
-                }
+            const int bin = row_base(cell) + bin_last;
+            if (in_grid && ring <= d_out && lo <= hi && bin + 1 < p.n_bboundaries) {
+                const int base = ((bin << (B - 1)) | halves) << 1;
+                seg_start = table_entry(p.cell_boundaries, base | (lo & 1));
+                seg_len = table_entry(p.cell_boundaries, (base | (hi & 1)) + 1) - seg_start;
             }
+            if (p.status && in_grid && ring <= d_out && lo <= hi && bin + 1 >= p.n_bboundaries) atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
         } else {
             constexpr int kCubes = B == 4 ? 1 : 3;
-            const int row = event_base + (int)__umul24(cell, nb_last);
+            // lanes without a row look at the own one
+            const int row = in_grid ? row_base(cell) : own_bin - qb_last;
             auto look = [&](int d) {  // the part of the row inside the cube of half-width d
                 const int from = max(qb_last - min(d, lo_most), 0), to = min(qb_last + min(d, hi_most), nb_last - 1) + 1;
                 seg_start = seg_len = 0;
-                if (in_grid && ring <= d && from < to) {
-                    if (row < p.n_bboundaries - to) {
+                if constexpr (CALLERS) {
+                    if (in_grid && ring <= d && from < to) callers_run(row + from, row + to);
+                } else {
+                    const bool wanted = in_grid && ring <= d && row < p.n_bboundaries - to;
+                    if (wanted) {
                         seg_start = table_entry(p.bin_boundaries, row + from);
                         seg_len = table_entry(p.bin_boundaries, row + to) - seg_start;
-                    } else if (p.status) {  // the reference prints "idx out of range" and skips the bin
-                        atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
                     }
+                    if (p.status && in_grid && ring <= d && !wanted) atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
                 }
                 return readlane_i32(wave_inclusive_sum(seg_len), kWave - 1);
             };
@@ -1124,7 +1161,7 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
                 }
                 if (rest >= 0.f && lo <= hi) {
                     if (FINE) {
-                        const int bin = event_base + (int)__umul24(cell, bins_last) + ((qb_last + lo) >> 1);
+                        const int bin = row_base(cell) + ((qb_last + lo) >> 1);
                         if (bin + 1 < p.n_bboundaries) {
                             const int base = ((bin << (B - 1)) | halves) << 1;
                             seg_start = table_entry(p.cell_boundaries, base | ((qb_last + lo) & 1));
@@ -1133,9 +1170,11 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
                             atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
                         }
                     } else {
-                        const int first = event_base + (int)__umul24(cell, nb_last) + qb_last + lo;
+                        const int first = row_base(cell) + qb_last + lo;
                         const int last = first + (hi - lo) + 1;
-                        if (last < p.n_bboundaries) {
+                        if constexpr (CALLERS) {
+                            callers_run(first, last);
+                        } else if (last < p.n_bboundaries) {
                             seg_start = table_entry(p.bin_boundaries, first);
                             seg_len = table_entry(p.bin_boundaries, last) - seg_start;
                         } else if (p.status) {
@@ -1221,7 +1260,7 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
 // NESTED: the search runs over a nested grid (see KnnParams::fine_bits): a query whose bin holds more
 // than fine_min_population points walks the nested grid (and the grid of bins after all when that
 // walk gives up), the others the grid of bins.
-template <int C, int NB, int S, bool MAPPED, bool WINDOW, bool NESTED>
+template <int C, int NB, int S, bool MAPPED, bool WINDOW, bool NESTED, bool CALLERS>
 __device__ __forceinline__ void search_query(const KnnParams &p, const int q, const int lane, uint8_t *const marks,
                                              uint64_t *const buffer) {
     constexpr bool kCollects = collects(C, NB, S, WINDOW);
@@ -1260,10 +1299,10 @@ __device__ __forceinline__ void search_query(const KnnParams &p, const int q, co
     if (searching) {
         if constexpr (kCollects) {
             if constexpr (NESTED) {
-                if (!crowded || !collect_nearest<C, NB, S, MAPPED, true>(p, q, lane, marks, buffer, Kn, key))
-                    collect_nearest<C, NB, S, MAPPED, false>(p, q, lane, marks, buffer, Kn, key);
+                if (!crowded || !collect_nearest<C, NB, S, MAPPED, true, CALLERS>(p, q, lane, marks, buffer, Kn, key))
+                    collect_nearest<C, NB, S, MAPPED, false, CALLERS>(p, q, lane, marks, buffer, Kn, key);
             } else {
-                collect_nearest<C, NB, S, MAPPED, false>(p, q, lane, marks, buffer, Kn, key);
+                collect_nearest<C, NB, S, MAPPED, false, CALLERS>(p, q, lane, marks, buffer, Kn, key);
             }
         } else {
             bool found = false;
@@ -1294,7 +1333,7 @@ __device__ __forceinline__ void search_query(const KnnParams &p, const int q, co
     }
 }
 
-template <int C, int NB, int S, bool MAPPED, bool WINDOW = false, bool NESTED = false>
+template <int C, int NB, int S, bool MAPPED, bool WINDOW = false, bool NESTED = false, bool CALLERS = false>
 __global__ __launch_bounds__(kWave)
 __attribute__((amdgpu_waves_per_eu(S <= 2 ? 8 : 1, 8)))
 void knn_wave_kernel(const KnnParams p) {
@@ -1303,11 +1342,11 @@ void knn_wave_kernel(const KnnParams p) {
     // queries come in bin order and differ a lot in cost from region to region:
     // chunks of 512 of them are dealt to the XCDs in turn
     const int q = xcd_chunked_block<512>(blockIdx.x, gridDim.x);
-    search_query<C, NB, S, MAPPED, WINDOW, NESTED>(p, q, lane_id(), marks, buffer);
+    search_query<C, NB, S, MAPPED, WINDOW, NESTED, CALLERS>(p, q, lane_id(), marks, buffer);
 }
 
 template <int C, int NB, bool MAPPED>
-int launch_levels(const KnnParams &p, hipStream_t s) {
+int launch_levels(const KnnParams &p, bool callers_table, hipStream_t s) {
     const int levels = std::max(1, ceil_div(p.K - 1, kWave));
     const dim3 grid(p.n_vert), block(kWave);
     if (levels > kBulkInsertMaxRuns) {  // more neighbours than the registers hold: one launch per window of ranks
@@ -1331,6 +1370,13 @@ int launch_levels(const KnnParams &p, hipStream_t s) {
             return check_launch("knn_wave_kernel (nested grid)");
         }
     }
+    if constexpr (collects(C, NB, 1, false)) {
+        if (callers_table && levels <= 2) {
+            if (levels == 1) knn_wave_kernel<C, NB, 1, MAPPED, false, false, true><<<grid, block, 0, s>>>(p);
+            else knn_wave_kernel<C, NB, 2, MAPPED, false, false, true><<<grid, block, 0, s>>>(p);
+            return check_launch("knn_wave_kernel (a caller's table)");
+        }
+    }
     switch (levels) {
         case 1: knn_wave_kernel<C, NB, 1, MAPPED><<<grid, block, 0, s>>>(p); break;
         case 2: knn_wave_kernel<C, NB, 2, MAPPED><<<grid, block, 0, s>>>(p); break;
@@ -1345,22 +1391,21 @@ int launch_levels(const KnnParams &p, hipStream_t s) {
 // wrapper's default, or min(4, coordinates), the pipeline's own grid) get kernels with both
 // numbers fixed at compile time, anything else the one that reads them.
 template <bool MAPPED>
-int launch_coords(const KnnParams &p, int bins_bound, hipStream_t s) {
-    // collect_nearest: 32-bit offsets into the table, 24-bit factors of bin numbers
-    if (p.n_bboundaries >= 1 << 30 || bins_bound >= 1 << 24) return launch_levels<0, 0, MAPPED>(p, s);
-    if (p.n_coords == 2 && p.n_bin_dim == 2) return launch_levels<2, 2, MAPPED>(p, s);
-    if (p.n_coords == 3 && p.n_bin_dim == 3) return launch_levels<3, 3, MAPPED>(p, s);
-    if (p.n_coords == 4 && p.n_bin_dim == 3) return launch_levels<4, 3, MAPPED>(p, s);
-    if (p.n_coords == 4 && p.n_bin_dim == 4) return launch_levels<4, 4, MAPPED>(p, s);
-    if (p.n_coords == 5 && p.n_bin_dim == 4) return launch_levels<5, 4, MAPPED>(p, s);
-    if (p.n_coords == 6 && p.n_bin_dim == 4) return launch_levels<6, 4, MAPPED>(p, s);
-    if (p.n_coords == 7 && p.n_bin_dim == 4) return launch_levels<7, 4, MAPPED>(p, s);
-    if (p.n_coords == 8 && p.n_bin_dim == 4) return launch_levels<8, 4, MAPPED>(p, s);
-    if (p.n_coords == 5 && p.n_bin_dim == 3) return launch_levels<5, 3, MAPPED>(p, s);
-    if (p.n_coords == 6 && p.n_bin_dim == 3) return launch_levels<6, 3, MAPPED>(p, s);
-    if (p.n_coords == 7 && p.n_bin_dim == 3) return launch_levels<7, 3, MAPPED>(p, s);
-    if (p.n_coords == 8 && p.n_bin_dim == 3) return launch_levels<8, 3, MAPPED>(p, s);
-    return launch_levels<0, 0, MAPPED>(p, s);
+int launch_coords(const KnnParams &p, bool callers_table, int bins_bound, hipStream_t s) {
+    if (p.n_bboundaries >= 1 << 30 || bins_bound >= 1 << 24) return launch_levels<0, 0, MAPPED>(p, callers_table, s);
+    if (p.n_coords == 2 && p.n_bin_dim == 2) return launch_levels<2, 2, MAPPED>(p, callers_table, s);
+    if (p.n_coords == 3 && p.n_bin_dim == 3) return launch_levels<3, 3, MAPPED>(p, callers_table, s);
+    if (p.n_coords == 4 && p.n_bin_dim == 3) return launch_levels<4, 3, MAPPED>(p, callers_table, s);
+    if (p.n_coords == 4 && p.n_bin_dim == 4) return launch_levels<4, 4, MAPPED>(p, callers_table, s);
+    if (p.n_coords == 5 && p.n_bin_dim == 4) return launch_levels<5, 4, MAPPED>(p, callers_table, s);
+    if (p.n_coords == 6 && p.n_bin_dim == 4) return launch_levels<6, 4, MAPPED>(p, callers_table, s);
+    if (p.n_coords == 7 && p.n_bin_dim == 4) return launch_levels<7, 4, MAPPED>(p, callers_table, s);
+    if (p.n_coords == 8 && p.n_bin_dim == 4) return launch_levels<8, 4, MAPPED>(p, callers_table, s);
+    if (p.n_coords == 5 && p.n_bin_dim == 3) return launch_levels<5, 3, MAPPED>(p, callers_table, s);
+    if (p.n_coords == 6 && p.n_bin_dim == 3) return launch_levels<6, 3, MAPPED>(p, callers_table, s);
+    if (p.n_coords == 7 && p.n_bin_dim == 3) return launch_levels<7, 3, MAPPED>(p, callers_table, s);
+    if (p.n_coords == 8 && p.n_bin_dim == 3) return launch_levels<8, 3, MAPPED>(p, callers_table, s);
+    return launch_levels<0, 0, MAPPED>(p, callers_table, s);
 }
 
 }  // namespace
@@ -1370,8 +1415,8 @@ int binned_select_knn_strided(const float *d_coord, const int *d_bin_idx, const 
                               const int *d_n_bins, const float *d_bin_width, const int *d_sorting,
                               const float *d_shift, float max_radius, int *d_indices, float *d_dist, int n_vert,
                               int n_neigh, int n_coords, int n_bin_dim, int n_bboundaries, int tf_compat,
-                              int use_direction, int bins_bound, const int *d_cell_boundaries, int fine_bits,
-                              int fine_min_population, hipStream_t s) {
+                              int use_direction, int bins_bound, bool callers_table,
+                              const int *d_cell_boundaries, int fine_bits, int fine_min_population, hipStream_t s) {
     // same conditions as the reference op (binned_select_knn_kernel.cc:336-352)
     HGC_REQUIRE(n_bin_dim > 1, "BinnedSelectKnnOp expects at least 2 binning dimensions.");
     HGC_REQUIRE(n_bin_dim < 6, "BinnedSelectKnnOp expects maximum 5 binning dimensions.");
@@ -1421,7 +1466,8 @@ int binned_select_knn_strided(const float *d_coord, const int *d_bin_idx, const 
     p.cell_boundaries = d_cell_boundaries;
     p.fine_bits = fine_bits;
     p.fine_min_population = fine_min_population;
-    return d_sorting ? launch_coords<true>(p, bins_bound, s) : launch_coords<false>(p, bins_bound, s);
+    // the package's own tables are read with 32-bit byte offsets, their bins per dimension are factors of 24 bits
+    return d_sorting ? launch_coords<true>(p, callers_table, bins_bound, s) : launch_coords<false>(p, callers_table, bins_bound, s);
 }
 
 }  // namespace hgc
@@ -1438,8 +1484,8 @@ int hgc_binned_select_knn_fused(const float *d_coord, const int *d_bin_idx, cons
                                 int use_direction, hgc_stream_t stream) {
     return binned_select_knn_strided(d_coord, d_bin_idx, d_direction, d_dim_bin_idx, d_bin_boundaries, d_n_bins,
                                      d_bin_width, d_sorting, d_shift, max_radius, d_indices, d_dist, n_vert, n_neigh,
-                                     n_coords, n_bin_dim, n_bboundaries, tf_compat, use_direction, n_bboundaries, nullptr, 0, 0,
-                                     as_stream(stream));
+                                     n_coords, n_bin_dim, n_bboundaries, tf_compat, use_direction, n_bboundaries, true,
+                                     nullptr, 0, 0, as_stream(stream));
 }
 
 int hgc_binned_select_knn(const float *d_coord, const int *d_bin_idx, const int *d_direction,

@@ -529,7 +529,7 @@ int hgc_binned_select_knn_pipeline(const float *d_coords, const int *d_row_split
     if (rc) return rc;
     return binned_select_knn_strided(scoords, sflat, sdir, sbinass, bin_starts, n_bins, bin_width,
                                      sorting, shift, max_radius, d_indices, d_dist, n_vert, n_neigh, n_coords,
-                                     n_bin_dims, L.total_bins_bound + 1, tf_compat, use_direction, n_bins_scalar + 1,
+                                     n_bin_dims, L.total_bins_bound + 1, tf_compat, use_direction, n_bins_scalar + 1, false,
                                      L.nested ? bounds : nullptr, L.nested ? n_bin_dims : 0, std::max(n_neigh - 1, 1) / kCrowdedBinFraction,
                                      as_stream(stream));
 }

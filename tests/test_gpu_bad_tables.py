@@ -58,9 +58,9 @@ def wrong_rows(binned, kind):
     return rows
 
 
-@pytest.mark.parametrize("dims", [2, 3, 4])
+@pytest.mark.parametrize("dims", [2, 3, 4, 5])
 @pytest.mark.parametrize("kind", ["above", "far above", "below", "another", "event"])
-@pytest.mark.parametrize("K,radius", [(6, 0.0), (6, 0.2), (100, 0.0)])
+@pytest.mark.parametrize("K,radius", [(6, 0.0), (6, 0.2), (100, 0.0), (140, 0.0), (140, 0.2)])
 def test_rows_that_do_not_name_the_own_bin(oracle, dims, kind, K, radius):
     """such a row says nothing about where its point is: the whole event is searched, of the event that its bin names"""
     from hgcalml_amd import ops
@@ -89,3 +89,35 @@ def test_bins_below_every_event_have_no_neighbours(oracle, dims, K):
     assert want[2] == 0 and flags == ops.FLAG_BIN_BEYOND_TABLE
     assert torch.equal(idx[~bad], want[0][~bad]) and torch.equal(dist[~bad], want[1][~bad])
     assert (idx[bad, 1:] == -1).all() and (dist[bad] == 0).all()
+
+
+@pytest.mark.parametrize("dims", [2, 3, 4])
+@pytest.mark.parametrize("K,radius", [(6, 0.0), (6, 0.2), (140, 0.0)])  # collected, and by shells
+@pytest.mark.parametrize("share", [0.1, 0.5, 0.93])
+def test_table_that_ends_inside_an_event(oracle, dims, K, radius, share):
+    """bins beyond the table hold nothing, the bins in front of its end keep their points (the rows of a point whose own
+    bin is beyond the table are left open)"""
+    from hgcalml_amd import ops
+    binned = Binned(oracle, dims)
+    n_bins_left = binned.cells + int(share * binned.cells)
+    x = torch.from_numpy(binned.x)
+    left = int(binned.bounds[n_bins_left])  # points in bin order
+    want = brute_force(x[:left], [0, SPLITS[1], left], K, radius, None)
+    idx, dist, flags = binned.search(K, radius, table=binned.bounds[:n_bins_left + 1])
+    assert flags == ops.FLAG_BIN_BEYOND_TABLE
+    assert torch.equal(idx[:left], want[0]) and torch.equal(dist[:left], want[1])
+    assert (idx[left:] < left).logical_or(idx[left:] == torch.arange(left, len(idx))[:, None]).all()
+
+
+@pytest.mark.parametrize("dims", [2, 3, 4])
+@pytest.mark.parametrize("K", [6, 140])
+@pytest.mark.parametrize("at,value", [(0, 0), (-1, 0), (0, -7), (-1, -7), (-1, 1 << 30)])
+def test_numbers_of_bins_that_no_grid_has(oracle, dims, K, at, value):
+    """the call ends, reports it and reads nothing beyond the table"""
+    from hgcalml_amd import ops
+    binned = Binned(oracle, dims)
+    binned.n_bins = binned.n_bins.copy()
+    binned.n_bins[at] = value
+    idx, dist, flags = binned.search(K)
+    assert flags == ops.FLAG_BIN_BEYOND_TABLE
+    assert (idx[:, 0] == torch.arange(len(idx))).all() and (idx[:, 1:] < len(idx)).all()
