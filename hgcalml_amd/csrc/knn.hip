@@ -1391,8 +1391,7 @@ int launch_levels(const KnnParams &p, bool callers_table, hipStream_t s) {
 // wrapper's default, or min(4, coordinates), the pipeline's own grid) get kernels with both
 // numbers fixed at compile time, anything else the one that reads them.
 template <bool MAPPED>
-int launch_coords(const KnnParams &p, bool callers_table, int bins_bound, hipStream_t s) {
-    if (p.n_bboundaries >= 1 << 30 || bins_bound >= 1 << 24) return launch_levels<0, 0, MAPPED>(p, callers_table, s);
+int launch_coords(const KnnParams &p, bool callers_table, hipStream_t s) {
     if (p.n_coords == 2 && p.n_bin_dim == 2) return launch_levels<2, 2, MAPPED>(p, callers_table, s);
     if (p.n_coords == 3 && p.n_bin_dim == 3) return launch_levels<3, 3, MAPPED>(p, callers_table, s);
     if (p.n_coords == 4 && p.n_bin_dim == 3) return launch_levels<4, 3, MAPPED>(p, callers_table, s);
@@ -1467,7 +1466,8 @@ int binned_select_knn_strided(const float *d_coord, const int *d_bin_idx, const 
     p.fine_bits = fine_bits;
     p.fine_min_population = fine_min_population;
     // the package's own tables are read with 32-bit byte offsets, their bins per dimension are factors of 24 bits
-    return d_sorting ? launch_coords<true>(p, callers_table, bins_bound, s) : launch_coords<false>(p, callers_table, bins_bound, s);
+    callers_table = callers_table || n_bboundaries >= 1 << 30 || bins_bound >= 1 << 24;
+    return d_sorting ? launch_coords<true>(p, callers_table, s) : launch_coords<false>(p, callers_table, s);
 }
 
 }  // namespace hgc
@@ -1484,7 +1484,7 @@ int hgc_binned_select_knn_fused(const float *d_coord, const int *d_bin_idx, cons
                                 int use_direction, hgc_stream_t stream) {
     return binned_select_knn_strided(d_coord, d_bin_idx, d_direction, d_dim_bin_idx, d_bin_boundaries, d_n_bins,
                                      d_bin_width, d_sorting, d_shift, max_radius, d_indices, d_dist, n_vert, n_neigh,
-                                     n_coords, n_bin_dim, n_bboundaries, tf_compat, use_direction, n_bboundaries, true,
+                                     n_coords, n_bin_dim, n_bboundaries, tf_compat, use_direction, 0, true,
                                      nullptr, 0, 0, as_stream(stream));
 }
 

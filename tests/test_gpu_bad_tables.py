@@ -121,3 +121,35 @@ def test_numbers_of_bins_that_no_grid_has(oracle, dims, K, at, value):
     idx, dist, flags = binned.search(K)
     assert flags == ops.FLAG_BIN_BEYOND_TABLE
     assert (idx[:, 0] == torch.arange(len(idx))).all() and (idx[:, 1:] < len(idx)).all()
+
+
+@pytest.mark.parametrize("dims,n_bins,events", [(3, 102, 16), (2, 2100, 4), (4, 64, 2)])
+@pytest.mark.parametrize("K", [9, 140])
+def test_tables_of_2_to_the_24_bins_and_more(dims, n_bins, events, K):
+    """bins per dimension are few, the bins of all events many: the same answers"""
+    from hgcalml_amd import ops
+    from hgcalml_amd._lib import check, lib, p, stream
+    gen = torch.Generator().manual_seed(dims)
+    n = 150 * events + 7
+    x = torch.rand(n, dims, generator=gen)
+    splits = [150 * e for e in range(events)] + [n]
+    bins = torch.tensor([n_bins] * dims, dtype=torch.int32, device=DEV)
+    width = torch.tensor([1.0 / n_bins], device=DEV)
+    total = events * n_bins ** dims
+    assert total >= 1 << 24
+    on_gpu = x.to(DEV)
+    rows, flat, count = torch.ops.hgcalml.bin_by_coordinates(on_gpu, torch.tensor(splits, dtype=torch.int32, device=DEV), width,
+                                                             bins, total, True)
+    order = torch.argsort(flat.long() * n + torch.arange(n, device=DEV))
+    table = torch.zeros(total + 1, dtype=torch.int32, device=DEV)
+    table[1:] = torch.cumsum(count, 0, dtype=torch.int32)
+    idx = torch.empty((n, K), dtype=torch.int32, device=DEV)
+    dist = torch.empty((n, K), dtype=torch.float32, device=DEV)
+    a = [on_gpu[order].contiguous(), flat[order].contiguous(), rows[order].contiguous()]
+    sorting = order.to(torch.int32)
+    flags = _status_after(lambda: check(lib.hgc_binned_select_knn_fused(
+        p(a[0]), p(a[1]), None, p(a[2]), p(table), p(bins), p(width), p(sorting), None, -1.0, p(idx), p(dist), n, K, dims, dims,
+        len(table), 0, 0, stream())))
+    want = brute_force(x, splits, K, 0.0, None)
+    assert flags in (0, ops.FLAG_COORDINATE_OUT_OF_GRID)
+    assert torch.equal(idx.cpu(), want[0]) and torch.equal(dist.cpu(), want[1])
