@@ -729,7 +729,8 @@ constexpr int kFineMaxCube = 3;  // on the nested grid a query gives up beyond t
 
 // keys 0 .. n of `buffer` cut down to between Kn and `most` of the smallest (Kn <= most <= n): returns how many are
 // left; the key (cut, cut_id) becomes one that the Kn-th smallest does not exceed. Distances first, and where more
-// than `most` keys share the Kn-th distance the indices decide.
+// than `most` keys share the Kn-th distance the indices decide. REPEATED: a key may be there several times.
+template <bool REPEATED>
 __device__ __forceinline__ int cut_to_smallest(uint64_t *const buffer, const int lane, const int n, const int Kn,
                                                const int most, uint32_t &cut, uint32_t &cut_id) {
     constexpr int kRegs = kBufferKeys / kWave;
@@ -804,7 +805,26 @@ __device__ __forceinline__ int cut_to_smallest(uint64_t *const buffer, const int
                 }
             }
             // one too many with the limit 1: points 0 and 1 share the Kn-th distance, and point 0 completes the list
-            if (left > most) tie_limit = 0;
+            if (!REPEATED && left > most) tie_limit = 0;
+            if (REPEATED && left > most) {  // that, or a key many times over, of which as many stay as fit
+                auto count_up_to = [&](uint64_t limit) {
+                    int c = 0;
+#pragma unroll
+                    for (int u = 0; u < kRegs; ++u) c += (int)__popcll(__builtin_amdgcn_ballot_w64(k[u] <= limit));
+                    return c;
+                };
+                const uint64_t first_id = (uint64_t)hi << 32;
+                if (tie_limit == 1 && count_up_to(first_id) >= Kn) tie_limit = 0;
+                const uint64_t limit = first_id | tie_limit;
+                int spare = most - (limit > 0 ? count_up_to(limit - 1) : 0);
+#pragma unroll
+                for (int u = 0; u < kRegs; ++u) {
+                    const uint64_t same = __builtin_amdgcn_ballot_w64(k[u] == limit);
+                    const int before = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0));
+                    if (k[u] == limit && before >= spare) k[u] = kEmptyKey;
+                    spare = max(0, spare - (int)__popcll(same));
+                }
+            }
         }
         const uint64_t limit = (uint64_t)hi << 32 | tie_limit;
         int at = 0;
@@ -842,7 +862,7 @@ __device__ __forceinline__ float bound_of(uint32_t pattern) { return __uint_as_f
 
 // The Kn smallest keys of query q, ascending, in `key` (ranks beyond the points there are: the empty key). FINE as in
 // walk_shells. False: nothing is decided (the grid of bins, or walk_shells, has to do it). CALLERS: bin rows and boundary table
-// were handed over by a caller, may contradict each other and be of any size; without, they are those of the package's own
+// were handed over by a caller, may contradict each other and be of any size, and `sorting` may repeat itself; without, they are those of the package's own
 // binning, which need no such checks (1.14 M points in 16 events on 43 bins: 1130 us with them, 1040 without, 1185 by shells).
 template <int C, int NB, int S, bool MAPPED, bool FINE, bool CALLERS>
 __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q, const int lane, uint8_t *const marks,
@@ -1232,7 +1252,7 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
                             enters &= __builtin_amdgcn_ballot_w64(ck <= ((uint64_t)cut << 32 | cut_id));
                             if (n_kept + (int)__popcll(enters) > kBufferKeys) {
                                 wave_lds_fence();
-                                n_kept = cut_to_smallest(buffer, lane, n_kept, Kn, kept, cut, cut_id);
+                                n_kept = cut_to_smallest<CALLERS>(buffer, lane, n_kept, Kn, kept, cut, cut_id);
                                 enters &= __builtin_amdgcn_ballot_w64(ck <= ((uint64_t)cut << 32 | cut_id));
                                 room = cut_id == 0xffffffffu ? kBufferKeys : 0;
                             }
@@ -1250,13 +1270,13 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
         d_in = d_out;
         if (n_kept >= Kn) {
             wave_lds_fence();
-            n_kept = cut_to_smallest(buffer, lane, n_kept, Kn, kept, cut, cut_id);
+            n_kept = cut_to_smallest<CALLERS>(buffer, lane, n_kept, Kn, kept, cut, cut_id);
         }
         d_out = d_out < 4 ? d_out + 1 : d_out + (d_out >> 1);
     }
 
     wave_lds_fence();
-    if (n_kept > S * kWave) n_kept = cut_to_smallest(buffer, lane, n_kept, Kn, S * kWave, cut, cut_id);
+    if (n_kept > S * kWave) n_kept = cut_to_smallest<CALLERS>(buffer, lane, n_kept, Kn, S * kWave, cut, cut_id);
     key[0] = wave_sort_u64(lane < n_kept ? buffer[lane] : kEmptyKey);
     if constexpr (S == 2) {
         key[1] = kEmptyKey;

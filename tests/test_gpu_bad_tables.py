@@ -153,3 +153,38 @@ def test_tables_of_2_to_the_24_bins_and_more(dims, n_bins, events, K):
     want = brute_force(x, splits, K, 0.0, None)
     assert flags in (0, ops.FLAG_COORDINATE_OUT_OF_GRID)
     assert torch.equal(idx.cpu(), want[0]) and torch.equal(dist.cpu(), want[1])
+
+
+@pytest.mark.parametrize("dims", [2, 3, 4])
+@pytest.mark.parametrize("K", [5, 17, 65, 129, 140])
+@pytest.mark.parametrize("again", [0, 1, 5, 650])
+def test_a_sorting_that_names_one_point_many_times(oracle, dims, K, again):
+    """300 points in one place are all called `again`: equal keys, more than the buffer of the collected search holds"""
+    from hgcalml_amd._lib import check, lib, p, stream
+    rng = np.random.default_rng(dims)
+    n = 1000
+    x = rng.random((n, dims)).astype(np.float32)
+    x[200:800] = 0.5
+    names = rng.permutation(n).astype(np.int32)
+    names[450:750] = again  # all of them in that place
+    rows, flat, n_bins, width, count = oracle.BinByCoordinates(x, np.array([0, n], np.int32), n_bins=4)
+    order = np.argsort(flat, kind="stable")
+    x, rows, flat, names = x[order], rows[order], flat[order], names[order]
+    bounds = np.concatenate([[0], np.cumsum(count)]).astype(np.int32)
+    on_gpu = [torch.from_numpy(np.ascontiguousarray(a)).to(DEV) for a in (x, flat, rows, bounds, n_bins, width, names)]
+    gx, gflat, grows, gbounds, gbins, gwidth, gnames = on_gpu
+    idx = torch.zeros((n, K), dtype=torch.int32, device=DEV)
+    dist = torch.zeros((n, K), dtype=torch.float32, device=DEV)
+    check(lib.hgc_binned_select_knn_fused(p(gx), p(gflat), None, p(grows), p(gbounds), p(gbins), p(gwidth), p(gnames), None, -1.0,
+                                          p(idx), p(dist), n, K, dims, dims, len(bounds), 0, 0, stream()))
+    idx, dist = idx.cpu().numpy(), dist.cpu().numpy()
+    d = np.zeros((n, n), np.float32)
+    for c in range(dims):
+        step = x[:, None, c] - x[None, :, c]
+        d = d + step * step
+    key = (d.view(np.uint32).astype(np.uint64) << np.uint64(32)) | names.astype(np.uint64)[None, :]
+    np.fill_diagonal(key, np.iinfo(np.uint64).max)
+    key = np.sort(key, axis=1)[:, :K - 1]
+    once = np.flatnonzero(np.bincount(names, minlength=n)[names] == 1)  # the rows that one point writes
+    assert (idx[names[once], 1:] == (key[once] & np.uint64(0xffffffff)).astype(np.int32)).all()
+    assert (dist[names[once], 1:].view(np.uint32) == (key[once] >> np.uint64(32)).astype(np.uint32)).all()
