@@ -395,7 +395,7 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
             bool rows_fit = true, is_grid = event_base >= 0 && nb_last > 0;  // false: a bin, or numbers of bins, that no grid has
             for (int i = 0; i < B - 1; ++i) {
                 grid_rows = min(grid_rows * nb[i], 1ll << 40);
-                rows_fit = rows_fit && nb[i] < (1 << 13);
+                rows_fit = rows_fit && (i == 0 || nb[i] < (1 << 13));  // the leading digit is what the divisions leave
                 is_grid = is_grid && nb[i] > 0;
             }
             // (flat bins are 32 bits)
@@ -909,7 +909,7 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
         qb[i] = readlane_i32(qb_v, i);
         if (i < B - 1) {
             grid_rows *= nb[i];
-            rows_fit = rows_fit && nb[i] < (1 << 13) && (!CALLERS || nb[i] > 0);
+            rows_fit = rows_fit && (i == 0 || nb[i] < (1 << 13)) && (!CALLERS || nb[i] > 0);
         }
     }
     const int nb_last = nb[B - 1], qb_last = qb[B - 1];
