@@ -278,6 +278,21 @@ constexpr float kNearFirst = 0.45f;
 // strip of segment marks (one byte of LDS each); a multiple of 512.
 constexpr int kMarkCap = 2048;
 
+// How far a place in a grid, in bins, and the bins that points were given may be off: three roundings of the place for the
+// query and two for a point, each 2^-24 of the number of bins, twice that for the hardware's reciprocal. A thousandth
+// of a bin, which the bounds below allow anyway, covers grids of up to kNarrowGrid bins per dimension; beyond that
+// edges count `edge` of a bin less and widths are taken `scale` of themselves (a neighbour beyond the next bin is at
+// least half a bin away; where the places are good to less than a quarter of a bin nothing is pruned).
+constexpr int kNarrowGrid = 1 << 10;
+struct GridSlack {
+    float edge, scale;
+};
+__device__ __forceinline__ GridSlack grid_slack(int most_bins) {
+    if (most_bins <= kNarrowGrid) return {1e-3f, 1.f};
+    const float off = (float)most_bins * 0x1p-21f;
+    return {fmaxf(1e-3f, off), off < 0.25f ? 1.f - 2.f * off : 0.f};
+}
+
 // q = x / w, r = x % w for 0 <= x < 2^22 and w < 2^13, without an integer divide: with inv_w
 // within an ulp of 1 / w (the hardware's approximate reciprocal will do) the float quotient is
 // off by at most one, the remainder says which way
@@ -356,8 +371,13 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
         const int nb_last = nb[B - 1], qb_last = qb[B - 1];
         const int bins_last = FINE ? nb_last >> 1 : nb_last;  // bins (not cells) along the last dimension
         const float bw = !placed ? 0.f : FINE ? 0.5f * p.bin_width[0] : p.bin_width[0];
+        int most_bins = 0;
+#pragma unroll
+        for (int i = 0; i < kDims; ++i) most_bins = max(most_bins, nb[i]);
+        const GridSlack slack = grid_slack(most_bins);
         const float inv_bw = 1.f / bw;
-        const float bins_per_unit = 1.001f * inv_bw;  // generous by 0.1 %, for the pruning bound only
+        const float gap_bw = bw * slack.scale;           // for lower bounds of distances
+        const float bins_per_unit = 1.001f / gap_bw;  // generous by 0.1 %, for the pruning bound only
 
         // Position of the query inside its own bin, in bin widths: to_lower[i] is a
         // lower bound of its distance to the bin's lower edge, to_upper[i] to the
@@ -371,8 +391,8 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
             if (i < B && p.shift) {
                 const float frac = (qrow[i] - p.shift[i]) * inv_bw - (float)qb[i];
                 if (frac >= 0.f && frac <= 1.f) {
-                    to_lower[i] = fmaxf(frac - 1e-3f, 0.f);
-                    to_upper[i] = fmaxf(1.f - frac - 1e-3f, 0.f);
+                    to_lower[i] = fmaxf(frac - slack.edge, 0.f);
+                    to_upper[i] = fmaxf(1.f - frac - slack.edge, 0.f);
                 }
             }
         }
@@ -546,13 +566,13 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
                                 cell = cell * nb[i] + k;
                             }
                             const float edge = o > 0 ? to_upper[i] : to_lower[i];
-                            const float g = o == 0 ? 0.f : ((float)(abs(o) - 1) + edge) * bw;
+                            const float g = o == 0 ? 0.f : ((float)(abs(o) - 1) + edge) * gap_bw;
                             gap2 += g * g;
                         }
                     }
                     // a whole run of the last dimension (rows on a face of the shell), or one of the
                     // two end caps
-                    const float cap_gap = ((float)(d - 1) + (second ? tu_last : tl_last)) * bw;
+                    const float cap_gap = ((float)(d - 1) + (second ? tu_last : tl_last)) * gap_bw;
                     const float cap2 = gap2 + cap_gap * cap_gap;
                     // bins of a run that are provably too far are cut off (bound
                     // generous by 0.1 % and a thousandth of a bin)
@@ -863,7 +883,7 @@ __device__ __forceinline__ float bound_of(uint32_t pattern) { return __uint_as_f
 // The Kn smallest keys of query q, ascending, in `key` (ranks beyond the points there are: the empty key). FINE as in
 // walk_shells. False: nothing is decided (the grid of bins, or walk_shells, has to do it). CALLERS: bin rows and boundary table
 // were handed over by a caller, may contradict each other and be of any size, and `sorting` may repeat itself; without, they are those of the package's own
-// binning, which need no such checks (1.14 M points in 16 events on 43 bins: 1130 us with them, 1040 without, 1185 by shells).
+// binning, which need no such checks (1.14 M points in 16 events on 43 bins: 1150 us with them, 1040 without, 1185 by shells).
 template <int C, int NB, int S, bool MAPPED, bool FINE, bool CALLERS>
 __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q, const int lane, uint8_t *const marks,
                                                 uint64_t *const buffer, const int Kn, uint64_t (&key)[S]) {
@@ -925,10 +945,20 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
     }
     const float bw = !placed ? 0.f : FINE ? 0.5f * p.bin_width[0] : p.bin_width[0];
     // Coordinates without bounds leave widths without a meaning: then nothing is pruned, the whole grid is walked.
-    const bool prunes = bw > 1e-30f && bw < 1e18f;  // (the square stays finite)
-    const float inv_bw = __builtin_amdgcn_rcpf(bw);  // within an ulp; used with margins of a thousandth of a bin
-    const float bins_per_unit = prunes ? 1.001f * inv_bw : 3.0e38f;
-    const float gap_scale = prunes ? 0.999f * (bw * bw) : 0.f;  // bounds are generous by 0.1 %
+    bool prunes = bw > 1e-30f && bw < 1e18f;  // (the square stays finite)
+    const float inv_bw = __builtin_amdgcn_rcpf(bw);  // within an ulp
+    float bins_per_unit = 1.001f * inv_bw, gap_scale = 0.999f * (bw * bw);  // bounds are generous by 0.1 %
+    GridSlack slack{1e-3f, 1.f};
+    if constexpr (CALLERS) {  // (the package's own grids are narrow)
+        int most_bins = nb_last;
+#pragma unroll
+        for (int i = 0; i < B - 1; ++i) most_bins = max(most_bins, nb[i]);
+        slack = grid_slack(most_bins);
+        prunes = prunes && slack.scale > 0.f;
+        bins_per_unit /= slack.scale;
+        gap_scale *= slack.scale * slack.scale;
+    }
+    if (!prunes) bins_per_unit = 3.0e38f, gap_scale = 0.f;
 
     // number of the first bin of a row of the grid, from the number of the row
     auto row_base = [&](int row) {
@@ -951,8 +981,8 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
     if (p.shift) {
         const float frac = (qrow[dim] - p.shift[dim]) * inv_bw - (float)qb_v;
         if (frac >= 0.f && frac <= 1.f) {
-            tl_v = fmaxf(frac - 1e-3f, 0.f);
-            tu_v = fmaxf(1.f - frac - 1e-3f, 0.f);
+            tl_v = fmaxf(frac - slack.edge, 0.f);
+            tu_v = fmaxf(1.f - frac - slack.edge, 0.f);
         }
     }
     float from_lower[B], from_upper[B];  // 1 - these bounds
@@ -1501,8 +1531,8 @@ int binned_select_knn_strided(const float *d_coord, const int *d_bin_idx, const 
     p.cell_boundaries = d_cell_boundaries;
     p.fine_bits = fine_bits;
     p.fine_min_population = fine_min_population;
-    // the package's own tables are read with 32-bit byte offsets, their bins per dimension are factors of 24 bits
-    callers_table = callers_table || n_bboundaries >= 1 << 30 || bins_bound >= 1 << 24;
+    // the package's own tables are read with 32-bit byte offsets, and their bins per dimension are few
+    callers_table = callers_table || n_bboundaries >= 1 << 30 || bins_bound > kNarrowGrid;
     return d_sorting ? launch_coords<true>(p, callers_table, s) : launch_coords<false>(p, callers_table, s);
 }
 
