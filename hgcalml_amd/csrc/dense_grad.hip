@@ -28,7 +28,7 @@ namespace {
 constexpr int kTile = 16, kStepRows = 4, kMostTiles = 4, kMostWaves = 16;
 // row slabs' parts: one workgroup per CU, half of that where the blocks of the result take more than one workgroup
 constexpr int kMostParts = 256;
-constexpr int kLeastRows = 16;  // of a wave
+constexpr int kLeastRows = 16;  // of a wave, before they are made whole batches of kStepRows * steps_ahead() rows
 constexpr int kWaves = 8;       // of a workgroup, or the next multiple of the four SIMDs that the blocks allow
 
 typedef float acc_t __attribute__((ext_vector_type(4)));
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(kMostWaves *kWave) void weight_grad_kernel(const We
         Cols<TM> a[2][U];
         Cols<TN> b[2][U];
         auto request = [&](int at, long long batch) {
-            const size_t row = (size_t)min(batch, batches - 1) * (kStepRows * U);
+            const size_t row = (size_t)batch * (kStepRows * U);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 a[at][u] = load_cols<TM>(g + (row + u * kStepRows) * p.O);
@@ -109,18 +109,24 @@ __global__ __launch_bounds__(kMostWaves *kWave) void weight_grad_kernel(const We
             }
             __builtin_amdgcn_sched_barrier(0);  // before what is multiplied meanwhile
         };
+        auto multiply_batch = [&](int at) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) multiply(a[at][u], b[at][u]);
+        };
         if (batches > 0) {
             request(0, 0);
-            for (long long batch = 0; batch < batches; batch += 2) {
+            long long batch = 0;
+            for (; batch + 2 < batches; batch += 2) {
                 request(1, batch + 1);
-#pragma unroll
-                for (int u = 0; u < U; ++u) multiply(a[0][u], b[0][u]);
+                multiply_batch(0);
                 request(0, batch + 2);
-                if (batch + 1 < batches) {
-#pragma unroll
-                    for (int u = 0; u < U; ++u) multiply(a[1][u], b[1][u]);
-                }
+                multiply_batch(1);
             }
+            // the last one or two, the first of them under way
+            const bool another = batch + 1 < batches;
+            if (another) request(1, batch + 1);
+            multiply_batch(0);
+            if (another) multiply_batch(1);
         }
         // what is left of the slab: rows behind it count as zeros
         for (long long row = first + batches * (kStepRows * U); row < end; row += kStepRows) {

@@ -40,6 +40,20 @@ def test_every_row_counts_once_and_rows_off_a_16_byte_boundary():
     assert torch.equal(bias, torch.full((n_out,), float(n), device=DEV))
 
 
+@pytest.mark.parametrize("n_out,n_in", [(1, 1), (3, 64), (4, 29), (16, 17), (22, 29), (31, 33), (48, 73), (49, 50), (64, 65),
+                                        (63, 130), (96, 112), (129, 193), (128, 192), (160, 352)])
+# from no batch to many in a slab, odd and even numbers of them, one part of the result to 256
+@pytest.mark.parametrize("n", [1, 15, 33, 64, 96, 100, 131, 1027, 2477, 8192, 40013, 70003, 150000])
+def test_every_row_counts_once_at_all_widths(n, n_out, n_in):
+    """whole numbers whose sums stay below 2^24 are exact in any order: no row, batch, slab or part lost or counted twice"""
+    row = torch.arange(n, device=DEV)[:, None]
+    g = ((row * 5 + torch.arange(n_out, device=DEV) * 3) % 7 - 2).float()   # -2 .. 4
+    x = ((row // 3 + torch.arange(n_in, device=DEV)) % 11 - 4).float()      # -4 .. 6
+    weight, bias = ops.dense_weight_grad(g, x)
+    assert torch.equal(weight.double(), g.double().t() @ x.double())
+    assert torch.equal(bias.double(), g.double().sum(0))
+
+
 def test_values_that_are_no_numbers_stay_in_their_columns():
     n, n_out, n_in = 1030, 30, 45
     gen = torch.Generator().manual_seed(5)
