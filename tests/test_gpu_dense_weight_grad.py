@@ -13,8 +13,12 @@ DEV = "cuda:0"
 def check(g, x):
     weight, bias = ops.dense_weight_grad(g, x)
     g64, x64 = g.cpu().double(), x.cpu().double()
-    # sums of n terms in 32 bits, in any order: n 2^-24 of the sum of the terms' sizes (and far less as they are split)
-    bound = max(len(g), 4) * 2.0 ** -24
+    # A term takes part in at most as many additions as a wave's slab has rows (256 parts of the rows, 128 or more where the
+    # result takes two workgroups, rounded up to a batch of 32), the four rows of a step and the slabs of a workgroup
+    # (16) and the parts (32 by one thread, 8 threads) add theirs, and it is rounded once itself: each addition is off by
+    # 2^-24 of the sum of the terms' sizes at most.
+    n = len(g)
+    bound = (min(n, n // 128 + 32) + 4 + 16 + 32 + 8 + 1) * 2.0 ** -24
     assert ((weight.cpu() - g64.t() @ x64).abs() <= bound * (g64.abs().t() @ x64.abs())).all()
     assert ((bias.cpu() - g64.sum(0)).abs() <= bound * g64.abs().sum(0)).all()
 
@@ -68,15 +72,46 @@ def test_values_that_are_no_numbers_stay_in_their_columns():
     assert torch.isinf(bias[7]) and torch.isfinite(bias).sum() == n_out - 1
 
 
+@pytest.fixture
+def passes(monkeypatch):
+    """the shapes that reach the one pass"""
+    seen, real = [], ops.dense_weight_grad
+
+    def spy(grad, x):
+        seen.append((tuple(grad.shape), tuple(x.shape)))
+        return real(grad, x)
+    monkeypatch.setattr(ops, "dense_weight_grad", spy)
+    return seen
+
+
+# up to 2^15 weights over any rows, up to 2^16 over 2^16 rows
+@pytest.mark.parametrize("n,n_in,n_out,taken", [(70000, 256, 128, True), (70000, 257, 128, False), (65536, 256, 256, True),
+                                                (65537, 256, 256, False), (300, 257, 256, False), (65537, 100, 70, True)])
+def test_which_layers_take_the_one_pass(n, n_in, n_out, taken, passes):
+    torch.manual_seed(1)
+    layer = TallLinear(n_in, n_out).to(DEV)
+    x = torch.randn(n, n_in, device=DEV)
+    g = torch.randn(n, n_out, device=DEV)
+    weight, bias = torch.autograd.grad(layer(x), [layer.weight, layer.bias], g)
+    assert passes == ([((n, n_out), (n, n_in))] if taken else [])
+    want = g.double().t() @ x.double()
+    # sums of n terms of either sign, in parts of n / 64 rows at the most: as in check()
+    bound = (n / 64 + 100) * 2.0 ** -24
+    assert ((weight.double() - want).abs() <= bound * (g.abs().double().t() @ x.abs().double())).all()
+    assert ((bias.double() - g.double().sum(0)).abs() <= bound * g.abs().double().sum(0)).all()
+
+
 @pytest.mark.parametrize("n", [1, 700, 5000])
-def test_layer_gradients(n):
+def test_layer_gradients(n, passes):
     """the layer's gradients with and without a second derivative asked for, and through a captured graph"""
     torch.manual_seed(n)
     layer = TallLinear(45, 30).to(DEV)
     x = torch.randn(n, 45, device=DEV, requires_grad=True)
     g = torch.randn(n, 30, device=DEV)
     one = torch.autograd.grad(layer(x), [x, layer.weight, layer.bias], g)
+    assert passes == [((n, 30), (n, 45))]
     two = torch.autograd.grad(layer(x), [x, layer.weight, layer.bias], g, create_graph=True)
+    assert len(passes) == 1  # a second derivative is left to the tensor operations
     for a, b in zip(one, two):
         assert (a - b).abs().max() <= 1e-5 * (b.abs().max() + 1)
     static = torch.empty_like(g)
