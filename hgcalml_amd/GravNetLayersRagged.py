@@ -45,8 +45,8 @@ def _sum_rows(t):
 
 def _weight_grad_in_one_pass(g, x):
     """Whether weight and bias gradient of a dense layer come from the library's one pass over g and x. Wide layers over
-    many rows are the batched product's (us with the bias' sums, one pass / batched: 240,000 rows, 160 x 352 376 / 290;
-    150,000, 160 x 256 140 / 135, 128 x 256 101 / 115; 60,000, 160 x 352 104 / 121; 20,000 43 / 69)."""
+    many rows are the batched product's (us with the bias' sums, one pass / batched: 240,000 rows, 160 x 352 371 / 300;
+    150,000, 160 x 256 139 / 141, 128 x 256 93 / 112; 65,536, 256 x 256 90 / 88; 60,000, 160 x 352 98 / 122; 20,000 43 / 85)."""
     widths = g.shape[1] * x.shape[1]
     return (not torch.is_grad_enabled() and _library_takes(g, x) and
             (widths <= 1 << 15 or (widths <= 1 << 16 and x.shape[0] <= 1 << 16)))

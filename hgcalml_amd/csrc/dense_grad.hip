@@ -13,10 +13,11 @@
 // the same order, and both write the same.
 //
 // Measured next to what it replaced, a batched library product over 64 slices of the rows, the slices' sum and the
-// gradient's column sums, us: 150,000 rows, 128 x 192 99 -> 76 to 84, 64 x 64 68 -> 23; 240,011, 96 x 112 90 -> 62;
-// 2477, 48 x 73 31 -> 10; its error against 64 bits is half as large. What keeps wide layers from the instruction's rate is
-// the L1, in which the blocks of a slab meet: 240,000 rows, 160 x 352 take 376 us, the batched product 290. Tried and taken
-// back: the rows through LDS, in lockstep (128 x 192 88 to 92 us, 240,000 rows, 96 x 112 72 to 77, 160 x 352 454).
+// gradient's column sums, us: 150,000 rows, 128 x 192 99 -> 81, 64 x 64 68 -> 23; 240,011, 96 x 112 90 -> 59; 2477, 48 x 73
+// 31 -> 10; its error against 64 bits is half as large. What keeps wide layers from the instruction's rate is the L1, in which
+// the blocks of a slab meet: 150,000 rows, 128 x 192 read their rows 1.7 times from L2 and keep the matrix cores 60 % busy,
+// 240,000 rows, 160 x 352 3.5 times and 57 % (393 us, the batched product 290). Tried and taken back:
+// the rows through LDS, in lockstep (128 x 192 88 to 92 us, 240,000 rows, 96 x 112 72 to 77, 160 x 352 454).
 #include <algorithm>
 
 #include "hgc_common.hpp"
@@ -63,7 +64,7 @@ struct WeightGrad {
 
 // Steps that are under way while as many are multiplied: enough bytes for narrow tiles. With wide ones the waves of a
 // slab drift apart the further they read ahead and miss each other's rows in the L1 (150,000 rows, 128 x 192, one, two
-// and four steps: 76, 88 and 97 us).
+// and four steps: 76, 88 and 97 us with requests beyond the slab's end, which are gone).
 constexpr int steps_ahead(int tiles) { return tiles > 8 ? 1 : tiles > 2 ? 4 : 8; }
 
 template <int TM, int TN>

@@ -260,18 +260,18 @@ __device__ __forceinline__ void merge_batch(uint64_t (&key)[S], uint64_t batch) 
 }
 
 // below this many entering candidates in a step of 64 the one-by-one insert is cheaper
-// (150k points in 4-D, K = 64, clusters / Gaussian blob: 0.519 / 0.924 ms at 12, 0.508 / 0.881 at 16,
-// 0.504 / 0.864 at 20 and 24, 0.517 / 0.899 at 32)
+// (150,000 points, walks by shells of both kinds, ms a call at 12 / 16 / 20 / 24 / 32: K = 200 4-D clusters 1.42 / 1.37 /
+// 1.34 / 1.35 / 1.42, 4-D Gaussian 2.15 / 2.04 / 2.01 / 2.03 / 2.18, 3-D uniform 1.26 / 1.15 / 1.09 / 1.09 / 1.18; K = 64 5-D
+// clusters 0.65 / 0.64 / 0.64 / 0.64 / 0.66, 6-D clusters 1.00 / 1.00 / 1.01 / 1.03 / 1.06)
 constexpr int kBulkInsertMin = 20;
 // lists of more runs than this would insert one by one (a merge costs 12 more steps per run)
 constexpr int kBulkInsertMaxRuns = 8;
 
-// NEAR_FIRST (the kernels of the nested grid, i.e. 48 neighbours and more: 16 events of 3-D points
-// with K = 32 and a radius ran 4 % slower with it): segments of a batch whose bins are at least
-// sqrt(kNearFirst) * d bin widths away (shell d) are walked after the nearer ones
-// (150,000 points in 4-D, K = 64, kernel: Gaussian blob 508 us without,
-// 455 / 464 / 464 / 473 us at 0.3 / 0.45 / 0.6 / 0.75; clusters + noise 409, 407 / 405 / 413 / 418;
-// uniform 347, 359 / 352 / 347 / 354)
+// NEAR_FIRST (the kernels of the nested grid that walk shells, i.e. 3-D and 4-D points with 130 to 513 neighbours):
+// segments of a batch whose bins are at least sqrt(kNearFirst) * d bin widths away (shell d) are walked after the nearer
+// ones (150,000 points, K = 200, ms a call without, and at 0.3 / 0.45 / 0.6 / 0.75: 4-D Gaussian 2.69, 1.95 / 2.01 / 2.11 /
+// 2.22; 4-D clusters 1.49, 1.35 / 1.32 / 1.31 / 1.33; 4-D uniform 1.79, 1.72 / 1.63 / 1.54 / 1.50; 3-D clusters 1.18, 1.10 /
+// 1.05 / 1.02 / 1.03; 3-D Gaussian 1.74, 1.31 / 1.36 / 1.42 / 1.49)
 constexpr float kNearFirst = 0.45f;
 
 // Candidates of one batch of segments that are walked per refill of a wave's
@@ -428,7 +428,7 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
         }
         // the first shell whose slots need more than one batch of 64 (walked whole: (2d+1)^(B-1)
         // rows and (2d-1)^(B-1) inner rows; on the nested grid d + 1 pieces per row)
-        const int first_cut_shell = FINE ? (B == 2 ? 5 : B == 3 ? 2 : B == 4 ? 2 : 1) : (B == 2 ? 17 : B == 3 ? 3 : B == 4 ? 2 : 1);
+        const int first_cut_shell = FINE ? 2 : (B == 2 ? 17 : B == 3 ? 3 : B == 4 ? 2 : 1);
 
         // Shell 0 (the query's own bin) never ends the search. When it cannot fill
         // the list either (so that it cannot prune shell 1), it is walked together
@@ -735,8 +735,8 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
 //   * then the Kn-th distance is bounded by bisection (counts are ballots) and what lies beyond is dropped;
 //   * then one pass over the rows of bins outside the cube that the bound reaches;
 //   * then the keys that are left are sorted, once.
-// Vector instructions per query: 16 events of 1.14 M 3-D points, K = 32, radius 0.1 about 700 -> 465, 150,000 4-D
-// points, K = 65 1475 -> 1087. The whole search, by shells -> collected: these two 1399 -> 1173 us and 429 -> 372 us;
+// Vector instructions per query: 16 events of 1.14 M 3-D points, K = 32, radius 0.1 about 700 -> 474, 150,000 4-D
+// points, K = 64 1476 -> 1074. The whole search, by shells -> collected: these two 1399 -> 1173 us and 429 -> 372 us;
 // 240,000 3-D points, K = 41 367 -> 307; 4-D Gaussian, K = 65 467 -> 410; 4-D uniform, K = 64 361 -> 305; 2-D
 // clusters, K = 32 186 -> 130; 3-D clusters, K = 96 489 -> 319. Tried and taken back: first regions that leave out the
 // corners of the cube (fewer candidates, but a second pass for every query: 4 to 13 % slower), up to three pieces of a
@@ -866,7 +866,7 @@ __device__ __forceinline__ int cut_to_smallest(uint64_t *const buffer, const int
     return left;
 }
 
-// table[i] with the table in scalar registers and a 32-bit byte offset (tables of collect_nearest stay below 2^30 entries)
+// table[i] with the table in scalar registers and a 32-bit byte offset (the package's own tables, below 2^30 entries)
 __device__ __forceinline__ int table_entry(const int *__restrict__ table, int i) {
     return *reinterpret_cast<const int *>(reinterpret_cast<const char *>(table) + ((uint32_t)i << 2));
 }
@@ -887,7 +887,7 @@ __device__ __forceinline__ float bound_of(uint32_t pattern) { return __uint_as_f
 template <int C, int NB, int S, bool MAPPED, bool FINE, bool CALLERS>
 __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q, const int lane, uint8_t *const marks,
                                                 uint64_t *const buffer, const int Kn, uint64_t (&key)[S]) {
-    static_assert(C > 0 && NB >= 2 && NB <= 4 && S <= 2);
+    static_assert(C > 0 && NB >= 2 && NB <= 4 && S <= 2 && (!FINE || NB >= 3));
     constexpr int B = NB;
     float qc[C];
     const float *qrow = p.coord + (size_t)q * C;
@@ -1012,7 +1012,7 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
         bool in_grid = true;
         if constexpr (FINE) {
             int row = lane >> 1;
-            in_grid = row < (B == 2 ? 3 : B == 3 ? 9 : 27);
+            in_grid = row < (B == 3 ? 9 : 27);
 #pragma unroll
             for (int i = B - 2; i >= 0; --i) {
                 off[i] = (i > 0 ? row % 3 : row) - 1;

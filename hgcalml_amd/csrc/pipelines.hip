@@ -34,36 +34,33 @@ namespace {
 //   * Up to four binned dimensions: binning the fourth coordinate of 4-D points too removes the
 //     candidates that are close in three coordinates and far in the fourth.
 //   * n_bins = 0.9 (points per event * 64 / K)^(1/dimensions) with K taken inside 32 .. 64 (0.85
-//     under a nested grid, below): a bit
-//     more than one point per bin at K = 64, and finer for fewer neighbours (16 events of 20,000 to
-//     120,000 3-D points, K = 32, radius 0.1: 1.72 ms -> 1.59 ms). For more than 64 neighbours a
-//     coarser grid did not pay (150,000 clustered 4-D points, K = 129 / 257: 0.96 / 2.23 ms on the
-//     grid for 64, 1.02 / 2.49 ms on one scaled further).
-//   * Where every coordinate is binned (2 to 4 of them) and the table stays small, a nested grid of
-//     half the bin width for the queries of crowded bins (bin_grouping's spatial mode,
-//     KnnParams::fine_bits): with it the bins themselves can be wider than a single grid would
-//     want them, which is what sparse regions like (their shells are mostly empty bins). Measured
-//     kernel times, 150,000 points in 4-D, K = 64, single grid of 20 bins -> nested grid on 18 bins:
-//     clusters + noise 450 -> 425 us, Gaussian blob 825 -> 515 us, uniform 418 -> 351 us. The whole
-//     call with and without it on the same bins, in ms (150,000 points; the nested grid's table is
-//     2^dimensions times larger, and few neighbours come from few candidates either way):
-//                               K = 8          16            32            64            129
-//       4-D clusters + noise  0.43 / 0.28   0.38 / 0.31   0.40 / 0.37   0.47 / 0.47   0.86 / 0.86
-//       4-D Gaussian blob     0.35 / 0.32   0.38 / 0.38   0.44 / 0.52   0.56 / 0.82   1.04 / 1.86
-//       3-D clusters + noise  0.31 / 0.23   0.30 / 0.25   0.32 / 0.30   0.36 / 0.36   0.61 / 0.64
-//       3-D uniform           0.33 / 0.21   0.29 / 0.24   0.33 / 0.29   0.35 / 0.32   0.55 / 0.53
-//       3-D Gaussian blob     0.26 / 0.25   0.29 / 0.29   0.33 / 0.36   0.37 / 0.52   0.70 / 0.96
-//       2-D clusters + noise  0.28 / 0.22   0.30 / 0.27   0.36 / 0.33   0.36 / 0.35   0.60 / 0.59
-//     so it is taken from 48 neighbours on and three binned dimensions on.
+//     under a nested grid, below): a bit more than one point per bin at K = 64, and finer for fewer neighbours.
+//     Whole calls on 0.85 / 1 / 1.15 of these bins, us (150,000 points): K = 16 4-D clusters 246 / 237 / 244, 4-D Gaussian 357 /
+//     332 / 328, 4-D uniform 213 / 215 / 242, 3-D clusters 191 / 192 / 192, 2-D clusters 172 / 179 / 181; K = 64 348 / 344 / 352,
+//     451 / 411 / 404, 294 / 313 / 358, 262 / 261 / 258, 222 / 231 / 236; 15 events of a million 3-D points, K = 32, radius 0.1
+//     1016 / 984 / 949: uniform points would like fewer bins, blobs more. Fewer still for more than 64 neighbours (64 / 129
+//     as the end of the rule, K = 129): 4-D clusters 461 / 471, 4-D Gaussian 597 / 647, 4-D uniform 526 / 416.
+//   * Where every coordinate is binned (3 or 4 of them) and the table stays small, a nested grid of half the bin width
+//     for the queries of crowded bins (bin_grouping's spatial mode, KnnParams::fine_bits): with it the bins
+//     themselves can be wider than a single grid would want them, which is what sparse regions like. It costs the
+//     grouping a table that is 2^dimensions times larger, and few neighbours come from few candidates either way.
+//     The whole call with and without it (single grid: 0.9, as above), in us (150,000 points):
+//                          K = 8        16         32         48         64         129
+//       4-D clusters     322 / 232  270 / 234  289 / 258  313 / 279  342 / 322  459 / 444
+//       4-D Gaussian     286 / 280  298 / 332  340 / 409  349 / 490  398 / 603  596 / 903
+//       4-D uniform      341 / 199  240 / 210  257 / 261  275 / 285  308 / 321  518 / 512
+//       3-D clusters     211 / 178  198 / 184  206 / 197  217 / 211  255 / 251  360 / 351
+//       3-D uniform      216 / 176  186 / 176  197 / 195  205 / 200  242 / 238  335 / 344
+//       3-D Gaussian     203 / 207  213 / 224  231 / 241  242 / 264  281 / 321  413 / 441
+//     so it is taken from 48 neighbours on: there it costs clusters 3 to 12 % and saves crowded blobs 8 to 34 %.
 //   * Points with more than four coordinates bin the first four, on the same rule (their bins hold
 //     every point along the other coordinates, so the neighbourhood is wide in bin widths however
-//     fine the grid; a nested grid does not pay there). 150,000 points, K = 64, three binned
+//     fine the grid; a nested grid does not pay there). They are searched by shells. 150,000 points, K = 64, three binned
 //     dimensions at 32 bins -> four at 18: 5-D Gaussian 2.07 -> 1.45 ms, 6-D Gaussian 2.91 -> 2.20 ms,
 //     6-D uniform 2.24 -> 1.62 ms, 8-D Gaussian 7.40 -> 5.85 ms. (Gaussians like more bins still,
 //     uniform boxes fewer: 24 / 11 bins give 1.17 / 2.32, 2.08 / 3.71, 2.71 / 1.23, 5.95 / 7.70 ms.)
-//   * Small events want fewer bins than that (most of a small grid is boundary): 200,000 uniform
-//     4-D points in 1000 events, K = 64: 0.80 ms at 4 bins, 0.52 at 3; in 4000 events 1.07 ms at
-//     4 bins, 0.31 at 2.
+//   * Small events want fewer bins than that (most of a small grid is boundary), us without and with that rule: 200,000
+//     uniform 4-D points, K = 64 in 200 events 403 / 362, in 1000 322 / 274; K = 16 in 4000 events 238 / 185.
 thread_local int g_callers_knn_grid = 0;
 
 struct SearchGrid {
@@ -78,7 +75,10 @@ SearchGrid callers_grid(int n_coords, int n_bins_scalar, int max_bin_dims) {
 // kSmallestGridK: the grid for this many neighbours or fewer is the finest one (it sizes the workspace)
 constexpr int kSmallestGridK = 32, kLargestGridK = 64;
 // a bin with more than (K - 1) / kCrowdedBinFraction points sends its queries to the nested grid
-constexpr int kCrowdedBinFraction = 3;  // 2 .. 6 measured: 3 is best by 1 to 3 % on clustered, Gaussian and uniform points
+// (us at 2 / 3 / 4 / 6: K = 64 4-D clusters 350 / 357 / 375 / 394, 4-D Gaussian 404 / 399 / 409 / 425, 3-D Gaussian 290 / 281 /
+// 284 / 290; K = 129 451 / 459 / 471 / 497, 657 / 596 / 588 / 606, 444 / 415 / 406 / 409; 4-D Gaussian, K = 200 2285 / 2006 / 1833 /
+// 1700; uniform points level)
+constexpr int kCrowdedBinFraction = 3;
 // fewer neighbours than this search on the single grid (see the table above own_grid)
 constexpr int kSmallestNestedK = 48;
 
@@ -89,9 +89,9 @@ SearchGrid own_grid(int n_vert, int n_coords, int n_rs, int n_neigh) {
     const double small = std::min(1.0, std::max(0.75, 0.75 + 0.25 * (std::log10(per_event) - 3.7)));
     const double k = std::min(std::max(n_neigh, kSmallestGridK), kLargestGridK);
     const bool nested = dims == n_coords && dims >= 3 && n_neigh >= kSmallestNestedK;
-    // under a nested grid the bins can be a little wider still (150,000 points, K = 64, factor 0.9 -> 0.85:
-    // clusters + noise and Gaussian blob unchanged, 4-D uniform 0.40 -> 0.385 ms, 3-D clusters 0.354 -> 0.346 ms;
-    // at 0.8 and below the blob loses 2 to 4 %)
+    // under a nested grid the bins can be a little wider still (150,000 points, K = 64, us at 0.9 / 0.85 / 0.8: 4-D clusters
+    // 361 / 357 / 370, 4-D Gaussian 402 / 399 / 406, 4-D uniform 330 / 310 / 297, 3-D clusters 255 / 256 / 256; K = 129 463 / 459 /
+    // 458, 592 / 596 / 586, 520 / 520 / 460, 355 / 361 / 358)
     const double n_bins = (nested ? 0.85 : 0.9) * small * std::pow(per_event * 64.0 / k, 1.0 / dims);
     return {dims, std::max(2, std::min((int)std::lround(n_bins), dims >= 4 ? 40 : dims == 3 ? 128 : 1024)), nested};
 }

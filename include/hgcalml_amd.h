@@ -170,7 +170,12 @@ int hgc_gather_rows(const void *d_in, const int *d_rows, void *d_out, int n_rows
  * than 45 bins each) ends there and sets HGC_FLAG_SHELL_TOO_WIDE in the status word;
  * without a registered status word that is silent and the rows of such queries
  * can miss neighbours (hgc_binned_select_knn_pipeline refuses such grids on the
- * host instead, whatever the status word). */
+ * host instead, whatever the status word).
+ * Bins beyond the end of the boundary table hold no points and set
+ * HGC_FLAG_BIN_BEYOND_TABLE, as do bins, or numbers of bins, that no grid has; a
+ * row of d_dim_bin_idx outside the grid, or of another bin than the point's own one,
+ * has the point searched in its whole event. The entries of the table themselves have
+ * to rise and to end at n_vert or before: they are not looked at. */
 int hgc_binned_select_knn(const float *d_coord, const int *d_bin_idx, const int *d_direction,
                           const int *d_dim_bin_idx, const int *d_bin_boundaries,
                           const int *d_n_bins, const float *d_bin_width,
