@@ -435,7 +435,7 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
         // with shell 1: every row of that shell then takes its whole run of the last
         // dimension, and the run of the centre row contains the own bin.
         bool with_own_bin = false;
-        if (reach_max > 0 && own_bin >= 0 && own_bin + 1 < p.n_bboundaries) {
+        if (reach_max > 0 && own_bin >= 0 && own_bin < p.n_bboundaries - 1) {
             if (FINE)
                 with_own_bin = p.cell_boundaries[own_cell + 1] - p.cell_boundaries[own_cell] <= Kn;
             else

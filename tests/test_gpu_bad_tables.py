@@ -79,12 +79,14 @@ def test_rows_that_do_not_name_the_own_bin(oracle, dims, kind, K, radius):
 
 @pytest.mark.parametrize("dims", [2, 3, 4])
 @pytest.mark.parametrize("K", [6, 140])  # collected, and by shells
-def test_bins_below_every_event_have_no_neighbours(oracle, dims, K):
+@pytest.mark.parametrize("n_bins", [3, 4, 5])
+@pytest.mark.parametrize("where", ["below", "the largest integer"])
+def test_bins_outside_every_event_have_no_neighbours(oracle, dims, K, n_bins, where):
     from hgcalml_amd import ops
-    binned = Binned(oracle, dims)
+    binned = Binned(oracle, dims, n_bins)
     want = binned.search(K)
     bad = torch.arange(len(binned.x)) % 11 == 0
-    binned.flat[bad.numpy()] = -binned.cells - 3
+    binned.flat[bad.numpy()] = -binned.cells - 3 if where == "below" else (1 << 31) - 1
     idx, dist, flags = binned.search(K)
     assert want[2] == 0 and flags == ops.FLAG_BIN_BEYOND_TABLE
     assert torch.equal(idx[~bad], want[0][~bad]) and torch.equal(dist[~bad], want[1][~bad])
