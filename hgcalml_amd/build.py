@@ -1,8 +1,7 @@
 """Builds libhgcalml_amd.so (HIP kernels + C ABI) for gfx950 with hipcc.
 
 Run as ``python -m hgcalml_amd.build``. hipcc cross-compiles, so no GPU is
-needed. The library is written next to the sources (in-tree) so that it travels
-with the repository snapshot to the GPU box.
+needed. The library is written next to the sources, where the package loads it.
 """
 import os
 import shutil

@@ -318,7 +318,7 @@ __device__ __forceinline__ void divmod_small(int x, int w, float inv_w, int &q, 
 // being binned, that is the rule where the bin's neighbourhood is about as crowded as the bin.
 constexpr int kFineMaxShell = 3;
 
-template <int C, int NB, int S, bool MAPPED, bool WINDOW, bool FINE, bool NEAR_FIRST>
+template <int C, int NB, int S, bool MAPPED, bool WINDOW, bool FINE, bool NEAR_FIRST, bool CALLERS>
 __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, const int lane, uint8_t *const marks,
                                             const int Kn, const uint64_t floor_key, uint64_t (&key)[S]) {
     constexpr int kDims = NB > 0 ? NB : kMaxBinDims;  // array extents
@@ -347,7 +347,7 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
                 qb[i] = uniform(p.dim_bin_idx[(size_t)q * (B + 1) + 1 + i]);
                 cells_per_event *= nb[i];
                 in_event = in_event * nb[i] + qb[i];
-                outside |= qb[i] | (nb[i] - 1 - qb[i]);
+                if (CALLERS) outside |= qb[i] | (nb[i] - 1 - qb[i]);
                 if (FINE) {
                     nb[i] *= 2;
                     qb[i] = 2 * qb[i] + ((own_cell >> (B - 1 - i)) & 1);
@@ -358,7 +358,7 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
         const int event_base = own_bin - own_bin % max(cells_per_event, 1);
         // A row outside the grid, or of another bin than the own one, does not say where the query is: then the whole grid
         // of the event is walked from the nearest bin inside, and (with bins of no width) nothing is pruned.
-        const bool placed = outside >= 0 && own_bin - event_base == in_event;
+        const bool placed = !CALLERS || (outside >= 0 && own_bin - event_base == in_event);
         if (!placed) {
             reach_max = 0;
 #pragma unroll
@@ -371,10 +371,13 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
         const int nb_last = nb[B - 1], qb_last = qb[B - 1];
         const int bins_last = FINE ? nb_last >> 1 : nb_last;  // bins (not cells) along the last dimension
         const float bw = !placed ? 0.f : FINE ? 0.5f * p.bin_width[0] : p.bin_width[0];
-        int most_bins = 0;
+        GridSlack slack{1e-3f, 1.f};
+        if constexpr (CALLERS) {  // (the package's own grids are narrow)
+            int most_bins = 0;
 #pragma unroll
-        for (int i = 0; i < kDims; ++i) most_bins = max(most_bins, nb[i]);
-        const GridSlack slack = grid_slack(most_bins);
+            for (int i = 0; i < kDims; ++i) most_bins = max(most_bins, nb[i]);
+            slack = grid_slack(most_bins);
+        }
         const float inv_bw = 1.f / bw;
         const float gap_bw = bw * slack.scale;           // for lower bounds of distances
         const float bins_per_unit = 1.001f / gap_bw;  // generous by 0.1 %, for the pruning bound only
@@ -419,7 +422,7 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
                 is_grid = is_grid && nb[i] > 0;
             }
             // (flat bins are 32 bits)
-            if (!FINE && grid_rows < (1ll << 22)) is_grid = is_grid && 2ll * event_base + grid_rows * nb_last <= 1ll << 32;
+            if (CALLERS && grid_rows < (1ll << 22)) is_grid = is_grid && 2ll * event_base + grid_rows * nb_last <= 1ll << 32;
             if (!rows_fit || grid_rows >= (1ll << 22) || !is_grid) {
                 if (FINE) return false;  // the grid of bins may do
                 if (p.status && lane == 0) atomicOr(p.status, is_grid ? HGC_FLAG_SHELL_TOO_WIDE : HGC_FLAG_BIN_BEYOND_TABLE);
@@ -613,12 +616,19 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
                             const int first = event_base + cell * nb_last + lo;
                             const int last = event_base + cell * nb_last + hi + 1;
                             // bins beyond the table are skipped, as by the reference, which prints "idx out of range"
-                            const int there = min(last, p.n_bboundaries - 1);
-                            if (first < there) {
+                            if constexpr (CALLERS) {
+                                const int there = min(last, p.n_bboundaries - 1);
+                                if (first < there) {
+                                    seg_start = p.bin_boundaries[first];
+                                    seg_len = p.bin_boundaries[there] - seg_start;
+                                }
+                                if (p.status && there < last) atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
+                            } else if (last < p.n_bboundaries) {
                                 seg_start = p.bin_boundaries[first];
-                                seg_len = p.bin_boundaries[there] - seg_start;
+                                seg_len = p.bin_boundaries[last] - seg_start;
+                            } else if (p.status) {
+                                atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
                             }
-                            if (p.status && there < last) atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
                         }
                     }
                 }
@@ -881,9 +891,7 @@ constexpr bool collects(int C, int NB, int S, bool window) { return C == NB && N
 __device__ __forceinline__ float bound_of(uint32_t pattern) { return __uint_as_float(max(pattern, 0x00800000u)); }
 
 // The Kn smallest keys of query q, ascending, in `key` (ranks beyond the points there are: the empty key). FINE as in
-// walk_shells. False: nothing is decided (the grid of bins, or walk_shells, has to do it). CALLERS: bin rows and boundary table
-// were handed over by a caller, may contradict each other and be of any size, and `sorting` may repeat itself; without, they are those of the package's own
-// binning, which need no such checks (1.14 M points in 16 events on 43 bins: 1150 us with them, 1040 without, 1185 by shells).
+// walk_shells. False: nothing is decided (the grid of bins, or walk_shells, has to do it). CALLERS as in knn_wave_kernel.
 template <int C, int NB, int S, bool MAPPED, bool FINE, bool CALLERS>
 __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q, const int lane, uint8_t *const marks,
                                                 uint64_t *const buffer, const int Kn, uint64_t (&key)[S]) {
@@ -1039,7 +1047,7 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
             }
         }
         // What the radius leaves of a row: with bins wider than the radius the cube is mostly beyond it (60,000 4-D Gaussian
-        // points, radius 0.1, K = 40: 139 -> 82 us a call; 16 events of 1.14 M points, radius 0.1: 1183 -> 1171).
+        // points, radius 0.1, K = 40: 139 -> 80 us a call; 16 events of 1.14 M points, radius 0.1: 1183 -> 1171).
         int lo_most = 1 << 30, hi_most = 1 << 30;
         if (has_radius && prunes) {
             float gap2 = 0.f;
@@ -1114,7 +1122,7 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
     for (;;) {
         const bool bounded = prunes && cut < 0x7f000000u;
         // Everything within the bound; where the list is not full and a radius reaches far, larger cubes come first (with
-        // radius 3 in the unit square, 60,000 points, K = 40 one pass over everything takes 1045 us, this 102).
+        // radius 3 in the unit square, 60,000 points, K = 40 one pass over everything takes 1045 us, this 97).
         const bool last_pass = bounded && d_in >= 0 && (n_kept >= Kn || d_radius <= 2 * d_in + 2);
         int below[B], width[B], below_in[B], width_in[B];
         float inv_width[B], inv_width_in[B];
@@ -1373,13 +1381,13 @@ __device__ __forceinline__ void search_query(const KnnParams &p, const int q, co
         } else {
             bool found = false;
             if constexpr (NESTED) {
-                found = crowded && walk_shells<C, NB, S, MAPPED, WINDOW, true, NESTED>(p, q, lane, marks, Kn, floor_key, key);
+                found = crowded && walk_shells<C, NB, S, MAPPED, WINDOW, true, NESTED, CALLERS>(p, q, lane, marks, Kn, floor_key, key);
                 if (!found) {
 #pragma unroll
                     for (int s = 0; s < S; ++s) key[s] = kEmptyKey;
                 }
             }
-            if (!found) walk_shells<C, NB, S, MAPPED, WINDOW, false, NESTED>(p, q, lane, marks, Kn, floor_key, key);
+            if (!found) walk_shells<C, NB, S, MAPPED, WINDOW, false, NESTED, CALLERS>(p, q, lane, marks, Kn, floor_key, key);
         }
     }
 
@@ -1399,7 +1407,11 @@ __device__ __forceinline__ void search_query(const KnnParams &p, const int q, co
     }
 }
 
-template <int C, int NB, int S, bool MAPPED, bool WINDOW = false, bool NESTED = false, bool CALLERS = false>
+// CALLERS: bin rows and boundary table were handed over by a caller, may contradict each other and be of any size, the
+// grid may be of any width, and `sorting` may repeat itself. Without, they are those of the package's own binning, which need
+// no such checks (1.14 M 3-D points in 16 events on 43 bins, K = 32: 1150 us with them, 1040 without, 1185 by shells; 4-D, K = 200
+// by shells 1525 and 1440; with checks for every call the searches on the package's own grid were 1 to 4 % slower).
+template <int C, int NB, int S, bool MAPPED, bool CALLERS, bool WINDOW = false, bool NESTED = false>
 __global__ __launch_bounds__(kWave)
 __attribute__((amdgpu_waves_per_eu(S <= 2 ? 8 : 1, 8)))
 void knn_wave_kernel(const KnnParams p) {
@@ -1411,44 +1423,37 @@ void knn_wave_kernel(const KnnParams p) {
     search_query<C, NB, S, MAPPED, WINDOW, NESTED, CALLERS>(p, q, lane_id(), marks, buffer);
 }
 
-template <int C, int NB, bool MAPPED>
-int launch_levels(const KnnParams &p, bool callers_table, hipStream_t s) {
+template <int C, int NB, bool MAPPED, bool CALLERS>
+int launch_levels(const KnnParams &p, hipStream_t s) {
     const int levels = std::max(1, ceil_div(p.K - 1, kWave));
     const dim3 grid(p.n_vert), block(kWave);
     if (levels > kBulkInsertMaxRuns) {  // more neighbours than the registers hold: one launch per window of ranks
         KnnParams window = p;
         for (window.rank_base = 0; window.rank_base < p.K - 1; window.rank_base += kBulkInsertMaxRuns * kWave) {
-            knn_wave_kernel<C, NB, kBulkInsertMaxRuns, MAPPED, true><<<grid, block, 0, s>>>(window);
+            knn_wave_kernel<C, NB, kBulkInsertMaxRuns, MAPPED, CALLERS, true><<<grid, block, 0, s>>>(window);
             const int rc = check_launch("knn_wave_kernel (window of ranks)");
             if (rc) return rc;
         }
         return HGC_OK;
     }
-    if constexpr (MAPPED && C == NB && NB >= 3 && NB <= 4) {  // all coordinates binned: a crowded bin has its neighbours close by
+    if constexpr (MAPPED && !CALLERS && C == NB && NB >= 3 && NB <= 4) {  // all coordinates binned: a crowded bin has its neighbours close by
         if (p.fine_bits > 0 && p.cell_boundaries) {
             switch (levels) {
-                case 1: knn_wave_kernel<C, NB, 1, MAPPED, false, true><<<grid, block, 0, s>>>(p); break;
-                case 2: knn_wave_kernel<C, NB, 2, MAPPED, false, true><<<grid, block, 0, s>>>(p); break;
+                case 1: knn_wave_kernel<C, NB, 1, MAPPED, CALLERS, false, true><<<grid, block, 0, s>>>(p); break;
+                case 2: knn_wave_kernel<C, NB, 2, MAPPED, CALLERS, false, true><<<grid, block, 0, s>>>(p); break;
                 case 3:
-                case 4: knn_wave_kernel<C, NB, 4, MAPPED, false, true><<<grid, block, 0, s>>>(p); break;
-                default: knn_wave_kernel<C, NB, 8, MAPPED, false, true><<<grid, block, 0, s>>>(p); break;
+                case 4: knn_wave_kernel<C, NB, 4, MAPPED, CALLERS, false, true><<<grid, block, 0, s>>>(p); break;
+                default: knn_wave_kernel<C, NB, 8, MAPPED, CALLERS, false, true><<<grid, block, 0, s>>>(p); break;
             }
             return check_launch("knn_wave_kernel (nested grid)");
         }
     }
-    if constexpr (collects(C, NB, 1, false)) {
-        if (callers_table && levels <= 2) {
-            if (levels == 1) knn_wave_kernel<C, NB, 1, MAPPED, false, false, true><<<grid, block, 0, s>>>(p);
-            else knn_wave_kernel<C, NB, 2, MAPPED, false, false, true><<<grid, block, 0, s>>>(p);
-            return check_launch("knn_wave_kernel (a caller's table)");
-        }
-    }
     switch (levels) {
-        case 1: knn_wave_kernel<C, NB, 1, MAPPED><<<grid, block, 0, s>>>(p); break;
-        case 2: knn_wave_kernel<C, NB, 2, MAPPED><<<grid, block, 0, s>>>(p); break;
+        case 1: knn_wave_kernel<C, NB, 1, MAPPED, CALLERS><<<grid, block, 0, s>>>(p); break;
+        case 2: knn_wave_kernel<C, NB, 2, MAPPED, CALLERS><<<grid, block, 0, s>>>(p); break;
         case 3:
-        case 4: knn_wave_kernel<C, NB, 4, MAPPED><<<grid, block, 0, s>>>(p); break;
-        default: knn_wave_kernel<C, NB, 8, MAPPED><<<grid, block, 0, s>>>(p); break;
+        case 4: knn_wave_kernel<C, NB, 4, MAPPED, CALLERS><<<grid, block, 0, s>>>(p); break;
+        default: knn_wave_kernel<C, NB, 8, MAPPED, CALLERS><<<grid, block, 0, s>>>(p); break;
     }
     return check_launch("knn_wave_kernel");
 }
@@ -1456,21 +1461,21 @@ int launch_levels(const KnnParams &p, bool callers_table, hipStream_t s) {
 // The usual shapes (up to 8 coordinates; binned dimensions = min(3, coordinates), the reference
 // wrapper's default, or min(4, coordinates), the pipeline's own grid) get kernels with both
 // numbers fixed at compile time, anything else the one that reads them.
-template <bool MAPPED>
-int launch_coords(const KnnParams &p, bool callers_table, hipStream_t s) {
-    if (p.n_coords == 2 && p.n_bin_dim == 2) return launch_levels<2, 2, MAPPED>(p, callers_table, s);
-    if (p.n_coords == 3 && p.n_bin_dim == 3) return launch_levels<3, 3, MAPPED>(p, callers_table, s);
-    if (p.n_coords == 4 && p.n_bin_dim == 3) return launch_levels<4, 3, MAPPED>(p, callers_table, s);
-    if (p.n_coords == 4 && p.n_bin_dim == 4) return launch_levels<4, 4, MAPPED>(p, callers_table, s);
-    if (p.n_coords == 5 && p.n_bin_dim == 4) return launch_levels<5, 4, MAPPED>(p, callers_table, s);
-    if (p.n_coords == 6 && p.n_bin_dim == 4) return launch_levels<6, 4, MAPPED>(p, callers_table, s);
-    if (p.n_coords == 7 && p.n_bin_dim == 4) return launch_levels<7, 4, MAPPED>(p, callers_table, s);
-    if (p.n_coords == 8 && p.n_bin_dim == 4) return launch_levels<8, 4, MAPPED>(p, callers_table, s);
-    if (p.n_coords == 5 && p.n_bin_dim == 3) return launch_levels<5, 3, MAPPED>(p, callers_table, s);
-    if (p.n_coords == 6 && p.n_bin_dim == 3) return launch_levels<6, 3, MAPPED>(p, callers_table, s);
-    if (p.n_coords == 7 && p.n_bin_dim == 3) return launch_levels<7, 3, MAPPED>(p, callers_table, s);
-    if (p.n_coords == 8 && p.n_bin_dim == 3) return launch_levels<8, 3, MAPPED>(p, callers_table, s);
-    return launch_levels<0, 0, MAPPED>(p, callers_table, s);
+template <bool MAPPED, bool CALLERS>
+int launch_coords(const KnnParams &p, hipStream_t s) {
+    if (p.n_coords == 2 && p.n_bin_dim == 2) return launch_levels<2, 2, MAPPED, CALLERS>(p, s);
+    if (p.n_coords == 3 && p.n_bin_dim == 3) return launch_levels<3, 3, MAPPED, CALLERS>(p, s);
+    if (p.n_coords == 4 && p.n_bin_dim == 3) return launch_levels<4, 3, MAPPED, CALLERS>(p, s);
+    if (p.n_coords == 4 && p.n_bin_dim == 4) return launch_levels<4, 4, MAPPED, CALLERS>(p, s);
+    if (p.n_coords == 5 && p.n_bin_dim == 4) return launch_levels<5, 4, MAPPED, CALLERS>(p, s);
+    if (p.n_coords == 6 && p.n_bin_dim == 4) return launch_levels<6, 4, MAPPED, CALLERS>(p, s);
+    if (p.n_coords == 7 && p.n_bin_dim == 4) return launch_levels<7, 4, MAPPED, CALLERS>(p, s);
+    if (p.n_coords == 8 && p.n_bin_dim == 4) return launch_levels<8, 4, MAPPED, CALLERS>(p, s);
+    if (p.n_coords == 5 && p.n_bin_dim == 3) return launch_levels<5, 3, MAPPED, CALLERS>(p, s);
+    if (p.n_coords == 6 && p.n_bin_dim == 3) return launch_levels<6, 3, MAPPED, CALLERS>(p, s);
+    if (p.n_coords == 7 && p.n_bin_dim == 3) return launch_levels<7, 3, MAPPED, CALLERS>(p, s);
+    if (p.n_coords == 8 && p.n_bin_dim == 3) return launch_levels<8, 3, MAPPED, CALLERS>(p, s);
+    return launch_levels<0, 0, MAPPED, CALLERS>(p, s);
 }
 
 }  // namespace
@@ -1533,7 +1538,8 @@ int binned_select_knn_strided(const float *d_coord, const int *d_bin_idx, const 
     p.fine_min_population = fine_min_population;
     // the package's own tables are read with 32-bit byte offsets, and their bins per dimension are few
     callers_table = callers_table || n_bboundaries >= 1 << 30 || bins_bound > kNarrowGrid;
-    return d_sorting ? launch_coords<true>(p, callers_table, s) : launch_coords<false>(p, callers_table, s);
+    if (!d_sorting) return launch_coords<false, true>(p, s);  // (the package's own points come with a sorting)
+    return callers_table ? launch_coords<true, true>(p, s) : launch_coords<true, false>(p, s);
 }
 
 }  // namespace hgc

@@ -246,7 +246,7 @@ __device__ __forceinline__ float divide_no_nan(float a, float b) { return b == 0
 // Index and weight as loads of every lane (the same address for the lanes of a vertex) cost as much of the L1's address
 // rate as the gathers themselves: 40,000 vertices, K = 32, F = 8, C = 4 26 us for the means and 37 for the covariance
 // before, the whole call with its search 161 -> 141 us. What bounds them now (18 and 29 us) is the latency of the gathered
-// rows: 5000 waves are five per SIMD, a third to 44 % of their time is waiting, and vector issue is 47 and 59 % busy.
+// rows: 5000 waves are five per SIMD, a third to 44 % of their time is waiting, and vector issue is 45 and 56 % busy.
 // Workgroups of one XCD take consecutive vertices.
 constexpr int kMomentSlots = 4, kMomentWaves = 4;
 

@@ -190,3 +190,17 @@ def test_a_sorting_that_names_one_point_many_times(oracle, dims, K, again):
     once = np.flatnonzero(np.bincount(names, minlength=n)[names] == 1)  # the rows that one point writes
     assert (idx[names[once], 1:] == (key[once] & np.uint64(0xffffffff)).astype(np.int32)).all()
     assert (dist[names[once], 1:].view(np.uint32) == (key[once] >> np.uint64(32)).astype(np.uint32)).all()
+
+
+@pytest.mark.parametrize("dims", [2, 3, 4])
+@pytest.mark.parametrize("K", [6, 140])
+def test_the_largest_integer_as_a_bin_of_a_grid_that_divides_it(oracle, dims, K):
+    """its event would end exactly where the integers do; the other rows are those of another grid and left open"""
+    from hgcalml_amd import ops
+    binned = Binned(oracle, dims)
+    binned.n_bins = np.full(dims, 4, np.int32)
+    bad = torch.arange(len(binned.x)) % 11 == 0
+    binned.flat[bad.numpy()] = (1 << 31) - 1
+    idx, dist, flags = binned.search(K)
+    assert flags & ops.FLAG_BIN_BEYOND_TABLE
+    assert (idx[bad, 1:] == -1).all() and (dist[bad] == 0).all()
