@@ -10,6 +10,7 @@ and through the dense layers (torch).
 """
 import torch
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from . import globals as gl
 from . import ops
@@ -91,10 +92,27 @@ class _JoinFn(torch.autograd.Function):
         return tuple(g if want else None for g, want in zip(out, ctx.needs_input_grad))
 
 
+def _weight_and_bias_grad(g, x, want_bias):
+    """(g^T x, sum over the rows of g): gradients of a dense layer over very many rows. The product reduces over those
+    rows into a small matrix; as one GEMM it runs on a handful of workgroups (0.35-0.44 ms for 150k rows of 64-192
+    columns). The library's pass forms it together with the bias gradient; where that one is not taken, a batch of 64 row
+    slices is added up afterwards."""
+    if _weight_grad_in_one_pass(g, x):
+        return ops.dense_weight_grad(g, x)
+    n, s = x.shape[0], _TallLinearFn.SLICES
+    whole = n // s * s
+    if whole >= 64 * s:
+        grad_w = torch.bmm(g[:whole].view(s, -1, g.shape[1]).transpose(1, 2), x[:whole].view(s, -1, x.shape[1]))
+        grad_w = _sum_rows(grad_w)
+        if whole < n:
+            grad_w = grad_w + g[whole:].t() @ x[whole:]
+    else:
+        grad_w = g.t() @ x
+    return grad_w, _sum_rows(g) if want_bias else None
+
+
 class _TallLinearFn(torch.autograd.Function):
-    """y = x W^T + b for x of very many rows. The weight gradient g^T x reduces over those rows into a small matrix; as one
-    GEMM it runs on a handful of workgroups (0.35-0.44 ms for 150k rows of 64-192 columns). The library's pass forms it
-    together with the bias gradient; where that one is not taken, a batch of 64 row slices is added up afterwards."""
+    """y = x W^T + b for x of very many rows, see _weight_and_bias_grad"""
 
     SLICES = 64
 
@@ -109,24 +127,84 @@ class _TallLinearFn(torch.autograd.Function):
         x, weight = ctx.saved_tensors
         g = g.contiguous()
         grad_x = g @ weight if ctx.needs_input_grad[0] else None
-        grad_w = None
         want_b = ctx.has_bias and ctx.needs_input_grad[2]
-        if ctx.needs_input_grad[1] and _weight_grad_in_one_pass(g, x):
-            grad_w, grad_b = ops.dense_weight_grad(g, x)
-            return grad_x, grad_w, grad_b if want_b else None
-        if ctx.needs_input_grad[1]:
-            n, s = x.shape[0], _TallLinearFn.SLICES
-            whole = n // s * s
-            if whole >= 64 * s:
-                grad_w = torch.bmm(g[:whole].view(s, -1, g.shape[1]).transpose(1, 2),
-                                   x[:whole].view(s, -1, x.shape[1]))
-                grad_w = _sum_rows(grad_w)
-                if whole < n:
-                    grad_w = grad_w + g[whole:].t() @ x[whole:]
-            else:
-                grad_w = g.t() @ x
-        grad_b = _sum_rows(g) if want_b else None
-        return grad_x, grad_w, grad_b
+        if not ctx.needs_input_grad[1]:
+            return grad_x, None, _sum_rows(g) if want_b else None
+        grad_w, grad_b = _weight_and_bias_grad(g, x, want_b)
+        return grad_x, grad_w, grad_b if want_b else None
+
+
+class _InputLayersFn(torch.autograd.Function):
+    """The block's two layers on x. Features and x leave twice, the second time as tensors of their own on the same
+    memory, for the block's last layer: what comes back for them is added in the pass that forms the gradient of x."""
+
+    @staticmethod
+    def forward(ctx, x, w_features, bias, w_coords, relu):
+        ctx.set_materialize_grads(False)
+        features = ops.gravnet_feature_layer(x, w_features, bias, relu)
+        coords = torch.nn.functional.linear(x, w_coords)
+        ctx.save_for_backward(x, w_features, w_coords, features)
+        ctx.relu = relu
+        return features, coords, features.data, x.data
+
+    @staticmethod
+    def backward(ctx, g_features, g_coords, g_features2, g_x):
+        x, w_features, w_coords, features = ctx.saved_tensors
+        want_x, want_wf, want_b, want_wc, _ = ctx.needs_input_grad
+        if g_features is None:
+            g_features, g_features2 = g_features2, None
+        grad_x = masked = None
+        if want_x and g_features is not None and not torch.is_grad_enabled():
+            grad_x, masked = ops.gravnet_input_layers_grad(g_features, g_features2, features, g_coords, g_x, w_features, w_coords,
+                                                           ctx.relu)
+        else:  # as tensor operations: derivatives of the derivative, or no gradient of x
+            if g_features is not None:
+                masked = g_features if g_features2 is None else g_features + g_features2
+                if ctx.relu:
+                    masked = torch.ops.aten.threshold_backward(masked, features, 0)
+                masked = masked.contiguous()
+            if want_x:
+                parts = [g_x] + [g @ w for g, w in ((masked, w_features), (g_coords, w_coords)) if g is not None]
+                grad_x = sum(part for part in parts if part is not None) if any(part is not None for part in parts) else None
+        grad_wf = grad_b = grad_wc = None
+        if masked is not None and want_wf:
+            grad_wf, grad_b = _weight_and_bias_grad(masked, x, want_b)
+        elif masked is not None and want_b:
+            grad_b = _sum_rows(masked)
+        if g_coords is not None and want_wc:
+            grad_wc, _ = _weight_and_bias_grad(g_coords.contiguous(), x, False)
+        return grad_x, grad_wf, grad_b if want_b else None, grad_wc, None
+
+
+class _OutputLayerFn(torch.autograd.Function):
+    """relu of the block's last layer on joined = [accumulated - (features | features) | x], which the weight gradient
+    reads; its parts are kept for the derivative of that gradient"""
+
+    @staticmethod
+    def forward(ctx, accumulated, features, x, weight, bias, with_joined):
+        out, joined = ops.gravnet_output_layer(accumulated, features, x, weight, bias, with_joined)
+        ctx.save_for_backward(weight, joined, out, accumulated, features, x)
+        return out
+
+    @staticmethod
+    def backward(ctx, g):
+        weight, joined, out, accumulated, features, x = ctx.saved_tensors
+        f = features.shape[1]
+        want_w, want_b = ctx.needs_input_grad[3:5]
+        if torch.is_grad_enabled() or not any(ctx.needs_input_grad[:3]):
+            masked = torch.ops.aten.threshold_backward(g, out, 0).contiguous()
+            grad = masked @ weight
+            grads = grad[:, :2 * f], -grad[:, :f] - grad[:, f:2 * f], grad[:, 2 * f:]
+            if torch.is_grad_enabled() and want_w:
+                joined = torch.cat([accumulated - features.repeat(1, 2), x], dim=1)
+        else:
+            *grads, masked = ops.gravnet_output_layer_grad(g, out, weight, f)
+        grad_w = grad_b = None
+        if want_w:
+            grad_w, grad_b = _weight_and_bias_grad(masked, joined, want_b)
+        elif want_b:
+            grad_b = _sum_rows(masked)
+        return (*(t if want else None for t, want in zip(grads, ctx.needs_input_grad)), grad_w, grad_b if want_b else None, None)
 
 
 class TallLinear(nn.Linear):
@@ -141,6 +219,9 @@ class TallLinear(nn.Linear):
 
 _ACTIVATIONS = {None: nn.Identity, "linear": nn.Identity, "relu": nn.ReLU, "elu": nn.ELU, "tanh": nn.Tanh,
                 "sigmoid": nn.Sigmoid, "selu": nn.SELU, "gelu": nn.GELU}
+
+
+_REPLACEABLE = {"compute_neighbours_and_distancesq", "collect_neighbours", "create_output_features", "update_dynamic_radius"}
 
 
 class RaggedGravNet(nn.Module):
@@ -217,8 +298,43 @@ class RaggedGravNet(nn.Module):
             joined = torch.cat([features - prev_feat.repeat(1, 2), x], dim=-1)
         return torch.relu(self.output_feature_transform(joined))
 
+    def _layers_in_one_pass(self, x):
+        """Whether the dense layers run as the library's passes: the block as it is here, its layers and activation
+        without hooks or replacements, so that nobody waits for their calls, and tensors that the passes take."""
+        if type(self) is not RaggedGravNet or not self.__dict__.keys().isdisjoint(_REPLACEABLE) or not x.is_contiguous():
+            return False
+        first, spatial, last = self.input_feature_transform, self.input_spatial_transform, self.output_feature_transform
+        if type(self.feature_activation) not in (nn.ReLU, nn.Identity) or _has_any_global_hook():
+            return False
+        for module in (first, spatial, last, self.feature_activation):
+            if (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks or
+                    "forward" in module.__dict__):
+                return False
+        if not all(type(layer) is TallLinear for layer in (first, spatial, last)):
+            return False
+        weights = first.weight, first.bias, spatial.weight, last.weight, last.bias
+        if any(w is None for w in weights) or spatial.bias is not None or not _library_takes(x, *weights):
+            return False
+        if not all(w.is_contiguous() for w in weights):
+            return False
+        f, i, o, c = first.weight.shape[0], x.shape[1], last.weight.shape[0], spatial.weight.shape[0]
+        if first.weight.shape[1] != i or spatial.weight.shape[1] != i or last.weight.shape[1] != 2 * f + i:
+            return False  # (the layers themselves say what is wrong)
+        return not (torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or x.shape[0] >= 1 << 31) and bool(
+            ops.lib.hgc_gravnet_dense_covers(f, i, o, c))
+
     def forward(self, x, row_splits):
         assert x.dim() == 2 and row_splits.dim() == 1
+        if self._layers_in_one_pass(x):
+            features, coordinates, features_again, x_again = _InputLayersFn.apply(
+                x, self.input_feature_transform.weight, self.input_feature_transform.bias, self.input_spatial_transform.weight,
+                type(self.feature_activation) is nn.ReLU)
+            nidx, ndist, sidx, sdist = self.compute_neighbours_and_distancesq(coordinates, row_splits)
+            accumulated = self.collect_neighbours(features, nidx, ndist)
+            last = self.output_feature_transform
+            outfeats = _OutputLayerFn.apply(accumulated, features_again, x_again, last.weight, last.bias,
+                                            torch.is_grad_enabled() and last.weight.requires_grad)
+            return (outfeats, coordinates, sidx, sdist) if self.return_self else (outfeats, coordinates, nidx, ndist)
         coordinates = self.input_spatial_transform(x)
         neighbour_indices, distancesq, sidx, sdist = self.compute_neighbours_and_distancesq(coordinates, row_splits)
         outfeats = self.create_output_features(x, neighbour_indices, distancesq)

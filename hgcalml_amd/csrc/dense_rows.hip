@@ -1,0 +1,488 @@
+// The dense layers of the GravNet block, rows in and rows out, with what stands around them in the same pass:
+//   input form        features = act(x Wf^T + b); the coordinates x Ws^T stay a library product, since their last bits decide
+//                     between neighbours at nearly equal distances
+//   output form       y = relu([mean - p | max - p | x] W^T + b), the joined rows kept for the weights' gradient on request
+//   output's gradient g where y > 0 times W: to the accumulation's rows, to p (minus both halves) and to x; the masked g kept
+//   input's gradient  (g1 + g2 where the features are > 0) Wf + g_coordinates Ws + g_x; the masked sum kept
+//
+// A contraction over at most a few hundred columns, for very many rows. Its bound is the float32 matrix instruction
+// (150,000 rows, 192 -> 128: 7.4 GFLOP, 47 us at its rate) or, for narrow layers, reading and writing the rows once.
+// The weights of a workgroup's columns lie in LDS for its whole life, in the order in which the instruction takes them (a
+// step of 16 columns of the input times 16 of the output is 64 lanes x 16 bytes, without bank conflicts), so nothing but
+// the first barrier keeps its waves together: each takes 16 rows at a time, streams them from memory with one batch of
+// steps requested ahead and has all output columns of the workgroup in registers. 16 rows a wave: many short tasks fill the
+// four SIMDs of 256 CUs evenly (9375 tasks for 150,000 rows).
+// Rows go in as the instruction's second operand, so that a lane holds four consecutive columns of one row in the end and
+// stores 16 bytes. At the end of a width that is no multiple of four a lane moves back onto the row's last four columns
+// (the ones it has twice count once), and behind the last row stands the last row again: no load or store is left out, so
+// none stands in a branch, which would make waiting for a load mean waiting for everything after it.
+// Measured next to the library products with join, activation, mask and sums as passes of their own, us: 150,000 rows, 64 inputs,
+// 64 features, 128 outputs: features 41 -> 21, output 156 -> 100, its gradient 171 -> 89, input's gradient 123 -> 40; 240,011 rows,
+// 48, 32, 96: 50 -> 16, 162 -> 73, 220 -> 83, 155 -> 36; a training step of the block 1976 -> 1741 and 2000 -> 1680, 2477
+// points 790 -> 594 (the host's time). What is left: the matrix instruction (61 % busy at 128 outputs) and the memory (the output layer without
+// its products 94). Error against 64 bits (2-norm, 150,000 rows): output 1.0e-7, library 1.5e-7. Tried and taken back: 8 waves
+// instead of 16 (output 108), weights' tiles multiplied onto the sum over all columns (error 2.1e-7), higher priority
+// while multiplying (level), whole ranges of rows per workgroup or XCD (108 to 127).
+#include <algorithm>
+
+#include "hgc_common.hpp"
+
+namespace hgc {
+namespace {
+
+constexpr int kTile = 16, kStepCols = 16;
+constexpr int kGroups = 256;               // workgroups at the most, one per CU
+constexpr int kLdsBytes = 160 * 1024;
+constexpr int kMostTiles = 12;             // of 16 output columns, in a wave's registers
+
+typedef float vec4 __attribute__((ext_vector_type(4)));
+
+enum class Form { Input, Output, OutputGrad, InputGrad };
+
+struct DenseRows {
+    const float *a0, *a1, *a2, *a3, *add;  // rows in
+    const float *w0, *w1, *bias;
+    float *o0, *o1, *o2, *side;            // rows out; side (may be null): the operand as it was multiplied
+    long long n;
+    int F, I, O, C;
+    int steps, steps0, steps1;             // of 16 input columns: all, up to the end of the first and of the second part
+    int tiles;                             // of 16 output columns, all of them
+    int relu, two;
+};
+
+__device__ __forceinline__ vec4 load4(const float *p) {
+    vec4 v;
+    __builtin_memcpy(&v, p, sizeof(v));
+    return v;
+}
+
+// Past the caches: what is written here is read by other kernels, after more than the L2 holds. (150,000 rows, output layer
+// 109 -> 99 us, its gradient 112 -> 87; 240,011 rows, 96 of 112 columns: 107 -> 74 and 116 -> 83)
+__device__ __forceinline__ void store4(float *p, const vec4 &v) {
+    typedef vec4 vec4_any __attribute__((aligned(4)));
+    __builtin_nontemporal_store(v, reinterpret_cast<vec4_any *>(p));
+}
+
+// the derivative of max(y, 0): NaN stays, as in torch
+__device__ __forceinline__ float where_positive(float g, float y) { return y <= 0.f ? 0.f : g; }
+
+// Four columns in sequence of a row of `width` >= 4, wanted from col on: the last ones move back onto the row's end.
+// Columns in front of `col` are then held twice.
+__device__ __forceinline__ int first_of_four(int col, int width) { return min(col, width - 4); }
+
+struct Part {  // of the input's columns
+    int index, col, width;
+};
+
+template <Form FORM>
+__device__ __forceinline__ Part part_of(const DenseRows &p, int step) {
+    if constexpr (FORM == Form::Input) return {0, step * kStepCols, p.I};
+    if constexpr (FORM == Form::OutputGrad) return {0, step * kStepCols, p.O};
+    if constexpr (FORM == Form::InputGrad) return {0, step * kStepCols, p.F};
+    const int index = step < p.steps0 ? 0 : step < p.steps1 ? 1 : 2;
+    const int before = index == 0 ? 0 : index == 1 ? p.steps0 : p.steps1;
+    return {index, (step - before) * kStepCols, index < 2 ? p.F : p.I};
+}
+
+// first weight of output column c of tile `tile` and the distance of its weights for consecutive input columns
+template <Form FORM>
+__device__ __forceinline__ const float *weights_of(const DenseRows &p, const Part &at, int tile, int c, size_t &pitch) {
+    const int tiles_f = (p.F + kTile - 1) / kTile;
+    auto column = [&](int tile, int width) { return first_of_four(tile * kTile + (c & ~3), width) + (c & 3); };
+    pitch = 1;
+    if constexpr (FORM == Form::Input) {
+        return p.w0 + (size_t)column(tile, p.F) * p.I;
+    } else if constexpr (FORM == Form::Output) {
+        return p.w0 + (size_t)column(tile, p.O) * (2 * p.F + p.I) + at.index * p.F;
+    } else if constexpr (FORM == Form::OutputGrad) {  // tiles of both halves in turn, then those of x
+        pitch = 2 * p.F + p.I;
+        return tile < 2 * tiles_f ? p.w0 + (tile & 1) * p.F + column(tile >> 1, p.F) : p.w0 + 2 * p.F + column(tile - 2 * tiles_f, p.I);
+    } else {
+        pitch = p.I;
+        return p.w0 + column(tile, p.I);
+    }
+}
+
+constexpr int sources(Form form) { return form == Form::Input ? 1 : form == Form::InputGrad ? 3 : 2; }
+
+template <int NSRC>
+struct Raw {
+    vec4 v[NSRC];
+};
+
+// Steps requested while as many are multiplied: 64 columns where few tiles leave little work for a step, 32 otherwise.
+constexpr int steps_ahead(Form form, int tiles) {
+    return tiles <= 4 && sources(form) == 1 ? 4 : tiles >= 6 && sources(form) == 3 ? 1 : 2;
+}
+// 16 waves of 128 registers, or 12 of 168 for many tiles
+constexpr int most_waves(int tiles) { return tiles <= 8 ? 16 : 12; }
+
+// SIDE: the operand is kept. COORDS: the gradient of the coordinates takes part (at most four of them: one more step of the
+// instruction).
+template <Form FORM, int NT, bool SIDE, bool COORDS>
+__global__ __launch_bounds__(most_waves(NT) *kWave) void dense_rows_kernel(const DenseRows p) {
+    constexpr int NSRC = sources(FORM), U = steps_ahead(FORM, NT);
+    extern __shared__ __align__(16) float s_weights[];
+    vec4 *const s_w = reinterpret_cast<vec4 *>(s_weights);
+    float *const s_bias = s_weights + (size_t)p.steps * NT * kWave * 4;  // or the weights of the coordinates
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id(), l = lane & 15, k = lane >> 4;
+    const int waves = blockDim.x / kWave, tile0 = blockIdx.y * NT;
+    const int tiles_f = (p.F + kTile - 1) / kTile;
+
+    // lane: output column l of the tile, four input columns of group k of the step; columns held twice count once
+    constexpr int kAtOnce = 4;
+    const int pieces = p.steps * NT;
+    for (int first = wave * kAtOnce; first < pieces; first += waves * kAtOnce) {
+        vec4 w[kAtOnce];
+#pragma unroll
+        for (int u = 0; u < kAtOnce; ++u) {
+            const int i = min(first + u, pieces - 1), step = i / NT;
+            const Part at = part_of<FORM>(p, step);
+            const int wanted = at.col + 4 * k, col = first_of_four(wanted, at.width);
+            size_t pitch;
+            const float *from = weights_of<FORM>(p, at, min(tile0 + i - step * NT, p.tiles - 1), l, pitch);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[u][e] = from[(col + e) * pitch];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[u][e] = col + e < wanted ? 0.f : w[u][e];
+        }
+#pragma unroll
+        for (int u = 0; u < kAtOnce; ++u)
+            if (first + u < pieces) s_w[(size_t)(first + u) * kWave + lane] = w[u];
+    }
+    if constexpr (FORM == Form::Input || FORM == Form::Output) {
+        const int width = FORM == Form::Input ? p.F : p.O;
+        for (int i = threadIdx.x; i < NT * kTile; i += blockDim.x)
+            s_bias[i] = p.bias[first_of_four(min(tile0 + i / kTile, p.tiles - 1) * kTile + (i & 12), width) + (i & 3)];
+    }
+    if constexpr (COORDS) {  // lane: output column l, coordinate k
+        for (int i = threadIdx.x; i < NT * kWave; i += blockDim.x) {
+            const int c = i & 15, coord = (i >> 4) & 3;
+            const int col = first_of_four(min(tile0 + i / kWave, p.tiles - 1) * kTile + (c & ~3), p.I) + (c & 3);
+            s_bias[i] = coord < p.C ? p.w1[(size_t)coord * p.I + col] : 0.f;
+        }
+    }
+    __syncthreads();
+
+    const long long tasks = (p.n + kTile - 1) / kTile, stride = (long long)waves * gridDim.x;
+    long long task = (long long)wave * gridDim.x + blockIdx.x;
+    if (task >= tasks) return;
+    const int batches = (p.steps + U - 1) / U;
+
+    // Rows behind the last one are the last one again, which is then written several times with the same values: loads and
+    // stores stand in no branch, so that waiting for a load never means waiting for what was asked for after it.
+    auto row_in = [&](long long task) { return (int)min((long long)l, p.n - 1 - task * kTile); };
+    auto request = [&](Raw<NSRC> (&raw)[U], float &coord, long long task, int batch) {
+        task = min(task, tasks - 1);
+        const unsigned row = row_in(task);
+        // (a base that is the same for all lanes and an offset of 32 bits)
+        auto at = [&](const float *from, int pitch, int first) { return from + task * kTile * pitch + (row * (unsigned)pitch + first); };
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const Part part = part_of<FORM>(p, min(batch * U + u, p.steps - 1));
+            const int col = first_of_four(part.col + 4 * k, part.width);
+            if constexpr (FORM == Form::Input) {
+                raw[u].v[0] = load4(at(p.a0, p.I, col));
+            } else if constexpr (FORM == Form::Output) {
+                const bool own = part.index < 2;
+                raw[u].v[0] = load4(at(own ? p.a0 + part.index * p.F : p.a2, own ? 2 * p.F : p.I, col));
+                raw[u].v[1] = load4(at(own ? p.a1 : p.a2, own ? p.F : p.I, col));
+            } else if constexpr (FORM == Form::OutputGrad) {
+                raw[u].v[0] = load4(at(p.a0, p.O, col));
+                raw[u].v[1] = load4(at(p.a1, p.O, col));
+            } else {
+                raw[u].v[0] = load4(at(p.a0, p.F, col));
+                raw[u].v[1] = load4(at(p.a1, p.F, col));
+                raw[u].v[2] = load4(at(p.a2, p.F, col));
+            }
+        }
+        if constexpr (COORDS) coord = *at(p.a3, p.C, min(k, p.C - 1));
+        __builtin_amdgcn_sched_barrier(0);  // before what is multiplied meanwhile
+    };
+
+    vec4 acc[NT];
+    auto clear = [&]() {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[t] = vec4{0.f, 0.f, 0.f, 0.f};
+    };
+    auto multiply = [&](const Raw<NSRC> (&raw)[U], long long task, int batch) {
+        const unsigned row = row_in(task);
+        const int here = min(U, p.steps - batch * U);
+        vec4 a[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const Part part = part_of<FORM>(p, min(batch * U + u, p.steps - 1));
+            const int wanted = part.col + 4 * k, col = first_of_four(wanted, part.width);
+            a[u] = raw[u].v[0];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (FORM == Form::Output) a[u][e] = part.index < 2 ? a[u][e] - raw[u].v[1][e] : a[u][e];
+                if constexpr (FORM == Form::OutputGrad) a[u][e] = where_positive(a[u][e], raw[u].v[1][e]);
+                if constexpr (FORM == Form::InputGrad) {
+                    a[u][e] = p.two ? a[u][e] + raw[u].v[1][e] : a[u][e];
+                    a[u][e] = p.relu ? where_positive(a[u][e], raw[u].v[2][e]) : a[u][e];
+                }
+            }
+            if constexpr (SIDE) {
+                const int pitch = FORM == Form::Output ? 2 * p.F + p.I : FORM == Form::OutputGrad ? p.O : p.F;
+                const int first = FORM == Form::Output ? part.index * p.F : 0;
+                if (tile0 == 0) store4(p.side + task * kTile * pitch + (row * (unsigned)pitch + first + col), a[u]);
+            }
+            if (part.col + kStepCols > part.width) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a[u][e] = col + e < wanted ? 0.f : a[u][e];
+            }
+        }
+        // The sum over two steps first, then onto the others: less rounding than one chain over all columns.
+#pragma unroll
+        for (int u0 = 0; u0 < U; u0 += 2) {
+            if (u0 > 0 && u0 >= here) break;
+#pragma unroll
+            for (int t0 = 0; t0 < NT; t0 += 4) {
+                constexpr int kMost = 4;
+                vec4 sum[kMost];
+#pragma unroll
+                for (int t = 0; t < kMost; ++t) sum[t] = vec4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int u = u0; u < u0 + 2 && u < U; ++u) {
+                    if (u > u0 && u >= here) break;
+                    vec4 w[kMost];
+#pragma unroll
+                    for (int t = 0; t < kMost && t0 + t < NT; ++t) w[t] = s_w[((batch * U + u) * NT + t0 + t) * kWave + lane];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+#pragma unroll
+                        for (int t = 0; t < kMost && t0 + t < NT; ++t)
+                            sum[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t][e], a[u][e], sum[t], 0, 0, 0);
+                }
+#pragma unroll
+                for (int t = 0; t < kMost && t0 + t < NT; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[t0 + t][e] = acc[t0 + t][e] + sum[t][e];
+            }
+        }
+    };
+    // lane: columns 4 k .. 4 k + 3 of every tile of row l
+    auto finish = [&](long long task, float coord) {
+        const long long row = task * kTile + row_in(task);
+        if constexpr (COORDS) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(s_bias[t * kWave + lane], k < p.C ? coord : 0.f, acc[t], 0, 0, 0);
+        }
+        auto with_bias = [&](int t) {
+            vec4 v = acc[t];
+            const vec4 b = *reinterpret_cast<const vec4 *>(s_bias + t * kTile + 4 * k);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                v[e] = v[e] + b[e];
+                v[e] = p.relu ? where_positive(v[e], v[e]) : v[e];
+            }
+            return v;
+        };
+        auto column = [&](int tile, int width) { return first_of_four(tile * kTile + 4 * k, width); };
+        if constexpr (FORM == Form::InputGrad) {
+            if (p.add) {
+#pragma unroll
+                for (int t0 = 0; t0 < NT; t0 += 4) {
+                    vec4 more[4];
+#pragma unroll
+                    for (int t = 0; t < 4 && t0 + t < NT; ++t)
+                        more[t] = load4(p.add + row * p.I + column(min(tile0 + t0 + t, p.tiles - 1), p.I));
+#pragma unroll
+                    for (int t = 0; t < 4 && t0 + t < NT; ++t)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[t0 + t][e] = acc[t0 + t][e] + more[t][e];
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            // (behind the last tile: that one again, weights and all)
+            const int tile = min(tile0 + t, p.tiles - 1);
+            if constexpr (FORM == Form::Input) {
+                store4(p.o0 + row * p.F + column(tile, p.F), with_bias(t));
+            } else if constexpr (FORM == Form::Output) {
+                store4(p.o0 + row * p.O + column(tile, p.O), with_bias(t));
+            } else if constexpr (FORM == Form::OutputGrad) {
+                if (tile0 + t < 2 * tiles_f) {
+                    if (t % 2 == 0) {
+                        const int col = column(tile >> 1, p.F);
+                        const vec4 &mean = acc[t], &max = acc[t + 1 < NT ? t + 1 : t];
+                        store4(p.o0 + row * 2 * p.F + col, mean);
+                        store4(p.o0 + (row * 2 + 1) * p.F + col, max);
+                        vec4 v;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] = -mean[e] - max[e];
+                        store4(p.o1 + row * p.F + col, v);
+                    }
+                } else {
+                    store4(p.o2 + row * p.I + column(tile - 2 * tiles_f, p.I), acc[t]);
+                }
+            } else {
+                store4(p.o0 + row * p.I + column(tile, p.I), acc[t]);
+            }
+        }
+    };
+
+    Raw<NSRC> now[U], ahead[U];
+    float coord_now = 0.f, coord_ahead = 0.f;
+    request(ahead, coord_ahead, task, 0);
+    for (int batch = 0;;) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) now[u] = ahead[u];
+        coord_now = coord_ahead;
+        const bool last = batch + 1 == batches;
+        const long long next_task = last ? task + stride : task;
+        const int next = last ? 0 : batch + 1;
+        request(ahead, coord_ahead, next_task, next);  // (behind the last task: its last row once more)
+        if (batch == 0) clear();
+        multiply(now, task, batch);
+        if (last) finish(task, coord_now);
+        if (next_task >= tasks) break;
+        task = next_task;
+        batch = next;
+    }
+}
+
+struct Plan {
+    int tiles, chunks;  // tiles of a workgroup, workgroups along the output's columns
+    size_t lds;
+};
+
+// Tiles of a workgroup: all output columns where registers and LDS hold them, otherwise equal shares.
+bool make_plan(Form form, int steps, int tiles, bool coords, Plan &plan) {
+    constexpr int offered[] = {1, 2, 3, 4, 5, 6, 8, 10, 12};
+    const bool pairs = form == Form::OutputGrad;
+    for (int chunks = 1; chunks <= tiles; ++chunks) {
+        const int share = (tiles + chunks - 1) / chunks;
+        for (int nt : offered) {
+            if (nt < share || (pairs && nt % 2)) continue;
+            const size_t lds = (size_t)steps * nt * kWave * sizeof(vec4) + nt * (coords ? kWave : kTile) * sizeof(float);
+            if (lds > kLdsBytes) break;
+            plan.tiles = nt;
+            plan.chunks = (tiles + nt - 1) / nt;
+            plan.lds = lds;
+            return true;
+        }
+    }
+    return false;
+}
+
+template <Form FORM, int NT, bool SIDE, bool COORDS>
+int launch_kernel(const DenseRows &p, const Plan &plan, hipStream_t s) {
+    const long long tasks = (p.n + kTile - 1) / kTile;
+    const int groups = (int)std::min<long long>(tasks, std::max(1, kGroups / plan.chunks));
+    const long long each = (tasks + groups - 1) / groups;
+    const int waves = (int)std::min<long long>(most_waves(NT), (each + 3) / 4 * 4);
+    if (plan.lds > 64 * 1024) {
+        HGC_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&dense_rows_kernel<FORM, NT, SIDE, COORDS>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));
+    }
+    dense_rows_kernel<FORM, NT, SIDE, COORDS><<<dim3(groups, plan.chunks), waves * kWave, plan.lds, s>>>(p);
+    return check_launch("dense_rows_kernel");
+}
+
+template <Form FORM, bool SIDE, bool COORDS>
+int launch(DenseRows p, int tiles, hipStream_t s) {
+    constexpr bool kPairs = FORM == Form::OutputGrad;
+    Plan plan;
+    p.tiles = tiles;
+    if (!make_plan(FORM, p.steps, tiles, COORDS, plan)) return fail(HGC_ERR_INVALID_ARGUMENT, "layer too wide");
+    switch (plan.tiles) {
+        case 1: if constexpr (!kPairs) return launch_kernel<FORM, 1, SIDE, COORDS>(p, plan, s); break;
+        case 2: return launch_kernel<FORM, 2, SIDE, COORDS>(p, plan, s);
+        case 3: if constexpr (!kPairs) return launch_kernel<FORM, 3, SIDE, COORDS>(p, plan, s); break;
+        case 4: return launch_kernel<FORM, 4, SIDE, COORDS>(p, plan, s);
+        case 5: if constexpr (!kPairs) return launch_kernel<FORM, 5, SIDE, COORDS>(p, plan, s); break;
+        case 6: return launch_kernel<FORM, 6, SIDE, COORDS>(p, plan, s);
+        case 8: return launch_kernel<FORM, 8, SIDE, COORDS>(p, plan, s);
+        case 10: return launch_kernel<FORM, 10, SIDE, COORDS>(p, plan, s);
+        case 12: return launch_kernel<FORM, 12, SIDE, COORDS>(p, plan, s);
+    }
+    return fail(HGC_ERR_INVALID_ARGUMENT, "no kernel for this number of tiles");
+}
+
+int steps_of(int width) { return ceil_div(width, kStepCols); }
+int tiles_of(int width) { return ceil_div(width, kTile); }
+
+// Rows of four columns and more, so that four in sequence exist; up to four coordinates, one step of the instruction. Wider
+// layers are the library product's, whose workgroups share what they read of the weights (240,000 rows, 352 -> 512 with
+// everything around it 1264 here, 983 there; 60,000 rows, 384 -> 256 170 and 154, the four passes of the block together
+// 368 and 463).
+constexpr int kWidestIn = 512, kWidestOut = 256;
+
+bool widths_fit(int f, int x, int o, int c) {
+    return f >= 4 && x >= 4 && o >= 4 && c >= 1 && f <= kWidestIn && x <= kWidestIn && 2 * f + x <= kWidestIn && o <= kWidestOut &&
+           c <= 4;
+}
+
+}  // namespace
+}  // namespace hgc
+
+using namespace hgc;
+
+extern "C" {
+
+int hgc_gravnet_dense_covers(int n_feat, int n_x, int n_out, int n_coords) {
+    return widths_fit(n_feat, n_x, n_out, n_coords);
+}
+
+int hgc_gravnet_feature_layer(const float *d_x, int n_vert, int n_x, const float *d_w, const float *d_bias, int n_feat,
+                              int relu, float *d_features, hgc_stream_t stream) {
+    HGC_REQUIRE(n_vert >= 0 && widths_fit(n_feat, n_x, 4, 1), "bad sizes");
+    if (n_vert == 0) return HGC_OK;
+    HGC_REQUIRE(d_x && d_w && d_bias && d_features, "null pointer");
+    DenseRows p{};
+    p.a0 = d_x, p.w0 = d_w, p.bias = d_bias, p.o0 = d_features;
+    p.n = n_vert, p.F = n_feat, p.I = n_x, p.relu = relu;
+    p.steps = steps_of(n_x);
+    return launch<Form::Input, false, false>(p, tiles_of(n_feat), as_stream(stream));
+}
+
+int hgc_gravnet_output_layer(const float *d_acc, const float *d_features, const float *d_x, int n_vert, int n_feat, int n_x,
+                             const float *d_w, const float *d_bias, int n_out, float *d_out, float *d_joined,
+                             hgc_stream_t stream) {
+    HGC_REQUIRE(n_vert >= 0 && widths_fit(n_feat, n_x, n_out, 1), "bad sizes");
+    if (n_vert == 0) return HGC_OK;
+    HGC_REQUIRE(d_acc && d_features && d_x && d_w && d_bias && d_out, "null pointer");
+    DenseRows p{};
+    p.a0 = d_acc, p.a1 = d_features, p.a2 = d_x, p.w0 = d_w, p.bias = d_bias, p.o0 = d_out, p.side = d_joined;
+    p.n = n_vert, p.F = n_feat, p.I = n_x, p.O = n_out, p.relu = 1;
+    p.steps0 = steps_of(n_feat), p.steps1 = 2 * p.steps0, p.steps = p.steps1 + steps_of(n_x);
+    return d_joined ? launch<Form::Output, true, false>(p, tiles_of(n_out), as_stream(stream))
+                    : launch<Form::Output, false, false>(p, tiles_of(n_out), as_stream(stream));
+}
+
+int hgc_gravnet_output_layer_grad(const float *d_grad, const float *d_out, int n_vert, int n_feat, int n_x, const float *d_w,
+                                  int n_out, float *d_masked, float *d_grad_acc, float *d_grad_features, float *d_grad_x,
+                                  hgc_stream_t stream) {
+    HGC_REQUIRE(n_vert >= 0 && widths_fit(n_feat, n_x, n_out, 1), "bad sizes");
+    if (n_vert == 0) return HGC_OK;
+    HGC_REQUIRE(d_grad && d_out && d_w && d_masked && d_grad_acc && d_grad_features && d_grad_x, "null pointer");
+    DenseRows p{};
+    p.a0 = d_grad, p.a1 = d_out, p.w0 = d_w, p.side = d_masked, p.o0 = d_grad_acc, p.o1 = d_grad_features, p.o2 = d_grad_x;
+    p.n = n_vert, p.F = n_feat, p.I = n_x, p.O = n_out, p.relu = 1;
+    p.steps = steps_of(n_out);
+    return launch<Form::OutputGrad, true, false>(p, 2 * tiles_of(n_feat) + tiles_of(n_x), as_stream(stream));
+}
+
+int hgc_gravnet_input_layers_grad(const float *d_grad_features, const float *d_grad_features2, const float *d_features,
+                                  const float *d_grad_coords, const float *d_grad_x, int n_vert, int n_x,
+                                  const float *d_w_feat, int n_feat, const float *d_w_coords, int n_coords, int relu,
+                                  float *d_masked, float *d_grad_in, hgc_stream_t stream) {
+    HGC_REQUIRE(n_vert >= 0 && widths_fit(n_feat, n_x, 4, n_coords), "bad sizes");
+    if (n_vert == 0) return HGC_OK;
+    HGC_REQUIRE(d_grad_features && (d_features || !relu) && d_w_feat && (d_w_coords || !d_grad_coords) && d_masked && d_grad_in,
+                "null pointer");
+    DenseRows p{};
+    p.a0 = d_grad_features, p.a1 = d_grad_features2 ? d_grad_features2 : d_grad_features, p.a2 = relu ? d_features : d_grad_features;
+    p.a3 = d_grad_coords, p.add = d_grad_x, p.two = d_grad_features2 != nullptr;
+    p.w0 = d_w_feat, p.w1 = d_w_coords, p.side = d_masked, p.o0 = d_grad_in;
+    p.n = n_vert, p.F = n_feat, p.I = n_x, p.C = n_coords, p.relu = relu;
+    p.steps = steps_of(n_feat);
+    return d_grad_coords ? launch<Form::InputGrad, true, true>(p, tiles_of(n_x), as_stream(stream))
+                         : launch<Form::InputGrad, true, false>(p, tiles_of(n_x), as_stream(stream));
+}
+
+}  // extern "C"

@@ -833,6 +833,68 @@ def dense_weight_grad(grad, x):
     return weight, bias
 
 
+@_op("gravnet_feature_layer(Tensor x, Tensor weight, Tensor bias, bool relu) -> Tensor")
+def gravnet_feature_layer(x, weight, bias, relu):
+    """x W^T + b, with relu the relu of it: the features [N, F] that the block propagates"""
+    dev = require_device(x, weight, bias)
+    x, w, b = f32(x), f32(weight), f32(bias)
+    (n, i), f = x.shape, w.shape[0]
+    if w.shape != (f, i) or b.shape != (f,):
+        raise ValueError("gravnet_feature_layer: x [N, X], a weight [F, X] and a bias [F] expected")
+    features = torch.empty((n, f), dtype=torch.float32, device=dev)
+    check(lib.hgc_gravnet_feature_layer(p(x), n, i, p(w), p(b), f, int(relu), p(features), stream()))
+    return features
+
+
+@_op("gravnet_input_layers_grad(Tensor grad_features, Tensor? grad_features2, Tensor features, Tensor? grad_coords, "
+     "Tensor? grad_x, Tensor w_features, Tensor w_coords, bool relu) -> (Tensor, Tensor)")
+def gravnet_input_layers_grad(grad_features, grad_features2, features, grad_coords, grad_x, w_features, w_coords, relu):
+    """(gradient w.r.t. x with grad_x added, gradient w.r.t. the features in front of their activation)"""
+    dev = require_device(grad_features, grad_features2, features, grad_coords, grad_x, w_features, w_coords)
+    g1, feat, wf, wc = f32(grad_features), f32(features), f32(w_features), f32(w_coords)
+    g2, gc, gx = (None if t is None else f32(t) for t in (grad_features2, grad_coords, grad_x))
+    (f, i), c, n = wf.shape, wc.shape[0], feat.shape[0]
+    if (g1.shape != (n, f) or feat.shape != (n, f) or wc.shape != (c, i) or (g2 is not None and g2.shape != (n, f)) or
+            (gc is not None and gc.shape != (n, c)) or (gx is not None and gx.shape != (n, i))):
+        raise ValueError("gravnet_input_layers_grad: gradients [N, F], [N, C] and [N, X] expected")
+    grad_in = torch.empty((n, i), dtype=torch.float32, device=dev)
+    masked = torch.empty((n, f), dtype=torch.float32, device=dev)
+    check(lib.hgc_gravnet_input_layers_grad(p(g1), p(g2), p(feat), p(gc), p(gx), n, i, p(wf), f, p(wc), c, int(relu), p(masked),
+                                            p(grad_in), stream()))
+    return grad_in, masked
+
+
+@_op("gravnet_output_layer(Tensor accumulated, Tensor features, Tensor x, Tensor weight, Tensor bias, bool with_joined) "
+     "-> (Tensor, Tensor)")
+def gravnet_output_layer(accumulated, features, x, weight, bias, with_joined):
+    """(relu(joined W^T + b), joined = gravnet_join(accumulated, features, x) if asked for, else empty)"""
+    dev = require_device(accumulated, features, x, weight, bias)
+    acc, feat, x, w, b = f32(accumulated), f32(features), f32(x), f32(weight), f32(bias)
+    n, f = feat.shape
+    i, o = x.shape[1], w.shape[0]
+    if acc.shape != (n, 2 * f) or x.shape != (n, i) or w.shape != (o, 2 * f + i) or b.shape != (o,):
+        raise ValueError("gravnet_output_layer: [N, 2F], [N, F], [N, X], a weight [O, 2F + X] and a bias [O] expected")
+    out = torch.empty((n, o), dtype=torch.float32, device=dev)
+    joined = torch.empty((n, 2 * f + i) if with_joined else (0,), dtype=torch.float32, device=dev)
+    check(lib.hgc_gravnet_output_layer(p(acc), p(feat), p(x), n, f, i, p(w), p(b), o, p(out), p(joined) if with_joined else None,
+                                       stream()))
+    return out, joined
+
+
+@_op("gravnet_output_layer_grad(Tensor grad, Tensor out, Tensor weight, int n_features) -> (Tensor, Tensor, Tensor, Tensor)")
+def gravnet_output_layer_grad(grad, out, weight, n_features):
+    """gradients w.r.t. accumulated [N, 2F], features [N, F] and x [N, X] of gravnet_output_layer, and the gradient in
+    front of its activation [N, O]"""
+    dev = require_device(grad, out, weight)
+    g, y, w = f32(grad), f32(out), f32(weight)
+    (n, o), f, i = y.shape, n_features, w.shape[1] - 2 * n_features
+    if g.shape != y.shape or w.shape[0] != o or f < 1 or i < 1:
+        raise ValueError("gravnet_output_layer_grad: gradient and result [N, O] and a weight [O, 2F + X] expected")
+    masked, g_acc, g_feat, g_x = (torch.empty((n, width), dtype=torch.float32, device=dev) for width in (o, 2 * f, f, i))
+    check(lib.hgc_gravnet_output_layer_grad(p(g), p(y), n, f, i, p(w), o, p(masked), p(g_acc), p(g_feat), p(g_x), stream()))
+    return g_acc, g_feat, g_x, masked
+
+
 # --------------------------------------------------------------------------- shapes without data
 
 # Fake ("meta") implementations: output shapes and dtypes from input shapes alone, so that
@@ -992,3 +1054,26 @@ def _(grad, normalised, norm, n_neighbours):
 @torch.library.register_fake("hgcalml::sumw_distance_grad")
 def _(norm_grad, weights, indices, distance_grad):
     return None
+
+
+@torch.library.register_fake("hgcalml::gravnet_feature_layer")
+def _(x, weight, bias, relu):
+    return _f32_like((x.shape[0], weight.shape[0]), x)
+
+
+@torch.library.register_fake("hgcalml::gravnet_input_layers_grad")
+def _(grad_features, grad_features2, features, grad_coords, grad_x, w_features, w_coords, relu):
+    return _f32_like((features.shape[0], w_features.shape[1]), features), _f32_like(features.shape, features)
+
+
+@torch.library.register_fake("hgcalml::gravnet_output_layer")
+def _(accumulated, features, x, weight, bias, with_joined):
+    n = x.shape[0]
+    return _f32_like((n, weight.shape[0]), x), _f32_like((n, weight.shape[1]) if with_joined else (0,), x)
+
+
+@torch.library.register_fake("hgcalml::gravnet_output_layer_grad")
+def _(grad, out, weight, n_features):
+    n = grad.shape[0]
+    widths = 2 * n_features, n_features, weight.shape[1] - 2 * n_features, weight.shape[0]
+    return tuple(_f32_like((n, width), grad) for width in widths)

@@ -1,0 +1,166 @@
+"""The GravNet block's dense layers as passes of the library (`hgc_gravnet_feature_layer`, `hgc_gravnet_output_layer` and
+their gradients) against the products in 64 bits, and which blocks take them."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def check(got, terms, addend=None):
+    """`terms`: (matrix, weight [out, in]) pairs whose products are added up. Every product and every addition is off by 2^-24
+    of a partial sum at the most, and the absolute values bound those."""
+    want = sum(a.double() @ w.double().t() for a, w in terms)
+    size = sum(a.double().abs() @ w.double().abs().t() for a, w in terms)
+    depth = sum(a.shape[1] for a, _ in terms)
+    if addend is not None:
+        want, size = want + addend.double(), size + addend.double().abs()
+    assert ((got.double() - want).abs() <= (depth + 2) * 2.0 ** -24 * size + 1e-37).all()
+    return want
+
+
+# tiles of 16 columns and rows, widths of 4 up, remainders of both, several workgroups along the columns, the widest layers
+@pytest.mark.parametrize("n", [1, 16, 17, 2061])
+@pytest.mark.parametrize("x_width,f,c,o", [(4, 4, 1, 4), (5, 7, 2, 6), (16, 16, 4, 16), (17, 31, 3, 33), (64, 64, 4, 128),
+                                           (96, 128, 4, 160), (13, 129, 3, 100), (256, 128, 4, 256), (412, 50, 2, 255)])
+def test_passes(n, x_width, f, c, o):
+    from hgcalml_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(n + f)
+
+    def normal(*shape):
+        return torch.randn(*shape, device=DEV, generator=gen)
+    # x starts four bytes into its memory
+    x = normal(n * x_width + 1)[1:].view(n, x_width)
+    w_feat, bias, w_coords = normal(f, x_width), normal(f), normal(c, x_width)
+    for relu in (True, False):
+        feat, linear = (ops.gravnet_feature_layer(x, w_feat, bias, r) for r in (relu, False))
+        check(linear, [(x, w_feat)], bias)
+        assert torch.equal(feat, torch.relu(linear) if relu else linear)
+
+    acc, w, b = normal(n, 2 * f), normal(o, 2 * f + x_width), normal(o)
+    joined = torch.cat([acc - feat.repeat(1, 2), x], dim=1)
+    out, kept = ops.gravnet_output_layer(acc, feat, x, w, b, True)
+    again, none = ops.gravnet_output_layer(acc, feat, x, w, b, False)
+    assert torch.equal(kept, joined) and torch.equal(out, again) and none.numel() == 0
+    # max(., 0) moves no two numbers apart: the bound of the sum holds for it too
+    want = joined.double() @ w.double().t() + b.double()
+    size = joined.double().abs() @ w.double().abs().t() + b.double().abs()
+    assert ((out.double() - want.clamp_min(0)).abs() <= (2 * f + x_width + 2) * 2.0 ** -24 * size).all() and (out >= 0).all()
+
+    g = normal(n, o)
+    g_acc, g_feat, g_x, masked = ops.gravnet_output_layer_grad(g, out, w, f)
+    assert torch.equal(masked, torch.where(out > 0, g, torch.zeros_like(g)))
+    check(g_acc, [(masked, w[:, :2 * f].t())])
+    check(g_x, [(masked, w[:, 2 * f:].t())])
+    assert torch.equal(g_feat, -g_acc[:, :f] - g_acc[:, f:])
+
+    feat = torch.relu(normal(n, f))
+    for g2, g_c, g_x2, relu in ((normal(n, f), normal(n, c), g_x, True), (None, None, None, True), (None, normal(n, c), None, False)):
+        g_in, masked = ops.gravnet_input_layers_grad(g_feat, g2, feat, g_c, g_x2, w_feat, w_coords, relu)
+        total = g_feat if g2 is None else g_feat + g2
+        assert torch.equal(masked, torch.where(feat > 0, total, torch.zeros_like(total)) if relu else total)
+        check(g_in, [(masked, w_feat.t())] + ([] if g_c is None else [(g_c, w_coords.t())]), g_x2)
+
+
+def test_non_finite_values_stay_in_their_rows():
+    from hgcalml_amd import ops
+    torch.manual_seed(3)
+    x = torch.randn(37, 13, device=DEV)
+    x[5, 12], x[20, 0] = float("nan"), float("inf")
+    w, b = torch.randn(10, 13, device=DEV), torch.randn(10, device=DEV)
+    want = torch.nn.functional.linear(x, w, b)
+    for got, ref in ((ops.gravnet_feature_layer(x, w, b, False), want), (ops.gravnet_feature_layer(x, w, b, True), torch.relu(want))):
+        assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(torch.isinf(got), torch.isinf(ref))
+        assert torch.isfinite(got[torch.arange(37, device=DEV) % 15 != 5]).all()
+
+
+@pytest.fixture
+def layers_taken(monkeypatch):
+    from hgcalml_amd import ops
+    seen, real = [], ops.gravnet_output_layer
+    monkeypatch.setattr(ops, "gravnet_output_layer", lambda *args: seen.append(1) or real(*args))
+    return seen
+
+
+def block(**kwargs):
+    from hgcalml_amd import RaggedGravNet
+    torch.manual_seed(8)
+    return RaggedGravNet(13, 9, 3, 30, 11, **kwargs).to(DEV)
+
+
+X = dict(row_splits=[0, 5, 400, 700])
+
+
+def step(layer, x, create_graph=False, second=False):
+    rs = torch.tensor(X["row_splits"], dtype=torch.int32, device=DEV)
+    layer.dynamic_radius.fill_(1.0)
+    out, coords, idx, dist = layer(x, rs)
+    wanted = [t for t in [x] + list(layer.parameters()) if t.requires_grad]
+    loss = (out * out).sum() + (coords * coords).sum()
+    if not second:
+        loss = loss + (dist * torch.linspace(0, 1, dist.numel(), device=DEV).view(dist.shape)).sum()
+    grads = torch.autograd.grad(loss, wanted, create_graph=create_graph)
+    if second:  # the last layer's weight gradient once more, with respect to that weight and its bias
+        last = layer.output_feature_transform
+        at = [i for i, t in enumerate(wanted) if t is last.weight][0]
+        grads = torch.autograd.grad((grads[at] * grads[at]).sum(), [last.weight, last.bias])
+    return [out.detach()] + [g.detach() for g in grads]
+
+
+def agree(a, b):
+    for s, t in zip(a, b):
+        assert (s.double() - t.double()).norm() <= 1e-5 * t.double().norm() + 1e-30
+
+
+@pytest.mark.parametrize("frozen", [(), ("input_feature_transform.weight",), ("output_feature_transform.weight",),
+                                    ("input_feature_transform.weight", "input_feature_transform.bias", "input_spatial_transform.weight")])
+@pytest.mark.parametrize("x_grad", [True, False])
+def test_block_with_parts_frozen(frozen, x_grad, layers_taken, monkeypatch):
+    """the same operations as the layers one by one but for the order of their sums: 1e-5"""
+    layer = block()
+    for name, weight in layer.named_parameters():
+        weight.requires_grad_(name not in frozen)
+    x = torch.randn(700, 13, device=DEV, requires_grad=x_grad)
+    got = step(layer, x)
+    assert layers_taken == [1]
+    monkeypatch.setattr(type(layer), "_layers_in_one_pass", lambda self, x: False)
+    agree(got, step(layer, x))
+    assert layers_taken == [1]
+
+
+@pytest.mark.parametrize("second", [False, True])
+def test_derivative_of_the_derivative(second, layers_taken, monkeypatch):
+    layer = block()
+    x = torch.randn(700, 13, device=DEV, requires_grad=True)
+    got = step(layer, x, create_graph=True, second=second)
+    assert layers_taken == [1]
+    monkeypatch.setattr(type(layer), "_layers_in_one_pass", lambda self, x: False)
+    agree(got, step(layer, x, create_graph=True, second=second))
+
+
+def test_blocks_that_are_left_alone(layers_taken):
+    """hooks, replaced layers and methods, other activations, autocast, widths and strides that the passes do not take"""
+    x = torch.randn(700, 13, device=DEV, requires_grad=True)
+    calls = []
+    layer = block()
+    layer.output_feature_transform.register_forward_hook(lambda *args: calls.append(1))
+    step(layer, x)
+    assert calls == [1]
+    layer = block()
+    layer.input_feature_transform = torch.nn.Linear(13, 11).to(DEV)
+    step(layer, x)
+    layer = block()
+    torch.nn.utils.parametrizations.weight_norm(layer.output_feature_transform)
+    step(layer, x)
+    layer = block()
+    layer.update_dynamic_radius = lambda dist: calls.append(2)
+    step(layer, x)
+    step(block(feature_activation="tanh"), x)
+    layer = block()
+    step(layer, x.detach().t().contiguous().t().requires_grad_(True))
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        layer(x, torch.tensor(X["row_splits"], dtype=torch.int32, device=DEV))
+    assert layers_taken == [] and calls == [1, 2]
+    with torch.no_grad():
+        layer(x, torch.tensor(X["row_splits"], dtype=torch.int32, device=DEV))
+    assert layers_taken == [1]
