@@ -528,16 +528,20 @@ int launch_records(const float *g, const float *feat, const uint4 *records, cons
 
 // ---- pass 3: weight gradients from list order to their slots -------------------
 
-// gw[inv_slots[e]] = gw_list[e] for the entries of all targets, four per thread. The
+// gw[inv_slots[e]] = gw_list[e] for the entries of all targets (unless *wanted is 0), four per thread. The
 // scattered 4-byte writes of one stretch of the list fall into the rows of the source
 // vertices around it; each XCD works on one contiguous stretch, so the lines stay in
-// its L2 until they are full.
-__global__ __launch_bounds__(256) void weight_grad_to_table_kernel(const int *__restrict__ inv_off,
+// its L2 until they are full. (As a loop over 2048 workgroups every load waits for the stores in front of it: 64 M entries
+// 1000 us in the place of 460.)
+constexpr int kToTableThreads = 1024;
+
+__global__ __launch_bounds__(kToTableThreads) void weight_grad_to_table_kernel(const int *__restrict__ inv_off,
                                                                    const int *__restrict__ inv_slots,
                                                                    const float *__restrict__ gw_list,
-                                                                   float *__restrict__ gw, int n_vert) {
+                                                                   float *__restrict__ gw, int n_vert, const int *__restrict__ wanted) {
+    if (wanted && !*wanted) return;
     const long long n_entries = inv_off[n_vert];
-    const long long e0 = ((long long)xcd_contiguous_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x) * 4;
+    const long long e0 = ((long long)xcd_contiguous_block(blockIdx.x, gridDim.x) * kToTableThreads + threadIdx.x) * 4;
     if (e0 + 4 <= n_entries) {
         const u32x4 slots = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(inv_slots + e0));
         const f32x4 vals = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(gw_list + e0));
@@ -559,6 +563,13 @@ bool records_layout(int F, uintptr_t align_or, int &vec, int &nb) {
 }
 
 }  // namespace
+
+// gw_list and inv_slots start on 16-byte boundaries; the list has at most `total` entries (fewer where slots are padded)
+int launch_weight_grad_to_table(const int *inv_off, const int *inv_slots, const float *gw_list, float *gw, int n_vert,
+                                long long total, const int *wanted, hipStream_t s) {
+    weight_grad_to_table_kernel<<<ceil_div(total, 4 * kToTableThreads), kToTableThreads, 0, s>>>(inv_off, inv_slots, gw_list, gw, n_vert, wanted);
+    return check_launch("weight_grad_to_table_kernel");
+}
 
 int launch_zero_padded_weight_grad(const int *inv_off, const int *inv_slots, float *gw, int n_vert, long long total,
                                    hipStream_t s);
@@ -614,10 +625,7 @@ int launch_accumulate_grad_records(const float *g, const float *w, const float *
     else rc = nb == 1 ? launch_records<1, 1, false>(HGC_ARGS) : launch_records<1, 2, false>(HGC_ARGS);
 #undef HGC_ARGS
     if (rc) return rc;
-    // the list has at most n_vert * K entries (fewer where slots are padded)
-    const long long blocks = ceil_div((long long)n_vert * K, 1024ll);
-    weight_grad_to_table_kernel<<<dim3((unsigned)blocks), 256, 0, s>>>(inv_off, inv_slots, gw_list, gw, n_vert);
-    return check_launch("weight_grad_to_table_kernel");
+    return launch_weight_grad_to_table(inv_off, inv_slots, gw_list, gw, n_vert, (long long)n_vert * K, nullptr, s);
 }
 
 }  // namespace hgc

@@ -40,6 +40,10 @@
 
 namespace hgc {
 
+// accumulate_grad_records.hip
+int launch_weight_grad_to_table(const int *inv_off, const int *inv_slots, const float *gw_list, float *gw, int n_vert,
+                                long long total, const int *wanted, hipStream_t s);
+
 namespace {
 
 using namespace acc;
@@ -56,6 +60,10 @@ struct GradRows {
     const unsigned char *maxslot;
     const int *inv_off, *inv_slots, *order;
     float *gw, *gfeat;
+    // Weight gradients in the order of the inverse index, moved to their slots by a pass of its own, where *scattered is
+    // set (see list_order_may_pay; both null: never)
+    float *gw_list;
+    const int *scattered;
     unsigned long long g_bytes, g_max_bytes, slot_bytes;  // sizes seen by the hardware's range check
     int n_vert, K, F, blocks, pitch;
     int skip;  // 1: the inverse index is that of a table with one more column in front (K + 1), which is left out
@@ -222,6 +230,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
     const __amdgpu_buffer_rsrc_t GX = make_rows(p.g_max, MAX ? p.g_max_bytes : 0);
     const __amdgpu_buffer_rsrc_t MS = make_rows(p.maxslot, MAX ? p.slot_bytes : 0);
     const float inv_divisor = 1.f / p.divisor;
+    const bool in_list_order = WGRAD && p.scattered && *p.scattered;
 
     // A lane at the end of a row that is no multiple of VEC, and the lanes behind it, take the last VEC
     // columns (never columns of the next row); what they share with another lane counts there (see TAIL).
@@ -338,7 +347,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
                 self_dot = in_group ? dot : self_dot;
             }
             if (MAX && selves.repeats) sum = __builtin_amdgcn_inverse_ballot_w64(selves.repeats) ? self_dot : sum;
-            if (en.slot >= 0 && task.block == 0) p.gw[en.slot] = p.negate ? -(sum * en.w) : sum;
+            if (en.slot >= 0 && task.block == 0) {
+                const float value = p.negate ? -(sum * en.w) : sum;
+                if (in_list_order) __builtin_nontemporal_store(value, p.gw_list + begin + c0 + entry_lane(l));
+                else p.gw[en.slot] = value;
+            }
         }
         slot_next = slot_after;
         en = next;
@@ -405,11 +418,48 @@ bool accumulate_grad_rows_covers(int n_feat, int n_neigh, bool mean_and_max, boo
            g_bytes <= kMaxRowBytes;
 }
 
+// The weight gradients of the targets in flight are 4-byte writes into the rows of everything that names them. Where those
+// rows, with the gradient rows and slots that are gathered, are more than an XCD's L2 holds, lines leave it before they are
+// whole and are written several times (fabric traffic five times the compulsory one at a million vertices, F = 128, window
+// +-2000). There the values leave in the order of the lists, in whole lines, and a pass moves them to their slots. us of the
+// gradient, scattered / in list order, banded tables of window +-2000: a million vertices, K = 64, F = 128 4612 / 4076, F = 64
+// 2700 / 2573, K = 24, F = 128 2454 / 2258; 300,000, K = 64, F = 128 1414 / 1219; 100,000 359 / 353; 20,000 87 / 93; window
+// +-1000, a million, K = 64, F = 128 3773 / 3912; +-300 3546 / 3761; tables of a search in bin order, 300,000 vertices, K = 40, F
+// = 128 907 / 1091. So the host asks for the size (asking and moving nothing costs 10 to 15 us) and leaves tables with a processing
+// order as they are, and the device looks at how far apart the vertices of a list are. (A mean alone gathers half as much.)
+constexpr int kSpanSamples = 1024;
+constexpr long long kSpanBytes = 3ll << 20;  // of the 4 MB of an XCD
+
+static bool list_order_may_pay(int n_vert, int n_feat, int n_neigh, bool mean_and_max) {
+    return mean_and_max && (long long)n_vert * n_neigh >= 16000000 && n_neigh >= 24 && n_feat >= 64;
+}
+
+// *scattered = whether the vertices between the first and the last one that name a target span more than kSpanBytes, on average
+__global__ __launch_bounds__(kSpanSamples) void list_span_kernel(const int *__restrict__ inv_off, const int *__restrict__ inv_slots,
+                                                                 int n_vert, int K, int row_bytes, int *__restrict__ scattered) {
+    __shared__ float s_span[kSpanSamples / kWave];
+    const int m = (int)((long long)threadIdx.x * n_vert / kSpanSamples);
+    const int begin = inv_off[m], end = inv_off[m + 1];
+    float span = begin < end ? (float)(inv_slots[end - 1] / K - inv_slots[begin] / K) : 0.f;
+    for (int off = kWave / 2; off > 0; off >>= 1) span += __shfl_xor(span, off);
+    if (lane_id() == 0) s_span[threadIdx.x / kWave] = span;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int i = 1; i < kSpanSamples / kWave; ++i) span += s_span[i];
+        *scattered = span * (1.f / kSpanSamples) * (float)row_bytes > (float)kSpanBytes;
+    }
+}
+
+static size_t quotient_bytes(int n_vert, int n_feat, float divisor) {
+    if (divisor == (float)(int)divisor && is_pow2((int)divisor)) return 0;
+    return align_up((size_t)n_vert * n_feat * sizeof(float));
+}
+
 size_t accumulate_grad_rows_scratch_bytes(int n_vert, int n_feat, int n_neigh, bool mean_and_max, float divisor) {
     const unsigned long long n = (unsigned long long)std::max(n_vert, 0) * std::max(n_feat, 0) * sizeof(float);
     if (!accumulate_grad_rows_covers(n_feat, n_neigh, mean_and_max, true, n * (mean_and_max ? 2 : 1))) return 0;
-    if (divisor == (float)(int)divisor && is_pow2((int)divisor)) return 0;
-    return align_up((size_t)n);
+    return quotient_bytes(std::max(n_vert, 0), n_feat, divisor) +
+           (list_order_may_pay(n_vert, n_feat, n_neigh, mean_and_max) ? align_up((size_t)n_vert * n_neigh * sizeof(float)) + align_up(sizeof(int)) : 0);
 }
 
 // Returns 1 where the shape is not covered. gw == nullptr: feature gradient only (mean only). scratch
@@ -426,9 +476,22 @@ int launch_accumulate_grad_rows(const float *g, const float *w, const float *fea
     GradRows p;
     Scale scale = kDivide;
     p.g = g;
+    const bool room = scratch && scratch_bytes >= accumulate_grad_rows_scratch_bytes(n_vert, F, K, mean_and_max, divisor);
+    p.gw_list = nullptr;
+    p.scattered = nullptr;
+    // (the list is read four entries at a time)
+    if (room && want_w && skip == 0 && !order && list_order_may_pay(n_vert, F, K, mean_and_max) && (reinterpret_cast<uintptr_t>(inv_slots) & 15u) == 0) {
+        char *const behind = static_cast<char *>(scratch) + quotient_bytes(n_vert, F, divisor);
+        int *const scattered = reinterpret_cast<int *>(behind + align_up((size_t)n_vert * K * sizeof(float)));
+        p.gw_list = reinterpret_cast<float *>(behind);
+        p.scattered = scattered;
+        const int row_bytes = 4 * g_cols + 4 * K + F;
+        list_span_kernel<<<1, kSpanSamples, 0, s>>>(inv_off, inv_slots, n_vert, K, row_bytes, scattered);
+        if (const int rc = check_launch("list_span_kernel")) return rc;
+    }
     if (divisor == (float)(int)divisor && is_pow2((int)divisor)) {
         scale = kPow2;
-    } else if (scratch && scratch_bytes >= accumulate_grad_rows_scratch_bytes(n_vert, F, K, mean_and_max, divisor)) {
+    } else if (room) {
         scale = kScaled;
         const long long total = (long long)n_vert * F;
         divide_mean_half_kernel<<<ceil_div(total, 256), 256, 0, s>>>(g, static_cast<float *>(scratch), total, F, g_cols, divisor);
@@ -457,14 +520,16 @@ int launch_accumulate_grad_rows(const float *g, const float *w, const float *fea
     p.div_k = make_fast_div(K + skip);
     p.divisor = divisor;
     p.negate = negate;
-    int vec;
+    int vec, rc;
     row_shape(F, vec, p.blocks);
     switch (vec) {
-        case 1: return launch_rows<1>(p, mean_and_max, want_w, scale, s);
-        case 2: return launch_rows<2>(p, mean_and_max, want_w, scale, s);
-        case 3: return launch_rows<3>(p, mean_and_max, want_w, scale, s);
-        default: return launch_rows<4>(p, mean_and_max, want_w, scale, s);
+        case 1: rc = launch_rows<1>(p, mean_and_max, want_w, scale, s); break;
+        case 2: rc = launch_rows<2>(p, mean_and_max, want_w, scale, s); break;
+        case 3: rc = launch_rows<3>(p, mean_and_max, want_w, scale, s); break;
+        default: rc = launch_rows<4>(p, mean_and_max, want_w, scale, s); break;
     }
+    if (rc || !p.gw_list) return rc;
+    return launch_weight_grad_to_table(inv_off, inv_slots, p.gw_list, gw, n_vert, (long long)n_vert * K, p.scattered, s);
 }
 
 }  // namespace hgc

@@ -33,7 +33,6 @@ namespace {
 constexpr int kTile = 16, kStepCols = 16;
 constexpr int kGroups = 256;               // workgroups at the most, one per CU
 constexpr int kLdsBytes = 160 * 1024;
-constexpr int kMostTiles = 12;             // of 16 output columns, in a wave's registers
 
 typedef float vec4 __attribute__((ext_vector_type(4)));
 
