@@ -68,6 +68,32 @@ struct KnnParams {
     int fine_bits, fine_min_population;
 };
 
+// The kernel's arguments, read again where they are needed: at eight waves a SIMD a wave has 78 scalar registers, and what
+// the compiler keeps in them from the first instruction on (it knows that arguments do not change) it moves to lanes of a
+// vector register and back, four at a time, by vector instructions, of which the search is made. (With these, the grid's
+// numbers by scalar loads, the first cube's prefix sum used again and no last merge for up to 32 keys: 474 -> 436 vector
+// instructions per query of the batch of 16 events, 1156 -> 1097 us; 100,000 2-D Gaussian points, K = 10 124 -> 117; 150,000 4-D
+// points, K = 64 1074 -> 1039, 362 -> 356. Seven waves with more registers: 1200. Half-widths 1 and 2 of the first cube
+// looked up together: 1115.)
+typedef const __attribute__((address_space(4))) KnnParams *KernelArgs;
+__device__ __forceinline__ KernelArgs kernel_args() {
+    KernelArgs a = (KernelArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(a));
+    return a;
+}
+
+// a value of its own, not one of four that were loaded together and stay together
+__device__ __forceinline__ int alone(int v) {
+    asm("" : "+s"(v));
+    return v;
+}
+
+// a data error of this lane, into the status word (if there is one)
+__device__ __forceinline__ void report(int flag) {
+    int *const status = kernel_args()->status;
+    if (status) atomicOr(status, flag);
+}
+
 template <int C>
 __device__ __forceinline__ float dist_sq(const float (&q)[C > 0 ? C : 1], const float *__restrict__ coord, int j,
                                          int n_coords, const float *__restrict__ qrow) {
@@ -221,14 +247,14 @@ __device__ __forceinline__ uint64_t bitonic_merge_steps(uint64_t key) {
     return compare_exchange<K, 1>(key);
 }
 
-// ascending sort of one key per lane
-__device__ __forceinline__ uint64_t wave_sort_u64(uint64_t key) {
+// ascending sort of one key per lane; the lanes from `n` on hold the empty key, and up to 32 keys need no last merge
+__device__ __forceinline__ uint64_t wave_sort_u64(uint64_t key, int n = kWave) {
     key = bitonic_merge_steps<2>(key);
     key = bitonic_merge_steps<4>(key);
     key = bitonic_merge_steps<8>(key);
     key = bitonic_merge_steps<16>(key);
     key = bitonic_merge_steps<32>(key);
-    return bitonic_merge_steps<64>(key);
+    return n <= kWave / 2 ? key : bitonic_merge_steps<64>(key);
 }
 
 // the 64 smallest of an ascending list and an ascending batch, ascending:
@@ -746,7 +772,7 @@ __device__ __forceinline__ bool walk_shells(const KnnParams &p, const int q, con
 //   * then one pass over the rows of bins outside the cube that the bound reaches;
 //   * then the keys that are left are sorted, once.
 // Vector instructions per query: 16 events of 1.14 M 3-D points, K = 32, radius 0.1 about 700 -> 474, 150,000 4-D
-// points, K = 64 1476 -> 1074. The whole search, by shells -> collected: these two 1399 -> 1173 us and 429 -> 372 us;
+// points, K = 64 1476 -> 1074 (now 436 and 1039, see kernel_args). The whole search, by shells -> collected: these two 1399 -> 1173 us and 429 -> 372 us;
 // 240,000 3-D points, K = 41 367 -> 307; 4-D Gaussian, K = 65 467 -> 410; 4-D uniform, K = 64 361 -> 305; 2-D
 // clusters, K = 32 186 -> 130; 3-D clusters, K = 96 489 -> 319. Tried and taken back: first regions that leave out the
 // corners of the cube (fewer candidates, but a second pass for every query: 4 to 13 % slower), up to three pieces of a
@@ -897,6 +923,8 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
                                                 uint64_t *const buffer, const int Kn, uint64_t (&key)[S]) {
     static_assert(C > 0 && NB >= 2 && NB <= 4 && S <= 2 && (!FINE || NB >= 3));
     constexpr int B = NB;
+    const int n_bboundaries = alone(p.n_bboundaries);
+    const bool use_direction = alone(p.use_direction) != 0;
     float qc[C];
     const float *qrow = p.coord + (size_t)q * C;
 #pragma unroll
@@ -909,10 +937,12 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
     const int dim = min(lane, B - 1);
     int nb_v = p.n_bins[dim], qb_v = p.dim_bin_idx[(size_t)q * (B + 1) + 1 + dim];
     int in_event = 0, cells_per_event = 1;  // number of the own bin inside its event
+    [[maybe_unused]] int nb_s[B], qb_s[B];  // the same by scalar loads
 #pragma unroll
     for (int i = 0; i < B; ++i) {
-        in_event = in_event * readlane_i32(nb_v, i) + readlane_i32(qb_v, i);
-        cells_per_event *= readlane_i32(nb_v, i);
+        nb_s[i] = p.n_bins[i], qb_s[i] = p.dim_bin_idx[(size_t)q * (B + 1) + 1 + i];
+        in_event = in_event * nb_s[i] + qb_s[i];
+        cells_per_event *= nb_s[i];
     }
     int event_base = own_bin - in_event;
     bool placed = true;
@@ -933,8 +963,8 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
     bool rows_fit = true;
 #pragma unroll
     for (int i = 0; i < B; ++i) {
-        nb[i] = readlane_i32(nb_v, i);
-        qb[i] = readlane_i32(qb_v, i);
+        nb[i] = FINE ? 2 * nb_s[i] : nb_s[i];
+        qb[i] = CALLERS ? readlane_i32(qb_v, i) : FINE ? 2 * qb_s[i] + ((own_cell >> (B - 1 - i)) & 1) : qb_s[i];
         if (i < B - 1) {
             grid_rows *= nb[i];
             rows_fit = rows_fit && (i == 0 || nb[i] < (1 << 13)) && (!CALLERS || nb[i] > 0);
@@ -945,10 +975,10 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
     grid_rows *= FINE ? bins_last + 1 : 2;  // slots of a pass
     bool no_grid = event_base < 0;  // a bin, or numbers of bins, that no grid has
     if (CALLERS && grid_rows < (1ll << 22))  // (grid_rows is twice the rows here; flat bins are 32 bits)
-        no_grid = no_grid || grid_rows <= 0 || nb_last < 1 || event_base >= p.n_bboundaries - 1 || 2ll * event_base + grid_rows * nb_last > 1ll << 32;
+        no_grid = no_grid || grid_rows <= 0 || nb_last < 1 || event_base >= n_bboundaries - 1 || 2ll * event_base + grid_rows * nb_last > 1ll << 32;
     if (!rows_fit || grid_rows >= (1ll << 22) || no_grid) {  // see divmod_small
         if (FINE) return false;  // the grid of bins may do
-        if (p.status && lane == 0) atomicOr(p.status, no_grid ? HGC_FLAG_BIN_BEYOND_TABLE : HGC_FLAG_SHELL_TOO_WIDE);
+        if (lane == 0) report(no_grid ? HGC_FLAG_BIN_BEYOND_TABLE : HGC_FLAG_SHELL_TOO_WIDE);
         return true;  // the list stays empty
     }
     const float bw = !placed ? 0.f : FINE ? 0.5f * p.bin_width[0] : p.bin_width[0];
@@ -976,12 +1006,12 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
     // as by the reference, which prints "idx out of range"
     int seg_start = 0, seg_len = 0;
     [[maybe_unused]] auto callers_run = [&](int first, int last) {
-        const int there = min(last, p.n_bboundaries - 1);
+        const int there = min(last, n_bboundaries - 1);
         if (first < there) {
             seg_start = p.bin_boundaries[first];
             seg_len = p.bin_boundaries[there] - seg_start;
         }
-        if (p.status && there < last) atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
+        if (there < last) report(HGC_FLAG_BIN_BEYOND_TABLE);
     };
 
     // lower bounds of the distance to the edges of the own bin, in bin widths, as in walk_shells
@@ -1012,6 +1042,7 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
     // the radius asks for). One lane per row of bins (on the nested grid per row and bin that the row's three cells
     // touch, always two).
     const int enough = Kn + (Kn >> kFirstCubeShift);
+    int first_end = 0;  // prefix sum of the rows' lengths
     int d_out, d_radius = 1 << 30;  // the cube of half-width d_radius holds everything within the radius
     if (has_radius && prunes)
         d_radius = max(1, uniform((int)fminf(__builtin_ceilf(__builtin_amdgcn_sqrtf(bound_of(__float_as_uint(p.radius_sq))) * bins_per_unit), 1.0e9f)));
@@ -1070,12 +1101,12 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
             const int lo = max(max(qb_last - min(d_out, lo_most), 0), 2 * bin_last);
             const int hi = min(min(qb_last + min(d_out, hi_most), nb_last - 1), 2 * bin_last + 1);
             const int bin = row_base(cell) + bin_last;
-            if (in_grid && ring <= d_out && lo <= hi && bin + 1 < p.n_bboundaries) {
+            if (in_grid && ring <= d_out && lo <= hi && bin + 1 < n_bboundaries) {
                 const int base = ((bin << (B - 1)) | halves) << 1;
                 seg_start = table_entry(p.cell_boundaries, base | (lo & 1));
                 seg_len = table_entry(p.cell_boundaries, (base | (hi & 1)) + 1) - seg_start;
             }
-            if (p.status && in_grid && ring <= d_out && lo <= hi && bin + 1 >= p.n_bboundaries) atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
+            if (in_grid && ring <= d_out && lo <= hi && bin + 1 >= n_bboundaries) report(HGC_FLAG_BIN_BEYOND_TABLE);
         } else {
             constexpr int kCubes = B == 4 ? 1 : 3;
             // lanes without a row look at the own one
@@ -1086,14 +1117,15 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
                 if constexpr (CALLERS) {
                     if (in_grid && ring <= d && from < to) callers_run(row + from, row + to);
                 } else {
-                    const bool wanted = in_grid && ring <= d && row < p.n_bboundaries - to;
+                    const bool wanted = in_grid && ring <= d && row < n_bboundaries - to;
                     if (wanted) {
                         seg_start = table_entry(p.bin_boundaries, row + from);
                         seg_len = table_entry(p.bin_boundaries, row + to) - seg_start;
                     }
-                    if (p.status && in_grid && ring <= d && !wanted) atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
+                    if (in_grid && ring <= d && !wanted) report(HGC_FLAG_BIN_BEYOND_TABLE);
                 }
-                return readlane_i32(wave_inclusive_sum(seg_len), kWave - 1);
+                first_end = wave_inclusive_sum(seg_len);
+                return readlane_i32(first_end, kWave - 1);
             };
             d_out = 1;
             const int held = look(1);
@@ -1103,13 +1135,14 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
                     d_out = 3;
                     look(3);
                 }
-            } else if (held > 4 * enough && placed && own_bin + 1 < p.n_bboundaries &&
+            } else if (held > 4 * enough && placed && own_bin + 1 < n_bboundaries &&
                        uniform(p.bin_boundaries[own_bin + 1]) - uniform(p.bin_boundaries[own_bin]) > enough) {
                 d_out = 0;  // crowded: the own bin does
                 look(0);
             }
             d_out = uniform(d_out);
         }
+        if (FINE) first_end = wave_inclusive_sum(seg_len);
     }
 
     int n_kept = 0;  // keys in the buffer
@@ -1231,28 +1264,28 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
                 if (rest >= 0.f && lo <= hi) {
                     if (FINE) {
                         const int bin = row_base(cell) + ((qb_last + lo) >> 1);
-                        if (bin + 1 < p.n_bboundaries) {
+                        if (bin + 1 < n_bboundaries) {
                             const int base = ((bin << (B - 1)) | halves) << 1;
                             seg_start = table_entry(p.cell_boundaries, base | ((qb_last + lo) & 1));
                             seg_len = table_entry(p.cell_boundaries, (base | ((qb_last + hi) & 1)) + 1) - seg_start;
-                        } else if (p.status) {
-                            atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
+                        } else {
+                            report(HGC_FLAG_BIN_BEYOND_TABLE);
                         }
                     } else {
                         const int first = row_base(cell) + qb_last + lo;
                         const int last = first + (hi - lo) + 1;
                         if constexpr (CALLERS) {
                             callers_run(first, last);
-                        } else if (last < p.n_bboundaries) {
+                        } else if (last < n_bboundaries) {
                             seg_start = table_entry(p.bin_boundaries, first);
                             seg_len = table_entry(p.bin_boundaries, last) - seg_start;
-                        } else if (p.status) {
-                            atomicOr(p.status, HGC_FLAG_BIN_BEYOND_TABLE);
+                        } else {
+                            report(HGC_FLAG_BIN_BEYOND_TABLE);
                         }
                     }
                 }
             }
-            const int seg_end = wave_inclusive_sum(seg_len);
+            const int seg_end = d_in >= 0 ? wave_inclusive_sum(seg_len) : first_end;
             const int seg_off = seg_end - seg_len;
             const int total = readlane_i32(seg_end, kWave - 1);
             // kept one lane up, so that the mark (lane number + 1) is the lane to read it from: see walk_shells
@@ -1279,8 +1312,8 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
                                                      reinterpret_cast<const char *>(p.sorting) + ((uint32_t)jj << 2))
                                                : (uint32_t)jj;
                     const float dsq = dist_sq<C>(qc, p.coord, jj, C, qrow);
-                    if (p.use_direction) {
-                        const int dj = p.direction[jj];
+                    if (use_direction) {
+                        const int dj = kernel_args()->direction[jj];
                         valid &= ~__builtin_amdgcn_ballot_w64(dj == 1 || dj == 2);  // may not be a neighbour
                     }
                     uint64_t enters = valid & __builtin_amdgcn_ballot_w64(__float_as_uint(dsq) <= cut);
@@ -1315,7 +1348,7 @@ __device__ __forceinline__ bool collect_nearest(const KnnParams &p, const int q,
 
     wave_lds_fence();
     if (n_kept > S * kWave) n_kept = cut_to_smallest<CALLERS>(buffer, lane, n_kept, Kn, S * kWave, cut, cut_id);
-    key[0] = wave_sort_u64(lane < n_kept ? buffer[lane] : kEmptyKey);
+    key[0] = wave_sort_u64(lane < n_kept ? buffer[lane] : kEmptyKey, n_kept);
     if constexpr (S == 2) {
         key[1] = kEmptyKey;
         if (n_kept > kWave) merge_batch<S>(key, wave_sort_u64(kWave + lane < n_kept ? buffer[kWave + lane] : kEmptyKey));
@@ -1392,17 +1425,22 @@ __device__ __forceinline__ void search_query(const KnnParams &p, const int q, co
     }
 
     // ---- write the row: slot 0 = self, then ascending (distance, index) ----
+    const KernelArgs args = kernel_args();
+    const int id = kCollects && MAPPED ? args->sorting[q] : self_id, pad = args->tf_compat ? id : -1;
+    const size_t row = (size_t)id * args->K;
+    int *const out_idx = args->out_idx;
+    float *const out_dist = args->out_dist;
     if (lane == 0 && rank_base == 0) {
-        p.out_idx[out_row] = self_id;
-        p.out_dist[out_row] = 0.f;
+        out_idx[row] = id;
+        out_dist[row] = 0.f;
     }
 #pragma unroll
     for (int s = 0; s < S; ++s) {
         const int rank = s * kWave + lane;
         if (rank < Kn) {
             const bool filled = key[s] != kEmptyKey;
-            p.out_idx[out_row + 1 + rank_base + rank] = filled ? (int)(uint32_t)key[s] : pad_idx;
-            p.out_dist[out_row + 1 + rank_base + rank] = filled ? __uint_as_float((uint32_t)(key[s] >> 32)) : 0.f;
+            out_idx[row + 1 + rank_base + rank] = filled ? (int)(uint32_t)key[s] : pad;
+            out_dist[row + 1 + rank_base + rank] = filled ? __uint_as_float((uint32_t)(key[s] >> 32)) : 0.f;
         }
     }
 }
