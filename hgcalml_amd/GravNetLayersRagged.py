@@ -54,25 +54,26 @@ def _weight_grad_in_one_pass(g, x):
 
 
 class _DropSelfFn(torch.autograd.Function):
-    """table and distances without the self column, and the distances themselves: the gradients of both come back in
-    one pass. The distances leave as a tensor of their own on the same memory, which may be written to (an input handed
+    """table and distances (times `scale`) without the self column, and the distances themselves: the gradients of both come
+    back in one pass. The distances leave as a tensor of their own on the same memory, which may be written to (an input handed
     back would be a view that refuses it): the block reads them no more, and neither does the search's gradient."""
 
     @staticmethod
-    def forward(ctx, idx, dist):
+    def forward(ctx, idx, dist, scale):
         ctx.set_materialize_grads(False)
-        nidx, ndist = ops.gravnet_drop_self(idx, dist)
+        ctx.scale = scale
+        nidx, ndist = ops.gravnet_drop_self(idx, dist, scale)
         ctx.mark_non_differentiable(nidx)
         return nidx, ndist, dist.data
 
     @staticmethod
     def backward(ctx, _grad_nidx, grad_narrow, grad_wide):
         if grad_narrow is None:
-            return None, grad_wide
+            return None, grad_wide, None
         if torch.is_grad_enabled():
-            grad = torch.nn.functional.pad(grad_narrow, (1, 0))
-            return None, grad if grad_wide is None else grad + grad_wide
-        return None, ops.gravnet_drop_self_grad(grad_narrow, grad_wide)
+            grad = torch.nn.functional.pad(ctx.scale * grad_narrow, (1, 0))
+            return None, grad if grad_wide is None else grad + grad_wide, None
+        return None, ops.gravnet_drop_self_grad(grad_narrow, grad_wide, ctx.scale), None
 
 
 class _JoinFn(torch.autograd.Function):
@@ -221,6 +222,7 @@ _ACTIVATIONS = {None: nn.Identity, "linear": nn.Identity, "relu": nn.ReLU, "elu"
                 "sigmoid": nn.Sigmoid, "selu": nn.SELU, "gelu": nn.GELU}
 
 
+_DISTANCE_SCALE = 10.0  # neighbours are weighted by exp(-10 d^2)
 _REPLACEABLE = {"compute_neighbours_and_distancesq", "collect_neighbours", "create_output_features", "update_dynamic_radius"}
 
 
@@ -263,15 +265,20 @@ class RaggedGravNet(nn.Module):
             self.dynamic_radius += 0.05 * (update - self.dynamic_radius)
 
     def compute_neighbours_and_distancesq(self, coordinates, row_splits):
+        return self._neighbours(coordinates, row_splits, 1.0)
+
+    def _neighbours(self, coordinates, row_splits, scale):
         idx, dist = BinnedSelectKnn(self.n_neighbours + 1, coordinates, row_splits, max_radius=-1.0,
                                     tf_compatible=False, n_bins=self.n_knn_bins)
         self.update_dynamic_radius(dist.detach())  # missing neighbours have distance 0
         # the table without its self column, as tensors of their own; it lists the
         # same vertices row by row, so the kNN's processing order applies to it too
         if _library_takes(dist):
-            nidx, ndist, dist = _DropSelfFn.apply(idx, dist)
+            nidx, ndist, dist = _DropSelfFn.apply(idx, dist, scale)
         else:
             nidx, ndist = idx[:, 1:].contiguous(), dist[:, 1:].contiguous()
+            if scale != 1.0:
+                ndist = scale * ndist
             if self.return_self:
                 dist = dist.clone()  # may be written to: the search keeps its own
         ops.share_vertex_order(idx, nidx)
@@ -281,10 +288,13 @@ class RaggedGravNet(nn.Module):
         return nidx, ndist, None, None
 
     def collect_neighbours(self, features, neighbour_indices, distancesq):
-        if self.sumwnorm and _library_takes(distancesq, features):
-            return _AccumulateSumwFn.apply(10.0 * distancesq, features, neighbour_indices)
+        return self._collect(features, neighbour_indices, _DISTANCE_SCALE * distancesq)
+
+    def _collect(self, features, neighbour_indices, distances):
+        if self.sumwnorm and _library_takes(distances, features):
+            return _AccumulateSumwFn.apply(distances, features, neighbour_indices)
         acc = AccumulateKnnSumw if self.sumwnorm else AccumulateKnn
-        f, _ = acc(10.0 * distancesq, features, neighbour_indices, mean_and_max=True)
+        f, _ = acc(distances, features, neighbour_indices, mean_and_max=True)
         return f
 
     def create_output_features(self, x, neighbour_indices, distancesq):
@@ -329,8 +339,10 @@ class RaggedGravNet(nn.Module):
             features, coordinates, features_again, x_again = _InputLayersFn.apply(
                 x, self.input_feature_transform.weight, self.input_feature_transform.bias, self.input_spatial_transform.weight,
                 type(self.feature_activation) is nn.ReLU)
-            nidx, ndist, sidx, sdist = self.compute_neighbours_and_distancesq(coordinates, row_splits)
-            accumulated = self.collect_neighbours(features, nidx, ndist)
+            # (where the distances without the self column are handed back, they are so without the factor)
+            scale = _DISTANCE_SCALE if self.return_self else 1.0
+            nidx, ndist, sidx, sdist = self._neighbours(coordinates, row_splits, scale)
+            accumulated = self._collect(features, nidx, ndist) if self.return_self else self.collect_neighbours(features, nidx, ndist)
             last = self.output_feature_transform
             outfeats = _OutputLayerFn.apply(accumulated, features_again, x_again, last.weight, last.bias,
                                             torch.is_grad_enabled() and last.weight.requires_grad)

@@ -69,6 +69,8 @@ _SIGNATURES = {
     "hgc_exp_neg_grad": (_c_int, [_ptr, _ptr, _ptr, ctypes.c_longlong, _ptr]),
     "hgc_gravnet_drop_self": (_c_int, [_ptr] * 2 + [_c_int] * 2 + [_ptr] * 3),
     "hgc_gravnet_drop_self_grad": (_c_int, [_ptr] * 2 + [_c_int] * 2 + [_ptr] * 2),
+    "hgc_gravnet_drop_self_scaled": (_c_int, [_ptr] * 2 + [_c_int] * 2 + [_c_float] + [_ptr] * 3),
+    "hgc_gravnet_drop_self_grad_scaled": (_c_int, [_ptr] * 2 + [_c_int] * 2 + [_c_float] + [_ptr] * 2),
     "hgc_gravnet_radius_step_workspace_bytes": (_c_size, []),
     "hgc_gravnet_radius_step": (_c_int, [_ptr, ctypes.c_longlong] + [_ptr] * 3 + [_c_size, _ptr]),
     "hgc_gravnet_join": (_c_int, [_ptr] * 3 + [_c_int] * 3 + [_ptr] * 2),

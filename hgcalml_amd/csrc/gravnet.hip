@@ -20,9 +20,11 @@ constexpr int kThreads = 256;
 
 // A thread moves four consecutive entries of the narrow table (16-byte stores); the wide rows start anywhere, their
 // loads are four dwords each that neighbouring lanes complete to whole lines.
+// (The block weights neighbours by exp(-10 d^2): its factor is taken here and in the gradient, where the values pass
+// anyway. As products of their own 13 us each way at 150k vertices, K = 64.)
 __global__ __launch_bounds__(kThreads) void drop_self_kernel(const int *__restrict__ idx, const float *__restrict__ dist,
-                                                             unsigned total, unsigned narrow, int *__restrict__ out_idx,
-                                                             float *__restrict__ out_dist) {
+                                                             unsigned total, unsigned narrow, float scale,
+                                                             int *__restrict__ out_idx, float *__restrict__ out_dist) {
     const unsigned first = (blockIdx.x * kThreads + threadIdx.x) * 4u;
     if (first >= total) return;
     unsigned row = first / narrow, col = first - row * narrow;
@@ -33,7 +35,7 @@ __global__ __launch_bounds__(kThreads) void drop_self_kernel(const int *__restri
     for (unsigned u = 0; u < 4; ++u) {
         if (u < count) {
             ai[u] = idx[first + u + row + 1];  // row * (narrow + 1) + col + 1
-            di[u] = dist[first + u + row + 1];
+            di[u] = scale * dist[first + u + row + 1];
         }
         if (++col == narrow) col = 0, ++row;
     }
@@ -47,10 +49,10 @@ __global__ __launch_bounds__(kThreads) void drop_self_kernel(const int *__restri
     }
 }
 
-// gradient w.r.t. the wide distances: that of the narrow ones moved up by a column, plus that of the wide ones (if any)
+// gradient w.r.t. the wide distances: that of the narrow ones, times the factor, moved up by a column, plus that of the wide ones (if any)
 __global__ __launch_bounds__(kThreads) void drop_self_grad_kernel(const float *__restrict__ g_narrow,
                                                                   const float *__restrict__ g_wide, unsigned total,
-                                                                  unsigned wide, float *__restrict__ out) {
+                                                                  unsigned wide, float scale, float *__restrict__ out) {
     const unsigned first = (blockIdx.x * kThreads + threadIdx.x) * 4u;
     if (first >= total) return;
     unsigned row = first / wide, col = first - row * wide;
@@ -66,7 +68,7 @@ __global__ __launch_bounds__(kThreads) void drop_self_grad_kernel(const float *_
     }
 #pragma unroll
     for (unsigned u = 0; u < 4; ++u) {
-        if (u < count && col > 0) vi[u] += g_narrow[first + u - row - 1];
+        if (u < count && col > 0) vi[u] += scale * g_narrow[first + u - row - 1];
         if (++col == wide) col = 0, ++row;
     }
     if (count == 4) {
@@ -402,8 +404,8 @@ using namespace hgc;
 
 extern "C" {
 
-int hgc_gravnet_drop_self(const int *d_idxs, const float *d_dist, int n_vert, int n_neigh, int *d_out_idxs,
-                          float *d_out_dist, hgc_stream_t stream) {
+int hgc_gravnet_drop_self_scaled(const int *d_idxs, const float *d_dist, int n_vert, int n_neigh, float scale, int *d_out_idxs,
+                                 float *d_out_dist, hgc_stream_t stream) {
     HGC_REQUIRE(n_vert >= 0 && n_neigh >= 2, "n_vert >= 0, n_neigh >= 2");
     HGC_REQUIRE((long long)n_vert * n_neigh < (1ll << 31), "n_vert * n_neigh must stay below 2^31");
     if (n_vert == 0) return HGC_OK;
@@ -411,12 +413,17 @@ int hgc_gravnet_drop_self(const int *d_idxs, const float *d_dist, int n_vert, in
     HGC_REQUIRE(aligned16({d_out_idxs, d_out_dist}), "outputs must lie on 16-byte boundaries");
     const unsigned total = (unsigned)n_vert * (unsigned)(n_neigh - 1);
     drop_self_kernel<<<ceil_div(total, 4 * kThreads), kThreads, 0, as_stream(stream)>>>(
-        d_idxs, d_dist, total, (unsigned)(n_neigh - 1), d_out_idxs, d_out_dist);
+        d_idxs, d_dist, total, (unsigned)(n_neigh - 1), scale, d_out_idxs, d_out_dist);
     return check_launch("gravnet_drop_self");
 }
 
-int hgc_gravnet_drop_self_grad(const float *d_grad_narrow, const float *d_grad_wide, int n_vert, int n_neigh,
-                               float *d_out_grad, hgc_stream_t stream) {
+int hgc_gravnet_drop_self(const int *d_idxs, const float *d_dist, int n_vert, int n_neigh, int *d_out_idxs,
+                          float *d_out_dist, hgc_stream_t stream) {
+    return hgc_gravnet_drop_self_scaled(d_idxs, d_dist, n_vert, n_neigh, 1.f, d_out_idxs, d_out_dist, stream);
+}
+
+int hgc_gravnet_drop_self_grad_scaled(const float *d_grad_narrow, const float *d_grad_wide, int n_vert, int n_neigh, float scale,
+                                      float *d_out_grad, hgc_stream_t stream) {
     HGC_REQUIRE(n_vert >= 0 && n_neigh >= 2, "n_vert >= 0, n_neigh >= 2");
     HGC_REQUIRE((long long)n_vert * n_neigh < (1ll << 31), "n_vert * n_neigh must stay below 2^31");
     if (n_vert == 0) return HGC_OK;
@@ -424,8 +431,13 @@ int hgc_gravnet_drop_self_grad(const float *d_grad_narrow, const float *d_grad_w
     HGC_REQUIRE(aligned16({d_grad_wide, d_out_grad}), "wide gradients must lie on 16-byte boundaries");
     const unsigned total = (unsigned)n_vert * (unsigned)n_neigh;
     drop_self_grad_kernel<<<ceil_div(total, 4 * kThreads), kThreads, 0, as_stream(stream)>>>(
-        d_grad_narrow, d_grad_wide, total, (unsigned)n_neigh, d_out_grad);
+        d_grad_narrow, d_grad_wide, total, (unsigned)n_neigh, scale, d_out_grad);
     return check_launch("gravnet_drop_self_grad");
+}
+
+int hgc_gravnet_drop_self_grad(const float *d_grad_narrow, const float *d_grad_wide, int n_vert, int n_neigh,
+                               float *d_out_grad, hgc_stream_t stream) {
+    return hgc_gravnet_drop_self_grad_scaled(d_grad_narrow, d_grad_wide, n_vert, n_neigh, 1.f, d_out_grad, stream);
 }
 
 size_t hgc_gravnet_radius_step_workspace_bytes(void) { return align_up(kRadiusBlocks * sizeof(MaxSum)); }

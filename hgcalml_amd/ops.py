@@ -705,9 +705,9 @@ def _aligned(t):
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
-@_op("gravnet_drop_self(Tensor indices, Tensor distances) -> (Tensor, Tensor)")
-def gravnet_drop_self(indices, distances):
-    """neighbour table and squared distances without their first column"""
+@_op("gravnet_drop_self(Tensor indices, Tensor distances, float scale=1.0) -> (Tensor, Tensor)")
+def gravnet_drop_self(indices, distances, scale=1.0):
+    """neighbour table and squared distances (times `scale`) without their first column"""
     dev = require_device(indices, distances)
     idx, d = i32(indices), f32(distances)
     n, k = idx.shape
@@ -715,12 +715,12 @@ def gravnet_drop_self(indices, distances):
         raise ValueError("gravnet_drop_self: indices and distances [N, K >= 2] expected")
     out_idx = torch.empty((n, k - 1), dtype=torch.int32, device=dev)
     out = torch.empty((n, k - 1), dtype=torch.float32, device=dev)
-    check(lib.hgc_gravnet_drop_self(p(idx), p(d), n, k, p(out_idx), p(out), stream()))
+    check(lib.hgc_gravnet_drop_self_scaled(p(idx), p(d), n, k, scale, p(out_idx), p(out), stream()))
     return out_idx, out
 
 
-@_op("gravnet_drop_self_grad(Tensor grad_narrow, Tensor? grad_wide) -> Tensor")
-def gravnet_drop_self_grad(grad_narrow, grad_wide):
+@_op("gravnet_drop_self_grad(Tensor grad_narrow, Tensor? grad_wide, float scale=1.0) -> Tensor")
+def gravnet_drop_self_grad(grad_narrow, grad_wide, scale=1.0):
     """gradient of gravnet_drop_self w.r.t. the distances, added to their own gradient (if there is one)"""
     dev = require_device(grad_narrow, grad_wide)
     narrow = f32(grad_narrow)
@@ -729,7 +729,7 @@ def gravnet_drop_self_grad(grad_narrow, grad_wide):
     if wide is not None and wide.shape != (n, k):
         raise ValueError("gravnet_drop_self_grad: gradients of shape [N, K - 1] and [N, K] expected")
     out = torch.empty((n, k), dtype=torch.float32, device=dev)
-    check(lib.hgc_gravnet_drop_self_grad(p(narrow), p(wide), n, k, p(out), stream()))
+    check(lib.hgc_gravnet_drop_self_grad_scaled(p(narrow), p(wide), n, k, scale, p(out), stream()))
     return out
 
 
@@ -1003,13 +1003,13 @@ def _(ccoords, dist, beta, no_condensation_mask, bins_flat, bin_splits, indices_
 
 
 @torch.library.register_fake("hgcalml::gravnet_drop_self")
-def _(indices, distances):
+def _(indices, distances, scale=1.0):
     n, k = indices.shape
     return _i32_like((n, k - 1), indices), _f32_like((n, k - 1), indices)
 
 
 @torch.library.register_fake("hgcalml::gravnet_drop_self_grad")
-def _(grad_narrow, grad_wide):
+def _(grad_narrow, grad_wide, scale=1.0):
     n, k = grad_narrow.shape
     return _f32_like((n, k + 1), grad_narrow)
 

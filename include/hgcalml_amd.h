@@ -581,11 +581,17 @@ int hgc_accumulate_knn_grad_whole_index(const float *d_grad_from_out_features, c
 /* Table and squared distances [n_vert, n_neigh] without column 0, the self
  * entry: outputs [n_vert, n_neigh - 1] on 16-byte boundaries. The gradient
  * w.r.t. the wide distances is that of the narrow ones moved up by a column
- * plus d_grad_wide (may be NULL: 0). */
+ * plus d_grad_wide (may be NULL: 0). The _scaled forms: the narrow distances are
+ * `scale` times the wide ones. */
 int hgc_gravnet_drop_self(const int *d_idxs, const float *d_dist, int n_vert, int n_neigh,
                           int *d_out_idxs, float *d_out_dist, hgc_stream_t stream);
 int hgc_gravnet_drop_self_grad(const float *d_grad_narrow, const float *d_grad_wide, int n_vert,
                                int n_neigh, float *d_out_grad, hgc_stream_t stream);
+
+int hgc_gravnet_drop_self_scaled(const int *d_idxs, const float *d_dist, int n_vert, int n_neigh,
+                                 float scale, int *d_out_idxs, float *d_out_dist, hgc_stream_t stream);
+int hgc_gravnet_drop_self_grad_scaled(const float *d_grad_narrow, const float *d_grad_wide, int n_vert,
+                                      int n_neigh, float scale, float *d_out_grad, hgc_stream_t stream);
 
 /* What update_dynamic_radius adds to the radius (GravNetLayersRagged.py:3180-3193):
  * 0.05 (u - radius), u = max(min(1.05 largest distance, 2), 2 mean distance) + 1e-3,

@@ -164,3 +164,17 @@ def test_blocks_that_are_left_alone(layers_taken):
     with torch.no_grad():
         layer(x, torch.tensor(X["row_splits"], dtype=torch.int32, device=DEV))
     assert layers_taken == [1]
+
+
+@pytest.mark.parametrize("n,k", [(1, 2), (700, 10), (333, 65)])
+def test_scaled_distances_without_the_self_column(n, k):
+    """the bits of the product by itself, both ways"""
+    from hgcalml_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    dist, narrow, wide = (torch.randn(n, c, device=DEV, generator=gen) for c in (k, k - 1, k))
+    idx = torch.randint(-1, n, (n, k), device=DEV, generator=gen, dtype=torch.int32)
+    out_idx, out = ops.gravnet_drop_self(idx, dist, 10.0)
+    assert torch.equal(out_idx, idx[:, 1:]) and torch.equal(out, 10.0 * dist[:, 1:])
+    moved = torch.nn.functional.pad(10.0 * narrow, (1, 0))
+    assert torch.equal(ops.gravnet_drop_self_grad(narrow, wide, 10.0), wide + moved)
+    assert torch.equal(ops.gravnet_drop_self_grad(narrow, None, 10.0), moved)
