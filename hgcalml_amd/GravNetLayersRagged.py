@@ -142,8 +142,11 @@ class _InputLayersFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w_features, bias, w_coords, relu):
         ctx.set_materialize_grads(False)
-        features = ops.gravnet_feature_layer(x, w_features, bias, relu)
+        # library products: their last bits decide which neighbours are near, largest and passed on at all
         coords = torch.nn.functional.linear(x, w_coords)
+        features = torch.nn.functional.linear(x, w_features, bias)
+        if relu:
+            features = features.relu_()
         ctx.save_for_backward(x, w_features, w_coords, features)
         ctx.relu = relu
         return features, coords, features.data, x.data

@@ -1,9 +1,11 @@
 // The dense layers of the GravNet block, rows in and rows out, with what stands around them in the same pass:
-//   input form        features = act(x Wf^T + b); the coordinates x Ws^T stay a library product, since their last bits decide
-//                     between neighbours at nearly equal distances
 //   output form       y = relu([mean - p | max - p | x] W^T + b), the joined rows kept for the weights' gradient on request
 //   output's gradient g where y > 0 times W: to the accumulation's rows, to p (minus both halves) and to x; the masked g kept
 //   input's gradient  (g1 + g2 where the features are > 0) Wf + g_coordinates Ws + g_x; the masked sum kept
+// The two first layers themselves stay library products: the last bits of coordinates decide between neighbours at nearly equal
+// distances, those of features between neighbours with nearly equal maxima and which side of 0 an activation falls on, and
+// single rows of the gradients change as a whole with that (by more than their root mean square in one step of ten, 150,000 and
+// 240,011 points; a pass of its own took 21 and 16 us for the features, the library and the activation 41 and 50).
 //
 // A contraction over at most a few hundred columns, for very many rows. Its bound is the float32 matrix instruction
 // (150,000 rows, 192 -> 128: 7.4 GFLOP, 47 us at its rate) or, for narrow layers, reading and writing the rows once.
@@ -17,11 +19,11 @@
 // (the ones it has twice count once), and behind the last row stands the last row again: no load or store is left out, so
 // none stands in a branch, which would make waiting for a load mean waiting for everything after it.
 // Measured next to the library products with join, activation, mask and sums as passes of their own, us: 150,000 rows, 64 inputs,
-// 64 features, 128 outputs: features 41 -> 21, output 156 -> 100, its gradient 171 -> 89, input's gradient 123 -> 40; 240,011 rows,
-// 48, 32, 96: 50 -> 16, 162 -> 73, 220 -> 83, 155 -> 36; a training step of the block 1976 -> 1741 and 2000 -> 1680, 2477
-// points 790 -> 594 (the host's time). What is left: the matrix instruction (61 % busy at 128 outputs) and the memory (the output layer without
-// its products 94). Error against 64 bits (2-norm, 150,000 rows): output 1.0e-7, library 1.5e-7. Tried and taken back: 8 waves
-// instead of 16 (output 108), weights' tiles multiplied onto the sum over all columns (error 2.1e-7), higher priority
+// 64 features, 128 outputs: output 156 -> 100, its gradient 171 -> 89, input's gradient 123 -> 40; 240,011 rows, 48, 32, 96: 162
+// -> 73, 220 -> 83, 155 -> 36. A training step of the block 1973 -> 1708 and 2001 -> 1661 (35 and 45 of it elsewhere), 2477
+// points 911 -> 668 (the host's time). What is left: the matrix instruction (61 % busy at 128 outputs) and the memory (the
+// output layer without its products 94). Error against 64 bits (2-norm, 150,000 rows): output 1.0e-7, library 1.5e-7. Tried and
+// taken back: 8 waves instead of 16 (output 108), one chain of products over all columns (error 2.1e-7), higher priority
 // while multiplying (level), whole ranges of rows per workgroup or XCD (108 to 127).
 #include <algorithm>
 
@@ -36,7 +38,7 @@ constexpr int kLdsBytes = 160 * 1024;
 
 typedef float vec4 __attribute__((ext_vector_type(4)));
 
-enum class Form { Input, Output, OutputGrad, InputGrad };
+enum class Form { Output, OutputGrad, InputGrad };
 
 struct DenseRows {
     const float *a0, *a1, *a2, *a3, *add;  // rows in
@@ -75,7 +77,6 @@ struct Part {  // of the input's columns
 
 template <Form FORM>
 __device__ __forceinline__ Part part_of(const DenseRows &p, int step) {
-    if constexpr (FORM == Form::Input) return {0, step * kStepCols, p.I};
     if constexpr (FORM == Form::OutputGrad) return {0, step * kStepCols, p.O};
     if constexpr (FORM == Form::InputGrad) return {0, step * kStepCols, p.F};
     const int index = step < p.steps0 ? 0 : step < p.steps1 ? 1 : 2;
@@ -89,9 +90,7 @@ __device__ __forceinline__ const float *weights_of(const DenseRows &p, const Par
     const int tiles_f = (p.F + kTile - 1) / kTile;
     auto column = [&](int tile, int width) { return first_of_four(tile * kTile + (c & ~3), width) + (c & 3); };
     pitch = 1;
-    if constexpr (FORM == Form::Input) {
-        return p.w0 + (size_t)column(tile, p.F) * p.I;
-    } else if constexpr (FORM == Form::Output) {
+    if constexpr (FORM == Form::Output) {
         return p.w0 + (size_t)column(tile, p.O) * (2 * p.F + p.I) + at.index * p.F;
     } else if constexpr (FORM == Form::OutputGrad) {  // tiles of both halves in turn, then those of x
         pitch = 2 * p.F + p.I;
@@ -102,17 +101,15 @@ __device__ __forceinline__ const float *weights_of(const DenseRows &p, const Par
     }
 }
 
-constexpr int sources(Form form) { return form == Form::Input ? 1 : form == Form::InputGrad ? 3 : 2; }
+constexpr int sources(Form form) { return form == Form::InputGrad ? 3 : 2; }
 
 template <int NSRC>
 struct Raw {
     vec4 v[NSRC];
 };
 
-// Steps requested while as many are multiplied: 64 columns where few tiles leave little work for a step, 32 otherwise.
-constexpr int steps_ahead(Form form, int tiles) {
-    return tiles <= 4 && sources(form) == 1 ? 4 : tiles >= 6 && sources(form) == 3 ? 1 : 2;
-}
+// Steps requested while as many are multiplied (three sources and many tiles: registers for one)
+constexpr int steps_ahead(Form form, int tiles) { return tiles >= 6 && sources(form) == 3 ? 1 : 2; }
 // 16 waves of 128 registers, or 12 of 168 for many tiles
 constexpr int most_waves(int tiles) { return tiles <= 8 ? 16 : 12; }
 
@@ -149,8 +146,8 @@ __global__ __launch_bounds__(most_waves(NT) *kWave) void dense_rows_kernel(const
         for (int u = 0; u < kAtOnce; ++u)
             if (first + u < pieces) s_w[(size_t)(first + u) * kWave + lane] = w[u];
     }
-    if constexpr (FORM == Form::Input || FORM == Form::Output) {
-        const int width = FORM == Form::Input ? p.F : p.O;
+    if constexpr (FORM == Form::Output) {
+        const int width = p.O;
         for (int i = threadIdx.x; i < NT * kTile; i += blockDim.x)
             s_bias[i] = p.bias[first_of_four(min(tile0 + i / kTile, p.tiles - 1) * kTile + (i & 12), width) + (i & 3)];
     }
@@ -180,9 +177,7 @@ __global__ __launch_bounds__(most_waves(NT) *kWave) void dense_rows_kernel(const
         for (int u = 0; u < U; ++u) {
             const Part part = part_of<FORM>(p, min(batch * U + u, p.steps - 1));
             const int col = first_of_four(part.col + 4 * k, part.width);
-            if constexpr (FORM == Form::Input) {
-                raw[u].v[0] = load4(at(p.a0, p.I, col));
-            } else if constexpr (FORM == Form::Output) {
+            if constexpr (FORM == Form::Output) {
                 const bool own = part.index < 2;
                 raw[u].v[0] = load4(at(own ? p.a0 + part.index * p.F : p.a2, own ? 2 * p.F : p.I, col));
                 raw[u].v[1] = load4(at(own ? p.a1 : p.a2, own ? p.F : p.I, col));
@@ -299,9 +294,7 @@ __global__ __launch_bounds__(most_waves(NT) *kWave) void dense_rows_kernel(const
         for (int t = 0; t < NT; ++t) {
             // (behind the last tile: that one again, weights and all)
             const int tile = min(tile0 + t, p.tiles - 1);
-            if constexpr (FORM == Form::Input) {
-                store4(p.o0 + row * p.F + column(tile, p.F), with_bias(t));
-            } else if constexpr (FORM == Form::Output) {
+            if constexpr (FORM == Form::Output) {
                 store4(p.o0 + row * p.O + column(tile, p.O), with_bias(t));
             } else if constexpr (FORM == Form::OutputGrad) {
                 if (tile0 + t < 2 * tiles_f) {
@@ -425,18 +418,6 @@ extern "C" {
 
 int hgc_gravnet_dense_covers(int n_feat, int n_x, int n_out, int n_coords) {
     return widths_fit(n_feat, n_x, n_out, n_coords);
-}
-
-int hgc_gravnet_feature_layer(const float *d_x, int n_vert, int n_x, const float *d_w, const float *d_bias, int n_feat,
-                              int relu, float *d_features, hgc_stream_t stream) {
-    HGC_REQUIRE(n_vert >= 0 && widths_fit(n_feat, n_x, 4, 1), "bad sizes");
-    if (n_vert == 0) return HGC_OK;
-    HGC_REQUIRE(d_x && d_w && d_bias && d_features, "null pointer");
-    DenseRows p{};
-    p.a0 = d_x, p.w0 = d_w, p.bias = d_bias, p.o0 = d_features;
-    p.n = n_vert, p.F = n_feat, p.I = n_x, p.relu = relu;
-    p.steps = steps_of(n_x);
-    return launch<Form::Input, false, false>(p, tiles_of(n_feat), as_stream(stream));
 }
 
 int hgc_gravnet_output_layer(const float *d_acc, const float *d_features, const float *d_x, int n_vert, int n_feat, int n_x,

@@ -833,19 +833,6 @@ def dense_weight_grad(grad, x):
     return weight, bias
 
 
-@_op("gravnet_feature_layer(Tensor x, Tensor weight, Tensor bias, bool relu) -> Tensor")
-def gravnet_feature_layer(x, weight, bias, relu):
-    """x W^T + b, with relu the relu of it: the features [N, F] that the block propagates"""
-    dev = require_device(x, weight, bias)
-    x, w, b = f32(x), f32(weight), f32(bias)
-    (n, i), f = x.shape, w.shape[0]
-    if w.shape != (f, i) or b.shape != (f,):
-        raise ValueError("gravnet_feature_layer: x [N, X], a weight [F, X] and a bias [F] expected")
-    features = torch.empty((n, f), dtype=torch.float32, device=dev)
-    check(lib.hgc_gravnet_feature_layer(p(x), n, i, p(w), p(b), f, int(relu), p(features), stream()))
-    return features
-
-
 @_op("gravnet_input_layers_grad(Tensor grad_features, Tensor? grad_features2, Tensor features, Tensor? grad_coords, "
      "Tensor? grad_x, Tensor w_features, Tensor w_coords, bool relu) -> (Tensor, Tensor)")
 def gravnet_input_layers_grad(grad_features, grad_features2, features, grad_coords, grad_x, w_features, w_coords, relu):
@@ -1054,11 +1041,6 @@ def _(grad, normalised, norm, n_neighbours):
 @torch.library.register_fake("hgcalml::sumw_distance_grad")
 def _(norm_grad, weights, indices, distance_grad):
     return None
-
-
-@torch.library.register_fake("hgcalml::gravnet_feature_layer")
-def _(x, weight, bias, relu):
-    return _f32_like((x.shape[0], weight.shape[0]), x)
 
 
 @torch.library.register_fake("hgcalml::gravnet_input_layers_grad")

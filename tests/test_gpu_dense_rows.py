@@ -1,5 +1,4 @@
-"""The GravNet block's dense layers as passes of the library (`hgc_gravnet_feature_layer`, `hgc_gravnet_output_layer` and
-their gradients) against the products in 64 bits, and which blocks take them."""
+"""The GravNet block's dense layers as passes of the library (`hgc_gravnet_output_layer` and the gradients of all three) against the products in 64 bits, and which blocks take them."""
 import pytest
 import torch
 
@@ -32,11 +31,7 @@ def test_passes(n, x_width, f, c, o):
     # x starts four bytes into its memory
     x = normal(n * x_width + 1)[1:].view(n, x_width)
     w_feat, bias, w_coords = normal(f, x_width), normal(f), normal(c, x_width)
-    for relu in (True, False):
-        feat, linear = (ops.gravnet_feature_layer(x, w_feat, bias, r) for r in (relu, False))
-        check(linear, [(x, w_feat)], bias)
-        assert torch.equal(feat, torch.relu(linear) if relu else linear)
-
+    feat = torch.relu(torch.nn.functional.linear(x, w_feat, bias))
     acc, w, b = normal(n, 2 * f), normal(o, 2 * f + x_width), normal(o)
     joined = torch.cat([acc - feat.repeat(1, 2), x], dim=1)
     out, kept = ops.gravnet_output_layer(acc, feat, x, w, b, True)
@@ -67,11 +62,17 @@ def test_non_finite_values_stay_in_their_rows():
     torch.manual_seed(3)
     x = torch.randn(37, 13, device=DEV)
     x[5, 12], x[20, 0] = float("nan"), float("inf")
-    w, b = torch.randn(10, 13, device=DEV), torch.randn(10, device=DEV)
-    want = torch.nn.functional.linear(x, w, b)
-    for got, ref in ((ops.gravnet_feature_layer(x, w, b, False), want), (ops.gravnet_feature_layer(x, w, b, True), torch.relu(want))):
-        assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(torch.isinf(got), torch.isinf(ref))
-        assert torch.isfinite(got[torch.arange(37, device=DEV) % 15 != 5]).all()
+    acc, feat = torch.randn(37, 20, device=DEV), torch.randn(37, 10, device=DEV)
+    acc[20, 3], feat[5, 9] = float("-inf"), float("nan")
+    w, b = torch.randn(18, 33, device=DEV), torch.randn(18, device=DEV)
+    out, joined = ops.gravnet_output_layer(acc, feat, x, w, b, True)
+    want = torch.relu(torch.nn.functional.linear(joined, w, b))
+    assert torch.equal(torch.isnan(out), torch.isnan(want)) and torch.equal(torch.isinf(out), torch.isinf(want))
+    assert torch.isfinite(out[torch.arange(37, device=DEV) % 15 != 5]).all()
+    # a result that is not a number passes its gradient on, as torch's relu does
+    g = torch.randn(37, 18, device=DEV)
+    masked = ops.gravnet_output_layer_grad(g, out, w, 10)[3]
+    assert torch.equal(masked, torch.ops.aten.threshold_backward(g, out, 0))
 
 
 @pytest.fixture
