@@ -142,7 +142,7 @@ class _InputLayersFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w_features, bias, w_coords, relu):
         ctx.set_materialize_grads(False)
-        # library products: their last bits decide which neighbours are near, largest and passed on at all
+        # library products: their last bits decide which neighbours are near, largest and passed on at all (dense_rows.hip)
         coords = torch.nn.functional.linear(x, w_coords)
         features = torch.nn.functional.linear(x, w_features, bias)
         if relu:
@@ -181,34 +181,39 @@ class _InputLayersFn(torch.autograd.Function):
 
 
 class _OutputLayerFn(torch.autograd.Function):
-    """relu of the block's last layer on joined = [accumulated - (features | features) | x], which the weight gradient
-    reads; its parts are kept for the derivative of that gradient"""
+    """relu of the block's last layer on joined = [accumulated - (features | features) | x], and joined itself: the weight
+    gradient reads it, and the derivative of that gradient comes back through it"""
 
     @staticmethod
-    def forward(ctx, accumulated, features, x, weight, bias, with_joined):
-        out, joined = ops.gravnet_output_layer(accumulated, features, x, weight, bias, with_joined)
-        ctx.save_for_backward(weight, joined, out, accumulated, features, x)
-        return out
+    def forward(ctx, accumulated, features, x, weight, bias):
+        ctx.set_materialize_grads(False)
+        joined = ops.gravnet_join(accumulated, features, x)
+        # (a library product too: its last bits decide which activations pass their gradient on)
+        out = torch.nn.functional.linear(joined, weight, bias).relu_()
+        ctx.n_features = features.shape[1]
+        ctx.save_for_backward(weight, out, joined if ctx.needs_input_grad[3] else None)
+        return out, joined
 
     @staticmethod
-    def backward(ctx, g):
-        weight, joined, out, accumulated, features, x = ctx.saved_tensors
-        f = features.shape[1]
-        want_w, want_b = ctx.needs_input_grad[3:5]
-        if torch.is_grad_enabled() or not any(ctx.needs_input_grad[:3]):
-            masked = torch.ops.aten.threshold_backward(g, out, 0).contiguous()
-            grad = masked @ weight
-            grads = grad[:, :2 * f], -grad[:, :f] - grad[:, f:2 * f], grad[:, 2 * f:]
-            if torch.is_grad_enabled() and want_w:
-                joined = torch.cat([accumulated - features.repeat(1, 2), x], dim=1)
-        else:
+    def backward(ctx, g, g_joined):
+        weight, out, joined = ctx.saved_tensors
+        f = ctx.n_features
+        wanted, (want_w, want_b) = ctx.needs_input_grad[:3], ctx.needs_input_grad[3:]
+        grads, masked = (None, None, None), None
+        if any(wanted) and g is not None and g_joined is None and not torch.is_grad_enabled():
             *grads, masked = ops.gravnet_output_layer_grad(g, out, weight, f)
+        else:  # as tensor operations: derivatives of the derivative, or no gradient of the rows
+            if g is not None:
+                masked = torch.ops.aten.threshold_backward(g, out, 0).contiguous()
+            if any(wanted) and (g is not None or g_joined is not None):
+                grad = g_joined if g is None else masked @ weight if g_joined is None else masked @ weight + g_joined
+                grads = grad[:, :2 * f], -grad[:, :f] - grad[:, f:2 * f], grad[:, 2 * f:]
         grad_w = grad_b = None
-        if want_w:
+        if masked is not None and want_w:
             grad_w, grad_b = _weight_and_bias_grad(masked, joined, want_b)
-        elif want_b:
+        elif masked is not None and want_b:
             grad_b = _sum_rows(masked)
-        return (*(t if want else None for t, want in zip(grads, ctx.needs_input_grad)), grad_w, grad_b if want_b else None, None)
+        return (*(t if want else None for t, want in zip(grads, wanted)), grad_w, grad_b if want_b else None)
 
 
 class TallLinear(nn.Linear):
@@ -347,8 +352,7 @@ class RaggedGravNet(nn.Module):
             nidx, ndist, sidx, sdist = self._neighbours(coordinates, row_splits, scale)
             accumulated = self._collect(features, nidx, ndist) if self.return_self else self.collect_neighbours(features, nidx, ndist)
             last = self.output_feature_transform
-            outfeats = _OutputLayerFn.apply(accumulated, features_again, x_again, last.weight, last.bias,
-                                            torch.is_grad_enabled() and last.weight.requires_grad)
+            outfeats, _ = _OutputLayerFn.apply(accumulated, features_again, x_again, last.weight, last.bias)
             return (outfeats, coordinates, sidx, sdist) if self.return_self else (outfeats, coordinates, nidx, ndist)
         coordinates = self.input_spatial_transform(x)
         neighbour_indices, distancesq, sidx, sdist = self.compute_neighbours_and_distancesq(coordinates, row_splits)

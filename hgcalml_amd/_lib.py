@@ -85,7 +85,6 @@ _SIGNATURES = {
     "hgc_dense_weight_grad_workspace_bytes": (_c_size, [ctypes.c_longlong] + [_c_int] * 2),
     "hgc_dense_weight_grad": (_c_int, [_ptr] * 2 + [ctypes.c_longlong] + [_c_int] * 2 + [_ptr] * 3 + [_c_size, _ptr]),
     "hgc_gravnet_dense_covers": (_c_int, [_c_int] * 4),
-    "hgc_gravnet_output_layer": (_c_int, [_ptr] * 3 + [_c_int] * 3 + [_ptr] * 2 + [_c_int] + [_ptr] * 3),
     "hgc_gravnet_output_layer_grad": (_c_int, [_ptr] * 2 + [_c_int] * 3 + [_ptr, _c_int] + [_ptr] * 5),
     "hgc_gravnet_input_layers_grad": (_c_int, [_ptr] * 5 + [_c_int] * 2 + [_ptr, _c_int, _ptr] + [_c_int] * 2 + [_ptr] * 3),
     "hgc_binned_assign_to_condensates_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int]),

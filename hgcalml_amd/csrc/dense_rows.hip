@@ -1,14 +1,15 @@
-// The dense layers of the GravNet block, rows in and rows out, with what stands around them in the same pass:
-//   output form       y = relu([mean - p | max - p | x] W^T + b), the joined rows kept for the weights' gradient on request
+// Gradients of the dense layers of the GravNet block, rows in and rows out, with what stands around them in the same pass:
 //   output's gradient g where y > 0 times W: to the accumulation's rows, to p (minus both halves) and to x; the masked g kept
+//                     (y = relu([mean - p | max - p | x] W^T + b))
 //   input's gradient  (g1 + g2 where the features are > 0) Wf + g_coordinates Ws + g_x; the masked sum kept
-// The two first layers themselves stay library products: the last bits of coordinates decide between neighbours at nearly equal
-// distances, those of features between neighbours with nearly equal maxima and which side of 0 an activation falls on, and
-// single rows of the gradients change as a whole with that (by more than their root mean square in one step of ten, 150,000 and
-// 240,011 points; a pass of its own took 21 and 16 us for the features, the library and the activation 41 and 50).
+// The three layers themselves are library products: the last bits of coordinates decide between neighbours at nearly equal
+// distances, those of features between neighbours with nearly equal maxima, and those in front of both activations which
+// gradients pass. With the last layer as a pass of its own about one activation of 20 million fell on the other side of 0, and single
+// rows of the gradients changed by up to 0.6 of their root mean square (10 of 34 steps by more than 0.01; none of them with the
+// library's product: 9e-6 at the most). It took 113 and 117 us in the steps below, join, product and activation 154 and 173.
 //
 // A contraction over at most a few hundred columns, for very many rows. Its bound is the float32 matrix instruction
-// (150,000 rows, 192 -> 128: 7.4 GFLOP, 47 us at its rate) or, for narrow layers, reading and writing the rows once.
+// (150,000 rows, 128 -> 192: 7.4 GFLOP, 47 us at its rate) or, for narrow layers, reading and writing the rows once.
 // The weights of a workgroup's columns lie in LDS for its whole life, in the order in which the instruction takes them (a
 // step of 16 columns of the input times 16 of the output is 64 lanes x 16 bytes, without bank conflicts), so nothing but
 // the first barrier keeps its waves together: each takes 16 rows at a time, streams them from memory with one batch of
@@ -18,13 +19,13 @@
 // stores 16 bytes. At the end of a width that is no multiple of four a lane moves back onto the row's last four columns
 // (the ones it has twice count once), and behind the last row stands the last row again: no load or store is left out, so
 // none stands in a branch, which would make waiting for a load mean waiting for everything after it.
-// Measured next to the library products with join, activation, mask and sums as passes of their own, us: 150,000 rows, 64 inputs,
-// 64 features, 128 outputs: output 156 -> 100, its gradient 171 -> 89, input's gradient 123 -> 40; 240,011 rows, 48, 32, 96: 162
-// -> 73, 220 -> 83, 155 -> 36. A training step of the block 1973 -> 1708 and 2001 -> 1661 (35 and 45 of it elsewhere), 2477
-// points 911 -> 668 (the host's time). What is left: the matrix instruction (61 % busy at 128 outputs) and the memory (the
-// output layer without its products 94). Error against 64 bits (2-norm, 150,000 rows): output 1.0e-7, library 1.5e-7. Tried and
-// taken back: 8 waves instead of 16 (output 108), one chain of products over all columns (error 2.1e-7), higher priority
-// while multiplying (level), whole ranges of rows per workgroup or XCD (108 to 127).
+// Measured next to the library products with mask, sums and the join's gradient as passes of their own, us, a gigabyte written
+// between calls (inputs come from memory): 150,000 rows, 64 inputs, 64 features, 128 outputs: output's gradient 197 -> 134, input's
+// 145 -> 80; 240,011 rows, 48, 32, 96: 248 -> 151, 173 -> 74; 20,000 rows, 64, 64, 128: 52 -> 30, 45 -> 17. In a training step of the block
+// the two take 122 and 52 us, and 135 and 48. The step 1973 -> 1759 and 1999 -> 1735 (35 and 45 of it elsewhere), 2477 points
+// 856 -> 730 (the host's time). Error against 64 bits (2-norm, 150,000 rows), here and library: gradient of the accumulated rows
+// 8.7e-8 and 1.5e-7, of the joined x the same, input's 5.6e-8 and 6.4e-8. Tried and taken back: 8 waves instead of 16, one chain of
+// products over all columns (twice the error), higher priority while multiplying, whole ranges of rows per workgroup or XCD.
 #include <algorithm>
 
 #include "hgc_common.hpp"
@@ -38,15 +39,15 @@ constexpr int kLdsBytes = 160 * 1024;
 
 typedef float vec4 __attribute__((ext_vector_type(4)));
 
-enum class Form { Output, OutputGrad, InputGrad };
+enum class Form { OutputGrad, InputGrad };
 
 struct DenseRows {
     const float *a0, *a1, *a2, *a3, *add;  // rows in
-    const float *w0, *w1, *bias;
-    float *o0, *o1, *o2, *side;            // rows out; side (may be null): the operand as it was multiplied
+    const float *w0, *w1;
+    float *o0, *o1, *o2, *masked;          // rows out; masked: the operand as it was multiplied
     long long n;
     int F, I, O, C;
-    int steps, steps0, steps1;             // of 16 input columns: all, up to the end of the first and of the second part
+    int steps;                             // of 16 input columns
     int tiles;                             // of 16 output columns, all of them
     int relu, two;
 };
@@ -57,8 +58,8 @@ __device__ __forceinline__ vec4 load4(const float *p) {
     return v;
 }
 
-// Past the caches: what is written here is read by other kernels, after more than the L2 holds. (150,000 rows, output layer
-// 109 -> 99 us, its gradient 112 -> 87; 240,011 rows, 96 of 112 columns: 107 -> 74 and 116 -> 83)
+// Past the caches: what is written here is read by other kernels, after more than the L2 holds. (Output's gradient, inputs in the
+// caches, 150,000 rows 112 -> 87 us; 240,011 rows, 96 of 112 columns: 116 -> 83)
 __device__ __forceinline__ void store4(float *p, const vec4 &v) {
     typedef vec4 vec4_any __attribute__((aligned(4)));
     __builtin_nontemporal_store(v, reinterpret_cast<vec4_any *>(p));
@@ -71,28 +72,16 @@ __device__ __forceinline__ float where_positive(float g, float y) { return y <= 
 // Columns in front of `col` are then held twice.
 __device__ __forceinline__ int first_of_four(int col, int width) { return min(col, width - 4); }
 
-struct Part {  // of the input's columns
-    int index, col, width;
-};
-
+// columns of a row that is multiplied
 template <Form FORM>
-__device__ __forceinline__ Part part_of(const DenseRows &p, int step) {
-    if constexpr (FORM == Form::OutputGrad) return {0, step * kStepCols, p.O};
-    if constexpr (FORM == Form::InputGrad) return {0, step * kStepCols, p.F};
-    const int index = step < p.steps0 ? 0 : step < p.steps1 ? 1 : 2;
-    const int before = index == 0 ? 0 : index == 1 ? p.steps0 : p.steps1;
-    return {index, (step - before) * kStepCols, index < 2 ? p.F : p.I};
-}
+__device__ __forceinline__ int width_in(const DenseRows &p) { return FORM == Form::OutputGrad ? p.O : p.F; }
 
 // first weight of output column c of tile `tile` and the distance of its weights for consecutive input columns
 template <Form FORM>
-__device__ __forceinline__ const float *weights_of(const DenseRows &p, const Part &at, int tile, int c, size_t &pitch) {
+__device__ __forceinline__ const float *weights_of(const DenseRows &p, int tile, int c, size_t &pitch) {
     const int tiles_f = (p.F + kTile - 1) / kTile;
     auto column = [&](int tile, int width) { return first_of_four(tile * kTile + (c & ~3), width) + (c & 3); };
-    pitch = 1;
-    if constexpr (FORM == Form::Output) {
-        return p.w0 + (size_t)column(tile, p.O) * (2 * p.F + p.I) + at.index * p.F;
-    } else if constexpr (FORM == Form::OutputGrad) {  // tiles of both halves in turn, then those of x
+    if constexpr (FORM == Form::OutputGrad) {  // tiles of both halves in turn, then those of x
         pitch = 2 * p.F + p.I;
         return tile < 2 * tiles_f ? p.w0 + (tile & 1) * p.F + column(tile >> 1, p.F) : p.w0 + 2 * p.F + column(tile - 2 * tiles_f, p.I);
     } else {
@@ -113,14 +102,14 @@ constexpr int steps_ahead(Form form, int tiles) { return tiles >= 6 && sources(f
 // 16 waves of 128 registers, or 12 of 168 for many tiles
 constexpr int most_waves(int tiles) { return tiles <= 8 ? 16 : 12; }
 
-// SIDE: the operand is kept. COORDS: the gradient of the coordinates takes part (at most four of them: one more step of the
-// instruction).
-template <Form FORM, int NT, bool SIDE, bool COORDS>
+// COORDS: the gradient of the coordinates takes part (at most four of them: one more step of the instruction).
+template <Form FORM, int NT, bool COORDS>
 __global__ __launch_bounds__(most_waves(NT) *kWave) void dense_rows_kernel(const DenseRows p) {
     constexpr int NSRC = sources(FORM), U = steps_ahead(FORM, NT);
+    const int width = width_in<FORM>(p);
     extern __shared__ __align__(16) float s_weights[];
     vec4 *const s_w = reinterpret_cast<vec4 *>(s_weights);
-    float *const s_bias = s_weights + (size_t)p.steps * NT * kWave * 4;  // or the weights of the coordinates
+    float *const s_coords = s_weights + (size_t)p.steps * NT * kWave * 4;  // weights of the coordinates
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_id(), l = lane & 15, k = lane >> 4;
     const int waves = blockDim.x / kWave, tile0 = blockIdx.y * NT;
     const int tiles_f = (p.F + kTile - 1) / kTile;
@@ -133,10 +122,9 @@ __global__ __launch_bounds__(most_waves(NT) *kWave) void dense_rows_kernel(const
 #pragma unroll
         for (int u = 0; u < kAtOnce; ++u) {
             const int i = min(first + u, pieces - 1), step = i / NT;
-            const Part at = part_of<FORM>(p, step);
-            const int wanted = at.col + 4 * k, col = first_of_four(wanted, at.width);
+            const int wanted = step * kStepCols + 4 * k, col = first_of_four(wanted, width);
             size_t pitch;
-            const float *from = weights_of<FORM>(p, at, min(tile0 + i - step * NT, p.tiles - 1), l, pitch);
+            const float *from = weights_of<FORM>(p, min(tile0 + i - step * NT, p.tiles - 1), l, pitch);
 #pragma unroll
             for (int e = 0; e < 4; ++e) w[u][e] = from[(col + e) * pitch];
 #pragma unroll
@@ -146,16 +134,11 @@ __global__ __launch_bounds__(most_waves(NT) *kWave) void dense_rows_kernel(const
         for (int u = 0; u < kAtOnce; ++u)
             if (first + u < pieces) s_w[(size_t)(first + u) * kWave + lane] = w[u];
     }
-    if constexpr (FORM == Form::Output) {
-        const int width = p.O;
-        for (int i = threadIdx.x; i < NT * kTile; i += blockDim.x)
-            s_bias[i] = p.bias[first_of_four(min(tile0 + i / kTile, p.tiles - 1) * kTile + (i & 12), width) + (i & 3)];
-    }
     if constexpr (COORDS) {  // lane: output column l, coordinate k
         for (int i = threadIdx.x; i < NT * kWave; i += blockDim.x) {
             const int c = i & 15, coord = (i >> 4) & 3;
             const int col = first_of_four(min(tile0 + i / kWave, p.tiles - 1) * kTile + (c & ~3), p.I) + (c & 3);
-            s_bias[i] = coord < p.C ? p.w1[(size_t)coord * p.I + col] : 0.f;
+            s_coords[i] = coord < p.C ? p.w1[(size_t)coord * p.I + col] : 0.f;
         }
     }
     __syncthreads();
@@ -175,20 +158,10 @@ __global__ __launch_bounds__(most_waves(NT) *kWave) void dense_rows_kernel(const
         auto at = [&](const float *from, int pitch, int first) { return from + task * kTile * pitch + (row * (unsigned)pitch + first); };
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const Part part = part_of<FORM>(p, min(batch * U + u, p.steps - 1));
-            const int col = first_of_four(part.col + 4 * k, part.width);
-            if constexpr (FORM == Form::Output) {
-                const bool own = part.index < 2;
-                raw[u].v[0] = load4(at(own ? p.a0 + part.index * p.F : p.a2, own ? 2 * p.F : p.I, col));
-                raw[u].v[1] = load4(at(own ? p.a1 : p.a2, own ? p.F : p.I, col));
-            } else if constexpr (FORM == Form::OutputGrad) {
-                raw[u].v[0] = load4(at(p.a0, p.O, col));
-                raw[u].v[1] = load4(at(p.a1, p.O, col));
-            } else {
-                raw[u].v[0] = load4(at(p.a0, p.F, col));
-                raw[u].v[1] = load4(at(p.a1, p.F, col));
-                raw[u].v[2] = load4(at(p.a2, p.F, col));
-            }
+            const int col = first_of_four(min(batch * U + u, p.steps - 1) * kStepCols + 4 * k, width);
+            raw[u].v[0] = load4(at(p.a0, width, col));
+            raw[u].v[1] = load4(at(p.a1, width, col));
+            if constexpr (FORM == Form::InputGrad) raw[u].v[2] = load4(at(p.a2, width, col));
         }
         if constexpr (COORDS) coord = *at(p.a3, p.C, min(k, p.C - 1));
         __builtin_amdgcn_sched_barrier(0);  // before what is multiplied meanwhile
@@ -205,24 +178,19 @@ __global__ __launch_bounds__(most_waves(NT) *kWave) void dense_rows_kernel(const
         vec4 a[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const Part part = part_of<FORM>(p, min(batch * U + u, p.steps - 1));
-            const int wanted = part.col + 4 * k, col = first_of_four(wanted, part.width);
+            const int first = min(batch * U + u, p.steps - 1) * kStepCols;
+            const int wanted = first + 4 * k, col = first_of_four(wanted, width);
             a[u] = raw[u].v[0];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                if constexpr (FORM == Form::Output) a[u][e] = part.index < 2 ? a[u][e] - raw[u].v[1][e] : a[u][e];
                 if constexpr (FORM == Form::OutputGrad) a[u][e] = where_positive(a[u][e], raw[u].v[1][e]);
                 if constexpr (FORM == Form::InputGrad) {
                     a[u][e] = p.two ? a[u][e] + raw[u].v[1][e] : a[u][e];
                     a[u][e] = p.relu ? where_positive(a[u][e], raw[u].v[2][e]) : a[u][e];
                 }
             }
-            if constexpr (SIDE) {
-                const int pitch = FORM == Form::Output ? 2 * p.F + p.I : FORM == Form::OutputGrad ? p.O : p.F;
-                const int first = FORM == Form::Output ? part.index * p.F : 0;
-                if (tile0 == 0) store4(p.side + task * kTile * pitch + (row * (unsigned)pitch + first + col), a[u]);
-            }
-            if (part.col + kStepCols > part.width) {
+            if (tile0 == 0) store4(p.masked + task * kTile * width + (row * (unsigned)width + col), a[u]);
+            if (first + kStepCols > width) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) a[u][e] = col + e < wanted ? 0.f : a[u][e];
             }
@@ -262,18 +230,8 @@ __global__ __launch_bounds__(most_waves(NT) *kWave) void dense_rows_kernel(const
         if constexpr (COORDS) {
 #pragma unroll
             for (int t = 0; t < NT; ++t)
-                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(s_bias[t * kWave + lane], k < p.C ? coord : 0.f, acc[t], 0, 0, 0);
+                acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(s_coords[t * kWave + lane], k < p.C ? coord : 0.f, acc[t], 0, 0, 0);
         }
-        auto with_bias = [&](int t) {
-            vec4 v = acc[t];
-            const vec4 b = *reinterpret_cast<const vec4 *>(s_bias + t * kTile + 4 * k);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                v[e] = v[e] + b[e];
-                v[e] = p.relu ? where_positive(v[e], v[e]) : v[e];
-            }
-            return v;
-        };
         auto column = [&](int tile, int width) { return first_of_four(tile * kTile + 4 * k, width); };
         if constexpr (FORM == Form::InputGrad) {
             if (p.add) {
@@ -294,9 +252,7 @@ __global__ __launch_bounds__(most_waves(NT) *kWave) void dense_rows_kernel(const
         for (int t = 0; t < NT; ++t) {
             // (behind the last tile: that one again, weights and all)
             const int tile = min(tile0 + t, p.tiles - 1);
-            if constexpr (FORM == Form::Output) {
-                store4(p.o0 + row * p.O + column(tile, p.O), with_bias(t));
-            } else if constexpr (FORM == Form::OutputGrad) {
+            if constexpr (FORM == Form::OutputGrad) {
                 if (tile0 + t < 2 * tiles_f) {
                     if (t % 2 == 0) {
                         const int col = column(tile >> 1, p.F);
@@ -350,7 +306,7 @@ bool make_plan(Form form, int steps, int tiles, bool coords, Plan &plan) {
         const int share = (tiles + chunks - 1) / chunks;
         for (int nt : offered) {
             if (nt < share || (pairs && nt % 2)) continue;
-            const size_t lds = (size_t)steps * nt * kWave * sizeof(vec4) + nt * (coords ? kWave : kTile) * sizeof(float);
+            const size_t lds = (size_t)steps * nt * kWave * sizeof(vec4) + (coords ? nt * kWave * sizeof(float) : 0);
             if (lds > kLdsBytes) break;
             plan.tiles = nt;
             plan.chunks = (tiles + nt - 1) / nt;
@@ -361,36 +317,36 @@ bool make_plan(Form form, int steps, int tiles, bool coords, Plan &plan) {
     return false;
 }
 
-template <Form FORM, int NT, bool SIDE, bool COORDS>
+template <Form FORM, int NT, bool COORDS>
 int launch_kernel(const DenseRows &p, const Plan &plan, hipStream_t s) {
     const long long tasks = (p.n + kTile - 1) / kTile;
     const int groups = (int)std::min<long long>(tasks, std::max(1, kGroups / plan.chunks));
     const long long each = (tasks + groups - 1) / groups;
     const int waves = (int)std::min<long long>(most_waves(NT), (each + 3) / 4 * 4);
     if (plan.lds > 64 * 1024) {
-        HGC_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&dense_rows_kernel<FORM, NT, SIDE, COORDS>),
+        HGC_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&dense_rows_kernel<FORM, NT, COORDS>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes));
     }
-    dense_rows_kernel<FORM, NT, SIDE, COORDS><<<dim3(groups, plan.chunks), waves * kWave, plan.lds, s>>>(p);
+    dense_rows_kernel<FORM, NT, COORDS><<<dim3(groups, plan.chunks), waves * kWave, plan.lds, s>>>(p);
     return check_launch("dense_rows_kernel");
 }
 
-template <Form FORM, bool SIDE, bool COORDS>
+template <Form FORM, bool COORDS>
 int launch(DenseRows p, int tiles, hipStream_t s) {
     constexpr bool kPairs = FORM == Form::OutputGrad;
     Plan plan;
     p.tiles = tiles;
     if (!make_plan(FORM, p.steps, tiles, COORDS, plan)) return fail(HGC_ERR_INVALID_ARGUMENT, "layer too wide");
     switch (plan.tiles) {
-        case 1: if constexpr (!kPairs) return launch_kernel<FORM, 1, SIDE, COORDS>(p, plan, s); break;
-        case 2: return launch_kernel<FORM, 2, SIDE, COORDS>(p, plan, s);
-        case 3: if constexpr (!kPairs) return launch_kernel<FORM, 3, SIDE, COORDS>(p, plan, s); break;
-        case 4: return launch_kernel<FORM, 4, SIDE, COORDS>(p, plan, s);
-        case 5: if constexpr (!kPairs) return launch_kernel<FORM, 5, SIDE, COORDS>(p, plan, s); break;
-        case 6: return launch_kernel<FORM, 6, SIDE, COORDS>(p, plan, s);
-        case 8: return launch_kernel<FORM, 8, SIDE, COORDS>(p, plan, s);
-        case 10: return launch_kernel<FORM, 10, SIDE, COORDS>(p, plan, s);
-        case 12: return launch_kernel<FORM, 12, SIDE, COORDS>(p, plan, s);
+        case 1: if constexpr (!kPairs) return launch_kernel<FORM, 1, COORDS>(p, plan, s); break;
+        case 2: return launch_kernel<FORM, 2, COORDS>(p, plan, s);
+        case 3: if constexpr (!kPairs) return launch_kernel<FORM, 3, COORDS>(p, plan, s); break;
+        case 4: return launch_kernel<FORM, 4, COORDS>(p, plan, s);
+        case 5: if constexpr (!kPairs) return launch_kernel<FORM, 5, COORDS>(p, plan, s); break;
+        case 6: return launch_kernel<FORM, 6, COORDS>(p, plan, s);
+        case 8: return launch_kernel<FORM, 8, COORDS>(p, plan, s);
+        case 10: return launch_kernel<FORM, 10, COORDS>(p, plan, s);
+        case 12: return launch_kernel<FORM, 12, COORDS>(p, plan, s);
     }
     return fail(HGC_ERR_INVALID_ARGUMENT, "no kernel for this number of tiles");
 }
@@ -399,9 +355,10 @@ int steps_of(int width) { return ceil_div(width, kStepCols); }
 int tiles_of(int width) { return ceil_div(width, kTile); }
 
 // Rows of four columns and more, so that four in sequence exist; up to four coordinates, one step of the instruction. Wider
-// layers are the library product's, whose workgroups share what they read of the weights (240,000 rows, 352 -> 512 with
-// everything around it 1264 here, 983 there; 60,000 rows, 384 -> 256 170 and 154, the four passes of the block together
-// 368 and 463).
+// layers are the library product's, whose workgroups share what they read of the weights. Up to the widest both gradients together
+// are faster here, us here / library, inputs from memory: last layer 384 -> 256 20,000 rows 90 / 142, 60,000 218 / 315, 240,000
+// 727 / 1138; 512 (256 of them x) -> 256 60,000 278 / 427, 150,000 627 / 1062, 240,000 959 / 1552; 512 (412 of them x) -> 255
+// 60,000 397 / 557, 240,000 1502 / 2047; 512 -> 64 240,000 607 / 1036.
 constexpr int kWidestIn = 512, kWidestOut = 256;
 
 bool widths_fit(int f, int x, int o, int c) {
@@ -420,20 +377,6 @@ int hgc_gravnet_dense_covers(int n_feat, int n_x, int n_out, int n_coords) {
     return widths_fit(n_feat, n_x, n_out, n_coords);
 }
 
-int hgc_gravnet_output_layer(const float *d_acc, const float *d_features, const float *d_x, int n_vert, int n_feat, int n_x,
-                             const float *d_w, const float *d_bias, int n_out, float *d_out, float *d_joined,
-                             hgc_stream_t stream) {
-    HGC_REQUIRE(n_vert >= 0 && widths_fit(n_feat, n_x, n_out, 1), "bad sizes");
-    if (n_vert == 0) return HGC_OK;
-    HGC_REQUIRE(d_acc && d_features && d_x && d_w && d_bias && d_out, "null pointer");
-    DenseRows p{};
-    p.a0 = d_acc, p.a1 = d_features, p.a2 = d_x, p.w0 = d_w, p.bias = d_bias, p.o0 = d_out, p.side = d_joined;
-    p.n = n_vert, p.F = n_feat, p.I = n_x, p.O = n_out, p.relu = 1;
-    p.steps0 = steps_of(n_feat), p.steps1 = 2 * p.steps0, p.steps = p.steps1 + steps_of(n_x);
-    return d_joined ? launch<Form::Output, true, false>(p, tiles_of(n_out), as_stream(stream))
-                    : launch<Form::Output, false, false>(p, tiles_of(n_out), as_stream(stream));
-}
-
 int hgc_gravnet_output_layer_grad(const float *d_grad, const float *d_out, int n_vert, int n_feat, int n_x, const float *d_w,
                                   int n_out, float *d_masked, float *d_grad_acc, float *d_grad_features, float *d_grad_x,
                                   hgc_stream_t stream) {
@@ -441,10 +384,10 @@ int hgc_gravnet_output_layer_grad(const float *d_grad, const float *d_out, int n
     if (n_vert == 0) return HGC_OK;
     HGC_REQUIRE(d_grad && d_out && d_w && d_masked && d_grad_acc && d_grad_features && d_grad_x, "null pointer");
     DenseRows p{};
-    p.a0 = d_grad, p.a1 = d_out, p.w0 = d_w, p.side = d_masked, p.o0 = d_grad_acc, p.o1 = d_grad_features, p.o2 = d_grad_x;
-    p.n = n_vert, p.F = n_feat, p.I = n_x, p.O = n_out, p.relu = 1;
+    p.a0 = d_grad, p.a1 = d_out, p.w0 = d_w, p.masked = d_masked, p.o0 = d_grad_acc, p.o1 = d_grad_features, p.o2 = d_grad_x;
+    p.n = n_vert, p.F = n_feat, p.I = n_x, p.O = n_out;
     p.steps = steps_of(n_out);
-    return launch<Form::OutputGrad, true, false>(p, 2 * tiles_of(n_feat) + tiles_of(n_x), as_stream(stream));
+    return launch<Form::OutputGrad, false>(p, 2 * tiles_of(n_feat) + tiles_of(n_x), as_stream(stream));
 }
 
 int hgc_gravnet_input_layers_grad(const float *d_grad_features, const float *d_grad_features2, const float *d_features,
@@ -458,11 +401,11 @@ int hgc_gravnet_input_layers_grad(const float *d_grad_features, const float *d_g
     DenseRows p{};
     p.a0 = d_grad_features, p.a1 = d_grad_features2 ? d_grad_features2 : d_grad_features, p.a2 = relu ? d_features : d_grad_features;
     p.a3 = d_grad_coords, p.add = d_grad_x, p.two = d_grad_features2 != nullptr;
-    p.w0 = d_w_feat, p.w1 = d_w_coords, p.side = d_masked, p.o0 = d_grad_in;
+    p.w0 = d_w_feat, p.w1 = d_w_coords, p.masked = d_masked, p.o0 = d_grad_in;
     p.n = n_vert, p.F = n_feat, p.I = n_x, p.C = n_coords, p.relu = relu;
     p.steps = steps_of(n_feat);
-    return d_grad_coords ? launch<Form::InputGrad, true, true>(p, tiles_of(n_x), as_stream(stream))
-                         : launch<Form::InputGrad, true, false>(p, tiles_of(n_x), as_stream(stream));
+    return d_grad_coords ? launch<Form::InputGrad, true>(p, tiles_of(n_x), as_stream(stream))
+                         : launch<Form::InputGrad, false>(p, tiles_of(n_x), as_stream(stream));
 }
 
 }  // extern "C"

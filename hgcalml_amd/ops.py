@@ -851,27 +851,10 @@ def gravnet_input_layers_grad(grad_features, grad_features2, features, grad_coor
     return grad_in, masked
 
 
-@_op("gravnet_output_layer(Tensor accumulated, Tensor features, Tensor x, Tensor weight, Tensor bias, bool with_joined) "
-     "-> (Tensor, Tensor)")
-def gravnet_output_layer(accumulated, features, x, weight, bias, with_joined):
-    """(relu(joined W^T + b), joined = gravnet_join(accumulated, features, x) if asked for, else empty)"""
-    dev = require_device(accumulated, features, x, weight, bias)
-    acc, feat, x, w, b = f32(accumulated), f32(features), f32(x), f32(weight), f32(bias)
-    n, f = feat.shape
-    i, o = x.shape[1], w.shape[0]
-    if acc.shape != (n, 2 * f) or x.shape != (n, i) or w.shape != (o, 2 * f + i) or b.shape != (o,):
-        raise ValueError("gravnet_output_layer: [N, 2F], [N, F], [N, X], a weight [O, 2F + X] and a bias [O] expected")
-    out = torch.empty((n, o), dtype=torch.float32, device=dev)
-    joined = torch.empty((n, 2 * f + i) if with_joined else (0,), dtype=torch.float32, device=dev)
-    check(lib.hgc_gravnet_output_layer(p(acc), p(feat), p(x), n, f, i, p(w), p(b), o, p(out), p(joined) if with_joined else None,
-                                       stream()))
-    return out, joined
-
-
 @_op("gravnet_output_layer_grad(Tensor grad, Tensor out, Tensor weight, int n_features) -> (Tensor, Tensor, Tensor, Tensor)")
 def gravnet_output_layer_grad(grad, out, weight, n_features):
-    """gradients w.r.t. accumulated [N, 2F], features [N, F] and x [N, X] of gravnet_output_layer, and the gradient in
-    front of its activation [N, O]"""
+    """out = relu(gravnet_join(accumulated, features, x) W^T + b): gradients w.r.t. accumulated [N, 2F], features [N, F] and
+    x [N, X], and the gradient in front of the activation [N, O]"""
     dev = require_device(grad, out, weight)
     g, y, w = f32(grad), f32(out), f32(weight)
     (n, o), f, i = y.shape, n_features, w.shape[1] - 2 * n_features
@@ -1046,12 +1029,6 @@ def _(norm_grad, weights, indices, distance_grad):
 @torch.library.register_fake("hgcalml::gravnet_input_layers_grad")
 def _(grad_features, grad_features2, features, grad_coords, grad_x, w_features, w_coords, relu):
     return _f32_like((features.shape[0], w_features.shape[1]), features), _f32_like(features.shape, features)
-
-
-@torch.library.register_fake("hgcalml::gravnet_output_layer")
-def _(accumulated, features, x, weight, bias, with_joined):
-    n = x.shape[0]
-    return _f32_like((n, weight.shape[0]), x), _f32_like((n, weight.shape[1]) if with_joined else (0,), x)
 
 
 @torch.library.register_fake("hgcalml::gravnet_output_layer_grad")

@@ -652,11 +652,10 @@ int hgc_dense_weight_grad(const float *d_grad, const float *d_x, long long n_row
                           int n_in, float *d_weight_grad, float *d_bias_grad, void *workspace,
                           size_t workspace_bytes, hgc_stream_t stream);
 
-/* The dense layers of the block, row-major matrices of n_vert rows, weights
+/* Gradients of the block's dense layers, row-major matrices of n_vert rows, weights
  * [out, in], each with what stands around it in one pass (float32 products and sums).
- *   output layer:  d_out [., n_out] = max(j W^T + bias, 0), j = the rows of hgc_gravnet_join,
- *                  left in d_joined [., 2 n_feat + n_x] unless that is NULL
- *   its gradient:  m = d_grad where d_out > 0, to d_masked; m W to
+ *   output layer d_out [., n_out] = max(j W^T + bias, 0), j = the rows of hgc_gravnet_join:
+ *                  m = d_grad where d_out > 0, to d_masked; m W to
  *                  d_grad_acc, d_grad_features and d_grad_x as in hgc_gravnet_join_grad
  *   gradient of the features x W_f^T + bias and the coordinates x W_c^T: m = d_grad_features + d_grad_features2 (may be NULL), with relu
  *                  where d_features > 0, to d_masked; d_grad_in = m W_f
@@ -665,9 +664,6 @@ int hgc_dense_weight_grad(const float *d_grad, const float *d_x, long long n_row
  * 256, n_coords 1 to 4). x needs no alignment beyond that of float.
  * No counterpart in the reference (Keras does it). */
 int hgc_gravnet_dense_covers(int n_feat, int n_x, int n_out, int n_coords);
-int hgc_gravnet_output_layer(const float *d_acc, const float *d_features, const float *d_x, int n_vert,
-                             int n_feat, int n_x, const float *d_w, const float *d_bias, int n_out,
-                             float *d_out, float *d_joined, hgc_stream_t stream);
 int hgc_gravnet_output_layer_grad(const float *d_grad, const float *d_out, int n_vert, int n_feat,
                                   int n_x, const float *d_w, int n_out, float *d_masked,
                                   float *d_grad_acc, float *d_grad_features, float *d_grad_x,

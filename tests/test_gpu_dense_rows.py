@@ -1,4 +1,7 @@
-"""The GravNet block's dense layers as passes of the library (`hgc_gravnet_output_layer` and the gradients of all three) against the products in 64 bits, and which blocks take them."""
+"""The gradients of the GravNet block's dense layers as passes of the library against the products in 64 bits, and which blocks take
+them."""
+import types
+
 import pytest
 import torch
 
@@ -33,15 +36,7 @@ def test_passes(n, x_width, f, c, o):
     w_feat, bias, w_coords = normal(f, x_width), normal(f), normal(c, x_width)
     feat = torch.relu(torch.nn.functional.linear(x, w_feat, bias))
     acc, w, b = normal(n, 2 * f), normal(o, 2 * f + x_width), normal(o)
-    joined = torch.cat([acc - feat.repeat(1, 2), x], dim=1)
-    out, kept = ops.gravnet_output_layer(acc, feat, x, w, b, True)
-    again, none = ops.gravnet_output_layer(acc, feat, x, w, b, False)
-    assert torch.equal(kept, joined) and torch.equal(out, again) and none.numel() == 0
-    # max(., 0) moves no two numbers apart: the bound of the sum holds for it too
-    want = joined.double() @ w.double().t() + b.double()
-    size = joined.double().abs() @ w.double().abs().t() + b.double().abs()
-    assert ((out.double() - want.clamp_min(0)).abs() <= (2 * f + x_width + 2) * 2.0 ** -24 * size).all() and (out >= 0).all()
-
+    out = torch.relu(torch.nn.functional.linear(ops.gravnet_join(acc, feat, x), w, b))
     g = normal(n, o)
     g_acc, g_feat, g_x, masked = ops.gravnet_output_layer_grad(g, out, w, f)
     assert torch.equal(masked, torch.where(out > 0, g, torch.zeros_like(g)))
@@ -65,21 +60,23 @@ def test_non_finite_values_stay_in_their_rows():
     acc, feat = torch.randn(37, 20, device=DEV), torch.randn(37, 10, device=DEV)
     acc[20, 3], feat[5, 9] = float("-inf"), float("nan")
     w, b = torch.randn(18, 33, device=DEV), torch.randn(18, device=DEV)
-    out, joined = ops.gravnet_output_layer(acc, feat, x, w, b, True)
-    want = torch.relu(torch.nn.functional.linear(joined, w, b))
-    assert torch.equal(torch.isnan(out), torch.isnan(want)) and torch.equal(torch.isinf(out), torch.isinf(want))
-    assert torch.isfinite(out[torch.arange(37, device=DEV) % 15 != 5]).all()
+    out = torch.relu(torch.nn.functional.linear(ops.gravnet_join(acc, feat, x), w, b))
+    assert torch.isnan(out).any()
     # a result that is not a number passes its gradient on, as torch's relu does
     g = torch.randn(37, 18, device=DEV)
-    masked = ops.gravnet_output_layer_grad(g, out, w, 10)[3]
-    assert torch.equal(masked, torch.ops.aten.threshold_backward(g, out, 0))
+    g[30, 17], g[31, 0] = float("nan"), float("-inf")
+    *grads, masked = ops.gravnet_output_layer_grad(g, out, w, 10)
+    want = torch.ops.aten.threshold_backward(g, out, 0)
+    assert torch.equal(masked.nan_to_num(7.0, 8.0, 9.0), want.nan_to_num(7.0, 8.0, 9.0))
+    for grad, part in zip(grads, (w[:, :20], w[:, :10] + w[:, 10:20], w[:, 20:])):
+        assert torch.equal(torch.isfinite(grad), torch.isfinite(want @ part))
 
 
 @pytest.fixture
 def layers_taken(monkeypatch):
-    from hgcalml_amd import ops
-    seen, real = [], ops.gravnet_output_layer
-    monkeypatch.setattr(ops, "gravnet_output_layer", lambda *args: seen.append(1) or real(*args))
+    from hgcalml_amd import GravNetLayersRagged as module
+    seen, real = [], module._InputLayersFn
+    monkeypatch.setattr(module, "_InputLayersFn", types.SimpleNamespace(apply=lambda *args: seen.append(1) or real.apply(*args)))
     return seen
 
 
@@ -101,10 +98,10 @@ def step(layer, x, create_graph=False, second=False):
     if not second:
         loss = loss + (dist * torch.linspace(0, 1, dist.numel(), device=DEV).view(dist.shape)).sum()
     grads = torch.autograd.grad(loss, wanted, create_graph=create_graph)
-    if second:  # the last layer's weight gradient once more, with respect to that weight and its bias
-        last = layer.output_feature_transform
+    if second:  # the last layer's weight gradient once more, with respect to that weight and its bias and what is in front of them
+        last, first = layer.output_feature_transform, layer.input_feature_transform
         at = [i for i, t in enumerate(wanted) if t is last.weight][0]
-        grads = torch.autograd.grad((grads[at] * grads[at]).sum(), [last.weight, last.bias])
+        grads = torch.autograd.grad((grads[at] * grads[at]).sum(), [last.weight, last.bias, first.weight, first.bias, x])
     return [out.detach()] + [g.detach() for g in grads]
 
 
@@ -127,6 +124,30 @@ def test_block_with_parts_frozen(frozen, x_grad, layers_taken, monkeypatch):
     monkeypatch.setattr(type(layer), "_layers_in_one_pass", lambda self, x: False)
     agree(got, step(layer, x))
     assert layers_taken == [1]
+
+
+@pytest.mark.parametrize("activation", ["relu", "linear"])
+def test_results_are_those_of_the_layers_one_by_one(activation, layers_taken, monkeypatch):
+    """Bit for bit: every activation then lets the same gradients pass, and those differ by the order of their sums alone, 400 terms
+    of float32 at the most in a row (400 * 2^-24 = 2.4e-5 of the terms' sizes, which a sum of the largest row's size is made of)."""
+    from hgcalml_amd import RaggedGravNet
+    torch.manual_seed(5)
+    layer = RaggedGravNet(64, 16, 3, 128, 64, feature_activation=activation).to(DEV)
+    x = torch.randn(60000, 64, device=DEV, requires_grad=True)
+    rs = torch.tensor([0, 60000], dtype=torch.int32, device=DEV)
+    weight = torch.randn(60000, 128, device=DEV)
+
+    def once():
+        layer.dynamic_radius.fill_(1.0)
+        results = layer(x, rs)
+        return results, torch.autograd.grad((results[0] * weight).sum(), [x] + list(layer.parameters()))
+    (results, grads), taken = once(), list(layers_taken)
+    monkeypatch.setattr(type(layer), "_layers_in_one_pass", lambda self, x: False)
+    one_by_one, want = once()
+    assert taken == layers_taken == [1]
+    assert all(torch.equal(a, b) for a, b in zip(results, one_by_one))
+    for a, b in zip(grads, want):
+        assert (a - b).abs().max() <= 2.4e-5 * b.abs().max()
 
 
 @pytest.mark.parametrize("second", [False, True])
