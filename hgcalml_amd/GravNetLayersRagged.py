@@ -319,6 +319,8 @@ class RaggedGravNet(nn.Module):
     def _layers_in_one_pass(self, x):
         """Whether the dense layers run as the library's passes: the block as it is here, its layers and activation
         without hooks or replacements, so that nobody waits for their calls, and tensors that the passes take."""
+        if torch.compiler.is_compiling():  # (asked first: a compiler traces this, but not the looks at hooks and dictionaries)
+            return False
         if type(self) is not RaggedGravNet or not self.__dict__.keys().isdisjoint(_REPLACEABLE) or not x.is_contiguous():
             return False
         first, spatial, last = self.input_feature_transform, self.input_spatial_transform, self.output_feature_transform
@@ -338,7 +340,7 @@ class RaggedGravNet(nn.Module):
         f, i, o, c = first.weight.shape[0], x.shape[1], last.weight.shape[0], spatial.weight.shape[0]
         if first.weight.shape[1] != i or spatial.weight.shape[1] != i or last.weight.shape[1] != 2 * f + i:
             return False  # (the layers themselves say what is wrong)
-        return not (torch.is_autocast_enabled("cuda") or torch.compiler.is_compiling() or x.shape[0] >= 1 << 31) and bool(
+        return not (torch.is_autocast_enabled("cuda") or x.shape[0] >= 1 << 31) and bool(
             ops.lib.hgc_gravnet_dense_covers(f, i, o, c))
 
     def forward(self, x, row_splits):
