@@ -232,6 +232,9 @@ _ACTIVATIONS = {None: nn.Identity, "linear": nn.Identity, "relu": nn.ReLU, "elu"
 
 _DISTANCE_SCALE = 10.0  # neighbours are weighted by exp(-10 d^2)
 _REPLACEABLE = {"compute_neighbours_and_distancesq", "collect_neighbours", "create_output_features", "update_dynamic_radius"}
+# what the layers in one pass stand for: with something else in its place (on the class, too) they run one by one
+_OWN_LAYER = {TallLinear: TallLinear.forward}
+_OWN_ACTIVATIONS = {cls: cls.forward for cls in (nn.ReLU, nn.Identity)}
 
 
 class RaggedGravNet(nn.Module):
@@ -324,14 +327,12 @@ class RaggedGravNet(nn.Module):
         if type(self) is not RaggedGravNet or not self.__dict__.keys().isdisjoint(_REPLACEABLE) or not x.is_contiguous():
             return False
         first, spatial, last = self.input_feature_transform, self.input_spatial_transform, self.output_feature_transform
-        if type(self.feature_activation) not in (nn.ReLU, nn.Identity) or _has_any_global_hook():
+        if _has_any_global_hook() or any(getattr(RaggedGravNet, name) is not method for name, method in _OWN_METHODS):
             return False
-        for module in (first, spatial, last, self.feature_activation):
-            if (module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks or
-                    "forward" in module.__dict__):
+        for module, known in ((first, _OWN_LAYER), (spatial, _OWN_LAYER), (last, _OWN_LAYER), (self.feature_activation, _OWN_ACTIVATIONS)):
+            if (known.get(type(module)) is not type(module).forward or "forward" in module.__dict__ or module._forward_hooks or
+                    module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks):
                 return False
-        if not all(type(layer) is TallLinear for layer in (first, spatial, last)):
-            return False
         weights = first.weight, first.bias, spatial.weight, last.weight, last.bias
         if any(w is None for w in weights) or spatial.bias is not None or not _library_takes(x, *weights):
             return False
@@ -362,3 +363,6 @@ class RaggedGravNet(nn.Module):
         if self.return_self:
             neighbour_indices, distancesq = sidx, sdist
         return outfeats, coordinates, neighbour_indices, distancesq
+
+
+_OWN_METHODS = [(name, getattr(RaggedGravNet, name)) for name in sorted(_REPLACEABLE)]
