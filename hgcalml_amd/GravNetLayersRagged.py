@@ -149,7 +149,12 @@ class _InputLayersFn(torch.autograd.Function):
             features = features.relu_()
         ctx.save_for_backward(x, w_features, w_coords, features)
         ctx.relu = relu
-        return features, coords, features.data, x.data
+        outputs = features, coords, features.data, x.data
+        # an output that depends on nothing that wants a gradient wants none either: what follows is spared its part of it
+        want_x, want_wf, want_b, want_wc, _ = ctx.needs_input_grad
+        wanted = want_x or want_wf or want_b, want_x or want_wc, want_x or want_wf or want_b, want_x
+        ctx.mark_non_differentiable(*(t for t, want in zip(outputs, wanted) if not want))
+        return outputs
 
     @staticmethod
     def backward(ctx, g_features, g_coords, g_features2, g_x):

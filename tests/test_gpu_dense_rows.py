@@ -150,6 +150,33 @@ def test_results_are_those_of_the_layers_one_by_one(activation, layers_taken, mo
         assert (a - b).abs().max() <= 2.4e-5 * b.abs().max()
 
 
+@pytest.mark.parametrize("frozen", [(), ("input_spatial_transform.weight",), ("input_feature_transform.weight", "input_feature_transform.bias"),
+                                    ("input_feature_transform.weight", "input_feature_transform.bias", "input_spatial_transform.weight")])
+@pytest.mark.parametrize("x_grad", [True, False])
+@pytest.mark.parametrize("return_self", [True, False])
+def test_frozen_parts_ask_for_no_gradient(frozen, x_grad, return_self, layers_taken, monkeypatch):
+    """which results carry a gradient, and which gradients of search and accumulation a step forms: those of the layers one by one"""
+    from hgcalml_amd import ops
+    layer = block(return_self=return_self)
+    for name, weight in layer.named_parameters():
+        weight.requires_grad_(name not in frozen)
+    x = torch.randn(700, 13, device=DEV, requires_grad=x_grad)
+    rs = torch.tensor(X["row_splits"], dtype=torch.int32, device=DEV)
+    calls = []
+    for name in ("gravnet_drop_self_grad", "accumulate_gradient_index"):
+        monkeypatch.setattr(ops, name, lambda *args, name=name, real=getattr(ops, name): calls.append(name) or real(*args))
+
+    def once():
+        calls.clear()
+        results = layer(x, rs)
+        results[0].sum().backward()
+        return [t.requires_grad for t in results], list(calls)
+    got, taken = once(), list(layers_taken)
+    monkeypatch.setattr(type(layer), "_layers_in_one_pass", lambda self, x: False)
+    assert got == once() and taken == layers_taken == [1]
+    assert got[0][0] and got[0][1] == (x_grad or "input_spatial_transform.weight" not in frozen)
+
+
 @pytest.mark.parametrize("second", [False, True])
 def test_derivative_of_the_derivative(second, layers_taken, monkeypatch):
     layer = block()
