@@ -421,20 +421,33 @@ bool accumulate_grad_rows_covers(int n_feat, int n_neigh, bool mean_and_max, boo
 // The weight gradients of the targets in flight are 4-byte writes into the rows of everything that names them. Where those
 // rows, with the gradient rows and slots that are gathered, are more than an XCD's L2 holds, lines leave it before they are
 // whole and are written several times (fabric traffic five times the compulsory one at a million vertices, F = 128, window
-// +-2000). There the values leave in the order of the lists, in whole lines, and a pass moves them to their slots. us of the
-// gradient, scattered / in list order, banded tables of window +-2000: a million vertices, K = 64, F = 128 4612 / 4076, F = 64
-// 2700 / 2573, K = 24, F = 128 2454 / 2258; 300,000, K = 64, F = 128 1414 / 1219; 100,000 359 / 353; 20,000 87 / 93; window
-// +-1000, a million, K = 64, F = 128 3773 / 3912; +-300 3546 / 3761; tables of a search in bin order, 300,000 vertices, K = 40, F
-// = 128 907 / 1091. So the host asks for the size (asking and moving nothing costs 10 to 15 us) and leaves tables with a processing
-// order as they are, and the device looks at how far apart the vertices of a list are. (A mean alone gathers half as much.)
+// +-2000). In the order of the lists the values leave in whole lines, and a pass moves them to their slots. Whether that pays
+// depends on how far apart the vertices of a list are; us of the gradient, slot by slot / in list order:
+//   span of the rows           table
+//   up to 2.6 MB   slower      a million, K = 64, F = 128, banded +-1000 3773 / 3912, +-300 3546 / 3761
+//   3.8 to 10 MB   faster      the same, +-1500 4318 / 3910, +-2000 4602 / 3985, +-3000 5127 / 4612, +-4000 6105 / 5966; K = 24, F = 64, +-4000 1680 /
+//                              1412, +-8000 2067 / 1996; 300,000, K = 64, F = 128, +-2000 1417 / 1216; 410,000, K = 40, F = 100, +-4000 1613 / 1492;
+//                              a search's table, hits ordered by a coordinate, K = 40, F = 128 1280 / 1273, a million, K = 64 4387 / 4100
+//   16 to 50 MB    slower      a million, K = 64, F = 128, +-6000 7358 / 7577, +-16000 8400 / 9018; K = 24, F = 64, +-16000 2420 / 2582; 300,000,
+//                              K = 64, F = 128, +-16000 2560 / 2805; search tables, hits in no order, 16 events of 410,000, K = 40, F = 128 2350 / 2426,
+//                              32 events of a million, K = 64 8249 / 8439
+//   beyond         slower      where all rows are up to 540 MB, twice the Infinity Cache: 300,000, K = 64, F = 128, +-32000 2869 / 3032; targets drawn at
+//                              random, 300,000, K = 64, F = 64 1808 / 1946, F = 128 2589 / 2812, 500,000, F = 64 2954 / 3318; a search's table of one event of
+//                              300,000, K = 64, F = 128 2592 / 2824; level: random, 410,000, K = 40, F = 128 2725 / 2726, 800,000, K = 24, F = 64 2352 / 2318
+//   beyond 79 MB   faster      where they are 670 MB and more: a million, K = 64, F = 128, +-32000 13385 / 11575, random 12771 / 11156; K = 24, F = 64, +-64000
+//                              3826 / 3384, random 3242 / 2950; random, 500,000, K = 64, F = 128 5263 / 4785, 700,000, K = 24, F = 128 3783 / 3482
+// So the host asks for the size (100,000, +-2000 359 / 353, 20,000 87 / 93; asking and moving nothing costs 10 to 15 us) and leaves tables with a
+// processing order as they are (300,000 vertices, K = 40, F = 128 907 / 1091), and the device looks at the span. (A mean alone gathers
+// half as much.)
 constexpr int kSpanSamples = 1024;
-constexpr long long kSpanBytes = 3ll << 20;  // of the 4 MB of an XCD
+constexpr float kSpanNear = 3 << 20, kSpanFar = 12 << 20, kSpanWhole = 64 << 20;  // bytes; an XCD's L2 has 4 MB
+constexpr long long kRowsWhole = 600ll << 20;
 
 static bool list_order_may_pay(int n_vert, int n_feat, int n_neigh, bool mean_and_max) {
     return mean_and_max && (long long)n_vert * n_neigh >= 16000000 && n_neigh >= 24 && n_feat >= 64;
 }
 
-// *scattered = whether the vertices between the first and the last one that name a target span more than kSpanBytes, on average
+// *scattered = whether list order pays by the span of the rows between the first and the last vertex that name a target, on average
 __global__ __launch_bounds__(kSpanSamples) void list_span_kernel(const int *__restrict__ inv_off, const int *__restrict__ inv_slots,
                                                                  int n_vert, int K, int row_bytes, int *__restrict__ scattered) {
     __shared__ float s_span[kSpanSamples / kWave];
@@ -446,7 +459,8 @@ __global__ __launch_bounds__(kSpanSamples) void list_span_kernel(const int *__re
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int i = 1; i < kSpanSamples / kWave; ++i) span += s_span[i];
-        *scattered = span * (1.f / kSpanSamples) * (float)row_bytes > (float)kSpanBytes;
+        const float bytes = span * (1.f / kSpanSamples) * (float)row_bytes;
+        *scattered = (bytes > kSpanNear && bytes <= kSpanFar) || (bytes > kSpanWhole && (long long)n_vert * row_bytes >= kRowsWhole);
     }
 }
 

@@ -54,3 +54,43 @@ def test_both_ways_give_the_same_bits(n, k, f, window, listed, mean_and_max):
         assert torch.equal(gw, gw_one) or not quotients == 0 and torch.allclose(gw, gw_one, rtol=1e-4, atol=1e-6)
         assert torch.equal(gx, gx_one)
         assert (gw[table < 0] == 0).all()
+
+
+# near lists, lists beyond an XCD's L2, and those far beyond it in tables that fit the cache behind it and that do not
+@pytest.mark.parametrize("n,k,f,window,listed", [(250000, 64, 64, 100, False), (250000, 64, 64, 2000, True), (250000, 64, 64, 3300, True),
+                                                 (250000, 64, 64, 20000, False), (250000, 64, 64, None, False), (400013, 40, 100, 2000, True),
+                                                 (400013, 40, 100, 20000, False), (950000, 24, 64, 16000, False), (950000, 24, 64, None, True)])
+def test_which_tables_take_which_way(n, k, f, window, listed):
+    """read out of the scratch memory: the device's answer and the list behind the quotients. A list that starts off a 16-byte boundary
+    goes slot by slot, with the quotients, and has the same bits."""
+    from hgcalml_amd import ops
+    from hgcalml_amd._lib import check, lib, p, stream, workspace
+    gen = torch.Generator(device=DEV).manual_seed(n + k)
+    if window is None:
+        table = torch.randint(0, n, (n, k), device=DEV, generator=gen, dtype=torch.int32)
+    else:
+        stratum = 2 * window // k
+        off = torch.arange(k, device=DEV, dtype=torch.int32) * stratum - window
+        rows = torch.arange(n, device=DEV, dtype=torch.int32)[:, None]
+        table = (rows + off + torch.randint(0, stratum, (n, k), device=DEV, generator=gen, dtype=torch.int32)) % n
+    table[::11, k - 2:] = -1
+    dist, feat, g = (torch.rand(*shape, device=DEV, generator=gen) for shape in ((n, k), (n, f), (n, 2 * f)))
+    _, arg, slots, w = torch.ops.hgcalml.accumulate_knn_exp_slots(dist, feat, table, 0, True)
+    off, inv = ops.inverse_neighbour_index(table)
+    need = lib.hgc_accumulate_knn_grad_scratch_bytes(n, k, f, 1)
+    list_at, flag_at = (need - 256 - n * k * 4) // 256 * 256, need - 256
+    moved = torch.empty(inv.numel() + 4, dtype=torch.int32, device=DEV)
+    results = []
+    for shift in (0, 1):
+        at = moved[shift:shift + inv.numel()]
+        at.copy_(inv)
+        ws = workspace(need, DEV)
+        ws.fill_(0x5a)
+        gw, gx = torch.full((n, k), 7.0, device=DEV), torch.empty(n, f, device=DEV)
+        check(lib.hgc_accumulate_knn_grad_scratch(p(g), p(w), p(feat), p(arg), p(slots), p(table), p(off), p(at), None, p(gw), p(gx), n,
+                                                  k, f, 2 * f, 1, 1, p(ws), need, stream()))
+        untouched = bool((ws[list_at:flag_at] == 0x5a).all())
+        flag = ws[flag_at:flag_at + 4].view(torch.int32).item()
+        assert (flag, untouched) == ((0x5a5a5a5a, True) if shift else (int(listed), not listed))
+        results.append((gw, gx))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
