@@ -37,6 +37,7 @@ int launch_accumulate_grad_fused(const float *g, const float *w, const float *fe
 // accumulate_grad_rows.hip: rows of 16 to 128 features; returns 1 when the shape is not covered. gw == nullptr:
 // feature gradient only. negate: gw receives -(gradient * w). scratch may be null.
 size_t accumulate_grad_rows_scratch_bytes(int n_vert, int n_feat, int n_neigh, bool mean_and_max, float divisor);
+size_t accumulate_grad_rows_quotient_bytes(int n_vert, int n_feat, int n_neigh, bool mean_and_max, float divisor);
 bool accumulate_grad_rows_covers(int n_feat, int n_neigh, bool mean_and_max, bool slots, unsigned long long g_bytes);
 int launch_accumulate_grad_rows(const float *g, const float *w, const float *feat, const unsigned char *maxslot,
                                 const int *inv_off, const int *inv_slots, float *gw, float *gfeat, int n_vert, int K, int F,
@@ -1383,7 +1384,7 @@ int hgc_accumulate_knn_grad_scratch(const float *d_grad_from_out_features, const
                                     int weights_are_exp, void *scratch, size_t scratch_bytes, hgc_stream_t stream) {
     HGC_REQUIRE(n_vert <= 0 || (d_out_grad_distances && d_out_grad_features), "null pointer");
     if (scratch && (!aligned256(scratch) ||
-                    scratch_bytes < hgc_accumulate_knn_grad_scratch_bytes(n_vert, n_neigh, n_feat, mean_and_max)))
+                    scratch_bytes < accumulate_grad_rows_quotient_bytes(n_vert, n_feat, n_neigh, mean_and_max != 0, (float)n_neigh)))
         return fail(HGC_ERR_WORKSPACE, "accumulate_knn_grad_scratch: scratch memory misaligned or too small");
     return accumulate_gradient(d_grad_from_out_features, d_distances, d_feat, d_max_feat_indices, d_max_slots,
                                d_neigh_indices, d_inv_offsets, d_inv_slots, d_out_grad_distances, d_out_grad_features,
@@ -1407,7 +1408,7 @@ int hgc_accumulate_knn_grad_whole_index(const float *d_grad_from_out_features, c
     HGC_REQUIRE(d_grad_from_out_features && d_distances && d_feat && d_inv_offsets && d_inv_slots &&
                     d_out_grad_distances && d_out_grad_features && (d_max_slots || !mean_and_max), "null pointer");
     if (scratch && (!aligned256(scratch) ||
-                    scratch_bytes < hgc_accumulate_knn_grad_scratch_bytes(n_vert, n_neigh, n_feat, mean_and_max)))
+                    scratch_bytes < accumulate_grad_rows_quotient_bytes(n_vert, n_feat, n_neigh, mean_and_max != 0, (float)n_neigh)))
         return fail(HGC_ERR_WORKSPACE, "accumulate_knn_grad_whole_index: scratch memory misaligned or too small");
     return launch_accumulate_grad_rows(d_grad_from_out_features, d_distances, d_feat, mean_and_max ? d_max_slots : nullptr,
                                        d_inv_offsets, d_inv_slots, d_out_grad_distances, d_out_grad_features, n_vert, n_neigh,

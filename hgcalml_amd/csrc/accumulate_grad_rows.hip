@@ -464,22 +464,29 @@ __global__ __launch_bounds__(kSpanSamples) void list_span_kernel(const int *__re
     }
 }
 
-static size_t quotient_bytes(int n_vert, int n_feat, float divisor) {
+static bool scratch_covers(int n_vert, int n_feat, int n_neigh, bool mean_and_max) {
+    const unsigned long long n = (unsigned long long)std::max(n_vert, 0) * std::max(n_feat, 0) * sizeof(float);
+    return accumulate_grad_rows_covers(n_feat, n_neigh, mean_and_max, true, n * (mean_and_max ? 2 : 1));
+}
+
+size_t accumulate_grad_rows_quotient_bytes(int n_vert, int n_feat, int n_neigh, bool mean_and_max, float divisor) {
+    if (!scratch_covers(n_vert, n_feat, n_neigh, mean_and_max)) return 0;
     if (divisor == (float)(int)divisor && is_pow2((int)divisor)) return 0;
-    return align_up((size_t)n_vert * n_feat * sizeof(float));
+    return align_up((size_t)std::max(n_vert, 0) * n_feat * sizeof(float));
 }
 
 size_t accumulate_grad_rows_scratch_bytes(int n_vert, int n_feat, int n_neigh, bool mean_and_max, float divisor) {
-    const unsigned long long n = (unsigned long long)std::max(n_vert, 0) * std::max(n_feat, 0) * sizeof(float);
-    if (!accumulate_grad_rows_covers(n_feat, n_neigh, mean_and_max, true, n * (mean_and_max ? 2 : 1))) return 0;
-    return quotient_bytes(std::max(n_vert, 0), n_feat, divisor) +
-           (list_order_may_pay(n_vert, n_feat, n_neigh, mean_and_max) ? align_up((size_t)n_vert * n_neigh * sizeof(float)) + align_up(sizeof(int)) : 0);
+    const size_t quotients = accumulate_grad_rows_quotient_bytes(n_vert, n_feat, n_neigh, mean_and_max, divisor);
+    if (!scratch_covers(n_vert, n_feat, n_neigh, mean_and_max) || !list_order_may_pay(n_vert, n_feat, n_neigh, mean_and_max)) return quotients;
+    return quotients + align_up((size_t)n_vert * n_neigh * sizeof(float)) + align_up(sizeof(int));
 }
 
-// Returns 1 where the shape is not covered. gw == nullptr: feature gradient only (mean only). scratch
-// (accumulate_grad_rows_scratch_bytes, may be null) holds the quotients g / divisor where the divisor is
-// no power of two: N F divides in a pass of their own instead of N K F inside the gather
-// (150,000 vertices, K = 40, F = 64: 287 -> 262 us).
+// Returns 1 where the shape is not covered. gw == nullptr: feature gradient only (mean only). scratch (may be null)
+// holds, where there is room for them,
+//   the quotients g / divisor where the divisor is no power of two (accumulate_grad_rows_quotient_bytes): N F divides in a
+//   pass of their own instead of N K F inside the gather (150,000 vertices, K = 40, F = 64: 287 -> 262 us);
+//   behind them the weight gradients in list order and whether they leave so (accumulate_grad_rows_scratch_bytes, see
+//   list_order_may_pay), for an index without `skip`, no processing order and inv_slots on a 16-byte boundary.
 int launch_accumulate_grad_rows(const float *g, const float *w, const float *feat, const unsigned char *maxslot,
                                 const int *inv_off, const int *inv_slots, float *gw, float *gfeat, int n_vert, int K, int F,
                                 int g_cols, bool mean_and_max, const int *order, float divisor, bool negate, int skip,
@@ -490,12 +497,13 @@ int launch_accumulate_grad_rows(const float *g, const float *w, const float *fea
     GradRows p;
     Scale scale = kDivide;
     p.g = g;
+    const size_t quotient_bytes = accumulate_grad_rows_quotient_bytes(n_vert, F, K, mean_and_max, divisor);
     const bool room = scratch && scratch_bytes >= accumulate_grad_rows_scratch_bytes(n_vert, F, K, mean_and_max, divisor);
     p.gw_list = nullptr;
     p.scattered = nullptr;
     // (the list is read four entries at a time)
     if (room && want_w && skip == 0 && !order && list_order_may_pay(n_vert, F, K, mean_and_max) && (reinterpret_cast<uintptr_t>(inv_slots) & 15u) == 0) {
-        char *const behind = static_cast<char *>(scratch) + quotient_bytes(n_vert, F, divisor);
+        char *const behind = static_cast<char *>(scratch) + quotient_bytes;
         int *const scattered = reinterpret_cast<int *>(behind + align_up((size_t)n_vert * K * sizeof(float)));
         p.gw_list = reinterpret_cast<float *>(behind);
         p.scattered = scattered;
@@ -505,7 +513,7 @@ int launch_accumulate_grad_rows(const float *g, const float *w, const float *fea
     }
     if (divisor == (float)(int)divisor && is_pow2((int)divisor)) {
         scale = kPow2;
-    } else if (room) {
+    } else if (scratch && scratch_bytes >= quotient_bytes) {
         scale = kScaled;
         const long long total = (long long)n_vert * F;
         divide_mean_half_kernel<<<ceil_div(total, 256), 256, 0, s>>>(g, static_cast<float *>(scratch), total, F, g_cols, divisor);

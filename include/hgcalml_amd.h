@@ -410,12 +410,19 @@ int hgc_accumulate_knn_grad_records(const float *d_grad_from_out_features, const
                                     int n_moments, int mean_and_max,
                                     void *workspace, size_t workspace_bytes, hgc_stream_t stream);
 
-/* hgc_accumulate_knn_grad_slots with scratch memory (may be NULL) for the
- * quotients g / n_neigh, n_vert * n_feat floats, where n_neigh is no power of
- * two and n_feat is 16..128 (the query returns 0 elsewhere, with mean_and_max
- * also beyond 254 neighbours, and for gradient matrices beyond 32-bit offsets):
- * one pass of n_vert * n_feat divides instead of one divide per gathered
- * element. Same bits either way. With
+/* hgc_accumulate_knn_grad_slots with scratch memory (may be NULL) in two parts,
+ * both for n_feat 16..128 (the query returns 0 elsewhere, with mean_and_max also
+ * beyond 254 neighbours, and for gradient matrices beyond 32-bit offsets):
+ *   where n_neigh is no power of two, the quotients g / n_neigh, n_vert * n_feat
+ *   floats: one pass of divides instead of one divide per gathered element;
+ *   with mean_and_max, n_vert * n_neigh >= 16,000,000, n_neigh >= 24 and
+ *   n_feat >= 64, n_vert * n_neigh floats and one int (each part rounded up to
+ *   256 bytes): the weight gradients of large tables whose lists reach far are
+ *   written in the order of d_inv_slots and moved to their slots. Not used with a
+ *   d_vertex_order or a d_inv_slots that is on no 16-byte boundary.
+ * Scratch that holds the first part alone is used for that (less is
+ * HGC_ERR_WORKSPACE). The feature gradient has the same bits whatever there is
+ * of it, and the weight gradient has them with and without the second part. With
  * weights_are_exp the weights are exp(-d) and d_out_grad_distances receives the
  * gradient w.r.t. d, -(gradient w.r.t. the weight * weight), the bits of
  * hgc_exp_neg_grad behind this call (outputs and d_distances then on 16-byte

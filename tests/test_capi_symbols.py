@@ -130,6 +130,27 @@ def test_scratch_of_the_accumulation_gradient(capi):
     assert f(5000000, 40, 128, 1) == 0 and f(5000000, 40, 128, 0) == 5000000 * 128 * 4   # rows beyond 32-bit offsets
 
 
+def test_scratch_of_the_weight_gradients_in_list_order(capi):
+    """from 16 million slots, 24 neighbours and 64 features on, with the maximum, one float per slot and an int behind the
+    quotients; a buffer that holds the quotients alone is taken, less is not (what is missing after that are only pointers)"""
+    f, call = capi.hgc_accumulate_knn_grad_scratch_bytes, capi.hgc_accumulate_knn_grad_scratch
+    f.restype, f.argtypes = ctypes.c_size_t, [ctypes.c_int] * 4
+    call.argtypes = [ctypes.c_void_p] * 11 + [ctypes.c_int] * 6 + [ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+
+    def up(n):
+        return (n + 255) // 256 * 256
+    at = ctypes.c_void_p(256)  # (an address that nothing looks at: each call ends before)
+    for n, k, feat, listed in ((250000, 64, 64, True), (249999, 64, 64, False), (400013, 40, 100, True), (700000, 23, 64, False),
+                               (300000, 60, 63, False), (666667, 24, 64, True)):
+        quotients = 0 if k & (k - 1) == 0 else up(n * feat * 4)
+        assert f(n, k, feat, 0) == quotients
+        assert f(n, k, feat, 1) == quotients + (up(n * k * 4) + 256 if listed else 0)
+        for size, code in ((quotients, -1), (quotients - 1, -2)):
+            if size >= 0:
+                rc = call(*[None] * 9, at, at, n, k, feat, 2 * feat, 1, 0, at, size, None)
+                assert rc == code, (n, k, feat, size, rc)
+
+
 def test_settings_are_per_thread(capi):
     """the status word, the choice of the kNN grid and the last error text belong to the thread that set
     them: another thread sees the initial state, and what it sets does not leak back"""

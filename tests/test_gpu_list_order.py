@@ -94,3 +94,28 @@ def test_which_tables_take_which_way(n, k, f, window, listed):
         assert (flag, untouched) == ((0x5a5a5a5a, True) if shift else (int(listed), not listed))
         results.append((gw, gx))
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("n,k,f", [(250000, 64, 64), (400013, 40, 100)])
+def test_scratch_of_the_quotients_alone(n, k, f):
+    """slot by slot, with the same bits"""
+    from hgcalml_amd import ops
+    from hgcalml_amd._lib import check, lib, p, stream, workspace
+    gen = torch.Generator(device=DEV).manual_seed(n)
+    rows = torch.arange(n, device=DEV, dtype=torch.int32)[:, None]
+    table = (rows + torch.arange(k, device=DEV, dtype=torch.int32) * (4000 // k) - 2000) % n
+    w, feat, g = (torch.rand(*shape, device=DEV, generator=gen) for shape in ((n, k), (n, f), (n, 2 * f)))
+    _, arg, slots = torch.ops.hgcalml.accumulate_knn_slots(w, feat, table, 0, True)
+    off, inv = ops.inverse_neighbour_index(table)
+    full = lib.hgc_accumulate_knn_grad_scratch_bytes(n, k, f, 1)
+    quotients = 0 if k & (k - 1) == 0 else (n * f * 4 + 255) // 256 * 256
+    results = []
+    for size in (full, quotients):
+        ws = workspace(full, DEV)
+        ws.fill_(0x5a)
+        gw, gx = torch.empty(n, k, device=DEV), torch.empty(n, f, device=DEV)
+        check(lib.hgc_accumulate_knn_grad_scratch(p(g), p(w), p(feat), p(arg), p(slots), p(table), p(off), p(inv), None, p(gw), p(gx),
+                                                  n, k, f, 2 * f, 1, 0, p(ws), size, stream()))
+        assert bool((ws[quotients:] == 0x5a).all()) == (size < full)
+        results.append((gw, gx))
+    assert all(torch.equal(a, b) for a, b in zip(*results))
