@@ -53,6 +53,7 @@ _SIGNATURES = {
     "hgc_accumulate_knn_grad_records_pays": (_c_int, [_c_int] * 4),
     "hgc_accumulate_knn_grad_records": (_c_int, [_ptr] * 11 + [_c_int] * 6 + [_ptr, _c_size, _ptr]),
     "hgc_accumulate_knn_grad_scratch_bytes": (_c_size, [_c_int] * 4),
+    "hgc_accumulate_knn_grad_quotient_bytes": (_c_size, [_c_int] * 4),
     "hgc_accumulate_knn_grad_scratch": (_c_int, [_ptr] * 11 + [_c_int] * 6 + [_ptr, _c_size, _ptr]),
     "hgc_accumulate_knn_grad_whole_index_covers": (_c_int, [_c_int] * 4),
     "hgc_accumulate_knn_grad_whole_index": (_c_int, [_ptr] * 9 + [_c_int] * 6 + [_ptr, _c_size, _ptr]),

@@ -1376,6 +1376,10 @@ size_t hgc_accumulate_knn_grad_scratch_bytes(int n_vert, int n_neigh, int n_feat
     return accumulate_grad_rows_scratch_bytes(n_vert, n_feat, n_neigh, mean_and_max != 0, (float)n_neigh);
 }
 
+size_t hgc_accumulate_knn_grad_quotient_bytes(int n_vert, int n_neigh, int n_feat, int mean_and_max) {
+    return accumulate_grad_rows_quotient_bytes(n_vert, n_feat, n_neigh, mean_and_max != 0, (float)n_neigh);
+}
+
 int hgc_accumulate_knn_grad_scratch(const float *d_grad_from_out_features, const float *d_distances, const float *d_feat,
                                     const int *d_max_feat_indices, const unsigned char *d_max_slots,
                                     const int *d_neigh_indices, const int *d_inv_offsets, const int *d_inv_slots,
@@ -1384,7 +1388,7 @@ int hgc_accumulate_knn_grad_scratch(const float *d_grad_from_out_features, const
                                     int weights_are_exp, void *scratch, size_t scratch_bytes, hgc_stream_t stream) {
     HGC_REQUIRE(n_vert <= 0 || (d_out_grad_distances && d_out_grad_features), "null pointer");
     if (scratch && (!aligned256(scratch) ||
-                    scratch_bytes < accumulate_grad_rows_quotient_bytes(n_vert, n_feat, n_neigh, mean_and_max != 0, (float)n_neigh)))
+                    scratch_bytes < hgc_accumulate_knn_grad_quotient_bytes(n_vert, n_neigh, n_feat, mean_and_max)))
         return fail(HGC_ERR_WORKSPACE, "accumulate_knn_grad_scratch: scratch memory misaligned or too small");
     return accumulate_gradient(d_grad_from_out_features, d_distances, d_feat, d_max_feat_indices, d_max_slots,
                                d_neigh_indices, d_inv_offsets, d_inv_slots, d_out_grad_distances, d_out_grad_features,
@@ -1408,7 +1412,7 @@ int hgc_accumulate_knn_grad_whole_index(const float *d_grad_from_out_features, c
     HGC_REQUIRE(d_grad_from_out_features && d_distances && d_feat && d_inv_offsets && d_inv_slots &&
                     d_out_grad_distances && d_out_grad_features && (d_max_slots || !mean_and_max), "null pointer");
     if (scratch && (!aligned256(scratch) ||
-                    scratch_bytes < accumulate_grad_rows_quotient_bytes(n_vert, n_feat, n_neigh, mean_and_max != 0, (float)n_neigh)))
+                    scratch_bytes < hgc_accumulate_knn_grad_quotient_bytes(n_vert, n_neigh, n_feat, mean_and_max)))
         return fail(HGC_ERR_WORKSPACE, "accumulate_knn_grad_whole_index: scratch memory misaligned or too small");
     return launch_accumulate_grad_rows(d_grad_from_out_features, d_distances, d_feat, mean_and_max ? d_max_slots : nullptr,
                                        d_inv_offsets, d_inv_slots, d_out_grad_distances, d_out_grad_features, n_vert, n_neigh,

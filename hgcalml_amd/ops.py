@@ -450,7 +450,7 @@ def _accumulate_backward(grad_from_out_features, distances, features, neigh_indi
     if exp_weights and n and inv_slots.numel() == n * (k + 1):  # accumulate_gradient_index: the index of the whole table
         if w.data_ptr() % 16:
             w = w.clone()
-        need = lib.hgc_accumulate_knn_grad_scratch_bytes(n, k, f, int(mean_and_max))
+        need = lib.hgc_accumulate_knn_grad_quotient_bytes(n, k, f, int(mean_and_max))
         ws = workspace(need, dev) if need else None
         check(lib.hgc_accumulate_knn_grad_whole_index(p(g), p(w), p(x), p(max_slots), p(inv_offsets), p(inv_slots),
                                                       p(vertex_order_of(neigh_indices)), p(gw), p(gx), n, k, f, g.shape[1],
@@ -468,10 +468,13 @@ def _accumulate_backward(grad_from_out_features, distances, features, neigh_indi
         return (exp_neg_grad(gw, w) if exp_weights else gw), gx
     if exp_weights and w.data_ptr() % 16:
         w = w.clone()
-    need = lib.hgc_accumulate_knn_grad_scratch_bytes(n, k, f, int(mean_and_max))
+    order = vertex_order_of(neigh_indices)
+    # (with a processing order the weight gradients go to their slots one by one, without room for them in list order)
+    bytes_of = lib.hgc_accumulate_knn_grad_scratch_bytes if order is None else lib.hgc_accumulate_knn_grad_quotient_bytes
+    need = bytes_of(n, k, f, int(mean_and_max))
     ws = workspace(need, dev) if need else None
     check(lib.hgc_accumulate_knn_grad_scratch(p(g), p(w), p(x), p(mi), p(max_slots), p(idx), p(inv_offsets),
-                                              p(inv_slots), p(vertex_order_of(neigh_indices)), p(gw), p(gx), n, k, f,
+                                              p(inv_slots), p(order), p(gw), p(gx), n, k, f,
                                               g.shape[1], int(mean_and_max), int(exp_weights), p(ws),
                                               ws.numel() if need else 0, stream()))
     return gw, gx

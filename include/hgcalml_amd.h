@@ -420,8 +420,8 @@ int hgc_accumulate_knn_grad_records(const float *d_grad_from_out_features, const
  *   256 bytes): the weight gradients of large tables whose lists reach far are
  *   written in the order of d_inv_slots and moved to their slots. Not used with a
  *   d_vertex_order or a d_inv_slots that is on no 16-byte boundary.
- * Scratch that holds the first part alone is used for that (less is
- * HGC_ERR_WORKSPACE). The feature gradient has the same bits whatever there is
+ * Scratch that holds the first part alone, of the second query's size, is used
+ * for that (less is HGC_ERR_WORKSPACE). The feature gradient has the same bits whatever there is
  * of it, and the weight gradient has them with and without the second part. With
  * weights_are_exp the weights are exp(-d) and d_out_grad_distances receives the
  * gradient w.r.t. d, -(gradient w.r.t. the weight * weight), the bits of
@@ -429,6 +429,7 @@ int hgc_accumulate_knn_grad_records(const float *d_grad_from_out_features, const
  * boundaries). No single counterpart in the reference
  * (modules/accknn_op.py:52,71-89). */
 size_t hgc_accumulate_knn_grad_scratch_bytes(int n_vert, int n_neigh, int n_feat, int mean_and_max);
+size_t hgc_accumulate_knn_grad_quotient_bytes(int n_vert, int n_neigh, int n_feat, int mean_and_max);
 int hgc_accumulate_knn_grad_scratch(const float *d_grad_from_out_features, const float *d_distances,
                                     const float *d_feat, const int *d_max_feat_indices,
                                     const unsigned char *d_max_slots, const int *d_neigh_indices,
@@ -571,8 +572,9 @@ int hgc_sort_distinct_keys(unsigned long long *d_keys, long long n, int value_bi
  * fed with the inverse index of that whole table, which the distance gradient
  * needs anyway: the entries of its column 0 are left out. Same results as with
  * the index of the table itself. For shapes the query accepts (rows of 16 to 128
- * features, d_max_slots given with mean_and_max). No counterpart in the
- * reference. */
+ * features, d_max_slots given with mean_and_max). Of the scratch memory only the
+ * quotients are used (hgc_accumulate_knn_grad_quotient_bytes). No counterpart in
+ * the reference. */
 int hgc_accumulate_knn_grad_whole_index_covers(int n_vert, int n_neigh, int n_feat, int mean_and_max);
 int hgc_accumulate_knn_grad_whole_index(const float *d_grad_from_out_features, const float *d_distances,
                                         const float *d_feat, const unsigned char *d_max_slots,

@@ -119,3 +119,23 @@ def test_scratch_of_the_quotients_alone(n, k, f):
         assert bool((ws[quotients:] == 0x5a).all()) == (size < full)
         results.append((gw, gx))
     assert all(torch.equal(a, b) for a, b in zip(*results))
+
+
+@pytest.mark.parametrize("kind,n,k,asked", [("ordered", 250000, 64, 0), ("ordered", 400013, 40, 1), ("clone", 250000, 64, 2), ("block", 250000, 64, 0),
+                                            ("block", 400013, 40, 1)])
+def test_memory_is_asked_for_where_it_is_used(kind, n, k, asked, monkeypatch):
+    """tables with a processing order and the block's (which reads the index of the whole table) have room for the quotients (1)
+    or none (0), and only a table without an order has more (2); 64 features"""
+    from hgcalml_amd import AccumulateKnn, BinnedSelectKnn, RaggedGravNet, ops
+    torch.manual_seed(3)
+    sizes, real = [], ops.workspace
+    rs = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+    if kind == "block":
+        out = RaggedGravNet(8, k, 3, 8, 64).to(DEV)(torch.rand(n, 8, device=DEV), rs)[0]
+    else:
+        idx, dist = BinnedSelectKnn(k, torch.rand(n, 3, device=DEV), rs)
+        out, _ = AccumulateKnn(dist, torch.rand(n, 64, device=DEV, requires_grad=True), idx.clone() if kind == "clone" else idx)
+    monkeypatch.setattr(ops, "workspace", lambda size, dev: sizes.append(size) or real(size, dev))
+    out.sum().backward()
+    full, quotients = ops.lib.hgc_accumulate_knn_grad_scratch_bytes(n, k, 64, 1), (n * 64 * 4 + 255) // 256 * 256
+    assert (full in sizes, quotients in sizes) == (asked == 2, asked == 1)
