@@ -339,7 +339,7 @@ int launch(DenseRows p, int tiles, hipStream_t s) {
     if (!make_plan(FORM, p.steps, tiles, COORDS, plan)) return fail(HGC_ERR_INVALID_ARGUMENT, "layer too wide");
     switch (plan.tiles) {
         case 1: if constexpr (!kPairs) return launch_kernel<FORM, 1, COORDS>(p, plan, s); break;
-        case 2: return launch_kernel<FORM, 2, COORDS>(p, plan, s);
+        case 2: if constexpr (!kPairs) return launch_kernel<FORM, 2, COORDS>(p, plan, s); break;
         case 3: if constexpr (!kPairs) return launch_kernel<FORM, 3, COORDS>(p, plan, s); break;
         case 4: return launch_kernel<FORM, 4, COORDS>(p, plan, s);
         case 5: if constexpr (!kPairs) return launch_kernel<FORM, 5, COORDS>(p, plan, s); break;
