@@ -21,10 +21,12 @@ def check(got, terms, addend=None):
     return want
 
 
-# tiles of 16 columns and rows, widths of 4 up, remainders of both, several workgroups along the columns, the widest layers
-@pytest.mark.parametrize("n", [1, 16, 17, 2061])
+# tiles of 16 columns and rows, widths of 4 up, remainders of both, several workgroups along the columns, the widest layers, every
+# number of tiles a workgroup takes (output's gradient 4, 6, 8, 10, 12, input's 1 to 6, 8, 10, 12); with 150,011 rows a wave takes several tasks
+@pytest.mark.parametrize("n", [1, 16, 17, 2061, 150011])
 @pytest.mark.parametrize("x_width,f,c,o", [(4, 4, 1, 4), (5, 7, 2, 6), (16, 16, 4, 16), (17, 31, 3, 33), (64, 64, 4, 128),
-                                           (96, 128, 4, 160), (13, 129, 3, 100), (256, 128, 4, 256), (412, 50, 2, 255)])
+                                           (96, 128, 4, 160), (13, 129, 3, 100), (256, 128, 4, 256), (412, 50, 2, 255),
+                                           (48, 32, 3, 96), (70, 16, 4, 160), (180, 20, 4, 40), (500, 5, 1, 9)])
 def test_passes(n, x_width, f, c, o):
     from hgcalml_amd import ops
     gen = torch.Generator(device=DEV).manual_seed(n + f)
@@ -80,10 +82,11 @@ def layers_taken(monkeypatch):
     return seen
 
 
-def block(**kwargs):
+def block(sizes=(13, 9, 3, 30, 11), **kwargs):
+    """inputs, neighbours, coordinates, outputs, features"""
     from hgcalml_amd import RaggedGravNet
     torch.manual_seed(8)
-    return RaggedGravNet(13, 9, 3, 30, 11, **kwargs).to(DEV)
+    return RaggedGravNet(*sizes, **kwargs).to(DEV)
 
 
 X = dict(row_splits=[0, 5, 400, 700])
@@ -177,6 +180,18 @@ def test_frozen_parts_ask_for_no_gradient(frozen, x_grad, return_self, layers_ta
     assert got[0][0] and got[0][1] == (x_grad or "input_spatial_transform.weight" not in frozen)
 
 
+@pytest.mark.parametrize("frozen", [False, True])
+def test_what_is_kept_for_the_gradient(frozen, layers_taken):
+    """of the last layer its result and, for the weight's gradient, the joined rows; not what those were joined from"""
+    layer = block()
+    layer.output_feature_transform.weight.requires_grad_(not frozen)
+    kept = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: kept.append(tuple(t.shape)) or t, lambda t: t):
+        layer(torch.randn(700, 13, device=DEV), torch.tensor(X["row_splits"], dtype=torch.int32, device=DEV))
+    assert layers_taken == [1]
+    assert kept.count((700, 22)) == 0 and kept.count((700, 35)) == int(not frozen) and kept.count((700, 30)) == 1
+
+
 @pytest.mark.parametrize("second", [False, True])
 def test_derivative_of_the_derivative(second, layers_taken, monkeypatch):
     layer = block()
@@ -207,6 +222,9 @@ def test_blocks_that_are_left_alone(layers_taken):
     step(block(feature_activation="tanh"), x)
     layer = block()
     step(layer, x.detach().t().contiguous().t().requires_grad_(True))
+    for widths in ((13, 9, 5, 30, 11), (13, 9, 3, 30, 3), (13, 9, 3, 257, 11), (13, 9, 3, 30, 250), (13, 9, 3, 3, 11)):
+        step(block(widths), x)
+    step(block((3, 9, 3, 30, 11)), x.detach()[:, :3].contiguous().requires_grad_(True))
     with torch.autocast("cuda", dtype=torch.bfloat16):
         layer(x, torch.tensor(X["row_splits"], dtype=torch.int32, device=DEV))
     assert layers_taken == [] and calls == [1, 2]
