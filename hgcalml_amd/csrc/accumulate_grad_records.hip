@@ -531,8 +531,8 @@ int launch_records(const float *g, const float *feat, const uint4 *records, cons
 // gw[inv_slots[e]] = gw_list[e] for the entries of all targets (unless *wanted is 0), four per thread. The
 // scattered 4-byte writes of one stretch of the list fall into the rows of the source
 // vertices around it; each XCD works on one contiguous stretch, so the lines stay in
-// its L2 until they are full. (As a loop over 2048 workgroups every load waits for the stores in front of it: 64 M entries
-// 1000 us in the place of 460.)
+// its L2 until they are full. (64 M entries, window +-2000: workgroups of 256 threads 460 us, of 1024 411; as a loop over 2048
+// workgroups, where every load waits for the stores in front of it, 1000.)
 constexpr int kToTableThreads = 1024;
 
 __global__ __launch_bounds__(kToTableThreads) void weight_grad_to_table_kernel(const int *__restrict__ inv_off,

@@ -423,22 +423,25 @@ bool accumulate_grad_rows_covers(int n_feat, int n_neigh, bool mean_and_max, boo
 // whole and are written several times (fabric traffic five times the compulsory one at a million vertices, F = 128, window
 // +-2000). In the order of the lists the values leave in whole lines, and a pass moves them to their slots. Whether that pays
 // depends on how far apart the vertices of a list are; us of the gradient, slot by slot / in list order:
-//   span of the rows           table
-//   up to 2.6 MB   slower      a million, K = 64, F = 128, banded +-1000 3773 / 3912, +-300 3546 / 3761
-//   3.8 to 10 MB   faster      the same, +-1500 4318 / 3910, +-2000 4602 / 3985, +-3000 5127 / 4612, +-4000 6105 / 5966; K = 24, F = 64, +-4000 1680 /
-//                              1412, +-8000 2067 / 1996; 300,000, K = 64, F = 128, +-2000 1417 / 1216; 410,000, K = 40, F = 100, +-4000 1613 / 1492;
-//                              a search's table, hits ordered by a coordinate, K = 40, F = 128 1280 / 1273, a million, K = 64 4387 / 4100
-//   16 to 50 MB    slower      a million, K = 64, F = 128, +-6000 7358 / 7577, +-16000 8400 / 9018; K = 24, F = 64, +-16000 2420 / 2582; 300,000,
-//                              K = 64, F = 128, +-16000 2560 / 2805; search tables, hits in no order, 16 events of 410,000, K = 40, F = 128 2350 / 2426,
-//                              32 events of a million, K = 64 8249 / 8439
-//   beyond         slower      where all rows are up to 540 MB, twice the Infinity Cache: 300,000, K = 64, F = 128, +-32000 2869 / 3032; targets drawn at
-//                              random, 300,000, K = 64, F = 64 1808 / 1946, F = 128 2589 / 2812, 500,000, F = 64 2954 / 3318; a search's table of one event of
-//                              300,000, K = 64, F = 128 2592 / 2824; level: random, 410,000, K = 40, F = 128 2725 / 2726, 800,000, K = 24, F = 64 2352 / 2318
-//   beyond 79 MB   faster      where they are 670 MB and more: a million, K = 64, F = 128, +-32000 13385 / 11575, random 12771 / 11156; K = 24, F = 64, +-64000
-//                              3826 / 3384, random 3242 / 2950; random, 500,000, K = 64, F = 128 5263 / 4785, 700,000, K = 24, F = 128 3783 / 3482
-// So the host asks for the size (100,000, +-2000 359 / 353, 20,000 87 / 93; asking and moving nothing costs 10 to 15 us) and leaves tables with a
-// processing order as they are (300,000 vertices, K = 40, F = 128 907 / 1091), and the device looks at the span. (A mean alone gathers
-// half as much.)
+//   up to 2.6 MB of rows  slower: a million, K = 64, F = 128, banded +-1000 3773 / 3912, +-300 3546 / 3761
+//   3.8 to 10 MB          faster: the same, +-1500 4318 / 3910, +-2000 4602 / 3985, +-3000 5127 / 4612, +-4000 6105 / 5966; K = 24,
+//                         F = 64, +-4000 1680 / 1412, +-8000 2067 / 1996; 300,000, K = 64, F = 128, +-2000 1417 / 1216; 410,000,
+//                         K = 40, F = 100, +-4000 1613 / 1492; a search's table, hits ordered by a coordinate, K = 40, F = 128
+//                         1280 / 1273, a million, K = 64 4387 / 4100
+//   16 to 50 MB           slower: a million, K = 64, F = 128, +-6000 7358 / 7577, +-16000 8400 / 9018; K = 24, F = 64, +-16000
+//                         2420 / 2582; 300,000, K = 64, F = 128, +-16000 2560 / 2805; search tables, hits in no order, 16 events of
+//                         410,000, K = 40, F = 128 2350 / 2426, 32 events of a million, K = 64 8249 / 8439 (but with K = 24 near
+//                         50 MB F = 64, +-32000 2828 / 2767, a search's table of 700,000, F = 128 3006 / 2939)
+//   beyond, where all     slower: 300,000, K = 64, F = 128, +-32000 2869 / 3032; targets drawn at random, 300,000, K = 64, F = 64
+//   rows are up to 540    1808 / 1946, F = 128 2589 / 2812, 500,000, F = 64 2954 / 3318; a search's table of one event of 300,000,
+//   MB, twice the         K = 64, F = 128 2592 / 2824; level: random, 410,000, K = 40, F = 128 2725 / 2726, 800,000, K = 24, F = 64
+//   Infinity Cache        2352 / 2318
+//   beyond 79 MB, where   faster: a million, K = 64, F = 128, +-32000 13385 / 11575, random 12771 / 11156; K = 24, F = 64, +-64000
+//   they are 670 MB and   3826 / 3384, random 3242 / 2950; random, 500,000, K = 64, F = 128 5263 / 4785, 700,000, K = 24, F = 128
+//   more                  3783 / 3482
+// So the host asks for the size (100,000, +-2000 359 / 353, 20,000 87 / 93; asking and moving nothing costs 10 to 20 us) and leaves
+// tables with a processing order as they are (300,000 vertices, K = 40, F = 128 907 / 1091), and the device looks at the span. (A
+// mean alone gathers half as much.)
 constexpr int kSpanSamples = 1024;
 constexpr float kSpanNear = 3 << 20, kSpanFar = 12 << 20, kSpanWhole = 64 << 20;  // bytes; an XCD's L2 has 4 MB
 constexpr long long kRowsWhole = 600ll << 20;

@@ -20,12 +20,14 @@
 // (the ones it has twice count once), and behind the last row stands the last row again: no load or store is left out, so
 // none stands in a branch, which would make waiting for a load mean waiting for everything after it.
 // Measured next to the library products with mask, sums and the join's gradient as passes of their own, us, a gigabyte written
-// between calls (inputs come from memory): 150,000 rows, 64 inputs, 64 features, 128 outputs: output's gradient 197 -> 134, input's
-// 145 -> 80; 240,011 rows, 48, 32, 96: 248 -> 151, 173 -> 74; 20,000 rows, 64, 64, 128: 52 -> 30, 45 -> 17. In a training step of the block
-// the two take 122 and 52 us, and 135 and 48. The step 1973 -> 1759 and 1999 -> 1735 (35 and 45 of it elsewhere), 2477 points
-// 856 -> 730 (the host's time). Error against 64 bits (2-norm, 150,000 rows), here and library: gradient of the accumulated rows
-// 8.7e-8 and 1.5e-7, of the joined x the same, input's 5.6e-8 and 6.4e-8. Tried and taken back: 8 waves instead of 16, one chain of
-// products over all columns (twice the error), higher priority while multiplying, whole ranges of rows per workgroup or XCD.
+// between calls (inputs come from memory): 150,000 rows, 64 inputs, 64 features, 128 outputs: output's gradient 197 -> 134,
+// input's 145 -> 80; 240,011 rows, 48, 32, 96: 248 -> 151, 173 -> 74; 20,000 rows, 64, 64, 128: 52 -> 30, 45 -> 17. In a training
+// step of the block the two take 122 and 52 us, and 135 and 48. The step 1973 -> 1759 and 1999 -> 1735 (35 and 45 of it elsewhere),
+// 2477 points 856 -> 730 (the host's time; runs of one side differ by 8 %). In the step of 150,000 points the matrix cores are busy
+// for 37 and 14 % of the two passes, and 3.9 and 4.9 TB/s move past the L2 (470 and 254 MB, 384 and 233 needed). Error against 64 bits
+// (2-norm, 150,000 rows), here and library: gradient of the accumulated rows 8.7e-8 and 1.5e-7, of the joined x the same, input's
+// 5.6e-8 and 6.4e-8. Tried and taken back: 8 waves instead of 16, one chain of products over all columns (twice the error), higher
+// priority while multiplying, whole ranges of rows per workgroup or XCD.
 #include <algorithm>
 
 #include "hgc_common.hpp"

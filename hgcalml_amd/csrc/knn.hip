@@ -73,8 +73,9 @@ struct KnnParams {
 // vector register and back, four at a time, by vector instructions, of which the search is made. (With these, the grid's
 // numbers by scalar loads, the first cube's prefix sum used again and no last merge for up to 32 keys: 474 -> 436 vector
 // instructions per query of the batch of 16 events, 1156 -> 1097 us; 100,000 2-D Gaussian points, K = 10 124 -> 117; 150,000 4-D
-// points, K = 64 1074 -> 1039, 362 -> 356. Seven waves with more registers: 1200. Half-widths 1 and 2 of the first cube
-// looked up together: 1115.)
+// points, K = 64 1074 -> 1039, 362 -> 356. One of the others taken out again, the batch, three runs each, 1109 to 1119 us with all of
+// them: scalar loads 1119 to 1124, prefix sum 1122 to 1133, last merge 1129 to 1137; 1174 without any. Seven waves with more
+// registers: 1200. Half-widths 1 and 2 of the first cube looked up together: 1115.)
 typedef const __attribute__((address_space(4))) KnnParams *KernelArgs;
 __device__ __forceinline__ KernelArgs kernel_args() {
     KernelArgs a = (KernelArgs)__builtin_amdgcn_kernarg_segment_ptr();
