@@ -666,11 +666,12 @@ int hgc_dense_weight_grad(const float *d_grad, const float *d_x, long long n_row
  *   output layer d_out [., n_out] = max(j W^T + bias, 0), j = the rows of hgc_gravnet_join:
  *                  m = d_grad where d_out > 0, to d_masked; m W to
  *                  d_grad_acc, d_grad_features and d_grad_x as in hgc_gravnet_join_grad
- *   gradient of the features x W_f^T + bias and the coordinates x W_c^T: m = d_grad_features + d_grad_features2 (may be NULL), with relu
+ *   features max(x W_f^T + bias, 0) (without relu: as they are) and coordinates x W_c^T:
+ *                  m = d_grad_features + d_grad_features2 (may be NULL), with relu
  *                  where d_features > 0, to d_masked; d_grad_in = m W_f
  *                  + d_grad_coords W_c + d_grad_x, the last two may be NULL
  * The query says whether the widths are covered (4 and more, 2 n_feat + n_x up to 512, n_out up to
- * 256, n_coords 1 to 4). x needs no alignment beyond that of float.
+ * 256, n_coords 1 to 4). No alignment beyond that of float.
  * No counterpart in the reference (Keras does it). */
 int hgc_gravnet_dense_covers(int n_feat, int n_x, int n_out, int n_coords);
 int hgc_gravnet_output_layer_grad(const float *d_grad, const float *d_out, int n_vert, int n_feat,

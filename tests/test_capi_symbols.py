@@ -118,7 +118,8 @@ def test_limits_of_the_gravnet_passes(capi):
 
 
 def test_scratch_of_the_accumulation_gradient(capi):
-    """one float per vertex and feature, and none where the kernel that reads it is not taken"""
+    """the quotients: one float per vertex and feature, and none where the kernel that reads it is not taken (small tables; large ones
+    in the next test)"""
     f = capi.hgc_accumulate_knn_grad_scratch_bytes
     f.restype, f.argtypes = ctypes.c_size_t, [ctypes.c_int] * 4
     for mean_and_max in (0, 1):
